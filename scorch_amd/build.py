@@ -98,6 +98,37 @@ def build_library(force: bool = False, verbose: bool = False) -> str:
     return LIB_PATH
 
 
+HOST_SRC = os.path.join(SRC_DIR, "host.cpp")
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
+
+
+def build_host(force: bool = False, verbose: bool = False) -> str:
+    """Compile csrc/host.cpp, the native call path of the Python layer (no device code), against
+    torch's headers and libscorch_hip.so.  Returns the module's path."""
+    if not force and not _newer(HOST_PATH, [HOST_SRC] + _headers()):
+        return HOST_PATH
+    import sysconfig
+    import torch
+    gxx = shutil.which("g++")
+    if not gxx:
+        raise RuntimeError("g++ not found: cannot build _host.so")
+    base = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = [gxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           "-isystem", os.path.join(base, "include"), "-isystem", os.path.join(base, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"], HOST_SRC,
+           "-L", PKG_DIR, "-l:libscorch_hip.so", "-L", os.path.join(base, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+           "-ltorch_python", "-lamdhip64", "-Wl,-rpath,$ORIGIN", "-o", HOST_PATH + ".tmp"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + proc.stdout)
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
+    return HOST_PATH
+
+
 HOST_DEMO_SRC = os.path.join(os.path.dirname(PKG_DIR), "tests", "host_c", "plan_demo.c")
 HOST_DEMO_BIN = os.path.join(os.path.dirname(PKG_DIR), "tests", "host_c", "plan_demo")
 
@@ -124,4 +155,5 @@ def build_host_demo(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     print(build_library(force="--force" in sys.argv, verbose=True))
+    print(build_host(force="--force" in sys.argv, verbose=True))
     print(build_host_demo(verbose=True))

@@ -71,6 +71,7 @@ class TensorFormat:
                 level_formats = list(level_formats)
             levels = [lf if isinstance(lf, LevelFormat) else LevelFormat(lf) for lf in level_formats]
         self._level_formats = levels
+        self._text = None
 
     def get_level_formats(self) -> List[LevelFormat]:
         return self._level_formats
@@ -85,7 +86,10 @@ class TensorFormat:
         return all(t == LevelType.DENSE for t in self.get_level_types())
 
     def __str__(self) -> str:
-        return ",".join(str(lf) for lf in self._level_formats)
+        text = self._text
+        if text is None:
+            text = self._text = ",".join(str(lf) for lf in self._level_formats)
+        return text
 
     __repr__ = __str__
 

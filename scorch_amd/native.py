@@ -165,6 +165,27 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native call path for products that have been decided (csrc/host.cpp), bound to this package."""
+    global _host
+    if _host is None:
+        handle = lib()          # (also builds both libraries if they are missing)
+        with _lock:
+            if _host is None:
+                if not os.path.exists(_build.HOST_PATH):
+                    _build.build_host()
+                from . import _host as module
+                from . import scorch_ops_hip
+                from .stensor import STensor
+                module.bind(vars(scorch_ops_hip), STensor, scorch_ops_hip._torch_empty, check)
+                _host = module
+        del handle
+    return _host
+
+
 def kernel_times(call):
     """Run ``call()`` (one library call, or several) and return the duration of each
     kernel it launched, in milliseconds, in launch order (scorch_hip_timing_begin /

@@ -19,7 +19,7 @@ from typing import Any, List, Optional, Union
 
 import torch
 
-from . import scorch_ops_hip
+from . import native, scorch_ops_hip
 from .format import TensorFormat, parse_format
 from .prebuilt_kernels import (_timed, execute_prebuilt_binary_kernel, resolve_prebuilt_fused,
                                resolve_prebuilt_matmul)
@@ -168,12 +168,15 @@ def _matmul_csr_dense_direct(a: STensor, b: torch.Tensor, kwargs) -> Optional[to
         return None
     if b.layout != torch.strided or b.dim() not in (1, 2) or a.dim() != 2 or not b.is_cuda:
         return None
-    if str(a.format) != "d,s" or a.index.mode_order != [0, 1] or not a.values.is_cuda:
+    a_format = str(a.format)
+    if a_format not in ("d,s", "o,o") or a.index.mode_order != [0, 1] or not a.values.is_cuda:
         return None
     if a.shape[1] != b.shape[0]:
         return None          # the general path words the error
     key = (a.values.dtype, b.dtype, b.dim())
-    fn = _direct_matmul.get(key)
+    fn = _direct_matmul.get(key) if a_format == "d,s" else _coo_matmul_symbol(key)
+    if fn is None and a_format == "o,o":
+        return None
     if fn is None:
         resolved = resolve_prebuilt_matmul(a, STensor.from_torch(b), output_format=None)
         if resolved is None or not resolved.output_format.is_dense():
@@ -186,7 +189,34 @@ def _matmul_csr_dense_direct(a: STensor, b: torch.Tensor, kwargs) -> Optional[to
     result = _timed(lambda: fn(result_shape, a.shape, a.index.mode_indices, a.values,
                                tuple(b.shape), [[] for _ in range(b.dim())], values),
                     a.values.device, kwargs.get("time_dict", None))
+    if values.data_ptr() == b.data_ptr():
+        scorch_ops_hip.remember_spmm(a, b.shape[1] if b.dim() == 2 else -1)
     return result.storage.value.view(result_shape)
+
+
+def _coo_matmul_symbol(key):
+    """The product of a coordinate operand and a dense matrix: one registry entry, fp32."""
+    return scorch_ops_hip.spmm_coo_float if key == (torch.float32, torch.float32, 2) else None
+
+
+# The native call path (csrc/host.cpp): serves products that have been decided, None for all others.
+def _decided_spmm(*args):
+    global _decided_spmm
+    if not torch.cuda.is_available():
+        return None
+    _decided_spmm = native.host().spmm
+    return _decided_spmm(*args)
+
+
+def _decided_sddmm(*args):
+    global _decided_sddmm
+    if not torch.cuda.is_available():
+        return None
+    _decided_sddmm = native.host().sddmm
+    return _decided_sddmm(*args)
+
+
+_DENSE_NAMES = {"dd": 2, "d": 1}
 
 
 def matmul(a: Union[torch.Tensor, STensor], b: Union[torch.Tensor, STensor],
@@ -194,6 +224,10 @@ def matmul(a: Union[torch.Tensor, STensor], b: Union[torch.Tensor, STensor],
     """Matrix product.  Keyword arguments as in the reference: ``format`` /
     ``output_format``, ``use_cache``, ``time_dict``."""
     if isinstance(a, STensor) and isinstance(b, torch.Tensor):
+        if not kwargs or (len(kwargs) == 1 and _DENSE_NAMES.get(kwargs.get("format", None)) == b.dim()):
+            out = _decided_spmm(a, b, None, 0)
+            if out is not None:
+                return out
         direct = _matmul_csr_dense_direct(a, b, kwargs)
         if direct is not None:
             return direct
@@ -292,7 +326,22 @@ def _sddmm_direct(mask, A, B, time_dict) -> Optional[STensor]:
                                    tuple(A.shape), dense_index, A.reshape(-1),
                                    tuple(B.shape), dense_index, B.reshape(-1)),
                         mask.values.device, time_dict)
+    scorch_ops_hip.remember_sddmm(mask, int(A.shape[1]))
     return _wrap(result_cpp, mask.shape, mask.format if mask_fmt == "o,o" else "oo")
+
+
+_coordinate_format = parse_format("oo")
+
+
+def _sddmm_result(mask: STensor, values: torch.Tensor, rows: Optional[torch.Tensor]) -> STensor:
+    """_wrap for a decided SDDMM: the mask's own index tensors (coordinates), or the pattern's row
+    coordinates and the mask's columns (CSR)."""
+    index = TensorIndex.__new__(TensorIndex)
+    modes = mask.index.mode_indices
+    index.format = mask.format if rows is None else _coordinate_format
+    index.mode_indices = modes if rows is None else [[rows], [modes[1][1]]]
+    index.mode_order = [0, 1]
+    return STensor(shape=mask.shape, index=index, value=values)
 
 
 def einsum(expression: str, *tensors: Optional[Union[torch.Tensor, STensor]],
@@ -306,11 +355,19 @@ def einsum(expression: str, *tensors: Optional[Union[torch.Tensor, STensor]],
     time_dict = kwargs.get("time_dict", None)
     requested = kwargs.get("format", kwargs.get("output_format", None))
     if canon == _SDDMM_EXPR and len(tensors) == 3 and requested is None:
+        if not kwargs:
+            decided = _decided_sddmm(*tensors)
+            if decided is not None:
+                return _sddmm_result(tensors[0], *decided)
         direct = _sddmm_direct(*tensors, time_dict)
         if direct is not None:
             return direct
     if canon in (_SPMM_EXPR, "ab,b->a") and len(tensors) == 2 and isinstance(tensors[0], STensor) \
             and isinstance(tensors[1], torch.Tensor) and tensors[1].dim() == (2 if canon == _SPMM_EXPR else 1):
+        if not kwargs:
+            out = _decided_spmm(tensors[0], tensors[1], None, 0)
+            if out is not None:
+                return out
         direct = _matmul_csr_dense_direct(tensors[0], tensors[1], kwargs)   # the same product as matmul's
         if direct is not None:
             return direct
@@ -403,6 +460,9 @@ def spmm_bias_act(a: STensor, b: Union[torch.Tensor, STensor], bias: torch.Tenso
     """``act(a @ b + bias)`` in one kernel: the call the reference's
     ``@scorch.compile`` makes when it recognises matmul -> add(bias) [-> relu]
     (src/scorch/trace.py:232-301).  Returns an (M, N) tensor."""
+    out = _decided_spmm(a, b, bias, 2 if relu else 1)
+    if out is not None:
+        return out
     kinds = ("add", "relu") if relu else ("add",)
     if isinstance(b, torch.Tensor) and b.layout == torch.strided and b.dim() == 2:
         # a dense torch operand is handed to the kernel as it is (no STensor around it)
@@ -427,4 +487,6 @@ def spmm_bias_act(a: STensor, b: Union[torch.Tensor, STensor], bias: torch.Tenso
             raise _not_on_device(values.device)
     M, N = a.shape[0], b_shape[1]
     out = fn((M, N), a.shape, a.index.mode_indices, a.values, b_shape, b_index, b_values, bias)
+    if isinstance(b, torch.Tensor):
+        scorch_ops_hip.remember_spmm(a, N, 2 if relu else 1)
     return out.storage.value.view(M, N)

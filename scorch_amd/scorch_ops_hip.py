@@ -32,7 +32,7 @@ from . import native
 
 # Every buffer this module allocates comes from these two names, so that a test can put a
 # poisoning allocator in their place: no kernel may depend on what a fresh buffer holds.
-_empty = torch.empty
+_torch_empty = _empty = torch.empty
 _empty_like = torch.empty_like
 
 HINT_MOSTLY_EMPTY_ROWS = 0x100      # SCORCH_HIP_HINT_MOSTLY_EMPTY_ROWS of include/scorch_hip.h
@@ -172,7 +172,7 @@ class _on_device:
 # pointer, a numpy or DLPack alias, a kernel of another library, or the replay of a recorded graph:
 # after such a write call forget(t), or mark the tensor volatile once.
 _CACHE_ATTRIBUTES = ("_scorch_plan", "_scorch_tiled", "_scorch_seen", "_scorch_ones", "_scorch_listed", "_scorch_coo_pos",
-                     "_scorch_block_mask", "_scorch_mask_checked", "_scorch_rows")
+                     "_scorch_block_mask", "_scorch_mask_checked", "_scorch_rows", "_scorch_row_order", "_scorch_attention")
 
 
 def _tensors_of(obj, seen=None):
@@ -220,11 +220,19 @@ def _same(ref, t: torch.Tensor) -> bool:
     return ref is not None and ref() is t
 
 
+def _decide_anew() -> None:
+    """Products that the native call path (csrc/host.cpp) serves without asking this module are all
+    decided again on their next call."""
+    if native._host is not None:
+        native._host.advance()
+
+
 def forget(*objs) -> None:
     """Drop everything this module has derived from the given tensors (or from the tensors of the
     given STensors, results, lists): the next call inspects, plans and copies anew.  For writes that
     PyTorch's version counter does not see -- ``t.data``, raw pointers, numpy / DLPack aliases,
     kernels of other libraries, replays of recorded graphs."""
+    _decide_anew()
     for t in _tensors_of(objs):
         for name in _CACHE_ATTRIBUTES:
             if hasattr(t, name):
@@ -243,6 +251,7 @@ def mark_volatile(*objs, volatile: bool = True) -> None:
     recorded graph, buffers another library writes): nothing derived from their values -- the
     column-tile copy, the all-ones verdict -- is kept or used from now on.  What is derived from an
     index tensor (a sparsity pattern) is not affected: use forget() when a pattern is rewritten."""
+    _decide_anew()
     for t in _tensors_of(objs):
         if volatile:
             for name in ("_scorch_tiled", "_scorch_seen", "_scorch_ones", "_scorch_listed"):
@@ -381,6 +390,15 @@ class BlockedCsr:
     __slots__ = ("n_active", "block_row_ptr", "block_col_idx", "block_words", "block_off", "block_cols", "block_nnz",
                  "sddmm_items", "spmm_items", "n_spmm_items", "spmm_split_rows", "n_spmm_split_rows", "n_spmm_slots",
                  "n_block_rows", "longest_block_row", "fill")
+
+    def sddmm_items_for(self, heads: int):
+        """(work items, their number) of an SDDMM of so many heads: the largest that still give every
+        workgroup slot of the chip one (1,024: 256 CUs x 4), else the smallest."""
+        for stretch in BLOCKED_STRETCHES:
+            items, n_items = self.sddmm_items[stretch]
+            if n_items * heads >= 1024:
+                break
+        return items, n_items
 
 
 def _describe_blocks(pos: torch.Tensor, crd: torch.Tensor, M: int, n_cols: int, min_fill: float = 0.0):
@@ -527,13 +545,8 @@ def _blocked(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, width: int)
 
 def _blocked_sddmm(L, bl: BlockedCsr, heads: int, M: int, n_cols: int, K: int, nnz: int, mask_vals,
                    a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, rows_ptr, stream: int) -> int:
-    """Launch the block SDDMM for `heads` pairs of dense operands over one pattern: with the
-    largest work items that still give every workgroup slot of the chip one (1,024: 256 CUs x 4),
-    else the smallest."""
-    for stretch in BLOCKED_STRETCHES:
-        items, n_items = bl.sddmm_items[stretch]
-        if n_items * heads >= 1024:
-            break
+    """Launch the block SDDMM for `heads` pairs of dense operands over one pattern."""
+    items, n_items = bl.sddmm_items_for(heads)
     return L.scorch_hip_sddmm_csr_blocked_f32(
         heads, M, n_cols, K, nnz, bl.n_active, bl.block_col_idx.data_ptr(), bl.block_words.data_ptr(),
         bl.block_off.data_ptr(), n_items, items.data_ptr(),
@@ -716,9 +729,7 @@ def _spmm(dtype, result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mod
             tiled = _tiled_operand(B_values, K, N, nnz, L)
         elif path == "tiled" and dtype == torch.float32:
             tiled = prepare_dense_operand(B_values, K, N)
-        # most rows empty and a result large enough for two more launches not to show: one streaming
-        # fill of the result, then only the rows that have entries (merge-path kernel)
-        fill_first = plan is not None and bias is None and 2 * plan.empty_rows >= M and M * N * elem >= (32 << 20)
+        fill_first = _fill_first(plan, M, N, elem, bias is not None)
         if path == "auto" and tiled is None and dtype == torch.float32 and bias is None and act == 0:
             bl = _blocked(plan, pos, crd, M, K, N)
             if bl is not None:
@@ -750,6 +761,74 @@ def _spmm(dtype, result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mod
     result = Tensor(out, [[], []])
     result.workspace = ws      # a buffer handed out during a graph capture lives as long as the result
     return result
+
+
+# What the native call path does with a decided product (the enum Kind of csrc/host.cpp)
+_ROUTE_ROWS, _ROUTE_PLANNED, _ROUTE_BLOCKED_SPMM, _ROUTE_SPMV, _ROUTE_SDDMM_CSR, _ROUTE_SDDMM_LISTED, _ROUTE_SDDMM_COO, \
+    _ROUTE_BLOCKED_SDDMM, _ROUTE_TILED = range(9)
+
+
+def remember_spmm(a, width: int, act: int = 0) -> None:
+    """After a product of the STensor `a` with a dense operand of `width` columns (-1: a vector) has
+    gone the general way: if nothing about such products is open any more -- the pattern is
+    planned, whether it is made of blocks is known -- hand the outcome to the native call path,
+    which serves the next ones.  `act` 0: no bias, 1: bias, 2: bias and ReLU."""
+    if SPMM_PATH != "auto" or torch.cuda.is_current_stream_capturing():
+        return
+    modes, vals = a.index.mode_indices, a.values
+    pos_of_coo = ()
+    if len(modes) == 2 and len(modes[1]) == 2:
+        pos, crd = modes[1]
+    elif len(modes) == 2 and len(modes[0]) == 1 and len(modes[1]) == 1:
+        known = _known_row_order(modes[0][0], int(a.shape[0]))
+        if known is None or known[1] is not None:           # (not in row order: its values are gathered on every call)
+            return
+        pos, crd = known[0], modes[1][0]
+        pos_of_coo = (None,) * 7 + (pos,)
+    else:
+        return
+    M, K, nnz = int(a.shape[0]), int(a.shape[1]), vals.numel()
+    if M == 0 or width == 0 or vals.dtype not in _SUFFIX:
+        return
+    plan = csr_plan(pos, crd, M, K, "A")
+    if plan is None:
+        return
+    L, elem, dev, host = native.lib(), vals.element_size(), vals.device, native.host()
+
+    def remember(kind, ints=(), tensors=(), workspace=0, may_tile=False):
+        if pos_of_coo:
+            tensors = tuple(tensors) + pos_of_coo[len(tensors):]
+        host.remember(a, kind, width, act, tuple(ints), tuple(tensors), workspace, may_tile, 0, None, SPMM_PATH, BLOCKED_PATH)
+
+    if width < 0:
+        if not pos_of_coo:
+            remember(_ROUTE_SPMV, workspace=L.scorch_hip_spmv_csr_workspace_bytes(M, nnz, elem))
+        return
+    may_tile = width >= 512 and vals.dtype == torch.float32 and bool(L.scorch_hip_dense_tiled_recommended(K, width, nnz, 4))
+    if act == 0 and vals.dtype == torch.float32 and BLOCKED_PATH != "off" and width in BLOCKED_WIDTHS:
+        if plan.blocked is None:
+            return
+        bl = _blocked(plan, pos, crd, M, K, width)
+        if bl is not None:
+            remember(_ROUTE_BLOCKED_SPMM, (bl.n_active, bl.n_spmm_items, bl.n_spmm_split_rows, bl.n_spmm_slots),
+                     (bl.block_col_idx, bl.block_words, bl.block_off, bl.block_cols, bl.spmm_items, bl.spmm_split_rows),
+                     L.scorch_hip_spmm_csr_blocked_workspace_bytes(1, bl.n_spmm_slots, width) if bl.n_spmm_slots else 0)
+            return
+    fill_first = _fill_first(plan, M, width, elem, act != 0)
+    if not may_tile and not fill_first and plan.max_row <= ROWS_KERNEL_MAX_ROW:
+        remember(_ROUTE_ROWS)
+        return
+    with _on_device(dev):
+        bounds = _chunk_bounds(plan, pos, M, nnz, width, elem, L, _stream(dev))
+    remember(_ROUTE_TILED if may_tile else _ROUTE_PLANNED,
+             (bounds.numel(), HINT_MOSTLY_EMPTY_ROWS if fill_first else 0, plan.max_row), (bounds,),
+             L.scorch_hip_spmm_csr_workspace_bytes(M, nnz, width, elem), may_tile)
+
+
+def _fill_first(plan: Optional[CsrPlan], M: int, N: int, elem: int, with_bias: bool) -> bool:
+    """Most rows empty and a result large enough for two more launches not to show: one streaming
+    fill of the result, then only the rows that have entries (merge-path kernel)."""
+    return plan is not None and not with_bias and 2 * plan.empty_rows >= M and M * N * elem >= (32 << 20)
 
 
 def _make_spmm(dtype):
@@ -953,6 +1032,12 @@ SDDMM_PATHS = ("auto", "plain", "listed")
 SDDMM_PATH = os.environ.get("SCORCH_HIP_SDDMM_PATH", "auto")
 
 
+def _lists_apply(nnz: int, n_cols: int, K: int) -> bool:
+    """Whether SDDMMs of this shape are served from per-XCD entry lists when their mask comes back: B
+    beyond one L2 and within the eight together, and used often enough."""
+    return 0 < K <= 256 and (8 << 20) <= n_cols * K * 4 <= (20 << 20) and nnz >= 4 * n_cols
+
+
 def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int, L, stream) -> Optional[torch.Tensor]:
     """The mask's per-XCD entry lists if this product should use them (built on the
     second such product with the mask), else None."""
@@ -961,8 +1046,7 @@ def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int,
     if SDDMM_PATH == "plain" or plan is None or K > 256 or K == 0 or crd.numel() == 0:
         return None
     if SDDMM_PATH == "auto":
-        b_bytes = n_cols * K * 4
-        if not (8 << 20) <= b_bytes <= (20 << 20) or crd.numel() < 4 * n_cols:
+        if not _lists_apply(crd.numel(), n_cols, K):
             return None
         plan.sddmm_uses += 1
         if plan.sddmm_lists is None and (plan.sddmm_uses < 2 or torch.cuda.is_current_stream_capturing()):
@@ -989,13 +1073,17 @@ def _sddmm_dense_args(S_shape, A_shape, A_values, B_shape, B_values):
     return M, n_cols, K, a, b
 
 
+def _coo_mask_may_be_blocked(row: torch.Tensor, M: int, n_cols: int, K: int) -> bool:
+    return not (BLOCKED_PATH == "off" or not plans_enabled() or K not in BLOCKED_WIDTHS or M % 64 or n_cols % 64
+                or row.numel() < 8 * M or M == 0)
+
+
 def _coo_mask_row_ptr(row: torch.Tensor, col: torch.Tensor, M: int, n_cols: int, K: int) -> Optional[torch.Tensor]:
     """The row pointer of a coordinate mask that may be one for the block kernels (dimensions
     multiples of 64, a dense width they serve, eight entries per row or more), once the same
     coordinate tensors have come back unchanged; None otherwise, and for coordinates that are
     not in row order.  Kept with the row tensor (one kernel and one host read, once)."""
-    if BLOCKED_PATH == "off" or not plans_enabled() or K not in BLOCKED_WIDTHS or M % 64 or n_cols % 64 \
-            or row.numel() < 8 * M or M == 0:
+    if not _coo_mask_may_be_blocked(row, M, n_cols, K):
         return None
     key = (_stamp(row), _stamp(col), M)
     seen = getattr(row, "_scorch_coo_pos", None)
@@ -1095,6 +1183,65 @@ def sddmm_csr_float(result_shape, S_shape, S_mode_indices, S_values, A_shape, A_
     return Tensor(out, [[rows], [crd]])
 
 
+def remember_sddmm(mask, K: int) -> None:
+    """remember_spmm for an SDDMM over the STensor `mask` with dense operands of depth K: handed over
+    once the kernel and what is known about the mask's values are settled."""
+    modes, vals = mask.index.mode_indices, mask.values
+    if SDDMM_PATH != "auto" or BLOCKED_PATH not in BLOCKED_PATHS or vals.dtype != torch.float32 or K == 0 \
+            or torch.cuda.is_current_stream_capturing() or is_volatile(vals) or vals.numel() == 0:
+        return
+    seen = getattr(vals, "_scorch_ones", None)
+    if seen is None or seen[0] != _stamp(vals) or seen[1] is None:
+        return
+    M, n_cols, nnz = int(mask.shape[0]), int(mask.shape[1]), vals.numel()
+    read_values = not seen[1]
+    host = native.host()
+
+    def remember(kind, ints=(), tensors=(), rows=None):
+        host.remember(mask, kind, K, 3, tuple(ints), tuple(tensors), 0, False, read_values, rows, SDDMM_PATH, BLOCKED_PATH)
+
+    def remember_blocked(bl, rows):
+        items, n_items = bl.sddmm_items_for(1)
+        remember(_ROUTE_BLOCKED_SDDMM, (bl.n_active, n_items), (bl.block_col_idx, bl.block_words, bl.block_off, items), rows)
+
+    if len(modes) == 2 and len(modes[1]) == 2:
+        pos, crd = modes[1]
+        plan = csr_plan(pos, crd, M, n_cols, "S")
+        if plan is None or plan.rows is None:
+            return
+        if BLOCKED_PATH != "off" and K in BLOCKED_WIDTHS:
+            if plan.blocked is None:
+                return
+            bl = _blocked(plan, pos, crd, M, n_cols, K)
+            if bl is not None:
+                remember_blocked(bl, plan.rows)
+                return
+        if _lists_apply(crd.numel(), n_cols, K):
+            listed = getattr(vals, "_scorch_listed", None)
+            if plan.sddmm_lists is None or (read_values and (listed is None or listed[0] != _stamp(vals)
+                                                             or listed[1] is not plan.sddmm_lists)):
+                return
+            remember(_ROUTE_SDDMM_LISTED, (plan.sddmm_lists.numel(),),
+                     (plan.sddmm_lists,) + ((listed[2],) if read_values else ()), plan.rows)
+            return
+        remember(_ROUTE_SDDMM_CSR, rows=plan.rows)
+    elif len(modes) == 2 and len(modes[0]) == 1 and len(modes[1]) == 1:
+        row, col = modes[0][0], modes[1][0]
+        if _coo_mask_may_be_blocked(row, M, n_cols, K):
+            seen = getattr(row, "_scorch_coo_pos", None)
+            if seen is None or seen[0] != (_stamp(row), _stamp(col), M) or not _same(seen[2], col) or seen[1] is None:
+                return
+            if seen[1] is not False:
+                plan = csr_plan(seen[1], col, M, n_cols, "S")
+                if plan is None or plan.blocked is None:
+                    return
+                bl = _blocked(plan, seen[1], col, M, n_cols, K)
+                if bl is not None:
+                    remember_blocked(bl, None)
+                    return
+        remember(_ROUTE_SDDMM_COO)
+
+
 # ---- neighbours of the path ---------------------------------------------------------
 SOFTMAX_SHORT_ROW = 4096     # rows up to this length never reach the row softmax's giant-row pass
 
@@ -1175,14 +1322,36 @@ def _coo_as_csr(mode_indices, values, n_rows: int, what: str):
     rows, cols = _index(mode_indices[0][0], what + " rows"), _index(mode_indices[1][0], what + " columns")
     if rows.numel() != cols.numel() or rows.numel() != values.numel():
         raise ValueError(f"scorch_ops_hip: {what}: coordinate and value arrays differ in length")
-    pos = coo_row_ptr(rows, n_rows)
-    if pos is None:
-        if rows.numel() and (int(rows.min()) < 0 or int(rows.max()) >= n_rows):
-            raise ValueError(f"scorch_ops_hip: {what} has a row coordinate outside [0, {n_rows})")
-        rows, order = torch.sort(rows, stable=True)
-        cols, values = cols[order].contiguous(), values[order].contiguous()
-        pos = coo_row_ptr(rows, n_rows)
+    known = _known_row_order(rows, n_rows)
+    if known is None:
+        pos, order = coo_row_ptr(rows, n_rows), None
+        if pos is None:
+            if rows.numel() and (int(rows.min()) < 0 or int(rows.max()) >= n_rows):
+                raise ValueError(f"scorch_ops_hip: {what} has a row coordinate outside [0, {n_rows})")
+            in_order, order = torch.sort(rows, stable=True)
+            pos = coo_row_ptr(in_order, n_rows)
+        known = (pos, order, {})
+        if plans_enabled():
+            try:
+                rows._scorch_row_order = (_stamp(rows), n_rows, known)
+            except (AttributeError, RuntimeError):
+                pass
+    pos, order, sorted_cols = known
+    if order is not None:
+        key = _stamp(cols)
+        kept = sorted_cols.get("cols")
+        if kept is None or kept[0] != key or not _same(kept[1], cols):
+            kept = sorted_cols["cols"] = (key, weakref.ref(cols), cols[order])
+        cols, values = kept[2], values[order]
     return pos, cols, values
+
+
+def _known_row_order(rows: torch.Tensor, n_rows: int):
+    """(row pointer, permutation into row order or None if they are in it, the columns in that order
+    once asked for) of row coordinates, kept with their tensor since an earlier product; None if
+    there is nothing (valid) kept."""
+    kept = getattr(rows, "_scorch_row_order", None)
+    return kept[2] if kept is not None and kept[0] == _stamp(rows) and kept[1] == n_rows else None
 
 
 def spmm_coo_float(result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mode_indices, B_values):
@@ -1520,11 +1689,48 @@ def sparse_attention_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row
     blocks with bit masks once (attention_block_mask) and the kernel computes every block that
     holds an entry.  Same result as sparse_attention_csr up to bf16 rounding of the operands, the
     probabilities and the result."""
+    out = native.host().attention(q, k, v, row_ptr, col_idx, scale, False)
+    if out is not None:
+        return out
     bm = attention_block_mask(row_ptr, col_idx, int(q.shape[1]))
     if bm.items is None:
-        return attn_blocksparse_bf16(q, k, v, bm.block_row_ptr, bm.block_col_idx, scale, block=bm.block,
-                                     block_mask_index=bm.block_mask_index, block_masks=bm.block_masks)
-    return attn_blocksparse_split_bf16(q, k, v, bm, scale)
+        out = attn_blocksparse_bf16(q, k, v, bm.block_row_ptr, bm.block_col_idx, scale, block=bm.block,
+                                    block_mask_index=bm.block_mask_index, block_masks=bm.block_masks)
+    else:
+        out = attn_blocksparse_split_bf16(q, k, v, bm, scale)
+    _remember_attention(q, row_ptr, col_idx, bm)
+    return out
+
+
+def _remember_attention(q: torch.Tensor, row_ptr: torch.Tensor, col_idx: torch.Tensor, bm: "BlockMask") -> None:
+    """After a fused attention call has gone the general way: hand what it was launched with to the
+    native call path, which serves the next ones over the same mask."""
+    if torch.cuda.is_current_stream_capturing() or not plans_enabled():
+        return
+    H, S, D = (int(x) for x in q.shape)
+    L, host = native.lib(), native.host()
+    if q.dtype == torch.float32:
+        items, split_rows, n_slots = _fp32_schedule(bm)
+        kind, pair, step = 2, False, 0
+        ws = L.scorch_hip_attn_blocksparse_f32_workspace_bytes(H, n_slots, D) if items is not None else 0
+    else:
+        if bm.items is not None:
+            items, split_rows, n_slots = bm.items, bm.split_rows, bm.n_slots
+            plan = bm.pairing.get(("items", H, D))
+        else:
+            schedule = _block_row_schedule(bm.block_row_ptr) if D in ATTENTION_WORKGROUPS_PER_CU else None
+            plan = schedule[2].get((H, D)) if schedule is not None else None
+            items, split_rows, n_slots = schedule[1] if schedule is not None else None, None, 0
+        if plan is None:
+            return
+        pair, step = plan
+        kind = 1 if bm.items is not None or pair or step else 0
+        ws = L.scorch_hip_attn_blocksparse_split_workspace_bytes(H, n_slots, D) if kind == 1 else 0
+    count = lambda t: t.numel() // 4 if t is not None else 0
+    host.remember_attention(
+        row_ptr, col_idx, weakref.ref(col_idx), kind, (H, S, D), q,
+        (bm.n_active_blocks, bm.n_masks, count(items), int(pair), int(step), count(split_rows), n_slots if count(items) else 0),
+        (bm.block_row_ptr, bm.block_col_idx, bm.block_mask_index, bm.block_masks, items, split_rows), ws)
 
 
 def sparse_attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_ptr: torch.Tensor,
@@ -1534,7 +1740,13 @@ def sparse_attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_
     sparse_attention_csr computes in three launches (the reference's per-head composition,
     bench/bench_sparse_transformer.py:354-372), to fp32 rounding.  The kernel computes every
     64 x 64 block that holds an entry, so it pays for masks that fill their blocks reasonably."""
-    return attn_blocksparse_f32(q, k, v, attention_block_mask(row_ptr, col_idx, int(q.shape[1])), scale)
+    out = native.host().attention(q, k, v, row_ptr, col_idx, scale, True)
+    if out is not None:
+        return out
+    bm = attention_block_mask(row_ptr, col_idx, int(q.shape[1]))
+    out = attn_blocksparse_f32(q, k, v, bm, scale)
+    _remember_attention(q, row_ptr, col_idx, bm)
+    return out
 
 
 FP32_ATTENTION_STRETCH = 16

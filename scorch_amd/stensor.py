@@ -43,9 +43,10 @@ class STensor(torch.nn.Module):
     def __init__(self, name: Optional[str] = None, shape: Optional[Tuple[int, ...]] = None,
                  storage: Optional[TensorStorage] = None, index: Optional[TensorIndex] = None,
                  value: Optional[torch.Tensor] = None, requires_grad: Optional[bool] = False) -> None:
-        super().__init__()
         # plain attributes (no parameter, buffer or sub-module among them): set past
-        # nn.Module.__setattr__, whose type checks cost more than everything else here
+        # nn.Module.__setattr__, whose type checks cost more than everything else here.  What
+        # nn.Module keeps for itself is made when something first asks for it (__getattr__): a
+        # result of every product is one of these objects
         put = object.__setattr__
         put(self, "_storage", storage if storage is not None else TensorStorage(index=index, value=value,
                                                                                 shape=shape))
@@ -58,6 +59,23 @@ class STensor(torch.nn.Module):
         else:
             put(self, "_dtype", torch.float32)
         put(self, "requires_grad", requires_grad)
+
+    def _module_state(self) -> None:
+        mine = dict(self.__dict__)
+        super().__init__()
+        self.__dict__.update(mine)
+
+    def __getattr__(self, name):
+        if "_parameters" not in self.__dict__:
+            self._module_state()
+            if name in self.__dict__:
+                return self.__dict__[name]
+        return super().__getattr__(name)
+
+    def __setattr__(self, name, value) -> None:
+        if "_parameters" not in self.__dict__:
+            self._module_state()
+        super().__setattr__(name, value)
 
     # ---- accessors the dispatch reads ------------------------------------------
     @property

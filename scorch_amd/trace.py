@@ -24,7 +24,7 @@ from typing import Any, Callable, Dict, List, Optional
 import torch
 import torch.fx
 
-from . import ops
+from . import ops, scorch_ops_hip
 from .prebuilt_kernels import resolve_prebuilt_fused
 from .stensor import STensor
 
@@ -182,11 +182,20 @@ def _try_prebuilt_fused(spec: FusionSpec, args: tuple) -> Optional[Callable]:
     bias_idx = spec.extra_arg_indices[0]
     kernel = resolved.fn
 
+    act = 2 if len(kinds) == 2 else 1
+
     def run(call_args: tuple) -> torch.Tensor:
-        lhs, rhs = _as_stensor(call_args[a_idx]), _as_stensor(call_args[b_idx])
+        lhs, rhs, bias = call_args[a_idx], call_args[b_idx], call_args[bias_idx]
+        result = ops._decided_spmm(lhs, rhs, bias, act)
+        if result is not None:
+            return result
+        lhs, dense = _as_stensor(lhs), rhs
+        rhs = _as_stensor(rhs)
         rows, cols = lhs.shape[0], rhs.shape[1]
         out = kernel([rows, cols], list(lhs.shape), lhs.index.mode_indices, lhs.values, list(rhs.shape),
-                     rhs.index.mode_indices, rhs.values, call_args[bias_idx])
+                     rhs.index.mode_indices, rhs.values, bias)
+        if isinstance(dense, torch.Tensor):
+            scorch_ops_hip.remember_spmm(lhs, cols, act)
         return out.storage.value.view(rows, cols)
 
     run.fused_symbol = resolved.symbol_name

@@ -1,0 +1,126 @@
+"""Products that have been decided are served by the native call path (scorch_amd/csrc/host.cpp): same
+results as the general way, and nothing stale after a write, a replaced tensor or forget()."""
+import numpy as np
+import pytest
+import torch
+
+import scorch_amd as scorch
+from conftest import random_csr
+from gpu_util import dev, host
+from scorch_amd import STensor, native
+from scorch_amd import scorch_ops_hip as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _operand(rng, M, K, dtype, form, long_row=0):
+    rp, ci, v = random_csr(rng, M, K, 0.05, dtype)
+    if long_row:
+        lens = np.diff(rp); lens[3] = long_row
+        rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        ci = rng.integers(0, K, rp[-1]).astype(np.int32)
+        v = rng.uniform(-1, 1, rp[-1]).astype(dtype)
+    rows = np.repeat(np.arange(M), np.diff(rp))
+    dense = torch.zeros(M, K, dtype=torch.float64)
+    dense.index_put_((torch.from_numpy(rows), torch.from_numpy(ci).long()), torch.from_numpy(v).double(), accumulate=True)
+    if form == "coo":
+        return STensor._coo((M, K), [dev(rows.astype(np.int32)), dev(ci)], dev(v), "A"), dense
+    return STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (M, K)), dense
+
+
+def _close(got, want, dtype):
+    tol = 1e-5 if dtype == np.float32 else 1e-12
+    return float((got.double().cpu() - want).norm()) <= tol * max(float(want.norm()), 1e-30)
+
+
+@pytest.mark.parametrize("form, dtype", [("csr", np.float32), ("csr", np.float64), ("coo", np.float32)])
+@pytest.mark.parametrize("long_row", [0, 700])
+@pytest.mark.parametrize("N", [None, 1, 37, 128])
+def test_decided_products_follow_their_operands(form, dtype, long_row, N):
+    if form == "coo" and N is None:
+        pytest.skip("coordinate operands have no matrix-vector kernel")
+    rng = np.random.default_rng(7)
+    M, K = 330, 290
+    A, dense = _operand(rng, M, K, dtype, form, long_row)
+    b = dev(rng.standard_normal((K, N) if N else K).astype(dtype))
+    for _ in range(3):
+        assert _close(scorch.matmul(A, b), dense @ b.double().cpu(), dtype)
+    decided = native.host().spmm
+    assert decided(A, b, None, 0) is not None
+    A.values.mul_(2)                                              # values are read on every call
+    assert _close(decided(A, b, None, 0), 2 * dense @ b.double().cpu(), dtype)
+    assert decided(A, b.float() if dtype == np.float64 else b.double(), None, 0) is None
+    assert decided(A, b[:-1], None, 0) is None
+    if N and N > 1:
+        assert decided(A, b.t().contiguous().t(), None, 0) is None    # a view goes the general way
+        assert _close(scorch.matmul(A, b.t().contiguous().t()), 2 * dense @ b.double().cpu(), dtype)
+    H.forget(A)
+    assert decided(A, b, None, 0) is None
+    for _ in range(2):                                            # (whether a pattern is made of blocks: from the second on)
+        assert _close(scorch.matmul(A, b), 2 * dense @ b.double().cpu(), dtype)
+    assert decided(A, b, None, 0) is not None
+    crd = A.index.mode_indices[1][-1]
+    crd[0] = K + 5                                                # a write to the pattern: inspected again, refused
+    assert decided(A, b, None, 0) is None
+    with pytest.raises(ValueError, match="column"):
+        scorch.matmul(A, b)
+
+
+def test_a_decided_product_keeps_to_pinned_paths_and_to_its_storage():
+    rng = np.random.default_rng(8)
+    A, dense = _operand(rng, 256, 256, np.float32, "csr")
+    b = torch.randn(256, 24, device="cuda")
+    scorch.matmul(A, b)
+    decided = native.host().spmm
+    assert decided(A, b, None, 0) is not None
+    H.SPMM_PATH = "merge"
+    try:
+        assert decided(A, b, None, 0) is None
+    finally:
+        H.SPMM_PATH = "auto"
+    assert decided(A, b, None, 0) is not None
+    A.storage._value = A.values * 3                               # another tensor in its place
+    assert decided(A, b, None, 0) is None
+    assert _close(scorch.matmul(A, b), 3 * dense @ b.double().cpu(), np.float32)
+
+
+@pytest.mark.parametrize("form", ["csr", "coo"])
+@pytest.mark.parametrize("unit", [True, False])
+def test_a_decided_sddmm_notices_new_mask_values(form, unit):
+    rng = np.random.default_rng(9)
+    M, n, K = 200, 170, 48
+    S, dense = _operand(rng, M, n, np.float32, form)
+    if unit:
+        S.values.fill_(1.0)
+        dense = (dense != 0).double()
+    q, k = torch.randn(M, K, device="cuda"), torch.randn(n, K, device="cuda")
+    want = (q.double() @ k.double().t()).cpu()
+    for _ in range(4):
+        out = scorch.einsum("ij,ik,jk->ij", S, q, k)
+    assert native.host().sddmm(S, q, k) is not None
+
+    def check(out, scale):
+        r, c = (out.index.mode_indices[i][0].long().cpu() for i in (0, 1))
+        assert torch.allclose(out.values.double().cpu(), scale * (dense * want)[r, c], rtol=1e-4, atol=1e-4)
+    check(scorch.einsum("ij,ik,jk->ij", S, q, k), 1)
+    S.values.mul_(0.5)
+    assert native.host().sddmm(S, q, k) is None                   # what was known about the values no longer holds
+    for _ in range(4):
+        check(scorch.einsum("ij,ik,jk->ij", S, q, k), 0.5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_decided_attention_is_the_general_ways_bit_for_bit(dtype):
+    from scorch_amd import workloads
+    S, Hn, D = 512, 4, 32
+    rp, ci = (dev(x) for x in workloads.longformer_mask(S))
+    q, k, v = (torch.randn(Hn, S, D, device="cuda").to(dtype) for _ in range(3))
+    fn = H.sparse_attention_bf16 if dtype == torch.bfloat16 else H.sparse_attention_f32
+    first = fn(q, k, v, rp, ci, 0.2)
+    f32 = dtype == torch.float32
+    assert torch.equal(native.host().attention(q, k, v, rp, ci, 0.2, f32), first)
+    assert native.host().attention(q, k, v, rp, ci.clone(), 0.2, f32) is None
+    assert native.host().attention(q, k, v, rp, ci, 0.2, not f32) is None
+    rp.add_(0)                                                    # written to, if only with what it held
+    assert native.host().attention(q, k, v, rp, ci, 0.2, f32) is None
+    assert torch.equal(fn(q, k, v, rp, ci, 0.2), first)
