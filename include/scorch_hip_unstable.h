@@ -258,6 +258,16 @@ SCORCH_HIP_API int scorch_hip_attn_blocksparse_f32(
     int64_t n_items, const int32_t *items, int64_t n_split_rows, const int32_t *split_rows, int64_t n_slots,
     const float *Q, const float *K, const float *V, float scale, float *O, void *workspace, size_t workspace_bytes,
     void *stream);
+/* The same with `block_cols` (one word per active block: the columns any of its rows refers to, as
+ * scorch_hip_csr_block_fill writes them; NULL: all): rows of K and V that no query of a block
+ * attends to are not read and count as zeros, and S may be any length, its last block row and
+ * column being live up to S only (block_mask_index is then required). */
+SCORCH_HIP_API int scorch_hip_attn_blocksparse_f32_cols(
+    int64_t H, int64_t S, int64_t D, int64_t block, int64_t n_active_blocks, const int32_t *block_row_ptr,
+    const int32_t *block_col_idx, const int32_t *block_mask_index, int64_t n_masks, const uint64_t *block_masks,
+    const uint64_t *block_cols, int64_t n_items, const int32_t *items, int64_t n_split_rows,
+    const int32_t *split_rows, int64_t n_slots, const float *Q, const float *K, const float *V, float scale, float *O,
+    void *workspace, size_t workspace_bytes, void *stream);
 
 /* ------------------------------------------------------------------------
  * SDDMM and SpMM in fp32 for a CSR operand whose entries cluster in 64 x 64

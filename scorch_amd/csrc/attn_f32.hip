@@ -19,6 +19,17 @@
 // takes is free as long as both operands agree: step c of slab j uses d = 16 j + 4 g + c, so a
 // lane's operands for four steps are 16 contiguous bytes of a row of K (one ds_read_b128) and of
 // its query's row of Q (kept in registers).
+//
+// Sequences of any length: S need not be a multiple of 64 when the caller hands over which columns
+// of every block are referred to (block_cols; a column beyond S never is).  Rows of K and V that no
+// query of a block attends to are then not read -- zeros stand in, so they may hold anything -- and
+// the last block row's queries beyond S compute on row S - 1 and are not stored.
+//
+// Blocks that are live in part are what a sliding window is made of: of the 64 queries x 64 keys
+// of its edge blocks, a wavefront's 16 queries attend to some of the four 16-key tiles only, and a
+// global token's block column holds one live key.  Tiles without a live position for the
+// wavefront are skipped in both products and in the exponentials (window of 64 and a global token:
+// 10.5 of 17 tiles remain).
 #include "common.hpp"
 
 namespace scorch {
@@ -52,14 +63,16 @@ struct Tile {
 
 constexpr float kDead = -3.0e38f;  // score of an entry the mask leaves out; also "no maximum yet"
 
-template <int D>
+// MASKED: blocks may be live in part (block_mask_index); without it every listed block is whole and
+// every operand exists, and the code for the rest is left out of the kernel (registers).
+template <int D, bool MASKED>
 __global__ __launch_bounds__(kBlockThreads)
 __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
     int S, int n_blocks, int n_heads, const int *__restrict__ block_row_ptr,
     const int *__restrict__ block_col_idx, const int *__restrict__ block_mask_index,
-    const unsigned long long *__restrict__ block_masks, const float *__restrict__ Q,
-    const float *__restrict__ K, const float *__restrict__ V, float scale_log2e, float *__restrict__ O,
-    int n_items, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
+    const unsigned long long *__restrict__ block_masks, const unsigned long long *__restrict__ block_cols,
+    const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float scale_log2e,
+    float *__restrict__ O, int n_items, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
   using T = Tile<D>;
   constexpr int kStride = T::kStride;
   constexpr int kSlabs = D / 16;  // contraction slabs of the first product (four MFMA steps each)
@@ -103,7 +116,8 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
   }
   const size_t head_off = (size_t)head * (size_t)S * D;
   const float *Kh = K + head_off, *Vh = V + head_off;
-  const int query = qb * kBlock + w * 16 + n;
+  const int query_at = qb * kBlock + w * 16 + n;
+  const int query = MASKED && query_at >= S ? S - 1 : query_at;
 
   // The query's row, scaled once: scores then come out of the matrix cores in base-2 exponent
   // units (a negative or zero scale needs nothing special).
@@ -123,18 +137,20 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
 
   // Tile traffic: thread `tid` moves chunks tid, tid + 256, ... (16 bytes each) of a 64 x D tile.
   floatx4 k_next[kCpt], v_next[kCpt];
-  auto fetch_k = [&](int it) {
-    const size_t tile = (size_t)uniform(block_col_idx[it]) * kBlock * D;
+  auto fetch = [&](floatx4 (&next)[kCpt], const float *from, int it) {
+    const float *tile = from + (size_t)uniform(block_col_idx[it]) * kBlock * D;
+    const unsigned long long cols = MASKED && block_cols ? block_cols[it] : ~0ull;
 #pragma unroll
-    for (int u = 0; u < kCpt; ++u)
-      k_next[u] = *reinterpret_cast<const floatx4 *>(Kh + tile + (size_t)(tid + u * kBlockThreads) * 4);
+    for (int u = 0; u < kCpt; ++u) {
+      const int chunk = tid + u * kBlockThreads;
+      if (!MASKED || ((cols >> (chunk / T::kChunksPerRow)) & 1ull))
+        next[u] = *reinterpret_cast<const floatx4 *>(tile + (size_t)chunk * 4);
+      else
+        next[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
   };
-  auto fetch_v = [&](int it) {
-    const size_t tile = (size_t)uniform(block_col_idx[it]) * kBlock * D;
-#pragma unroll
-    for (int u = 0; u < kCpt; ++u)
-      v_next[u] = *reinterpret_cast<const floatx4 *>(Vh + tile + (size_t)(tid + u * kBlockThreads) * 4);
-  };
+  auto fetch_k = [&](int it) { fetch(k_next, Kh, it); };
+  auto fetch_v = [&](int it) { fetch(v_next, Vh, it); };
   auto store_tile = [&]() {
 #pragma unroll
     for (int u = 0; u < kCpt; ++u) {
@@ -153,94 +169,136 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
   }
   __syncthreads();
 
+  // a block that is only partly live: bit j of word i of its mask says whether query i of the block
+  // row attends to key j of the block.  The words of the next block are requested a block ahead.
+  auto mask_of = [&](int it) { return MASKED ? uniform(block_mask_index[it]) : -1; };
+  auto live_word = [&](int mask_at) {
+    return mask_at >= 0 ? block_masks[(size_t)mask_at * kBlock + my_query_in_block] : 0ull;
+  };
+  // the lane's own sixteen bits of its query's word: bit 4 t + r is key 16 t + 4 g + r
+  auto own_bits = [&](unsigned long long word) {
+    unsigned bits = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) bits |= ((unsigned)(word >> (16 * t + 4 * g)) & 0xfu) << (4 * t);
+    return bits;
+  };
+  int mask_at = kb_begin < kb_end ? mask_of(kb_begin) : -1;
+  unsigned live = own_bits(live_word(mask_at));
+
   for (int it = kb_begin; it < kb_end; ++it) {
     const bool more = it + 1 < kb_end;
     if (more) fetch_k(it + 1);  // in flight while this block is computed (V follows after the scores:
                                 // the two sets of staging registers are then not live at once with
                                 // the K operands)
+    const int next_mask_at = more ? mask_of(it + 1) : -1;
+    const unsigned long long next_live = live_word(next_mask_at);
 
-    // S^T = K Q^T: tile t holds keys 16 t + 4 g + r (r = 0 .. 3) against query n
-    floatx4 st[4];
+    // One block.  WHOLE: every tile has live positions and (unless `partly`) all of them are; otherwise
+    // only the 16-key tiles in `tiles` are computed (bits 0 .. 3, the same for the whole wavefront).
+    auto block = [&](auto whole, bool partly, unsigned tiles) {
+      constexpr bool kWhole = decltype(whole)::value;
+      auto on = [&](int t) { return kWhole || ((tiles >> t) & 1u); };
+      // S^T = K Q^T: tile t holds keys 16 t + 4 g + r (r = 0 .. 3) against query n
+      floatx4 st[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) st[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < 4; ++t) st[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kWhole) {
 #pragma unroll
-    for (int j = 0; j < kSlabs; ++j) {
-      floatx4 k_op[4];
+        for (int j = 0; j < kSlabs; ++j) {
+          floatx4 k_op[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        k_op[t] = *reinterpret_cast<const floatx4 *>(&s_k[(16 * t + n) * kStride + 16 * j + 4 * g]);
+          for (int t = 0; t < 4; ++t)
+            k_op[t] = *reinterpret_cast<const floatx4 *>(&s_k[(16 * t + n) * kStride + 16 * j + 4 * g]);
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+              st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_op[t][c], q_op[j][c], st[t], 0, 0, 0);
+        }
+      } else {
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_op[t][c], q_op[j][c], st[t], 0, 0, 0);
-    }
+          if (on(t)) {
+#pragma unroll
+            for (int j = 0; j < kSlabs; ++j) {
+              const floatx4 k_op = *reinterpret_cast<const floatx4 *>(&s_k[(16 * t + n) * kStride + 16 * j + 4 * g]);
+#pragma unroll
+              for (int c = 0; c < 4; ++c)
+                st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_op[c], q_op[j][c], st[t], 0, 0, 0);
+            }
+          }
+      }
 
-    if (more) fetch_v(it + 1);
+      if (more) fetch_v(it + 1);
 
-    // a block that is only partly live: bit j of word i of its mask says whether query i of the
-    // block row attends to key j of the block
-    unsigned long long live = ~0ull;
-    bool partly_live = false;  // the same for the whole workgroup
-    if (block_mask_index) {
-      const int mask_at = uniform(block_mask_index[it]);
-      if (mask_at >= 0) {
-        partly_live = true;
-        live = block_masks[(size_t)mask_at * kBlock + my_query_in_block] >> (4 * g);
+      if (partly) {
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (!((live >> (16 * t + r)) & 1ull)) st[t][r] = kDead;
+            if (!((live >> (4 * t + r)) & 1u)) st[t][r] = kDead;
       }
-    }
 
-    // online softmax, base 2
-    float mx = st[0][0];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[t][r]);
-    mx = combine_query_lanes(mx, [](float a, float b) { return fmaxf(a, b); });
-    if (__any(mx > m_run)) {  // some query's maximum rises: after a row's first key blocks, seldom
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // (no maximum yet: the sums are 0)
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < kFeat; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o_acc[dt][r] *= alpha;
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) st[t][r] = __builtin_amdgcn_exp2f(st[t][r] - m_run);
-    if (partly_live) {
-      // an entry the mask leaves out: exp2(kDead - m_run) is 0 already unless the query has had no
-      // live key so far (m_run = kDead), so it is set
+      // online softmax, base 2
+      float mx = kDead;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (!((live >> (16 * t + r)) & 1ull)) st[t][r] = 0.0f;
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) l_run += st[t][r];
-
-    // O^T += V^T P^T: step (t, r) contracts keys 16 t + 4 g + r, whose probabilities lane (g, n)
-    // holds for query n; the V^T operand is V[that key][16 dt + n]
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float *v_row = &s_v[(16 * t + 4 * g + r) * kStride + n];
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, st[t][r]);
+      mx = combine_query_lanes(mx, [](float a, float b) { return fmaxf(a, b); });
+      if (__any(mx > m_run)) {  // some query's maximum rises: after a row's first key blocks, seldom
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // (no maximum yet: the sums are 0)
+        m_run = m_new;
+        l_run *= alpha;
 #pragma unroll
         for (int dt = 0; dt < kFeat; ++dt)
-          o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_row[16 * dt], st[t][r], o_acc[dt], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o_acc[dt][r] *= alpha;
       }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (on(t)) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) st[t][r] = __builtin_amdgcn_exp2f(st[t][r] - m_run);
+          if (partly) {
+            // an entry the mask leaves out: exp2(kDead - m_run) is 0 already unless the query has had no
+            // live key so far (m_run = kDead), so it is set
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (!((live >> (4 * t + r)) & 1u)) st[t][r] = 0.0f;
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) l_run += st[t][r];
+        }
+
+      // O^T += V^T P^T: step (t, r) contracts keys 16 t + 4 g + r, whose probabilities lane (g, n)
+      // holds for query n; the V^T operand is V[that key][16 dt + n]
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (on(t)) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float *v_row = &s_v[(16 * t + 4 * g + r) * kStride + n];
+#pragma unroll
+            for (int dt = 0; dt < kFeat; ++dt)
+              o_acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_row[16 * dt], st[t][r], o_acc[dt], 0, 0, 0);
+          }
+        }
+    };
+    if constexpr (!MASKED) {
+      block(std::true_type{}, false, 0xfu);
+    } else {
+      unsigned tiles = 0xfu;
+      if (mask_at >= 0) {
+        tiles = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) tiles |= __any((live >> (4 * t)) & 0xfu) ? 1u << t : 0u;
+      }
+      block(std::false_type{}, mask_at >= 0, (unsigned)uniform((int)tiles));
+    }
+    mask_at = next_mask_at;
+    live = own_bits(next_live);
 
     __syncthreads();  // every wavefront is done with this tile
     if (more) store_tile();
@@ -259,6 +317,7 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
     }
     return;
   }
+  if (MASKED && query_at >= S) return;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;  // queries without a live key give zeros
   float *out = O + head_off + (size_t)query * D;
 #pragma unroll
@@ -301,6 +360,7 @@ __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, in
       for (int r = 0; r < 4; ++r) acc[j + r] += weight * o[r];
     }
   }
+  if (row.x * kBlock + q >= S) return;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
   float *out = O + ((size_t)head * S + (size_t)row.x * kBlock + q) * D + quarter * kMine;
 #pragma unroll
@@ -315,13 +375,13 @@ __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, in
 template <int D>
 static int launch(dim3 grid, hipStream_t s, int S, int n_blocks, int H, const int32_t *block_row_ptr,
                   const int32_t *block_col_idx, const int32_t *block_mask_index,
-                  const unsigned long long *block_masks, const float *q, const float *k, const float *v,
-                  float scale_log2e, float *o, int n_items, const int4 *items, int n_slots, float *partials,
+                  const unsigned long long *block_masks, const unsigned long long *block_cols, const float *q,
+                  const float *k, const float *v, float scale_log2e, float *o, int n_items, const int4 *items, int n_slots, float *partials,
                   int n_split_rows, const int4 *split_rows) {
   mark_launch(s);
-  attn_f32_kernel<D><<<grid, kBlockThreads, 0, s>>>(S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index,
-                                                    block_masks, q, k, v, scale_log2e, o, n_items, items, n_slots,
-                                                    partials);
+  auto kernel = block_mask_index ? &attn_f32_kernel<D, true> : &attn_f32_kernel<D, false>;
+  kernel<<<grid, kBlockThreads, 0, s>>>(S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index, block_masks,
+                                        block_cols, q, k, v, scale_log2e, o, n_items, items, n_slots, partials);
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(s);
   if (n_split_rows > 0) {
@@ -347,6 +407,18 @@ extern "C" int scorch_hip_attn_blocksparse_f32(
     int64_t n_items, const int32_t *items, int64_t n_split_rows, const int32_t *split_rows, int64_t n_slots,
     const float *Q, const float *K, const float *V, float scale, float *O, void *workspace, size_t workspace_bytes,
     void *stream) {
+  return scorch_hip_attn_blocksparse_f32_cols(H, S, D, block, n_active_blocks, block_row_ptr, block_col_idx,
+                                              block_mask_index, n_masks, block_masks, nullptr, n_items, items,
+                                              n_split_rows, split_rows, n_slots, Q, K, V, scale, O, workspace,
+                                              workspace_bytes, stream);
+}
+
+extern "C" int scorch_hip_attn_blocksparse_f32_cols(
+    int64_t H, int64_t S, int64_t D, int64_t block, int64_t n_active_blocks, const int32_t *block_row_ptr,
+    const int32_t *block_col_idx, const int32_t *block_mask_index, int64_t n_masks, const uint64_t *block_masks,
+    const uint64_t *block_cols, int64_t n_items, const int32_t *items, int64_t n_split_rows, const int32_t *split_rows, int64_t n_slots,
+    const float *Q, const float *K, const float *V, float scale, float *O, void *workspace, size_t workspace_bytes,
+    void *stream) {
   using namespace scorch;
   const char *fn = "scorch_hip_attn_blocksparse_f32";
   if (H < 0 || S < 0 || D < 0 || block <= 0 || n_active_blocks < 0 || n_masks < 0 || n_items < 0 ||
@@ -356,9 +428,9 @@ extern "C" int scorch_hip_attn_blocksparse_f32(
   if ((D != 32 && D != 64 && D != 128) || block != attn32::kBlock)
     return fail(SCORCH_HIP_EUNSUPPORTED, "%s: only head dimensions 32, 64 and 128 and %d x %d mask blocks are "
                 "built (got D=%lld block=%lld)", fn, attn32::kBlock, attn32::kBlock, (long long)D, (long long)block);
-  if (S % attn32::kBlock != 0)
-    return fail(SCORCH_HIP_EINVAL, "%s: S=%lld is not a multiple of the block size", fn, (long long)S);
-  if (H * (S / attn32::kBlock) > INT32_MAX || S * D > INT32_MAX || n_items * H > INT32_MAX || n_slots > INT32_MAX)
+  if (S % attn32::kBlock != 0 && (!block_cols || !block_mask_index))
+    return fail(SCORCH_HIP_EINVAL, "%s: S=%lld is not a multiple of the block size (and no block_cols)", fn, (long long)S);
+  if (H * (S / attn32::kBlock + 1) > INT32_MAX || S * D > INT32_MAX || n_items * H > INT32_MAX || n_slots > INT32_MAX)
     return fail(SCORCH_HIP_EUNSUPPORTED, "%s: H=%lld, S=%lld or the item count too large", fn, (long long)H,
                 (long long)S);
   if (H == 0 || S == 0) return SCORCH_HIP_OK;
@@ -371,7 +443,8 @@ extern "C" int scorch_hip_attn_blocksparse_f32(
     SCORCH_REQUIRE(n_masks == 0 || block_masks != nullptr, "%s: block_masks is NULL", fn);
     SCORCH_REQUIRE(aligned_to(block_masks, 8), "%s: block_masks must be 8-byte aligned", fn);
   }
-  const int n_blocks = (int)(S / attn32::kBlock);
+  SCORCH_REQUIRE(aligned_to(block_cols, 8), "%s: block_cols must be 8-byte aligned", fn);
+  const int n_blocks = (int)((S + attn32::kBlock - 1) / attn32::kBlock);
   int work = n_blocks;
   const int4 *item_list = nullptr, *rows = nullptr;
   float *partials = nullptr;
@@ -396,7 +469,7 @@ extern "C" int scorch_hip_attn_blocksparse_f32(
   const unsigned long long *masks = reinterpret_cast<const unsigned long long *>(block_masks);
 #define SCORCH_ATTN32(DIM)                                                                                     \
   return attn32::launch<DIM>(grid, s, (int)S, n_blocks, (int)H, block_row_ptr, block_col_idx, block_mask_index, \
-                             masks, Q, K, V, scale_log2e, O, work, item_list, (int)n_slots, partials,          \
+                             masks, reinterpret_cast<const unsigned long long *>(block_cols), Q, K, V, scale_log2e, O, work, item_list, (int)n_slots, partials,          \
                              (int)n_split_rows, rows)
   if (D == 32) SCORCH_ATTN32(32);
   if (D == 64) SCORCH_ATTN32(64);

@@ -471,7 +471,7 @@ struct AttentionRoute {
   at::ScalarType dtype;
   int kind;
   int64_t workspace, p[8];
-  const void *q[6];
+  const void *q[7];
   PyObject *keep;
 };
 struct Attention {
@@ -508,7 +508,8 @@ Attention *attention_of(PyObject *row, PyObject *col) {
   return t;
 }
 
-// attention(q, k, v, row_ptr, col_idx, scale, whether in fp32).  None: not decided yet.
+// attention(q, k, v, row_ptr, col_idx, scale, form).  `form` 0: bf16; 1: fp32; 2: fp32, for a caller that wants the three
+// separate steps where the mask fills its blocks too thinly for the fused kernel.  None: not decided yet.
 PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 7 || !g_ops) return none();
   Attention *t = attention_of(args[3], args[4]);
@@ -521,7 +522,8 @@ PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
   for (int i = 0; i < 3; ++i)
     if (!THPVariable_CheckExact(args[i])) return none();
   const at::Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
-  if (q.scalar_type() != (args[6] == Py_True ? at::kFloat : at::kBFloat16) || !q.is_cuda() || q.dim() != 3 || q.sizes() != k.sizes() || q.sizes() != v.sizes() || !q.is_contiguous() ||
+  const long form = PyLong_AsLong(args[6]);
+  if (q.scalar_type() != (form ? at::kFloat : at::kBFloat16) || !q.is_cuda() || q.dim() != 3 || q.sizes() != k.sizes() || q.sizes() != v.sizes() || !q.is_contiguous() ||
       !k.is_contiguous() || !v.is_contiguous() || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() ||
       k.device() != q.device() || v.device() != q.device() || q.device() != THPVariable_Unpack(args[3]).device() ||
       q.is_neg() || k.is_neg() || v.is_neg())
@@ -531,7 +533,7 @@ PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
   for (AttentionRoute &x : *t->routes)
     if (x.H == H && x.S == S && x.D == D && x.dtype == q.scalar_type()) r = &x;
   const int device = q.get_device();
-  if (!r || c10::hip::current_device() != device) return none();
+  if (!r || (form == 2 && !r->p[7]) || c10::hip::current_device() != device) return none();
   hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
   void *ws = nullptr;
   size_t ws_bytes = 0;
@@ -543,7 +545,7 @@ PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
   int rc = SCORCH_HIP_EINVAL;
   const int64_t *p = r->p;
   const auto i32 = [&](int i) { return at_<int32_t>(r->q[i]); };
-  switch (r->kind) {  // p: active blocks, masks, items, pair, priority step, split rows, slots
+  switch (r->kind) {  // p: active blocks, masks, items, pair, priority step, split rows, slots, fills its blocks
     case kRowsBf16:
       rc = r->q[2] ? scorch_hip_attn_blocksparse_masked_bf16(H, S, D, 64, p[0], i32(0), i32(1), i32(2), p[1],
                                                              at_<uint64_t>(r->q[3]), Q, K, V, scale, O, stream)
@@ -555,9 +557,10 @@ PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
                                                   ws_bytes, stream);
       break;
     case kF32:
-      rc = scorch_hip_attn_blocksparse_f32(H, S, D, 64, p[0], i32(0), i32(1), i32(2), p[1], at_<uint64_t>(r->q[3]), p[2],
-                                           i32(4), p[5], i32(5), p[6], at_<float>(Q), at_<float>(K), at_<float>(V), scale,
-                                           static_cast<float *>(O), ws, ws_bytes, stream);
+      rc = scorch_hip_attn_blocksparse_f32_cols(H, S, D, 64, p[0], i32(0), i32(1), i32(2), p[1], at_<uint64_t>(r->q[3]),
+                                                at_<uint64_t>(r->q[6]), p[2], i32(4), p[5], i32(5), p[6], at_<float>(Q),
+                                                at_<float>(K), at_<float>(V), scale, static_cast<float *>(O), ws, ws_bytes,
+                                                stream);
       break;
     default: return none();
   }
@@ -573,7 +576,7 @@ PyObject *host_remember_attention(PyObject *, PyObject *args) {
                         &PyTuple_Type, &tensors, &ws))
     return nullptr;
   if (!THPVariable_CheckExact(row) || !THPVariable_CheckExact(col) || !THPVariable_Check(model) ||
-      !PyWeakref_CheckRef(ref) || PyTuple_GET_SIZE(ints) > 8 || PyTuple_GET_SIZE(tensors) > 6)
+      !PyWeakref_CheckRef(ref) || PyTuple_GET_SIZE(ints) > 8 || PyTuple_GET_SIZE(tensors) > 7)
     return none();
   Attention *t = attention_of(row, col);
   if (!t) {

@@ -119,6 +119,9 @@ SIGNATURES = {
     "scorch_hip_attn_blocksparse_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr, _i64,
                                                        _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, ctypes.c_float, _ptr,
                                                        _ptr, _size, _ptr]),
+    "scorch_hip_attn_blocksparse_f32_cols": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr,
+                                                            _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr,
+                                                            ctypes.c_float, _ptr, _ptr, _size, _ptr]),
     "scorch_hip_sddmm_csr_blocked_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _ptr,
                                                         _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "scorch_hip_spmm_csr_blocked_workspace_bytes": (_size, [_i64, _i64, _i64]),

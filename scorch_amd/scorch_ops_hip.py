@@ -295,7 +295,7 @@ class CsrPlan:
     row-pointer tensor, so it is dropped with the operand, and is rebuilt when
     either index tensor has been written to since."""
     __slots__ = ("key", "partner", "max_row", "empty_rows", "sorted_rows", "runs", "bounds", "sddmm_lists",
-                 "sddmm_uses", "rows", "blocked", "blocked_uses")
+                 "sddmm_uses", "rows", "blocked", "blocked_uses", "attention", "attention_uses")
 
     def __init__(self, key, max_row: int, empty_rows: int, sorted_rows: bool = False, runs: int = 0):
         self.key = key
@@ -310,6 +310,8 @@ class CsrPlan:
         self.rows: Optional[torch.Tensor] = None           # the row coordinate of every entry (SDDMM results)
         self.blocked = None                                # BlockedCsr, False (looked at: not blocky), None (not yet)
         self.blocked_uses = 0                              # products that could have gone to the block kernels
+        self.attention = None                              # BlockMask, False (blocks too thinly filled), None (not yet)
+        self.attention_uses = 0                            # sparse_attention_csr calls
 
 
 def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, what: str = "operand") -> Optional[CsrPlan]:
@@ -1489,12 +1491,52 @@ def sparse_attention_csr(row_ptr: torch.Tensor, col_idx: torch.Tensor, q: torch.
     """softmax(scale * q k^T restricted to a CSR mask) v for q, k, v of shape (H, S, D), fp32: the
     reference's sparse attention (bench/bench_sparse_transformer.py:354-372: SDDMM, row softmax and
     SpMM per head) as three launches for all heads.  Any mask, any head dimension; rows of the mask
-    without entries give zero rows."""
+    without entries give zero rows.  A mask that fills its 64 x 64 blocks and comes back is served by
+    the fused fp32 kernel, which never writes the scores to memory: the same result to rounding."""
+    if SPMM_PATH == "auto" and SDDMM_PATH == "auto" and BLOCKED_PATH == "auto":
+        out = native.host().attention(q, k, v, row_ptr, col_idx, scale, 2)
+        if out is not None:
+            return out
+        bm = _fused_attention_mask(row_ptr, col_idx, q, k, v)
+        if bm is not None:
+            out = attn_blocksparse_f32(q, k, v, bm, scale)
+            _remember_attention(q, row_ptr, col_idx, bm)
+            return out
     H, S, D = (int(x) for x in q.shape)
     mask = [[], [row_ptr, col_idx]]
     scores, _ = sddmm_csr_float_batched([S, S], mask, None, q, k)
     probs = softmax_csr_float_batched(row_ptr, scores, scale)
     return spmm_csr_float_batched([S, S], mask, probs, v)
+
+
+def _fused_attention_mask(row_ptr, col_idx, q, k, v) -> Optional["BlockMask"]:
+    """The mask by blocks if sparse_attention_csr goes to the fused fp32 kernel: fp32 operands of a
+    width it serves, columns that increase strictly in every row (a repeated entry would count
+    twice in the three steps), and blocks filled as the block kernels ask for (BLOCKED_MIN_FILL).
+    Decided on a mask's second call, as there, and for any sequence length."""
+    if q.dim() != 3 or q.shape != k.shape or q.shape != v.shape or q.numel() == 0 or int(q.shape[2]) not in BLOCKED_MIN_FILL \
+            or any(t.dtype != torch.float32 or not t.is_cuda for t in (q, k, v)) \
+            or any(t.dtype != torch.int32 or not t.is_contiguous() for t in (row_ptr, col_idx)):
+        return None
+    S, D, nnz = int(q.shape[1]), int(q.shape[2]), col_idx.numel()
+    plan = csr_plan(row_ptr, col_idx, S, S, "S")
+    if plan is None:
+        return None
+    if plan.attention is None:
+        plan.attention_uses += 1
+        if torch.cuda.is_current_stream_capturing() or plan.attention_uses < 2:
+            return None
+        least = min(BLOCKED_MIN_FILL.values())
+        block_cols = -(-S // 64)
+        plan.attention = False
+        if plan.sorted_rows and 0 < nnz <= BLOCKED_MAX_NNZ and nnz >= least * 64 * plan.runs \
+                and block_cols <= BLOCKED_MAX_BLOCK_COLS and block_cols ** 2 <= BLOCKED_MAX_BLOCKS:
+            if S % 64:
+                plan.attention = _block_mask(row_ptr, col_idx, S)
+            elif _blocked(plan, row_ptr, col_idx, S, S, D) is not None or plan.blocked:
+                plan.attention = attention_block_mask(row_ptr, col_idx, S)
+    bm = plan.attention or None
+    return bm if bm is not None and bm.density_in_blocks >= BLOCKED_MIN_FILL[D] else None
 
 
 class BlockMask:
@@ -1503,7 +1545,7 @@ class BlockMask:
     of its 64-word bit mask (bit j of word r: query r of the block row attends to key j of the
     block).  Blocks with equal masks share one."""
     __slots__ = ("S", "block", "block_row_ptr", "block_col_idx", "block_mask_index", "block_masks", "nnz",
-                 "items", "split_rows", "n_slots", "schedule32", "block_row_lens", "pairing")
+                 "items", "split_rows", "n_slots", "schedule32", "block_row_lens", "pairing", "block_cols")
 
     def __init__(self, S, block, block_row_ptr, block_col_idx, block_mask_index, block_masks, nnz):
         self.S, self.block, self.nnz = S, block, nnz
@@ -1514,6 +1556,7 @@ class BlockMask:
         self.n_slots = 0
         self.schedule32 = None      # the fp32 kernel's own sharing-out (see _fp32_schedule)
         self.block_row_lens = None  # active blocks per block row, on the host (numpy), once it has been read
+        self.block_cols = None      # int64 per active block: the columns some row of it refers to (None: all)
         self.pairing = {}           # (item list, heads, head dimension) -> (workgroups take two items?, priority step)
 
     def row_lens(self):
@@ -1544,16 +1587,25 @@ def block_mask_from_csr(row_ptr: torch.Tensor, col_idx: torch.Tensor, S: int) ->
     kernel passes of _describe_blocks over the entries, then the blocks that are not fully stored
     are compared with one another so that equal masks are kept once.  Done once per mask (see
     attention_block_mask for the cached form); repeated entries and unsorted rows are tolerated."""
-    block = 64
-    if S % block:
+    if S % 64:
         raise ValueError("scorch_ops_hip: S must be a multiple of 64")
     pos, crd = _index(row_ptr, "row_ptr"), _index(col_idx, "col_idx")
-    dev = _device_of(pos, crd)
+    _device_of(pos, crd)
     if pos.numel() != S + 1:
         raise ValueError("scorch_ops_hip: row_ptr length does not match S")
     csr_plan(pos, crd, S, S, "mask")                      # validates the index (ValueError), once per tensor pair
-    nb = S // block
-    brp, arrays = _describe_blocks(pos, crd, S, S)
+    return _block_mask(pos, crd, S)
+
+
+def _block_mask(pos: torch.Tensor, crd: torch.Tensor, S: int) -> BlockMask:
+    """The work of block_mask_from_csr on a checked pattern, for any S: up to the next multiple of 64
+    the rows are empty and no entry names a column."""
+    block = 64
+    dev = pos.device
+    nb = -(-S // block)
+    if S % block:
+        pos = torch.cat([pos, pos[-1:].expand(nb * block - S)])
+    brp, arrays = _describe_blocks(pos, crd, nb * block, nb * block)
     if arrays is None:                                    # no entries at all
         empty = lambda dtype: torch.zeros(0, dtype=dtype, device=dev)
         bm = BlockMask(S, block, torch.zeros(nb + 1, dtype=torch.int32, device=dev), empty(torch.int32),
@@ -1572,6 +1624,8 @@ def block_mask_from_csr(row_ptr: torch.Tensor, col_idx: torch.Tensor, S: int) ->
     bm = BlockMask(S, block, arrays["block_row_ptr"], arrays["block_col_idx"], mask_index,
                    masks.contiguous().view(-1), int(stored.sum()))
     bm.block_row_lens = brp[1:] - brp[:-1]
+    if partial.numel():
+        bm.block_cols = arrays["block_cols"]
     return bm
 
 
@@ -1689,7 +1743,7 @@ def sparse_attention_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row
     blocks with bit masks once (attention_block_mask) and the kernel computes every block that
     holds an entry.  Same result as sparse_attention_csr up to bf16 rounding of the operands, the
     probabilities and the result."""
-    out = native.host().attention(q, k, v, row_ptr, col_idx, scale, False)
+    out = native.host().attention(q, k, v, row_ptr, col_idx, scale, 0)
     if out is not None:
         return out
     bm = attention_block_mask(row_ptr, col_idx, int(q.shape[1]))
@@ -1727,10 +1781,13 @@ def _remember_attention(q: torch.Tensor, row_ptr: torch.Tensor, col_idx: torch.T
         kind = 1 if bm.items is not None or pair or step else 0
         ws = L.scorch_hip_attn_blocksparse_split_workspace_bytes(H, n_slots, D) if kind == 1 else 0
     count = lambda t: t.numel() // 4 if t is not None else 0
+    # (a mask of whole blocks has an index without a bit mask to name: the fp32 kernel for whole blocks takes it)
+    mask_index = bm.block_mask_index if bm.n_masks or q.dtype != torch.float32 else None
     host.remember_attention(
         row_ptr, col_idx, weakref.ref(col_idx), kind, (H, S, D), q,
-        (bm.n_active_blocks, bm.n_masks, count(items), int(pair), int(step), count(split_rows), n_slots if count(items) else 0),
-        (bm.block_row_ptr, bm.block_col_idx, bm.block_mask_index, bm.block_masks, items, split_rows), ws)
+        (bm.n_active_blocks, bm.n_masks, count(items), int(pair), int(step), count(split_rows), n_slots if count(items) else 0,
+         int(D in BLOCKED_MIN_FILL and bm.density_in_blocks >= BLOCKED_MIN_FILL[D])),
+        (bm.block_row_ptr, bm.block_col_idx, mask_index, bm.block_masks, items, split_rows, bm.block_cols), ws)
 
 
 def sparse_attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_ptr: torch.Tensor,
@@ -1740,7 +1797,7 @@ def sparse_attention_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row_
     sparse_attention_csr computes in three launches (the reference's per-head composition,
     bench/bench_sparse_transformer.py:354-372), to fp32 rounding.  The kernel computes every
     64 x 64 block that holds an entry, so it pays for masks that fill their blocks reasonably."""
-    out = native.host().attention(q, k, v, row_ptr, col_idx, scale, True)
+    out = native.host().attention(q, k, v, row_ptr, col_idx, scale, 1)
     if out is not None:
         return out
     bm = attention_block_mask(row_ptr, col_idx, int(q.shape[1]))
@@ -1801,10 +1858,10 @@ def attn_blocksparse_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bm: 
         stream = _stream(dev)
         need = L.scorch_hip_attn_blocksparse_f32_workspace_bytes(H, n_slots, D) if n_items else 0
         ws = _workspace(dev, stream, need) if need else None
-        rc = L.scorch_hip_attn_blocksparse_f32(
+        n_masks = bm.n_masks if bm.block_masks is not None else 0
+        rc = L.scorch_hip_attn_blocksparse_f32_cols(
             H, S, D, bm.block, bm.n_active_blocks, ptr(bm.block_row_ptr), ptr(bm.block_col_idx),
-            ptr(bm.block_mask_index), bm.n_masks if bm.block_masks is not None else 0, ptr(bm.block_masks),
-            n_items, ptr(items), n_split, ptr(split_rows), n_slots if n_items else 0,
+            ptr(bm.block_mask_index) if n_masks else None, n_masks, ptr(bm.block_masks), ptr(bm.block_cols), n_items, ptr(items), n_split, ptr(split_rows), n_slots if n_items else 0,
             q.data_ptr(), k.data_ptr(), v.data_ptr(), float(scale), out.data_ptr(),
             ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, stream)
     native.check(rc)

@@ -134,3 +134,33 @@ def test_keys_the_mask_leaves_out_may_hold_anything_in_k(oracle):
     to16 = lambda a: dev(a).to(torch.bfloat16)
     out16 = H.sparse_attention_bf16(to16(q), to16(k_bad), to16(v), dev(rp), dev(ci), D ** -0.5).float().cpu().numpy()
     assert np.isfinite(out16).all() and oracle.rel_fro(out16, ref) <= 1e-2
+
+
+@pytest.mark.parametrize("S", [1, 63, 65, 130, 447, 513])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("kind", ["window", "causal", "dense"])
+def test_sequences_of_any_length_through_the_three_step_call(oracle, S, D, kind):
+    """sparse_attention_csr over a mask that fills its blocks goes to the fused kernel when the mask comes
+    back, whatever the sequence length: the last block row and column are live up to S only, nothing
+    beyond S is read or written, and rows no query refers to may hold anything."""
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = {"window": (abs(i - j) <= 40) | (i == 0) | (j == 0), "causal": j <= i, "dense": j >= 0}[kind] & np.ones((S, S), bool)
+    unused = S // 2 if S > 3 else None
+    if unused is not None:
+        mask[:, unused] = False
+        mask[unused, :] = False                           # a query without keys: a zero row
+    rng = np.random.default_rng(S + D)
+    q, k, v = (rng.standard_normal((3, S, D)).astype(np.float32) for _ in range(3))
+    rp, ci = (dev(x) for x in csr_of(mask))
+    ref = np.stack([oracle.attention_dense_fp64(q[h], k[h], v[h], mask, D ** -0.5) for h in range(3)])
+    if unused is not None:
+        k[:, unused] = v[:, unused] = np.nan
+    def followed_by_nan(x):
+        buffer = torch.full((x.size + 64 * D,), float("nan"), device="cuda")
+        buffer[:x.size] = dev(x).reshape(-1)
+        return buffer[:x.size].view(x.shape)
+    dq, dk, dv = (followed_by_nan(x) for x in (q, k, v))
+    for call in range(3):
+        out = H.sparse_attention_csr(rp, ci, dq, dk, dv, D ** -0.5)
+        assert oracle.rel_fro(out.cpu().numpy(), ref) <= TOL
+    assert isinstance(rp._scorch_plan.attention, H.BlockMask) == (S > 1)    # (one entry fills no block)

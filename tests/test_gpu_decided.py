@@ -117,10 +117,10 @@ def test_decided_attention_is_the_general_ways_bit_for_bit(dtype):
     q, k, v = (torch.randn(Hn, S, D, device="cuda").to(dtype) for _ in range(3))
     fn = H.sparse_attention_bf16 if dtype == torch.bfloat16 else H.sparse_attention_f32
     first = fn(q, k, v, rp, ci, 0.2)
-    f32 = dtype == torch.float32
+    f32 = int(dtype == torch.float32)
     assert torch.equal(native.host().attention(q, k, v, rp, ci, 0.2, f32), first)
     assert native.host().attention(q, k, v, rp, ci.clone(), 0.2, f32) is None
-    assert native.host().attention(q, k, v, rp, ci, 0.2, not f32) is None
+    assert native.host().attention(q, k, v, rp, ci, 0.2, 1 - f32) is None
     rp.add_(0)                                                    # written to, if only with what it held
     assert native.host().attention(q, k, v, rp, ci, 0.2, f32) is None
     assert torch.equal(fn(q, k, v, rp, ci, 0.2), first)
