@@ -1764,7 +1764,7 @@ def _remember_attention(q: torch.Tensor, row_ptr: torch.Tensor, col_idx: torch.T
     H, S, D = (int(x) for x in q.shape)
     L, host = native.lib(), native.host()
     if q.dtype == torch.float32:
-        items, split_rows, n_slots = _fp32_schedule(bm)
+        items, split_rows, n_slots = _fp32_launch_schedule(bm, H, D)
         kind, pair, step = 2, False, 0
         ws = L.scorch_hip_attn_blocksparse_f32_workspace_bytes(H, n_slots, D) if items is not None else 0
     else:
@@ -1832,6 +1832,43 @@ def _fp32_schedule(bm: BlockMask):
     return bm.schedule32
 
 
+def _fp32_stretch(lens, heads: int, D: int, n_cus: int) -> Optional[int]:
+    """Key blocks per stretch that a launch of so many heads wants, or None for what _fp32_schedule takes
+    whatever the heads.  A key block keeps a workgroup's matrix cores busy for 1.7 us (D = 64) and
+    a workgroup for 3.3, so a launch is over when its longest item is: while the block rows are
+    longer than half as much again as a CU's share of all blocks, they go out in stretches, the
+    shorter the fewer there are to go round -- two blocks where a CU's share is less than two, four
+    up to 16 (in units of D = 64), eight up to 64.  Measured in us with stretches of 10 and now: S =
+    3,001, 8 heads, window 64 and a global token 47.5 -> 29.4; S = 4,096, D = 32 33.5 -> 23.5; S = 512,
+    4 heads 31 -> 15; S = 8,192, 16 heads 101 -> 96.  Rows of nearly the chip's share each stay
+    whole (S = 2,048, 8 heads, strided blocks: 22.7, in fours 26.1)."""
+    longest = int(lens.max()) if lens.size else 0
+    share = float(lens.sum()) * heads / n_cus
+    if longest <= max(2, 1.5 * share) or share * D / 64 >= 64:
+        return None
+    return 2 if share < 2 else 4 if share * D / 64 < 16 else 8
+
+
+def _fp32_launch_schedule(bm: BlockMask, heads: int, D: int):
+    """_fp32_schedule for a launch of so many heads, kept with the BlockMask."""
+    key = ("fp32", heads, D)
+    kept = bm.pairing.get(key)
+    if kept is None:
+        kept = _fp32_schedule(bm)
+        if bm.schedule32 is None:          # (being recorded, with nothing decided before)
+            return kept
+        stretch = _fp32_stretch(bm.row_lens(), heads, D, _cu_count(bm.block_row_ptr.device))
+        if stretch is not None and not torch.cuda.is_current_stream_capturing():
+            plain = BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)
+            plain.block_row_lens = bm.row_lens()
+            split_long_block_rows(plain, stretch, list_unequal_rows=True)
+            kept = (plain.items, plain.split_rows, plain.n_slots)
+        elif stretch is not None:
+            return kept
+        bm.pairing[key] = kept
+    return kept
+
+
 def attn_blocksparse_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bm: BlockMask, scale: float) -> torch.Tensor:
     """The fp32 fused attention kernel over a BlockMask (block_mask_index / block_masks may be None:
     every listed block fully live; rows that split_long_block_rows shared out go through a
@@ -1849,7 +1886,7 @@ def attn_blocksparse_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bm: 
     if S != bm.S:
         raise ValueError("scorch_ops_hip: the BlockMask was built for another sequence length")
     ptr = lambda t: t.data_ptr() if t is not None and t.numel() else None
-    items, split_rows, n_slots = _fp32_schedule(bm)
+    items, split_rows, n_slots = _fp32_launch_schedule(bm, int(H), int(D))
     n_items = items.numel() // 4 if items is not None else 0
     n_split = split_rows.numel() // 4 if split_rows is not None else 0
     out = _empty_like(q)
