@@ -55,7 +55,7 @@ MEASURED_TRAFFIC = {
     ("gcn_powerlaw", "merge"): {"bytes": 9_790_300_000, "sources": _SPMM_SOURCES, "sha16": "f03cdf8f7d11457c",
                                 "profile": "profiles/spmm_merge_kernel_gcn_powerlaw.md"},
     ("spmm_uniform", "rows"): {"bytes": 10_830_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp",
-                                                                _CSRC + "common.hpp"), "sha16": "36b7f160411c76eb",
+                                                                _CSRC + "common.hpp"), "sha16": "",
                                "profile": "profiles/spmm_rows_kernel_uniform_4096.md"},
     ("sae_decoder", "tiled"): {"bytes": 344_100_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp",
                                                                  _CSRC + "common.hpp"), "sha16": "ea9b5c43570e7930",

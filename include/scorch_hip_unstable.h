@@ -85,6 +85,10 @@ SCORCH_HIP_API int scorch_hip_spmm_csr_f32_timed(int64_t M, int64_t K, int64_t N
 #define SCORCH_HIP_INSPECT_REPORT_INTS 8
 SCORCH_HIP_API int scorch_hip_csr_inspect(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr,
                            const int32_t *col_idx, int32_t *report /* device, [8] */, void *stream);
+/* The same with the report in host memory when the call returns: one launch, whose last workgroup
+ * hands it to the waiting host thread.  Not for a stream that is being captured. */
+SCORCH_HIP_API int scorch_hip_csr_inspect_now(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr,
+                                  const int32_t *col_idx, int32_t *report, void *stream);
 
 /* Row-split SpMM for matrices whose rows are all short: C = act(A * B + bias)
  * in one launch, without workspace (a team of lanes per row; no rows are cut,
@@ -381,6 +385,40 @@ SCORCH_HIP_API int scorch_hip_spmm_csr_batched_f32(int64_t batch, int64_t M, int
  * No counterpart in the reference. */
 SCORCH_HIP_API int scorch_hip_values_differ_f32(int64_t n, const float *vals, float value,
                                  int32_t *differ /* device */, void *stream);
+
+/* ------------------------------------------------------------------------
+ * SpGEMM whose two passes share what the first found out: _symbolic_planned is
+ * scorch_hip_spgemm_csr_symbolic and returns with `report` (host memory, 7 words: entries of the
+ * result or -1 for 2^31 and more, then the numbers of rows per tier) filled in, which takes the
+ * place of the caller's read of c_row_ptr[M]; _numeric_planned_<T> takes that report and the SAME
+ * workspace, unchanged in between, reads the row lists from it and launches only what has rows.
+ * Not for a stream that is being captured.
+ * ---------------------------------------------------------------------- */
+#define SCORCH_HIP_SPGEMM_REPORT_WORDS 7
+SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const int32_t *b_row_ptr, const int32_t *b_col_idx,
+                                   int32_t *c_row_ptr, void *workspace, size_t workspace_bytes, int64_t *report,
+                                   void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_f32(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const float *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const float *b_vals, const int32_t *c_row_ptr,
+                                   int32_t *c_col_idx, float *c_vals, void *workspace, size_t workspace_bytes,
+                                   const int64_t *report, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_f64(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const double *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const double *b_vals, const int32_t *c_row_ptr,
+                                   int32_t *c_col_idx, double *c_vals, void *workspace, size_t workspace_bytes,
+                                   const int64_t *report, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_i32(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const int32_t *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const int32_t *b_vals, const int32_t *c_row_ptr,
+                                   int32_t *c_col_idx, int32_t *c_vals, void *workspace, size_t workspace_bytes,
+                                   const int64_t *report, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_i64(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const int64_t *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const int64_t *b_vals, const int32_t *c_row_ptr,
+                                   int32_t *c_col_idx, int64_t *c_vals, void *workspace, size_t workspace_bytes,
+                                   const int64_t *report, void *stream);
 
 #ifdef __cplusplus
 }

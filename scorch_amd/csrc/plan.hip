@@ -22,6 +22,7 @@ hipError_t preload_spgemm();
 hipError_t preload_spmm();
 hipError_t preload_spmm_rows();
 hipError_t preload_spmm_tiled();
+hipError_t preload_sync();
 }  // namespace scorch
 
 namespace {
@@ -182,7 +183,7 @@ int scorch_hip_init(void) {
   hipError_t (*const loaders[])() = {scorch::preload_attn,      scorch::preload_attn_f32, scorch::preload_blockdesc,
                                      scorch::preload_blocked,   scorch::preload_misc,     scorch::preload_sddmm,
                                      scorch::preload_spgemm,    scorch::preload_spmm,     scorch::preload_spmm_rows,
-                                     scorch::preload_spmm_tiled};
+                                     scorch::preload_spmm_tiled, scorch::preload_sync};
   for (auto load : loaders) SCORCH_HIP_CHECK(load());
   return SCORCH_HIP_OK;
 }

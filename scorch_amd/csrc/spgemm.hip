@@ -16,6 +16,8 @@
 //   up to 4096 products  B of at most 131,072 columns: a bitmap of the columns in LDS
 //                        (256 threads, see below); wider B: one workgroup, hash
 //                        table of 8192 slots in LDS
+//   more, and more than a 128th of all such rows' products
+//                        several workgroups (see "rows shared out among workgroups")
 //   more                 one workgroup of 1024 threads with a bitmap of the columns
 //                        in LDS, 524,288 columns at a time (B of up to 4.2 M
 //                        columns is covered in up to eight such ranges, walking the
@@ -36,7 +38,7 @@
 // integer results are exact.
 #include <climits>
 
-#include "common.hpp"
+#include "sync.hpp"
 
 namespace scorch {
 
@@ -48,6 +50,7 @@ constexpr int kMediumWorkgroups = 2048;
 constexpr int kMinHugeWorkgroups = 64;
 constexpr int kMaxHugeWorkgroups = 1024;
 constexpr size_t kHugeSlabBudget = (size_t)1 << 30;
+constexpr int kNarrowColumns = 32 * 4096;              // widest B whose bitmap leaves room for other workgroups in a CU's LDS
 constexpr int kLdsBitmapColumns = 8 * 32 * 16384;  // widest B served by the LDS bitmap (in up to 8 ranges of columns)
 
 // Number of bitmap workgroups: as many slabs (N bits and N / 32 ranks) as fit
@@ -284,6 +287,22 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
 constexpr int kScanPerThread = 16;
 constexpr int kScanTile = kBlockThreads * kScanPerThread;
 
+// counters: [0] medium rows, [1] huge rows, [2] small rows, [5] giant rows listed; [3], [4] next row to hand out;
+// [6..7] one 64-bit sum: the number of entries of the result; [8] rows shared out, [9] their slices; [10..11] one
+// 64-bit sum: the giant rows' products
+constexpr int kSpgemmCounters = 16;
+
+// The symbolic pass is over: the numeric pass hands its longest rows out from the first again, and
+// the host thread, if it waits, gets the report (SpgemmReport).
+__device__ __forceinline__ void end_of_symbolic(int *counters, unsigned long long entries, int64_t *report, int64_t sequence) {
+  if (report) {
+    const int64_t words[7] = {entries > (unsigned long long)INT32_MAX ? -1 : (int64_t)entries,
+                              counters[2], counters[0], counters[1], counters[5], counters[8], counters[9]};
+    sync_publish(report, sequence, words, 7);
+  }
+  counters[3] = 0;
+}
+
 // (*grand_total also receives the sum of all counts in 64 bits: the row pointer is int32,
 // and a result of 2^31 entries or more must be reported, not wrapped)
 __global__ __launch_bounds__(kBlockThreads) void scan_tile_totals_kernel(const int *__restrict__ data,
@@ -307,8 +326,11 @@ __global__ __launch_bounds__(kBlockThreads) void scan_tile_totals_kernel(const i
   if (wave_lane() == 0 && wide > 0) atomicAdd(grand_total, (unsigned long long)wide);
 }
 
+// (also, at the end of the symbolic pass: see end_of_symbolic)
 __global__ __launch_bounds__(kBlockThreads) void scan_spine_kernel(int *__restrict__ totals,
-                                                                   int64_t n_tiles) {
+                                                                   int64_t n_tiles, int *__restrict__ counters,
+                                                                   int64_t *__restrict__ report, int64_t sequence) {
+  if (threadIdx.x == 0) end_of_symbolic(counters, *reinterpret_cast<const unsigned long long *>(counters + 6), report, sequence);
   __shared__ int s_scan[kWavesPerBlock + 1];
   int carried = 0;
   for (int64_t base = 0; base < n_tiles; base += kBlockThreads) {
@@ -341,6 +363,50 @@ __global__ __launch_bounds__(kBlockThreads) void scan_apply_kernel(int *__restri
   }
 }
 
+// The same for few rows, in one workgroup and one launch.
+constexpr int kScanOneGroup = 65536;
+constexpr int kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void scan_one_group_kernel(int *__restrict__ data, int n, int *__restrict__ counters,
+                                                                      int64_t *__restrict__ report, int64_t sequence) {
+  constexpr int kPer = 16;
+  __shared__ int s_scan[kScanThreads / kWaveSize];
+  int carried = 0;
+  unsigned long long wide = 0;
+  for (int base = 0; base < n; base += kScanThreads * kPer) {
+    const int first = base + (int)threadIdx.x * kPer;
+    int v[kPer], mine = 0;
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+      v[e] = first + e < n ? data[first + e] : 0;
+      mine += v[e];
+      wide += (unsigned)v[e];
+    }
+    int total = 0;
+    int running = carried + block_exclusive_scan_n<kScanThreads / kWaveSize>(mine, s_scan, total);
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+      if (first + e < n) data[first + e] = running;
+      running += v[e];
+    }
+    carried += total;
+  }
+#pragma unroll
+  for (int off = kWaveSize / 2; off > 0; off >>= 1) {
+    const unsigned lo = (unsigned)__shfl_xor((int)(unsigned)wide, off), hi = (unsigned)__shfl_xor((int)(unsigned)(wide >> 32), off);
+    wide += ((unsigned long long)hi << 32) | lo;
+  }
+  __shared__ unsigned long long s_wide;
+  if (threadIdx.x == 0) s_wide = 0;
+  __syncthreads();
+  if (wave_lane() == 0) atomicAdd(&s_wide, wide);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *reinterpret_cast<unsigned long long *>(counters + 6) = s_wide;
+    end_of_symbolic(counters, s_wide, report, sequence);
+    if (s_wide > (unsigned long long)INT32_MAX) data[n - 1] = -1;
+  }
+}
+
 // ---- pass 0: products per row, and the lists of rows too big for a wavefront ----
 // A workgroup takes up to kBoundsRows consecutive rows, eight lanes per row; rows
 // of A with more than kBoundsLongRow entries are queued in LDS and summed
@@ -368,8 +434,7 @@ inline int bounds_rows_per_group(int64_t M) {
 __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     int M, int rows_per_group, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
     const int *__restrict__ b_pos, int *__restrict__ products, int *__restrict__ small_rows,
-    int *__restrict__ medium_rows, int *__restrict__ huge_rows, int *__restrict__ counters,
-    const int *__restrict__ c_pos_if_narrow) {
+    int *__restrict__ medium_rows, int *__restrict__ huge_rows, int *__restrict__ counters) {
   constexpr int G = 8;  // lanes per row
   constexpr int kStep = kBlockThreads / G;
   __shared__ int s_long[kBoundsRows];
@@ -378,18 +443,17 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
   __shared__ int s_n[6];                  // [4], [5]: long and very long rows queued
   __shared__ int s_base[4];
   __shared__ long long s_part[kWavesPerBlock];
+  __shared__ unsigned long long s_giant_products;
   if (threadIdx.x < 6) s_n[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_giant_products = 0;
   __syncthreads();
   auto file_row = [&](int row, long long sum) {
     const int bound = sum > INT_MAX ? INT_MAX : (int)sum;
     products[row] = bound;
-    int list = bound >= kGiantProducts ? 3 : bound > kMediumProducts ? 1 : bound > kSmallProducts ? 0
+    const int list = bound >= kGiantProducts ? 3 : bound > kMediumProducts ? 1 : bound > kSmallProducts ? 0
                      : bound > kTinyProducts ? 2 : -1;
-    // The numeric pass knows the row's length: a row of many products but at most
-    // kMediumProducts distinct columns fits the sums of the tier below, whose
-    // smaller workgroups share a compute unit (B no wider than its bitmap).
-    if (list == 1 && c_pos_if_narrow && c_pos_if_narrow[row + 1] - c_pos_if_narrow[row] <= kMediumProducts) list = 0;
     if (list >= 0) s_list[list][atomicAdd(&s_n[list], 1)] = row;
+    if (list == 3) atomicAdd(&s_giant_products, (unsigned long long)bound);
   };
 
   const int t = threadIdx.x % G;
@@ -456,6 +520,8 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
   __syncthreads();
   if (threadIdx.x < 4 && s_n[threadIdx.x] > 0)
     s_base[threadIdx.x] = atomicAdd(&counters[threadIdx.x < 3 ? threadIdx.x : 5], s_n[threadIdx.x]);
+  if (threadIdx.x == 0 && s_giant_products > 0)
+    atomicAdd(reinterpret_cast<unsigned long long *>(counters + 10), s_giant_products);
   __syncthreads();
   int *const lists[3] = {medium_rows, huge_rows, small_rows};
 #pragma unroll
@@ -469,11 +535,15 @@ __device__ __forceinline__ int huge_row(const int *__restrict__ rows, int M, int
   return idx < n_giant ? rows[M - 1 - idx] : rows[idx - n_giant];
 }
 
-// counters: [0] medium rows, [1] huge rows, [2] small rows, [5] giant rows listed; [3], [4] next row to hand out;
-// [6..7] one 64-bit sum: the number of entries of the result
-__global__ void spgemm_reset_kernel(int *counters, int *c_pos_last) {
-  if (threadIdx.x < 8) counters[threadIdx.x] = 0;
-  if (threadIdx.x == 0 && c_pos_last) *c_pos_last = 0;
+// (The bitmaps of the rows that may be shared out start clear)
+__global__ __launch_bounds__(kBlockThreads) void spgemm_reset_kernel(int *counters, int *c_pos_last, int64_t clear_words,
+                                                                     unsigned *bits) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < kSpgemmCounters) counters[threadIdx.x] = 0;
+    if (threadIdx.x == 0 && c_pos_last) *c_pos_last = 0;
+  }
+  const int64_t stride = (int64_t)gridDim.x * kBlockThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x; i < clear_words; i += stride) bits[i] = 0u;
 }
 
 // ---- rows of at most kMicroProducts products: a quarter wavefront each -----------------
@@ -646,9 +716,9 @@ __device__ __forceinline__ void spgemm_team_row(
 // products by its four quarters at once, then those of up to kTinyProducts one
 // after the other with all its lanes (rows beyond that belong to the workgroup
 // kernels).  The two kinds of table share the wavefront's LDS.
-// QUARTERS = false: one row per wavefront, all lanes on it whatever its size; for
-// matrices of too few rows to fill the chip four to a wavefront.
-template <typename T, bool NUMERIC, bool QUARTERS>
+// (One row per wavefront, for matrices of too few rows to fill the chip four to a wavefront, is
+// spgemm_small_matrix_kernel's.)
+template <typename T, bool NUMERIC>
 __global__ __launch_bounds__(kBlockThreads) void spgemm_tiny_kernel(
     int M, const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
     const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
@@ -656,15 +726,6 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_tiny_kernel(
     T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
   constexpr int kQuarters = kWaveSize / kMicroTeam;
-  if (!QUARTERS) {
-    __shared__ TeamTables<A, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts> one;
-    const int w = threadIdx.x / kWaveSize;
-    const int64_t row = xcd_contiguous(blockIdx.x, gridDim.x) * kWavesPerBlock + w;
-    if (row >= M || products[row] > kTinyProducts) return;
-    spgemm_team_row<T, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts>(
-        one, w, wave_lane(), (int)row, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
-    return;
-  }
   union Tables {
     TeamTables<A, NUMERIC, kWaveSize, 1, kTinySlots, kTinyProducts> wave;
     TeamTables<A, NUMERIC, kMicroTeam, kQuarters, kMicroSlots, kMicroProducts> quarter;
@@ -697,8 +758,22 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_tiny_kernel(
 // ---- rows of at most PRODUCTS products: one workgroup each, 2 * PRODUCTS hash slots ----
 // THREADS: workgroup size (the tables of the larger form leave room for one workgroup per
 // CU: it is given 1024 threads rather than 256).
+template <typename A, bool NUMERIC, int PRODUCTS, int THREADS>
+struct MediumTables {
+  A vals[NUMERIC ? 2 * PRODUCTS : 1];
+  A cv[NUMERIC ? PRODUCTS : 1];
+  ProductBatch<THREADS, A> batch;
+  int keys[2 * PRODUCTS];
+  int ck[NUMERIC ? PRODUCTS : 1];
+  int scan[(THREADS / kWaveSize) + 1];
+  int red[2][(THREADS / kWaveSize)];
+  int cnt[NUMERIC ? PRODUCTS / 2 : 1];
+};
+
+// The rows `block`, block + n_blocks, ... of the list.
 template <typename T, bool NUMERIC, int PRODUCTS, int COUNTER, int THREADS>
-__global__ __launch_bounds__(THREADS) void spgemm_medium_kernel(
+__device__ __forceinline__ void spgemm_medium_rows(
+    MediumTables<typename Acc<T>::type, NUMERIC, PRODUCTS, THREADS> &lds, int block, int n_blocks,
     const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
     const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
     const int *__restrict__ rows, const int *__restrict__ counters, int *__restrict__ c_pos,
@@ -707,21 +782,21 @@ __global__ __launch_bounds__(THREADS) void spgemm_medium_kernel(
   constexpr int kSlots = 2 * PRODUCTS;
   constexpr int kBuckets = PRODUCTS / 2;
   constexpr int kBucketCrowd = 32;  // a fuller bucket sends the row to the bitonic sort
-  __shared__ int s_keys[kSlots];
-  __shared__ A s_vals[NUMERIC ? kSlots : 1];
-  __shared__ int s_ck[NUMERIC ? PRODUCTS : 1];
-  __shared__ A s_cv[NUMERIC ? PRODUCTS : 1];
-  __shared__ int s_scan[(THREADS / kWaveSize) + 1];
-  __shared__ int s_red[2][(THREADS / kWaveSize)];
-  __shared__ int s_cnt[NUMERIC ? kBuckets : 1];
-  __shared__ ProductBatch<THREADS, A> s_batch;
+  auto &s_keys = lds.keys;
+  auto &s_vals = lds.vals;
+  auto &s_ck = lds.ck;
+  auto &s_cv = lds.cv;
+  auto &s_scan = lds.scan;
+  auto &s_red = lds.red;
+  auto &s_cnt = lds.cnt;
+  auto &s_batch = lds.batch;
 
   const int tid = threadIdx.x;
   const int n_rows = counters[COUNTER];
 
   // (rows handed out one at a time through a counter, as in the bitmap tiers, measured
   // slower: these rows are short enough for the counter's round trip to show)
-  for (int idx = blockIdx.x; idx < n_rows; idx += gridDim.x) {
+  for (int idx = block; idx < n_rows; idx += n_blocks) {
     const int row = rows[idx];
     for (int s = tid; s < kSlots; s += THREADS) {
       s_keys[s] = -1;
@@ -854,6 +929,17 @@ __global__ __launch_bounds__(THREADS) void spgemm_medium_kernel(
   }
 }
 
+template <typename T, bool NUMERIC, int PRODUCTS, int COUNTER, int THREADS>
+__global__ __launch_bounds__(THREADS) void spgemm_medium_kernel(
+    const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
+    const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
+    const int *__restrict__ rows, const int *__restrict__ counters, int *__restrict__ c_pos,
+    int *__restrict__ c_crd, T *__restrict__ c_val) {
+  __shared__ MediumTables<typename Acc<T>::type, NUMERIC, PRODUCTS, THREADS> lds;
+  spgemm_medium_rows<T, NUMERIC, PRODUCTS, COUNTER, THREADS>(lds, blockIdx.x, gridDim.x, a_pos, a_crd, a_val, b_pos,
+                                                             b_crd, b_val, rows, counters, c_pos, c_crd, c_val);
+}
+
 // ---- rows beyond that: a bitmap over all columns -------------------------------------------
 // Workgroups of 1024 threads: such a row has tens of thousands of products and
 // is one workgroup's alone, so its width is the row's parallelism.  The
@@ -964,27 +1050,43 @@ constexpr int kLdsBudget = 160 * 1024 - 1024;
 
 // THREADS: workgroup size.  ACC: LDS sums to provide (0: all the LDS that is left).
 // LIST, WORK: which of `counters` holds the length of `rows` and the next row to hand out.
+template <typename A, bool NUMERIC, int WORDS, int THREADS, int ACC>
+struct BitmapTables {
+  static constexpr int kGroups = WORDS / 4;
+  static constexpr int kFixed = WORDS * 4 + (NUMERIC ? kGroups * 4 : 0) + (int)sizeof(ProductBatch<THREADS, A>) + 512;
+  static constexpr int kAccEntries = !NUMERIC ? 1 : ACC > 0 ? ACC : (kLdsBudget - kFixed) / (int)sizeof(A);
+  alignas(16) unsigned bits[WORDS];
+  int rank[NUMERIC ? kGroups : 1];  // rank of the first column of every group of four words
+  A acc[kAccEntries];
+  ProductBatch<THREADS, A> batch;
+  int scan[THREADS / kWaveSize];
+  int next;
+};
+
+// Block number `block` of n_blocks.  `narrow_rows`: the list of the tier above (its length in counters[1]), whose rows
+// of at most kMediumProducts distinct columns -- known in the numeric pass -- are taken here as well; null: none.
 template <typename T, bool NUMERIC, int WORDS, int THREADS, int ACC, int LIST, int WORK>
-__global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
+__device__ __forceinline__ void spgemm_lds_bitmap_rows(
+    BitmapTables<typename Acc<T>::type, NUMERIC, WORDS, THREADS, ACC> &lds, int block, int n_blocks,
     int M, int N, const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
     const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
-    const int *__restrict__ rows, int *__restrict__ counters, int *__restrict__ c_pos,
-    int *__restrict__ c_crd, T *__restrict__ c_val) {
+    const int *__restrict__ rows, const int *__restrict__ narrow_rows, int *__restrict__ counters,
+    int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
-  constexpr int kGroups = WORDS / 4;
-  constexpr int kFixed = WORDS * 4 + (NUMERIC ? kGroups * 4 : 0) + (int)sizeof(ProductBatch<THREADS, A>) + 512;
-  constexpr int kAccEntries = !NUMERIC ? 1 : ACC > 0 ? ACC : (kLdsBudget - kFixed) / (int)sizeof(A);
+  using Tables = BitmapTables<A, NUMERIC, WORDS, THREADS, ACC>;
+  constexpr int kAccEntries = Tables::kAccEntries;
   constexpr int kWaves = THREADS / kWaveSize;
-  __shared__ __align__(16) unsigned s_bits[WORDS];
-  __shared__ int s_rank[NUMERIC ? kGroups : 1];  // rank of the first column of every group of four words
-  __shared__ A s_acc[kAccEntries];
-  __shared__ ProductBatch<THREADS, A> s_batch;
-  __shared__ int s_scan[kWaves];
-  __shared__ int s_next;
+  auto &s_bits = lds.bits;
+  auto &s_rank = lds.rank;
+  auto &s_acc = lds.acc;
+  auto &s_batch = lds.batch;
+  auto &s_scan = lds.scan;
+  int &s_next = lds.next;
   const int tid = threadIdx.x;
   const int n_giant = LIST == 1 ? counters[5] : 0;  // only the list of the longest rows has the class
-  const int n_rows = counters[LIST] + n_giant;
-  if ((int)blockIdx.x >= n_rows) return;  // more workgroups than rows: no need to queue at the counter
+  const int n_own = counters[LIST] + n_giant;
+  const int n_rows = n_own + (narrow_rows ? counters[1] : 0);
+  if (block >= n_rows) return;  // more workgroups than rows: no need to queue at the counter
   constexpr int kRangeColumns = 32 * WORDS;
   A *acc = reinterpret_cast<A *>(c_val);
   // B with no more columns than the LDS holds sums: the numeric pass keeps a sum
@@ -1003,10 +1105,21 @@ __global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
       __syncthreads();
       idx = s_next;
     } else {
-      idx = (int)blockIdx.x + turn * (int)gridDim.x;
+      idx = block + turn * n_blocks;
     }
     if (idx >= n_rows) return;  // the same for every thread
-    const int row = LIST == 1 ? huge_row(rows, M, n_giant, idx) : rows[idx];
+    int row;
+    if (LIST == 1) {
+      row = huge_row(rows, M, n_giant, idx);
+      if (row < 0) continue;  // shared out among workgroups
+      // (of few distinct columns: the tier below's, whose smaller workgroups share a compute unit)
+      if (NUMERIC && N <= kNarrowColumns && idx >= n_giant && c_pos[row + 1] - c_pos[row] <= kMediumProducts) continue;
+    } else if (idx < n_own) {
+      row = rows[idx];
+    } else {
+      row = narrow_rows[idx - n_own];
+      if (c_pos[row + 1] - c_pos[row] > kMediumProducts) continue;
+    }
     const int a_lo = a_pos[row], a_hi = a_pos[row + 1];
     const int out = NUMERIC ? c_pos[row] : 0;
     int done = 0;  // distinct columns found in the ranges before this one
@@ -1103,8 +1216,236 @@ __global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
   }
 }
 
+template <typename T, bool NUMERIC, int WORDS, int THREADS, int ACC, int LIST, int WORK>
+__global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
+    int M, int N, const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
+    const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
+    const int *__restrict__ rows, const int *__restrict__ narrow_rows, int *__restrict__ counters,
+    int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
+  __shared__ BitmapTables<typename Acc<T>::type, NUMERIC, WORDS, THREADS, ACC> lds;
+  spgemm_lds_bitmap_rows<T, NUMERIC, WORDS, THREADS, ACC, LIST, WORK>(lds, blockIdx.x, gridDim.x, M, N, a_pos, a_crd,
+                                                                      a_val, b_pos, b_crd, b_val, rows, narrow_rows,
+                                                                      counters, c_pos, c_crd, c_val);
+}
+
+// ---- a matrix of few rows: the three kinds of 256-thread work in one launch --------------------
+// Below 32,768 rows the tiers' kernels are short and what a product costs is launches, 3 to 5 us
+// each: workgroups [0, n_bitmap) take bitmap rows, the next n_medium hash rows of up to
+// kSmallProducts products, the rest four rows of up to kTinyProducts each, the longest kinds first.
+// The kinds share the workgroup's LDS (40 KB with fp32 sums, four workgroups to a CU).
+template <typename T, bool NUMERIC>
+__global__ __launch_bounds__(kBlockThreads) void spgemm_small_matrix_kernel(
+    int M, int N, int n_bitmap, int n_medium, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
+    const T *__restrict__ a_val, const int *__restrict__ b_pos, const int *__restrict__ b_crd,
+    const T *__restrict__ b_val, const int *__restrict__ products, const int *__restrict__ small_rows,
+    const int *__restrict__ medium_rows, const int *__restrict__ narrow_rows, int *__restrict__ counters,
+    int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
+  using A = typename Acc<T>::type;
+  union Tables {
+    BitmapTables<A, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts> bitmap;
+    MediumTables<A, NUMERIC, kSmallProducts, kBlockThreads> medium;
+    TeamTables<A, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts> tiny;
+  };
+  __shared__ Tables lds;
+  int block = blockIdx.x;
+  if (block < n_bitmap) {
+    spgemm_lds_bitmap_rows<T, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts, 0, 4>(
+        lds.bitmap, block, n_bitmap, M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, medium_rows, narrow_rows, counters,
+        c_pos, c_crd, c_val);
+    return;
+  }
+  block -= n_bitmap;
+  if (block < n_medium) {
+    spgemm_medium_rows<T, NUMERIC, kSmallProducts, 2, kBlockThreads>(lds.medium, block, n_medium, a_pos, a_crd, a_val, b_pos,
+                                                                    b_crd, b_val, small_rows, counters, c_pos, c_crd, c_val);
+    return;
+  }
+  block -= n_medium;
+  const int w = threadIdx.x / kWaveSize;
+  const int row = block * kWavesPerBlock + w;
+  if (row >= M || products[row] > kTinyProducts) return;
+  spgemm_team_row<T, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts>(
+      lds.tiny, w, wave_lane(), row, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
+}
+
+// ---- rows shared out among workgroups --------------------------------------------------------
+// A row is one workgroup's in every tier above, so a tier ends when its longest row does: a hub of
+// 50,000 entries in a graph of 131,072 nodes has 850,000 products, 0.31 ms of the symbolic pass
+// and 1.25 ms of the numeric one on one CU (its 131,000 sums mostly miss the LDS), while the other
+// rows of the tier take a tenth of that on the whole chip.  A giant row with more than a 128th of
+// the giant rows' products -- twice a CU's share -- and at least kSplitProducts goes out in slices
+// of its A entries instead.  A slice ORs a bitmap of its columns, kept in LDS, into the row's
+// bitmap in memory, and adds its products to one sum per column there with device-wide
+// atomics: the row's columns are many and its products spread over them, so no address is
+// contended (a row with few distinct columns is not in this class: the numeric pass files it
+// below).  A pass over bitmap and sums then writes the row.  At most `pool` rows; where more
+// qualify there are enough rows to keep the chip busy and the rest stay one workgroup's.
+constexpr int kSplitProducts = 32768;
+constexpr int kSplitSliceProducts = 8192;   // aimed at: a row of p products gets p / 8192 slices, at most 64
+constexpr int kSplitMaxSlices = 64;
+constexpr int kSplitMaxRows = 64;
+constexpr int kSplitMaxColumns = 32 * 16384;  // the slice's bitmap is in LDS
+constexpr int kSplitMinColumns = 4096;        // a narrower B: a hub row has few products, and its sums fit the LDS
+constexpr size_t kSplitBudget = (size_t)64 << 20;
+
+inline int split_pool(int64_t N) {
+  if (N < kSplitMinColumns || N > kSplitMaxColumns) return 0;
+  const size_t fit = kSplitBudget / ((size_t)N * 8);
+  return (int)(fit < kSplitMaxRows ? fit : kSplitMaxRows);
+}
+
+// split_rows[slot] = row; items[i] = (slot, slice, slices, 0).  One workgroup.
+__global__ __launch_bounds__(kBlockThreads) void spgemm_split_select_kernel(
+    int M, int pool, const int *__restrict__ a_pos, const int *__restrict__ products, int *__restrict__ huge_rows,
+    int *__restrict__ counters, int *__restrict__ split_rows, int4 *__restrict__ items) {
+  __shared__ int s_rows, s_items;
+  if (threadIdx.x == 0) s_rows = s_items = 0;
+  __syncthreads();
+  const int n_giant = counters[5];
+  const unsigned long long share = *reinterpret_cast<const unsigned long long *>(counters + 10) / 128;
+  for (int i = threadIdx.x; i < n_giant; i += kBlockThreads) {
+    const int row = huge_rows[M - 1 - i];
+    const int p = products[row];
+    if (p < kSplitProducts || (unsigned long long)p < share) continue;
+    const int slot = atomicAdd(&s_rows, 1);
+    if (slot >= pool) continue;
+    huge_rows[M - 1 - i] = -1;
+    split_rows[slot] = row;
+    const int entries = a_pos[row + 1] - a_pos[row];
+    int slices = p / kSplitSliceProducts;
+    slices = slices > kSplitMaxSlices ? kSplitMaxSlices : slices;
+    slices = slices > entries ? entries : slices;
+    const int at = atomicAdd(&s_items, slices);  // at most pool * kSplitMaxSlices in all
+    for (int j = 0; j < slices; ++j) items[at + j] = make_int4(slot, j, slices, 0);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    counters[8] = s_rows < pool ? s_rows : pool;
+    counters[9] = s_items;
+  }
+}
+
+template <typename A>
+__global__ __launch_bounds__(kBlockThreads) void spgemm_split_clear_kernel(int N, const int *__restrict__ counters,
+                                                                           A *__restrict__ sums) {
+  const int64_t n = (int64_t)counters[8] * N, stride = (int64_t)gridDim.x * kBlockThreads;
+  for (int64_t i = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x; i < n; i += stride) sums[i] = (A)0;
+}
+
+// A slice's A entries.
+__device__ __forceinline__ void split_slice(const int4 &item, const int *a_pos, int row, int &from, int &to) {
+  const int lo = a_pos[row], entries = a_pos[row + 1] - lo;
+  from = lo + (int)((int64_t)entries * item.y / item.z);
+  to = lo + (int)((int64_t)entries * (item.y + 1) / item.z);
+}
+
+template <int WORDS>
+__global__ __launch_bounds__(kHugeThreads) void spgemm_split_columns_kernel(
+    int words, const int *__restrict__ a_pos, const int *__restrict__ a_crd, const int *__restrict__ b_pos,
+    const int *__restrict__ b_crd, const int *__restrict__ counters, const int *__restrict__ split_rows,
+    const int4 *__restrict__ items, unsigned *__restrict__ bits) {
+  __shared__ unsigned s_bits[WORDS];
+  __shared__ ProductBatch<kHugeThreads, float> s_batch;
+  __shared__ int s_scan[kHugeWaves];
+  const int tid = threadIdx.x;
+  const int n_items = counters[9];
+  for (int i = blockIdx.x; i < n_items; i += gridDim.x) {  // uniform
+    const int4 item = items[i];
+    int from, to;
+    split_slice(item, a_pos, split_rows[item.x], from, to);
+    for (int w = tid; w < words; w += kHugeThreads) s_bits[w] = 0u;
+    __syncthreads();
+    for_each_product<kHugeThreads, false, float, float>(from, to, tid, a_crd, nullptr, b_pos, b_crd, nullptr, s_batch, s_scan,
+                                                        [&](int k, float) { atomicOr(&s_bits[k >> 5], 1u << (k & 31)); });
+    __syncthreads();
+    unsigned *row_bits = bits + (size_t)item.x * (size_t)words;
+    for (int w = tid; w < words; w += kHugeThreads)
+      if (s_bits[w]) atomicOr(&row_bits[w], s_bits[w]);
+    __syncthreads();
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kHugeThreads) void spgemm_split_sums_kernel(
+    int N, const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
+    const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
+    const int *__restrict__ counters, const int *__restrict__ split_rows, const int4 *__restrict__ items,
+    typename Acc<T>::type *__restrict__ sums) {
+  using A = typename Acc<T>::type;
+  __shared__ ProductBatch<kHugeThreads, A> s_batch;
+  __shared__ int s_scan[kHugeWaves];
+  const int n_items = counters[9];
+  for (int i = blockIdx.x; i < n_items; i += gridDim.x) {  // uniform
+    const int4 item = items[i];
+    int from, to;
+    split_slice(item, a_pos, split_rows[item.x], from, to);
+    A *row_sums = sums + (size_t)item.x * (size_t)N;
+    for_each_product<kHugeThreads, true, T, A>(from, to, threadIdx.x, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan,
+                                               [&](int k, A product) { atomic_accumulate<A>(&row_sums[k], product); });
+  }
+}
+
+struct SplitCount {
+  const int *rows;
+  const unsigned *bits;
+  int words;
+};
+__global__ __launch_bounds__(kBlockThreads) void spgemm_split_count_kernel(const int *__restrict__ counters, SplitCount split,
+                                                                           int *__restrict__ c_pos) {
+  __shared__ int s_scan[kWavesPerBlock];
+  const int slot = blockIdx.x;
+  if (slot >= counters[8]) return;
+  int mine = 0, total = 0;
+  for (int w = threadIdx.x; w < split.words; w += kBlockThreads) mine += __popc(split.bits[(size_t)slot * split.words + w]);
+  (void)block_exclusive_scan(mine, s_scan, total);
+  if (threadIdx.x == 0) c_pos[split.rows[slot]] = total;
+}
+
+// Writes the shared-out rows.  grid: (pieces of kEmitWords bitmap words, rows).
+constexpr int kEmitWords = 1024;
+template <typename T>
+__global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
+    int N, int words, const int *__restrict__ counters, const int *__restrict__ split_rows,
+    const unsigned *__restrict__ bits, const typename Acc<T>::type *__restrict__ sums, const int *__restrict__ c_pos,
+    int *__restrict__ c_crd, T *__restrict__ c_val) {
+  __shared__ unsigned s_bits[kEmitWords];
+  __shared__ int s_rank[kEmitWords];
+  __shared__ int s_scan[kHugeWaves];
+  const int slot = blockIdx.y;
+  if (slot >= counters[8]) return;
+  const int tid = threadIdx.x, lane = wave_lane();
+  const unsigned *row_bits = bits + (size_t)slot * (size_t)words;
+  const int first = (int)blockIdx.x * kEmitWords;
+  int mine = 0, before = 0;
+  for (int w = tid; w < first; w += kHugeThreads) mine += __popc(row_bits[w]);
+  (void)block_exclusive_scan_n<kHugeWaves>(mine, s_scan, before);
+  const unsigned word = first + tid < words ? row_bits[first + tid] : 0u;
+  int unused = 0;
+  s_rank[tid] = block_exclusive_scan_n<kHugeWaves>(__popc(word), s_scan, unused);
+  s_bits[tid] = word;
+  __syncthreads();
+  const size_t out = (size_t)c_pos[split_rows[slot]] + before;
+  const typename Acc<T>::type *row_sums = sums + (size_t)slot * (size_t)N;
+  // two bitmap words, 64 columns, per wavefront and step: sums are read and entries written coalesced
+  for (int w = 2 * (tid / kWaveSize); w < kEmitWords; w += 2 * kHugeWaves) {
+    const int mine_at = w + (lane >> 5), bit = lane & 31;
+    const unsigned b = s_bits[mine_at];
+    if ((b >> bit) & 1u) {
+      const int col = (first + mine_at) * 32 + bit;
+      const size_t at = out + s_rank[mine_at] + __popc(b & ((1u << bit) - 1u));
+      c_crd[at] = col;
+      c_val[at] = (T)row_sums[col];
+    }
+  }
+}
+
 // ---- host side ------------------------------------------------------------------------------
 struct SpgemmWorkspace {
+  int pool;               // rows that can be shared out among workgroups
+  int *split_rows;
+  int4 *split_items;
+  unsigned *split_bits;
+  void *split_sums;
   int *products, *small_rows, *medium_rows, *huge_rows, *counters;
   int huge_pool;
   int *scan_totals;
@@ -1123,7 +1464,12 @@ inline SpgemmWorkspace spgemm_layout(char *base, int64_t M, int64_t N, size_t el
   ws.small_rows = reinterpret_cast<int *>(take((size_t)M * 4));
   ws.medium_rows = reinterpret_cast<int *>(take((size_t)M * 4));
   ws.huge_rows = reinterpret_cast<int *>(take((size_t)M * 4));
-  ws.counters = reinterpret_cast<int *>(take(32));
+  ws.counters = reinterpret_cast<int *>(take(kSpgemmCounters * 4));
+  ws.pool = split_pool(N);
+  ws.split_rows = reinterpret_cast<int *>(take((size_t)ws.pool * 4));
+  ws.split_items = reinterpret_cast<int4 *>(take((size_t)ws.pool * kSplitMaxSlices * sizeof(int4)));
+  ws.split_bits = reinterpret_cast<unsigned *>(take((size_t)ws.pool * ((size_t)(N + 31) / 32) * 4));
+  ws.split_sums = take((size_t)ws.pool * (size_t)N * 8);
   ws.scan_totals = reinterpret_cast<int *>(take(((size_t)(M + 1) / kScanTile + 1) * 4));
   ws.huge_pool = huge_workgroups(N);
   // up to kLdsBitmapColumns columns the bitmap tier lives in LDS and needs no slabs
@@ -1155,73 +1501,140 @@ inline int spgemm_check(const char *fn, int64_t M, int64_t K, int64_t N, const v
   return SCORCH_HIP_OK;
 }
 
+// What the symbolic pass found out, for a numeric pass over the same workspace.
+struct SpgemmReport {
+  int64_t entries;                                         // of the result; -1: 2^31 or more
+  int64_t small, medium, huge, giant, split, split_items;  // rows listed per tier; slices of the rows shared out
+};
+constexpr int kSpgemmReportWords = 7;
+
+// `known`: the numeric pass finds the row lists of the symbolic pass in the workspace and launches what has rows.
+// `sync`: the symbolic pass hands its report over.
 template <typename T, bool NUMERIC>
 int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val, const int *b_pos,
                const int *b_crd, const T *b_val, int *c_pos, int *c_crd, T *c_val,
-               const SpgemmWorkspace &ws, hipStream_t stream) {
-  spgemm_reset_kernel<<<1, 64, 0, stream>>>(ws.counters, NUMERIC ? nullptr : c_pos + M);
-  SCORCH_HIP_CHECK(hipGetLastError());
-  const int rows_per_group = bounds_rows_per_group(M);
-  const unsigned row_groups = (unsigned)(((int64_t)M + rows_per_group - 1) / rows_per_group);
-  spgemm_bounds_kernel<<<row_groups, kBlockThreads, 0, stream>>>(M, rows_per_group, a_pos, a_crd, b_pos, ws.products,
-                                                                ws.small_rows, ws.medium_rows,
-                                                                ws.huge_rows, ws.counters,
-                                                                NUMERIC && N <= 32 * 4096 ? c_pos : nullptr);
-  SCORCH_HIP_CHECK(hipGetLastError());
-  // four rows to a wavefront once that still leaves every wavefront slot of the chip a wavefront
-  if ((int64_t)M >= 4 * 8192) {
+               const SpgemmWorkspace &ws, hipStream_t stream, const SpgemmReport *known = nullptr,
+               SyncCall *sync = nullptr) {
+  using A = typename Acc<T>::type;
+  const int words = (N + 31) / 32;
+  if (!known) {
+    const int64_t clear_words = (int64_t)ws.pool * words;
+    const unsigned clear_blocks = (unsigned)(1 + (clear_words < 1 << 18 ? clear_words : 1 << 18) / 1024);
+    spgemm_reset_kernel<<<clear_blocks, kBlockThreads, 0, stream>>>(ws.counters, NUMERIC ? nullptr : c_pos + M, clear_words,
+                                                                    ws.split_bits);
+    SCORCH_HIP_CHECK(hipGetLastError());
+    const int rows_per_group = bounds_rows_per_group(M);
+    const unsigned row_groups = (unsigned)(((int64_t)M + rows_per_group - 1) / rows_per_group);
+    spgemm_bounds_kernel<<<row_groups, kBlockThreads, 0, stream>>>(M, rows_per_group, a_pos, a_crd, b_pos, ws.products,
+                                                                  ws.small_rows, ws.medium_rows,
+                                                                  ws.huge_rows, ws.counters);
+    SCORCH_HIP_CHECK(hipGetLastError());
+  }
+  if (ws.pool > 0 && (!known || known->split > 0)) {
+    A *sums = static_cast<A *>(ws.split_sums);
+    if (!known) {
+      spgemm_split_select_kernel<<<1, kBlockThreads, 0, stream>>>(M, ws.pool, a_pos, ws.products, ws.huge_rows, ws.counters,
+                                                                 ws.split_rows, ws.split_items);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      auto columns_of = words <= 4096 ? &spgemm_split_columns_kernel<4096> : &spgemm_split_columns_kernel<kSplitMaxColumns / 32>;
+      columns_of<<<512, kHugeThreads, 0, stream>>>(words, a_pos, a_crd, b_pos, b_crd, ws.counters, ws.split_rows,
+                                                   ws.split_items, ws.split_bits);
+      SCORCH_HIP_CHECK(hipGetLastError());
+    }
+    if (NUMERIC) {
+      const int64_t n_sums = (int64_t)(known ? (int)known->split : ws.pool) * N;
+      spgemm_split_clear_kernel<A><<<(unsigned)(1 + (n_sums < 1 << 20 ? n_sums : 1 << 20) / 1024), kBlockThreads, 0, stream>>>(
+          N, ws.counters, sums);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      const unsigned slices = known ? (unsigned)known->split_items : 512u;
+      spgemm_split_sums_kernel<T><<<slices, kHugeThreads, 0, stream>>>(N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.counters,
+                                                                      ws.split_rows, ws.split_items, sums);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      const unsigned pieces = (unsigned)((words + kEmitWords - 1) / kEmitWords);
+      spgemm_split_emit_kernel<T><<<dim3(pieces, (unsigned)(known ? known->split : ws.pool)), kHugeThreads, 0, stream>>>(
+          N, words, ws.counters, ws.split_rows, ws.split_bits, sums, c_pos, c_crd, c_val);
+      SCORCH_HIP_CHECK(hipGetLastError());
+    }
+  }
+  const bool narrow = N <= kNarrowColumns;
+  // rows the 256-thread bitmap kernel goes through; with the result's row pointer known, also those of the tier above
+  // that turn out to have few distinct columns
+  const int *narrow_rows = NUMERIC && narrow ? ws.huge_rows : nullptr;
+  const auto blocks_for = [&](int64_t rows) { return (unsigned)(rows < kMediumWorkgroups ? rows : kMediumWorkgroups); };
+  const unsigned small_blocks = blocks_for(known ? known->small : M);
+  const unsigned bitmap_blocks = blocks_for(known ? known->medium + (narrow_rows ? known->huge : 0) : M);
+  if (M < 4 * 8192 && narrow) {
+    const unsigned tiny_blocks = (unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock);
+    spgemm_small_matrix_kernel<T, NUMERIC><<<bitmap_blocks + small_blocks + tiny_blocks, kBlockThreads, 0, stream>>>(
+        M, N, (int)bitmap_blocks, (int)small_blocks, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows,
+        ws.medium_rows, narrow_rows, ws.counters, c_pos, c_crd, c_val);
+    SCORCH_HIP_CHECK(hipGetLastError());
+  } else {
+    // four rows to a wavefront
     const int64_t rows_per_block = kWavesPerBlock * (kWaveSize / kMicroTeam);
     const unsigned tiny_blocks = (unsigned)round_up_8(((int64_t)M + rows_per_block - 1) / rows_per_block);
-    spgemm_tiny_kernel<T, NUMERIC, true><<<tiny_blocks, kBlockThreads, 0, stream>>>(
+    spgemm_tiny_kernel<T, NUMERIC><<<tiny_blocks, kBlockThreads, 0, stream>>>(
         M, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, c_pos, c_crd, c_val);
-  } else {
-    const unsigned tiny_blocks = (unsigned)round_up_8(((int64_t)M + kWavesPerBlock - 1) / kWavesPerBlock);
-    spgemm_tiny_kernel<T, NUMERIC, false><<<tiny_blocks, kBlockThreads, 0, stream>>>(
-        M, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, c_pos, c_crd, c_val);
+    SCORCH_HIP_CHECK(hipGetLastError());
+    if (small_blocks) {
+      spgemm_medium_kernel<T, NUMERIC, kSmallProducts, 2, kBlockThreads><<<small_blocks, kBlockThreads, 0, stream>>>(
+          a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.small_rows, ws.counters, c_pos, c_crd, c_val);
+      SCORCH_HIP_CHECK(hipGetLastError());
+    }
+    if (bitmap_blocks && narrow) {
+      // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
+      spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts, 0, 4>
+          <<<bitmap_blocks, kBlockThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
+                                                        narrow_rows, ws.counters, c_pos, c_crd, c_val);
+    } else if (bitmap_blocks) {
+      // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
+      // beside them (with 8-byte sums, no more than 256)
+      constexpr int kThreads = sizeof(A) > 4 ? kBlockThreads : kHugeThreads;
+      spgemm_medium_kernel<T, NUMERIC, kMediumProducts, 0, kThreads><<<bitmap_blocks, kThreads, 0, stream>>>(
+          a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
+    }
+    SCORCH_HIP_CHECK(hipGetLastError());
   }
-  SCORCH_HIP_CHECK(hipGetLastError());
-  const unsigned medium_blocks = (unsigned)(M < kMediumWorkgroups ? M : kMediumWorkgroups);
-  spgemm_medium_kernel<T, NUMERIC, kSmallProducts, 2, kBlockThreads><<<medium_blocks, kBlockThreads, 0, stream>>>(
-      a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.small_rows, ws.counters, c_pos, c_crd, c_val);
-  SCORCH_HIP_CHECK(hipGetLastError());
-  if (N <= 32 * 4096) {
-    // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
-    spgemm_lds_bitmap_kernel<T, NUMERIC, 4096, kBlockThreads, kMediumProducts, 0, 4>
-        <<<medium_blocks, kBlockThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val,
-                                                      ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
-  } else {
-    // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
-    // beside them (with 8-byte sums, no more than 256)
-    constexpr int kThreads = sizeof(typename Acc<T>::type) > 4 ? kBlockThreads : kHugeThreads;
-    spgemm_medium_kernel<T, NUMERIC, kMediumProducts, 0, kThreads><<<medium_blocks, kThreads, 0, stream>>>(
-        a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
-  }
-  SCORCH_HIP_CHECK(hipGetLastError());
   // one workgroup per CU's worth of LDS; more only queue up behind them
-  const unsigned lds_pool = (unsigned)(M < 512 ? M : 512);
-  if (N <= 32 * 4096)
-    spgemm_lds_bitmap_kernel<T, NUMERIC, 4096, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
-        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, ws.counters, c_pos, c_crd, c_val);
-  else if (!NUMERIC && N > 32 * 16384 && N <= 32 * 32768)
+  const int64_t huge_rows = known ? known->huge + known->giant - known->split : M;
+  const unsigned lds_pool = (unsigned)(huge_rows < 512 ? huge_rows : 512);
+  if (lds_pool == 0) {
+  } else if (narrow) {
+    spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
+        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, nullptr, ws.counters, c_pos, c_crd, c_val);
+  } else if (!NUMERIC && N > 32 * 16384 && N <= 32 * 32768) {
     // the symbolic pass keeps no ranks or sums: its bitmap can be twice as wide, one range instead of two
     spgemm_lds_bitmap_kernel<T, NUMERIC, NUMERIC ? 16384 : 32768, kHugeThreads, 0, 1, 3>
         <<<lds_pool, kHugeThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows,
-                                                ws.counters, c_pos, c_crd, c_val);
-  else if (N <= kLdsBitmapColumns)
+                                                nullptr, ws.counters, c_pos, c_crd, c_val);
+  } else if (N <= kLdsBitmapColumns) {
     spgemm_lds_bitmap_kernel<T, NUMERIC, 16384, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
-        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, ws.counters, c_pos, c_crd, c_val);
-  else
+        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, nullptr, ws.counters, c_pos, c_crd, c_val);
+  } else {
     spgemm_huge_kernel<T, NUMERIC><<<ws.huge_pool, kHugeThreads, 0, stream>>>(
         M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, ws.counters, ws.bitmaps,
         ws.ranks, c_pos, c_crd, c_val);
+  }
   SCORCH_HIP_CHECK(hipGetLastError());
   if (!NUMERIC) {
     const int64_t n = (int64_t)M + 1;
-    const unsigned tiles = (unsigned)((n + kScanTile - 1) / kScanTile);
     unsigned long long *grand_total = reinterpret_cast<unsigned long long *>(ws.counters + 6);
+    const SplitCount split = {ws.pool > 0 ? ws.split_rows : nullptr, ws.split_bits, words};
+    int64_t *report = sync ? sync->target() : nullptr;
+    const int64_t sequence = sync ? sync->sequence() : 0;
+    if (ws.pool > 0) {
+      spgemm_split_count_kernel<<<(unsigned)ws.pool, kBlockThreads, 0, stream>>>(ws.counters, split, c_pos);
+      SCORCH_HIP_CHECK(hipGetLastError());
+    }
+    if (n <= kScanOneGroup) {
+      scan_one_group_kernel<<<1, kScanThreads, 0, stream>>>(c_pos, (int)n, ws.counters, report, sequence);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      return SCORCH_HIP_OK;
+    }
+    const unsigned tiles = (unsigned)((n + kScanTile - 1) / kScanTile);
     scan_tile_totals_kernel<<<tiles, kBlockThreads, 0, stream>>>(c_pos, n, ws.scan_totals, grand_total);
     SCORCH_HIP_CHECK(hipGetLastError());
-    scan_spine_kernel<<<1, kBlockThreads, 0, stream>>>(ws.scan_totals, tiles);
+    scan_spine_kernel<<<1, kBlockThreads, 0, stream>>>(ws.scan_totals, tiles, ws.counters, report, sequence);
     SCORCH_HIP_CHECK(hipGetLastError());
     scan_apply_kernel<<<tiles, kBlockThreads, 0, stream>>>(c_pos, n, ws.scan_totals, grand_total);
     SCORCH_HIP_CHECK(hipGetLastError());
@@ -1233,15 +1646,18 @@ template <typename T>
 int spgemm_numeric_entry(const char *fn, int64_t M, int64_t K, int64_t N, const int32_t *a_pos,
                          const int32_t *a_crd, const T *a_val, const int32_t *b_pos,
                          const int32_t *b_crd, const T *b_val, const int32_t *c_pos, int32_t *c_crd,
-                         T *c_val, void *workspace, size_t workspace_bytes, void *stream) {
+                         T *c_val, void *workspace, size_t workspace_bytes, void *stream,
+                         const int64_t *report = nullptr) {
   if (int rc = spgemm_check(fn, M, K, N, a_pos, a_crd, b_pos, b_crd, c_pos, workspace, workspace_bytes,
                             sizeof(T)))
     return rc;
   if (M == 0 || N == 0 || K == 0) return SCORCH_HIP_OK;
   const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, sizeof(T));
+  SpgemmReport known;
+  if (report) known = {report[0], report[1], report[2], report[3], report[4], report[5], report[6]};
   return spgemm_run<T, true>((int)M, (int)N, a_pos, a_crd, a_val, b_pos, b_crd, b_val,
                              const_cast<int32_t *>(c_pos), c_crd, c_val, ws,
-                             static_cast<hipStream_t>(stream));
+                             static_cast<hipStream_t>(stream), report ? &known : nullptr);
 }
 
 }  // namespace scorch
@@ -1264,13 +1680,39 @@ int scorch_hip_spgemm_csr_symbolic(int64_t M, int64_t K, int64_t N, const int32_
     return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (M == 0) {
-    spgemm_reset_kernel<<<1, 64, 0, s>>>(static_cast<int *>(workspace), c_row_ptr);
+    spgemm_reset_kernel<<<1, kBlockThreads, 0, s>>>(static_cast<int *>(workspace), c_row_ptr, 0, nullptr);
     SCORCH_HIP_CHECK(hipGetLastError());
     return SCORCH_HIP_OK;
   }
   const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, 1);
   return spgemm_run<float, false>((int)M, (int)N, a_row_ptr, a_col_idx, nullptr, b_row_ptr, b_col_idx,
                                   nullptr, c_row_ptr, nullptr, nullptr, ws, s);
+}
+
+int scorch_hip_spgemm_csr_symbolic_planned(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                           const int32_t *a_col_idx, const int32_t *b_row_ptr,
+                                           const int32_t *b_col_idx, int32_t *c_row_ptr, void *workspace,
+                                           size_t workspace_bytes, int64_t *report, void *stream) {
+  using namespace scorch;
+  const char *fn = "scorch_hip_spgemm_csr_symbolic_planned";
+  if (int rc = spgemm_check(fn, M, K, N, a_row_ptr, a_col_idx, b_row_ptr, b_col_idx, c_row_ptr,
+                            workspace, workspace_bytes, 1))
+    return rc;
+  SCORCH_REQUIRE(report != nullptr, "%s: report is NULL", fn);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  for (int i = 0; i < kSpgemmReportWords; ++i) report[i] = 0;
+  if (M == 0) {
+    spgemm_reset_kernel<<<1, kBlockThreads, 0, s>>>(static_cast<int *>(workspace), c_row_ptr, 0, nullptr);
+    SCORCH_HIP_CHECK(hipGetLastError());
+    return SCORCH_HIP_OK;
+  }
+  SyncCall sync;
+  if (sync.null()) return fail(SCORCH_HIP_ERUNTIME, "%s: no memory for the report", fn);
+  const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, 1);
+  if (int rc = spgemm_run<float, false>((int)M, (int)N, a_row_ptr, a_col_idx, nullptr, b_row_ptr, b_col_idx, nullptr,
+                                        c_row_ptr, nullptr, nullptr, ws, s, nullptr, &sync))
+    return rc;
+  return sync.wait(fn, s, report, kSpgemmReportWords);
 }
 
 #define SCORCH_DEFINE_SPGEMM(SUFFIX, T)                                                             \
@@ -1283,6 +1725,18 @@ int scorch_hip_spgemm_csr_symbolic(int64_t M, int64_t K, int64_t N, const int32_
                                            a_row_ptr, a_col_idx, a_vals, b_row_ptr, b_col_idx,      \
                                            b_vals, c_row_ptr, c_col_idx, c_vals, workspace,         \
                                            workspace_bytes, stream);                                \
+  }                                                                                                 \
+  int scorch_hip_spgemm_csr_numeric_planned_##SUFFIX(                                                \
+      int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr, const int32_t *a_col_idx,           \
+      const T *a_vals, const int32_t *b_row_ptr, const int32_t *b_col_idx, const T *b_vals,          \
+      const int32_t *c_row_ptr, int32_t *c_col_idx, T *c_vals, void *workspace,                      \
+      size_t workspace_bytes, const int64_t *report, void *stream) {                                 \
+    SCORCH_REQUIRE(report && report[0] >= 0, "scorch_hip_spgemm_csr_numeric_planned_" #SUFFIX         \
+                   ": no report of a symbolic pass");                                               \
+    return scorch::spgemm_numeric_entry<T>("scorch_hip_spgemm_csr_numeric_planned_" #SUFFIX, M, K, N, \
+                                           a_row_ptr, a_col_idx, a_vals, b_row_ptr, b_col_idx,      \
+                                           b_vals, c_row_ptr, c_col_idx, c_vals, workspace,         \
+                                           workspace_bytes, stream, report);                        \
   }
 
 SCORCH_DEFINE_SPGEMM(f32, float)

@@ -25,6 +25,7 @@
 // inspection pass below reports it) choose between this kernel and the
 // merge-path one.
 #include "spmm.hpp"
+#include "sync.hpp"
 
 namespace scorch {
 
@@ -222,10 +223,21 @@ __global__ void csr_inspect_clear_kernel(int *__restrict__ report) {
   if (threadIdx.x < kInspectReportInts) report[threadIdx.x] = 0;
 }
 
+// PUBLISH: the report goes to the host thread that waits for it.  Every workgroup leaves its totals in `partials`
+// (kInspectReportInts ints each) and takes a ticket; the one that takes the last adds them up.  (Otherwise: added into
+// `report` with atomics, which another launch has cleared.  Workgroups by the thousand queue up at those: 46 us for
+// 600,000 entries, 15 us for 131,072; with at most 512 of them and one ticket each 12 and 6.)
+struct InspectSync {
+  int *tickets;
+  unsigned tickets_before;
+  int64_t *to;
+  int64_t sequence;
+};
+template <bool PUBLISH>
 __global__ __launch_bounds__(kBlockThreads) void csr_inspect_kernel(int M, int K, int64_t nnz,
                                                                     const int *__restrict__ row_ptr,
                                                                     const int *__restrict__ col_idx,
-                                                                    int *__restrict__ report) {
+                                                                    int *__restrict__ report, InspectSync sync) {
   const int64_t stride = (int64_t)gridDim.x * kBlockThreads;
   const int64_t first = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x;
   int bad_rows = 0, bad_cols = 0, longest = 0, empty = 0;
@@ -304,6 +316,15 @@ __global__ __launch_bounds__(kBlockThreads) void csr_inspect_kernel(int M, int K
       descents += s_descents[w];
       runs += s_runs[w];
     }
+    if constexpr (PUBLISH) {
+      int *mine = report + (size_t)blockIdx.x * kInspectReportInts;
+      const int totals[6] = {s_bad_rows, s_bad_cols, longest, empty, descents, runs};
+#pragma unroll
+      for (int i = 0; i < 6; ++i) __hip_atomic_store(mine + i, totals[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned ticket = __hip_atomic_fetch_add(reinterpret_cast<unsigned *>(sync.tickets), 1u, __ATOMIC_ACQ_REL,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+      s_bad_rows = ticket - sync.tickets_before == gridDim.x - 1;  // the last one
+    } else {
     if (s_bad_rows) atomicOr(&report[0], 1);
     if (s_bad_cols) atomicOr(&report[1], 1);
     if (longest > 0) atomicMax(&report[2], longest);
@@ -311,6 +332,48 @@ __global__ __launch_bounds__(kBlockThreads) void csr_inspect_kernel(int M, int K
     // partial sums may be negative (the row loop's corrections); the totals lie in [0, nnz]
     if (descents != 0) atomicAdd(&report[4], descents);
     if (runs != 0) atomicAdd(&report[5], runs);
+    }
+  }
+  if constexpr (PUBLISH) {
+    __syncthreads();
+    if (!s_bad_rows) return;
+    int sums[6] = {0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += kBlockThreads) {
+      const int *of = report + (size_t)b * kInspectReportInts;
+      int v[6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) v[i] = __hip_atomic_load(of + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sums[0] |= v[0];
+      sums[1] |= v[1];
+      sums[2] = v[2] > sums[2] ? v[2] : sums[2];
+      sums[3] += v[3];
+      sums[4] += v[4];
+      sums[5] += v[5];
+    }
+    __shared__ int s_sums[kWavesPerBlock][6];
+#pragma unroll
+    for (int off = kWaveSize / 2; off > 0; off >>= 1)
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        const int other = __shfl_xor(sums[i], off);
+        sums[i] = i < 2 ? sums[i] | other : i == 2 ? (other > sums[i] ? other : sums[i]) : sums[i] + other;
+      }
+    if (wave_lane() == 0)
+#pragma unroll
+      for (int i = 0; i < 6; ++i) s_sums[threadIdx.x / kWaveSize][i] = sums[i];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int64_t words[6];
+      for (int i = 0; i < 6; ++i) {
+        int t = s_sums[0][i];
+        for (int w = 1; w < kWavesPerBlock; ++w) {
+          const int other = s_sums[w][i];
+          t = i < 2 ? t | other : i == 2 ? (other > t ? other : t) : t + other;
+        }
+        words[i] = t;
+      }
+      sync_publish(sync.to, sync.sequence, words, 6);
+    }
   }
 }
 
@@ -357,9 +420,38 @@ int scorch_hip_csr_inspect(int64_t M, int64_t K, int64_t nnz, const int32_t *row
   const int64_t work = (M > nnz ? M : nnz) + 1;
   int64_t blocks = (work + scorch::kBlockThreads - 1) / scorch::kBlockThreads;
   if (blocks > 2048) blocks = 2048;
-  scorch::csr_inspect_kernel<<<dim3((unsigned)blocks), scorch::kBlockThreads, 0, s>>>((int)M, (int)K, nnz, row_ptr,
-                                                                                    col_idx, report);
+  scorch::csr_inspect_kernel<false><<<dim3((unsigned)blocks), scorch::kBlockThreads, 0, s>>>(
+      (int)M, (int)K, nnz, row_ptr, col_idx, report, scorch::InspectSync{});
   SCORCH_HIP_CHECK(hipGetLastError());
+  return SCORCH_HIP_OK;
+}
+
+int scorch_hip_csr_inspect_now(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
+                               int32_t *report, void *stream) {
+  using namespace scorch;
+  const char *fn = "scorch_hip_csr_inspect_now";
+  if (M < 0 || K < 0 || nnz < 0)
+    return fail(SCORCH_HIP_EINVAL, "%s: negative size (M=%lld K=%lld nnz=%lld)", fn, (long long)M, (long long)K,
+                (long long)nnz);
+  if (M >= INT32_MAX || K > INT32_MAX || nnz > INT32_MAX)
+    return fail(SCORCH_HIP_EUNSUPPORTED, "%s: M, K and nnz must fit the int32 index arrays", fn);
+  SCORCH_REQUIRE(row_ptr != nullptr && report != nullptr, "%s: row_ptr or report is NULL", fn);
+  SCORCH_REQUIRE(nnz == 0 || col_idx != nullptr, "%s: col_idx is NULL with nnz=%lld", fn, (long long)nnz);
+  SCORCH_REQUIRE(aligned_to(row_ptr, 4) && aligned_to(col_idx, 4), "%s: arrays must be 4-byte aligned", fn);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  SyncCall sync;
+  if (sync.null()) return fail(SCORCH_HIP_ERUNTIME, "%s: no memory for the report", fn);
+  const int64_t work = (M > nnz ? M : nnz) + 1;
+  int64_t blocks = (work + 2 * kBlockThreads - 1) / (2 * kBlockThreads);
+  constexpr int64_t kMost = (kSyncDeviceInts - 16) / kInspectReportInts;
+  if (blocks > kMost) blocks = kMost;
+  const InspectSync how = {sync.scratch(), sync.tickets_before((unsigned)blocks), sync.target(), sync.sequence()};
+  csr_inspect_kernel<true><<<dim3((unsigned)blocks), kBlockThreads, 0, s>>>((int)M, (int)K, nnz, row_ptr, col_idx,
+                                                                          sync.scratch() + 16, how);
+  SCORCH_HIP_CHECK(hipGetLastError());
+  int64_t words[6];
+  if (int rc = sync.wait(fn, s, words, 6)) return rc;
+  for (int i = 0; i < kInspectReportInts; ++i) report[i] = i < 6 ? (int32_t)words[i] : 0;
   return SCORCH_HIP_OK;
 }
 

@@ -78,6 +78,11 @@ SIGNATURES = {
     "scorch_hip_spgemm_csr_numeric_f64": (ctypes.c_int, _SPGEMM),
     "scorch_hip_spgemm_csr_numeric_i32": (ctypes.c_int, _SPGEMM),
     "scorch_hip_spgemm_csr_numeric_i64": (ctypes.c_int, _SPGEMM),
+    "scorch_hip_spgemm_csr_symbolic_planned": (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
+                                                              _size, ctypes.POINTER(_i64), _ptr]),
+    **{"scorch_hip_spgemm_csr_numeric_planned_" + t: (ctypes.c_int, _SPGEMM[:-1] + [ctypes.POINTER(_i64), _ptr])
+       for t in ("f32", "f64", "i32", "i64")},
+    "scorch_hip_csr_inspect_now": (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, ctypes.POINTER(ctypes.c_int32), _ptr]),
     "scorch_hip_sddmm_coo_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,
                                                 _ptr, _ptr]),
     "scorch_hip_sddmm_csr_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,

@@ -21,6 +21,7 @@ is re-stored once by column tiles (see CsrPlan and _tiled_operand below).
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 import weakref
@@ -37,6 +38,7 @@ _empty_like = torch.empty_like
 
 HINT_MOSTLY_EMPTY_ROWS = 0x100      # SCORCH_HIP_HINT_MOSTLY_EMPTY_ROWS of include/scorch_hip.h
 INSPECT_REPORT_INTS = 8             # SCORCH_HIP_INSPECT_REPORT_INTS
+SPGEMM_REPORT_WORDS = 7             # SCORCH_HIP_SPGEMM_REPORT_WORDS
 _SUFFIX = {torch.float32: "f32", torch.float64: "f64", torch.int32: "i32", torch.int64: "i64"}
 
 
@@ -315,8 +317,8 @@ class CsrPlan:
 
 
 def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, what: str = "operand") -> Optional[CsrPlan]:
-    """The plan of (pos, crd), built on first sight: one inspection kernel and
-    one read of its four-integer report (a synchronisation).  Raises ValueError
+    """The plan of (pos, crd), built on first sight: one inspection kernel whose
+    report the host waits for.  Raises ValueError
     for a malformed index -- row pointers that do not start at 0, end at
     len(crd) or decrease, column indices outside [0, n_cols) -- before any
     kernel dereferences it.  None when planning is switched off or the stream
@@ -332,11 +334,11 @@ def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, wha
     if torch.cuda.is_current_stream_capturing():
         return None
     dev = pos.device
-    report = _empty(INSPECT_REPORT_INTS, dtype=torch.int32, device=dev)
+    report = (ctypes.c_int32 * INSPECT_REPORT_INTS)()
     with _on_device(dev):
-        native.check(native.lib().scorch_hip_csr_inspect(n_rows, n_cols, crd.numel(), pos.data_ptr(),
-                                                         crd.data_ptr(), report.data_ptr(), _stream(dev)))
-    bad_rows, bad_cols, max_row, empty_rows, descents, runs = report.tolist()[:6]
+        native.check(native.lib().scorch_hip_csr_inspect_now(n_rows, n_cols, crd.numel(), pos.data_ptr(),
+                                                             crd.data_ptr(), report, _stream(dev)))
+    bad_rows, bad_cols, max_row, empty_rows, descents, runs = report[:6]
     if bad_rows or bad_cols:
         problems = []
         if bad_rows:
@@ -903,23 +905,26 @@ def _make_spgemm(dtype):
         L = native.lib()
         with _on_device(dev):
             stream = _stream(dev)
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("scorch_ops_hip: the size of a CSR x CSR product has to be read by the host; it cannot "
+                                   "be recorded in a graph")
             need = L.scorch_hip_spgemm_csr_workspace_bytes(M, N, a_val.element_size())
             ws = _workspace(dev, stream, need)
             c_pos = _empty(M + 1, dtype=torch.int32, device=dev)
-            native.check(L.scorch_hip_spgemm_csr_symbolic(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(),
-                                                          b_pos.data_ptr(), b_crd.data_ptr(),
-                                                          c_pos.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                          stream))
-            nnz = int(c_pos[-1].item())
+            report = (ctypes.c_int64 * SPGEMM_REPORT_WORDS)()
+            native.check(L.scorch_hip_spgemm_csr_symbolic_planned(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(),
+                                                                  b_pos.data_ptr(), b_crd.data_ptr(), c_pos.data_ptr(),
+                                                                  ws.data_ptr(), ws.numel(), report, stream))
+            nnz = report[0]
             if nnz < 0:
                 raise native.ScorchHipError(native.EUNSUPPORTED,
                                             "SpGEMM: the result has 2^31 entries or more, beyond its int32 row pointer")
             c_crd = _empty(nnz, dtype=torch.int32, device=dev)
             c_val = _empty(nnz, dtype=dtype, device=dev)
-            fn = getattr(L, "scorch_hip_spgemm_csr_numeric_" + _SUFFIX[dtype])
+            fn = getattr(L, "scorch_hip_spgemm_csr_numeric_planned_" + _SUFFIX[dtype])
             native.check(fn(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(),
                             b_pos.data_ptr(), b_crd.data_ptr(), b_val.data_ptr(), c_pos.data_ptr(),
-                            c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), stream))
+                            c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), report, stream))
         return Tensor(c_val, [[], [c_pos, c_crd]])
     return kernel
 

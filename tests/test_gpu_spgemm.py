@@ -389,3 +389,50 @@ def test_reproducible_mode_gives_the_same_bits_on_every_run(oracle, monkeypatch)
                                [3, 3], [[], [dev(np.array([0, 1, 2, 3], np.int32)), dev(np.array([1, 2, 0], np.int32))]],
                                dev(np.array([4.0, 0.25, -1.0], np.float32)))
     assert host(small.storage.value).tolist() == [-0.5, -8.0, 0.75]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("N", [4095, 4096, 32_769, 131_073, 524_288, 524_289])
+def test_hub_rows_shared_out_among_workgroups(oracle, dtype, N):
+    """Rows of far more products than the rest -- a hub of many short B rows, one of few long ones, one
+    whose products meet in few columns -- at the widths where their treatment changes, between
+    rows of every other size."""
+    rng = np.random.default_rng(N)
+    M, K = 70, 3000
+    blens = rng.integers(0, 40, K)
+    blens[:4] = [min(N, 40_000), min(N, 9000), 0, 1]
+    brp = np.concatenate([[0], np.cumsum(blens)]).astype(np.int32)
+    bci = np.concatenate([np.sort(rng.choice(N if j % 3 else min(N, 700), n, replace=False)) if n <= 700 or j % 3
+                          else np.sort(rng.choice(N, n, replace=False)) for j, n in enumerate(blens) if n]).astype(np.int32)
+    alens = rng.integers(0, 12, M)
+    alens[5], alens[6], alens[7], alens[40] = K, 4, 900, 1500
+    rows = [np.sort(rng.choice(K, n, replace=False)) for n in alens]
+    rows[6] = np.array([0, 1, 2, 3])
+    rows[7] = np.arange(0, 2700, 3)                        # B rows over the first 700 columns
+    aci = np.concatenate(rows).astype(np.int32)
+    arp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    value = (lambda n: rng.integers(-9, 9, n).astype(dtype)) if np.issubdtype(dtype, np.integer) else \
+        (lambda n: rng.uniform(-1, 1, n).astype(dtype))
+    check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
+    if dtype in (np.float32, np.int64):                    # the two calls of the stable header, which share nothing
+        from scorch_amd import native
+        L, t = native.lib(), {np.float32: ("f32", torch.float32), np.int64: ("i64", torch.int64)}[dtype]
+        ap, ac, av, bp, bc, bv = (dev(x) for x in (arp, aci, value(aci.size), brp, bci, value(bci.size)))
+        ws = torch.full((L.scorch_hip_spgemm_csr_workspace_bytes(M, N, 8),), 0x7F, dtype=torch.uint8, device="cuda")
+        c_pos = torch.empty(M + 1, dtype=torch.int32, device="cuda")
+        native.check(L.scorch_hip_spgemm_csr_symbolic(M, K, N, ap.data_ptr(), ac.data_ptr(), bp.data_ptr(), bc.data_ptr(),
+                                                      c_pos.data_ptr(), ws.data_ptr(), ws.numel(), None))
+        nnz = int(c_pos[-1])
+        ws.fill_(0x7F)
+        c_crd = torch.full((nnz,), -1, dtype=torch.int32, device="cuda")
+        c_val = torch.zeros(nnz, dtype=t[1], device="cuda")
+        native.check(getattr(L, "scorch_hip_spgemm_csr_numeric_" + t[0])(
+            M, K, N, ap.data_ptr(), ac.data_ptr(), av.data_ptr(), bp.data_ptr(), bc.data_ptr(), bv.data_ptr(),
+            c_pos.data_ptr(), c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), None))
+        wrp, wci, wv = oracle.spgemm_csr_typed(arp, aci, host(av), brp, bci, host(bv), N)
+        assert np.array_equal(host(c_pos), wrp) and np.array_equal(host(c_crd), wci)
+        if dtype == np.int64:
+            assert np.array_equal(host(c_val), wv)
+        else:
+            assert oracle.rel_fro(host(c_val), oracle.spgemm_csr_typed(arp, aci, host(av).astype(np.float64), brp, bci,
+                                                                       host(bv).astype(np.float64), N)[2]) <= 1e-5
