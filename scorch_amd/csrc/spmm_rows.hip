@@ -182,7 +182,16 @@ int spmm_rows_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz
   while (vec > 1 && !(N % vec == 0 && aligned_to(B, sizeof(T) * vec) && aligned_to(C, sizeof(T) * vec)))
     vec /= 2;
   // lanes that cover a row of B (at most a wavefront: wider rows take several column tiles)
-  const int64_t lanes = (N + vec - 1) / vec;
+  int64_t lanes = (N + vec - 1) / vec;
+  if (lanes > kWaveSize) lanes = kWaveSize;
+  // Few rows of many entries (a weight matrix: 1024 rows of 205, N = 256) are too few wavefronts at a
+  // wavefront per row and tile of 64 lanes: narrower tiles, down to the 128 bytes of a cache
+  // line, and more lane groups to a row, until they fill half of the chip's 8192 slots (31.8 -> 13 us;
+  // 512 rows: 30 -> 8; beyond half a narrower tile costs: 4096 rows of 41, N = 64 5.5 -> 6.0).
+  const int64_t mean = (nnz + M - 1) / M;
+  while (lanes > 8 && lanes * vec * (int64_t)sizeof(T) > 128 && mean >= 2 * kRowsBatch &&
+         M * ((N + lanes * vec - 1) / (lanes * vec)) < 4096)
+    lanes = lanes > 32 ? 32 : lanes > 16 ? 16 : 8;
 #define SCORCH_ROWS(VEC, LPR) \
   return launch_spmm_rows<T, VEC, LPR>(m, n, nnz, row_ptr, col_idx, vals, B, bias, relu, C, s, (int)batch, K)
 #define SCORCH_ROWS_LANES(VEC)              \
