@@ -420,6 +420,10 @@ SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_i64(int64_t M, int64_t 
                                    int32_t *c_col_idx, int64_t *c_vals, void *workspace, size_t workspace_bytes,
                                    const int64_t *report, void *stream);
 
+/* B (K, N) row by row from its transpose X, an (N, K) array: what a product with a transposed view
+ * needs first. */
+SCORCH_HIP_API int scorch_hip_dense_to_rows_f32(int64_t K, int64_t N, const float *X, float *B, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

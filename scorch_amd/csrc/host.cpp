@@ -171,12 +171,14 @@ Operand *operand_of(PyObject *a) {
   return o;
 }
 
-// A tensor argument that a kernel can read as it is.
-bool fits(PyObject *obj, const Operand *o, int64_t dims, at::ScalarType dtype) {
+// A tensor argument that a kernel can read as it is (or, `transposed`: that is the transpose of one).
+bool fits(PyObject *obj, const Operand *o, int64_t dims, at::ScalarType dtype, bool transposed = false) {
   if (!THPVariable_CheckExact(obj)) return false;
   const at::Tensor &t = THPVariable_Unpack(obj);
   return t.layout() == at::kStrided && t.is_cuda() && t.get_device() == o->device && t.scalar_type() == dtype &&
-         t.dim() == dims && t.is_contiguous() && !t.is_neg();
+         t.dim() == dims && !t.is_neg() &&
+         (transposed ? dims == 2 && t.stride(0) == 1 && t.stride(1) == t.size(0) && t.size(0) > 1 && t.size(1) > 1
+                     : t.is_contiguous());
 }
 
 // Memory for a result, from torch's allocator -- through the module's own name for it when somebody
@@ -275,7 +277,9 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!o || !THPVariable_CheckExact(b)) return none();
   const at::Tensor &bt = THPVariable_Unpack(b);
   const int64_t dims = bt.dim();
-  if (dims < 1 || dims > 2 || !fits(b, o, dims, o->dtype) || bt.size(0) != o->cols) return none();
+  if (dims < 1 || dims > 2 || bt.size(0) != o->cols) return none();
+  const bool transposed = !bt.is_contiguous();
+  if (!fits(b, o, dims, o->dtype, transposed) || (transposed && o->dtype != at::kFloat)) return none();
   const int64_t N = dims == 2 ? bt.size(1) : -1;
   Route *r = find_route(o, N, act);
   if (!r || r->spmm_path != item(g_ops, n_spmm_path) || r->other_path != item(g_ops, n_blocked_path)) return none();
@@ -297,6 +301,7 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (r->workspace || r->may_tile) {
     if (capturing(stream)) return none();
     if (r->may_tile) {
+      if (transposed) return none();
       if (tiles_switched_off()) return none();
       tiles = tile_copy(b, o->cols, N);
       if (!tiles) return none();  // the general path counts the product and may make the copy
@@ -307,8 +312,15 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const int64_t M = o->rows, K = o->cols, nnz = o->second.numel;
   const bool got = N >= 0 ? allocate(out, {M, N}, o->dtype, o->device, bt) : allocate(out, {M}, o->dtype, o->device, bt);
   if (!got) return nullptr;
+  at::Tensor by_rows;  // (its memory goes back to torch's allocator for this stream when the call returns)
+  if (transposed) {
+    if (!allocate(by_rows, {K, N}, o->dtype, o->device, bt)) return nullptr;
+    const int rc = scorch_hip_dense_to_rows_f32(K, N, at_<float>(bt.const_data_ptr()),
+                                                static_cast<float *>(by_rows.mutable_data_ptr()), stream);
+    if (rc != SCORCH_HIP_OK) return finished(rc, out);
+  }
   const int32_t *pos = at_<int32_t>(r->row_ptr ? r->row_ptr : o->first.data), *crd = at_<int32_t>(o->second.data);
-  const void *v = vt.const_data_ptr(), *B = bt.const_data_ptr();
+  const void *v = vt.const_data_ptr(), *B = transposed ? by_rows.const_data_ptr() : bt.const_data_ptr();
   void *C = out.mutable_data_ptr();
   const int flag = act == 2 ? 1 : 0;
   int rc = SCORCH_HIP_EINVAL;

@@ -189,7 +189,7 @@ def _matmul_csr_dense_direct(a: STensor, b: torch.Tensor, kwargs) -> Optional[to
     result = _timed(lambda: fn(result_shape, a.shape, a.index.mode_indices, a.values,
                                tuple(b.shape), [[] for _ in range(b.dim())], values),
                     a.values.device, kwargs.get("time_dict", None))
-    if values.data_ptr() == b.data_ptr():
+    if b.is_contiguous() or b.t().is_contiguous():
         scorch_ops_hip.remember_spmm(a, b.shape[1] if b.dim() == 2 else -1)
     return result.storage.value.view(result_shape)
 
