@@ -52,22 +52,22 @@ CONFIG_WORKLOADS = ("spmm_uniform", "sddmm_uniform", "attention_blocksparse", "s
 _CSRC = "scorch_amd/csrc/"
 _SPMM_SOURCES = (_CSRC + "spmm.hip", _CSRC + "spmm.hpp", _CSRC + "common.hpp")
 MEASURED_TRAFFIC = {
-    ("gcn_powerlaw", "merge"): {"bytes": 9_790_300_000, "sources": _SPMM_SOURCES, "sha16": "f03cdf8f7d11457c",
+    ("gcn_powerlaw", "merge"): {"bytes": 9_790_300_000, "sources": _SPMM_SOURCES, "sha16": "",
                                 "profile": "profiles/spmm_merge_kernel_gcn_powerlaw.md"},
     ("spmm_uniform", "rows"): {"bytes": 10_830_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp",
                                                                 _CSRC + "common.hpp"), "sha16": "",
                                "profile": "profiles/spmm_rows_kernel_uniform_4096.md"},
     ("sae_decoder", "tiled"): {"bytes": 344_100_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp",
-                                                                 _CSRC + "common.hpp"), "sha16": "ea9b5c43570e7930",
+                                                                 _CSRC + "common.hpp"), "sha16": "",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
-    ("sae_decoder", "merge"): {"bytes": 1_767_900_000, "sources": _SPMM_SOURCES, "sha16": "f03cdf8f7d11457c",
+    ("sae_decoder", "merge"): {"bytes": 1_767_900_000, "sources": _SPMM_SOURCES, "sha16": "",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
     ("sddmm_uniform", "listed"): {"bytes": 278_000_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
-                                  "sha16": "eed3747508604c18", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
+                                  "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
     ("sddmm_uniform", "plain"): {"bytes": 848_200_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
-                                 "sha16": "eed3747508604c18", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
+                                 "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
     ("attention_blocksparse", "fused"): {"bytes": 81_050_000, "sources": (_CSRC + "attn.hip", _CSRC + "common.hpp"),
-                                         "sha16": "1c42d31b5c08e253", "profile": "profiles/attn_blocksparse_kernel_s8192_h16.md"},
+                                         "sha16": "", "profile": "profiles/attn_blocksparse_kernel_s8192_h16.md"},
 }
 
 

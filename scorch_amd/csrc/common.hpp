@@ -94,6 +94,23 @@ template <> struct Acc<int64_t> { using type = uint64_t; };
 // ---- device helpers ---------------------------------------------------------
 template <typename T, int V> struct alignas(sizeof(T) * V) Vec { T v[V]; };
 
+// V elements at any address aligned to one element, moved by one instruction all the same (global
+// memory takes 16-byte accesses at 4-byte alignment): rows of an odd number of elements start
+// anywhere.
+template <typename T, int V>
+__device__ __forceinline__ Vec<T, V> load_vec(const T *p) {
+  typedef T Native __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+  typedef T Aligned __attribute__((ext_vector_type(V)));
+  const Aligned x = *reinterpret_cast<const Native *>(p);
+  return __builtin_bit_cast(Vec<T, V>, x);
+}
+template <typename T, int V>
+__device__ __forceinline__ void store_vec(T *p, const Vec<T, V> &x) {
+  typedef T Native __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+  typedef T Aligned __attribute__((ext_vector_type(V)));
+  *reinterpret_cast<Native *>(p) = __builtin_bit_cast(Aligned, x);
+}
+
 // Sum over the GS lanes of a group (GS a power of two, groups aligned), every lane receiving the
 // total, with the pairing x(i) + x(i ^ off) for off = GS / 2 down to 1.  Within a row of 16 lanes
 // the exchanges are row rotations carried by the add itself (DPP): once the steps above have made
@@ -128,8 +145,10 @@ __device__ __forceinline__ void store_streaming(T *p, T x) {
 }
 template <typename T, int V>
 __device__ __forceinline__ void store_streaming(T *p, const Vec<T, V> &x) {
-  typedef T Native __attribute__((ext_vector_type(V)));
-  __builtin_nontemporal_store(__builtin_bit_cast(Native, x), reinterpret_cast<Native *>(p));
+  typedef T Native __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+  typedef T Aligned __attribute__((ext_vector_type(V)));
+  const Native n = __builtin_bit_cast(Aligned, x);
+  __builtin_nontemporal_store(n, reinterpret_cast<Native *>(p));
 }
 
 __device__ __forceinline__ int wave_lane() { return threadIdx.x & (kWaveSize - 1); }

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
   const int w = threadIdx.x / kWaveSize;
   const TileMap where = map_workgroup(blockIdx.x, n_tiles, blocks_per_tile);
   const int64_t chunk = where.block * kWavesPerBlock + w;
-  const int col0 = (where.tile * kWaveSize + lane) * VEC;
+  const int col0 = lane_column<VEC>((where.tile * kWaveSize + lane) * VEC, N);
   const bool active = col0 < N;
 
   const int64_t d0 = chunk * items_per_chunk;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
     const int j = uniform(s_col[w][k]);
     VecT b;
     if (active) {
-      b = *reinterpret_cast<const VecT *>(B + (size_t)j * (size_t)N + col0);
+      b = load_vec<T, VEC>(B + (size_t)j * (size_t)N + col0);
     } else {
 #pragma unroll
       for (int v = 0; v < VEC; ++v) b.v[v] = (T)0;
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
     VecT o;
 #pragma unroll
     for (int v = 0; v < VEC; ++v) o.v[v] = (T)acc[v];
-    *reinterpret_cast<VecT *>(carry_val + (size_t)chunk * (size_t)N + col0) = o;
+    store_vec<T, VEC>(carry_val + (size_t)chunk * (size_t)N + col0, o);
   }
 }
 
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
   const int t = lane % LPR;
   const TileMap where = map_workgroup(blockIdx.x, n_tiles, blocks_per_tile);
   const int64_t span = where.block * kWavesPerBlock + w;
-  const int col0 = (where.tile * LPR + t) * VEC;
+  const int col0 = lane_column<VEC>((where.tile * LPR + t) * VEC, N);
   const bool active = col0 < N;
 
   const int64_t d0 = span * items_per_chunk;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
 
   auto add_entry = [&](A (&acc)[VEC], int k) {
     const A a = (A)s_val[w][k];
-    const VecT b = *reinterpret_cast<const VecT *>(B + (size_t)s_col[w][k] * (size_t)N + col0);
+    const VecT b = load_vec<T, VEC>(B + (size_t)s_col[w][k] * (size_t)N + col0);
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] += a * (A)b.v[v];
   };
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           a[u] = (A)s_val[w][k + u];
-          b[u] = *reinterpret_cast<const VecT *>(B + (size_t)s_col[w][k + u] * (size_t)N + col0);
+          b[u] = load_vec<T, VEC>(B + (size_t)s_col[w][k + u] * (size_t)N + col0);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
       } else if (len > 0) {
 #pragma unroll
         for (int v = 0; v < VEC; ++v) o.v[v] = (T)acc[v];
-        *reinterpret_cast<VecT *>(carry_val + (size_t)span * (size_t)N + col0) = o;
+        store_vec<T, VEC>(carry_val + (size_t)span * (size_t)N + col0, o);
       }
     }
     if (live && slot == n_rows && where.tile == 0 && t == 0 && blockIdx.y == 0) carry_row[span] = len > 0 ? x1 : -1;
@@ -409,8 +409,11 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
   if (timer) SCORCH_HIP_CHECK(hipEventRecord(timer->ev[1], stream));
   mark_launch(stream);
   const int64_t fix_per_block = kWavesPerBlock * kFixupChunks;
-  spmm_fixup_kernel<T, VEC, EPI><<<dim3((unsigned)((chunks + fix_per_block - 1) / fix_per_block), (unsigned)batch),
-                                   kBlockThreads, 0, stream>>>(N, chunks, carry_row, carry_val, C, bias, strides);
+  // (the fix-up adds to C where it stands: no column may be two lanes')
+  const bool whole = N % VEC == 0 && aligned_to(C, sizeof(T) * VEC) && aligned_to(carry_val, sizeof(T) * VEC);
+  auto fixup = whole ? &spmm_fixup_kernel<T, VEC, EPI> : &spmm_fixup_kernel<T, 1, EPI>;
+  fixup<<<dim3((unsigned)((chunks + fix_per_block - 1) / fix_per_block), (unsigned)batch), kBlockThreads, 0, stream>>>(
+      N, chunks, carry_row, carry_val, C, bias, strides);
   SCORCH_HIP_CHECK(hipGetLastError());
   if (timer) SCORCH_HIP_CHECK(hipEventRecord(timer->ev[2], stream));
   mark_launch(stream);
@@ -512,32 +515,25 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int m = (int)M, n = (int)N;
   if (const int tile_bytes = timer ? 0 : narrow_tile_bytes(K, N, nnz, sizeof(T))) {
-    // widest vector (at most 16 bytes) that divides N and is aligned; lanes to cover the tile
-    constexpr int kMaxVec = (int)(16 / sizeof(T));
-    int vec = kMaxVec;
-    while (vec > 1 && !(N % vec == 0 && aligned_to(B, sizeof(T) * vec) && aligned_to(C, sizeof(T) * vec)))
-      vec /= 2;
-    const int64_t tile_elems = tile_bytes / (int)sizeof(T) < N ? tile_bytes / (int)sizeof(T) : N;
-    const int64_t lanes = (tile_elems + vec - 1) / vec;
+    const int vec = narrow_vec<T>(N);
+    const int64_t lanes = (tile_bytes / (int)sizeof(T) + vec - 1) / vec;  // at most 16: 256 bytes in vectors of 16
 #define SCORCH_GROUPED(VEC, LPR) \
   return launch_spmm_grouped<T, VEC, LPR, EPI>(m, n, nnz, row_ptr, col_idx, vals, B, bias, C, workspace, s, bounds, \
                                                (int)batch, K)
-#define SCORCH_GROUPED_LANES(VEC)                      \
-  do {                                                 \
-    if (lanes <= 8) SCORCH_GROUPED(VEC, 8);            \
-    if (lanes <= 16) SCORCH_GROUPED(VEC, 16);          \
-    if (lanes <= 32) SCORCH_GROUPED(VEC, 32);          \
-  } while (0)
-    if constexpr (sizeof(T) == 4) {
-      if (vec == 4) SCORCH_GROUPED_LANES(4);
+    constexpr int kMaxVec = (int)(16 / sizeof(T));
+    if (vec == kMaxVec) {
+      if (lanes <= 2) SCORCH_GROUPED(kMaxVec, 2);
+      if (lanes <= 4) SCORCH_GROUPED(kMaxVec, 4);
+      if (lanes <= 8) SCORCH_GROUPED(kMaxVec, 8);
+      SCORCH_GROUPED(kMaxVec, 16);
     }
-    if (vec == 2) SCORCH_GROUPED_LANES(2);
-    if (vec == 1) SCORCH_GROUPED_LANES(1);
-#undef SCORCH_GROUPED_LANES
+    if constexpr (kMaxVec > 2) {
+      if (vec == 2) SCORCH_GROUPED(2, 2);
+    }
+    SCORCH_GROUPED(1, 2);
 #undef SCORCH_GROUPED
-    // more than 32 lanes needed (odd N with scalar lanes): the wide kernel handles it
   }
-  const int vec = pick_vec<T>(N, B, C, workspace);
+  const int vec = pick_vec<T>(N);
   if constexpr (sizeof(T) == 4) {
     if (vec == 4)
       return launch_spmm<T, 4, EPI>(m, n, nnz, row_ptr, col_idx, vals, B, bias, C, workspace, s, timer, bounds,

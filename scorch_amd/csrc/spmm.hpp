@@ -151,21 +151,36 @@ inline size_t spmm_batched_workspace_bytes(int64_t batch, int64_t M, int64_t nnz
   return align_up(chunks * sizeof(int), 256) + align_up((size_t)batch * chunks * (size_t)N * elem, 256);
 }
 
-// Elements per lane.  Preferred: the widest vector (at most 16 bytes) that
-// divides N, is aligned and still keeps all 64 lanes busy (64 * VEC <= N).
-// Narrow N: the narrowest vector that covers N with one column tile.
+// Elements per lane.  Rows of B and C need no alignment beyond their elements' (load_vec), and N
+// need not be a multiple of the vector: the last lane of a row takes its last VEC columns, some of
+// which its neighbour computes as well, to the same bits.  (An odd N with one element per lane
+// took longer: a product with N = 37 on 50,021 nodes 43 -> 37 us, N = 15 on 100,000 27 -> 19.)  A full wavefront per row: the widest
+// vector (at most 16 bytes) that keeps all 64 lanes busy (64 * VEC <= N), else the narrowest that
+// covers N with one column tile.
 template <typename T>
-int pick_vec(int64_t N, const void *B, const void *C, const void *ws) {
+int pick_vec(int64_t N) {
   constexpr int kMaxVec = (int)(16 / sizeof(T));
-  auto usable = [&](int vec) {
-    const size_t bytes = sizeof(T) * vec;
-    return N % vec == 0 && aligned_to(B, bytes) && aligned_to(C, bytes) && aligned_to(ws, bytes);
-  };
   for (int vec = kMaxVec; vec > 1; vec /= 2)
-    if (usable(vec) && (int64_t)kWaveSize * vec <= N) return vec;
+    if ((int64_t)kWaveSize * vec <= N) return vec;
   for (int vec = 2; vec <= kMaxVec; vec *= 2)
-    if (usable(vec) && (int64_t)kWaveSize * vec >= N && (int64_t)kWaveSize * (vec / 2) < N) return vec;
+    if (vec <= N && (int64_t)kWaveSize * vec >= N && (int64_t)kWaveSize * (vec / 2) < N) return vec;
   return 1;
+}
+
+// A lane group per row: the widest vector not wider than the row, and the lanes (a power of two,
+// two at least) that cover it.
+template <typename T>
+int narrow_vec(int64_t N) {
+  int vec = (int)(16 / sizeof(T));
+  while (vec > 1 && vec > N) vec /= 2;
+  return vec;
+}
+
+// First column of a lane: its place in the row, moved back where the vector would pass the end.
+// (>= N: the lane has nothing to do.)
+template <int VEC>
+__device__ __forceinline__ int lane_column(int col, int N) {
+  return col < N && col + VEC > N ? N - VEC : col;
 }
 
 // End of the run of equal carry rows that starts at `start` (a member): a 64-way

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_rows_kernel(
   const int64_t row64 = (where.block * kWavesPerBlock + w) * rows_per_wave + member;
   const bool live = row64 < M;
   const int row = live ? (int)row64 : 0;
-  const int col0 = (where.tile * LPR + t) * VEC;
+  const int col0 = lane_column<VEC>((where.tile * LPR + t) * VEC, N);
   const bool active = col0 < N;
 
   int begin = 0, end = 0;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_rows_kernel(
     for (int u = 0; u < kRowsBatch; ++u) {
       av[u] = (A)a[u];
       if (c[u] >= 0 && active) {
-        b[u] = *reinterpret_cast<const VecT *>(B + (size_t)c[u] * (size_t)N + col0);
+        b[u] = load_vec<T, VEC>(B + (size_t)c[u] * (size_t)N + col0);
       } else {
 #pragma unroll
         for (int v = 0; v < VEC; ++v) b[u].v[v] = (T)0;
@@ -176,11 +176,8 @@ int spmm_rows_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz
   const int m = (int)M, n = (int)N;
   const int relu = act == SCORCH_HIP_ACT_RELU;
 
-  // widest vector (at most 16 bytes) that divides N and is aligned
   constexpr int kMaxVec = (int)(16 / sizeof(T));
-  int vec = kMaxVec;
-  while (vec > 1 && !(N % vec == 0 && aligned_to(B, sizeof(T) * vec) && aligned_to(C, sizeof(T) * vec)))
-    vec /= 2;
+  const int vec = narrow_vec<T>(N);
   // lanes that cover a row of B (at most a wavefront: wider rows take several column tiles)
   int64_t lanes = (N + vec - 1) / vec;
   if (lanes > kWaveSize) lanes = kWaveSize;
@@ -196,16 +193,18 @@ int spmm_rows_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz
   return launch_spmm_rows<T, VEC, LPR>(m, n, nnz, row_ptr, col_idx, vals, B, bias, relu, C, s, (int)batch, K)
 #define SCORCH_ROWS_LANES(VEC)              \
   do {                                      \
+    if (lanes <= 2) SCORCH_ROWS(VEC, 2);    \
+    if (lanes <= 4) SCORCH_ROWS(VEC, 4);    \
     if (lanes <= 8) SCORCH_ROWS(VEC, 8);    \
     if (lanes <= 16) SCORCH_ROWS(VEC, 16);  \
     if (lanes <= 32) SCORCH_ROWS(VEC, 32);  \
     SCORCH_ROWS(VEC, 64);                   \
   } while (0)
-  if constexpr (sizeof(T) == 4) {
-    if (vec == 4) SCORCH_ROWS_LANES(4);
+  if (vec == kMaxVec) SCORCH_ROWS_LANES(kMaxVec);
+  if constexpr (kMaxVec > 2) {
+    if (vec == 2) SCORCH_ROWS(2, 2);
   }
-  if (vec == 2) SCORCH_ROWS_LANES(2);
-  SCORCH_ROWS_LANES(1);
+  SCORCH_ROWS(1, 2);
 #undef SCORCH_ROWS_LANES
 #undef SCORCH_ROWS
 }
