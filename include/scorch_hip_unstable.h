@@ -420,6 +420,32 @@ SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_i64(int64_t M, int64_t 
                                    int32_t *c_col_idx, int64_t *c_vals, void *workspace, size_t workspace_bytes,
                                    const int64_t *report, void *stream);
 
+/* ------------------------------------------------------------------------
+ * scorch_hip_spmm_csr_planned_<T> (and, in fp32, its batched form: `batch` products over one pattern,
+ * value arrays, B, C one after the other) in one launch: the chunks that share a row count
+ * themselves in `counters` and the last of them adds their parts up, the same bits as the second
+ * launch gives.  `counters` must hold scorch_hip_spmm_csr_planned_counters() int32 that are zero;
+ * they are zero again when the launch is done, and launches that may overlap must not share them.
+ * With fewer (n_counters = 0) the second launch is made.  workspace: as for _planned / _batched.
+ * ---------------------------------------------------------------------- */
+SCORCH_HIP_API int64_t scorch_hip_spmm_csr_planned_counters(int64_t batch, int64_t M, int64_t nnz, int64_t N, size_t elem_size);
+SCORCH_HIP_API int scorch_hip_spmm_csr_planned_counted_f32(
+    int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
+    const float *vals, const float *B, const float *bias, int act, float *C, const void *bounds, size_t bounds_bytes, void *workspace,
+    size_t workspace_bytes, int32_t *counters, int64_t n_counters, void *stream);
+SCORCH_HIP_API int scorch_hip_spmm_csr_planned_counted_f64(
+    int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
+    const double *vals, const double *B, const double *bias, int act, double *C, const void *bounds, size_t bounds_bytes, void *workspace,
+    size_t workspace_bytes, int32_t *counters, int64_t n_counters, void *stream);
+SCORCH_HIP_API int scorch_hip_spmm_csr_planned_counted_i32(
+    int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
+    const int32_t *vals, const int32_t *B, const int32_t *bias, int act, int32_t *C, const void *bounds, size_t bounds_bytes, void *workspace,
+    size_t workspace_bytes, int32_t *counters, int64_t n_counters, void *stream);
+SCORCH_HIP_API int scorch_hip_spmm_csr_planned_counted_i64(
+    int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
+    const int64_t *vals, const int64_t *B, const int64_t *bias, int act, int64_t *C, const void *bounds, size_t bounds_bytes, void *workspace,
+    size_t workspace_bytes, int32_t *counters, int64_t n_counters, void *stream);
+
 /* B (K, N) row by row from its transpose X, an (N, K) array: what a product with a transposed view
  * needs first. */
 SCORCH_HIP_API int scorch_hip_dense_to_rows_f32(int64_t K, int64_t N, const float *X, float *B, void *stream);

@@ -28,7 +28,7 @@ namespace {
 
 // ---- names and objects looked up once ---------------------------------------------------------
 PyObject *n_storage, *n_index, *n_value, *n_shape, *n_mode_indices, *n_format, *n_routes, *n_spmm_path, *n_blocked_path,
-    *n_sddmm_path, *n_empty, *n_workspaces, *n_tiled, *n_volatile, *n_epoch, *n_attention, *n_dtype, *n_device;
+    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_volatile, *n_epoch, *n_attention, *n_dtype, *n_device;
 PyObject *g_ops = nullptr;        // scorch_ops_hip's namespace
 PyObject *g_stensor = nullptr;    // the STensor type
 PyObject *g_torch_empty = nullptr;
@@ -210,10 +210,10 @@ bool capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// Scratch memory for (device, stream): the buffer the general path keeps, if it is there and large
+// Scratch memory for (device, stream), or another of the module's buffers per stream: the buffer the general path keeps, if it is there and large
 // enough; null otherwise (the general path then makes it).
-void *workspace(int device, hipStream_t stream, int64_t bytes, size_t *have) {
-  PyObject *all = item(g_ops, n_workspaces);
+void *workspace(int device, hipStream_t stream, int64_t count, size_t *have, PyObject *which = nullptr) {
+  PyObject *all = item(g_ops, which ? which : n_workspaces);
   if (!all || !PyDict_CheckExact(all)) return nullptr;
   PyObject *d = PyLong_FromLong(device), *s = PyLong_FromUnsignedLongLong(reinterpret_cast<unsigned long long>(stream));
   PyObject *key = PyTuple_Pack(2, d, s);
@@ -223,7 +223,7 @@ void *workspace(int device, hipStream_t stream, int64_t bytes, size_t *have) {
   Py_DECREF(key);
   if (!buf || !THPVariable_Check(buf)) return nullptr;
   const at::Tensor &t = THPVariable_Unpack(buf);
-  if (t.numel() < bytes) return nullptr;
+  if (t.numel() < count) return nullptr;
   *have = (size_t)t.numel();
   return t.mutable_data_ptr();
 }
@@ -295,8 +295,8 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
   }
   if (c10::hip::current_device() != o->device) return none();
   hipStream_t stream = c10::hip::getCurrentHIPStream(o->device).stream();
-  void *ws = nullptr;
-  size_t ws_bytes = 0;
+  void *ws = nullptr, *counters = nullptr;
+  size_t ws_bytes = 0, n_counted = 0;
   const at::Tensor *tiles = nullptr;
   if (r->workspace || r->may_tile) {
     if (capturing(stream)) return none();
@@ -307,6 +307,7 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
       if (!tiles) return none();  // the general path counts the product and may make the copy
     }
     if (r->workspace && !(ws = workspace(o->device, stream, r->workspace, &ws_bytes))) return none();
+    if (r->kind == kPlanned && !(counters = workspace(o->device, stream, r->p[3], &n_counted, n_counters))) return none();
   }
   at::Tensor out;
   const int64_t M = o->rows, K = o->cols, nnz = o->second.numel;
@@ -344,8 +345,9 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
 #undef SCORCH_CALL
   } else if (r->kind == kPlanned) {
 #define SCORCH_CALL(S, T)                                                                                             \
-  scorch_hip_spmm_csr_planned_##S(M, K, N, nnz, pos, crd, at_<T>(v), at_<T>(B), at_<T>(bias_ptr), flag | (int)r->p[1], \
-                                  static_cast<T *>(C), r->q[0], (size_t)r->p[0], ws, ws_bytes, stream)
+  scorch_hip_spmm_csr_planned_counted_##S(1, M, K, N, nnz, pos, crd, at_<T>(v), at_<T>(B), at_<T>(bias_ptr),          \
+                                          flag | (int)r->p[1], static_cast<T *>(C), r->q[0], (size_t)r->p[0], ws,     \
+                                          ws_bytes, static_cast<int32_t *>(counters), (int64_t)n_counted, stream)
     SCORCH_BY_TYPE(SCORCH_CALL)
 #undef SCORCH_CALL
   } else if (r->kind == kSpmv) {
@@ -669,7 +671,7 @@ PyMODINIT_FUNC PyInit__host() {
   } names[] = {{&n_storage, "_storage"}, {&n_index, "_index"}, {&n_value, "_value"}, {&n_shape, "_shape"},
                {&n_mode_indices, "mode_indices"}, {&n_format, "format"}, {&n_routes, "_routes"},
                {&n_spmm_path, "SPMM_PATH"}, {&n_blocked_path, "BLOCKED_PATH"}, {&n_sddmm_path, "SDDMM_PATH"},
-               {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_tiled, "_scorch_tiled"},
+               {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_counters, "_counter_buffers"}, {&n_tiled, "_scorch_tiled"},
                {&n_volatile, "_scorch_volatile"}, {&n_epoch, "_scorch_epoch"}, {&n_attention, "_scorch_attention"},
                {&n_dtype, "dtype"}, {&n_device, "device"}};
   for (const auto &x : names) *x.slot = PyUnicode_InternFromString(x.text);

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
     const T *__restrict__ vals, const T *__restrict__ B, T *__restrict__ C,
     const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int n_tiles,
     int64_t blocks_per_tile, int *__restrict__ carry_row, T *__restrict__ carry_val,
-    const Boundary *__restrict__ bounds, SpmmBatch batch, int zero_filled) {
+    const Boundary *__restrict__ bounds, SpmmBatch batch, int zero_filled, int *__restrict__ counters) {
   using A = typename Acc<T>::type;
   using VecT = Vec<T, VEC>;
   constexpr int kSlots = kItemsPerWave + kSnapItems;
@@ -114,7 +114,9 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
 #pragma unroll
       for (int v = 0; v < VEC; ++v)
         o.v[v] = partial ? (T)acc[v] : apply_epilogue<T, EPI>(acc[v], bias_v[v]);
-      store_streaming(C + (size_t)x * (size_t)N + col0, o);
+      T *dst = C + (size_t)x * (size_t)N + col0;
+      if (partial && counters) store_part<T, VEC>(dst, o);
+      else store_streaming(dst, o);
     }
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = (A)0;
@@ -157,12 +159,25 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
   // Whatever is left belongs to row x1, whose marker lies in a later chunk.
   const int row_start = uniform(s_rp[w][n_rows]);  // row_ptr[x1]
   const int tail = y1 - (row_start > y0 ? row_start : y0);
-  if (where.tile == 0 && lane == 0 && blockIdx.y == 0) carry_row[chunk] = tail > 0 ? x1 : -1;
+  if (!counters && where.tile == 0 && lane == 0 && blockIdx.y == 0) carry_row[chunk] = tail > 0 ? x1 : -1;
   if (tail > 0 && active) {
     VecT o;
 #pragma unroll
     for (int v = 0; v < VEC; ++v) o.v[v] = (T)acc[v];
-    store_vec<T, VEC>(carry_val + (size_t)chunk * (size_t)N + col0, o);
+    T *dst = carry_val + (size_t)chunk * (size_t)N + col0;
+    if (counters) store_part<T, VEC>(dst, o);
+    else store_vec<T, VEC>(dst, o);
+  }
+  if (counters) {
+    const int shift = __builtin_ctz(items_per_chunk);
+    const int64_t chunks = (total_items + items_per_chunk - 1) >> shift;
+    counters += 2 * ((int64_t)blockIdx.y * n_tiles + where.tile) * chunks;
+    auto finish = [&](int row, int begin, int end, bool carry) {
+      finish_part<T, VEC, EPI>(row, begin, end, chunk, carry, shift, snap, chunks, counters, N, col0, active, carry_val, C,
+                               bias_v);
+    };
+    if (carry_in && n_rows > 0) finish(x0, uniform(s_rp[w][0]), uniform(s_rp[w][1]), false);
+    if (tail > 0) finish(x1, row_start, uniform(s_rp[w][n_rows + 1]), true);
   }
 }
 
@@ -185,7 +200,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
     const T *__restrict__ vals, const T *__restrict__ B, T *__restrict__ C,
     const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int n_tiles,
     int64_t blocks_per_tile, int *__restrict__ carry_row, T *__restrict__ carry_val,
-    const Boundary *__restrict__ bounds, SpmmBatch batch) {
+    const Boundary *__restrict__ bounds, SpmmBatch batch, int *__restrict__ counters) {
   using A = typename Acc<T>::type;
   using VecT = Vec<T, VEC>;
   constexpr int G = kWaveSize / LPR;
@@ -301,14 +316,31 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
 #pragma unroll
         for (int v = 0; v < VEC; ++v)
           o.v[v] = partial ? (T)acc[v] : apply_epilogue<T, EPI>(acc[v], bias_v[v]);
-        store_streaming(C + (size_t)(x0 + slot) * (size_t)N + col0, o);
+        T *dst = C + (size_t)(x0 + slot) * (size_t)N + col0;
+        if (partial && counters) store_part<T, VEC>(dst, o);
+        else store_streaming(dst, o);
       } else if (len > 0) {
 #pragma unroll
         for (int v = 0; v < VEC; ++v) o.v[v] = (T)acc[v];
-        store_vec<T, VEC>(carry_val + (size_t)span * (size_t)N + col0, o);
+        T *dst = carry_val + (size_t)span * (size_t)N + col0;
+        if (counters) store_part<T, VEC>(dst, o);
+        else store_vec<T, VEC>(dst, o);
       }
     }
-    if (live && slot == n_rows && where.tile == 0 && t == 0 && blockIdx.y == 0) carry_row[span] = len > 0 ? x1 : -1;
+    if (!counters && live && slot == n_rows && where.tile == 0 && t == 0 && blockIdx.y == 0)
+      carry_row[span] = len > 0 ? x1 : -1;
+  }
+  if (counters) {
+    const int shift = __builtin_ctz(items_per_chunk);
+    const int64_t chunks = (total_items + items_per_chunk - 1) >> shift;
+    counters += 2 * ((int64_t)blockIdx.y * n_tiles + where.tile) * chunks;
+    auto finish = [&](int row, int begin, int end, bool carry) {
+      finish_part<T, VEC, EPI>(row, begin, end, span, carry, shift, snap, chunks, counters, N, col0, active && g == 0,
+                               carry_val, C, bias_v);
+    };
+    if (carry_in && n_rows > 0) finish(x0, uniform(s_rp[w][0]), uniform(s_rp[w][1]), false);
+    const int tail_begin = uniform(s_rp[w][n_rows]);
+    if (y1 > (tail_begin > y0 ? tail_begin : y0)) finish(x1, tail_begin, uniform(s_rp[w][n_rows + 1]), true);
   }
 }
 
@@ -375,7 +407,8 @@ struct KernelTimer {
 template <typename T, int VEC, int EPI>
 int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_idx, const T *vals,
                 const T *B, const T *bias, T *C, void *workspace, hipStream_t stream,
-                KernelTimer *timer, const Boundary *bounds, int batch, int64_t K, bool zero_fill = false) {
+                KernelTimer *timer, const Boundary *bounds, int batch, int64_t K, int *counters,
+                int64_t counters_given, bool zero_fill = false) {
   const SpmmSplit split = spmm_split(M, nnz, N, sizeof(T));
   const int64_t chunks = split.spans;
   const SpmmBatch strides = {nnz, K * N, (int64_t)M * N, chunks * N};
@@ -391,6 +424,7 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
     return fail(SCORCH_HIP_EUNSUPPORTED, "SpMM: %lld workgroups exceed the launch limit",
                 (long long)(blocks_per_tile * n_tiles));
   const dim3 grid((unsigned)(blocks_per_tile * n_tiles), (unsigned)batch);
+  if (counters_given < 2 * (int64_t)batch * n_tiles * chunks) counters = nullptr;  // the launch below folds the carries
   if (timer) SCORCH_HIP_CHECK(hipEventRecord(timer->ev[0], stream));
   mark_launch(stream);
   zero_fill = zero_fill && EPI == kEpiNone && aligned_to(C, 16) && ((int64_t)batch * M * N * (int64_t)sizeof(T)) % 16 == 0;
@@ -404,10 +438,11 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
   }
   spmm_merge_kernel<T, VEC, EPI><<<grid, kBlockThreads, 0, stream>>>(
       M, N, row_ptr, col_idx, vals, B, C, bias, (int64_t)M + nnz, split.items_per_chunk,
-      split.snap, n_tiles, blocks_per_tile, carry_row, carry_val, bounds, strides, zero_fill ? 1 : 0);
+      split.snap, n_tiles, blocks_per_tile, carry_row, carry_val, bounds, strides, zero_fill ? 1 : 0, counters);
   SCORCH_HIP_CHECK(hipGetLastError());
   if (timer) SCORCH_HIP_CHECK(hipEventRecord(timer->ev[1], stream));
   mark_launch(stream);
+  if (counters) return SCORCH_HIP_OK;
   const int64_t fix_per_block = kWavesPerBlock * kFixupChunks;
   // (the fix-up adds to C where it stands: no column may be two lanes')
   const bool whole = N % VEC == 0 && aligned_to(C, sizeof(T) * VEC) && aligned_to(carry_val, sizeof(T) * VEC);
@@ -426,7 +461,8 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
 template <typename T, int VEC, int LPR, int EPI>
 int launch_spmm_grouped(int M, int N, int64_t nnz, const int *row_ptr, const int *col_idx,
                         const T *vals, const T *B, const T *bias, T *C, void *workspace,
-                        hipStream_t stream, const Boundary *bounds, int batch, int64_t K) {
+                        hipStream_t stream, const Boundary *bounds, int batch, int64_t K, int *counters,
+                        int64_t counters_given) {
   const int64_t total = (int64_t)M + nnz;
   const int tile = LPR * VEC;
   const int n_tiles = (N + tile - 1) / tile;
@@ -453,12 +489,14 @@ int launch_spmm_grouped(int M, int N, int64_t nnz, const int *row_ptr, const int
                 (long long)(blocks_per_tile * n_tiles));
   mark_launch(stream);
   const SpmmBatch strides = {nnz, K * N, (int64_t)M * N, spans * N};
+  if (counters_given < 2 * (int64_t)batch * n_tiles * spans) counters = nullptr;  // the launch below folds the carries
   spmm_grouped_kernel<T, VEC, LPR, EPI><<<dim3((unsigned)(blocks_per_tile * n_tiles), (unsigned)batch), kBlockThreads,
                                           0, stream>>>(
       M, N, row_ptr, col_idx, vals, B, C, bias, total, ipc, ipc < kSnapItems ? ipc : kSnapItems, n_tiles,
-      blocks_per_tile, carry_row, carry_val, bounds, strides);
+      blocks_per_tile, carry_row, carry_val, bounds, strides, counters);
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(stream);
+  if (counters) return SCORCH_HIP_OK;
   const int64_t fix_per_block = kWavesPerBlock * kFixupChunks;
   spmm_fixup_kernel<T, 1, EPI><<<dim3((unsigned)((spans + fix_per_block - 1) / fix_per_block), (unsigned)batch),
                                  kBlockThreads, 0, stream>>>(N, spans, carry_row, carry_val, C, bias, strides);
@@ -483,7 +521,8 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
                const int32_t *col_idx, const T *vals, const T *B, const T *bias, T *C,
                void *workspace, size_t workspace_bytes, void *stream,
                KernelTimer *timer = nullptr, const void *bounds_buffer = nullptr, size_t bounds_bytes = 0,
-               int64_t batch = 1, bool mostly_empty_rows = false) {
+               int64_t batch = 1, bool mostly_empty_rows = false, int *counters = nullptr,
+               int64_t counters_given = 0) {
   if (batch < 0 || batch > 65535)
     return fail(SCORCH_HIP_EUNSUPPORTED, "%s: batch=%lld is outside [0, 65535]", fn, (long long)batch);
   if (batch == 0) return SCORCH_HIP_OK;
@@ -519,7 +558,7 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
     const int64_t lanes = (tile_bytes / (int)sizeof(T) + vec - 1) / vec;  // at most 16: 256 bytes in vectors of 16
 #define SCORCH_GROUPED(VEC, LPR) \
   return launch_spmm_grouped<T, VEC, LPR, EPI>(m, n, nnz, row_ptr, col_idx, vals, B, bias, C, workspace, s, bounds, \
-                                               (int)batch, K)
+                                               (int)batch, K, counters, counters_given)
     constexpr int kMaxVec = (int)(16 / sizeof(T));
     if (vec == kMaxVec) {
       if (lanes <= 2) SCORCH_GROUPED(kMaxVec, 2);
@@ -533,17 +572,17 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
     SCORCH_GROUPED(1, 2);
 #undef SCORCH_GROUPED
   }
-  const int vec = pick_vec<T>(N);
+  const int vec = pick_vec(N, sizeof(T));
   if constexpr (sizeof(T) == 4) {
     if (vec == 4)
       return launch_spmm<T, 4, EPI>(m, n, nnz, row_ptr, col_idx, vals, B, bias, C, workspace, s, timer, bounds,
-                                  (int)batch, K, mostly_empty_rows);
+                                  (int)batch, K, counters, counters_given, mostly_empty_rows);
   }
   if (vec == 2)
     return launch_spmm<T, 2, EPI>(m, n, nnz, row_ptr, col_idx, vals, B, bias, C, workspace, s, timer, bounds,
-                                  (int)batch, K, mostly_empty_rows);
+                                  (int)batch, K, counters, counters_given, mostly_empty_rows);
   return launch_spmm<T, 1, EPI>(m, n, nnz, row_ptr, col_idx, vals, B, bias, C, workspace, s, timer, bounds,
-                                  (int)batch, K, mostly_empty_rows);
+                                  (int)batch, K, counters, counters_given, mostly_empty_rows);
 }
 
 
@@ -952,6 +991,47 @@ SCORCH_DEFINE_SPMM_PLANNED(f32, float)
 SCORCH_DEFINE_SPMM_PLANNED(f64, double)
 SCORCH_DEFINE_SPMM_PLANNED(i32, int32_t)
 SCORCH_DEFINE_SPMM_PLANNED(i64, int64_t)
+
+#define SCORCH_DEFINE_SPMM_PLANNED_COUNTED(SUFFIX, T)                                                      \
+  int scorch_hip_spmm_csr_planned_counted_##SUFFIX(                                                         \
+      int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,                  \
+      const int32_t *col_idx, const T *vals, const T *B, const T *bias, int act, T *C, const void *bounds,  \
+      size_t bounds_bytes, void *workspace, size_t workspace_bytes, int32_t *counters, int64_t n_counters,  \
+      void *stream) {                                                                                       \
+    const char *fn = "scorch_hip_spmm_csr_planned_counted_" #SUFFIX;                                        \
+    const bool mostly_empty = (act & SCORCH_HIP_HINT_MOSTLY_EMPTY_ROWS) != 0;                               \
+    act &= ~SCORCH_HIP_HINT_MOSTLY_EMPTY_ROWS;                                                              \
+    SCORCH_REQUIRE(n_counters >= 0 && (n_counters == 0 || counters) && scorch::aligned_to(counters, 4),     \
+                   "%s: counters are NULL or misaligned", fn);                                              \
+    if (!bias && act == SCORCH_HIP_ACT_NONE)                                                                \
+      return scorch::spmm_entry<T, scorch::kEpiNone>(fn, M, K, N, nnz, row_ptr, col_idx, vals, B, nullptr,  \
+                                                     C, workspace, workspace_bytes, stream, nullptr,        \
+                                                     bounds, bounds_bytes, batch, mostly_empty, counters,   \
+                                                     n_counters);                                           \
+    if (bias && act == SCORCH_HIP_ACT_NONE)                                                                 \
+      return scorch::spmm_entry<T, scorch::kEpiBias>(fn, M, K, N, nnz, row_ptr, col_idx, vals, B, bias, C,  \
+                                                     workspace, workspace_bytes, stream, nullptr, bounds,   \
+                                                     bounds_bytes, batch, false, counters, n_counters);     \
+    if (bias && act == SCORCH_HIP_ACT_RELU)                                                                 \
+      return scorch::spmm_entry<T, scorch::kEpiBiasRelu>(fn, M, K, N, nnz, row_ptr, col_idx, vals, B, bias, \
+                                                         C, workspace, workspace_bytes, stream, nullptr,    \
+                                                         bounds, bounds_bytes, batch, false, counters,      \
+                                                         n_counters);                                       \
+    return scorch::fail(SCORCH_HIP_EINVAL, "%s: activation %d (with%s bias) is not supported", fn, act,     \
+                        bias ? "" : "out");                                                                 \
+  }
+
+SCORCH_DEFINE_SPMM_PLANNED_COUNTED(f32, float)
+SCORCH_DEFINE_SPMM_PLANNED_COUNTED(f64, double)
+SCORCH_DEFINE_SPMM_PLANNED_COUNTED(i32, int32_t)
+SCORCH_DEFINE_SPMM_PLANNED_COUNTED(i64, int64_t)
+
+int64_t scorch_hip_spmm_csr_planned_counters(int64_t batch, int64_t M, int64_t nnz, int64_t N, size_t elem_size) {
+  if (batch <= 0 || M < 0 || nnz < 0 || N <= 0 || elem_size == 0) return 0;
+  const int64_t columns = 64 * (int64_t)scorch::pick_vec(N, elem_size);
+  const int64_t tiles = N * (int64_t)elem_size <= 256 ? 1 : (N + columns - 1) / columns;
+  return 2 * batch * tiles * scorch::spmm_num_chunks(M, nnz, N, elem_size);
+}
 
 size_t scorch_hip_spmm_csr_batched_workspace_bytes(int64_t batch, int64_t M, int64_t nnz, int64_t N) {
   if (batch <= 0 || M < 0 || nnz < 0 || N < 0) return 0;

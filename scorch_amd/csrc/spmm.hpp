@@ -115,6 +115,127 @@ struct SpmmSplit {
   int64_t spans;   // chunks = wavefronts with work = carry records
 };
 
+// ---- rows cut by chunk boundaries, folded without a second launch -----------------------------
+// The chunks that share a row leave their parts (carry_val, and the chunk that ends the row its
+// part in C) and take a ticket from the row's counter; the one that takes the last adds the parts up
+// in the order spmm_fixup_kernel keeps: the same bits, one launch less (3 to 8 us of a product that
+// takes 7 to 20; 24 of 1,340 on the million-node graph).
+//   Counters are zero before a launch and after it: whoever takes a counter's last ticket clears it.  They live in memory of their own, one
+// buffer per stream, since launches that overlap must not share them.
+//   Parts and counters cross between XCDs, whose L2s are not coherent with each other: parts are
+// written and read with agent-scope accesses, which go past the L2, and a wavefront waits until
+// its own have been acknowledged before it takes its ticket.  (A release fence instead would make
+// the L2 write all of its dirty lines back, at every row.)
+struct RowSpan {
+  int first, last;  // chunks; the last one ends the row
+};
+// Row `row`'s chunks: nominal positions of its first entry and its end marker, the latter's chunk
+// corrected for a boundary inside the row that has moved past the marker (chunk_boundary).
+__device__ __forceinline__ RowSpan row_span(int row, int begin, int end, int shift, int snap) {
+  const int64_t p0 = (int64_t)begin + row, marker = (int64_t)end + row;
+  RowSpan s;
+  s.first = (int)(p0 >> shift);
+  s.last = (int)(marker >> shift);
+  const int64_t d = (int64_t)s.last << shift;
+  if (d > p0 && marker + 1 - d <= snap) --s.last;
+  return s;
+}
+
+// Whether this wavefront is the last of the row's to get here.  Its own parts are in memory when
+// its ticket is taken.
+__device__ __forceinline__ bool last_ticket(int *counter, int parts) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  int taken = 0;
+  if (wave_lane() == 0)
+    taken = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  taken = uniform(taken);
+  if (taken != parts - 1) return false;
+  if (wave_lane() == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+template <typename T, int VEC>
+__device__ __forceinline__ void store_part(T *p, const Vec<T, VEC> &x) {
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) __hip_atomic_store(p + v, x.v[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T, int VEC>
+__device__ __forceinline__ Vec<T, VEC> load_part(const T *p) {
+  Vec<T, VEC> x;
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) x.v[v] = __hip_atomic_load(p + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return x;
+}
+
+// The sum of the parts of chunks from, from + step, ... (count of them) in their order.  One lane, VEC columns.
+template <typename T, int VEC>
+__device__ __forceinline__ Vec<T, VEC> sum_parts(const T *__restrict__ carry_val, int N, int col0, int from, int step, int count) {
+  using A = typename Acc<T>::type;
+  A sum[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) sum[v] = (A)0;
+  constexpr int kBatch = 8;  // in flight
+  auto part_at = [&](int i) { return load_part<T, VEC>(carry_val + (size_t)(from + i * step) * (size_t)N + col0); };
+  int i = 0;
+  for (; i + kBatch <= count; i += kBatch) {
+    Vec<T, VEC> part[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) part[u] = part_at(i + u);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) sum[v] += (A)part[u].v[v];
+  }
+  for (; i < count; ++i) {
+    const Vec<T, VEC> part = part_at(i);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) sum[v] += (A)part.v[v];
+  }
+  Vec<T, VEC> o;
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) o.v[v] = (T)sum[v];
+  return o;
+}
+
+// A chunk's part of row `row` (entries [begin, end)) is in memory: take its ticket and, as the last, fold
+// the row into C.  carry: the part is chunk's carry; else what the row's last chunk has stored in C.
+// A row of more than kFoldGroup carries is folded in two levels -- groups of kFoldGroup consecutive carries,
+// then the groups' sums, kept where each group's first carry was -- so that a 50,000-entry row neither
+// queues up hundreds of chunks at one counter nor ends in one wavefront adding hundreds of parts (with
+// one level 100,000 nodes at N = 16 took 49 us, with a second launch 28).
+// counters: two per chunk, the groups' and the rows', each at the first chunk of its own.
+constexpr int kFoldGroup = 16;
+template <typename T, int VEC, int EPI>
+__device__ __forceinline__ void finish_part(int row, int begin, int end, int64_t chunk, bool carry, int shift, int snap,
+                                            int64_t n_chunks, int *__restrict__ counters, int N, int col0, bool folds,
+                                            T *__restrict__ carry_val, T *__restrict__ C, const T (&bias_v)[VEC]) {
+  using A = typename Acc<T>::type;
+  const RowSpan span = row_span(row, begin, end, shift, snap);
+  const int n = span.last - span.first;
+  int *const rows = counters + n_chunks;
+  int parts = n, step = 1;
+  if (n > kFoldGroup) {
+    parts = (n + kFoldGroup - 1) / kFoldGroup;
+    step = kFoldGroup;
+    if (carry) {
+      const int first = span.first + ((int)chunk - span.first) / kFoldGroup * kFoldGroup;
+      const int count = span.last - first < kFoldGroup ? span.last - first : kFoldGroup;
+      if (!last_ticket(counters + first, count)) return;
+      if (folds) {
+        const Vec<T, VEC> sum = sum_parts<T, VEC>(carry_val, N, col0, first, 1, count);
+        store_part<T, VEC>(carry_val + (size_t)first * (size_t)N + col0, sum);
+      }
+    }
+  }
+  if (!last_ticket(rows + span.first, parts + 1) || !folds) return;
+  T *dst = C + (size_t)row * (size_t)N + col0;
+  Vec<T, VEC> o = load_part<T, VEC>(dst);
+  const Vec<T, VEC> sum = sum_parts<T, VEC>(carry_val, N, col0, span.first, step, parts);
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) o.v[v] = apply_epilogue<T, EPI>((A)sum.v[v] + (A)o.v[v], bias_v[v]);
+  store_vec<T, VEC>(dst, o);
+}
+
 inline SpmmSplit spmm_split(int64_t M, int64_t nnz, int64_t N, size_t elem) {
   const int64_t total = M + nnz;
   SpmmSplit sp;
@@ -157,9 +278,8 @@ inline size_t spmm_batched_workspace_bytes(int64_t batch, int64_t M, int64_t nnz
 // took longer: a product with N = 37 on 50,021 nodes 43 -> 37 us, N = 15 on 100,000 27 -> 19.)  A full wavefront per row: the widest
 // vector (at most 16 bytes) that keeps all 64 lanes busy (64 * VEC <= N), else the narrowest that
 // covers N with one column tile.
-template <typename T>
-int pick_vec(int64_t N) {
-  constexpr int kMaxVec = (int)(16 / sizeof(T));
+inline int pick_vec(int64_t N, size_t elem) {
+  const int kMaxVec = (int)(16 / elem);
   for (int vec = kMaxVec; vec > 1; vec /= 2)
     if ((int64_t)kWaveSize * vec <= N) return vec;
   for (int vec = 2; vec <= kMaxVec; vec *= 2)
@@ -239,25 +359,42 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_fixup_kernel(
     for (int col0 = lane * VEC; col0 < N; col0 += kWaveSize * VEC) {
       VecT *dst = reinterpret_cast<VecT *>(C + (size_t)r * (size_t)N + col0);
       VecT o = *dst;  // issued before the carries so that both are in flight together
+      // groups of kFoldGroup carries, then the groups' sums: the order of finish_part
       A sum[VEC];
 #pragma unroll
       for (int v = 0; v < VEC; ++v) sum[v] = (A)0;
       int64_t e = start;
-      constexpr int kBatch = 32;  // loads in flight: a long row spans hundreds of chunks
+      constexpr int kBatch = 2 * kFoldGroup;  // loads in flight: a long row spans hundreds of chunks
       for (; e + kBatch <= end; e += kBatch) {
         VecT part[kBatch];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u)
           part[u] = *reinterpret_cast<const VecT *>(carry_val + (size_t)(e + u) * (size_t)N + col0);
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u)
+        for (int h = 0; h < kBatch; h += kFoldGroup) {
+          A group[VEC];
 #pragma unroll
-          for (int v = 0; v < VEC; ++v) sum[v] += (A)part[u].v[v];
+          for (int v = 0; v < VEC; ++v) group[v] = (A)0;
+#pragma unroll
+          for (int u = 0; u < kFoldGroup; ++u)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) group[v] += (A)part[h + u].v[v];
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) sum[v] += (A)(T)group[v];
+        }
       }
-      for (; e < end; ++e) {
-        const VecT part = *reinterpret_cast<const VecT *>(carry_val + (size_t)e * (size_t)N + col0);
+      while (e < end) {
+        A group[VEC];
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) sum[v] += (A)part.v[v];
+        for (int v = 0; v < VEC; ++v) group[v] = (A)0;
+        const int64_t stop = e + kFoldGroup < end ? e + kFoldGroup : end;
+        for (; e < stop; ++e) {
+          const VecT part = *reinterpret_cast<const VecT *>(carry_val + (size_t)e * (size_t)N + col0);
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) group[v] += (A)part.v[v];
+        }
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) sum[v] += (A)(T)group[v];
       }
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {

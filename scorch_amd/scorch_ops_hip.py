@@ -90,6 +90,23 @@ def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
     return buf
 
 
+_counter_buffers = {}
+
+
+def _counters(device: torch.device, stream: int, count: int):
+    """(pointer, number) of int32 counters for a launch on (device, stream) that are zero and left
+    zero: one buffer per stream, since launches that overlap must not share it.  None under stream
+    capture, where a buffer fresh from the graph's pool would have to be cleared by every replay."""
+    if count <= 0 or torch.cuda.is_current_stream_capturing():
+        return None, 0
+    key = (device.index, stream)
+    buf = _counter_buffers.get(key)
+    if buf is None or buf.numel() < count:
+        buf = torch.zeros(max(count, 1 << 14), dtype=torch.int32, device=device)
+        _counter_buffers[key] = buf
+    return buf.data_ptr(), buf.numel()
+
+
 def _device_of(*tensors: torch.Tensor) -> torch.device:
     dev = tensors[0].device
     if dev.type != "cuda":
@@ -822,10 +839,13 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
     if not may_tile and not fill_first and plan.max_row <= ROWS_KERNEL_MAX_ROW:
         remember(_ROUTE_ROWS)
         return
+    counters = L.scorch_hip_spmm_csr_planned_counters(1, M, nnz, width, elem)
     with _on_device(dev):
         bounds = _chunk_bounds(plan, pos, M, nnz, width, elem, L, _stream(dev))
+        if not may_tile:
+            _counters(dev, _stream(dev), counters)
     remember(_ROUTE_TILED if may_tile else _ROUTE_PLANNED,
-             (bounds.numel(), HINT_MOSTLY_EMPTY_ROWS if fill_first else 0, plan.max_row), (bounds,),
+             (bounds.numel(), HINT_MOSTLY_EMPTY_ROWS if fill_first else 0, plan.max_row, counters), (bounds,),
              L.scorch_hip_spmm_csr_workspace_bytes(M, nnz, width, elem), may_tile)
 
 
@@ -1482,11 +1502,11 @@ def spmm_csr_float_batched(A_shape, A_mode_indices, A_values: torch.Tensor, B: t
             ws = _workspace(dev, stream, L.scorch_hip_spmm_csr_batched_workspace_bytes(H, M, nnz, N))
             bounds = _chunk_bounds(plan, pos, M, nnz, N, 4, L, stream) \
                 if plan is not None and SPMM_PATH != "merge_unplanned" else None
-            rc = L.scorch_hip_spmm_csr_batched_f32(H, M, K, N, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(),
-                                                   b.data_ptr(), out.data_ptr(),
-                                                   bounds.data_ptr() if bounds is not None else None,
-                                                   bounds.numel() if bounds is not None else 0, ws.data_ptr(),
-                                                   ws.numel(), stream)
+            rc = L.scorch_hip_spmm_csr_planned_counted_f32(
+                H, M, K, N, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(), b.data_ptr(), None, 0, out.data_ptr(),
+                bounds.data_ptr() if bounds is not None else None, bounds.numel() if bounds is not None else 0,
+                ws.data_ptr(), ws.numel(), *_counters(dev, stream, L.scorch_hip_spmm_csr_planned_counters(H, M, nnz, N, 4)),
+                stream)
     native.check(rc)
     return out
 

@@ -126,3 +126,32 @@ def test_decided_attention_is_the_general_ways_bit_for_bit(dtype):
     rp.add_(0)                                                    # written to, if only with what it held
     assert native.host().attention(q, k, v, rp, ci, 0.2, f32) is None
     assert torch.equal(fn(q, k, v, rp, ci, 0.2), first)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("N", [1, 2, 3, 5, 16, 61, 65, 130, 300])
+@pytest.mark.parametrize("relu", [None, True])
+def test_rows_folded_in_one_launch_are_the_second_launchs_bit_for_bit(dtype, N, relu):
+    """The decided product lets the last of the chunks that share a row add their parts up; the general way
+    makes a second launch for it.  Rows that end at, just before and just after a chunk's boundary,
+    over two chunks and over hundreds; many launches one after the other on the same counters."""
+    if relu and dtype != np.float32:
+        pytest.skip("the fused epilogue is fp32")
+    rng = np.random.default_rng(N)
+    K = 500
+    lens = rng.integers(0, 9, 4000)
+    lens[[3, 700, 701, 2500, 3999]] = [20_000, 300, 31, 5000, 2000]
+    lens[1000:1040] = np.arange(225, 265)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    integer = np.issubdtype(dtype, np.integer)
+    ci = rng.integers(0, K, rp[-1]).astype(np.int32)
+    v = (rng.integers(-9, 9, rp[-1]) if integer else rng.uniform(-1, 1, rp[-1])).astype(dtype)
+    A = STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (lens.size, K))
+    b = dev((rng.integers(-9, 9, (K, N)) if integer else rng.standard_normal((K, N))).astype(dtype))
+    bias = torch.randn(N, device="cuda") if relu else None
+    general = (lambda: scorch.spmm_bias_act(A, b, bias, relu=True)) if relu else (lambda: scorch.matmul(A, b))
+    want = general()
+    for _ in range(20):
+        got = native.host().spmm(A, b, bias, 2 if relu else 0)
+        assert got is not None and torch.equal(got, want)
+    assert all(int(c.abs().sum()) == 0 for c in H._counter_buffers.values())
