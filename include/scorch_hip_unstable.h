@@ -446,6 +446,32 @@ SCORCH_HIP_API int scorch_hip_spmm_csr_planned_counted_i64(
     const int64_t *vals, const int64_t *B, const int64_t *bias, int act, int64_t *C, const void *bounds, size_t bounds_bytes, void *workspace,
     size_t workspace_bytes, int32_t *counters, int64_t n_counters, void *stream);
 
+/* ------------------------------------------------------------------------
+ * SpMV with its chunk boundaries computed once (scorch_hip_spmv_csr_bounds; NULL: searched for) and, with
+ * scorch_hip_spmv_csr_planned_counters() counters as above, in one launch (n_counters = 0: two).
+ * workspace: scorch_hip_spmv_csr_workspace_bytes.
+ * ---------------------------------------------------------------------- */
+SCORCH_HIP_API int64_t scorch_hip_spmv_csr_planned_counters(int64_t M, int64_t nnz);
+SCORCH_HIP_API size_t scorch_hip_spmv_csr_bounds_bytes(int64_t M, int64_t nnz);
+SCORCH_HIP_API int scorch_hip_spmv_csr_bounds(int64_t M, int64_t nnz, const int32_t *row_ptr, void *bounds, size_t bounds_bytes,
+                                   void *stream);
+SCORCH_HIP_API int scorch_hip_spmv_csr_planned_f32(
+    int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx, const float *vals, const float *x, float *y,
+    const void *bounds, size_t bounds_bytes, void *workspace, size_t workspace_bytes, int32_t *counters, int64_t n_counters,
+    void *stream);
+SCORCH_HIP_API int scorch_hip_spmv_csr_planned_f64(
+    int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx, const double *vals, const double *x, double *y,
+    const void *bounds, size_t bounds_bytes, void *workspace, size_t workspace_bytes, int32_t *counters, int64_t n_counters,
+    void *stream);
+SCORCH_HIP_API int scorch_hip_spmv_csr_planned_i32(
+    int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx, const int32_t *vals, const int32_t *x, int32_t *y,
+    const void *bounds, size_t bounds_bytes, void *workspace, size_t workspace_bytes, int32_t *counters, int64_t n_counters,
+    void *stream);
+SCORCH_HIP_API int scorch_hip_spmv_csr_planned_i64(
+    int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx, const int64_t *vals, const int64_t *x, int64_t *y,
+    const void *bounds, size_t bounds_bytes, void *workspace, size_t workspace_bytes, int32_t *counters, int64_t n_counters,
+    void *stream);
+
 /* B (K, N) row by row from its transpose X, an (N, K) array: what a product with a transposed view
  * needs first. */
 SCORCH_HIP_API int scorch_hip_dense_to_rows_f32(int64_t K, int64_t N, const float *X, float *B, void *stream);

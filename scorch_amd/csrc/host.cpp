@@ -307,7 +307,7 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
       if (!tiles) return none();  // the general path counts the product and may make the copy
     }
     if (r->workspace && !(ws = workspace(o->device, stream, r->workspace, &ws_bytes))) return none();
-    if (r->kind == kPlanned && !(counters = workspace(o->device, stream, r->p[3], &n_counted, n_counters))) return none();
+    if ((r->kind == kPlanned || r->kind == kSpmv) && !(counters = workspace(o->device, stream, r->p[3], &n_counted, n_counters))) return none();
   }
   at::Tensor out;
   const int64_t M = o->rows, K = o->cols, nnz = o->second.numel;
@@ -352,7 +352,9 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
 #undef SCORCH_CALL
   } else if (r->kind == kSpmv) {
 #define SCORCH_CALL(S, T)                                                                                     \
-  scorch_hip_spmv_csr_##S(M, K, nnz, pos, crd, at_<T>(v), at_<T>(B), static_cast<T *>(C), ws, ws_bytes, stream)
+  scorch_hip_spmv_csr_planned_##S(M, K, nnz, pos, crd, at_<T>(v), at_<T>(B), static_cast<T *>(C), r->q[0],             \
+                                  (size_t)r->p[0], ws, ws_bytes, static_cast<int32_t *>(counters), (int64_t)n_counted, \
+                                  stream)
     SCORCH_BY_TYPE(SCORCH_CALL)
 #undef SCORCH_CALL
   } else if (r->kind == kBlockedSpmm) {

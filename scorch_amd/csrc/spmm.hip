@@ -169,11 +169,10 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
     else store_vec<T, VEC>(dst, o);
   }
   if (counters) {
-    const int shift = __builtin_ctz(items_per_chunk);
-    const int64_t chunks = (total_items + items_per_chunk - 1) >> shift;
+    const int64_t chunks = (total_items + items_per_chunk - 1) >> __builtin_ctz(items_per_chunk);
     counters += 2 * ((int64_t)blockIdx.y * n_tiles + where.tile) * chunks;
     auto finish = [&](int row, int begin, int end, bool carry) {
-      finish_part<T, VEC, EPI>(row, begin, end, chunk, carry, shift, snap, chunks, counters, N, col0, active, carry_val, C,
+      finish_part<T, VEC, EPI>(row, begin, end, chunk, carry, items_per_chunk, snap, chunks, counters, N, col0, active, carry_val, C,
                                bias_v);
     };
     if (carry_in && n_rows > 0) finish(x0, uniform(s_rp[w][0]), uniform(s_rp[w][1]), false);
@@ -331,11 +330,10 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
       carry_row[span] = len > 0 ? x1 : -1;
   }
   if (counters) {
-    const int shift = __builtin_ctz(items_per_chunk);
-    const int64_t chunks = (total_items + items_per_chunk - 1) >> shift;
+    const int64_t chunks = (total_items + items_per_chunk - 1) >> __builtin_ctz(items_per_chunk);
     counters += 2 * ((int64_t)blockIdx.y * n_tiles + where.tile) * chunks;
     auto finish = [&](int row, int begin, int end, bool carry) {
-      finish_part<T, VEC, EPI>(row, begin, end, span, carry, shift, snap, chunks, counters, N, col0, active && g == 0,
+      finish_part<T, VEC, EPI>(row, begin, end, span, carry, items_per_chunk, snap, chunks, counters, N, col0, active && g == 0,
                                carry_val, C, bias_v);
     };
     if (carry_in && n_rows > 0) finish(x0, uniform(s_rp[w][0]), uniform(s_rp[w][1]), false);
@@ -593,8 +591,14 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
 // sums the products of the r-th row the chunk touches.  A row with many entries
 // in the chunk is summed by the whole wavefront instead (strided partial sums,
 // butterfly reduction).  The part of the last row that continues in the next
-// chunk becomes a carry, folded into y by spmv_fixup_kernel in a fixed order,
-// so results are bit-reproducible.
+// chunk becomes a carry, folded into y in a fixed order, so results are bit-reproducible: by the
+// last of the row's chunks (finish_part) where the caller has counters, else by spmv_fixup_kernel.
+//
+// Bound: the gathers of x, one L2 request each; past 4 MB of x most of them miss their XCD's L2 and
+// are bound by the fabric (1 M rows, 11 M entries, fp64, power-law: 203 us, 7 TB/s of 128-byte lines;
+// without a plan's boundaries and with the second launch 211 us).  Small matrices are bound by the launch: 2000
+// rows 19.1 -> 6.1 us per call, 100 k rows x 10 19.7 -> 10.8 us with one launch instead of two and
+// boundaries read instead of searched for.
 constexpr int kSpmvItems = 512;
 // large matrices take chunks twice the size: 16 loads per lane in flight instead of 8, half
 // the chunks to start and to fix up (0.124 -> 0.117 ms on a 17 M-nonzero graph); smaller
@@ -607,7 +611,8 @@ template <typename T, int ITEMS>
 __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
     int M, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
     const T *__restrict__ vals, const T *__restrict__ x, T *__restrict__ y, int64_t total_items,
-    int *__restrict__ carry_row, T *__restrict__ carry_val) {
+    int *__restrict__ carry_row, T *__restrict__ carry_val, const Boundary *__restrict__ bounds,
+    int *__restrict__ counters) {
   using A = typename Acc<T>::type;
   __shared__ A s_prod[kWavesPerBlock][ITEMS];
   __shared__ int s_rp[kWavesPerBlock][ITEMS + 2];
@@ -616,14 +621,23 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
   const int w = threadIdx.x / kWaveSize;
   // the grid is a multiple of 8 workgroups; every XCD takes a contiguous eighth of the spans
   const int64_t span = xcd_contiguous(blockIdx.x, gridDim.x) * kWavesPerBlock + w;
-  int64_t d0 = span * ITEMS;
+  // Where the chunk begins: read from a plan's table, whose boundaries move forward to a row's end by up to
+  // kSnapItems items (few rows are then cut at all; chunks are that much shorter nominally, so that
+  // one still holds at most ITEMS), or searched for in row_ptr (four dependent loads).
+  const int items = bounds ? ITEMS - kSnapItems : ITEMS;
+  const int64_t d0 = span * items;
   if (d0 >= total_items) return;  // nothing here uses workgroup barriers
-  int64_t d1 = d0 + ITEMS;
+  int64_t d1 = d0 + items;
   d1 = d1 < total_items ? d1 : total_items;
-
-  auto row_end_key = [&](int i) { return (int64_t)row_ptr[i + 1] + i; };
-  const int x0 = wave_count_below(M, d0, row_end_key);
-  const int y0 = uniform((int)(d0 - x0));
+  int x0, y0;
+  if (bounds) {
+    const Boundary from = load_boundary(bounds, span);
+    x0 = from.x, y0 = from.y;
+  } else {
+    auto row_end_key = [&](int i) { return (int64_t)row_ptr[i + 1] + i; };
+    x0 = wave_count_below(M, d0, row_end_key);
+    y0 = uniform((int)(d0 - x0));
+  }
 
   // Everything the chunk can touch is known from its start alone: at most
   // ITEMS nonzeros from y0 and ITEMS + 1 row pointers from x0.  All
@@ -637,7 +651,22 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
   // (a chunk that lies inside the arrays reads them at constant offsets from a scalar base:
   // no address arithmetic and no bounds checks per element)
   const bool inside = (int64_t)y0 + ITEMS <= nnz;
-  if (inside) {
+  // With the chunk's end known as well nothing beyond it is read: a gathered x is an L2 request, and
+  // those bound the kernel.
+  int n_rows = 0, y1 = 0, n_nz = ITEMS;
+  if (bounds) {
+    const Boundary to = load_boundary(bounds, span + 1);
+    n_rows = to.x - x0;
+    y1 = to.y;
+    n_nz = y1 - y0;
+#pragma unroll
+    for (int u = 0; u < kNzLoads; ++u) {
+      const int k = lane + u * kWaveSize;
+      const bool ok = k < n_nz;
+      col[u] = ok ? col_idx[y0 + k] : -1;
+      val[u] = ok ? vals[y0 + k] : (T)0;
+    }
+  } else if (inside) {
     const int *c0 = col_idx + y0;
     const T *v0 = vals + y0;
 #pragma unroll
@@ -655,7 +684,9 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
     }
   }
   int rp[kRpLoads];
-  if ((int64_t)x0 + kRpLoads * kWaveSize <= M) {
+  if (bounds) {
+    for (int k = lane; k <= n_rows + 1; k += kWaveSize) s_rp[w][k] = row_ptr[x0 + k < M ? x0 + k : M];
+  } else if ((int64_t)x0 + kRpLoads * kWaveSize <= M) {
     const int *r0 = row_ptr + x0;
 #pragma unroll
     for (int u = 0; u < kRpLoads; ++u) rp[u] = r0[lane + u * kWaveSize];
@@ -666,7 +697,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
       rp[u] = row_ptr[r < M ? r : M];
     }
   }
-  if (inside) {
+  if (inside && !bounds) {
 #pragma unroll
     for (int u = 0; u < kNzLoads; ++u) s_prod[w][lane + u * kWaveSize] = (A)val[u] * (A)x[col[u]];
   } else {
@@ -676,17 +707,22 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
       s_prod[w][lane + u * kWaveSize] = (A)val[u] * xv;
     }
   }
+  if (!bounds) {
 #pragma unroll
-  for (int u = 0; u < kRpLoads; ++u)
-    if (lane + u * kWaveSize < ITEMS + 2) s_rp[w][lane + u * kWaveSize] = rp[u];
+    for (int u = 0; u < kRpLoads; ++u)
+      if (lane + u * kWaveSize < ITEMS + 2) s_rp[w][lane + u * kWaveSize] = rp[u];
+  }
   wave_lds_sync();
 
   // rows ending inside the chunk: row x0 + j ends at merged position s_rp[j + 1] + x0 + j,
   // and no row from x0 + ITEMS on can end before d1
-  const int reach = M - x0 < ITEMS ? M - x0 : ITEMS;
-  const int n_rows = wave_count_below(reach, d1, [&](int j) { return (int64_t)s_rp[w][j + 1] + x0 + j; });
+  if (!bounds) {
+    const int reach = M - x0 < ITEMS ? M - x0 : ITEMS;
+    n_rows = wave_count_below(reach, d1, [&](int j) { return (int64_t)s_rp[w][j + 1] + x0 + j; });
+    y1 = uniform((int)(d1 - x0 - n_rows));
+  }
   const int x1 = x0 + n_rows;
-  const int y1 = uniform((int)(d1 - x1));
+  const bool carry_in = uniform(s_rp[w][0]) < y0;  // row x0 began in an earlier chunk
 
   // Row slot r is row x0 + r; slot n_rows is the row that continues past the chunk.
   for (int base = 0; base <= n_rows; base += kWaveSize) {
@@ -717,22 +753,35 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_merge_kernel(
     }
     if (live) {
       if (r < n_rows) {
-        y[x0 + r] = (T)sum;
+        if (counters && carry_in && r == 0) store_part<T, 1>(y + x0, Vec<T, 1>{(T)sum});
+        else y[x0 + r] = (T)sum;
+      } else if (counters) {
+        if (len > 0) store_part<T, 1>(carry_val + span, Vec<T, 1>{(T)sum});
       } else {
         carry_row[span] = len > 0 ? x1 : -1;
         if (len > 0) carry_val[span] = (T)sum;
       }
     }
   }
+  if (counters) {  // rows cut by chunk boundaries: see finish_part
+    const T none[1] = {(T)0};
+    const int64_t spans = (total_items + items - 1) / items;
+    auto finish = [&](int row, int begin, int end, bool carry) {
+      finish_part<T, 1, kEpiNone>(row, begin, end, span, carry, items, bounds ? kSnapItems : 0, spans, counters, 1, 0, lane == 0,
+                                  carry_val, y, none);
+    };
+    if (carry_in && n_rows > 0) finish(x0, uniform(s_rp[w][0]), uniform(s_rp[w][1]), false);
+    const int tail_begin = uniform(s_rp[w][n_rows]);
+    if (y1 > (tail_begin > y0 ? tail_begin : y0)) finish(x1, tail_begin, uniform(s_rp[w][n_rows + 1]), true);
+  }
 }
 
 // The carries of SpMV are single values, so a wavefront per chunk (spmm_fixup_kernel)
 // would leave 63 lanes idle.  Here a thread looks at one chunk: if it heads a run
 // of equal carry rows it adds the run, in chunk order, to y.  Runs of more than
-// kSpmvShortRun carries (a row spread over that many wavefronts) are then taken
-// one after the other by the whole wavefront: lane l sums members l, l + 64, ...
-// and the lanes' sums are combined in a fixed order.  Same result on every run.
-constexpr int kSpmvShortRun = 32;
+// kFoldGroup carries (a row spread over that many wavefronts) are then taken
+// one after the other by the whole wavefront: a lane sums a group of kFoldGroup, and the
+// groups' sums are added up in order, as finish_part does.
 
 template <typename T>
 __global__ __launch_bounds__(kBlockThreads) void spmv_fixup_kernel(int64_t spans,
@@ -754,8 +803,8 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_fixup_kernel(int64_t spans
     if (row >= 0) {
       if (after == row) {
         int64_t e = c + 1;
-        for (; e < spans && e < c + kSpmvShortRun && carry_row[e] == row; ++e) sum += (A)carry_val[e];
-        long_run = e == c + kSpmvShortRun && e < spans && carry_row[e] == row;
+        for (; e < spans && e < c + kFoldGroup && carry_row[e] == row; ++e) sum += (A)carry_val[e];
+        long_run = e == c + kFoldGroup && e < spans && carry_row[e] == row;
       }
       if (!long_run) y[row] = (T)(sum + (A)y[row]);
     }
@@ -767,17 +816,26 @@ __global__ __launch_bounds__(kBlockThreads) void spmv_fixup_kernel(int64_t spans
     const int64_t start = c - lane + owner;
     const int r = __shfl(row, owner);
     const int64_t end = carry_run_end(carry_row, start, spans, r);
-    A part = (A)0;
-    for (int64_t e = start + lane; e < end; e += kWaveSize) part += (A)carry_val[e];
-#pragma unroll
-    for (int off = kWaveSize / 2; off > 0; off >>= 1) part += (A)__shfl_xor((T)part, off);
-    if (lane == owner) y[r] = (T)(part + (A)y[r]);
+    A total = (A)0;
+    for (int64_t base = start; base < end; base += kWaveSize * kFoldGroup) {
+      A part = (A)0;
+      for (int j = 0; j < kFoldGroup; ++j) {
+        const int64_t e = base + lane * kFoldGroup + j;
+        if (e < end) part += (A)carry_val[e];
+      }
+      const int64_t left = (end - base + kFoldGroup - 1) / kFoldGroup;
+      const int groups = left < kWaveSize ? (int)left : kWaveSize;
+      for (int g = 0; g < groups; ++g) total += (A)__shfl((T)part, g);
+    }
+    if (lane == owner) y[r] = (T)(total + (A)y[r]);
   }
 }
 
+inline int spmv_items(int64_t M, int64_t nnz) { return M + nnz >= kSpmvLargeFrom ? kSpmvItemsLarge : kSpmvItems; }
+
 // (the most spans a call can use: the workspace is sized by it)
 inline int64_t spmv_num_spans(int64_t M, int64_t nnz) {
-  return (M + nnz + kSpmvItems - 1) / kSpmvItems;
+  return (M + nnz + kSpmvItems - kSnapItems - 1) / (kSpmvItems - kSnapItems);
 }
 
 inline size_t spmv_workspace_bytes(int64_t M, int64_t nnz, size_t elem) {
@@ -788,7 +846,8 @@ inline size_t spmv_workspace_bytes(int64_t M, int64_t nnz, size_t elem) {
 template <typename T>
 int spmv_entry(const char *fn, int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr,
                const int32_t *col_idx, const T *vals, const T *x, T *y, void *workspace,
-               size_t workspace_bytes, void *stream) {
+               size_t workspace_bytes, void *stream, const void *bounds_buffer = nullptr, size_t bounds_bytes = 0,
+               int *counters = nullptr, int64_t counters_given = 0) {
   if (int rc = check_csr_args(fn, M, K, nnz, row_ptr, col_idx, vals)) return rc;
   if (M == 0) return SCORCH_HIP_OK;
   SCORCH_REQUIRE(y != nullptr, "%s: y is NULL", fn);
@@ -801,20 +860,27 @@ int spmv_entry(const char *fn, int64_t M, int64_t K, int64_t nnz, const int32_t 
                 workspace ? workspace_bytes : (size_t)0);
   SCORCH_REQUIRE(aligned_to(workspace, 256), "%s: workspace must be 256-byte aligned", fn);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool large = M + nnz >= kSpmvLargeFrom;
-  const int64_t items_per_span = large ? kSpmvItemsLarge : kSpmvItems;
+  const bool large = spmv_items(M, nnz) == kSpmvItemsLarge;
+  const int items_per_span = spmv_items(M, nnz) - (bounds_buffer ? kSnapItems : 0);
   const int64_t spans = (M + nnz + items_per_span - 1) / items_per_span;
+  const Boundary *bounds = static_cast<const Boundary *>(bounds_buffer);
+  if (bounds && bounds_bytes < (size_t)(spans + 1) * sizeof(Boundary))
+    return fail(SCORCH_HIP_EWORKSPACE, "%s: chunk boundaries of %zu bytes needed, %zu given", fn,
+                (size_t)(spans + 1) * sizeof(Boundary), bounds_bytes);
+  SCORCH_REQUIRE(aligned_to(bounds, 8) && aligned_to(counters, 4), "%s: boundaries or counters are misaligned", fn);
+  if (counters_given < 2 * spans) counters = nullptr;  // the launch below folds the carries
   int *carry_row = static_cast<int *>(workspace);
   T *carry_val = reinterpret_cast<T *>(static_cast<char *>(workspace) +
                                        align_up((size_t)spans * sizeof(int), 256));
   const int64_t blocks = round_up_8((spans + kWavesPerBlock - 1) / kWavesPerBlock);
   if (large)
     spmv_merge_kernel<T, kSpmvItemsLarge><<<dim3((unsigned)blocks), kBlockThreads, 0, s>>>(
-        (int)M, row_ptr, col_idx, vals, x, y, M + nnz, carry_row, carry_val);
+        (int)M, row_ptr, col_idx, vals, x, y, M + nnz, carry_row, carry_val, bounds, counters);
   else
     spmv_merge_kernel<T, kSpmvItems><<<dim3((unsigned)blocks), kBlockThreads, 0, s>>>(
-        (int)M, row_ptr, col_idx, vals, x, y, M + nnz, carry_row, carry_val);
+        (int)M, row_ptr, col_idx, vals, x, y, M + nnz, carry_row, carry_val, bounds, counters);
   SCORCH_HIP_CHECK(hipGetLastError());
+  if (counters) return SCORCH_HIP_OK;
   spmv_fixup_kernel<T><<<dim3((unsigned)((spans + kBlockThreads - 1) / kBlockThreads)), kBlockThreads, 0, s>>>(
       spans, carry_row, carry_val, y);
   SCORCH_HIP_CHECK(hipGetLastError());
@@ -893,6 +959,49 @@ SCORCH_DEFINE_SPMV(f32, float)
 SCORCH_DEFINE_SPMV(f64, double)
 SCORCH_DEFINE_SPMV(i32, int32_t)
 SCORCH_DEFINE_SPMV(i64, int64_t)
+
+#define SCORCH_DEFINE_SPMV_PLANNED(SUFFIX, T)                                                   \
+  int scorch_hip_spmv_csr_planned_##SUFFIX(                                                      \
+      int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,        \
+      const T *vals, const T *x, T *y, const void *bounds, size_t bounds_bytes, void *workspace, \
+      size_t workspace_bytes, int32_t *counters, int64_t n_counters, void *stream) {            \
+    return scorch::spmv_entry<T>("scorch_hip_spmv_csr_planned_" #SUFFIX, M, K, nnz, row_ptr,     \
+                                 col_idx, vals, x, y, workspace, workspace_bytes, stream, bounds, \
+                                 bounds_bytes, counters, counters ? n_counters : 0);            \
+  }
+
+SCORCH_DEFINE_SPMV_PLANNED(f32, float)
+SCORCH_DEFINE_SPMV_PLANNED(f64, double)
+SCORCH_DEFINE_SPMV_PLANNED(i32, int32_t)
+SCORCH_DEFINE_SPMV_PLANNED(i64, int64_t)
+
+int64_t scorch_hip_spmv_csr_planned_counters(int64_t M, int64_t nnz) {
+  return M < 0 || nnz < 0 ? 0 : 2 * scorch::spmv_num_spans(M, nnz);
+}
+
+size_t scorch_hip_spmv_csr_bounds_bytes(int64_t M, int64_t nnz) {
+  return M < 0 || nnz < 0 ? 0 : (size_t)(scorch::spmv_num_spans(M, nnz) + 1) * sizeof(scorch::Boundary);
+}
+
+int scorch_hip_spmv_csr_bounds(int64_t M, int64_t nnz, const int32_t *row_ptr, void *bounds, size_t bounds_bytes,
+                               void *stream) {
+  const char *fn = "scorch_hip_spmv_csr_bounds";
+  if (M < 0 || nnz < 0 || M >= INT32_MAX || nnz > INT32_MAX)
+    return scorch::fail(SCORCH_HIP_EINVAL, "%s: M=%lld or nnz=%lld is negative or too large", fn, (long long)M, (long long)nnz);
+  SCORCH_REQUIRE(row_ptr != nullptr && bounds != nullptr, "%s: row_ptr or bounds is NULL", fn);
+  SCORCH_REQUIRE(scorch::aligned_to(row_ptr, 4) && scorch::aligned_to(bounds, 8),
+                 "%s: row_ptr must be 4-byte and bounds 8-byte aligned", fn);
+  const int items = scorch::spmv_items(M, nnz) - scorch::kSnapItems;
+  const int64_t num_bounds = (M + nnz + items - 1) / items + 1;
+  if (bounds_bytes < (size_t)num_bounds * sizeof(scorch::Boundary))
+    return scorch::fail(SCORCH_HIP_EWORKSPACE, "%s: %zu bytes needed for the boundaries, %zu given", fn,
+                        (size_t)num_bounds * sizeof(scorch::Boundary), bounds_bytes);
+  scorch::spmm_bounds_kernel<<<dim3((unsigned)((num_bounds + scorch::kBlockThreads - 1) / scorch::kBlockThreads)),
+                               scorch::kBlockThreads, 0, static_cast<hipStream_t>(stream)>>>(
+      (int)M, M + nnz, items, scorch::kSnapItems, num_bounds, row_ptr, static_cast<scorch::Boundary *>(bounds));
+  SCORCH_HIP_CHECK(hipGetLastError());
+  return SCORCH_HIP_OK;
+}
 
 int scorch_hip_spmm_csr_f32_timed(int64_t M, int64_t K, int64_t N, int64_t nnz,
                                   const int32_t *row_ptr, const int32_t *col_idx, const float *vals,

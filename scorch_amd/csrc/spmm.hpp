@@ -131,12 +131,12 @@ struct RowSpan {
 };
 // Row `row`'s chunks: nominal positions of its first entry and its end marker, the latter's chunk
 // corrected for a boundary inside the row that has moved past the marker (chunk_boundary).
-__device__ __forceinline__ RowSpan row_span(int row, int begin, int end, int shift, int snap) {
-  const int64_t p0 = (int64_t)begin + row, marker = (int64_t)end + row;
+__device__ __forceinline__ RowSpan row_span(int row, int begin, int end, int items, int snap) {
+  const int64_t p0 = (int64_t)begin + row, marker = (int64_t)end + row;  // below 2^32
   RowSpan s;
-  s.first = (int)(p0 >> shift);
-  s.last = (int)(marker >> shift);
-  const int64_t d = (int64_t)s.last << shift;
+  s.first = (int)((unsigned)p0 / (unsigned)items);
+  s.last = (int)((unsigned)marker / (unsigned)items);
+  const int64_t d = (int64_t)s.last * items;
   if (d > p0 && marker + 1 - d <= snap) --s.last;
   return s;
 }
@@ -206,11 +206,11 @@ __device__ __forceinline__ Vec<T, VEC> sum_parts(const T *__restrict__ carry_val
 // counters: two per chunk, the groups' and the rows', each at the first chunk of its own.
 constexpr int kFoldGroup = 16;
 template <typename T, int VEC, int EPI>
-__device__ __forceinline__ void finish_part(int row, int begin, int end, int64_t chunk, bool carry, int shift, int snap,
+__device__ __forceinline__ void finish_part(int row, int begin, int end, int64_t chunk, bool carry, int items, int snap,
                                             int64_t n_chunks, int *__restrict__ counters, int N, int col0, bool folds,
                                             T *__restrict__ carry_val, T *__restrict__ C, const T (&bias_v)[VEC]) {
   using A = typename Acc<T>::type;
-  const RowSpan span = row_span(row, begin, end, shift, snap);
+  const RowSpan span = row_span(row, begin, end, items, snap);
   const int n = span.last - span.first;
   int *const rows = counters + n_chunks;
   int parts = n, step = 1;

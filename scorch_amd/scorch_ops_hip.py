@@ -823,7 +823,13 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
 
     if width < 0:
         if not pos_of_coo:
-            remember(_ROUTE_SPMV, workspace=L.scorch_hip_spmv_csr_workspace_bytes(M, nnz, elem))
+            bounds = plan.bounds.get("spmv")
+            if bounds is None:
+                return
+            counters = L.scorch_hip_spmv_csr_planned_counters(M, nnz)
+            _counters(dev, _stream(dev), counters)
+            remember(_ROUTE_SPMV, (bounds.numel(), 0, 0, counters), (bounds,),
+                     L.scorch_hip_spmv_csr_workspace_bytes(M, nnz, elem))
         return
     may_tile = width >= 512 and vals.dtype == torch.float32 and bool(L.scorch_hip_dense_tiled_recommended(K, width, nnz, 4))
     if act == 0 and vals.dtype == torch.float32 and BLOCKED_PATH != "off" and width in BLOCKED_WIDTHS:
@@ -1021,6 +1027,16 @@ prebuilt_spmspm_csr_i32 = _make_spgemm(torch.int32)
 prebuilt_spmspm_csr_i64 = _make_spgemm(torch.int64)
 
 
+def _spmv_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, L, stream) -> Optional[torch.Tensor]:
+    """Chunk boundaries of the matrix-vector product, computed once."""
+    bounds = plan.bounds.get("spmv")
+    if bounds is None and M > 0:
+        bounds = _empty(L.scorch_hip_spmv_csr_bounds_bytes(M, nnz), dtype=torch.uint8, device=pos.device)
+        native.check(L.scorch_hip_spmv_csr_bounds(M, nnz, pos.data_ptr(), bounds.data_ptr(), bounds.numel(), stream))
+        plan.bounds["spmv"] = bounds
+    return bounds
+
+
 # ---- SpMV ----------------------------------------------------------------------
 def _make_spmv(dtype):
     def kernel(result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mode_indices, B_values):
@@ -1031,16 +1047,18 @@ def _make_spmv(dtype):
         if pos.numel() != M + 1 or x.numel() != K or crd.numel() != a_val.numel():
             raise ValueError("scorch_ops_hip: array lengths do not match the shapes")
         dev = _device_of(pos, crd, a_val, x)
-        csr_plan(pos, crd, M, K, "A")
+        plan = csr_plan(pos, crd, M, K, "A")
         y = _empty(M, dtype=dtype, device=dev)
         L = native.lib()
+        nnz = a_val.numel()
         with _on_device(dev):
             stream = _stream(dev)
-            ws = _workspace(dev, stream, L.scorch_hip_spmv_csr_workspace_bytes(M, a_val.numel(),
-                                                                              a_val.element_size()))
-            fn = getattr(L, "scorch_hip_spmv_csr_" + _SUFFIX[dtype])
-            rc = fn(M, K, a_val.numel(), pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(), x.data_ptr(),
-                    y.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+            ws = _workspace(dev, stream, L.scorch_hip_spmv_csr_workspace_bytes(M, nnz, a_val.element_size()))
+            bounds = _spmv_bounds(plan, pos, M, nnz, L, stream) if plan is not None else None
+            fn = getattr(L, "scorch_hip_spmv_csr_planned_" + _SUFFIX[dtype])
+            rc = fn(M, K, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(), x.data_ptr(), y.data_ptr(),
+                    bounds.data_ptr() if bounds is not None else None, bounds.numel() if bounds is not None else 0,
+                    ws.data_ptr(), ws.numel(), *_counters(dev, stream, L.scorch_hip_spmv_csr_planned_counters(M, nnz)), stream)
         native.check(rc)
         return Tensor(y, [[]])
     return kernel

@@ -155,3 +155,31 @@ def test_rows_folded_in_one_launch_are_the_second_launchs_bit_for_bit(dtype, N, 
         got = native.host().spmm(A, b, bias, 2 if relu else 0)
         assert got is not None and torch.equal(got, want)
     assert all(int(c.abs().sum()) == 0 for c in H._counter_buffers.values())
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("rows, entries", [(1, 0), (1, 447), (1, 448), (3, 1500), (5000, 20_000), (900_000, 5_000_000)])
+def test_vector_product_from_a_plans_boundaries(dtype, rows, entries):
+    """One short chunk, a row that ends at a chunk's end, rows over many chunks, and the larger chunks of
+    large matrices: against float64, and launch after launch on the same counters."""
+    rng = np.random.default_rng(rows)
+    K = 3000
+    lens = rng.multinomial(entries // 2, np.full(rows, 1 / rows))
+    lens[rows // 2] += entries - entries // 2
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    integer = np.issubdtype(dtype, np.integer)
+    ci = rng.integers(0, K, entries).astype(np.int32)
+    v = (rng.integers(-9, 9, entries) if integer else rng.uniform(-1, 1, entries)).astype(dtype)
+    x = (rng.integers(-9, 9, K) if integer else rng.standard_normal(K)).astype(dtype)
+    A = STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (rows, K))
+    xd = dev(x)
+    want = np.bincount(np.repeat(np.arange(rows), lens), v.astype(np.float64) * x[ci], minlength=rows)
+    got = scorch.matmul(A, xd)
+    if integer:
+        assert np.array_equal(host(got), want.astype(dtype))
+    else:
+        tol = 1e-5 if dtype == np.float32 else 1e-12
+        assert np.linalg.norm(host(got) - want) <= tol * max(np.linalg.norm(want), 1e-30)
+    for _ in range(10):
+        assert torch.equal(scorch.matmul(A, xd), got)
+    assert all(int(c.abs().sum()) == 0 for c in H._counter_buffers.values())
