@@ -244,6 +244,8 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
   const int v_chunk = (n & 3) >> 1;
   const int my_query_in_block = w * 16 + n;
 
+  int next_mask = -1;  // MASKED: where the next block's bit mask is (-1: it has none)
+  if (MASKED && kb_begin < kb_end) next_mask = uniform(block_mask_index[kb_begin]);
   if (kb_begin < kb_end) load_tile(Even{}, kb_begin);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -253,6 +255,17 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
     using Other = std::integral_constant<int, buf ^ 1>;
     const unsigned char *k_src = buf ? s_k1 : s_k0;
     const unsigned char *v_src = buf ? s_v1 : s_v0;
+    // A block that is only partly live brings a 64 x 64 bit mask: bit j of word i says whether
+    // query i of the block row attends to key j of the block.  A lane holds the scores of its
+    // query against keys 16t + 4g + r (bit 16t + r of the word shifted down by 4g); dead ones are
+    // kept out of the maximum and get probability zero below.  The word is requested ahead of the
+    // tile (loads come back in order) and its place one block ahead, so that neither is waited for.
+    const int mask_at = next_mask;
+    unsigned long long live = ~0ull;
+    if constexpr (MASKED) {
+      if (mask_at >= 0) live = block_masks[(size_t)mask_at * kAttnBlock + my_query_in_block];
+      if (it + 1 < kb_end) next_mask = uniform(block_mask_index[it + 1]);
+    }
     if (it + 1 < kb_end) load_tile(Other{}, it + 1);  // its last readers passed the previous barrier
 
     floatx4 st[4];
@@ -271,11 +284,11 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
     // while the vector ALU does the softmax; requested one by one just before their MFMAs, every
     // MFMA of the second product waits an LDS round trip.  (The masked kernel at D = 64 has no
     // registers left for that and requests them after the softmax.)
-    constexpr bool kEarlyV = !(MASKED && D == 64);
+    constexpr int kEarlyV = MASKED && D == 64 ? 3 : kFeat;
     bf16x8 v_ops[kFeat][2];
-    auto request_v_operands = [&]() {
+    auto request_v_operands = [&](int from, int to) {
 #pragma unroll
-      for (int dt = 0; dt < kFeat; ++dt)
+      for (int dt = from; dt < to; ++dt)
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
           const int at = 32 * kRowBytes * s + v_off + (((2 * dt + v_chunk) ^ v_swz) * 16);
@@ -285,19 +298,12 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
           v_ops[dt][s] = __builtin_bit_cast(bf16x8, packed);
         }
     };
-    if constexpr (kEarlyV) request_v_operands();
+    request_v_operands(0, kEarlyV);
     __builtin_amdgcn_sched_barrier(0);  // (the scheduler would move the reads back down to their uses)
 
-    // A block that is only partly live brings a 64 x 64 bit mask: bit j of word i says whether
-    // query i of the block row attends to key j of the block.  A lane holds the scores of its
-    // query against keys 16t + 4g + r (bit 16t + r of the word shifted down by 4g); dead ones are
-    // kept out of the maximum here and get probability zero below.
-    int mask_at = -1;
-    unsigned long long live = ~0ull;
     if constexpr (MASKED) {
-      mask_at = uniform(block_mask_index[it]);
       if (mask_at >= 0) {
-        live = block_masks[(size_t)mask_at * kAttnBlock + my_query_in_block] >> (4 * g);
+        live >>= 4 * g;
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -338,14 +344,23 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[t][r], scale_log2e, -m_run));
-        if constexpr (MASKED) {
-          if (!((live >> (16 * t + r)) & 1ull)) p = 0.0f;
-        }
-        p_op[t >> 1][(t & 1) * 4 + r] = (__bf16)p;
+        st[t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[t][r], scale_log2e, -m_run));
       }
+    if constexpr (MASKED) {
+      if (mask_at >= 0) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (!((live >> (16 * t + r)) & 1ull)) st[t][r] = 0.0f;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p_op[t >> 1][(t & 1) * 4 + r] = (__bf16)st[t][r];
 
-    if constexpr (!kEarlyV) request_v_operands();
+    request_v_operands(kEarlyV, kFeat);
 #pragma unroll
     for (int dt = 0; dt < kFeat; ++dt)
 #pragma unroll
@@ -399,44 +414,39 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
 
 // Combines the stretches of a block row that was shared out: with m* the largest of the
 // stretches' reference maxima (base-2 exponents), O = sum_p 2^(m_p - m*) O_p / sum_p 2^(m_p - m*) l_p.
-// One workgroup per (split row, head); thread t takes query t / 4 and a quarter of the features.
+// A thread takes four features of a query: a row has few stretches (a dozen) and a launch few such rows (a
+// global token's), so it is the number of loads in flight that counts (S = 8,192, 16 heads, one shared-out
+// row of 13 stretches: 10.3 us with a quarter of the features per thread and one workgroup per row and head).
 template <int D>
 __global__ __launch_bounds__(kBlockThreads) void attn_merge_kernel(int S, int n_slots,
                                                                    const int4 *__restrict__ split_rows,
                                                                    const float *__restrict__ partials,
                                                                    __bf16 *__restrict__ O) {
+  constexpr int kLanes = D / 4, kQueries = kBlockThreads / kLanes;  // threads per query, queries per workgroup
   const int4 row = split_rows[blockIdx.x];  // x: block row, y: first slot, z: number of stretches
   const int head = blockIdx.y;
-  const int q = threadIdx.x >> 2, quarter = threadIdx.x & 3;
-  constexpr int kMine = D / 4;  // features per thread
+  const int q = blockIdx.z * kQueries + threadIdx.x / kLanes, feature = threadIdx.x % kLanes * 4;
   const float *base = partials + (((size_t)head * n_slots + row.y) * kAttnBlock + q) * (D + 4);
   const size_t part_stride = (size_t)kAttnBlock * (D + 4);
   float m_star = -3.0e38f;
+#pragma unroll 8
   for (int p = 0; p < row.z; ++p) m_star = fmaxf(m_star, base[p * part_stride + D]);
-  float acc[kMine];
-#pragma unroll
-  for (int j = 0; j < kMine; ++j) acc[j] = 0.0f;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   float l = 0.0f;
+#pragma unroll 4
   for (int p = 0; p < row.z; ++p) {
     const float *part = base + p * part_stride;
     const float weight = __builtin_amdgcn_exp2f(part[D] - m_star);
     l += weight * part[D + 1];
+    const floatx4 o = *reinterpret_cast<const floatx4 *>(part + feature);
 #pragma unroll
-    for (int j = 0; j < kMine; j += 4) {
-      const floatx4 o = *reinterpret_cast<const floatx4 *>(part + quarter * kMine + j);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[j + r] += weight * o[r];
-    }
+    for (int r = 0; r < 4; ++r) acc[r] += weight * o[r];
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  __bf16 *out = O + ((size_t)head * S + (size_t)row.x * kAttnBlock + q) * D + quarter * kMine;
+  bf16x4 o;
 #pragma unroll
-  for (int j = 0; j < kMine; j += 4) {
-    bf16x4 o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[j + r] * inv);
-    *reinterpret_cast<bf16x4 *>(out + j) = o;
-  }
+  for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[r] * inv);
+  *reinterpret_cast<bf16x4 *>(O + ((size_t)head * S + (size_t)row.x * kAttnBlock + q) * D + feature) = o;
 }
 
 }  // namespace scorch
@@ -534,6 +544,7 @@ static int attn_entry(const char *fn, int64_t H, int64_t S, int64_t D, int64_t b
                *v = static_cast<const __bf16 *>(V);
   __bf16 *o = static_cast<__bf16 *>(O);
   const unsigned long long *masks = reinterpret_cast<const unsigned long long *>(block_masks);
+  if (!masks) block_mask_index = nullptr;  // no bit masks to name: every block is whole
   mark_launch(s);
   if (D == 32)
     attn_launch_dim<32>(grid, s, scale < 0.0f, (int)S, n_blocks, (int)H, block_row_ptr, block_col_idx,
@@ -547,7 +558,7 @@ static int attn_entry(const char *fn, int64_t H, int64_t S, int64_t D, int64_t b
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(s);
   if (split && split->n_split_rows > 0) {
-    const dim3 merge_grid((unsigned)split->n_split_rows, (unsigned)H);
+    const dim3 merge_grid((unsigned)split->n_split_rows, (unsigned)H, (unsigned)(kAttnBlock * D / 4 / kBlockThreads));
     const int4 *rows = reinterpret_cast<const int4 *>(split->split_rows);
     if (D == 32) attn_merge_kernel<32><<<merge_grid, kBlockThreads, 0, s>>>((int)S, n_slots, rows, partials, o);
     else if (D == 64) attn_merge_kernel<64><<<merge_grid, kBlockThreads, 0, s>>>((int)S, n_slots, rows, partials, o);
@@ -585,8 +596,8 @@ extern "C" int scorch_hip_attn_blocksparse_masked_bf16(
     SCORCH_REQUIRE(aligned_to(block_masks, 8), "%s: block_masks must be 8-byte aligned", fn);
   }
   return attn_entry(fn, H, S, D, block, n_active_blocks, block_row_ptr, block_col_idx,
-                    n_active_blocks > 0 ? block_mask_index : nullptr, block_masks, Q, K, V, scale,
-                    O, stream);
+                    n_active_blocks > 0 ? block_mask_index : nullptr, n_masks > 0 ? block_masks : nullptr, Q, K, V,
+                    scale, O, stream);
 }
 
 extern "C" size_t scorch_hip_attn_blocksparse_split_workspace_bytes(int64_t H, int64_t n_slots, int64_t D) {
@@ -618,8 +629,8 @@ extern "C" int scorch_hip_attn_blocksparse_split_bf16(
   split.split_rows = split_rows;
   split.workspace = workspace;
   split.workspace_bytes = workspace_bytes;
-  return attn_entry(fn, H, S, D, block, n_active_blocks, nullptr, block_col_idx, block_mask_index, block_masks,
-                    Q, K, V, scale, O, stream, &split);
+  return attn_entry(fn, H, S, D, block, n_active_blocks, nullptr, block_col_idx, block_mask_index,
+                    n_masks > 0 ? block_masks : nullptr, Q, K, V, scale, O, stream, &split);
 }
 
 SCORCH_DEFINE_PRELOAD(attn)

@@ -339,37 +339,29 @@ __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, in
                                                                        float *__restrict__ O) {
   const int4 row = split_rows[blockIdx.x];  // x: block row, y: first slot, z: number of stretches
   const int head = blockIdx.y;
-  const int q = threadIdx.x >> 2, quarter = threadIdx.x & 3;
-  constexpr int kMine = D / 4;
+  constexpr int kLanes = D / 4, kQueries = kBlockThreads / kLanes;  // threads per query, queries per workgroup
+  const int q = blockIdx.z * kQueries + threadIdx.x / kLanes, feature = threadIdx.x % kLanes * 4;
   const float *base = partials + (((size_t)head * n_slots + row.y) * kBlock + q) * (D + 4);
   const size_t part_stride = (size_t)kBlock * (D + 4);
   float m_star = kDead;
+#pragma unroll 8
   for (int p = 0; p < row.z; ++p) m_star = fmaxf(m_star, base[p * part_stride + D]);
-  float acc[kMine];
-#pragma unroll
-  for (int j = 0; j < kMine; ++j) acc[j] = 0.0f;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   float l = 0.0f;
+#pragma unroll 4
   for (int p = 0; p < row.z; ++p) {
     const float *part = base + p * part_stride;
     const float weight = __builtin_amdgcn_exp2f(part[D] - m_star);
     l += weight * part[D + 1];
+    const floatx4 o = *reinterpret_cast<const floatx4 *>(part + feature);
 #pragma unroll
-    for (int j = 0; j < kMine; j += 4) {
-      const floatx4 o = *reinterpret_cast<const floatx4 *>(part + quarter * kMine + j);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[j + r] += weight * o[r];
-    }
+    for (int r = 0; r < 4; ++r) acc[r] += weight * o[r];
   }
   if (row.x * kBlock + q >= S) return;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  float *out = O + ((size_t)head * S + (size_t)row.x * kBlock + q) * D + quarter * kMine;
 #pragma unroll
-  for (int j = 0; j < kMine; j += 4) {
-    floatx4 o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = acc[j + r] * inv;
-    *reinterpret_cast<floatx4 *>(out + j) = o;
-  }
+  for (int r = 0; r < 4; ++r) acc[r] *= inv;
+  *reinterpret_cast<floatx4 *>(O + ((size_t)head * S + (size_t)row.x * kBlock + q) * D + feature) = acc;
 }
 
 template <int D>
@@ -385,8 +377,8 @@ static int launch(dim3 grid, hipStream_t s, int S, int n_blocks, int H, const in
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(s);
   if (n_split_rows > 0) {
-    attn_f32_merge_kernel<D><<<dim3((unsigned)n_split_rows, (unsigned)H), kBlockThreads, 0, s>>>(S, n_slots, split_rows,
-                                                                                               partials, o);
+    const dim3 merge_grid((unsigned)n_split_rows, (unsigned)H, (unsigned)(kBlock * D / 4 / kBlockThreads));
+    attn_f32_merge_kernel<D><<<merge_grid, kBlockThreads, 0, s>>>(S, n_slots, split_rows, partials, o);
     SCORCH_HIP_CHECK(hipGetLastError());
     mark_launch(s);
   }
