@@ -1673,7 +1673,7 @@ def _block_mask(pos: torch.Tensor, crd: torch.Tensor, S: int) -> BlockMask:
 
 
 # workgroups of the fused bf16 attention kernel a CU holds at once, by head dimension
-ATTENTION_WORKGROUPS_PER_CU = {32: 6, 64: 4, 128: 2}
+ATTENTION_WORKGROUPS_PER_CU = {32: 5, 64: 4, 128: 2}
 
 
 _cu_counts: Dict[int, int] = {}
@@ -1690,20 +1690,27 @@ def pair_attention_items(lens, heads: int, D: int, n_cus: int = 256) -> bool:
     """Whether the fused bf16 attention kernel should give every workgroup two work items, the
     k-th longest and then the k-th shortest (scorch_hip_attn_blocksparse_split_bf16, pair_items).
     `lens`: key blocks per item.  Pairing evens the workgroups out and halves their number; it
-    pays where the items differ in length, or are so short that a workgroup's start and end
+    pays where the items differ in length, or are all so short that a workgroup's start and end
     weigh, and the launch is between about 0.6 and 4 times what the chip holds at once, and costs
     elsewhere (S = 8192, 16 heads, D = 64, measured: the benchmark's causal strided mask -7 %,
     four blocks in every row -9 %, twelve +1 %; a causal mask at S = 4096 -15 % with 16 heads,
-    +7 % with 4, -3 % with 128; at S = 16384 with D = 128 +3 %)."""
+    +7 % with 4, -3 % with 128; at S = 16384 with D = 128 +3 %).  Items that differ by less than a
+    causal mask's need a launch that does not fit the chip at once as it is (strided masks of 64 to 128
+    block rows: 1.1 to 1.6 rounds -3 to -15 %, 0.8 to 1.0 rounds +6 to +9 %), short ones among
+    them are best left alone (a window with a global token, 2 rounds: +9 %), and pairs that
+    leave a second round nearly empty lose all they gain (2.2 rounds: +22 %)."""
     import numpy as np
     lens = np.asarray(lens)
     if lens.size < 2 or D not in ATTENTION_WORKGROUPS_PER_CU:
         return False
     slots = n_cus * ATTENTION_WORKGROUPS_PER_CU[D]
     rounds = lens.size * heads / slots
-    mean = float(lens.mean())
-    uneven = float(lens.max()) > 1.25 * mean
-    return 0.6 <= rounds <= 4.0 and mean <= 64 and (uneven or mean <= 6)
+    mean, most = float(lens.mean()), float(lens.max())
+    if not 0.6 <= rounds <= 4.0 or mean > 64 or 2.0 < rounds < 8 / 3:
+        return False
+    if most <= 1.25 * mean:
+        return mean <= 6
+    return mean > 7 and (most > 1.75 * mean or rounds > 1.05)
 
 
 def attention_priority_step(lens, heads: int, D: int, pair: bool, n_cus: int = 256) -> int:
@@ -1790,7 +1797,11 @@ def sparse_attention_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, row
     if out is not None:
         return out
     bm = attention_block_mask(row_ptr, col_idx, int(q.shape[1]))
-    if bm.items is None:
+    shared_out = _bf16_launch_schedule(bm, int(q.shape[0]), int(q.shape[2]))
+    if shared_out is not None:
+        items, split_rows, n_slots, pair, step = shared_out
+        out = _attn_bf16_items(*_attn_bf16_args(q, k, v), bm, items, split_rows, n_slots, scale, pair, step)
+    elif bm.items is None:
         out = attn_blocksparse_bf16(q, k, v, bm.block_row_ptr, bm.block_col_idx, scale, block=bm.block,
                                     block_mask_index=bm.block_mask_index, block_masks=bm.block_masks)
     else:
@@ -1811,9 +1822,10 @@ def _remember_attention(q: torch.Tensor, row_ptr: torch.Tensor, col_idx: torch.T
         kind, pair, step = 2, False, 0
         ws = L.scorch_hip_attn_blocksparse_f32_workspace_bytes(H, n_slots, D) if items is not None else 0
     else:
-        if bm.items is not None:
-            items, split_rows, n_slots = bm.items, bm.split_rows, bm.n_slots
-            plan = bm.pairing.get(("items", H, D))
+        shared_out = _bf16_launch_schedule(bm, H, D)
+        if shared_out is not None:
+            items, split_rows, n_slots = shared_out[:3]
+            plan = shared_out[3:]
         else:
             schedule = _block_row_schedule(bm.block_row_ptr) if D in ATTENTION_WORKGROUPS_PER_CU else None
             plan = schedule[2].get((H, D)) if schedule is not None else None
@@ -1821,7 +1833,7 @@ def _remember_attention(q: torch.Tensor, row_ptr: torch.Tensor, col_idx: torch.T
         if plan is None:
             return
         pair, step = plan
-        kind = 1 if bm.items is not None or pair or step else 0
+        kind = 1 if shared_out is not None or pair or step else 0
         ws = L.scorch_hip_attn_blocksparse_split_workspace_bytes(H, n_slots, D) if kind == 1 else 0
     count = lambda t: t.numel() // 4 if t is not None else 0
     # (a mask of whole blocks has an index without a bit mask to name: the fp32 kernel for whole blocks takes it)
@@ -1991,6 +2003,48 @@ def _attn_bf16_items(q, k, v, bm: BlockMask, items: torch.Tensor, split_rows: Op
 # workgroup / leave the wavefronts' priorities alone whatever the mask looks like.
 ATTENTION_PAIRING = os.environ.get("SCORCH_HIP_ATTN_PAIRING", "1") not in ("", "0")
 ATTENTION_PRIORITY = os.environ.get("SCORCH_HIP_ATTN_PRIORITY", "1") not in ("", "0")
+
+
+def _bf16_stretch(lens, heads: int, D: int, n_cus: int) -> Optional[int]:
+    """Key blocks per stretch for a bf16 launch of so many heads, or None where every block row is best
+    left whole.  Rows more than twice as long as most (a global token's) would be what the launch
+    waits for: they go out in stretches of eight blocks, or twice a usual row's if that is more, and
+    where the launch leaves a quarter of the chip idle in half of that (a window of 64 with a
+    global token, us in stretches of ten and now: S = 2,048, 8 heads 11.9 -> 9.9; S = 4,096, 8 heads 13.5 ->
+    12.6; S = 8,192, 16 heads 30.4 -> 30.0).  A launch that reaches half the CUs at most shares out rows
+    of 16 blocks and more as well (S = 8,192, one head, strided: 12.3 -> 11.4; rows of seven: 6.5 -> 9)."""
+    import numpy as np
+    most = int(lens.max()) if lens.size else 0
+    if D not in ATTENTION_WORKGROUPS_PER_CU:
+        return None
+    if most <= max(8, 2 * -(-int(lens.sum()) // max(int(lens.size), 1))):
+        return 8 if most >= 16 and lens.size * heads <= n_cus // 2 else None
+    usual = int(np.median(lens))
+    if lens.size * heads < 0.75 * n_cus * ATTENTION_WORKGROUPS_PER_CU[D]:
+        return max(4, usual)
+    return max(8, 2 * usual)
+
+
+def _bf16_launch_schedule(bm: BlockMask, heads: int, D: int):
+    """(items, split rows, slots, pair the items?, priority step) for a bf16 launch of so many heads over
+    a mask with rows that are shared out, kept with the BlockMask; None where no row is, and while
+    the stream is capturing and nothing is known yet."""
+    key = ("bf16", heads, D)
+    if key not in bm.pairing:
+        if bm.block_row_ptr.is_cuda and torch.cuda.is_current_stream_capturing():
+            return None
+        lens = bm.row_lens()
+        stretch = _bf16_stretch(lens, heads, D, _cu_count(bm.block_row_ptr.device))
+        kept = None
+        if stretch is not None:
+            plain = BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)
+            plain.block_row_lens = lens
+            split_long_block_rows(plain, stretch)
+            rows = plain.items.view(-1, 4).cpu().numpy()
+            kept = (plain.items, plain.split_rows, plain.n_slots,
+                    *_launch_plan(rows[:, 2] - rows[:, 1], heads, D, bm.block_row_ptr.device))
+        bm.pairing[key] = kept
+    return bm.pairing[key]
 
 
 def _launch_plan(lens, heads: int, D: int, device):

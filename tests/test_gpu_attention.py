@@ -384,3 +384,34 @@ def test_the_dispatch_pairs_items_where_it_was_measured_to_pay():
             heads, 64 * nb, 64, 64, t_bci.numel(), t_brp.data_ptr(), t_bci.data_ptr(), q.data_ptr(), k.data_ptr(),
             v.data_ptr(), 0.125, rc_out.data_ptr(), torch.cuda.current_stream().cuda_stream))
         assert torch.equal(out, rc_out)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("S, heads, window, stretch", [
+    (512, 2, 40, None),        # rows no longer than a launch shares out
+    (1024, 4, 40, 4),          # a global token's row, a launch that leaves most of the chip idle
+    (1024, 1, 1024, 8),        # every row whole and alike: shared out because a few CUs would do all of it
+    (2048, 33, 130, 16),       # one that fills the chip, with usual rows of eight blocks
+])
+def test_rows_shared_out_by_the_size_of_the_launch(oracle, D, S, heads, window, stretch):
+    """What _bf16_stretch takes for a launch, through the public entry and against float64; the second
+    and later calls take the native path and are the same bit for bit."""
+    at = np.arange(S)
+    mask = np.abs(at[:, None] - at[None, :]) <= window
+    mask[0, :] = mask[:, 0] = True
+    lens = np.array([mask[i:i + 64].reshape(64, -1, 64).any(axis=(0, 2)).sum() for i in range(0, S, 64)])
+    chosen = H._bf16_stretch(lens, heads, D, H._cu_count("cuda"))
+    assert chosen == stretch
+    rp, ci = csr_of(mask)
+    rp, ci = dev(rp), dev(ci)
+    gen = torch.Generator().manual_seed(S + D)
+    q, k, v = (torch.randn(heads, S, D, generator=gen).to(torch.bfloat16).cuda() for _ in range(3))
+    out = H.sparse_attention_bf16(q, k, v, rp, ci, D ** -0.5)
+    kept = H.attention_block_mask(rp, ci, S).pairing[("bf16", heads, D)]
+    assert (kept is None) == (stretch is None)
+    for _ in range(3):
+        assert torch.equal(H.sparse_attention_bf16(q, k, v, rp, ci, D ** -0.5), out)
+    for h in (0, heads - 1):
+        ref = oracle.attention_dense_fp64(q[h].float().cpu().numpy(), k[h].float().cpu().numpy(),
+                                          v[h].float().cpu().numpy(), mask, D ** -0.5)
+        assert oracle.rel_fro(out[h].float().cpu().numpy(), ref) <= 5e-3
