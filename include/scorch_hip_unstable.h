@@ -90,6 +90,15 @@ SCORCH_HIP_API int scorch_hip_csr_inspect(int64_t M, int64_t K, int64_t nnz, con
 SCORCH_HIP_API int scorch_hip_csr_inspect_now(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr,
                                   const int32_t *col_idx, int32_t *report, void *stream);
 
+/* New column indices under row pointers that an earlier inspection has found well formed.  _begin
+ * queues one kernel that copies col_idx to `checked`, with columns outside [0, K) replaced by 0, so that a
+ * product over `checked` may be queued right behind it, and returns at once; _end waits for the
+ * verdict -- *outside: whether a column was replaced, i.e. the product is not to be used -- and ends the call.
+ * Every _begin that succeeded needs its _end.  Not for a stream that is being captured. */
+SCORCH_HIP_API int scorch_hip_csr_columns_begin(int64_t K, int64_t nnz, const int32_t *col_idx, int32_t *checked /* device, [nnz] */,
+                                    void *stream, void **pending);
+SCORCH_HIP_API int scorch_hip_csr_columns_end(void *pending, int32_t *outside);
+
 /* Row-split SpMM for matrices whose rows are all short: C = act(A * B + bias)
  * in one launch, without workspace (a team of lanes per row; no rows are cut,
  * so there are no carries to fold).  Same contraction as

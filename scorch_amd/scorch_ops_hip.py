@@ -314,7 +314,7 @@ class CsrPlan:
     row-pointer tensor, so it is dropped with the operand, and is rebuilt when
     either index tensor has been written to since."""
     __slots__ = ("key", "partner", "max_row", "empty_rows", "sorted_rows", "runs", "bounds", "sddmm_lists",
-                 "sddmm_uses", "rows", "blocked", "blocked_uses", "attention", "attention_uses")
+                 "sddmm_uses", "rows", "blocked", "blocked_uses", "attention", "attention_uses", "other_columns")
 
     def __init__(self, key, max_row: int, empty_rows: int, sorted_rows: bool = False, runs: int = 0):
         self.key = key
@@ -331,6 +331,31 @@ class CsrPlan:
         self.blocked_uses = 0                              # products that could have gone to the block kernels
         self.attention = None                              # BlockMask, False (blocks too thinly filled), None (not yet)
         self.attention_uses = 0                            # sparse_attention_csr calls
+        self.other_columns = None                          # (weak reference, stamp): column indices last multiplied over these rows
+
+
+def _plan_at_hand(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int) -> Optional[CsrPlan]:
+    """The plan of (pos, crd) if it has been made and both tensors are what they were."""
+    plan = getattr(pos, "_scorch_plan", None)
+    if plan is not None and plan.key == (_stamp(pos), _stamp(crd), n_rows, n_cols) and _same(plan.partner, crd):
+        return plan
+    return None
+
+
+def _plan_of_rows(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int) -> Optional[CsrPlan]:
+    """The plan of these unchanged row pointers with other column indices, for column indices that
+    come along for the first time: what it knows about rows holds for them too, and only their
+    range is open.  From their second product on they get a plan of their own."""
+    plan = getattr(pos, "_scorch_plan", None)
+    if plan is None or n_cols == 0 or crd.numel() == 0 or not plans_enabled() or torch.cuda.is_current_stream_capturing():
+        return None
+    (of_pos, of_crd, *sizes), stamp = plan.key, _stamp(crd)
+    if of_pos != _stamp(pos) or of_crd[3] != stamp[3] or sizes != [n_rows, n_cols]:
+        return None
+    if _same(plan.partner, crd):           # the plan's own column indices: as they were, or written to since
+        return None
+    seen, plan.other_columns = plan.other_columns, (weakref.ref(crd), stamp)
+    return None if seen is not None and _same(seen[0], crd) and seen[1] == stamp else plan
 
 
 def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, what: str = "operand") -> Optional[CsrPlan]:
@@ -340,12 +365,12 @@ def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, wha
     len(crd) or decrease, column indices outside [0, n_cols) -- before any
     kernel dereferences it.  None when planning is switched off or the stream
     is being captured (no synchronisation is possible there)."""
-    key = (_stamp(pos), _stamp(crd), n_rows, n_cols)
-    plan = getattr(pos, "_scorch_plan", None)
-    if plan is not None and plan.key == key and _same(plan.partner, crd):
+    plan = _plan_at_hand(pos, crd, n_rows, n_cols)
+    if plan is not None:
         return plan
     if not plans_enabled():
         return None
+    key = (_stamp(pos), _stamp(crd), n_rows, n_cols)
     if pos.numel() != n_rows + 1:
         raise ValueError(f"scorch_ops_hip: {what}: row pointer has {pos.numel()} entries, expected {n_rows + 1}")
     if torch.cuda.is_current_stream_capturing():
@@ -362,7 +387,7 @@ def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, wha
             problems.append(f"row_ptr must start at 0, never decrease and end at {crd.numel()}")
         if bad_cols:
             problems.append(f"a column index lies outside [0, {n_cols})")
-        raise ValueError(f"scorch_ops_hip: {what}: malformed CSR index: " + "; ".join(problems))
+        raise _malformed(what, problems)
     plan = CsrPlan(key, max_row, empty_rows, descents == 0, runs)
     plan.partner = weakref.ref(crd)
     try:
@@ -370,6 +395,10 @@ def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, wha
     except (AttributeError, RuntimeError):      # an object that takes no attributes: plan per call
         pass
     return plan
+
+
+def _malformed(what: str, problems) -> ValueError:
+    return ValueError(f"scorch_ops_hip: {what}: malformed CSR index: " + "; ".join(problems))
 
 
 def _chunk_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, N: int, elem: int, L, stream) -> torch.Tensor:
@@ -736,7 +765,39 @@ def _spmm(dtype, result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mod
         bias_ptr = bias.data_ptr()
     if SPMM_PATH not in SPMM_PATHS:
         raise ValueError(f"scorch_ops_hip: SPMM_PATH is {SPMM_PATH!r}, expected one of {SPMM_PATHS}")
+    if SPMM_PATH == "auto" and BLOCKED_PATH != "always" and M > 0 and N > 0:
+        rows = _plan_of_rows(pos, crd, M, K)
+        if rows is not None:
+            return _spmm_new_columns(rows, dtype, M, K, N, pos, crd, a_val, b_val, B_values, bias_ptr, act)
     plan = csr_plan(pos, crd, M, K, "A")
+    return _spmm_launch(plan, True, dtype, M, K, N, pos, crd, a_val, b_val, B_values, bias_ptr, act)
+
+
+def _spmm_new_columns(plan: CsrPlan, dtype, M, K, N, pos, crd, a_val, b_val, B_values, bias_ptr, act):
+    """A product with new column indices over row pointers that `plan` knows: the product is queued
+    behind the check of the columns' range (it reads a copy without columns out of range), and the
+    verdict is read while it runs."""
+    L, dev = native.lib(), pos.device
+    checked = _empty(crd.numel(), dtype=torch.int32, device=dev)
+    pending, outside = ctypes.c_void_p(), ctypes.c_int32(1)
+    with _on_device(dev):
+        native.check(L.scorch_hip_csr_columns_begin(K, crd.numel(), crd.data_ptr(), checked.data_ptr(), _stream(dev),
+                                                    ctypes.byref(pending)))
+        try:
+            result = _spmm_launch(plan, False, dtype, M, K, N, pos, checked, a_val, b_val, B_values, bias_ptr, act)
+        finally:
+            rc = L.scorch_hip_csr_columns_end(pending, ctypes.byref(outside))
+        native.check(rc)
+    if outside.value:
+        raise _malformed("A", [f"a column index lies outside [0, {K})"])
+    return result
+
+
+def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N, pos, crd, a_val, b_val, B_values,
+                 bias_ptr, act):
+    """Choose the kernel of a checked product and queue it.  `of_these_columns`: `plan` was made for
+    these column indices, not only for the row pointers."""
+    dev, nnz = pos.device, a_val.numel()
     out = _empty(M * N, dtype=dtype, device=dev)
     L = native.lib()
     suffix = _SUFFIX[dtype]
@@ -750,8 +811,8 @@ def _spmm(dtype, result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mod
             tiled = _tiled_operand(B_values, K, N, nnz, L)
         elif path == "tiled" and dtype == torch.float32:
             tiled = prepare_dense_operand(B_values, K, N)
-        fill_first = _fill_first(plan, M, N, elem, bias is not None)
-        if path == "auto" and tiled is None and dtype == torch.float32 and bias is None and act == 0:
+        fill_first = _fill_first(plan, M, N, elem, bias_ptr is not None)
+        if path == "auto" and of_these_columns and tiled is None and dtype == torch.float32 and bias_ptr is None and act == 0:
             bl = _blocked(plan, pos, crd, M, K, N)
             if bl is not None:
                 native.check(_blocked_spmm(L, bl, 1, M, K, N, nnz, a_val, b_val, out, stream))
@@ -811,7 +872,7 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
     M, K, nnz = int(a.shape[0]), int(a.shape[1]), vals.numel()
     if M == 0 or width == 0 or vals.dtype not in _SUFFIX:
         return
-    plan = csr_plan(pos, crd, M, K, "A")
+    plan = _plan_at_hand(pos, crd, M, K)
     if plan is None:
         return
     L, elem, dev, host = native.lib(), vals.element_size(), vals.device, native.host()

@@ -183,3 +183,41 @@ def test_vector_product_from_a_plans_boundaries(dtype, rows, entries):
     for _ in range(10):
         assert torch.equal(scorch.matmul(A, xd), got)
     assert all(int(c.abs().sum()) == 0 for c in H._counter_buffers.values())
+
+
+@pytest.mark.parametrize("rows, K, N, per_row", [(1, 1, 3, 1), (37, 50, 5, 7), (64, 500, 64, 300), (4096, 2048, 1024, 8)])
+def test_new_columns_under_known_row_pointers(rows, K, N, per_row):
+    """New column indices with every product, the same row pointers: each product is its own, a column out
+    of range is refused after any number of good ones (and leaves the next one alone), columns multiplied
+    a second time are planned, and a rewritten row pointer is looked at again."""
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    rp = torch.arange(0, rows * per_row + 1, per_row, dtype=torch.int32, device="cuda")
+    b = torch.randn(K, N, device="cuda", generator=gen)
+
+    def product(ci, vals):
+        return scorch.matmul(STensor.from_csr_arrays(rp, ci, vals, (rows, K)), b)
+
+    def check(ci, vals):
+        want = torch.zeros(rows, K, dtype=torch.float64)
+        at = torch.arange(rows).repeat_interleave(per_row)
+        want.index_put_((at, ci.long().cpu()), vals.double().cpu(), accumulate=True)
+        assert _close(product(ci, vals), want @ b.double().cpu(), np.float32)
+
+    for turn in range(6):
+        ci = torch.randint(K, (rows * per_row,), device="cuda", generator=gen, dtype=torch.int32 if turn % 2 else torch.int64)
+        vals = torch.randn(rows * per_row, device="cuda", generator=gen)
+        check(ci, vals)
+        if turn == 2:
+            for outside in (K, -1, 2**31 - 1):
+                bad = ci.to(torch.int32)
+                bad[-1] = outside
+                with pytest.raises(ValueError, match="column"):
+                    product(bad, vals)
+    first = rp._scorch_plan
+    ci = ci.to(torch.int32)
+    for _ in range(3):
+        check(ci, vals)
+    assert rp._scorch_plan is not first and H._plan_at_hand(rp, ci, rows, K) is rp._scorch_plan
+    rp[-1] += 1
+    with pytest.raises(ValueError, match="row_ptr"):
+        product(torch.zeros_like(ci), vals)
