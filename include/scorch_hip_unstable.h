@@ -95,9 +95,9 @@ SCORCH_HIP_API int scorch_hip_csr_inspect_now(int64_t M, int64_t K, int64_t nnz,
  * product over `checked` may be queued right behind it, and returns at once; _end waits for the
  * verdict -- *outside: whether a column was replaced, i.e. the product is not to be used -- and ends the call.
  * Every _begin that succeeded needs its _end.  Not for a stream that is being captured. */
-SCORCH_HIP_API int scorch_hip_csr_columns_begin(int64_t K, int64_t nnz, const int32_t *col_idx, int32_t *checked /* device, [nnz] */,
+SCORCH_HIP_API int scorch_hip_csr_inspect_columns_begin(int64_t K, int64_t nnz, const int32_t *col_idx, int32_t *checked /* device, [nnz] */,
                                     void *stream, void **pending);
-SCORCH_HIP_API int scorch_hip_csr_columns_end(void *pending, int32_t *outside);
+SCORCH_HIP_API int scorch_hip_csr_inspect_columns_end(void *pending, int32_t *outside);
 
 /* Row-split SpMM for matrices whose rows are all short: C = act(A * B + bias)
  * in one launch, without workspace (a team of lanes per row; no rows are cut,
@@ -182,6 +182,23 @@ SCORCH_HIP_API int scorch_hip_spmm_csr_tiled_f32(int64_t M, int64_t K, int64_t N
                                   const float *Bt, size_t bt_bytes, const float *bias, int act, float *C,
                                   const void *bounds, size_t bounds_bytes,
                                   void *workspace, size_t workspace_bytes, int64_t longest_row, void *stream);
+
+/* SpMM of a matrix of up to 10,239 columns whose rows are about equally long -- a sparse weight
+ * matrix -- with B by column panels in LDS: C = act(A * B + bias), bias NULL or of N elements.
+ * transposed: B is handed over as its transpose, N rows of K elements, and is read as it lies (the
+ * product W @ x.T of a layer, csrc/spmm.h:28-150 with the operand the reference copies first).
+ * Correct for rows of any length; bit-reproducible.
+ *   ..._rows_panels_recommended: whether this is the kernel to take; longest_row as scorch_hip_csr_inspect
+ *     reports it.
+ *   ..._rows_recommended: the same question for scorch_hip_spmm_csr_rows_<T> against the merge-path kernels.
+ *   ..._tiled_recommended: the same for scorch_hip_spmm_csr_tiled_f32, given that the tiled copy of B is there. */
+SCORCH_HIP_API int scorch_hip_spmm_csr_rows_panels_f32(int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,
+                                   const int32_t *col_idx, const float *vals, const float *B, int transposed,
+                                   const float *bias, int act, float *C, void *stream);
+SCORCH_HIP_API int scorch_hip_spmm_csr_rows_panels_recommended(int64_t M, int64_t K, int64_t N, int64_t nnz, int64_t longest_row,
+                                   int transposed);
+SCORCH_HIP_API int scorch_hip_spmm_csr_rows_recommended(int64_t M, int64_t nnz, int64_t longest_row);
+SCORCH_HIP_API int scorch_hip_spmm_csr_tiled_recommended(int64_t M, int64_t K, int64_t N, int64_t nnz);
 
 /* SDDMM for a CSR mask whose pattern is used again and again (an attention mask
  * serves every head, layer and step), with B larger than one of the GPU's eight

@@ -28,7 +28,7 @@ namespace {
 
 // ---- names and objects looked up once ---------------------------------------------------------
 PyObject *n_storage, *n_index, *n_value, *n_shape, *n_mode_indices, *n_format, *n_routes, *n_spmm_path, *n_blocked_path,
-    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_volatile, *n_epoch, *n_attention, *n_dtype, *n_device;
+    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_dtype, *n_device;
 PyObject *g_ops = nullptr;        // scorch_ops_hip's namespace
 PyObject *g_stensor = nullptr;    // the STensor type
 PyObject *g_torch_empty = nullptr;
@@ -70,7 +70,7 @@ bool unchanged(const Mark &m) {
   return t.const_data_ptr() == m.data && version_of(t) == m.version && t.numel() == m.numel;
 }
 
-enum Kind { kRows = 0, kPlanned = 1, kBlockedSpmm = 2, kSpmv = 3, kSddmmCsr = 4, kSddmmListed = 5, kSddmmCoo = 6, kBlockedSddmm = 7, kTiledOnly = 8 };
+enum Kind { kRows = 0, kPlanned = 1, kBlockedSpmm = 2, kSpmv = 3, kSddmmCsr = 4, kSddmmListed = 5, kSddmmCoo = 6, kBlockedSddmm = 7 };
 
 // One decided product: everything about the call that does not change from call to call.
 struct Route {
@@ -243,6 +243,24 @@ Route *find_route(Operand *o, int64_t width, int act) {
   return nullptr;
 }
 
+// Whether a dense operand without a column-tile copy is a new one: then it is marked as seen once, as
+// the general path does (its second product makes the copy), and this product goes without.
+bool first_sight(PyObject *b, int64_t K, int64_t N) {
+  PyObject *d = dict_of(b);
+  PyObject *volatile_ = item(d, n_volatile);
+  if (volatile_ && volatile_ != Py_False) return true;
+  if (item(d, n_seen) || item(d, n_tiled)) return false;
+  PyObject *epoch = item(d, n_epoch);
+  const at::Tensor &t = THPVariable_Unpack(b);
+  PyObject *stamp = Py_BuildValue("(kKLLl)", (unsigned long)version_of(t),
+                                  (unsigned long long)reinterpret_cast<uintptr_t>(t.const_data_ptr()), (long long)K, (long long)N,
+                                  epoch ? PyLong_AsLong(epoch) : 0L);
+  const bool marked = stamp && PyObject_SetAttr(b, n_seen, stamp) == 0;
+  Py_XDECREF(stamp);
+  if (!marked) PyErr_Clear();
+  return marked;
+}
+
 // The column-tile copy of a dense operand, if the operand carries a valid one.
 const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N) {
   PyObject *d = dict_of(b);
@@ -298,15 +316,15 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
   void *ws = nullptr, *counters = nullptr;
   size_t ws_bytes = 0, n_counted = 0;
   const at::Tensor *tiles = nullptr;
+  const bool panels = (r->kind == kRows || r->kind == kPlanned) && (r->p[4] & (transposed ? 2 : 1));
   if (r->workspace || r->may_tile) {
     if (capturing(stream)) return none();
-    if (r->may_tile) {
-      if (transposed) return none();
-      if (tiles_switched_off()) return none();
+    if (r->may_tile && !transposed && !tiles_switched_off()) {
       tiles = tile_copy(b, o->cols, N);
-      if (!tiles) return none();  // the general path counts the product and may make the copy
+      if (!tiles && !first_sight(b, o->cols, N)) return none();  // the general path makes the copy
+      if (!r->p[5]) tiles = nullptr;                             // (which is for other products of this operand)
     }
-    if (r->workspace && !(ws = workspace(o->device, stream, r->workspace, &ws_bytes))) return none();
+    if (r->workspace && (tiles || r->kind != kRows) && !(ws = workspace(o->device, stream, r->workspace, &ws_bytes))) return none();
     if ((r->kind == kPlanned || r->kind == kSpmv) && !(counters = workspace(o->device, stream, r->p[3], &n_counted, n_counters))) return none();
   }
   at::Tensor out;
@@ -314,14 +332,14 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const bool got = N >= 0 ? allocate(out, {M, N}, o->dtype, o->device, bt) : allocate(out, {M}, o->dtype, o->device, bt);
   if (!got) return nullptr;
   at::Tensor by_rows;  // (its memory goes back to torch's allocator for this stream when the call returns)
-  if (transposed) {
+  if (transposed && !panels) {
     if (!allocate(by_rows, {K, N}, o->dtype, o->device, bt)) return nullptr;
     const int rc = scorch_hip_dense_to_rows_f32(K, N, at_<float>(bt.const_data_ptr()),
                                                 static_cast<float *>(by_rows.mutable_data_ptr()), stream);
     if (rc != SCORCH_HIP_OK) return finished(rc, out);
   }
   const int32_t *pos = at_<int32_t>(r->row_ptr ? r->row_ptr : o->first.data), *crd = at_<int32_t>(o->second.data);
-  const void *v = vt.const_data_ptr(), *B = transposed ? by_rows.const_data_ptr() : bt.const_data_ptr();
+  const void *v = vt.const_data_ptr(), *B = transposed && !panels ? by_rows.const_data_ptr() : bt.const_data_ptr();
   void *C = out.mutable_data_ptr();
   const int flag = act == 2 ? 1 : 0;
   int rc = SCORCH_HIP_EINVAL;
@@ -337,6 +355,9 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
     rc = scorch_hip_spmm_csr_tiled_f32(M, K, N, nnz, pos, crd, at_<float>(v), at_<float>(tiles->const_data_ptr()),
                                        tiles->numel() * 4, at_<float>(bias_ptr), flag, static_cast<float *>(C), r->q[0],
                                        (size_t)r->p[0], ws, ws_bytes, r->p[2], stream);
+  } else if (panels) {
+    rc = scorch_hip_spmm_csr_rows_panels_f32(M, K, N, nnz, pos, crd, at_<float>(v), at_<float>(B), transposed, at_<float>(bias_ptr),
+                                        flag, static_cast<float *>(C), stream);
   } else if (r->kind == kRows) {
 #define SCORCH_CALL(S, T)                                                                                      \
   scorch_hip_spmm_csr_rows_##S(M, K, N, nnz, pos, crd, at_<T>(v), at_<T>(B), at_<T>(bias_ptr), flag,           \
@@ -673,7 +694,7 @@ PyMODINIT_FUNC PyInit__host() {
   } names[] = {{&n_storage, "_storage"}, {&n_index, "_index"}, {&n_value, "_value"}, {&n_shape, "_shape"},
                {&n_mode_indices, "mode_indices"}, {&n_format, "format"}, {&n_routes, "_routes"},
                {&n_spmm_path, "SPMM_PATH"}, {&n_blocked_path, "BLOCKED_PATH"}, {&n_sddmm_path, "SDDMM_PATH"},
-               {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_counters, "_counter_buffers"}, {&n_tiled, "_scorch_tiled"},
+               {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_counters, "_counter_buffers"}, {&n_tiled, "_scorch_tiled"}, {&n_seen, "_scorch_seen"},
                {&n_volatile, "_scorch_volatile"}, {&n_epoch, "_scorch_epoch"}, {&n_attention, "_scorch_attention"},
                {&n_dtype, "dtype"}, {&n_device, "device"}};
   for (const auto &x : names) *x.slot = PyUnicode_InternFromString(x.text);

@@ -20,6 +20,7 @@ hipError_t preload_misc();
 hipError_t preload_sddmm();
 hipError_t preload_spgemm();
 hipError_t preload_spmm();
+hipError_t preload_spmm_panels();
 hipError_t preload_spmm_rows();
 hipError_t preload_spmm_tiled();
 hipError_t preload_sync();
@@ -28,7 +29,6 @@ hipError_t preload_sync();
 namespace {
 
 constexpr int kPlanWidths = 8;              // chunk boundaries kept for this many values of N
-constexpr int64_t kRowsKernelMaxRow = 256;  // longest row the row-split kernel is chosen for
 constexpr int64_t kSoftmaxShortRow = 4096;  // rows up to this length: the one-launch softmax
 constexpr int64_t kFillFirstBytes = (int64_t)32 << 20;
 constexpr int64_t kListsMinDense = (int64_t)8 << 20, kListsMaxDense = (int64_t)20 << 20;
@@ -106,7 +106,11 @@ bool spmm_fills_first(const scorch_hip_csr_plan *plan, int64_t N, bool has_bias)
 }
 bool spmm_by_rows(const scorch_hip_csr_plan *plan, int64_t N, bool has_bias) {
   return plan->M == 0 || N == 0 ||
-         (!spmm_fills_first(plan, N, has_bias) && plan->longest_row() <= kRowsKernelMaxRow);
+         (!spmm_fills_first(plan, N, has_bias) && scorch_hip_spmm_csr_rows_recommended(plan->M, plan->nnz, plan->longest_row()));
+}
+
+bool spmm_by_panels(const scorch_hip_csr_plan *plan, int64_t N) {
+  return scorch_hip_spmm_csr_rows_panels_recommended(plan->M, plan->n_cols, N, plan->nnz, plan->longest_row(), 0) != 0;
 }
 
 // Boundaries and workspace of the merge-path kernels for dense width N (nothing for a product
@@ -182,7 +186,7 @@ extern "C" {
 int scorch_hip_init(void) {
   hipError_t (*const loaders[])() = {scorch::preload_attn,      scorch::preload_attn_f32, scorch::preload_blockdesc,
                                      scorch::preload_blocked,   scorch::preload_misc,     scorch::preload_sddmm,
-                                     scorch::preload_spgemm,    scorch::preload_spmm,     scorch::preload_spmm_rows,
+                                     scorch::preload_spgemm,    scorch::preload_spmm,     scorch::preload_spmm_rows, scorch::preload_spmm_panels,
                                      scorch::preload_spmm_tiled, scorch::preload_sync};
   for (auto load : loaders) SCORCH_HIP_CHECK(load());
   return SCORCH_HIP_OK;
@@ -278,6 +282,9 @@ int scorch_hip_spmm_csr_plan_f32(scorch_hip_csr_plan *plan, int64_t N, const flo
   if (act != SCORCH_HIP_ACT_NONE && act != SCORCH_HIP_ACT_RELU)
     return fail(SCORCH_HIP_EINVAL, "scorch_hip_spmm_csr_plan_f32: act %d is not a scorch_hip_act", act);
   if (N < 0) return fail(SCORCH_HIP_EINVAL, "scorch_hip_spmm_csr_plan_f32: negative N");
+  if (spmm_by_panels(plan, N))
+    return scorch_hip_spmm_csr_rows_panels_f32(plan->M, plan->n_cols, N, plan->nnz, plan->row_ptr, plan->col_idx, vals, B, 0,
+                                          bias, act, C, stream);
   if (spmm_by_rows(plan, N, bias != nullptr))
     return scorch_hip_spmm_csr_rows_f32(plan->M, plan->n_cols, N, plan->nnz, plan->row_ptr, plan->col_idx, vals, B,
                                         bias, act, C, stream);
@@ -383,7 +390,7 @@ int scorch_hip_spmm_csr_plan_dense_f32(scorch_hip_csr_plan *plan, const float *v
                 fn, (long long)dense->K, (long long)dense->N, dense->device, (long long)plan->M,
                 (long long)plan->n_cols, plan->device);
   const int64_t N = dense->N;
-  if (!dense->tiles || plan->M == 0 || !scorch_hip_dense_tiled_recommended(dense->K, N, plan->nnz, 4))
+  if (!dense->tiles || plan->M == 0 || !scorch_hip_spmm_csr_tiled_recommended(plan->M, dense->K, N, plan->nnz))
     return scorch_hip_spmm_csr_plan_f32(plan, N, vals, dense->B, bias, act, C, stream);
   Boundaries *bounds = nullptr;
   if (int rc = prepare_spmm(plan, N, static_cast<hipStream_t>(stream), &bounds, true)) return rc;

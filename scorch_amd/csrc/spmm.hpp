@@ -257,12 +257,30 @@ inline int64_t spmm_num_chunks(int64_t M, int64_t nnz, int64_t N, size_t elem) {
   return (M + nnz + sp.items_per_chunk - 1) / sp.items_per_chunk;
 }
 
+// The tiled kernel's split (spmm_tiled.hip): one chunk for every wavefront of a resident grid, if the
+// chunks are small enough for that; a chunk is then staged once for all tiles.  512 chunks are four
+// wavefronts to each of an XCD's 128 SIMDs, 768 six (what its registers allow); other numbers leave
+// some CUs with one workgroup more than others, and the XCD waits for them in every tile (528 chunks 0.190 ms, 512
+// 0.158 on the decoder shape).  Few items make short chunks: 512 rows of 32, N = 4,096, 64 -> 28 us, 4,096 rows of 64
+// of 16,384, N = 512, 172 -> 31.  (spans 0: the shape does not split this way.)
+constexpr int kTiledItemsMax = 384;
+inline SpmmSplit tiled_split(int64_t M, int64_t nnz, int64_t N, size_t elem) {
+  for (const int64_t wavefronts : {512, 768}) {
+    int64_t items = (M + nnz + wavefronts - 1) / wavefronts;
+    if (items > kTiledItemsMax || N * (int64_t)elem < 2048 || wavefronts * N * (int64_t)elem > ((int64_t)64 << 20)) continue;
+    if (items < 16) items = 16;
+    return {(int)items, kSnapItems, (M + nnz + items - 1) / items};
+  }
+  return {0, 0, 0};
+}
+
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Workspace layout: carry_row int32[num_chunks] padded to 256 bytes, then
 // carry_val T[num_chunks * N] padded likewise.
 inline size_t spmm_workspace_bytes(int64_t M, int64_t nnz, int64_t N, size_t elem) {
-  const size_t chunks = (size_t)spmm_num_chunks(M, nnz, N, elem);
+  const size_t usual = (size_t)spmm_num_chunks(M, nnz, N, elem), tiled = (size_t)tiled_split(M, nnz, N, elem).spans;
+  const size_t chunks = usual > tiled ? usual : tiled;
   return align_up(chunks * sizeof(int), 256) + align_up(chunks * (size_t)N * elem, 256);
 }
 
@@ -404,6 +422,27 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_fixup_kernel(
       *dst = o;
     }
   }
+}
+
+// ---- which kernel: estimates in microseconds --------------------------------------------------------
+// Fitted to 70 shapes between 256 x 1,024 and 8,192 x 8,192, 8 to 800 entries a row, N = 32 to 4,096, on
+// which they are within a third; kernels that differ by less than that are close to each other anyway.
+//
+// The row-split kernel: what the L2s hand out, 21 TB/s while the K rows of a column tile (1 KiB) fit one
+// of them, 9.5 when most gathers miss.
+inline double spmm_rows_us(int64_t M, int64_t K, int64_t N, int64_t nnz) {
+  const double slice = (double)K * (double)(N * 4 < 1024 ? N * 4 : 1024) / (1 << 20);
+  return 2.5 + (double)nnz * (double)N * 4 / (slice <= 4 ? 21e6 : slice <= 8 ? 15e6 : 9.5e6) + (double)M * (double)N * 4 / 4e6;
+}
+// Turning a transposed operand first, and reading it from memory rather than the L2s after that.
+inline double dense_turn_us(int64_t K, int64_t N) {
+  const double us = 4.5 + (double)K * (double)N * 4 / 0.7e6;
+  return us < 12 ? us : 12;
+}
+// The tiled kernel: an XCD's tiles one after the other.
+inline double spmm_tiled_us(int64_t K, int64_t N, int64_t nnz) {
+  const int64_t rounds = ((N * 4 + 127) / 128 + 7) / 8;
+  return 2.5 + (double)rounds * (1.0 + (double)nnz * 128 / (K <= 4096 ? 4.2e6 : 3.3e6));
 }
 
 }  // namespace scorch

@@ -34,7 +34,6 @@ namespace scorch {
 constexpr int kTileBytes = 128;                // bytes of one row of a column tile
 constexpr int64_t kTiledSliceMax = 3 << 20;    // K * kTileBytes must fit an L2 beside A
 constexpr int kTiledGroupRowMax = 64;          // longer in-chunk rows are shared by all groups
-constexpr int kTiledItemsMax = 320;            // most merge items per chunk (the split may exceed the usual 256)
 // A chunk stages what lies between its two boundaries, and its end may move forward by up to
 // kSnapItems items to a row's end (chunk_boundary), so a wavefront's staging arrays hold this many.
 constexpr int kTiledSlots = kTiledItemsMax + kSnapItems;
@@ -148,10 +147,16 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
         for (int v = 0; v < VEC; ++v) acc[v] += a * (A)b.v[v];
       };
 
-      // Row slot r is row x0 + r; slot n_rows is the row that continues past the chunk.
-      for (int base = 0; base <= n_rows; base += G) {
-        const int slot = base + g;
-        const bool live = slot <= n_rows;
+      // Row slot r is row x0 + r; slot n_rows is the row that continues past the chunk, if one does.
+      // With fewer slots than lane groups several groups take a row, every 2nd, 4th or 8th entry each.
+      const int n_slots = n_rows + (y1 > uniform(s_rp[w][n_rows]));
+      int team_shift = 0;
+      while (team_shift < 3 && (n_slots << (team_shift + 1)) <= G) ++team_shift;
+      const int team = 1 << team_shift, sub = g & (team - 1);
+      if (n_slots == n_rows && tile == 0 && lane == 0) carry_row[span] = -1;
+      for (int base = 0; base < n_slots; base += G >> team_shift) {
+        const int slot = base + (g >> team_shift);
+        const bool live = slot < n_slots;
         int lo = 0, hi = 0;
         if (live) {
           const int begin = s_rp[w][slot], end = s_rp[w][slot + 1];
@@ -164,26 +169,33 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
 #pragma unroll
         for (int v = 0; v < VEC; ++v) acc[v] = (A)0;
 
-        if (len <= kTiledGroupRowMax) {
-          int k = lo;
-          for (; k + kTiledBatch <= hi; k += kTiledBatch) {
+        auto walk = [&](int k, int step, int last) {  // entries k, k + step, ... below `last`
+          for (; k + (kTiledBatch - 1) * step < last; k += kTiledBatch * step) {
             VecT b[kTiledBatch];
             A a[kTiledBatch];
 #pragma unroll
             for (int u = 0; u < kTiledBatch; ++u) {
-              a[u] = (A)s_val[w][k + u];
-              b[u] = *reinterpret_cast<const VecT *>(slice + ((unsigned)s_col[w][k + u] + lane_bytes));
+              a[u] = (A)s_val[w][k + u * step];
+              b[u] = *reinterpret_cast<const VecT *>(slice + ((unsigned)s_col[w][k + u * step] + lane_bytes));
             }
 #pragma unroll
             for (int u = 0; u < kTiledBatch; ++u)
 #pragma unroll
               for (int v = 0; v < VEC; ++v) acc[v] += a[u] * (A)b[u].v[v];
           }
-          for (; k < hi; ++k) add_entry(acc, k);
+          for (; k < last; k += step) add_entry(acc, k);
+        };
+        if (team_shift > 0) {
+          walk(lo + sub, team, hi);
+          for (int off = LPR; off < LPR << team_shift; off <<= 1)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) acc[v] += (A)__shfl_xor((T)acc[v], off);
+        } else if (len <= kTiledGroupRowMax) {
+          walk(lo, 1, hi);
         }
 
         // Rows with many entries in the chunk: one at a time, all groups.
-        unsigned long long pending = __ballot(len > kTiledGroupRowMax && t == 0);
+        unsigned long long pending = __ballot(team_shift == 0 && len > kTiledGroupRowMax && t == 0);
         while (pending) {
           const int owner_lane = __ffsll(pending) - 1;  // lane 0 of the owning group
           pending &= pending - 1;
@@ -202,7 +214,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
           }
         }
 
-        if (live && active) {
+        if (live && active && sub == 0) {
           const bool whole_row = slot < n_rows;
           if (whole_row || len > 0) {
             const bool partial = !whole_row || (carry_in && slot == 0);
@@ -221,7 +233,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
             }
           }
         }
-        if (live && slot == n_rows && tile == 0 && t == 0) carry_row[span] = len > 0 ? x1 : -1;
+        if (live && slot == n_rows && tile == 0 && t == 0 && sub == 0) carry_row[span] = len > 0 ? x1 : -1;
       }
     }
   }
@@ -255,19 +267,10 @@ int spmm_tiled_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nn
   SCORCH_REQUIRE(aligned_to(workspace, 256), "%s: workspace must be 256-byte aligned", fn);
   SpmmSplit split = spmm_split(M, nnz, N, sizeof(T));
   const Boundary *bounds = static_cast<const Boundary *>(bounds_buffer);
-  // When every wavefront gets one chunk anyway (the whole grid is resident), cut the work into a
-  // multiple of 128 chunks, i.e. the same number of wavefronts for each of an XCD's 128 SIMDs:
-  // 528 chunks of 256 items leave some CUs with five workgroups and others with four, and the
-  // XCD then waits for the fuller ones in every tile (0.190 against 0.158 ms with 512 chunks of
-  // 264 items on the decoder shape).  Boundaries computed for the usual split do not apply then.
-  if (split.spans > 128 && split.spans <= (int64_t)kTiledMaxWorkgroupsPerXcd * kWavesPerBlock) {
-    const int64_t even = split.spans / 128 * 128;
-    const int64_t ipc = (M + nnz + even - 1) / even;
-    if (even != split.spans && ipc <= kTiledItemsMax) {
-      split.items_per_chunk = (int)ipc;
-      split.spans = (M + nnz + ipc - 1) / ipc;
-      bounds = nullptr;
-    }
+  // (One chunk to a wavefront: its boundaries are looked for once, so none computed beforehand are needed.)
+  if (const SpmmSplit resident = tiled_split(M, nnz, N, sizeof(T)); resident.spans > 0) {
+    split = resident;
+    bounds = nullptr;
   }
   if (split.items_per_chunk + split.snap > kTiledSlots)
     return fail(SCORCH_HIP_ERUNTIME, "%s: chunks of %d + %d items exceed the %d staging slots", fn,
@@ -321,6 +324,12 @@ int scorch_hip_dense_tiled_recommended(int64_t K, int64_t N, int64_t nnz, size_t
   // are gathered more than once on average
   return N * (int64_t)elem_size >= 16 * scorch::kTileBytes && K * scorch::kTileBytes <= scorch::kTiledSliceMax &&
          nnz >= 2 * K;
+}
+
+int scorch_hip_spmm_csr_tiled_recommended(int64_t M, int64_t K, int64_t N, int64_t nnz) {
+  // several chunks to a wavefront are staged again in every tile: 20,000 rows of 20 at N = 512 take 127 us, 98 row by row
+  return scorch_hip_dense_tiled_recommended(K, N, nnz, 4) && scorch::tiled_split(M, nnz, N, 4).spans > 0 &&
+         scorch::spmm_tiled_us(K, N, nnz) < scorch::spmm_rows_us(M, K, N, nnz);
 }
 
 int scorch_hip_dense_to_tiled_f32(int64_t K, int64_t N, const float *B, float *Bt, size_t bt_bytes,

@@ -91,8 +91,13 @@ SIGNATURES = {
     **{"scorch_hip_spmv_csr_planned_" + t: (ctypes.c_int, [_i64] * 3 + [_ptr] * 6 + [_size, _ptr, _size, _ptr, _i64, _ptr])
        for t in ("f32", "f64", "i32", "i64")},
     "scorch_hip_dense_to_rows_f32": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr]),
-    "scorch_hip_csr_columns_begin": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr, ctypes.POINTER(_ptr)]),
-    "scorch_hip_csr_columns_end": (ctypes.c_int, [_ptr, ctypes.POINTER(ctypes.c_int32)]),
+    "scorch_hip_csr_inspect_columns_begin": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr, ctypes.POINTER(_ptr)]),
+    "scorch_hip_csr_inspect_columns_end": (ctypes.c_int, [_ptr, ctypes.POINTER(ctypes.c_int32)]),
+    "scorch_hip_spmm_csr_rows_panels_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, ctypes.c_int, _ptr,
+                                                      ctypes.c_int, _ptr, _ptr]),
+    "scorch_hip_spmm_csr_rows_panels_recommended": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, ctypes.c_int]),
+    "scorch_hip_spmm_csr_rows_recommended": (ctypes.c_int, [_i64, _i64, _i64]),
+    "scorch_hip_spmm_csr_tiled_recommended": (ctypes.c_int, [_i64, _i64, _i64, _i64]),
     "scorch_hip_csr_inspect_now": (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, ctypes.POINTER(ctypes.c_int32), _ptr]),
     "scorch_hip_sddmm_coo_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,
                                                 _ptr, _ptr]),

@@ -293,7 +293,7 @@ def plans_enabled() -> bool:
     return os.environ.get("SCORCH_HIP_PLAN", "1") not in ("", "0")
 
 
-ROWS_KERNEL_MAX_ROW = 256   # longest row for which the row-split kernel is chosen
+ROWS_KERNEL_MAX_ROW = 256   # longest row for which the row-split kernel is chosen whatever the others' lengths
 
 # Which SpMM kernel serves a product.  "auto" (the default; SCORCH_HIP_SPMM_PATH
 # overrides it at import) decides from the operand's plan; the other values pin one
@@ -781,12 +781,12 @@ def _spmm_new_columns(plan: CsrPlan, dtype, M, K, N, pos, crd, a_val, b_val, B_v
     checked = _empty(crd.numel(), dtype=torch.int32, device=dev)
     pending, outside = ctypes.c_void_p(), ctypes.c_int32(1)
     with _on_device(dev):
-        native.check(L.scorch_hip_csr_columns_begin(K, crd.numel(), crd.data_ptr(), checked.data_ptr(), _stream(dev),
+        native.check(L.scorch_hip_csr_inspect_columns_begin(K, crd.numel(), crd.data_ptr(), checked.data_ptr(), _stream(dev),
                                                     ctypes.byref(pending)))
         try:
             result = _spmm_launch(plan, False, dtype, M, K, N, pos, checked, a_val, b_val, B_values, bias_ptr, act)
         finally:
-            rc = L.scorch_hip_csr_columns_end(pending, ctypes.byref(outside))
+            rc = L.scorch_hip_csr_inspect_columns_end(pending, ctypes.byref(outside))
         native.check(rc)
     if outside.value:
         raise _malformed("A", [f"a column index lies outside [0, {K})"])
@@ -809,6 +809,8 @@ def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N
         tiled = None
         if path == "auto":
             tiled = _tiled_operand(B_values, K, N, nnz, L)
+            if tiled is not None and not L.scorch_hip_spmm_csr_tiled_recommended(M, K, N, nnz):
+                tiled = None
         elif path == "tiled" and dtype == torch.float32:
             tiled = prepare_dense_operand(B_values, K, N)
         fill_first = _fill_first(plan, M, N, elem, bias_ptr is not None)
@@ -817,8 +819,13 @@ def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N
             if bl is not None:
                 native.check(_blocked_spmm(L, bl, 1, M, K, N, nnz, a_val, b_val, out, stream))
                 return Tensor(out, [[], []])
+        if tiled is None and path == "auto" and plan is not None and dtype == torch.float32 and \
+                L.scorch_hip_spmm_csr_rows_panels_recommended(M, K, N, nnz, plan.max_row, 0):
+            native.check(L.scorch_hip_spmm_csr_rows_panels_f32(M, K, N, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(),
+                                                          b_val.data_ptr(), 0, bias_ptr, act, out.data_ptr(), stream))
+            return Tensor(out, [[], []])
         if tiled is None and (path == "rows" or (path == "auto" and plan is not None and not fill_first
-                                                 and plan.max_row <= ROWS_KERNEL_MAX_ROW)):
+                                                 and L.scorch_hip_spmm_csr_rows_recommended(M, nnz, plan.max_row))):
             # every row is short: one launch of the row-split kernel, no workspace
             rc = getattr(L, "scorch_hip_spmm_csr_rows_" + suffix)(
                 M, K, N, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(), b_val.data_ptr(), bias_ptr, act,
@@ -847,7 +854,7 @@ def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N
 
 # What the native call path does with a decided product (the enum Kind of csrc/host.cpp)
 _ROUTE_ROWS, _ROUTE_PLANNED, _ROUTE_BLOCKED_SPMM, _ROUTE_SPMV, _ROUTE_SDDMM_CSR, _ROUTE_SDDMM_LISTED, _ROUTE_SDDMM_COO, \
-    _ROUTE_BLOCKED_SDDMM, _ROUTE_TILED = range(9)
+    _ROUTE_BLOCKED_SDDMM = range(8)
 
 
 def remember_spmm(a, width: int, act: int = 0) -> None:
@@ -892,7 +899,6 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
             remember(_ROUTE_SPMV, (bounds.numel(), 0, 0, counters), (bounds,),
                      L.scorch_hip_spmv_csr_workspace_bytes(M, nnz, elem))
         return
-    may_tile = width >= 512 and vals.dtype == torch.float32 and bool(L.scorch_hip_dense_tiled_recommended(K, width, nnz, 4))
     if act == 0 and vals.dtype == torch.float32 and BLOCKED_PATH != "off" and width in BLOCKED_WIDTHS:
         if plan.blocked is None:
             return
@@ -902,18 +908,24 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
                      (bl.block_col_idx, bl.block_words, bl.block_off, bl.block_cols, bl.spmm_items, bl.spmm_split_rows),
                      L.scorch_hip_spmm_csr_blocked_workspace_bytes(1, bl.n_spmm_slots, width) if bl.n_spmm_slots else 0)
             return
+    fp32 = vals.dtype == torch.float32
     fill_first = _fill_first(plan, M, width, elem, act != 0)
-    if not may_tile and not fill_first and plan.max_row <= ROWS_KERNEL_MAX_ROW:
-        remember(_ROUTE_ROWS)
+    # the dense operand may have, or get, a column-tile copy, and this product may read that; or it is taken by
+    # panels in LDS, as it lies (1) or handed over as its transpose (2)
+    may_tile = fp32 and bool(L.scorch_hip_dense_tiled_recommended(K, width, nnz, 4))
+    tiles = may_tile and L.scorch_hip_spmm_csr_tiled_recommended(M, K, width, nnz)
+    panels = sum(bit for bit, turned in ((1, 0), (2, 1))
+                 if fp32 and L.scorch_hip_spmm_csr_rows_panels_recommended(M, K, width, nnz, plan.max_row, turned))
+    workspace = L.scorch_hip_spmm_csr_workspace_bytes(M, nnz, width, elem)
+    if not fill_first and L.scorch_hip_spmm_csr_rows_recommended(M, nnz, plan.max_row):
+        remember(_ROUTE_ROWS, (0, 0, plan.max_row, 0, panels, tiles), (), workspace if may_tile else 0, may_tile)
         return
     counters = L.scorch_hip_spmm_csr_planned_counters(1, M, nnz, width, elem)
     with _on_device(dev):
         bounds = _chunk_bounds(plan, pos, M, nnz, width, elem, L, _stream(dev))
-        if not may_tile:
-            _counters(dev, _stream(dev), counters)
-    remember(_ROUTE_TILED if may_tile else _ROUTE_PLANNED,
-             (bounds.numel(), HINT_MOSTLY_EMPTY_ROWS if fill_first else 0, plan.max_row, counters), (bounds,),
-             L.scorch_hip_spmm_csr_workspace_bytes(M, nnz, width, elem), may_tile)
+        _counters(dev, _stream(dev), counters)
+    remember(_ROUTE_PLANNED, (bounds.numel(), HINT_MOSTLY_EMPTY_ROWS if fill_first else 0, plan.max_row, counters, panels, tiles),
+             (bounds,), workspace, may_tile)
 
 
 def _fill_first(plan: Optional[CsrPlan], M: int, N: int, elem: int, with_bias: bool) -> bool:
@@ -1574,7 +1586,8 @@ def spmm_csr_float_batched(A_shape, A_mode_indices, A_values: torch.Tensor, B: t
         bl = _blocked(plan, pos, crd, M, K, N) if SPMM_PATH == "auto" else None
         if bl is not None:
             rc = _blocked_spmm(L, bl, H, M, K, N, nnz, a_val, b, out, stream)
-        elif SPMM_PATH == "rows" or (SPMM_PATH == "auto" and plan is not None and plan.max_row <= ROWS_KERNEL_MAX_ROW):
+        elif SPMM_PATH == "rows" or (SPMM_PATH == "auto" and plan is not None and
+                                    L.scorch_hip_spmm_csr_rows_recommended(M, nnz, plan.max_row)):
             rc = L.scorch_hip_spmm_csr_rows_batched_f32(H, M, K, N, nnz, pos.data_ptr(), crd.data_ptr(),
                                                         a_val.data_ptr(), b.data_ptr(), out.data_ptr(), stream)
         else:

@@ -466,3 +466,52 @@ def test_direct_calls_on_a_large_square_like_the_references_perf_test():
         assert torch.allclose(result.cpu().view_as(reference), reference, atol=1e-3, rtol=1e-3), name
     out = scorch.matmul(a, b)
     assert torch.allclose(out.cpu(), reference, atol=1e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("M, K, N, per_row", [(1, 1, 1, 1), (3, 40, 33, 20), (17, 5000, 7, 100), (40, 10_239, 9, 300), (33, 1247, 64, 65),
+                                             (70, 1300, 61, 64), (1040, 2500, 40, 30), (257, 200, 1000, 129)])
+@pytest.mark.parametrize("transposed", [0, 1])
+def test_panels_of_the_dense_operand_in_lds(oracle, M, K, N, per_row, transposed):
+    """Every panel width (K decides), a ragged last panel, fewer rows than wavefronts and more than 64 to a
+    wavefront, empty rows and rows of several batches, a bias with and without ReLU; the operand as it
+    lies and as its transpose: against fp64, and the same bits again."""
+    from scorch_amd import native
+    rng = np.random.default_rng(M + N)
+    lens = np.clip(rng.integers(per_row // 2, per_row + per_row // 2 + 1, M), 0, K)
+    if M > 16:
+        lens[[0, M // 2]], lens[M - 1] = 0, K
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = np.concatenate([np.sort(rng.choice(K, n, replace=False)) for n in lens]).astype(np.int32)
+    v = rng.uniform(-1, 1, ci.size).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    want = oracle.spmm_fp64(rp, ci, v, B)
+    d_rp, d_ci, d_v, d_bias, d_B = dev(rp), dev(ci), dev(v), dev(bias), dev(np.ascontiguousarray(B.T) if transposed else B)
+    L = native.lib()
+    for with_bias, relu in ((False, 0), (True, 0), (True, 1)):
+        outs = []
+        for _ in range(2):
+            out = torch.full((M, N), float("nan"), device="cuda")
+            native.check(L.scorch_hip_spmm_csr_rows_panels_f32(
+                M, K, N, ci.size, d_rp.data_ptr(), d_ci.data_ptr(), d_v.data_ptr(), d_B.data_ptr(), transposed,
+                d_bias.data_ptr() if with_bias else None, relu, out.data_ptr(), torch.cuda.current_stream().cuda_stream))
+            outs.append(host(out))
+        expect = want + bias if with_bias else want
+        assert oracle.rel_fro(outs[0], np.maximum(expect, 0) if relu else expect) <= 1e-5
+        assert np.array_equal(*outs)
+    assert L.scorch_hip_spmm_csr_rows_panels_recommended(M, 20_000, N, ci.size, per_row, transposed) == 0   # no panel fits
+
+
+@pytest.mark.parametrize("M, K, per_row", [(2, 900, 900), (100, 64, 33), (512, 1024, 64), (520, 1024, 65), (4096, 2000, 64), (3000, 2000, 70)])
+def test_tiled_kernel_with_several_lane_groups_to_a_row(oracle, M, K, per_row):
+    """Chunks of one, two and four rows (eight, four and two lane groups to each), rows that end at a chunk's
+    end and rows cut by it, 512 and 768 chunks."""
+    rng = np.random.default_rng(M)
+    N = 520
+    rp = (np.arange(M + 1) * per_row).astype(np.int32)
+    ci = rng.integers(0, K, M * per_row).astype(np.int32)
+    v = rng.uniform(-1, 1, ci.size).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    got = hip_spmm(rp, ci, v, B, path="tiled")
+    assert oracle.rel_fro(got, oracle.spmm_fp64(rp, ci, v, B)) <= 1e-5
+    assert np.array_equal(got, hip_spmm(rp, ci, v, B, path="tiled"))
