@@ -413,38 +413,62 @@ SCORCH_HIP_API int scorch_hip_values_differ_f32(int64_t n, const float *vals, fl
                                  int32_t *differ /* device */, void *stream);
 
 /* ------------------------------------------------------------------------
- * SpGEMM whose two passes share what the first found out: _symbolic_planned is
- * scorch_hip_spgemm_csr_symbolic and returns with `report` (host memory, 7 words: entries of the
- * result or -1 for 2^31 and more, then the numbers of rows per tier) filled in, which takes the
- * place of the caller's read of c_row_ptr[M]; _numeric_planned_<T> takes that report and the SAME
- * workspace, unchanged in between, reads the row lists from it and launches only what has rows.
+ * SpGEMM whose two passes share what the first found out.  _symbolic_planned_begin counts the
+ * products of every row, lists the rows by size, queues the short rows' counting and returns with
+ * `report` (host memory, 9 words) partly filled in and with the bytes of memory that the long rows'
+ * products take, sorted by ranges of columns: *bin_bytes, 0 where they are not sorted (no such rows,
+ * more than 131,072 columns, or more than 4 GiB).  _symbolic_planned_<T> counts the long rows, in
+ * `bins` (256-byte aligned, NULL: the other way), makes c_row_ptr, and completes the report: word 0
+ * is the number of entries of the result or -1 for 2^31 and more, which takes the place of the
+ * caller's read of c_row_ptr[M].  _numeric_planned_<T> takes that report and the SAME workspace and
+ * bins, unchanged in between, and launches only what has rows.
  * Not for a stream that is being captured.
  * ---------------------------------------------------------------------- */
-#define SCORCH_HIP_SPGEMM_REPORT_WORDS 7
-SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+#define SCORCH_HIP_SPGEMM_REPORT_WORDS 9
+SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned_begin(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
                                    const int32_t *a_col_idx, const int32_t *b_row_ptr, const int32_t *b_col_idx,
-                                   int32_t *c_row_ptr, void *workspace, size_t workspace_bytes, int64_t *report,
-                                   void *stream);
+                                   int32_t *c_row_ptr, void *workspace, size_t workspace_bytes, size_t elem_size,
+                                   int64_t *report, size_t *bin_bytes, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned_f32(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const float *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const float *b_vals, int32_t *c_row_ptr,
+                                   void *workspace, size_t workspace_bytes, void *bins, size_t bin_bytes,
+                                   int64_t *report, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned_f64(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const double *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const double *b_vals, int32_t *c_row_ptr,
+                                   void *workspace, size_t workspace_bytes, void *bins, size_t bin_bytes,
+                                   int64_t *report, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned_i32(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const int32_t *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const int32_t *b_vals, int32_t *c_row_ptr,
+                                   void *workspace, size_t workspace_bytes, void *bins, size_t bin_bytes,
+                                   int64_t *report, void *stream);
+SCORCH_HIP_API int scorch_hip_spgemm_csr_symbolic_planned_i64(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                   const int32_t *a_col_idx, const int64_t *a_vals, const int32_t *b_row_ptr,
+                                   const int32_t *b_col_idx, const int64_t *b_vals, int32_t *c_row_ptr,
+                                   void *workspace, size_t workspace_bytes, void *bins, size_t bin_bytes,
+                                   int64_t *report, void *stream);
 SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_f32(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
                                    const int32_t *a_col_idx, const float *a_vals, const int32_t *b_row_ptr,
                                    const int32_t *b_col_idx, const float *b_vals, const int32_t *c_row_ptr,
                                    int32_t *c_col_idx, float *c_vals, void *workspace, size_t workspace_bytes,
-                                   const int64_t *report, void *stream);
+                                   void *bins, size_t bin_bytes, const int64_t *report, void *stream);
 SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_f64(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
                                    const int32_t *a_col_idx, const double *a_vals, const int32_t *b_row_ptr,
                                    const int32_t *b_col_idx, const double *b_vals, const int32_t *c_row_ptr,
                                    int32_t *c_col_idx, double *c_vals, void *workspace, size_t workspace_bytes,
-                                   const int64_t *report, void *stream);
+                                   void *bins, size_t bin_bytes, const int64_t *report, void *stream);
 SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_i32(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
                                    const int32_t *a_col_idx, const int32_t *a_vals, const int32_t *b_row_ptr,
                                    const int32_t *b_col_idx, const int32_t *b_vals, const int32_t *c_row_ptr,
                                    int32_t *c_col_idx, int32_t *c_vals, void *workspace, size_t workspace_bytes,
-                                   const int64_t *report, void *stream);
+                                   void *bins, size_t bin_bytes, const int64_t *report, void *stream);
 SCORCH_HIP_API int scorch_hip_spgemm_csr_numeric_planned_i64(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
                                    const int32_t *a_col_idx, const int64_t *a_vals, const int32_t *b_row_ptr,
                                    const int32_t *b_col_idx, const int64_t *b_vals, const int32_t *c_row_ptr,
                                    int32_t *c_col_idx, int64_t *c_vals, void *workspace, size_t workspace_bytes,
-                                   const int64_t *report, void *stream);
+                                   void *bins, size_t bin_bytes, const int64_t *report, void *stream);
 
 /* ------------------------------------------------------------------------
  * scorch_hip_spmm_csr_planned_<T> (and, in fp32, its batched form: `batch` products over one pattern,

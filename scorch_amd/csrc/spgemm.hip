@@ -16,6 +16,9 @@
 //   up to 4096 products  B of at most 131,072 columns: a bitmap of the columns in LDS
 //                        (256 threads, see below); wider B: one workgroup, hash
 //                        table of 8192 slots in LDS
+//   more, B of at most 131,072 columns, and the two passes share what they find out
+//                        the products sorted by ranges of columns (see "the longest rows by
+//                        bins of columns")
 //   more, and more than a 128th of all such rows' products
 //                        several workgroups (see "rows shared out among workgroups")
 //   more                 one workgroup of 1024 threads with a bitmap of the columns
@@ -76,10 +79,9 @@ __device__ __forceinline__ int hash_insert(int *keys, int mask, int key) {
   }
 }
 
-// *addr += v, atomically (LDS or global memory).  Floating-point sums use the
-// hardware's add instructions (global_atomic_add_f32 / _f64, ds_add_f32 / _f64)
-// rather than a compare-and-swap loop; they are exact for ordinary device
-// memory, which is what the workspace must be.
+// *addr += v, atomically, in global memory.  Floating-point sums use the hardware's add
+// instructions (global_atomic_add_f32 / _f64) rather than a compare-and-swap loop; they are exact
+// for ordinary device memory, which is what the workspace must be.
 template <typename A>
 __device__ __forceinline__ void atomic_accumulate(A *addr, A v) { atomicAdd(addr, v); }
 template <>
@@ -89,6 +91,22 @@ __device__ __forceinline__ void atomic_accumulate<double>(double *addr, double v
 template <>
 __device__ __forceinline__ void atomic_accumulate<uint64_t>(uint64_t *addr, uint64_t v) {
   atomicAdd(reinterpret_cast<unsigned long long *>(addr), (unsigned long long)v);
+}
+
+// The same in LDS.  What a CU takes for an instruction of 64 lanes at random addresses, in clocks: reads
+// and writes 7, integer or / add 8, compare-and-swap 12, ds_add_f64 21, and ds_add_f32 193, three
+// for every lane.  fp32 sums are therefore compare-and-swapped starting
+// from the guess that this is the first product of its column, as it mostly is.
+template <typename A>
+__device__ __forceinline__ void lds_accumulate(A *addr, A v) { atomic_accumulate<A>(addr, v); }
+template <>
+__device__ __forceinline__ void lds_accumulate<float>(float *addr, float v) {
+  unsigned *const bits = reinterpret_cast<unsigned *>(addr);
+  for (unsigned seen = 0u;;) {
+    const unsigned found = atomicCAS(bits, seen, __builtin_bit_cast(unsigned, __builtin_bit_cast(float, seen) + v));
+    if (found == seen) return;
+    seen = found;
+  }
 }
 
 // A workgroup's slab in global memory is private to it: its wavefronts share one
@@ -288,19 +306,25 @@ constexpr int kScanPerThread = 16;
 constexpr int kScanTile = kBlockThreads * kScanPerThread;
 
 // counters: [0] medium rows, [1] huge rows, [2] small rows, [5] giant rows listed; [3], [4] next row to hand out;
-// [6..7] one 64-bit sum: the number of entries of the result; [8] rows shared out, [9] their slices; [10..11] one
-// 64-bit sum: the giant rows' products
-constexpr int kSpgemmCounters = 16;
+// [6] (64 bits) the number of entries of the result; [8] rows shared out, [9] their slices; [10] (64 bits) the giant
+// rows' products; [12] (64 bits) the products of all rows beyond kMediumProducts, and [14] their batches of kBinEntries
+// entries; [15] workgroups of pass 0 that are through; [16..18] the bins' totals (Bins)
+// Every counter has a 128-byte line of its own: atomics on one line follow one another at 12 ns each, whatever
+// they address (512 workgroups with eight counts each: 71 us on one line).
+constexpr int kSpgemmCounters = 20;
+__host__ __device__ constexpr int counter(int i) { return 32 * i; }
+constexpr int kBinEntries = 512;
 
 // The symbolic pass is over: the numeric pass hands its longest rows out from the first again, and
 // the host thread, if it waits, gets the report (SpgemmReport).
 __device__ __forceinline__ void end_of_symbolic(int *counters, unsigned long long entries, int64_t *report, int64_t sequence) {
   if (report) {
     const int64_t words[7] = {entries > (unsigned long long)INT32_MAX ? -1 : (int64_t)entries,
-                              counters[2], counters[0], counters[1], counters[5], counters[8], counters[9]};
+                              counters[counter(2)], counters[counter(0)], counters[counter(1)],
+                              counters[counter(5)], counters[counter(8)], counters[counter(9)]};
     sync_publish(report, sequence, words, 7);
   }
-  counters[3] = 0;
+  counters[counter(3)] = 0;
 }
 
 // (*grand_total also receives the sum of all counts in 64 bits: the row pointer is int32,
@@ -330,7 +354,7 @@ __global__ __launch_bounds__(kBlockThreads) void scan_tile_totals_kernel(const i
 __global__ __launch_bounds__(kBlockThreads) void scan_spine_kernel(int *__restrict__ totals,
                                                                    int64_t n_tiles, int *__restrict__ counters,
                                                                    int64_t *__restrict__ report, int64_t sequence) {
-  if (threadIdx.x == 0) end_of_symbolic(counters, *reinterpret_cast<const unsigned long long *>(counters + 6), report, sequence);
+  if (threadIdx.x == 0) end_of_symbolic(counters, *reinterpret_cast<const unsigned long long *>(counters + counter(6)), report, sequence);
   __shared__ int s_scan[kWavesPerBlock + 1];
   int carried = 0;
   for (int64_t base = 0; base < n_tiles; base += kBlockThreads) {
@@ -401,7 +425,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_one_group_kernel(int *__res
   if (wave_lane() == 0) atomicAdd(&s_wide, wide);
   __syncthreads();
   if (threadIdx.x == 0) {
-    *reinterpret_cast<unsigned long long *>(counters + 6) = s_wide;
+    *reinterpret_cast<unsigned long long *>(counters + counter(6)) = s_wide;
     end_of_symbolic(counters, s_wide, report, sequence);
     if (s_wide > (unsigned long long)INT32_MAX) data[n - 1] = -1;
   }
@@ -434,7 +458,8 @@ inline int bounds_rows_per_group(int64_t M) {
 __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     int M, int rows_per_group, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
     const int *__restrict__ b_pos, int *__restrict__ products, int *__restrict__ small_rows,
-    int *__restrict__ medium_rows, int *__restrict__ huge_rows, int *__restrict__ counters) {
+    int *__restrict__ medium_rows, int *__restrict__ huge_rows, int *__restrict__ counters,
+    int64_t *__restrict__ report, int64_t sequence) {
   constexpr int G = 8;  // lanes per row
   constexpr int kStep = kBlockThreads / G;
   __shared__ int s_long[kBoundsRows];
@@ -443,17 +468,22 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
   __shared__ int s_n[6];                  // [4], [5]: long and very long rows queued
   __shared__ int s_base[4];
   __shared__ long long s_part[kWavesPerBlock];
-  __shared__ unsigned long long s_giant_products;
+  __shared__ unsigned long long s_giant_products, s_big_products;
+  __shared__ int s_big_batches;
   if (threadIdx.x < 6) s_n[threadIdx.x] = 0;
-  if (threadIdx.x == 0) s_giant_products = 0;
+  if (threadIdx.x == 0) s_giant_products = s_big_products = 0, s_big_batches = 0;
   __syncthreads();
-  auto file_row = [&](int row, long long sum) {
+  auto file_row = [&](int row, long long sum, int entries) {
     const int bound = sum > INT_MAX ? INT_MAX : (int)sum;
     products[row] = bound;
     const int list = bound >= kGiantProducts ? 3 : bound > kMediumProducts ? 1 : bound > kSmallProducts ? 0
                      : bound > kTinyProducts ? 2 : -1;
     if (list >= 0) s_list[list][atomicAdd(&s_n[list], 1)] = row;
     if (list == 3) atomicAdd(&s_giant_products, (unsigned long long)bound);
+    if (list & 1 && list > 0) {
+      atomicAdd(&s_big_products, (unsigned long long)sum);
+      atomicAdd(&s_big_batches, (entries + kBinEntries - 1) / kBinEntries);
+    }
   };
 
   const int t = threadIdx.x % G;
@@ -465,7 +495,8 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
       lo = a_pos[row];
       hi = a_pos[row + 1];
     }
-    const bool is_long = hi - lo > kBoundsLongRow;
+    const int entries = hi - lo;
+    const bool is_long = entries > kBoundsLongRow;
     if (is_long) {
       if (t == 0) {
         if (hi - lo > kBoundsWaveRow) s_very_long[atomicAdd(&s_n[5], 1)] = (int)row;
@@ -480,7 +511,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     }
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    if (row < M && t == 0 && !is_long) file_row((int)row, sum);
+    if (row < M && t == 0 && !is_long) file_row((int)row, sum, entries);
   }
   __syncthreads();
 
@@ -495,7 +526,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     }
 #pragma unroll
     for (int off = kWaveSize / 2; off > 0; off >>= 1) part += __shfl_xor(part, off);
-    if (wave_lane() == 0) file_row(r, part);
+    if (wave_lane() == 0) file_row(r, part, a_pos[r + 1] - a_pos[r]);
   }
   const int n_very_long = s_n[5];
   for (int i = 0; i < n_very_long; ++i) {  // uniform over the workgroup
@@ -514,15 +545,29 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     if (threadIdx.x == 0) {
       long long total = 0;
       for (int w = 0; w < kWavesPerBlock; ++w) total += s_part[w];
-      file_row(r, total);
+      file_row(r, total, a_pos[r + 1] - a_pos[r]);
     }
   }
   __syncthreads();
   if (threadIdx.x < 4 && s_n[threadIdx.x] > 0)
-    s_base[threadIdx.x] = atomicAdd(&counters[threadIdx.x < 3 ? threadIdx.x : 5], s_n[threadIdx.x]);
+    s_base[threadIdx.x] = atomicAdd(&counters[counter(threadIdx.x < 3 ? threadIdx.x : 5)], s_n[threadIdx.x]);
   if (threadIdx.x == 0 && s_giant_products > 0)
-    atomicAdd(reinterpret_cast<unsigned long long *>(counters + 10), s_giant_products);
+    atomicAdd(reinterpret_cast<unsigned long long *>(counters + counter(10)), s_giant_products);
+  if (threadIdx.x == 0 && s_big_batches > 0) {
+    atomicAdd(reinterpret_cast<unsigned long long *>(counters + counter(12)), s_big_products);
+    atomicAdd(&counters[counter(14)], s_big_batches);
+  }
+  if (report) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's counts are in memory
   __syncthreads();
+  if (report && threadIdx.x == 0 &&  // the last workgroup hands the totals to the host thread
+      __hip_atomic_fetch_add(&counters[counter(15)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1) {
+    const auto total = [&](int i) { return __hip_atomic_load(&counters[counter(i)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    const int64_t words[6] = {total(2), total(0), total(1), total(5),
+                              (int64_t)__hip_atomic_load(reinterpret_cast<unsigned long long *>(counters + counter(12)),
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                              total(14)};
+    sync_publish(report, sequence, words, 6);
+  }
   int *const lists[3] = {medium_rows, huge_rows, small_rows};
 #pragma unroll
   for (int l = 0; l < 3; ++l)
@@ -539,7 +584,7 @@ __device__ __forceinline__ int huge_row(const int *__restrict__ rows, int M, int
 __global__ __launch_bounds__(kBlockThreads) void spgemm_reset_kernel(int *counters, int *c_pos_last, int64_t clear_words,
                                                                      unsigned *bits) {
   if (blockIdx.x == 0) {
-    if (threadIdx.x < kSpgemmCounters) counters[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < counter(kSpgemmCounters); i += kBlockThreads) counters[i] = 0;
     if (threadIdx.x == 0 && c_pos_last) *c_pos_last = 0;
   }
   const int64_t stride = (int64_t)gridDim.x * kBlockThreads;
@@ -591,7 +636,7 @@ __device__ __forceinline__ void spgemm_team_row(
       a_pos[row], a_pos[row + 1], t, a_crd, a_val, b_pos, b_crd, b_val, lds.batch[team], nullptr,
       [&](int col, A product) {
         const int slot = hash_insert(lds.keys[team], SLOTS - 1, col);
-        if (NUMERIC) atomic_accumulate<A>(&lds.vals[team][slot], product);
+        if (NUMERIC) lds_accumulate<A>(&lds.vals[team][slot], product);
       });
   wave_lds_sync();
 
@@ -792,7 +837,7 @@ __device__ __forceinline__ void spgemm_medium_rows(
   auto &s_batch = lds.batch;
 
   const int tid = threadIdx.x;
-  const int n_rows = counters[COUNTER];
+  const int n_rows = counters[counter(COUNTER)];
 
   // (rows handed out one at a time through a counter, as in the bitmap tiers, measured
   // slower: these rows are short enough for the counter's round trip to show)
@@ -810,7 +855,7 @@ __device__ __forceinline__ void spgemm_medium_rows(
         a_pos[row], a_pos[row + 1], tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan,
         [&](int col, A product) {
           const int slot = hash_insert(s_keys, kSlots - 1, col);
-          if (NUMERIC) atomic_accumulate<A>(&s_vals[slot], product);
+          if (NUMERIC) lds_accumulate<A>(&s_vals[slot], product);
         });
     __syncthreads();
 
@@ -965,8 +1010,8 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_huge_kernel(
   __shared__ ProductBatch<kHugeThreads, A> s_batch;
   __shared__ int s_cols[NUMERIC ? kHugeEmitWords * 32 : 1];
   const int tid = threadIdx.x;
-  const int n_giant = counters[5];
-  const int n_rows = counters[1] + n_giant;
+  const int n_giant = counters[counter(5)];
+  const int n_rows = counters[counter(1)] + n_giant;
   if ((int)blockIdx.x >= n_rows) return;
 
   const int words = (N + 31) / 32;
@@ -1049,7 +1094,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_huge_kernel(
 constexpr int kLdsBudget = 160 * 1024 - 1024;
 
 // THREADS: workgroup size.  ACC: LDS sums to provide (0: all the LDS that is left).
-// LIST, WORK: which of `counters` holds the length of `rows` and the next row to hand out.
+// LIST, WORK: which of the counters holds the length of `rows` and the next row to hand out.
 template <typename A, bool NUMERIC, int WORDS, int THREADS, int ACC>
 struct BitmapTables {
   static constexpr int kGroups = WORDS / 4;
@@ -1063,7 +1108,7 @@ struct BitmapTables {
   int next;
 };
 
-// Block number `block` of n_blocks.  `narrow_rows`: the list of the tier above (its length in counters[1]), whose rows
+// Block number `block` of n_blocks.  `narrow_rows`: the list of the tier above (its length in counter 1), whose rows
 // of at most kMediumProducts distinct columns -- known in the numeric pass -- are taken here as well; null: none.
 template <typename T, bool NUMERIC, int WORDS, int THREADS, int ACC, int LIST, int WORK>
 __device__ __forceinline__ void spgemm_lds_bitmap_rows(
@@ -1083,9 +1128,9 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
   auto &s_scan = lds.scan;
   int &s_next = lds.next;
   const int tid = threadIdx.x;
-  const int n_giant = LIST == 1 ? counters[5] : 0;  // only the list of the longest rows has the class
-  const int n_own = counters[LIST] + n_giant;
-  const int n_rows = n_own + (narrow_rows ? counters[1] : 0);
+  const int n_giant = LIST == 1 ? counters[counter(5)] : 0;  // only the list of the longest rows has the class
+  const int n_own = counters[counter(LIST)] + n_giant;
+  const int n_rows = n_own + (narrow_rows ? counters[counter(1)] : 0);
   if (block >= n_rows) return;  // more workgroups than rows: no need to queue at the counter
   constexpr int kRangeColumns = 32 * WORDS;
   A *acc = reinterpret_cast<A *>(c_val);
@@ -1101,7 +1146,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
     __syncthreads();  // everyone is done with the previous row (and with s_next)
     int idx;
     if (LIST == 1) {
-      if (tid == 0) s_next = atomicAdd(&counters[WORK], 1);
+      if (tid == 0) s_next = atomicAdd(&counters[counter(WORK)], 1);
       __syncthreads();
       idx = s_next;
     } else {
@@ -1139,7 +1184,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
         for_each_product<THREADS, true, T, A>(
             a_lo, a_hi, tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan, [&](int k, A product) {
               atomicOr(&s_bits[k >> 5], 1u << (k & 31));
-              atomic_accumulate<A>(&s_acc[k], product);
+              lds_accumulate<A>(&s_acc[k], product);
             });
       } else {
         for_each_product<THREADS, false, T, A>(
@@ -1204,7 +1249,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
                              __popc(grp.y & (sub == 1 ? below : sub > 1 ? ~0u : 0u)) +
                              __popc(grp.z & (sub == 2 ? below : sub > 2 ? ~0u : 0u)) +
                              __popc(grp.w & (sub == 3 ? below : 0u));
-              if (at < kAccEntries) atomic_accumulate<A>(&s_acc[at], product);
+              if (at < kAccEntries) lds_accumulate<A>(&s_acc[at], product);
               else __hip_atomic_fetch_add(&acc[first + at], product, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             });
         __syncthreads();
@@ -1301,8 +1346,8 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_split_select_kernel(
   __shared__ int s_rows, s_items;
   if (threadIdx.x == 0) s_rows = s_items = 0;
   __syncthreads();
-  const int n_giant = counters[5];
-  const unsigned long long share = *reinterpret_cast<const unsigned long long *>(counters + 10) / 128;
+  const int n_giant = counters[counter(5)];
+  const unsigned long long share = *reinterpret_cast<const unsigned long long *>(counters + counter(10)) / 128;
   for (int i = threadIdx.x; i < n_giant; i += kBlockThreads) {
     const int row = huge_rows[M - 1 - i];
     const int p = products[row];
@@ -1320,15 +1365,15 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_split_select_kernel(
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    counters[8] = s_rows < pool ? s_rows : pool;
-    counters[9] = s_items;
+    counters[counter(8)] = s_rows < pool ? s_rows : pool;
+    counters[counter(9)] = s_items;
   }
 }
 
 template <typename A>
 __global__ __launch_bounds__(kBlockThreads) void spgemm_split_clear_kernel(int N, const int *__restrict__ counters,
                                                                            A *__restrict__ sums) {
-  const int64_t n = (int64_t)counters[8] * N, stride = (int64_t)gridDim.x * kBlockThreads;
+  const int64_t n = (int64_t)counters[counter(8)] * N, stride = (int64_t)gridDim.x * kBlockThreads;
   for (int64_t i = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x; i < n; i += stride) sums[i] = (A)0;
 }
 
@@ -1348,7 +1393,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_columns_kernel(
   __shared__ ProductBatch<kHugeThreads, float> s_batch;
   __shared__ int s_scan[kHugeWaves];
   const int tid = threadIdx.x;
-  const int n_items = counters[9];
+  const int n_items = counters[counter(9)];
   for (int i = blockIdx.x; i < n_items; i += gridDim.x) {  // uniform
     const int4 item = items[i];
     int from, to;
@@ -1374,7 +1419,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_sums_kernel(
   using A = typename Acc<T>::type;
   __shared__ ProductBatch<kHugeThreads, A> s_batch;
   __shared__ int s_scan[kHugeWaves];
-  const int n_items = counters[9];
+  const int n_items = counters[counter(9)];
   for (int i = blockIdx.x; i < n_items; i += gridDim.x) {  // uniform
     const int4 item = items[i];
     int from, to;
@@ -1394,7 +1439,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_split_count_kernel(const
                                                                            int *__restrict__ c_pos) {
   __shared__ int s_scan[kWavesPerBlock];
   const int slot = blockIdx.x;
-  if (slot >= counters[8]) return;
+  if (slot >= counters[counter(8)]) return;
   int mine = 0, total = 0;
   for (int w = threadIdx.x; w < split.words; w += kBlockThreads) mine += __popc(split.bits[(size_t)slot * split.words + w]);
   (void)block_exclusive_scan(mine, s_scan, total);
@@ -1412,7 +1457,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
   __shared__ int s_rank[kEmitWords];
   __shared__ int s_scan[kHugeWaves];
   const int slot = blockIdx.y;
-  if (slot >= counters[8]) return;
+  if (slot >= counters[counter(8)]) return;
   const int tid = threadIdx.x, lane = wave_lane();
   const unsigned *row_bits = bits + (size_t)slot * (size_t)words;
   const int first = (int)blockIdx.x * kEmitWords;
@@ -1435,6 +1480,352 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
       const size_t at = out + s_rank[mine_at] + __popc(b & ((1u << bit) - 1u));
       c_crd[at] = col;
       c_val[at] = (T)row_sums[col];
+    }
+  }
+}
+
+// ---- the longest rows by bins of columns -------------------------------------------------------
+// One sum per column of a row beyond kMediumProducts does not fit LDS (131,072 columns), so the kernels
+// above walk such a row twice, first for its columns, and a hub's sums are added up in memory (20
+// products a nanosecond, however many workgroups do it).  Here the products are made once and
+// sorted by ranges of columns: a workgroup turns 2,048 products at a time into runs of equal
+// range in LDS and writes them out (a window: 16 bits of column within the range and the value each, 6
+// bytes in fp32).  The columns of one range of one row are then counted, and later its sums added up
+// in LDS, by a workgroup that reads its runs from all of the row's windows: streams instead of
+// gathers, as many workgroups to a row as it has ranges, and a hub shared out by itself.
+// Both passes over these rows of a power-law graph squared (131,072 nodes, 16 entries a row, 19 M
+// products of this kind), fp32: 300 us (lists 19, sort 106, count 52, sums 123); the numeric pass alone took 512.  The sort is
+// bound by the gathers from B (a line for about two entries), the sums by LDS atomics.  (Ranges
+// without the windows, each item bisecting the rows of B for its piece, fetch those lines once
+// per range: 411 us for the numeric pass alone.)
+// For products of up to kNarrowColumns columns whose two passes share what they find out.
+constexpr int kBinThreads = kBinEntries;
+constexpr int kBinProducts = 4 * kBinThreads;  // to a window
+constexpr int kBinShare = 4 * kBinProducts;    // products of a batch of entries to a workgroup
+constexpr int kBinColumns = 8192;              // most columns to a range; a power of two
+constexpr int kMaxBins = kNarrowColumns / kBinColumns;
+constexpr int64_t kBinBudget = (int64_t)4 << 30;
+
+struct BinWindow {
+  int first;                            // its products in `columns` and `values`
+  unsigned short at[kMaxBins + 2];      // where its runs begin
+};
+struct BinRow {
+  int row, batches, first_window, first_product, first_item, items;
+};
+struct BinItem {
+  int row, batch, share, shares;  // of the batch's windows this one takes those from `share` on, `shares` apart
+};
+
+struct Bins {
+  int shift = 0, n = 0;                 // ranges of 2^shift columns, n of them; n 0: not used
+  int64_t rows = 0, items = 0;
+  int *totals;                          // products, windows, items handed out to rows so far (counters of pass 0)
+  BinRow *row;
+  unsigned long long *used;             // per row: windows (upper half) and products written
+  BinItem *item;
+  BinWindow *window;
+  int *counts;                          // [row][n]: distinct columns
+  unsigned short *columns;
+  void *values;
+  size_t total = 0;
+};
+
+inline Bins spgemm_bins(char *base, int *counters, int64_t N, size_t elem, int64_t rows, int64_t products, int64_t batches) {
+  Bins b;
+  if (rows == 0 || N > kNarrowColumns || products * (int64_t)(2 + elem) > kBinBudget || products > INT32_MAX / 2) return b;
+  b.shift = 10;  // eight ranges and more, for the sake of narrow matrices' hubs
+  while ((2 << b.shift) <= kBinColumns && (8 << b.shift) < N) ++b.shift;
+  b.n = (int)((N + (1 << b.shift) - 1) >> b.shift);
+  b.rows = rows;
+  b.items = batches + products / kBinShare;
+  size_t off = 0;
+  auto take = [&](size_t bytes) { char *p = base ? base + off : nullptr; off += (bytes + 255) / 256 * 256; return p; };
+  b.totals = counters ? counters + counter(16) : nullptr;
+  b.row = reinterpret_cast<BinRow *>(take((size_t)rows * sizeof(BinRow)));
+  b.used = reinterpret_cast<unsigned long long *>(take((size_t)rows * 8));
+  b.item = reinterpret_cast<BinItem *>(take((size_t)b.items * sizeof(BinItem)));
+  b.window = reinterpret_cast<BinWindow *>(take((size_t)(products / kBinProducts + batches) * sizeof(BinWindow)));
+  b.counts = reinterpret_cast<int *>(take((size_t)(rows * b.n) * 4));
+  b.columns = reinterpret_cast<unsigned short *>(take((size_t)products * 2));
+  b.values = take((size_t)products * elem);
+  b.total = off;
+  return b;
+}
+
+// Places for the rows' products, windows and work items.
+__global__ __launch_bounds__(kBlockThreads) void spgemm_bin_rows_kernel(int M, Bins bins, const int *__restrict__ a_pos,
+                                                                        const int *__restrict__ products,
+                                                                        const int *__restrict__ huge_rows,
+                                                                        const int *__restrict__ counters,
+                                                                        int *__restrict__ c_pos) {
+  __shared__ int s_scan[kWavesPerBlock], s_base[3];
+  const int64_t i = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x;
+  const bool mine = i < bins.rows;
+  BinRow r = {};
+  int p = 0;
+  if (mine) {
+    r.row = huge_row(huge_rows, M, counters[counter(5)], (int)i);
+    p = products[r.row];
+    r.batches = (a_pos[r.row + 1] - a_pos[r.row] + kBinEntries - 1) / kBinEntries;
+    r.items = r.batches + p / kBinShare;  // at most
+  }
+  const int want[3] = {p, mine ? p / kBinProducts + r.batches : 0, r.items};
+  int at[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    int total = 0;
+    at[k] = block_exclusive_scan(want[k], s_scan, total);
+    if (threadIdx.x == (unsigned)k) s_base[k] = atomicAdd(bins.totals + counter(k), total);
+  }
+  __syncthreads();
+  if (!mine) return;
+  r.first_product = s_base[0] + at[0];
+  r.first_window = s_base[1] + at[1];
+  r.first_item = s_base[2] + at[2];
+  bins.row[i] = r;
+  bins.used[i] = 0;
+  c_pos[r.row] = 0;
+}
+
+// A row's work items: a wavefront to a batch of entries.
+constexpr int kBinItemThreads = 512;
+__global__ __launch_bounds__(kBinItemThreads) void spgemm_bin_items_kernel(Bins bins, const int *__restrict__ a_pos,
+                                                                           const int *__restrict__ a_crd,
+                                                                           const int *__restrict__ b_pos) {
+  constexpr int kPer = kBinEntries / kWaveSize;
+  __shared__ int s_items;
+  if (threadIdx.x == 0) s_items = 0;
+  __syncthreads();
+  const int lane = wave_lane();
+  const BinRow r = bins.row[blockIdx.x];
+  const int lo = a_pos[r.row], hi = a_pos[r.row + 1];
+  for (int batch = threadIdx.x / kWaveSize; batch < r.batches; batch += kBinItemThreads / kWaveSize) {
+    int at[kPer], total = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int p = lo + batch * kBinEntries + i * kWaveSize + lane;
+      at[i] = p < hi ? a_crd[p] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      if (at[i] >= 0) total += b_pos[at[i] + 1] - b_pos[at[i]];
+#pragma unroll
+    for (int off = kWaveSize / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
+    const int shares = 1 + total / kBinShare;
+    int first = 0;
+    if (lane == 0) first = atomicAdd(&s_items, shares);
+    first = r.first_item + uniform(first);
+    for (int j = lane; j < shares; j += kWaveSize) bins.item[first + j] = {(int)blockIdx.x, batch, j, shares};
+  }
+  __syncthreads();
+  for (int j = s_items + (int)threadIdx.x; j < r.items; j += kBinItemThreads) bins.item[r.first_item + j] = {0, 0, 0, 0};  // none
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
+    Bins bins, const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
+    const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val) {
+  using A = typename Acc<T>::type;
+  constexpr int U = kBinProducts / kBinThreads;
+  __shared__ ProductBatch<kBinEntries, A> s_batch;
+  __shared__ A s_value[kBinProducts];
+  __shared__ unsigned short s_column[kBinProducts];
+  __shared__ int s_scan[kBinThreads / kWaveSize], s_count[kMaxBins + 1], s_at[kMaxBins + 1], s_first, s_window;
+  if ((int)blockIdx.x >= bins.totals[counter(2)]) return;
+  const int tid = threadIdx.x;
+  const BinItem item = bins.item[blockIdx.x];
+  if (item.shares == 0) return;
+  const BinRow r = bins.row[item.row];
+  const int lo = a_pos[r.row] + item.batch * kBinEntries, hi = min(lo + kBinEntries, a_pos[r.row + 1]);
+  {
+    int first = 0, len = 0;
+    A av = (A)0;
+    if (lo + tid < hi) {
+      const int j = a_crd[lo + tid];
+      first = b_pos[j];
+      len = b_pos[j + 1] - first;
+      av = (A)a_val[lo + tid];
+    }
+    int unused = 0;
+    s_batch.index[tid] = block_exclusive_scan_n<kBinThreads / kWaveSize>(len, s_scan, unused);
+    s_batch.index[kBinEntries + tid] = first;
+    s_batch.a_val[tid] = av;
+    if (tid == kBinThreads - 1) s_first = unused;
+  }
+  __syncthreads();
+  const int total = s_first;
+  for (int x0 = item.share * kBinProducts; x0 < total; x0 += item.shares * kBinProducts) {  // uniform
+    const int n = min(kBinProducts, total - x0);
+    int q[U], e[U], col[U], rank[U];
+    A b[U];
+    unsigned long long used = 0;  // (the round trip passes while the products are gathered)
+    if (tid == kBinThreads - 1) used = atomicAdd(&bins.used[item.row], (1ull << 32) + (unsigned)n);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int x = min(x0 + u * kBinThreads + tid, total - 1);
+      e[u] = 0;  // as in product_step
+#pragma unroll
+      for (int step = kBinEntries / 2; step > 0; step >>= 1)
+        if (s_batch.index[e[u] + step] <= x) e[u] += step;
+      q[u] = s_batch.index[kBinEntries + e[u]] + (x - s_batch.index[e[u]]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      col[u] = b_crd[q[u]];
+      b[u] = (A)b_val[q[u]];
+    }
+    __syncthreads();  // everyone is done with the previous window (and has read s_first)
+    if (tid <= kMaxBins) s_count[tid] = 0;
+    if (tid == kBinThreads - 1) {
+      s_first = (int)(unsigned)used;
+      s_window = (int)(used >> 32);
+    }
+    __syncthreads();
+    int bin[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      bin[u] = col[u] >> bins.shift;
+      if (u * kBinThreads + tid < n) rank[u] = atomicAdd(&s_count[bin[u]], 1);
+    }
+    __syncthreads();
+    if (tid <= bins.n) {
+      int at = 0;
+      for (int i = 0; i < tid; ++i) at += s_count[i];
+      s_at[tid] = at;
+      bins.window[r.first_window + s_window].at[tid] = (unsigned short)at;
+    }
+    if (tid == 0) bins.window[r.first_window + s_window].first = r.first_product + s_first;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u * kBinThreads + tid < n) {
+        const int at = s_at[bin[u]] + rank[u];
+        s_column[at] = (unsigned short)(col[u] - (bin[u] << bins.shift));
+        s_value[at] = s_batch.a_val[e[u]] * b[u];
+      }
+    __syncthreads();
+    const int64_t first = (int64_t)r.first_product + s_first;
+    A *values = static_cast<A *>(bins.values) + first;
+    for (int i = tid; i < n; i += kBinThreads) {
+      bins.columns[first + i] = s_column[i];
+      values[i] = s_value[i];
+    }
+  }
+}
+
+// fn(place) for every product of range `bin` of a row, `place` indexing columns and values: 64 windows' runs are
+// looked up at a time, a wavefront takes a run.
+template <int WAVES, typename Fn>
+__device__ __forceinline__ void for_each_binned(const Bins &bins, const BinRow &r, int windows, int bin, Fn fn) {
+  const int lane = wave_lane(), w = threadIdx.x / kWaveSize;
+  for (int base = w; base < windows; base += WAVES * kWaveSize) {
+    int first = 0, last = 0;
+    if (base + lane * WAVES < windows) {
+      const BinWindow &win = bins.window[r.first_window + base + lane * WAVES];
+      first = win.first + win.at[bin];
+      last = win.first + win.at[bin + 1];
+    }
+    const int here = min(kWaveSize, (windows - base + WAVES - 1) / WAVES);
+    for (int i = 0; i < here; ++i) {
+      const int from = __builtin_amdgcn_readlane(first, i), to = __builtin_amdgcn_readlane(last, i);
+      for (int p = from + lane; p < to; p += 4 * kWaveSize) fn(p, to);
+    }
+  }
+}
+
+constexpr int kBinCountThreads = 256;
+__global__ __launch_bounds__(kBinCountThreads) void spgemm_bin_count_kernel(Bins bins, int *__restrict__ c_pos) {
+  constexpr int kWaves = kBinCountThreads / kWaveSize;
+  __shared__ unsigned s_bits[kBinColumns / 32];
+  __shared__ int s_scan[kWaves];
+  const int idx = (int)(blockIdx.x / (unsigned)bins.n), bin = (int)(blockIdx.x % (unsigned)bins.n);
+  const BinRow r = bins.row[idx];
+  const int windows = (int)(bins.used[idx] >> 32), words = (1 << bins.shift) / 32;
+  for (int i = threadIdx.x; i < words; i += kBinCountThreads) s_bits[i] = 0u;
+  __syncthreads();
+  for_each_binned<kWaves>(bins, r, windows, bin, [&](int p, int to) {
+    int c[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) c[u] = p + u * kWaveSize < to ? bins.columns[p + u * kWaveSize] : -1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c[u] >= 0) atomicOr(&s_bits[c[u] >> 5], 1u << (c[u] & 31));
+  });
+  __syncthreads();
+  int mine = 0, total = 0;
+  for (int i = threadIdx.x; i < words; i += kBinCountThreads) mine += __popc(s_bits[i]);
+  (void)block_exclusive_scan_n<kWaves>(mine, s_scan, total);
+  if (threadIdx.x == 0) {
+    bins.counts[(size_t)idx * bins.n + bin] = total;
+    if (total) atomicAdd(&c_pos[r.row], total);
+  }
+}
+
+constexpr int kBinSumThreads = 512;
+template <typename T>
+__global__ __launch_bounds__(kBinSumThreads) void spgemm_bin_sums_kernel(Bins bins, const int *__restrict__ c_pos,
+                                                                         int *__restrict__ c_crd, T *__restrict__ c_val) {
+  using A = typename Acc<T>::type;
+  constexpr int kWaves = kBinSumThreads / kWaveSize;
+  __shared__ A s_sum[kBinColumns];
+  __shared__ unsigned s_bits[kBinColumns / 32];
+  __shared__ int s_rank[kBinColumns / 32];
+  __shared__ int s_scan[kWaves];
+  const int tid = threadIdx.x, lane = wave_lane();
+  const int idx = (int)(blockIdx.x / (unsigned)bins.n), bin = (int)(blockIdx.x % (unsigned)bins.n);
+  const int *counts = bins.counts + (size_t)idx * bins.n;
+  const int n = counts[bin];
+  const BinRow r = bins.row[idx];
+  const int windows = (int)(bins.used[idx] >> 32), columns = 1 << bins.shift, words = columns / 32;
+  for (int i = tid; i < columns; i += kBinSumThreads) s_sum[i] = (A)0;
+  for (int i = tid; i < words; i += kBinSumThreads) s_bits[i] = 0u;
+  int out = c_pos[r.row];
+  for (int i = 0; i < bin; ++i) out += counts[i];
+  if (n == 0) return;
+  __syncthreads();
+  const A *values = static_cast<const A *>(bins.values);
+  for_each_binned<kWaves>(bins, r, windows, bin, [&](int p, int to) {
+    int c[4];
+    A v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int at = p + u * kWaveSize;
+      c[u] = at < to ? bins.columns[at] : -1;
+      v[u] = at < to ? values[at] : (A)0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c[u] >= 0) {
+        atomicOr(&s_bits[c[u] >> 5], 1u << (c[u] & 31));
+        lds_accumulate<A>(&s_sum[c[u]], v[u]);
+      }
+  });
+  __syncthreads();
+  int unused = 0;
+  const int rank = block_exclusive_scan_n<kWaves>(tid < words ? __popc(s_bits[tid]) : 0, s_scan, unused);
+  const int first_column = bin << bins.shift;
+  if (4 * n < columns) {  // a thread per word of the bitmap
+    if (tid < words) {
+      int at = out + rank;
+      for (unsigned bits = s_bits[tid]; bits; bits &= bits - 1, ++at) {
+        const int col = tid * 32 + __ffs(bits) - 1;
+        c_crd[at] = first_column + col;
+        c_val[at] = (T)s_sum[col];
+      }
+    }
+    return;
+  }
+  if (tid < words) s_rank[tid] = rank;
+  __syncthreads();
+  // two bitmap words, 64 columns, per wavefront and step
+  for (int w = 2 * (tid / kWaveSize); w < words; w += 2 * kWaves) {
+    const int mine = w + (lane >> 5), bit = lane & 31;
+    const unsigned b = s_bits[mine];
+    if ((b >> bit) & 1u) {
+      const int at = out + s_rank[mine] + __popc(b & ((1u << bit) - 1u));
+      c_crd[at] = first_column + mine * 32 + bit;
+      c_val[at] = (T)s_sum[mine * 32 + bit];
     }
   }
 }
@@ -1464,7 +1855,7 @@ inline SpgemmWorkspace spgemm_layout(char *base, int64_t M, int64_t N, size_t el
   ws.small_rows = reinterpret_cast<int *>(take((size_t)M * 4));
   ws.medium_rows = reinterpret_cast<int *>(take((size_t)M * 4));
   ws.huge_rows = reinterpret_cast<int *>(take((size_t)M * 4));
-  ws.counters = reinterpret_cast<int *>(take(kSpgemmCounters * 4));
+  ws.counters = reinterpret_cast<int *>(take(counter(kSpgemmCounters) * 4));
   ws.pool = split_pool(N);
   ws.split_rows = reinterpret_cast<int *>(take((size_t)ws.pool * 4));
   ws.split_items = reinterpret_cast<int4 *>(take((size_t)ws.pool * kSplitMaxSlices * sizeof(int4)));
@@ -1505,124 +1896,140 @@ inline int spgemm_check(const char *fn, int64_t M, int64_t K, int64_t N, const v
 struct SpgemmReport {
   int64_t entries;                                         // of the result; -1: 2^31 or more
   int64_t small, medium, huge, giant, split, split_items;  // rows listed per tier; slices of the rows shared out
+  int64_t products, batches;                               // of the rows beyond kMediumProducts
 };
-constexpr int kSpgemmReportWords = 7;
+constexpr int kSpgemmReportWords = 9;
+inline SpgemmReport report_of(const int64_t *w) { return {w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8]}; }
 
 // `known`: the numeric pass finds the row lists of the symbolic pass in the workspace and launches what has rows.
-// `sync`: the symbolic pass hands its report over.
+// `sync`: the symbolic pass hands its report over (its short rows' part what pass 0 found, the long rows' part the rest).
+// `bins`: the rows beyond kMediumProducts go by bins (the symbolic pass has counted them there already).
+constexpr int kShortRows = 1, kLongRows = 2;
 template <typename T, bool NUMERIC>
 int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val, const int *b_pos,
                const int *b_crd, const T *b_val, int *c_pos, int *c_crd, T *c_val,
-               const SpgemmWorkspace &ws, hipStream_t stream, const SpgemmReport *known = nullptr,
-               SyncCall *sync = nullptr) {
+               const SpgemmWorkspace &ws, hipStream_t stream, int parts = kShortRows | kLongRows,
+               const SpgemmReport *known = nullptr, SyncCall *sync = nullptr, const Bins *bins = nullptr) {
   using A = typename Acc<T>::type;
   const int words = (N + 31) / 32;
-  if (!known) {
-    const int64_t clear_words = (int64_t)ws.pool * words;
-    const unsigned clear_blocks = (unsigned)(1 + (clear_words < 1 << 18 ? clear_words : 1 << 18) / 1024);
-    spgemm_reset_kernel<<<clear_blocks, kBlockThreads, 0, stream>>>(ws.counters, NUMERIC ? nullptr : c_pos + M, clear_words,
-                                                                    ws.split_bits);
-    SCORCH_HIP_CHECK(hipGetLastError());
-    const int rows_per_group = bounds_rows_per_group(M);
-    const unsigned row_groups = (unsigned)(((int64_t)M + rows_per_group - 1) / rows_per_group);
-    spgemm_bounds_kernel<<<row_groups, kBlockThreads, 0, stream>>>(M, rows_per_group, a_pos, a_crd, b_pos, ws.products,
-                                                                  ws.small_rows, ws.medium_rows,
-                                                                  ws.huge_rows, ws.counters);
-    SCORCH_HIP_CHECK(hipGetLastError());
-  }
-  if (ws.pool > 0 && (!known || known->split > 0)) {
-    A *sums = static_cast<A *>(ws.split_sums);
-    if (!known) {
-      spgemm_split_select_kernel<<<1, kBlockThreads, 0, stream>>>(M, ws.pool, a_pos, ws.products, ws.huge_rows, ws.counters,
-                                                                 ws.split_rows, ws.split_items);
-      SCORCH_HIP_CHECK(hipGetLastError());
-      auto columns_of = words <= 4096 ? &spgemm_split_columns_kernel<4096> : &spgemm_split_columns_kernel<kSplitMaxColumns / 32>;
-      columns_of<<<512, kHugeThreads, 0, stream>>>(words, a_pos, a_crd, b_pos, b_crd, ws.counters, ws.split_rows,
-                                                   ws.split_items, ws.split_bits);
-      SCORCH_HIP_CHECK(hipGetLastError());
-    }
-    if (NUMERIC) {
-      const int64_t n_sums = (int64_t)(known ? (int)known->split : ws.pool) * N;
-      spgemm_split_clear_kernel<A><<<(unsigned)(1 + (n_sums < 1 << 20 ? n_sums : 1 << 20) / 1024), kBlockThreads, 0, stream>>>(
-          N, ws.counters, sums);
-      SCORCH_HIP_CHECK(hipGetLastError());
-      const unsigned slices = known ? (unsigned)known->split_items : 512u;
-      spgemm_split_sums_kernel<T><<<slices, kHugeThreads, 0, stream>>>(N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.counters,
-                                                                      ws.split_rows, ws.split_items, sums);
-      SCORCH_HIP_CHECK(hipGetLastError());
-      const unsigned pieces = (unsigned)((words + kEmitWords - 1) / kEmitWords);
-      spgemm_split_emit_kernel<T><<<dim3(pieces, (unsigned)(known ? known->split : ws.pool)), kHugeThreads, 0, stream>>>(
-          N, words, ws.counters, ws.split_rows, ws.split_bits, sums, c_pos, c_crd, c_val);
-      SCORCH_HIP_CHECK(hipGetLastError());
-    }
-  }
   const bool narrow = N <= kNarrowColumns;
-  // rows the 256-thread bitmap kernel goes through; with the result's row pointer known, also those of the tier above
-  // that turn out to have few distinct columns
-  const int *narrow_rows = NUMERIC && narrow ? ws.huge_rows : nullptr;
-  const auto blocks_for = [&](int64_t rows) { return (unsigned)(rows < kMediumWorkgroups ? rows : kMediumWorkgroups); };
-  const unsigned small_blocks = blocks_for(known ? known->small : M);
-  const unsigned bitmap_blocks = blocks_for(known ? known->medium + (narrow_rows ? known->huge : 0) : M);
-  if (M < 4 * 8192 && narrow) {
-    const unsigned tiny_blocks = (unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock);
-    spgemm_small_matrix_kernel<T, NUMERIC><<<bitmap_blocks + small_blocks + tiny_blocks, kBlockThreads, 0, stream>>>(
-        M, N, (int)bitmap_blocks, (int)small_blocks, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows,
-        ws.medium_rows, narrow_rows, ws.counters, c_pos, c_crd, c_val);
-    SCORCH_HIP_CHECK(hipGetLastError());
-  } else {
-    // four rows to a wavefront
-    const int64_t rows_per_block = kWavesPerBlock * (kWaveSize / kMicroTeam);
-    const unsigned tiny_blocks = (unsigned)round_up_8(((int64_t)M + rows_per_block - 1) / rows_per_block);
-    spgemm_tiny_kernel<T, NUMERIC><<<tiny_blocks, kBlockThreads, 0, stream>>>(
-        M, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, c_pos, c_crd, c_val);
-    SCORCH_HIP_CHECK(hipGetLastError());
-    if (small_blocks) {
-      spgemm_medium_kernel<T, NUMERIC, kSmallProducts, 2, kBlockThreads><<<small_blocks, kBlockThreads, 0, stream>>>(
-          a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.small_rows, ws.counters, c_pos, c_crd, c_val);
+  if (parts & kShortRows) {
+    if (!known) {
+      const int64_t clear_words = (int64_t)ws.pool * words;
+      const unsigned clear_blocks = (unsigned)(1 + (clear_words < 1 << 18 ? clear_words : 1 << 18) / 1024);
+      spgemm_reset_kernel<<<clear_blocks, kBlockThreads, 0, stream>>>(ws.counters, NUMERIC ? nullptr : c_pos + M, clear_words,
+                                                                      ws.split_bits);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      const int rows_per_group = bounds_rows_per_group(M);
+      const unsigned row_groups = (unsigned)(((int64_t)M + rows_per_group - 1) / rows_per_group);
+      spgemm_bounds_kernel<<<row_groups, kBlockThreads, 0, stream>>>(M, rows_per_group, a_pos, a_crd, b_pos, ws.products,
+                                                                    ws.small_rows, ws.medium_rows,
+                                                                    ws.huge_rows, ws.counters,
+                                                                    sync ? sync->target() : nullptr, sync ? sync->sequence() : 0);
       SCORCH_HIP_CHECK(hipGetLastError());
     }
-    if (bitmap_blocks && narrow) {
-      // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
-      spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts, 0, 4>
-          <<<bitmap_blocks, kBlockThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
-                                                        narrow_rows, ws.counters, c_pos, c_crd, c_val);
-    } else if (bitmap_blocks) {
-      // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
-      // beside them (with 8-byte sums, no more than 256)
-      constexpr int kThreads = sizeof(A) > 4 ? kBlockThreads : kHugeThreads;
-      spgemm_medium_kernel<T, NUMERIC, kMediumProducts, 0, kThreads><<<bitmap_blocks, kThreads, 0, stream>>>(
-          a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
+    // rows the 256-thread bitmap kernel goes through; with the result's row pointer known, also those of the tier above
+    // that turn out to have few distinct columns
+    const int *narrow_rows = NUMERIC && narrow && !bins ? ws.huge_rows : nullptr;
+    const auto blocks_for = [&](int64_t rows) { return (unsigned)(rows < kMediumWorkgroups ? rows : kMediumWorkgroups); };
+    const unsigned small_blocks = blocks_for(known ? known->small : M);
+    const unsigned bitmap_blocks = blocks_for(known ? known->medium + (narrow_rows ? known->huge : 0) : M);
+    if (M < 4 * 8192 && narrow) {
+      const unsigned tiny_blocks = (unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock);
+      spgemm_small_matrix_kernel<T, NUMERIC><<<bitmap_blocks + small_blocks + tiny_blocks, kBlockThreads, 0, stream>>>(
+          M, N, (int)bitmap_blocks, (int)small_blocks, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows,
+          ws.medium_rows, narrow_rows, ws.counters, c_pos, c_crd, c_val);
+      SCORCH_HIP_CHECK(hipGetLastError());
+    } else {
+      // four rows to a wavefront
+      const int64_t rows_per_block = kWavesPerBlock * (kWaveSize / kMicroTeam);
+      const unsigned tiny_blocks = (unsigned)round_up_8(((int64_t)M + rows_per_block - 1) / rows_per_block);
+      spgemm_tiny_kernel<T, NUMERIC><<<tiny_blocks, kBlockThreads, 0, stream>>>(
+          M, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, c_pos, c_crd, c_val);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      if (small_blocks) {
+        spgemm_medium_kernel<T, NUMERIC, kSmallProducts, 2, kBlockThreads><<<small_blocks, kBlockThreads, 0, stream>>>(
+            a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.small_rows, ws.counters, c_pos, c_crd, c_val);
+        SCORCH_HIP_CHECK(hipGetLastError());
+      }
+      if (bitmap_blocks && narrow) {
+        // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
+        spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts, 0, 4>
+            <<<bitmap_blocks, kBlockThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
+                                                          narrow_rows, ws.counters, c_pos, c_crd, c_val);
+      } else if (bitmap_blocks) {
+        // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
+        // beside them (with 8-byte sums, no more than 256)
+        constexpr int kThreads = sizeof(A) > 4 ? kBlockThreads : kHugeThreads;
+        spgemm_medium_kernel<T, NUMERIC, kMediumProducts, 0, kThreads><<<bitmap_blocks, kThreads, 0, stream>>>(
+            a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
+      }
+      SCORCH_HIP_CHECK(hipGetLastError());
+    }
+  }
+  if (!(parts & kLongRows)) return SCORCH_HIP_OK;
+  const int64_t listed = known ? known->huge + known->giant : M;  // rows beyond kMediumProducts, at most
+  if (bins) {
+    if constexpr (NUMERIC) {
+      spgemm_bin_sums_kernel<T><<<(unsigned)(bins->rows * bins->n), kBinSumThreads, 0, stream>>>(*bins, c_pos, c_crd, c_val);
+      SCORCH_HIP_CHECK(hipGetLastError());
+    }
+  } else if (listed > 0) {
+    if (ws.pool > 0 && (!known || !NUMERIC || known->split > 0)) {
+      A *sums = static_cast<A *>(ws.split_sums);
+      if (!NUMERIC || !known) {
+        spgemm_split_select_kernel<<<1, kBlockThreads, 0, stream>>>(M, ws.pool, a_pos, ws.products, ws.huge_rows, ws.counters,
+                                                                   ws.split_rows, ws.split_items);
+        SCORCH_HIP_CHECK(hipGetLastError());
+        auto columns_of = words <= 4096 ? &spgemm_split_columns_kernel<4096> : &spgemm_split_columns_kernel<kSplitMaxColumns / 32>;
+        columns_of<<<512, kHugeThreads, 0, stream>>>(words, a_pos, a_crd, b_pos, b_crd, ws.counters, ws.split_rows,
+                                                     ws.split_items, ws.split_bits);
+        SCORCH_HIP_CHECK(hipGetLastError());
+      }
+      if (NUMERIC) {
+        const int64_t n_sums = (int64_t)(known ? (int)known->split : ws.pool) * N;
+        spgemm_split_clear_kernel<A><<<(unsigned)(1 + (n_sums < 1 << 20 ? n_sums : 1 << 20) / 1024), kBlockThreads, 0, stream>>>(
+            N, ws.counters, sums);
+        SCORCH_HIP_CHECK(hipGetLastError());
+        const unsigned slices = known ? (unsigned)known->split_items : 512u;
+        spgemm_split_sums_kernel<T><<<slices, kHugeThreads, 0, stream>>>(N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.counters,
+                                                                        ws.split_rows, ws.split_items, sums);
+        SCORCH_HIP_CHECK(hipGetLastError());
+        const unsigned pieces = (unsigned)((words + kEmitWords - 1) / kEmitWords);
+        spgemm_split_emit_kernel<T><<<dim3(pieces, (unsigned)(known ? known->split : ws.pool)), kHugeThreads, 0, stream>>>(
+            N, words, ws.counters, ws.split_rows, ws.split_bits, sums, c_pos, c_crd, c_val);
+        SCORCH_HIP_CHECK(hipGetLastError());
+      }
+    }
+    // one workgroup per CU's worth of LDS; more only queue up behind them
+    const int64_t huge_rows = listed - (known && NUMERIC ? known->split : 0);
+    const unsigned lds_pool = (unsigned)(huge_rows < 512 ? huge_rows : 512);
+    if (lds_pool == 0) {
+    } else if (narrow) {
+      spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
+          M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, nullptr, ws.counters, c_pos, c_crd, c_val);
+    } else if (!NUMERIC && N > 32 * 16384 && N <= 32 * 32768) {
+      // the symbolic pass keeps no ranks or sums: its bitmap can be twice as wide, one range instead of two
+      spgemm_lds_bitmap_kernel<T, NUMERIC, NUMERIC ? 16384 : 32768, kHugeThreads, 0, 1, 3>
+          <<<lds_pool, kHugeThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows,
+                                                  nullptr, ws.counters, c_pos, c_crd, c_val);
+    } else if (N <= kLdsBitmapColumns) {
+      spgemm_lds_bitmap_kernel<T, NUMERIC, 16384, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
+          M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, nullptr, ws.counters, c_pos, c_crd, c_val);
+    } else {
+      spgemm_huge_kernel<T, NUMERIC><<<ws.huge_pool, kHugeThreads, 0, stream>>>(
+          M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, ws.counters, ws.bitmaps,
+          ws.ranks, c_pos, c_crd, c_val);
     }
     SCORCH_HIP_CHECK(hipGetLastError());
   }
-  // one workgroup per CU's worth of LDS; more only queue up behind them
-  const int64_t huge_rows = known ? known->huge + known->giant - known->split : M;
-  const unsigned lds_pool = (unsigned)(huge_rows < 512 ? huge_rows : 512);
-  if (lds_pool == 0) {
-  } else if (narrow) {
-    spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
-        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, nullptr, ws.counters, c_pos, c_crd, c_val);
-  } else if (!NUMERIC && N > 32 * 16384 && N <= 32 * 32768) {
-    // the symbolic pass keeps no ranks or sums: its bitmap can be twice as wide, one range instead of two
-    spgemm_lds_bitmap_kernel<T, NUMERIC, NUMERIC ? 16384 : 32768, kHugeThreads, 0, 1, 3>
-        <<<lds_pool, kHugeThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows,
-                                                nullptr, ws.counters, c_pos, c_crd, c_val);
-  } else if (N <= kLdsBitmapColumns) {
-    spgemm_lds_bitmap_kernel<T, NUMERIC, 16384, kHugeThreads, 0, 1, 3><<<lds_pool, kHugeThreads, 0, stream>>>(
-        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, nullptr, ws.counters, c_pos, c_crd, c_val);
-  } else {
-    spgemm_huge_kernel<T, NUMERIC><<<ws.huge_pool, kHugeThreads, 0, stream>>>(
-        M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.huge_rows, ws.counters, ws.bitmaps,
-        ws.ranks, c_pos, c_crd, c_val);
-  }
-  SCORCH_HIP_CHECK(hipGetLastError());
   if (!NUMERIC) {
     const int64_t n = (int64_t)M + 1;
-    unsigned long long *grand_total = reinterpret_cast<unsigned long long *>(ws.counters + 6);
+    unsigned long long *grand_total = reinterpret_cast<unsigned long long *>(ws.counters + counter(6));
     const SplitCount split = {ws.pool > 0 ? ws.split_rows : nullptr, ws.split_bits, words};
     int64_t *report = sync ? sync->target() : nullptr;
     const int64_t sequence = sync ? sync->sequence() : 0;
-    if (ws.pool > 0) {
+    if (ws.pool > 0 && !bins && listed > 0) {
       spgemm_split_count_kernel<<<(unsigned)ws.pool, kBlockThreads, 0, stream>>>(ws.counters, split, c_pos);
       SCORCH_HIP_CHECK(hipGetLastError());
     }
@@ -1647,17 +2054,63 @@ int spgemm_numeric_entry(const char *fn, int64_t M, int64_t K, int64_t N, const 
                          const int32_t *a_crd, const T *a_val, const int32_t *b_pos,
                          const int32_t *b_crd, const T *b_val, const int32_t *c_pos, int32_t *c_crd,
                          T *c_val, void *workspace, size_t workspace_bytes, void *stream,
-                         const int64_t *report = nullptr) {
+                         const int64_t *report = nullptr, void *bin_memory = nullptr, size_t bin_bytes = 0) {
   if (int rc = spgemm_check(fn, M, K, N, a_pos, a_crd, b_pos, b_crd, c_pos, workspace, workspace_bytes,
                             sizeof(T)))
     return rc;
   if (M == 0 || N == 0 || K == 0) return SCORCH_HIP_OK;
   const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, sizeof(T));
   SpgemmReport known;
-  if (report) known = {report[0], report[1], report[2], report[3], report[4], report[5], report[6]};
+  Bins bins;
+  if (report) {
+    known = report_of(report);
+    if (bin_memory) bins = spgemm_bins(static_cast<char *>(bin_memory), ws.counters, N, sizeof(T), known.huge + known.giant,
+                                       known.products, known.batches);
+    if (bins.total > bin_bytes)
+      return fail(SCORCH_HIP_EWORKSPACE, "%s: bins of %zu bytes needed, %zu given", fn, bins.total, bin_bytes);
+  }
   return spgemm_run<T, true>((int)M, (int)N, a_pos, a_crd, a_val, b_pos, b_crd, b_val,
                              const_cast<int32_t *>(c_pos), c_crd, c_val, ws,
-                             static_cast<hipStream_t>(stream), report ? &known : nullptr);
+                             static_cast<hipStream_t>(stream), kShortRows | kLongRows, report ? &known : nullptr, nullptr,
+                             bins.n > 0 ? &bins : nullptr);
+}
+
+// The second half of the symbolic pass.
+template <typename T>
+int spgemm_symbolic_entry(const char *fn, int64_t M, int64_t K, int64_t N, const int32_t *a_pos,
+                          const int32_t *a_crd, const T *a_val, const int32_t *b_pos, const int32_t *b_crd, const T *b_val,
+                          int32_t *c_pos, void *workspace, size_t workspace_bytes, void *bin_memory, size_t bin_bytes,
+                          int64_t *report, void *stream) {
+  if (int rc = spgemm_check(fn, M, K, N, a_pos, a_crd, b_pos, b_crd, c_pos, workspace, workspace_bytes,
+                            sizeof(T)))
+    return rc;
+  SCORCH_REQUIRE(report != nullptr, "%s: report is NULL", fn);
+  if (M == 0) return SCORCH_HIP_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  SpgemmReport known = report_of(report);
+  const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, sizeof(T));
+  Bins bins;
+  if (bin_memory) bins = spgemm_bins(static_cast<char *>(bin_memory), ws.counters, N, sizeof(T), known.huge + known.giant,
+                                     known.products, known.batches);
+  if (bins.total > bin_bytes)
+    return fail(SCORCH_HIP_EWORKSPACE, "%s: bins of %zu bytes needed, %zu given", fn, bins.total, bin_bytes);
+  SyncCall sync;
+  if (sync.null()) return fail(SCORCH_HIP_ERUNTIME, "%s: no memory for the report", fn);
+  if (bins.n > 0) {
+    spgemm_bin_rows_kernel<<<(unsigned)((bins.rows + kBlockThreads - 1) / kBlockThreads), kBlockThreads, 0, s>>>(
+        (int)M, bins, a_pos, ws.products, ws.huge_rows, ws.counters, c_pos);
+    SCORCH_HIP_CHECK(hipGetLastError());
+    spgemm_bin_items_kernel<<<(unsigned)bins.rows, kBinItemThreads, 0, s>>>(bins, a_pos, a_crd, b_pos);
+    SCORCH_HIP_CHECK(hipGetLastError());
+    spgemm_bin_kernel<T><<<(unsigned)bins.items, kBinThreads, 0, s>>>(bins, a_pos, a_crd, a_val, b_pos, b_crd, b_val);
+    SCORCH_HIP_CHECK(hipGetLastError());
+    spgemm_bin_count_kernel<<<(unsigned)(bins.rows * bins.n), kBinCountThreads, 0, s>>>(bins, c_pos);
+    SCORCH_HIP_CHECK(hipGetLastError());
+  }
+  if (int rc = spgemm_run<float, false>((int)M, (int)N, a_pos, a_crd, nullptr, b_pos, b_crd, nullptr, c_pos, nullptr, nullptr, ws,
+                                        s, kLongRows, &known, &sync, bins.n > 0 ? &bins : nullptr))
+    return rc;
+  return sync.wait(fn, s, report, 7);
 }
 
 }  // namespace scorch
@@ -1689,18 +2142,21 @@ int scorch_hip_spgemm_csr_symbolic(int64_t M, int64_t K, int64_t N, const int32_
                                   nullptr, c_row_ptr, nullptr, nullptr, ws, s);
 }
 
-int scorch_hip_spgemm_csr_symbolic_planned(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
-                                           const int32_t *a_col_idx, const int32_t *b_row_ptr,
-                                           const int32_t *b_col_idx, int32_t *c_row_ptr, void *workspace,
-                                           size_t workspace_bytes, int64_t *report, void *stream) {
+int scorch_hip_spgemm_csr_symbolic_planned_begin(int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr,
+                                                 const int32_t *a_col_idx, const int32_t *b_row_ptr,
+                                                 const int32_t *b_col_idx, int32_t *c_row_ptr, void *workspace,
+                                                 size_t workspace_bytes, size_t elem_size, int64_t *report,
+                                                 size_t *bin_bytes, void *stream) {
   using namespace scorch;
-  const char *fn = "scorch_hip_spgemm_csr_symbolic_planned";
+  const char *fn = "scorch_hip_spgemm_csr_symbolic_planned_begin";
   if (int rc = spgemm_check(fn, M, K, N, a_row_ptr, a_col_idx, b_row_ptr, b_col_idx, c_row_ptr,
                             workspace, workspace_bytes, 1))
     return rc;
-  SCORCH_REQUIRE(report != nullptr, "%s: report is NULL", fn);
+  SCORCH_REQUIRE(report != nullptr && bin_bytes != nullptr, "%s: report or bin_bytes is NULL", fn);
+  SCORCH_REQUIRE(elem_size == 4 || elem_size == 8, "%s: values of %zu bytes", fn, elem_size);
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (int i = 0; i < kSpgemmReportWords; ++i) report[i] = 0;
+  *bin_bytes = 0;
   if (M == 0) {
     spgemm_reset_kernel<<<1, kBlockThreads, 0, s>>>(static_cast<int *>(workspace), c_row_ptr, 0, nullptr);
     SCORCH_HIP_CHECK(hipGetLastError());
@@ -1708,11 +2164,16 @@ int scorch_hip_spgemm_csr_symbolic_planned(int64_t M, int64_t K, int64_t N, cons
   }
   SyncCall sync;
   if (sync.null()) return fail(SCORCH_HIP_ERUNTIME, "%s: no memory for the report", fn);
-  const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, 1);
+  const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, elem_size);
   if (int rc = spgemm_run<float, false>((int)M, (int)N, a_row_ptr, a_col_idx, nullptr, b_row_ptr, b_col_idx, nullptr,
-                                        c_row_ptr, nullptr, nullptr, ws, s, nullptr, &sync))
+                                        c_row_ptr, nullptr, nullptr, ws, s, kShortRows, nullptr, &sync))
     return rc;
-  return sync.wait(fn, s, report, kSpgemmReportWords);
+  int64_t words[6];
+  if (int rc = sync.wait(fn, s, words, 6)) return rc;  // (the short rows' kernels are still at work)
+  for (int i = 0; i < 4; ++i) report[1 + i] = words[i];
+  report[7] = words[4], report[8] = words[5];
+  *bin_bytes = spgemm_bins(nullptr, nullptr, N, elem_size, words[2] + words[3], words[4], words[5]).total;
+  return SCORCH_HIP_OK;
 }
 
 #define SCORCH_DEFINE_SPGEMM(SUFFIX, T)                                                             \
@@ -1726,17 +2187,27 @@ int scorch_hip_spgemm_csr_symbolic_planned(int64_t M, int64_t K, int64_t N, cons
                                            b_vals, c_row_ptr, c_col_idx, c_vals, workspace,         \
                                            workspace_bytes, stream);                                \
   }                                                                                                 \
+  int scorch_hip_spgemm_csr_symbolic_planned_##SUFFIX(                                               \
+      int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr, const int32_t *a_col_idx,           \
+      const T *a_vals, const int32_t *b_row_ptr, const int32_t *b_col_idx, const T *b_vals,          \
+      int32_t *c_row_ptr, void *workspace, size_t workspace_bytes, void *bins, size_t bin_bytes,     \
+      int64_t *report, void *stream) {                                                               \
+    return scorch::spgemm_symbolic_entry<T>("scorch_hip_spgemm_csr_symbolic_planned_" #SUFFIX, M, K, \
+                                            N, a_row_ptr, a_col_idx, a_vals, b_row_ptr, b_col_idx,   \
+                                            b_vals, c_row_ptr, workspace, workspace_bytes, bins,     \
+                                            bin_bytes, report, stream);                              \
+  }                                                                                                 \
   int scorch_hip_spgemm_csr_numeric_planned_##SUFFIX(                                                \
       int64_t M, int64_t K, int64_t N, const int32_t *a_row_ptr, const int32_t *a_col_idx,           \
       const T *a_vals, const int32_t *b_row_ptr, const int32_t *b_col_idx, const T *b_vals,          \
       const int32_t *c_row_ptr, int32_t *c_col_idx, T *c_vals, void *workspace,                      \
-      size_t workspace_bytes, const int64_t *report, void *stream) {                                 \
+      size_t workspace_bytes, void *bins, size_t bin_bytes, const int64_t *report, void *stream) {   \
     SCORCH_REQUIRE(report && report[0] >= 0, "scorch_hip_spgemm_csr_numeric_planned_" #SUFFIX         \
                    ": no report of a symbolic pass");                                               \
     return scorch::spgemm_numeric_entry<T>("scorch_hip_spgemm_csr_numeric_planned_" #SUFFIX, M, K, N, \
                                            a_row_ptr, a_col_idx, a_vals, b_row_ptr, b_col_idx,      \
                                            b_vals, c_row_ptr, c_col_idx, c_vals, workspace,         \
-                                           workspace_bytes, stream, report);                        \
+                                           workspace_bytes, stream, report, bins, bin_bytes);       \
   }
 
 SCORCH_DEFINE_SPGEMM(f32, float)

@@ -78,9 +78,14 @@ SIGNATURES = {
     "scorch_hip_spgemm_csr_numeric_f64": (ctypes.c_int, _SPGEMM),
     "scorch_hip_spgemm_csr_numeric_i32": (ctypes.c_int, _SPGEMM),
     "scorch_hip_spgemm_csr_numeric_i64": (ctypes.c_int, _SPGEMM),
-    "scorch_hip_spgemm_csr_symbolic_planned": (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
-                                                              _size, ctypes.POINTER(_i64), _ptr]),
-    **{"scorch_hip_spgemm_csr_numeric_planned_" + t: (ctypes.c_int, _SPGEMM[:-1] + [ctypes.POINTER(_i64), _ptr])
+    "scorch_hip_spgemm_csr_symbolic_planned_begin": (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
+                                                                    _size, _size, ctypes.POINTER(_i64),
+                                                                    ctypes.POINTER(_size), _ptr]),
+    **{"scorch_hip_spgemm_csr_symbolic_planned_" + t: (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
+                                                                      _ptr, _size, _ptr, _size, ctypes.POINTER(_i64), _ptr])
+       for t in ("f32", "f64", "i32", "i64")},
+    **{"scorch_hip_spgemm_csr_numeric_planned_" + t: (ctypes.c_int,
+                                                      _SPGEMM[:-1] + [_ptr, _size, ctypes.POINTER(_i64), _ptr])
        for t in ("f32", "f64", "i32", "i64")},
     "scorch_hip_spmm_csr_planned_counters": (_i64, [_i64, _i64, _i64, _i64, _size]),
     **{"scorch_hip_spmm_csr_planned_counted_" + t: (ctypes.c_int, [_i64] * 5 + [_ptr] * 5 + [

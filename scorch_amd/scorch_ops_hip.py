@@ -38,7 +38,7 @@ _empty_like = torch.empty_like
 
 HINT_MOSTLY_EMPTY_ROWS = 0x100      # SCORCH_HIP_HINT_MOSTLY_EMPTY_ROWS of include/scorch_hip.h
 INSPECT_REPORT_INTS = 8             # SCORCH_HIP_INSPECT_REPORT_INTS
-SPGEMM_REPORT_WORDS = 7             # SCORCH_HIP_SPGEMM_REPORT_WORDS
+SPGEMM_REPORT_WORDS = 9             # SCORCH_HIP_SPGEMM_REPORT_WORDS
 _SUFFIX = {torch.float32: "f32", torch.float64: "f64", torch.int32: "i32", torch.int64: "i64"}
 
 
@@ -986,8 +986,8 @@ def spmm_csr_bias_relu_float(result_shape, A_shape, A_mode_indices, A_values, B_
 # ---- SpGEMM --------------------------------------------------------------------
 def _make_spgemm(dtype):
     def kernel(result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mode_indices, B_values):
-        """C = A @ B, all CSR (reference: csrc/kernels.h:52-202).  Two kernels
-        passes with one host read of the result size in between."""
+        """C = A @ B, all CSR (reference: csrc/kernels.h:52-202).  Two
+        passes; the host reads how much memory the long rows take and how large the result is."""
         M, K, N = int(A_shape[0]), int(A_shape[1]), int(B_shape[1])
         if int(B_shape[0]) != K:
             raise ValueError(f"scorch_ops_hip: shape mismatch A{tuple(A_shape)} B{tuple(B_shape)}")
@@ -1010,10 +1010,15 @@ def _make_spgemm(dtype):
             need = L.scorch_hip_spgemm_csr_workspace_bytes(M, N, a_val.element_size())
             ws = _workspace(dev, stream, need)
             c_pos = _empty(M + 1, dtype=torch.int32, device=dev)
-            report = (ctypes.c_int64 * SPGEMM_REPORT_WORDS)()
-            native.check(L.scorch_hip_spgemm_csr_symbolic_planned(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(),
-                                                                  b_pos.data_ptr(), b_crd.data_ptr(), c_pos.data_ptr(),
-                                                                  ws.data_ptr(), ws.numel(), report, stream))
+            report, bin_bytes = (ctypes.c_int64 * SPGEMM_REPORT_WORDS)(), ctypes.c_size_t()
+            native.check(L.scorch_hip_spgemm_csr_symbolic_planned_begin(
+                M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), b_pos.data_ptr(), b_crd.data_ptr(), c_pos.data_ptr(),
+                ws.data_ptr(), ws.numel(), a_val.element_size(), report, ctypes.byref(bin_bytes), stream))
+            bins = _empty(bin_bytes.value, dtype=torch.uint8, device=dev) if bin_bytes.value else None
+            bins_ptr = bins.data_ptr() if bins is not None else None
+            native.check(getattr(L, "scorch_hip_spgemm_csr_symbolic_planned_" + _SUFFIX[dtype])(
+                M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(), b_pos.data_ptr(), b_crd.data_ptr(),
+                b_val.data_ptr(), c_pos.data_ptr(), ws.data_ptr(), ws.numel(), bins_ptr, bin_bytes, report, stream))
             nnz = report[0]
             if nnz < 0:
                 raise native.ScorchHipError(native.EUNSUPPORTED,
@@ -1023,7 +1028,7 @@ def _make_spgemm(dtype):
             fn = getattr(L, "scorch_hip_spgemm_csr_numeric_planned_" + _SUFFIX[dtype])
             native.check(fn(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(),
                             b_pos.data_ptr(), b_crd.data_ptr(), b_val.data_ptr(), c_pos.data_ptr(),
-                            c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), report, stream))
+                            c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), bins_ptr, bin_bytes, report, stream))
         return Tensor(c_val, [[], [c_pos, c_crd]])
     return kernel
 

@@ -436,3 +436,27 @@ def test_hub_rows_shared_out_among_workgroups(oracle, dtype, N):
         else:
             assert oracle.rel_fro(host(c_val), oracle.spgemm_csr_typed(arp, aci, host(av).astype(np.float64), brp, bci,
                                                                        host(bv).astype(np.float64), N)[2]) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("N", [1, 1023, 1025, 8193, 65_537, 131_072])
+def test_long_rows_sorted_by_ranges_of_columns(oracle, dtype, N):
+    """Rows just beyond 4096 products and around the windows of 2048 products and the batches of 512 entries that
+    they are sorted in, with B rows that are empty, that lie in one range and that touch the first and last column."""
+    rng = np.random.default_rng(N)
+    K = 2600
+    width = min(N, 60)
+    blens = rng.integers(0, width + 1, K)
+    blens[:8] = [0, width, min(N, 4097), min(N, 8192), min(N, 30_000), min(N, 2), min(N, 8193), 1]
+    where = [np.sort(rng.choice(N, n, replace=False)) if n > 2 else np.array([0, N - 1][2 - n:], int) for n in blens]
+    where[1] = np.arange(N - width, N)                       # the last columns only
+    brp = np.concatenate([[0], np.cumsum(blens)]).astype(np.int32)
+    bci = np.concatenate(where).astype(np.int32)
+    rows = [np.array(r) for r in ([2], [3], [4], [0, 2, 7], [6], [0], [1], np.arange(511), np.arange(512), np.arange(513),
+                                  np.arange(1024), np.arange(8, 1033), np.arange(K), np.full(1, 5))]
+    rows.insert(4, np.flatnonzero(blens == 0))   # many entries, no products
+    aci = np.concatenate(rows).astype(np.int32)
+    arp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    value = (lambda n: rng.integers(-9, 9, n).astype(dtype)) if np.issubdtype(dtype, np.integer) else \
+        (lambda n: rng.uniform(-1, 1, n).astype(dtype))
+    check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
