@@ -70,10 +70,11 @@ __device__ __forceinline__ int hash_slot(int key, int mask) {
 }
 
 // Slot of `key` in an open-addressing table (empty = -1); inserts it if absent.
-__device__ __forceinline__ int hash_insert(int *keys, int mask, int key) {
+__device__ __forceinline__ int hash_insert(int *keys, int mask, int key, bool &fresh) {
   int s = hash_slot(key, mask);
   for (;;) {
     const int prev = atomicCAS(&keys[s], -1, key);
+    fresh = prev == -1;
     if (prev == -1 || prev == key) return s;
     s = (s + 1) & mask;
   }
@@ -123,18 +124,50 @@ __device__ __forceinline__ void workgroup_store(A *p, A v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Prefix sums and maxima over TEAM lanes (16, or the 64 of a wavefront), inclusive: the exchanges are
+// carried by the operation itself (DPP: row_shr 1, 2, 4, 8 within rows of 16 lanes, then
+// row_bcast 15 and 31 across them).  A shuffle goes through the LDS pipe and is waited for at
+// every step.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or_zero(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+template <int TEAM>
+__device__ __forceinline__ int team_inclusive_sum(int x) {
+  static_assert(TEAM == 16 || TEAM == kWaveSize, "a row of lanes or a wavefront");
+  x += dpp_or_zero<0x111, 0xf>(x);
+  x += dpp_or_zero<0x112, 0xf>(x);
+  x += dpp_or_zero<0x114, 0xf>(x);
+  x += dpp_or_zero<0x118, 0xf>(x);
+  if (TEAM == 16) return x;
+  x += dpp_or_zero<0x142, 0xa>(x);
+  return x + dpp_or_zero<0x143, 0xc>(x);
+}
+template <int TEAM>  // of numbers from 0 up
+__device__ __forceinline__ int team_inclusive_max(int x) {
+  static_assert(TEAM == 16 || TEAM == kWaveSize, "a row of lanes or a wavefront");
+  x = max(x, dpp_or_zero<0x111, 0xf>(x));
+  x = max(x, dpp_or_zero<0x112, 0xf>(x));
+  x = max(x, dpp_or_zero<0x114, 0xf>(x));
+  x = max(x, dpp_or_zero<0x118, 0xf>(x));
+  if (TEAM == 16) return x;
+  x = max(x, dpp_or_zero<0x142, 0xa>(x));
+  return max(x, dpp_or_zero<0x143, 0xc>(x));
+}
+// The last lane's value, for every lane of the team.
+template <int TEAM>
+__device__ __forceinline__ int team_last(int x) {
+  if (TEAM == kWaveSize) return __builtin_amdgcn_readlane(x, kWaveSize - 1);
+  return __shfl(x, wave_lane() | (TEAM - 1));
+}
+
 // Exclusive prefix sum of one int per thread over a workgroup of WAVES
 // wavefronts; `total` receives the sum.  `scratch` holds WAVES ints.
 template <int WAVES>
 __device__ __forceinline__ int block_exclusive_scan_n(int v, int *scratch, int &total) {
   const int lane = wave_lane();
   const int w = threadIdx.x / kWaveSize;
-  int incl = v;
-#pragma unroll
-  for (int off = 1; off < kWaveSize; off <<= 1) {
-    const int up = __shfl_up(incl, off);
-    if (lane >= off) incl += up;
-  }
+  const int incl = team_inclusive_sum<kWaveSize>(v);
   __syncthreads();  // scratch may still be read from a previous call
   if (lane == kWaveSize - 1) scratch[w] = incl;
   __syncthreads();
@@ -154,27 +187,18 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *scratch, int &to
 }
 
 // Exclusive scan of `v` over a workgroup of WAVES wavefronts and, behind the same two
-// barriers, the workgroup's minimum of `lo` and maximum of `hi`.
+// barriers, the workgroup's minimum of `lo` (from 0 up) and maximum of `hi` (from -1 up).
 template <int WAVES>
 __device__ __forceinline__ int block_scan_min_max(int v, int &total, int &lo, int &hi, int *scan_scratch,
                                                   int *min_scratch, int *max_scratch) {
   const int lane = wave_lane();
   const int w = threadIdx.x / kWaveSize;
-  int incl = v;
-#pragma unroll
-  for (int off = 1; off < kWaveSize; off <<= 1) {
-    const int up = __shfl_up(incl, off);
-    if (lane >= off) incl += up;
-  }
-#pragma unroll
-  for (int off = kWaveSize / 2; off > 0; off >>= 1) {
-    const int l = __shfl_xor(lo, off), h = __shfl_xor(hi, off);
-    lo = l < lo ? l : lo;
-    hi = h > hi ? h : hi;
-  }
+  const int incl = team_inclusive_sum<kWaveSize>(v);
+  lo = INT_MAX - team_inclusive_max<kWaveSize>(INT_MAX - lo);
+  hi = team_inclusive_max<kWaveSize>(hi + 1) - 1;
   __syncthreads();  // the scratch arrays may still be read from a previous call
-  if (lane == kWaveSize - 1) scan_scratch[w] = incl;
-  if (lane == 0) {
+  if (lane == kWaveSize - 1) {
+    scan_scratch[w] = incl;
     min_scratch[w] = lo;
     max_scratch[w] = hi;
   }
@@ -185,8 +209,8 @@ __device__ __forceinline__ int block_scan_min_max(int v, int &total, int &lo, in
     const int part = scan_scratch[i];
     if (i < w) before += part;
     all += part;
-    lo = min_scratch[i] < lo ? min_scratch[i] : lo;
-    hi = max_scratch[i] > hi ? max_scratch[i] : hi;
+    lo = i == 0 ? min_scratch[0] : min(lo, min_scratch[i]);
+    hi = i == 0 ? max_scratch[0] : max(hi, max_scratch[i]);
   }
   total = all;
   return before + incl - v;
@@ -201,12 +225,29 @@ __device__ __forceinline__ int block_scan_min_max(int v, int &total, int &lo, in
 // TEAM entries of A at once -- thread t reads entry t, its B row's start and
 // length -- turns the lengths into offsets with a prefix sum, and then walks the
 // batch's products flat: product x belongs to the entry e with off[e] <= x <
-// off[e + 1], found by bisection in LDS.  All lanes stay busy and consecutive
-// lanes read consecutive entries of a B row.
+// off[e + 1].  Workgroups find it by bisection in LDS.  Teams of up to a wavefront
+// mark the first product of every entry that has any and take the running maximum of
+// the marks: six vector instructions per product instead of six dependent LDS reads with their
+// compares.  All lanes stay busy and consecutive lanes read consecutive entries of a B row.
+constexpr int kProductsInFlight = 4;
+
 template <int TEAM, typename A>
 struct ProductBatch {
   int index[2 * TEAM];  // [e]: first product of entry e within the batch; [TEAM + e]: where its B row starts
   A a_val[TEAM];
+};
+template <typename A>
+struct MarkedBatch {
+  int start[kWaveSize];                                 // where entry e's B row starts, less its first product
+  A a_val[kWaveSize];
+  unsigned mark[kProductsInFlight * kWaveSize / 4];     // a byte per product: the entry it is the first of, or 0
+};
+template <typename A> struct ProductBatch<kWaveSize, A> : MarkedBatch<A> {};
+template <typename A>
+struct ProductBatch<16, A> {
+  int start[16];
+  A a_val[16];
+  unsigned mark[kProductsInFlight * 16 / 4];
 };
 
 // Teams of up to a wavefront (64 lanes, or an aligned part of one) need no
@@ -219,19 +260,10 @@ __device__ __forceinline__ void team_sync() {
 template <int TEAM>
 __device__ __forceinline__ int team_exclusive_scan(int v, int *scratch, int &total) {
   if (TEAM > kWaveSize) return block_exclusive_scan_n<TEAM / kWaveSize>(v, scratch, total);
-  const int lane = wave_lane();
-  const int t = lane % TEAM;
-  int incl = v;
-#pragma unroll
-  for (int off = 1; off < TEAM; off <<= 1) {
-    const int up = __shfl_up(incl, off);
-    if (t >= off) incl += up;
-  }
-  total = __shfl(incl, lane - t + TEAM - 1);
+  const int incl = team_inclusive_sum<TEAM <= kWaveSize ? TEAM : kWaveSize>(v);
+  total = team_last<TEAM>(incl);
   return incl - v;
 }
-
-constexpr int kProductsInFlight = 4;
 
 // One step of the walk over a batch's products: products x0, x0 + TEAM, ... (U of
 // them) of this thread.  Their bisections interleave and their loads from B are all
@@ -264,6 +296,42 @@ __device__ __forceinline__ void product_step(int x0, int total, const int *__res
     if (!PARTIAL || x0 + u * TEAM < total) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
 }
 
+// The same for a team of up to a wavefront, U = kProductsInFlight: `first` and `len` are this lane's entry's
+// products, `carried` the last entry that began before the step (its products may go on).
+template <int TEAM, bool NUMERIC, typename T, typename A, typename Fn>
+__device__ __forceinline__ void marked_step(int x0, int total, int t, int first, int len, int &carried,
+                                            const int *__restrict__ b_crd, const T *__restrict__ b_val,
+                                            ProductBatch<TEAM, A> &batch, Fn &fn) {
+  constexpr int U = kProductsInFlight;
+  unsigned char *const marks = reinterpret_cast<unsigned char *>(batch.mark);
+  batch.mark[t] = 0u;
+  wave_lds_sync();
+  // (entries with products start at different ones: no two lanes write one byte)
+  if (len > 0 && first >= x0 && first < x0 + U * TEAM) marks[first - x0] = (unsigned char)t;
+  wave_lds_sync();
+  int e[U], q[U], col[U];
+  A b[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) e[u] = team_inclusive_max<TEAM>(marks[u * TEAM + t]);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int last = team_last<TEAM>(e[u]);
+    e[u] = max(e[u], carried);
+    carried = max(carried, last);
+    // (slots beyond the last product read that product again and hand nothing to fn)
+    q[u] = min(x0 + u * TEAM + t, total - 1) + batch.start[e[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u > 0 && x0 + u * TEAM >= total) break;  // uniform over the team
+    col[u] = b_crd[q[u]];
+    b[u] = NUMERIC ? (A)b_val[q[u]] : (A)0;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (x0 + u * TEAM + t < total) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
+}
+
 // fn(column, product) for every product of A entries [a_lo, a_hi); `t` is the
 // thread's number in the team.  Uniform over the team.
 template <int TEAM, bool NUMERIC, typename T, typename A, typename Fn>
@@ -285,6 +353,14 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
     int total = 0;
     const int first = team_exclusive_scan<TEAM>(len, scan_scratch, total);
     team_sync<TEAM>();  // the previous batch has been read by everyone
+    if constexpr (TEAM <= kWaveSize) {
+      batch.start[t] = lo - first;
+      if (NUMERIC) batch.a_val[t] = av;
+      int carried = 0;
+      for (int x = 0; x < total; x += U * TEAM)
+        marked_step<TEAM, NUMERIC, T, A>(x, total, t, first, len, carried, b_crd, b_val, batch, fn);
+      continue;
+    } else {
     batch.index[t] = first;
     batch.index[TEAM + t] = lo;
     if (NUMERIC) batch.a_val[t] = av;
@@ -296,6 +372,7 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
       product_step<TEAM, NUMERIC, U, true, T, A>(x + t, total, b_crd, b_val, batch, fn);
     else if (x + t < total)
       product_step<TEAM, NUMERIC, 1, false, T, A>(x + t, total, b_crd, b_val, batch, fn);
+    }
   }
 }
 
@@ -455,6 +532,23 @@ inline int bounds_rows_per_group(int64_t M) {
   return (int)(rows < 32 ? 32 : rows > kBoundsRows ? kBoundsRows : rows);
 }
 
+// Products of entries p, p + stride, ... (N of them, those before hi): all of A's columns are requested before the
+// first is used, then all of B's row pointers.
+template <int N>
+__device__ __forceinline__ long long products_of_entries(int p, int stride, int hi, const int *__restrict__ a_crd,
+                                                   const int *__restrict__ b_pos) {
+  int j[N];
+  long long sum = 0;
+#pragma unroll
+  for (int u = 0; u < N; ++u) j[u] = a_crd[min(p + u * stride, hi - 1)];
+  Vec<int, 2> b[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) b[u] = load_vec<int, 2>(b_pos + j[u]);
+#pragma unroll
+  for (int u = 0; u < N; ++u) sum += p + u * stride < hi ? b[u].v[1] - b[u].v[0] : 0;
+  return sum;
+}
+
 __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     int M, int rows_per_group, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
     const int *__restrict__ b_pos, int *__restrict__ products, int *__restrict__ small_rows,
@@ -462,6 +556,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     int64_t *__restrict__ report, int64_t sequence) {
   constexpr int G = 8;  // lanes per row
   constexpr int kStep = kBlockThreads / G;
+  constexpr int kRowsAtOnce = 4;          // whose loads a lane has in flight together
   __shared__ int s_long[kBoundsRows];
   __shared__ int s_very_long[kBoundsRows];
   __shared__ int s_list[4][kBoundsRows];  // medium, huge, small, giant
@@ -488,30 +583,47 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
 
   const int t = threadIdx.x % G;
   const int64_t first = (int64_t)blockIdx.x * rows_per_group;
-  for (int it = 0; it < rows_per_group / kStep; ++it) {
-    const int64_t row = first + it * kStep + threadIdx.x / G;
-    int lo = 0, hi = 0;
-    if (row < M) {
-      lo = a_pos[row];
-      hi = a_pos[row + 1];
-    }
-    const int entries = hi - lo;
-    const bool is_long = entries > kBoundsLongRow;
-    if (is_long) {
-      if (t == 0) {
-        if (hi - lo > kBoundsWaveRow) s_very_long[atomicAdd(&s_n[5], 1)] = (int)row;
-        else s_long[atomicAdd(&s_n[4], 1)] = (int)row;
-      }
-      hi = lo;
-    }
-    long long sum = 0;
-    for (int p = lo + t; p < hi; p += G) {
-      const int j = a_crd[p];
-      sum += b_pos[j + 1] - b_pos[j];
+  const int64_t end = min(first + rows_per_group, (int64_t)M);
+  for (int64_t base = first + threadIdx.x / G; base < end; base += kRowsAtOnce * kStep) {
+    int lo[kRowsAtOnce], hi[kRowsAtOnce], j[kRowsAtOnce][2];
+    Vec<int, 2> b[kRowsAtOnce][2];
+#pragma unroll
+    for (int r = 0; r < kRowsAtOnce; ++r) {
+      const int64_t row = min(base + r * kStep, end - 1);
+      lo[r] = a_pos[row];
+      hi[r] = a_pos[row + 1];
     }
 #pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    if (row < M && t == 0 && !is_long) file_row((int)row, sum, entries);
+    for (int r = 0; r < kRowsAtOnce; ++r)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        j[r][u] = -1;
+        if (lo[r] + t + u * G < hi[r]) j[r][u] = a_crd[lo[r] + t + u * G];
+      }
+#pragma unroll
+    for (int r = 0; r < kRowsAtOnce; ++r)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        b[r][u].v[0] = b[r][u].v[1] = 0;
+        if (j[r][u] >= 0) b[r][u] = load_vec<int, 2>(b_pos + j[r][u]);
+      }
+#pragma unroll
+    for (int r = 0; r < kRowsAtOnce; ++r) {
+      const int64_t row = base + r * kStep;
+      if (row >= end) break;
+      const int entries = hi[r] - lo[r];
+      if (entries > kBoundsLongRow) {
+        if (t > 0) continue;
+        if (entries > kBoundsWaveRow) s_very_long[atomicAdd(&s_n[5], 1)] = (int)row;
+        else s_long[atomicAdd(&s_n[4], 1)] = (int)row;
+        continue;
+      }
+      long long sum = (long long)(b[r][0].v[1] - b[r][0].v[0]) + (b[r][1].v[1] - b[r][1].v[0]);
+      for (int p = lo[r] + t + 2 * G; p < hi[r]; p += 4 * G) sum += products_of_entries<4>(p, G, hi[r], a_crd, b_pos);
+#pragma unroll
+      for (int off = G / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+      if (t == 0) file_row((int)row, sum, entries);
+    }
   }
   __syncthreads();
 
@@ -519,11 +631,9 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
   for (int i = threadIdx.x / kWaveSize; i < n_long; i += kWavesPerBlock) {  // uniform over the wavefront
     const int r = s_long[i];
     long long part = 0;
-#pragma unroll 4
-    for (int p = a_pos[r] + wave_lane(); p < a_pos[r + 1]; p += kWaveSize) {
-      const int j = a_crd[p];
-      part += b_pos[j + 1] - b_pos[j];
-    }
+    const int hi = a_pos[r + 1];
+    for (int p = a_pos[r] + wave_lane(); p < hi; p += 8 * kWaveSize)
+      part += products_of_entries<8>(p, kWaveSize, hi, a_crd, b_pos);
 #pragma unroll
     for (int off = kWaveSize / 2; off > 0; off >>= 1) part += __shfl_xor(part, off);
     if (wave_lane() == 0) file_row(r, part, a_pos[r + 1] - a_pos[r]);
@@ -532,11 +642,9 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
   for (int i = 0; i < n_very_long; ++i) {  // uniform over the workgroup
     const int r = s_very_long[i];
     long long part = 0;
-#pragma unroll 4
-    for (int p = a_pos[r] + (int)threadIdx.x; p < a_pos[r + 1]; p += kBlockThreads) {
-      const int j = a_crd[p];
-      part += b_pos[j + 1] - b_pos[j];
-    }
+    const int hi = a_pos[r + 1];
+    for (int p = a_pos[r] + (int)threadIdx.x; p < hi; p += 8 * kBlockThreads)
+      part += products_of_entries<8>(p, kBlockThreads, hi, a_crd, b_pos);
 #pragma unroll
     for (int off = kWaveSize / 2; off > 0; off >>= 1) part += __shfl_xor(part, off);
     __syncthreads();
@@ -609,7 +717,7 @@ constexpr int kMicroSlots = 64;
 // entries being walked.
 template <typename A, bool NUMERIC, int TEAM, int TEAMS, int SLOTS, int PRODUCTS>
 struct TeamTables {
-  int keys[TEAMS][SLOTS];
+  alignas(16) int keys[TEAMS][SLOTS];
   A vals[TEAMS][NUMERIC ? SLOTS : 1];
   ProductBatch<TEAM, A> batch[TEAMS];
 };
@@ -617,56 +725,65 @@ struct TeamTables {
 // One row of C by team number `team` of TEAM lanes (a wavefront or an aligned
 // part of one; this lane is its number t): hash the row's products, count or
 // compact the occupied slots, sort by rank.
+// `bound`: the row's products.
+// The table is as large as the row asks for, twice its entries (numeric pass: known) or products and
+// at least TEAM: most rows of a tier are short, and clearing and going through 512 slots for a
+// row of 40 entries cost more than its products.
 template <typename T, bool NUMERIC, int TEAM, int TEAMS, int SLOTS, int PRODUCTS>
 __device__ __forceinline__ void spgemm_team_row(
-    TeamTables<typename Acc<T>::type, NUMERIC, TEAM, TEAMS, SLOTS, PRODUCTS> &lds, int team, int t, int row,
+    TeamTables<typename Acc<T>::type, NUMERIC, TEAM, TEAMS, SLOTS, PRODUCTS> &lds, int team, int t, int row, int bound,
     const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
     const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
     int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
   const int lane = wave_lane();
 
-  for (int s = t; s < SLOTS; s += TEAM) {
+  const int out = NUMERIC ? c_pos[row] : 0;
+  const int n = NUMERIC ? c_pos[row + 1] - out : 0;
+  const int most = 2 * (NUMERIC ? n : bound);
+  int slots = TEAM;  // uniform over the team
+  while (slots < most) slots <<= 1;
+  for (int s = t; s < slots; s += TEAM) {
     lds.keys[team][s] = -1;
     if (NUMERIC) lds.vals[team][s] = (A)0;
   }
   wave_lds_sync();
 
+  int found = 0;
+
   for_each_product<TEAM, NUMERIC, T, A>(
       a_pos[row], a_pos[row + 1], t, a_crd, a_val, b_pos, b_crd, b_val, lds.batch[team], nullptr,
       [&](int col, A product) {
-        const int slot = hash_insert(lds.keys[team], SLOTS - 1, col);
+        bool fresh;
+        const int slot = hash_insert(lds.keys[team], slots - 1, col, fresh);
         if (NUMERIC) lds_accumulate<A>(&lds.vals[team][slot], product);
+        else found += fresh ? 1 : 0;
       });
-  wave_lds_sync();
-
-  // Count the occupied slots; in the numeric pass, also compact them, in place: a
-  // step's TEAM slots are read by all lanes before any is written, and entry
-  // number `at` never lies beyond the slot it came from.
-  int n = 0;
-  for (int base = 0; base < SLOTS; base += TEAM) {
-    const int key = lds.keys[team][base + t];
-    A val = (A)0;
-    if (NUMERIC) val = lds.vals[team][base + t];
-    unsigned long long occupied = __ballot(key != -1) >> (lane - t);  // the team's lanes from bit 0
-    if (TEAM < kWaveSize) occupied &= (1ull << (TEAM % kWaveSize)) - 1ull;
-    if (NUMERIC) {
-      wave_lds_sync();  // everyone has read this step's slots
-      if (key != -1) {
-        const int at = n + __popcll(occupied & ((1ull << t) - 1ull));
-        lds.keys[team][at] = key;
-        lds.vals[team][at] = val;
-      }
-    }
-    n += __popcll(occupied);
-  }
   if (!NUMERIC) {
-    if (t == 0) c_pos[row] = n;
+    found = team_inclusive_sum<TEAM>(found);
+    if (t == TEAM - 1) c_pos[row] = found;
     return;
   }
   wave_lds_sync();
 
-  const int out = c_pos[row];
+  // The occupied slots are compacted in place: a step's TEAM slots are read by all
+  // lanes before any is written, and entry number `at` never lies beyond the slot it came from.
+  int compacted = 0;
+  for (int base = 0; base < slots; base += TEAM) {
+    const int key = lds.keys[team][base + t];
+    const A val = lds.vals[team][base + t];
+    unsigned long long occupied = __ballot(key != -1) >> (lane - t);  // the team's lanes from bit 0
+    if (TEAM < kWaveSize) occupied &= (1ull << (TEAM % kWaveSize)) - 1ull;
+    wave_lds_sync();  // everyone has read this step's slots
+    if (key != -1) {
+      const int at = compacted + __popcll(occupied & ((1ull << t) - 1ull));
+      lds.keys[team][at] = key;
+      lds.vals[team][at] = val;
+    }
+    compacted += __popcll(occupied);
+  }
+  wave_lds_sync();
+
   // Whole wavefronts with more than a key per lane sort by buckets: counting
   // ranks below costs n compares per key, half of this tier's time at 256 keys a
   // row.  The keys' range is cut into 2 * TEAM equal power-of-two intervals; a
@@ -679,7 +796,8 @@ __device__ __forceinline__ void spgemm_team_row(
     constexpr int kBuckets = 2 * TEAM;
     constexpr int kPerLane = PRODUCTS / TEAM;
     constexpr int kCrowd = 16;
-    int *const cnt = lds.batch[team].index;
+    static_assert(TEAM < kWaveSize || sizeof(lds.batch[team]) >= kBuckets * sizeof(int), "the counts lie where the batch was");
+    int *const cnt = reinterpret_cast<int *>(&lds.batch[team]);
     int key[kPerLane], pos[kPerLane];
     int key_min = INT_MAX, key_max = -1;
 #pragma unroll
@@ -691,12 +809,8 @@ __device__ __forceinline__ void spgemm_team_row(
         key_max = key[i] > key_max ? key[i] : key_max;
       }
     }
-#pragma unroll
-    for (int off = TEAM / 2; off > 0; off >>= 1) {
-      const int lo = __shfl_xor(key_min, off), hi = __shfl_xor(key_max, off);
-      key_min = lo < key_min ? lo : key_min;
-      key_max = hi > key_max ? hi : key_max;
-    }
+    key_min = INT_MAX - team_last<TEAM>(team_inclusive_max<TEAM>(INT_MAX - key_min));
+    key_max = team_last<TEAM>(team_inclusive_max<TEAM>(key_max));  // (every lane has a key)
     int shift = 0;
     while (((key_max - key_min) >> shift) >= kBuckets) ++shift;
     cnt[t] = 0;
@@ -710,11 +824,7 @@ __device__ __forceinline__ void spgemm_team_row(
     int unused = 0;
     const int before = team_exclusive_scan<TEAM>(c0 + c1, nullptr, unused);
     int crowd = c0 > c1 ? c0 : c1;
-#pragma unroll
-    for (int off = TEAM / 2; off > 0; off >>= 1) {
-      const int other = __shfl_xor(crowd, off);
-      crowd = other > crowd ? other : crowd;
-    }
+    crowd = team_last<TEAM>(team_inclusive_max<TEAM>(crowd));
     if (crowd <= kCrowd) {  // uniform
       wave_lds_sync();  // everyone has read the counts
       cnt[2 * t] = before;
@@ -747,11 +857,18 @@ __device__ __forceinline__ void spgemm_team_row(
     }
   }
 
-  // Rank = number of smaller keys (keys are distinct): the sorted position.
+  // Rank = number of smaller keys (keys are distinct): the sorted position.  Four keys to a read, the
+  // last ones padded (n is at most half of the table's slots, or a multiple of four).
+  if (t < (-n & 3)) lds.keys[team][n + t] = INT_MAX;
+  wave_lds_sync();
+  const int4 *const fours = reinterpret_cast<const int4 *>(lds.keys[team]);
   for (int e = t; e < n; e += TEAM) {
     const int key = lds.keys[team][e];
     int rank = 0;
-    for (int x = 0; x < n; ++x) rank += lds.keys[team][x] < key ? 1 : 0;
+    for (int x = 0; 4 * x < n; ++x) {
+      const int4 k = fours[x];
+      rank += (k.x < key ? 1 : 0) + (k.y < key ? 1 : 0) + (k.z < key ? 1 : 0) + (k.w < key ? 1 : 0);
+    }
     c_crd[out + rank] = key;
     c_val[out + rank] = (T)lds.vals[team][e];
   }
@@ -787,7 +904,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_tiny_kernel(
   const int bound = mine < M ? products[mine] : INT_MAX;
   if (bound <= kMicroProducts)
     spgemm_team_row<T, NUMERIC, kMicroTeam, kQuarters, kMicroSlots, kMicroProducts>(
-        lds[w].quarter, q, lane % kMicroTeam, (int)mine, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd,
+        lds[w].quarter, q, lane % kMicroTeam, (int)mine, bound, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd,
         c_val);
 #pragma unroll
   for (int i = 0; i < kQuarters; ++i) {
@@ -795,7 +912,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_tiny_kernel(
     if (b > kMicroProducts && b <= kTinyProducts) {
       wave_lds_sync();  // the tables' previous users are done
       spgemm_team_row<T, NUMERIC, kWaveSize, 1, kTinySlots, kTinyProducts>(
-          lds[w].wave, 0, lane, (int)(first + i), a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
+          lds[w].wave, 0, lane, (int)(first + i), b, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
     }
   }
 }
@@ -821,10 +938,9 @@ __device__ __forceinline__ void spgemm_medium_rows(
     MediumTables<typename Acc<T>::type, NUMERIC, PRODUCTS, THREADS> &lds, int block, int n_blocks,
     const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
     const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
-    const int *__restrict__ rows, const int *__restrict__ counters, int *__restrict__ c_pos,
-    int *__restrict__ c_crd, T *__restrict__ c_val) {
+    const int *__restrict__ products, const int *__restrict__ rows, const int *__restrict__ counters,
+    int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
-  constexpr int kSlots = 2 * PRODUCTS;
   constexpr int kBuckets = PRODUCTS / 2;
   constexpr int kBucketCrowd = 32;  // a fuller bucket sends the row to the bitonic sort
   auto &s_keys = lds.keys;
@@ -843,7 +959,11 @@ __device__ __forceinline__ void spgemm_medium_rows(
   // slower: these rows are short enough for the counter's round trip to show)
   for (int idx = block; idx < n_rows; idx += n_blocks) {
     const int row = rows[idx];
-    for (int s = tid; s < kSlots; s += THREADS) {
+    const int out = NUMERIC ? c_pos[row] : 0;
+    const int most = 2 * (NUMERIC ? c_pos[row + 1] - out : products[row]);
+    int slots = THREADS;  // a table as large as the row asks for; uniform
+    while (slots < most) slots <<= 1;
+    for (int s = tid; s < slots; s += THREADS) {
       s_keys[s] = -1;
       if (NUMERIC) s_vals[s] = (A)0;
     }
@@ -851,20 +971,29 @@ __device__ __forceinline__ void spgemm_medium_rows(
       for (int bkt = tid; bkt < kBuckets; bkt += THREADS) s_cnt[bkt] = 0;
     __syncthreads();
 
+    int found = 0;
     for_each_product<THREADS, NUMERIC, T, A>(
         a_pos[row], a_pos[row + 1], tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan,
         [&](int col, A product) {
-          const int slot = hash_insert(s_keys, kSlots - 1, col);
+          bool fresh;
+          const int slot = hash_insert(s_keys, slots - 1, col, fresh);
           if (NUMERIC) lds_accumulate<A>(&s_vals[slot], product);
+          else found += fresh ? 1 : 0;
         });
+    if (!NUMERIC) {
+      int n = 0;
+      (void)block_exclusive_scan_n<THREADS / kWaveSize>(found, s_scan, n);
+      if (tid == 0) c_pos[row] = n;
+      continue;  // (the scan's barriers have everyone past the table)
+    }
     __syncthreads();
 
-    // Each thread owns kRun slots, a workgroup's width apart (neighbouring threads
+    // Each thread owns `run` slots, a workgroup's width apart (neighbouring threads
     // on neighbouring LDS banks); an exclusive scan of the per-thread counts
     // places the occupied ones.
-    constexpr int kRun = kSlots / THREADS;
+    const int run = slots / THREADS;
     int mine = 0, key_min = INT_MAX, key_max = -1;
-    for (int s = 0; s < kRun; ++s) {
+    for (int s = 0; s < run; ++s) {
       const int key = s_keys[s * THREADS + tid];
       if (key != -1) {
         ++mine;
@@ -873,13 +1002,7 @@ __device__ __forceinline__ void spgemm_medium_rows(
       }
     }
     int n = 0;
-    int at = NUMERIC ? block_scan_min_max<THREADS / kWaveSize>(mine, n, key_min, key_max, s_scan, s_red[0], s_red[1])
-                     : block_exclusive_scan_n<THREADS / kWaveSize>(mine, s_scan, n);
-    if (!NUMERIC) {
-      if (tid == 0) c_pos[row] = n;
-      __syncthreads();
-      continue;
-    }
+    int at = block_scan_min_max<THREADS / kWaveSize>(mine, n, key_min, key_max, s_scan, s_red[0], s_red[1]);
 
     // Sorting the row's (column, value) pairs.  First choice: buckets.  The
     // columns' range [min, max] is cut into kBuckets equal power-of-two intervals
@@ -890,7 +1013,7 @@ __device__ __forceinline__ void spgemm_medium_rows(
     // of the whole row takes over.
     int shift = 0;
     while (((key_max - key_min) >> shift) >= kBuckets) ++shift;  // n > 0 here: the row has products
-    for (int s = 0; s < kRun; ++s) {  // (the counts were cleared with the tables)
+    for (int s = 0; s < run; ++s) {  // (the counts were cleared with the tables)
       const int key = s_keys[s * THREADS + tid];
       if (key != -1) atomicAdd(&s_cnt[(key - key_min) >> shift], 1);
     }
@@ -911,7 +1034,7 @@ __device__ __forceinline__ void spgemm_medium_rows(
         start += c;
       }
       __syncthreads();
-      for (int s = 0; s < kRun; ++s) {
+      for (int s = 0; s < run; ++s) {
         const int key = s_keys[s * THREADS + tid];
         if (key != -1) {
           const int pos = atomicAdd(&s_cnt[(key - key_min) >> shift], 1);  // ends as the bucket's end
@@ -920,7 +1043,6 @@ __device__ __forceinline__ void spgemm_medium_rows(
         }
       }
       __syncthreads();
-      const int out = c_pos[row];
       for (int e = tid; e < n; e += THREADS) {
         const int key = s_ck[e];
         const int bkt = (key - key_min) >> shift;
@@ -933,7 +1055,7 @@ __device__ __forceinline__ void spgemm_medium_rows(
       __syncthreads();
       continue;
     } else {
-      for (int s = 0; s < kRun; ++s) {
+      for (int s = 0; s < run; ++s) {
         const int key = s_keys[s * THREADS + tid];
         if (key != -1) {
           s_ck[at] = key;
@@ -965,7 +1087,6 @@ __device__ __forceinline__ void spgemm_medium_rows(
         }
       }
     }
-    const int out = c_pos[row];
     for (int e = tid; e < n; e += THREADS) {
       c_crd[out + e] = s_ck[e];
       c_val[out + e] = (T)s_cv[e];
@@ -978,11 +1099,11 @@ template <typename T, bool NUMERIC, int PRODUCTS, int COUNTER, int THREADS>
 __global__ __launch_bounds__(THREADS) void spgemm_medium_kernel(
     const int *__restrict__ a_pos, const int *__restrict__ a_crd, const T *__restrict__ a_val,
     const int *__restrict__ b_pos, const int *__restrict__ b_crd, const T *__restrict__ b_val,
-    const int *__restrict__ rows, const int *__restrict__ counters, int *__restrict__ c_pos,
-    int *__restrict__ c_crd, T *__restrict__ c_val) {
+    const int *__restrict__ products, const int *__restrict__ rows, const int *__restrict__ counters,
+    int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
   __shared__ MediumTables<typename Acc<T>::type, NUMERIC, PRODUCTS, THREADS> lds;
   spgemm_medium_rows<T, NUMERIC, PRODUCTS, COUNTER, THREADS>(lds, blockIdx.x, gridDim.x, a_pos, a_crd, a_val, b_pos,
-                                                             b_crd, b_val, rows, counters, c_pos, c_crd, c_val);
+                                                             b_crd, b_val, products, rows, counters, c_pos, c_crd, c_val);
 }
 
 // ---- rows beyond that: a bitmap over all columns -------------------------------------------
@@ -1302,15 +1423,17 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_small_matrix_kernel(
   block -= n_bitmap;
   if (block < n_medium) {
     spgemm_medium_rows<T, NUMERIC, kSmallProducts, 2, kBlockThreads>(lds.medium, block, n_medium, a_pos, a_crd, a_val, b_pos,
-                                                                    b_crd, b_val, small_rows, counters, c_pos, c_crd, c_val);
+                                                                    b_crd, b_val, products, small_rows, counters, c_pos,
+                                                                    c_crd, c_val);
     return;
   }
   block -= n_medium;
   const int w = threadIdx.x / kWaveSize;
   const int row = block * kWavesPerBlock + w;
-  if (row >= M || products[row] > kTinyProducts) return;
+  const int bound = row < M ? products[row] : INT_MAX;
+  if (bound > kTinyProducts) return;
   spgemm_team_row<T, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts>(
-      lds.tiny, w, wave_lane(), row, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
+      lds.tiny, w, wave_lane(), row, bound, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
 }
 
 // ---- rows shared out among workgroups --------------------------------------------------------
@@ -1949,7 +2072,7 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
       SCORCH_HIP_CHECK(hipGetLastError());
       if (small_blocks) {
         spgemm_medium_kernel<T, NUMERIC, kSmallProducts, 2, kBlockThreads><<<small_blocks, kBlockThreads, 0, stream>>>(
-            a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.small_rows, ws.counters, c_pos, c_crd, c_val);
+            a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows, ws.counters, c_pos, c_crd, c_val);
         SCORCH_HIP_CHECK(hipGetLastError());
       }
       if (bitmap_blocks && narrow) {
@@ -1962,7 +2085,7 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
         // beside them (with 8-byte sums, no more than 256)
         constexpr int kThreads = sizeof(A) > 4 ? kBlockThreads : kHugeThreads;
         spgemm_medium_kernel<T, NUMERIC, kMediumProducts, 0, kThreads><<<bitmap_blocks, kThreads, 0, stream>>>(
-            a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
+            a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
       }
       SCORCH_HIP_CHECK(hipGetLastError());
     }
