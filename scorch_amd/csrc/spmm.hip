@@ -45,7 +45,7 @@ template <typename T, int VEC, int EPI>
 __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
     int M, int N, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
     const T *__restrict__ vals, const T *__restrict__ B, T *__restrict__ C,
-    const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int n_tiles,
+    const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int n_tiles, int lanes_per_tile,
     int64_t blocks_per_tile, int *__restrict__ carry_row, T *__restrict__ carry_val,
     const Boundary *__restrict__ bounds, SpmmBatch batch, int zero_filled, int *__restrict__ counters) {
   using A = typename Acc<T>::type;
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
   const int w = threadIdx.x / kWaveSize;
   const TileMap where = map_workgroup(blockIdx.x, n_tiles, blocks_per_tile);
   const int64_t chunk = where.block * kWavesPerBlock + w;
-  const int col0 = lane_column<VEC>((where.tile * kWaveSize + lane) * VEC, N);
+  const int col0 = lane < lanes_per_tile ? lane_column<VEC>((where.tile * lanes_per_tile + lane) * VEC, N) : N;
   const bool active = col0 < N;
 
   const int64_t d0 = chunk * items_per_chunk;
@@ -414,7 +414,7 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
   T *carry_val = reinterpret_cast<T *>(
       static_cast<char *>(workspace) +
       align_up((size_t)spmm_num_chunks(M, nnz, N, sizeof(T)) * sizeof(int), 256));
-  const int tile = kWaveSize * VEC;
+  const int lanes = tile_lanes(N, VEC), tile = lanes * VEC;
   const int n_tiles = (N + tile - 1) / tile;
   // a multiple of 8 (see map_workgroup); workgroups past the last chunk find nothing to do
   const int64_t blocks_per_tile = round_up_8((chunks + kWavesPerBlock - 1) / kWavesPerBlock);
@@ -436,7 +436,7 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
   }
   spmm_merge_kernel<T, VEC, EPI><<<grid, kBlockThreads, 0, stream>>>(
       M, N, row_ptr, col_idx, vals, B, C, bias, (int64_t)M + nnz, split.items_per_chunk,
-      split.snap, n_tiles, blocks_per_tile, carry_row, carry_val, bounds, strides, zero_fill ? 1 : 0, counters);
+      split.snap, n_tiles, lanes, blocks_per_tile, carry_row, carry_val, bounds, strides, zero_fill ? 1 : 0, counters);
   SCORCH_HIP_CHECK(hipGetLastError());
   if (timer) SCORCH_HIP_CHECK(hipEventRecord(timer->ev[1], stream));
   mark_launch(stream);
@@ -1137,7 +1137,8 @@ SCORCH_DEFINE_SPMM_PLANNED_COUNTED(i64, int64_t)
 
 int64_t scorch_hip_spmm_csr_planned_counters(int64_t batch, int64_t M, int64_t nnz, int64_t N, size_t elem_size) {
   if (batch <= 0 || M < 0 || nnz < 0 || N <= 0 || elem_size == 0) return 0;
-  const int64_t columns = 64 * (int64_t)scorch::pick_vec(N, elem_size);
+  const int vec = scorch::pick_vec(N, elem_size);
+  const int64_t columns = (int64_t)scorch::tile_lanes(N, vec) * vec;
   const int64_t tiles = N * (int64_t)elem_size <= 256 ? 1 : (N + columns - 1) / columns;
   return 2 * batch * tiles * scorch::spmm_num_chunks(M, nnz, N, elem_size);
 }

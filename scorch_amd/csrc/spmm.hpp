@@ -314,6 +314,19 @@ int narrow_vec(int64_t N) {
   return vec;
 }
 
+// Vectors in a column tile, one lane each.  A vector moved back from the row's end (lane_column) shares
+// columns with the one before it.  Lanes of one wavefront may: they do everything in step.  Two tiles
+// may not: the wavefronts that fold a row (finish_part) read its sums where they stand, and one would
+// read what the other has written.  So a last tile of a single such vector is given another by tiles of
+// fewer lanes (N = 257: 63 + 2 vectors instead of 64 + 1; as many tiles, the same loads of B).
+inline int tile_lanes(int64_t N, int vec) {
+  const int64_t vectors = (N + vec - 1) / vec;
+  int lanes = kWaveSize;
+  if (N % vec != 0)
+    while (vectors > lanes && vectors % lanes == 1) --lanes;
+  return lanes;
+}
+
 // First column of a lane: its place in the row, moved back where the vector would pass the end.
 // (>= N: the lane has nothing to do.)
 template <int VEC>

@@ -157,6 +157,47 @@ def test_rows_folded_in_one_launch_are_the_second_launchs_bit_for_bit(dtype, N, 
     assert all(int(c.abs().sum()) == 0 for c in H._counter_buffers.values())
 
 
+@pytest.mark.parametrize("dtype, N", [(np.float32, 129), (np.float32, 257), (np.float32, 258), (np.float32, 259), (np.float32, 513),
+                                      (np.float32, 771), (np.int32, 257), (np.float64, 129), (np.float64, 257), (np.float64, 385),
+                                      (np.int64, 513)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_folded_rows_of_widths_whose_last_column_tile_is_one_ragged_vector(dtype, N, act, monkeypatch):
+    """A last vector that is moved back from the row's end shares columns with the one before it: were that
+    another column tile's, the tiles' folds would read one another's sums, and count a part or the
+    bias twice.  Rows of two to sixteen chunks, of more than sixteen, and many such rows at once."""
+    if act and dtype != np.float32:
+        pytest.skip("the fused epilogue is fp32")
+    monkeypatch.setenv("SCORCH_HIP_TILED", "0")                   # (a copy by column tiles would take the wide ones)
+    rng = np.random.default_rng(N)
+    K = 300
+    lens = rng.integers(0, 5, 1500)
+    lens[::50] = rng.integers(300, 900, 30)
+    lens[[7, 702, 1499]] = [30_000, 12_000, 9000]
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    integer = np.issubdtype(dtype, np.integer)
+    ci = rng.integers(0, K, rp[-1]).astype(np.int32)
+    v = (rng.integers(-9, 9, rp[-1]) if integer else rng.uniform(-1, 1, rp[-1])).astype(dtype)
+    b = (rng.integers(-9, 9, (K, N)) if integer else rng.standard_normal((K, N))).astype(dtype)
+    A = STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (lens.size, K))
+    bd, bias = dev(b), torch.randn(N, device="cuda") if act else None
+    general = (lambda: scorch.spmm_bias_act(A, bd, bias)) if act else (lambda: scorch.matmul(A, bd))
+    first = general()
+    dense = np.zeros((lens.size, K))
+    np.add.at(dense, (np.repeat(np.arange(lens.size), lens), ci), v.astype(np.float64))
+    want = dense @ b.astype(np.float64) + (host(bias).astype(np.float64) if act else 0)
+    # a row's error is below its entries' count, in fp32's or fp64's unit, times the sum of magnitudes (first
+    # 1, then n additions); integers are exact
+    unit = 0.0 if integer else np.finfo(dtype).eps
+    bound = np.zeros_like(dense)
+    np.add.at(bound, (np.repeat(np.arange(lens.size), lens), ci), np.abs(v.astype(np.float64)))
+    bound = unit * (lens[:, None] + 2) * (bound @ np.abs(b.astype(np.float64)) + 10)
+    assert (np.abs(host(first).astype(np.float64) - want) <= bound).all()
+    for _ in range(30):
+        got = native.host().spmm(A, bd, bias, act)
+        assert got is not None and torch.equal(got, first)
+    assert all(int(c.abs().sum()) == 0 for c in H._counter_buffers.values())
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
 @pytest.mark.parametrize("rows, entries", [(1, 0), (1, 447), (1, 448), (3, 1500), (5000, 20_000), (900_000, 5_000_000)])
 def test_vector_product_from_a_plans_boundaries(dtype, rows, entries):
