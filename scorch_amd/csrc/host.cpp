@@ -17,9 +17,11 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdlib>
+#include <exception>
 #include <vector>
 
 #include "../../include/scorch_hip_unstable.h"
@@ -51,6 +53,17 @@ struct Mark {
   uint32_t version = 0;
   int64_t numel = 0;
 };
+
+// Runs an entry point's body: whatever C++ throws in it (no memory for the result, an operand without
+// storage) leaves as the Python exception that torch itself would raise.
+template <typename Body> PyObject *guarded(Body body) {
+  try {
+    return body();
+  } catch (...) {
+    torch::translate_exception_to_python(std::current_exception());
+    return nullptr;
+  }
+}
 
 uint32_t version_of(const at::Tensor &t) { return t.unsafeGetTensorImpl()->version_counter().current_version(); }
 
@@ -172,11 +185,12 @@ Operand *operand_of(PyObject *a) {
 }
 
 // A tensor argument that a kernel can read as it is (or, `transposed`: that is the transpose of one).
+// (Without storage: what torch.vmap and torch.func.grad hand in.)
 bool fits(PyObject *obj, const Operand *o, int64_t dims, at::ScalarType dtype, bool transposed = false) {
   if (!THPVariable_CheckExact(obj)) return false;
   const at::Tensor &t = THPVariable_Unpack(obj);
   return t.layout() == at::kStrided && t.is_cuda() && t.get_device() == o->device && t.scalar_type() == dtype &&
-         t.dim() == dims && !t.is_neg() &&
+         t.dim() == dims && !t.is_neg() && t.has_storage() &&
          (transposed ? dims == 2 && t.stride(0) == 1 && t.stride(1) == t.size(0) && t.size(0) > 1 && t.size(1) > 1
                      : t.is_contiguous());
 }
@@ -249,9 +263,10 @@ bool first_sight(PyObject *b, int64_t K, int64_t N) {
   PyObject *d = dict_of(b);
   PyObject *volatile_ = item(d, n_volatile);
   if (volatile_ && volatile_ != Py_False) return true;
+  const at::Tensor &t = THPVariable_Unpack(b);
+  if (t.is_inference()) return true;  // (no version counter: writes go unseen, so no copy is ever kept of it)
   if (item(d, n_seen) || item(d, n_tiled)) return false;
   PyObject *epoch = item(d, n_epoch);
-  const at::Tensor &t = THPVariable_Unpack(b);
   PyObject *stamp = Py_BuildValue("(kKLLl)", (unsigned long)version_of(t),
                                   (unsigned long long)reinterpret_cast<uintptr_t>(t.const_data_ptr()), (long long)K, (long long)N,
                                   epoch ? PyLong_AsLong(epoch) : 0L);
@@ -268,7 +283,7 @@ const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N) {
   if (!c || !PyTuple_CheckExact(c) || PyTuple_GET_SIZE(c) != 6) return nullptr;
   const at::Tensor &t = THPVariable_Unpack(b);
   PyObject *volatile_ = item(d, n_volatile), *epoch = item(d, n_epoch);
-  if (volatile_ && volatile_ != Py_False) return nullptr;
+  if (t.is_inference() || (volatile_ && volatile_ != Py_False)) return nullptr;
   const long e = epoch ? PyLong_AsLong(epoch) : 0;
   if (PyLong_AsUnsignedLong(PyTuple_GET_ITEM(c, 0)) != version_of(t) ||
       PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(c, 1)) != reinterpret_cast<unsigned long long>(t.const_data_ptr()) ||
@@ -287,7 +302,7 @@ bool tiles_switched_off() {
 template <typename T> const T *at_(const void *p) { return static_cast<const T *>(p); }
 
 // spmm(a, b, bias or None, act): C = act(A @ B + bias), or y = A @ x for a vector.  None: not decided yet.
-PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
+PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
   if (n != 4 || !g_ops) return none();
   PyObject *a = args[0], *b = args[1], *bias = args[2];
   const int act = PyLong_AsLong(args[3]);
@@ -390,7 +405,7 @@ PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // sddmm(mask, A, B): (values, row coordinates or None).  None: not decided yet.
-PyObject *host_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
+PyObject *sddmm_body(PyObject *const *args, Py_ssize_t n) {
   if (n != 3 || !g_ops) return none();
   Operand *o = operand_of(args[0]);
   if (!o || o->dtype != at::kFloat || !fits(args[1], o, 2, at::kFloat) || !fits(args[2], o, 2, at::kFloat)) return none();
@@ -437,7 +452,7 @@ PyObject *host_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n) {
 
 // remember(a, kind, width, act, ints, tensors, workspace, may_tile, mask_values, rows, path, other_path): keep a decided
 // product with the STensor it was decided for.  The last of eight `tensors` is the row pointer of a coordinate operand.
-PyObject *host_remember(PyObject *, PyObject *args) {
+PyObject *remember_body(PyObject *args) {
   PyObject *a, *ints, *tensors, *rows, *path, *other;
   int kind, act, may_tile, mask_values;
   long long width, ws;
@@ -547,7 +562,7 @@ Attention *attention_of(PyObject *row, PyObject *col) {
 
 // attention(q, k, v, row_ptr, col_idx, scale, form).  `form` 0: bf16; 1: fp32; 2: fp32, for a caller that wants the three
 // separate steps where the mask fills its blocks too thinly for the fused kernel.  None: not decided yet.
-PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
+PyObject *attention_body(PyObject *const *args, Py_ssize_t n) {
   if (n != 7 || !g_ops) return none();
   Attention *t = attention_of(args[3], args[4]);
   if (!t) return none();
@@ -563,7 +578,7 @@ PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (q.scalar_type() != (form ? at::kFloat : at::kBFloat16) || !q.is_cuda() || q.dim() != 3 || q.sizes() != k.sizes() || q.sizes() != v.sizes() || !q.is_contiguous() ||
       !k.is_contiguous() || !v.is_contiguous() || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() ||
       k.device() != q.device() || v.device() != q.device() || q.device() != THPVariable_Unpack(args[3]).device() ||
-      q.is_neg() || k.is_neg() || v.is_neg())
+      q.is_neg() || k.is_neg() || v.is_neg() || !q.has_storage() || !k.has_storage() || !v.has_storage())
     return none();
   const int64_t H = q.size(0), S = q.size(1), D = q.size(2);
   AttentionRoute *r = nullptr;
@@ -605,7 +620,7 @@ PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // remember_attention(row_ptr, col_idx, weakref(col_idx), kind, (H, S, D), model tensor, ints, tensors, workspace)
-PyObject *host_remember_attention(PyObject *, PyObject *args) {
+PyObject *remember_attention_body(PyObject *args) {
   PyObject *row, *col, *ref, *model, *ints, *tensors;
   int kind;
   long long H, S, D, ws;
@@ -618,7 +633,7 @@ PyObject *host_remember_attention(PyObject *, PyObject *args) {
   Attention *t = attention_of(row, col);
   if (!t) {
     const at::Tensor &r = THPVariable_Unpack(row), &c = THPVariable_Unpack(col);
-    if (r.is_inference() || c.is_inference()) return none();
+    if (r.is_inference() || c.is_inference() || !r.has_storage() || !c.has_storage()) return none();
     t = reinterpret_cast<Attention *>(AttentionType.tp_alloc(&AttentionType, 0));
     if (!t) return nullptr;
     t->routes = new std::vector<AttentionRoute>();
@@ -672,6 +687,14 @@ PyObject *host_advance(PyObject *, PyObject *) {
   ++g_generation;
   return none();
 }
+
+PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) { return guarded([&] { return spmm_body(args, n); }); }
+PyObject *host_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n) { return guarded([&] { return sddmm_body(args, n); }); }
+PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  return guarded([&] { return attention_body(args, n); });
+}
+PyObject *host_remember(PyObject *, PyObject *args) { return guarded([&] { return remember_body(args); }); }
+PyObject *host_remember_attention(PyObject *, PyObject *args) { return guarded([&] { return remember_attention_body(args); }); }
 
 PyMethodDef methods[] = {
     {"bind", host_bind, METH_VARARGS, nullptr},

@@ -283,7 +283,9 @@ def mark_volatile(*objs, volatile: bool = True) -> None:
 
 
 def is_volatile(t: torch.Tensor) -> bool:
-    return bool(getattr(t, "_scorch_volatile", False)) or \
+    """Whether nothing derived from the tensor's values is kept: it is marked so, or is an inference
+    tensor, which has no version counter to tell a write by."""
+    return t.is_inference() or bool(getattr(t, "_scorch_volatile", False)) or \
         bool(getattr(getattr(t, "_scorch_origin", None), "_scorch_volatile", False))
 
 

@@ -262,3 +262,61 @@ def test_new_columns_under_known_row_pointers(rows, K, N, per_row):
     rp[-1] += 1
     with pytest.raises(ValueError, match="row_ptr"):
         product(torch.zeros_like(ci), vals)
+
+
+def test_no_memory_for_a_decided_products_result_is_an_error_to_catch(monkeypatch):
+    """The native call path allocates the result itself: without memory for it the caller gets torch's
+    OutOfMemoryError, as from the general way, and the next product works."""
+    monkeypatch.setattr(H, "_empty", H._torch_empty)              # (the allocation in native code, not the tests' poisoned one)
+    rows, N = 1 << 19, 512                                        # a result of 1 GiB, from operands of a few MB
+    rp = torch.arange(rows + 1, dtype=torch.int32, device="cuda")
+    ci = torch.arange(rows, dtype=torch.int32, device="cuda") % 64
+    A = STensor.from_csr_arrays(rp, ci, torch.ones(rows, device="cuda"), (rows, 64))
+    b = torch.randn(64, N, device="cuda")
+    S = 1 << 14
+    mask = (torch.arange(0, S + 1, dtype=torch.int32, device="cuda") * 64,
+            torch.arange(S * 64, dtype=torch.int32, device="cuda") % 64 + torch.arange(S, dtype=torch.int32, device="cuda").div(
+                64, rounding_mode="floor").repeat_interleave(64) * 64)
+    q = torch.randn(128, S, 64, device="cuda").to(torch.bfloat16)     # 256 MiB
+    for _ in range(3):
+        scorch.matmul(A, b)
+        H.sparse_attention_bf16(q, q, q, *mask, 0.125)
+    assert native.host().spmm(A, b, None, 0) is not None and native.host().attention(q, q, q, *mask, 0.125, 0) is not None
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            native.host().spmm(A, b, None, 0)
+        with pytest.raises(torch.OutOfMemoryError):
+            scorch.matmul(A, b)
+        with pytest.raises(torch.OutOfMemoryError):
+            H.sparse_attention_bf16(q, q, q, *mask, 0.125)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(scorch.matmul(A, b)[:64], b)
+
+
+@pytest.mark.parametrize("N", [8, 512])
+def test_decided_products_of_inference_and_of_wrapped_tensors(N, monkeypatch):
+    """A dense operand without a version counter is multiplied like any other (and never copied by column
+    tiles); one without storage -- torch.vmap, torch.func.grad -- is an error to catch, not an abort."""
+    monkeypatch.setattr(H, "_empty", H._torch_empty)
+    rng = np.random.default_rng(3)
+    A, dense = _operand(rng, 400, 300, np.float32, "csr")
+    b = torch.randn(300, N, device="cuda")
+    for _ in range(3):
+        scorch.matmul(A, b)
+    with torch.inference_mode():
+        inner = torch.randn(300, N, device="cuda")
+        for _ in range(4):
+            assert _close(scorch.matmul(A, inner), dense @ inner.double().cpu(), np.float32)
+            inner.mul_(0.5)
+    for _ in range(2):
+        assert _close(scorch.matmul(A, inner), dense @ inner.double().cpu(), np.float32)
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda x: scorch.matmul(A, x))(torch.stack([b, b]))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: scorch.matmul(A, x).sum())(b)
+    assert native.host().spmm(A, torch.randn(300, N, device="cuda"), None, 0) is not None

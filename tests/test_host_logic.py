@@ -569,3 +569,27 @@ def test_when_attention_workgroups_take_two_items():
     assert step(np.full(nb, nb), 16, 64, False) == 32 and step(np.full(nb, 4), 64, 64, False) == 0   # eight rounds
     assert step(causal(256), 8, 128, False) == 0                                # four rounds of two workgroups per CU
     assert step(np.array([], np.int64), 16, 64, False) == 0 and step(c4, 16, 48, False) == 0
+
+
+def test_cpp_exceptions_in_the_native_call_path_become_python_exceptions():
+    """An operand without storage (torch.vmap hands one in) makes torch's C++ throw: the caller gets a Python
+    exception, and the process goes on."""
+    import weakref
+
+    from scorch_amd import native
+    host = native.host()
+    row, col = torch.zeros(65, dtype=torch.int32), torch.zeros(4, dtype=torch.int32)
+
+    def throws(x):
+        host.remember_attention(row, col, weakref.ref(col), 2, (1, 64, 32), x, (), (x,), 0)
+        return x
+
+    with pytest.raises(RuntimeError, match="storage"):
+        torch.vmap(throws)(torch.zeros(2, 5))
+
+    def answers_none(x):
+        assert host.remember_attention(x, col, weakref.ref(col), 2, (1, 64, 32), row, (), (), 0) is None
+        assert host.attention(x, x, x, x, col, 1.0, 1) is None
+        return x
+
+    torch.vmap(answers_none)(torch.zeros(2, 5, dtype=torch.int32))
