@@ -219,12 +219,18 @@ def _decided_sddmm(*args):
 _DENSE_NAMES = {"dd": 2, "d": 1}
 
 
+def _named_dense(fmt) -> Optional[int]:
+    """The order of the dense format that a string names; None for anything else (lists and TensorFormat
+    objects name formats too, and are left to the general path)."""
+    return _DENSE_NAMES.get(fmt) if isinstance(fmt, str) else None
+
+
 def matmul(a: Union[torch.Tensor, STensor], b: Union[torch.Tensor, STensor],
            **kwargs: Any) -> Union[torch.Tensor, STensor]:
     """Matrix product.  Keyword arguments as in the reference: ``format`` /
     ``output_format``, ``use_cache``, ``time_dict``."""
     if isinstance(a, STensor) and isinstance(b, torch.Tensor):
-        if not kwargs or (len(kwargs) == 1 and _DENSE_NAMES.get(kwargs.get("format", None)) == b.dim()):
+        if not kwargs or (len(kwargs) == 1 and _named_dense(kwargs.get("format", None)) == b.dim()):
             out = _decided_spmm(a, b, None, 0)
             if out is not None:
                 return out

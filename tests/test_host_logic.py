@@ -593,3 +593,14 @@ def test_cpp_exceptions_in_the_native_call_path_become_python_exceptions():
         return x
 
     torch.vmap(answers_none)(torch.zeros(2, 5, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("fmt", ["dd", ["dense", "dense"], ["d", "d"], parse_format("dd"), ("d", "d")])
+def test_format_arguments_of_every_documented_form_reach_the_dispatch(fmt):
+    """Strings, lists, tuples and TensorFormat objects: on the CPU all of them end at the same refusal."""
+    a, b = sparse_dense_pair()
+    A = STensor.from_torch(a.to_sparse_csr())
+    for call in (lambda: scorch.matmul(A, b, format=fmt), lambda: scorch.matmul(A, b, output_format=fmt),
+                 lambda: scorch.einsum("ij,jk->ik", A, b, format=fmt)):
+        with pytest.raises(RuntimeError, match="HIP devices only"):
+            call()
