@@ -30,6 +30,13 @@
 // global token's block column holds one live key.  Tiles without a live position for the
 // wavefront are skipped in both products and in the exponentials (window of 64 and a global token:
 // 10.5 of 17 tiles remain).
+//
+// A NaN or infinity in a row of V belongs to the queries that attend to that key, and in such a block
+// not to the others, whose probability for it is 0 (0 x NaN is NaN): the three steps never multiply
+// the two.  What goes into LDS is therefore looked at (one fma for two elements); where a partly live
+// block has something non-finite in V, those elements become zeros in LDS and leave a flag (NaN,
+// infinity, -infinity) at the result elements they belong to, which are given it at the end.  (The
+// look costs 1 % -- S = 3,001, 8 heads, D = 64, window of 64 and a global token: 27.0 -> 27.3 us.)
 #include "common.hpp"
 
 namespace scorch {
@@ -80,6 +87,9 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
   constexpr int kCpt = T::kChunksPerThread;
   __shared__ __attribute__((aligned(16))) float s_k[T::kFloats];
   __shared__ __attribute__((aligned(16))) float s_v[T::kFloats];
+  constexpr int kFlagWords = kBlock * D / 32;
+  __shared__ int s_wild;  // MASKED: the last partly live block whose V holds something non-finite
+  __shared__ unsigned s_flags[MASKED ? 3 : 1][MASKED ? kFlagWords : 1];  // bit d of query q's words: result (q, d)
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWaveSize - 1);
@@ -151,7 +161,7 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
   };
   auto fetch_k = [&](int it) { fetch(k_next, Kh, it); };
   auto fetch_v = [&](int it) { fetch(v_next, Vh, it); };
-  auto store_tile = [&]() {
+  auto store_tile = [&](int it, bool partly) {
 #pragma unroll
     for (int u = 0; u < kCpt; ++u) {
       const int chunk = tid + u * kBlockThreads;
@@ -159,15 +169,18 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
       *reinterpret_cast<floatx4 *>(&s_k[at]) = k_next[u];
       *reinterpret_cast<floatx4 *>(&s_v[at]) = v_next[u];
     }
+    if (MASKED && partly) {
+      // infinite or NaN if some element is (a product may overflow too: the block is then looked through in vain)
+      float sum = 0.0f, more = 0.0f;
+#pragma unroll
+      for (int u = 0; u < kCpt; ++u) {
+        sum = fmaf(v_next[u][0], v_next[u][1], sum);
+        more = fmaf(v_next[u][2], v_next[u][3], more);
+      }
+      if (!(fabsf(sum + more) < __builtin_inff())) s_wild = it;
+    }
   };
   const int my_query_in_block = w * 16 + n;
-
-  if (kb_begin < kb_end) {
-    fetch_k(kb_begin);
-    fetch_v(kb_begin);
-    store_tile();
-  }
-  __syncthreads();
 
   // a block that is only partly live: bit j of word i of its mask says whether query i of the block
   // row attends to key j of the block.  The words of the next block are requested a block ahead.
@@ -183,8 +196,16 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
     return bits;
   };
   int mask_at = kb_begin < kb_end ? mask_of(kb_begin) : -1;
+  // (s_wild needs no first value: a number it holds by chance has a block looked through in vain, by everybody)
+  if (kb_begin < kb_end) {
+    fetch_k(kb_begin);
+    fetch_v(kb_begin);
+    store_tile(kb_begin, mask_at >= 0);
+  }
+  __syncthreads();
   unsigned live = own_bits(live_word(mask_at));
 
+  bool flagged = false;  // (the same for the whole workgroup, as what it depends on is)
   for (int it = kb_begin; it < kb_end; ++it) {
     const bool more = it + 1 < kb_end;
     if (more) fetch_k(it + 1);  // in flight while this block is computed (V follows after the scores:
@@ -192,6 +213,7 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
                                 // the K operands)
     const int next_mask_at = more ? mask_of(it + 1) : -1;
     const unsigned long long next_live = live_word(next_mask_at);
+    const int wild_at = MASKED ? s_wild : -1;  // (looked at after the first product, when it has long arrived)
 
     // One block.  WHOLE: every tile has live positions and (unless `partly`) all of them are; otherwise
     // only the 16-key tiles in `tiles` are computed (bits 0 .. 3, the same for the whole wavefront).
@@ -272,6 +294,30 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
           for (int r = 0; r < 4; ++r) l_run += st[t][r];
         }
 
+      if constexpr (!kWhole)
+        if (partly && uniform(wild_at) == it) {  // the whole workgroup comes here, before its second product, or nobody does
+          int own = threadIdx.x;
+          asm volatile("" : "+v"(own));  // (addresses made from it stay in here: the loop has no registers to spare)
+          if (!flagged) {
+            for (int i = own; i < 3 * kFlagWords; i += kBlockThreads) s_flags[i / kFlagWords][i % kFlagWords] = 0u;
+            __syncthreads();
+            flagged = true;
+          }
+          const unsigned long long *words = block_masks + (size_t)mask_at * kBlock;
+#pragma unroll 1
+          for (int i = own; i < kBlock * D; i += kBlockThreads) {
+            const int key = i / D, d = i % D;
+            float &v = s_v[key * kStride + d];
+            if (fabsf(v) < __builtin_inff()) continue;
+            unsigned *flags = s_flags[v > 0.0f ? 1 : v < 0.0f ? 2 : 0] + d / 32;
+#pragma unroll 1
+            for (int q = 0; q < kBlock; ++q)
+              if ((words[q] >> key) & 1ull) atomicOr(flags + q * (D / 32), 1u << (d % 32));
+            v = 0.0f;
+          }
+          __syncthreads();
+        }
+
       // O^T += V^T P^T: step (t, r) contracts keys 16 t + 4 g + r, whose probabilities lane (g, n)
       // holds for query n; the V^T operand is V[that key][16 dt + n]
 #pragma unroll
@@ -301,10 +347,23 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
     live = own_bits(next_live);
 
     __syncthreads();  // every wavefront is done with this tile
-    if (more) store_tile();
+    if (more) store_tile(it + 1, mask_at >= 0);
     __syncthreads();
   }
 
+  if (MASKED && flagged) {
+#pragma unroll
+    for (int dt = 0; dt < kFeat; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int word = my_query_in_block * (D / 32) + dt / 2, bit = 16 * (dt % 2) + 4 * g + r;
+        const bool nan = (s_flags[0][word] >> bit) & 1u, up = (s_flags[MASKED ? 1 : 0][word] >> bit) & 1u,
+                   down = (s_flags[MASKED ? 2 : 0][word] >> bit) & 1u;
+        if (nan || (up && down)) o_acc[dt][r] = __builtin_nanf("");
+        else if (up) o_acc[dt][r] += __builtin_inff();
+        else if (down) o_acc[dt][r] -= __builtin_inff();
+      }
+  }
   const float l = combine_query_lanes(l_run, [](float a, float b) { return a + b; });
   if (part_slot >= 0) {
     // a stretch of a block row: unnormalised sums, their reference maximum and the row sum

@@ -1616,7 +1616,9 @@ def sparse_attention_csr(row_ptr: torch.Tensor, col_idx: torch.Tensor, q: torch.
     reference's sparse attention (bench/bench_sparse_transformer.py:354-372: SDDMM, row softmax and
     SpMM per head) as three launches for all heads.  Any mask, any head dimension; rows of the mask
     without entries give zero rows.  A mask that fills its 64 x 64 blocks and comes back is served by
-    the fused fp32 kernel, which never writes the scores to memory: the same result to rounding."""
+    the fused fp32 kernel, which never writes the scores to memory: the same result to rounding, and
+    a NaN or infinity in a row of v reaches the queries that attend to that key only.  (Where S is a
+    multiple of 64 a first call's SpMM may go by blocks, in which it reaches the block's 64 queries.)"""
     if SPMM_PATH == "auto" and SDDMM_PATH == "auto" and BLOCKED_PATH == "auto":
         out = native.host().attention(q, k, v, row_ptr, col_idx, scale, 2)
         if out is not None:

@@ -164,3 +164,49 @@ def test_sequences_of_any_length_through_the_three_step_call(oracle, S, D, kind)
         out = H.sparse_attention_csr(rp, ci, dq, dk, dv, D ** -0.5)
         assert oracle.rel_fro(out.cpu().numpy(), ref) <= TOL
     assert isinstance(rp._scorch_plan.attention, H.BlockMask) == (S > 1)    # (one entry fills no block)
+
+
+@pytest.mark.parametrize("S", [65, 130, 447, 512, 1500])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_a_non_finite_row_of_v_reaches_the_queries_that_attend_to_it_and_no_others(S, D):
+    """From the first call (three steps) to the later ones (the fused kernel, whose tiles hold the row for all
+    64 queries of a block): NaN, either infinity, both in one sum, values whose products overflow; a
+    key that every query attends to, one that few do, one in a whole block."""
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = (abs(i - j) <= 40) | (i == 0)
+    mask[: S // 2] |= j[:, :] == 5
+    rng = np.random.default_rng(S + D)
+    q, k, v = (rng.standard_normal((2, S, D)).astype(np.float32) for _ in range(3))
+    v[0, 5, 3] = np.inf
+    v[0, S // 2] = np.nan
+    v[0, S - 1, ::2] = -np.inf
+    v[0, S - 2, 1::3] = np.inf                            # (with the row before: NaN where both meet)
+    v[1, S // 3, D - 1] = -np.inf
+    v[1, 7] = 3e38                                        # finite, though a product of two is not
+    v[1, 9] = -3e38
+    scale = 0.5 * D ** -0.5                               # (no probability underflows)
+    want = np.empty((2, S, D))
+    with np.errstate(all="ignore"):
+        for h in range(2):
+            for row in range(S):
+                keys = np.flatnonzero(mask[row])
+                s = scale * (k[h, keys].astype(np.float64) @ q[h, row].astype(np.float64))
+                p = np.exp(s - s.max())
+                want[h, row] = (p / p.sum()) @ v[h, keys].astype(np.float64)
+    rp, ci = (dev(x) for x in csr_of(mask))
+    dq, dk, dv = (dev(x) for x in (q, k, v))
+    finite = np.isfinite(want)
+    assert not finite.all() and finite.mean() > 0.3
+    size = np.abs(want[finite])
+    for call in range(3):
+        out = H.sparse_attention_csr(rp, ci, dq, dk, dv, scale).cpu().numpy()
+        if call == 0 and S % 64 == 0:
+            continue                                      # (the first call's SpMM is by blocks: a block's rows share)
+        np.testing.assert_array_equal(np.isnan(out), np.isnan(want))
+        np.testing.assert_array_equal(np.isposinf(out), np.isposinf(want))
+        np.testing.assert_array_equal(np.isneginf(out), np.isneginf(want))
+        # sums of up to S terms that may cancel, each rounded a few times: against the magnitudes that go in
+        assert (np.abs(out[finite] - want[finite]) <= 1e-5 * np.maximum(size, np.where(size > 1e6, 3e38, 4.0))).all()
+    assert isinstance(rp._scorch_plan.attention, H.BlockMask)
+    if S % 64 == 0:
+        assert np.array_equal(H.sparse_attention_f32(dq, dk, dv, rp, ci, scale).cpu().numpy(), out, equal_nan=True)
