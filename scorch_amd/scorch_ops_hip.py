@@ -1003,36 +1003,50 @@ def _make_spgemm(dtype):
         dev = _device_of(a_pos, a_crd, a_val, b_pos, b_crd, b_val)
         csr_plan(a_pos, a_crd, M, K, "A")      # validates the indices (once per operand)
         csr_plan(b_pos, b_crd, K, N, "B")
-        L = native.lib()
-        with _on_device(dev):
-            stream = _stream(dev)
-            if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError("scorch_ops_hip: the size of a CSR x CSR product has to be read by the host; it cannot "
-                                   "be recorded in a graph")
-            need = L.scorch_hip_spgemm_csr_workspace_bytes(M, N, a_val.element_size())
-            ws = _workspace(dev, stream, need)
-            c_pos = _empty(M + 1, dtype=torch.int32, device=dev)
-            report, bin_bytes = (ctypes.c_int64 * SPGEMM_REPORT_WORDS)(), ctypes.c_size_t()
-            native.check(L.scorch_hip_spgemm_csr_symbolic_planned_begin(
-                M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), b_pos.data_ptr(), b_crd.data_ptr(), c_pos.data_ptr(),
-                ws.data_ptr(), ws.numel(), a_val.element_size(), report, ctypes.byref(bin_bytes), stream))
-            bins = _empty(bin_bytes.value, dtype=torch.uint8, device=dev) if bin_bytes.value else None
-            bins_ptr = bins.data_ptr() if bins is not None else None
-            native.check(getattr(L, "scorch_hip_spgemm_csr_symbolic_planned_" + _SUFFIX[dtype])(
-                M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(), b_pos.data_ptr(), b_crd.data_ptr(),
-                b_val.data_ptr(), c_pos.data_ptr(), ws.data_ptr(), ws.numel(), bins_ptr, bin_bytes, report, stream))
-            nnz = report[0]
-            if nnz < 0:
-                raise native.ScorchHipError(native.EUNSUPPORTED,
-                                            "SpGEMM: the result has 2^31 entries or more, beyond its int32 row pointer")
-            c_crd = _empty(nnz, dtype=torch.int32, device=dev)
-            c_val = _empty(nnz, dtype=dtype, device=dev)
-            fn = getattr(L, "scorch_hip_spgemm_csr_numeric_planned_" + _SUFFIX[dtype])
-            native.check(fn(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(),
-                            b_pos.data_ptr(), b_crd.data_ptr(), b_val.data_ptr(), c_pos.data_ptr(),
-                            c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), bins_ptr, bin_bytes, report, stream))
-        return Tensor(c_val, [[], [c_pos, c_crd]])
+        args = (M, K, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, dev)
+        try:
+            return _spgemm_product(*args)
+        except torch.OutOfMemoryError:
+            pass            # (left before the second try: the exception keeps the first one's memory alive)
+        return _spgemm_product(*args, sort_products=False)
     return kernel
+
+
+def _spgemm_product(M, K, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, dev, sort_products: bool = True) -> Tensor:
+    """The two passes over checked operands.  `sort_products`: the products of the long rows are sorted
+    by ranges of columns, in memory taken for the call (up to 4 GiB); without it they go another, slower
+    way, which needs none."""
+    dtype, L = a_val.dtype, native.lib()
+    with _on_device(dev):
+        stream = _stream(dev)
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("scorch_ops_hip: the size of a CSR x CSR product has to be read by the host; it cannot "
+                               "be recorded in a graph")
+        need = L.scorch_hip_spgemm_csr_workspace_bytes(M, N, a_val.element_size())
+        ws = _workspace(dev, stream, need)
+        c_pos = _empty(M + 1, dtype=torch.int32, device=dev)
+        report, bin_bytes = (ctypes.c_int64 * SPGEMM_REPORT_WORDS)(), ctypes.c_size_t()
+        native.check(L.scorch_hip_spgemm_csr_symbolic_planned_begin(
+            M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), b_pos.data_ptr(), b_crd.data_ptr(), c_pos.data_ptr(),
+            ws.data_ptr(), ws.numel(), a_val.element_size(), report, ctypes.byref(bin_bytes), stream))
+        if not sort_products:
+            bin_bytes.value = 0
+        bins = _empty(bin_bytes.value, dtype=torch.uint8, device=dev) if bin_bytes.value else None
+        bins_ptr = bins.data_ptr() if bins is not None else None
+        native.check(getattr(L, "scorch_hip_spgemm_csr_symbolic_planned_" + _SUFFIX[dtype])(
+            M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(), b_pos.data_ptr(), b_crd.data_ptr(),
+            b_val.data_ptr(), c_pos.data_ptr(), ws.data_ptr(), ws.numel(), bins_ptr, bin_bytes, report, stream))
+        nnz = report[0]
+        if nnz < 0:
+            raise native.ScorchHipError(native.EUNSUPPORTED,
+                                        "SpGEMM: the result has 2^31 entries or more, beyond its int32 row pointer")
+        c_crd = _empty(nnz, dtype=torch.int32, device=dev)
+        c_val = _empty(nnz, dtype=dtype, device=dev)
+        fn = getattr(L, "scorch_hip_spgemm_csr_numeric_planned_" + _SUFFIX[dtype])
+        native.check(fn(M, K, N, a_pos.data_ptr(), a_crd.data_ptr(), a_val.data_ptr(),
+                        b_pos.data_ptr(), b_crd.data_ptr(), b_val.data_ptr(), c_pos.data_ptr(),
+                        c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), bins_ptr, bin_bytes, report, stream))
+    return Tensor(c_val, [[], [c_pos, c_crd]])
 
 
 _spgemm_f32_atomic = _make_spgemm(torch.float32)

@@ -460,3 +460,37 @@ def test_long_rows_sorted_by_ranges_of_columns(oracle, dtype, N):
     value = (lambda n: rng.integers(-9, 9, n).astype(dtype)) if np.issubdtype(dtype, np.integer) else \
         (lambda n: rng.uniform(-1, 1, n).astype(dtype))
     check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("N", [900, 4095, 8193, 65_537, 131_072])
+@pytest.mark.parametrize("refuse", ["products", "result"])
+def test_without_memory_for_the_sorted_products_the_long_rows_go_the_other_way(oracle, dtype, N, refuse, monkeypatch):
+    """The products of the long rows are sorted in memory that a call takes for itself, up to 4 GiB: where
+    there is none, or none left for the result beside it, the product is made without it, a hub row shared
+    out among workgroups included."""
+    rng = np.random.default_rng(N)
+    M, K = 60, 2500
+    blens = rng.integers(0, min(N, 40), K)
+    blens[:3] = [min(N, 40_000), min(N, 9000), 0]
+    brp = np.concatenate([[0], np.cumsum(blens)]).astype(np.int32)
+    bci = np.concatenate([np.sort(rng.choice(N, n, replace=False)) for n in blens if n]).astype(np.int32)
+    rows = [np.sort(rng.choice(K, n, replace=False)) for n in rng.integers(0, 12, M)]
+    rows[5], rows[6], rows[40] = np.arange(K), np.array([0, 1, 2]), np.arange(0, K, 2)
+    aci = np.concatenate(rows).astype(np.int32)
+    arp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    value = (lambda n: rng.integers(-9, 9, n).astype(dtype)) if np.issubdtype(dtype, np.integer) else \
+        (lambda n: rng.uniform(-1, 1, n).astype(dtype))
+    av, bv = value(aci.size), value(bci.size)
+    rp, ci, _ = check(oracle, arp, aci, av, brp, bci, bv, N)  # (the workspace is as large as it needs to be from here on)
+    allocate, refused = H._empty, []
+
+    def without_memory(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8 if refuse == "products" else args[0] == rp[-1] and not refused:
+            refused.append(args)
+            raise torch.OutOfMemoryError("no memory, says the test")
+        return allocate(*args, **kwargs)
+
+    monkeypatch.setattr(H, "_empty", without_memory)
+    other_rp, other_ci, _ = check(oracle, arp, aci, av, brp, bci, bv, N)
+    assert len(refused) == 1 and np.array_equal(rp, other_rp) and np.array_equal(ci, other_ci)
