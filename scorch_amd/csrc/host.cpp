@@ -6,8 +6,8 @@
 // first times an operand comes along.  Once every decision for (operand, width) has been made it
 // hands the outcome -- a Route: which entry point, with which constants -- to this module, which
 // keeps it with the operand and serves the calls that follow: it checks that the operand is
-// still the same unwritten tensors (identity, address, version counter and the generation that
-// forget() and mark_volatile() advance), that the dense operand fits, allocates the result, and
+// still the same unwritten tensors (identity, address, version counter, and the epoch that
+// forget() advances), that the dense operand fits, allocates the result, and
 // calls the library.  Anything else -- another dtype, a view, a graph being captured that would
 // need scratch memory, a pinned kernel path -- is answered with None, and the caller takes the
 // general way, which also words every error.
@@ -30,12 +30,11 @@ namespace {
 
 // ---- names and objects looked up once ---------------------------------------------------------
 PyObject *n_storage, *n_index, *n_value, *n_shape, *n_mode_indices, *n_format, *n_routes, *n_spmm_path, *n_blocked_path,
-    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_dtype, *n_device;
+    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_ones, *n_dtype, *n_device;
 PyObject *g_ops = nullptr;        // scorch_ops_hip's namespace
 PyObject *g_stensor = nullptr;    // the STensor type
 PyObject *g_torch_empty = nullptr;
 PyObject *g_check = nullptr;      // native.check
-int64_t g_generation = 0;         // advanced by forget() and mark_volatile()
 
 PyObject *item(PyObject *dict, PyObject *name) {  // borrowed, or null
   return dict ? PyDict_GetItem(dict, name) : nullptr;
@@ -48,7 +47,8 @@ PyObject *none() { Py_RETURN_NONE; }
 
 // An index tensor as it was when the decisions were made.
 struct Mark {
-  PyObject *obj = nullptr;  // strong
+  PyObject *obj = nullptr;    // strong
+  PyObject *epoch = nullptr;  // strong: the attribute that forget() replaces; null before the first time
   const void *data = nullptr;
   uint32_t version = 0;
   int64_t numel = 0;
@@ -67,12 +67,21 @@ template <typename Body> PyObject *guarded(Body body) {
 
 uint32_t version_of(const at::Tensor &t) { return t.unsafeGetTensorImpl()->version_counter().current_version(); }
 
+// The epoch of a tensor (borrowed, or null).  forget() puts another number in its place, so the same
+// object means that it has not been called.
+PyObject *epoch_of(PyObject *tensor) { return item(dict_of(tensor), n_epoch); }
+bool is_volatile(PyObject *tensor) {
+  PyObject *v = item(dict_of(tensor), n_volatile);
+  return v && v != Py_False;
+}
+
 bool take_mark(Mark &m, PyObject *obj) {
   if (!THPVariable_Check(obj)) return false;
   const at::Tensor &t = THPVariable_Unpack(obj);
   if (!t.is_cuda() || t.is_inference() || !t.is_contiguous()) return false;
   Py_INCREF(obj);
   m.obj = obj;
+  Py_XINCREF(m.epoch = epoch_of(obj));
   m.data = t.const_data_ptr();
   m.version = version_of(t);
   m.numel = t.numel();
@@ -80,7 +89,7 @@ bool take_mark(Mark &m, PyObject *obj) {
 }
 bool unchanged(const Mark &m) {
   const at::Tensor &t = THPVariable_Unpack(m.obj);
-  return t.const_data_ptr() == m.data && version_of(t) == m.version && t.numel() == m.numel;
+  return t.const_data_ptr() == m.data && version_of(t) == m.version && t.numel() == m.numel && epoch_of(m.obj) == m.epoch;
 }
 
 enum Kind { kRows = 0, kPlanned = 1, kBlockedSpmm = 2, kSpmv = 3, kSddmmCsr = 4, kSddmmListed = 5, kSddmmCoo = 6, kBlockedSddmm = 7 };
@@ -99,15 +108,16 @@ struct Route {
   PyObject *keep;     // strong: what `q` and `row_ptr` point into
   PyObject *spmm_path, *other_path;   // strong: the module settings the decision was made under
   uint32_t value_version;
+  PyObject *verdict;                  // SDDMM: the attribute that says whether the mask's values are all 1 (strong, or null)
   const void *value_data;             // SDDMM: the mask's values the verdict in mask_values is about
   PyObject *rows;                     // SDDMM over a CSR mask: the result's row coordinates (strong)
 };
 
 struct Operand {
   PyObject_HEAD
-  int64_t generation;
   PyObject *index, *format, *mode_indices, *value, *shape;  // strong
   Mark first, second;
+  PyObject *value_epoch;  // strong, or null
   bool csr;
   int64_t rows, cols;
   int device;
@@ -119,14 +129,12 @@ void operand_dealloc(PyObject *self) {
   Operand *o = reinterpret_cast<Operand *>(self);
   if (o->routes) {
     for (Route &r : *o->routes) {
-      Py_XDECREF(r.keep);
-      Py_XDECREF(r.spmm_path);
-      Py_XDECREF(r.other_path);
-      Py_XDECREF(r.rows);
+      for (PyObject *p : {r.keep, r.spmm_path, r.other_path, r.rows, r.verdict}) Py_XDECREF(p);
     }
     delete o->routes;
   }
-  for (PyObject *p : {o->index, o->format, o->mode_indices, o->value, o->shape, o->first.obj, o->second.obj})
+  for (PyObject *p : {o->index, o->format, o->mode_indices, o->value, o->shape, o->first.obj, o->second.obj, o->first.epoch,
+                      o->second.epoch, o->value_epoch})
     Py_XDECREF(p);
   Py_TYPE(self)->tp_free(self);
 }
@@ -177,10 +185,10 @@ Operand *operand_of(PyObject *a) {
   PyObject *found = item(p.storage_dict, n_routes);
   if (!found || Py_TYPE(found) != &OperandType) return nullptr;
   Operand *o = reinterpret_cast<Operand *>(found);
-  if (o->generation != g_generation || o->index != p.index || o->format != p.format || o->mode_indices != p.mode_indices ||
+  if (o->index != p.index || o->format != p.format || o->mode_indices != p.mode_indices ||
       o->value != p.value || o->shape != p.shape || o->first.obj != p.first || o->second.obj != p.second)
     return nullptr;
-  if (!unchanged(o->first) || !unchanged(o->second)) return nullptr;
+  if (!unchanged(o->first) || !unchanged(o->second) || epoch_of(o->value) != o->value_epoch) return nullptr;
   return o;
 }
 
@@ -260,13 +268,12 @@ Route *find_route(Operand *o, int64_t width, int act) {
 // Whether a dense operand without a column-tile copy is a new one: then it is marked as seen once, as
 // the general path does (its second product makes the copy), and this product goes without.
 bool first_sight(PyObject *b, int64_t K, int64_t N) {
-  PyObject *d = dict_of(b);
-  PyObject *volatile_ = item(d, n_volatile);
-  if (volatile_ && volatile_ != Py_False) return true;
   const at::Tensor &t = THPVariable_Unpack(b);
-  if (t.is_inference()) return true;  // (no version counter: writes go unseen, so no copy is ever kept of it)
+  // (an inference tensor has no version counter: writes go unseen, so no copy is ever kept of it)
+  if (t.is_inference() || is_volatile(b)) return true;
+  PyObject *d = dict_of(b);
   if (item(d, n_seen) || item(d, n_tiled)) return false;
-  PyObject *epoch = item(d, n_epoch);
+  PyObject *epoch = epoch_of(b);
   PyObject *stamp = Py_BuildValue("(kKLLl)", (unsigned long)version_of(t),
                                   (unsigned long long)reinterpret_cast<uintptr_t>(t.const_data_ptr()), (long long)K, (long long)N,
                                   epoch ? PyLong_AsLong(epoch) : 0L);
@@ -282,8 +289,8 @@ const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N) {
   PyObject *c = item(d, n_tiled);
   if (!c || !PyTuple_CheckExact(c) || PyTuple_GET_SIZE(c) != 6) return nullptr;
   const at::Tensor &t = THPVariable_Unpack(b);
-  PyObject *volatile_ = item(d, n_volatile), *epoch = item(d, n_epoch);
-  if (t.is_inference() || (volatile_ && volatile_ != Py_False)) return nullptr;
+  if (t.is_inference() || is_volatile(b)) return nullptr;
+  PyObject *epoch = epoch_of(b);
   const long e = epoch ? PyLong_AsLong(epoch) : 0;
   if (PyLong_AsUnsignedLong(PyTuple_GET_ITEM(c, 0)) != version_of(t) ||
       PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(c, 1)) != reinterpret_cast<unsigned long long>(t.const_data_ptr()) ||
@@ -416,6 +423,7 @@ PyObject *sddmm_body(PyObject *const *args, Py_ssize_t n) {
   if (!r || r->spmm_path != item(g_ops, n_sddmm_path) || r->other_path != item(g_ops, n_blocked_path)) return none();
   // what is known about the mask's values was found out about these values
   const at::Tensor &vt = THPVariable_Unpack(o->value);
+  if (item(dict_of(o->value), n_ones) != r->verdict) return none();  // (mark_volatile() takes it away)
   if (vt.const_data_ptr() != r->value_data || version_of(vt) != r->value_version || vt.numel() != o->second.numel) return none();
   if (c10::hip::current_device() != o->device) return none();
   hipStream_t stream = c10::hip::getCurrentHIPStream(o->device).stream();
@@ -470,7 +478,7 @@ PyObject *remember_body(PyObject *args) {
     o = reinterpret_cast<Operand *>(OperandType.tp_alloc(&OperandType, 0));
     if (!o) return nullptr;
     o->routes = new std::vector<Route>();
-    o->generation = g_generation;
+    Py_XINCREF(o->value_epoch = epoch_of(p.value));
     o->index = p.index, o->format = p.format, o->mode_indices = p.mode_indices, o->value = p.value, o->shape = p.shape;
     for (PyObject *x : {o->index, o->format, o->mode_indices, o->value, o->shape}) Py_INCREF(x);
     o->csr = p.csr;
@@ -498,9 +506,10 @@ PyObject *remember_body(PyObject *args) {
   r.value_data = vt.const_data_ptr();
   r.value_version = version_of(vt);
   r.keep = tensors, r.spmm_path = path, r.other_path = other, r.rows = rows == Py_None ? nullptr : rows;
-  for (PyObject *x : {r.keep, r.spmm_path, r.other_path, r.rows}) Py_XINCREF(x);
+  r.verdict = item(dict_of(p.value), n_ones);
+  for (PyObject *x : {r.keep, r.spmm_path, r.other_path, r.rows, r.verdict}) Py_XINCREF(x);
   auto drop = [](Route &x) {
-    for (PyObject *y : {x.keep, x.spmm_path, x.other_path, x.rows}) Py_XDECREF(y);
+    for (PyObject *y : {x.keep, x.spmm_path, x.other_path, x.rows, x.verdict}) Py_XDECREF(y);
   };
   if (Route *old = find_route(o, width, act)) {
     std::swap(*old, r);
@@ -528,7 +537,7 @@ struct AttentionRoute {
 };
 struct Attention {
   PyObject_HEAD
-  int64_t generation;
+  PyObject *row_epoch, *col_epoch;  // strong, or null
   const void *row_data, *col_data;
   uint32_t row_version, col_version;
   int64_t row_numel, col_numel;
@@ -541,7 +550,7 @@ void attention_dealloc(PyObject *self) {
     for (AttentionRoute &r : *t->routes) Py_XDECREF(r.keep);
     delete t->routes;
   }
-  Py_XDECREF(t->col_ref);
+  for (PyObject *p : {t->col_ref, t->row_epoch, t->col_epoch}) Py_XDECREF(p);
   Py_TYPE(self)->tp_free(self);
 }
 PyTypeObject AttentionType = {PyVarObject_HEAD_INIT(nullptr, 0)};
@@ -551,7 +560,7 @@ Attention *attention_of(PyObject *row, PyObject *col) {
   PyObject *found = item(dict_of(row), n_attention);
   if (!found || Py_TYPE(found) != &AttentionType) return nullptr;
   Attention *t = reinterpret_cast<Attention *>(found);
-  if (t->generation != g_generation || PyWeakref_GET_OBJECT(t->col_ref) != col) return nullptr;
+  if (PyWeakref_GET_OBJECT(t->col_ref) != col || epoch_of(row) != t->row_epoch || epoch_of(col) != t->col_epoch) return nullptr;
   const at::Tensor &r = THPVariable_Unpack(row), &c = THPVariable_Unpack(col);
   if (r.is_inference() || c.is_inference() || r.const_data_ptr() != t->row_data || version_of(r) != t->row_version ||
       r.numel() != t->row_numel || c.const_data_ptr() != t->col_data || version_of(c) != t->col_version ||
@@ -637,7 +646,8 @@ PyObject *remember_attention_body(PyObject *args) {
     t = reinterpret_cast<Attention *>(AttentionType.tp_alloc(&AttentionType, 0));
     if (!t) return nullptr;
     t->routes = new std::vector<AttentionRoute>();
-    t->generation = g_generation;
+    Py_XINCREF(t->row_epoch = epoch_of(row));
+    Py_XINCREF(t->col_epoch = epoch_of(col));
     t->row_data = r.const_data_ptr(), t->row_version = version_of(r), t->row_numel = r.numel();
     t->col_data = c.const_data_ptr(), t->col_version = version_of(c), t->col_numel = c.numel();
     Py_INCREF(ref);
@@ -683,11 +693,6 @@ PyObject *host_bind(PyObject *, PyObject *args) {
   return none();
 }
 
-PyObject *host_advance(PyObject *, PyObject *) {
-  ++g_generation;
-  return none();
-}
-
 PyObject *host_spmm(PyObject *, PyObject *const *args, Py_ssize_t n) { return guarded([&] { return spmm_body(args, n); }); }
 PyObject *host_sddmm(PyObject *, PyObject *const *args, Py_ssize_t n) { return guarded([&] { return sddmm_body(args, n); }); }
 PyObject *host_attention(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -698,7 +703,6 @@ PyObject *host_remember_attention(PyObject *, PyObject *args) { return guarded([
 
 PyMethodDef methods[] = {
     {"bind", host_bind, METH_VARARGS, nullptr},
-    {"advance", host_advance, METH_NOARGS, nullptr},
     {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(host_spmm)), METH_FASTCALL, nullptr},
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(host_sddmm)), METH_FASTCALL, nullptr},
     {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(host_attention)), METH_FASTCALL, nullptr},
@@ -719,7 +723,7 @@ PyMODINIT_FUNC PyInit__host() {
                {&n_spmm_path, "SPMM_PATH"}, {&n_blocked_path, "BLOCKED_PATH"}, {&n_sddmm_path, "SDDMM_PATH"},
                {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_counters, "_counter_buffers"}, {&n_tiled, "_scorch_tiled"}, {&n_seen, "_scorch_seen"},
                {&n_volatile, "_scorch_volatile"}, {&n_epoch, "_scorch_epoch"}, {&n_attention, "_scorch_attention"},
-               {&n_dtype, "dtype"}, {&n_device, "device"}};
+               {&n_ones, "_scorch_ones"}, {&n_dtype, "dtype"}, {&n_device, "device"}};
   for (const auto &x : names) *x.slot = PyUnicode_InternFromString(x.text);
   OperandType.tp_name = "scorch_amd._host.Operand";
   OperandType.tp_basicsize = sizeof(Operand);

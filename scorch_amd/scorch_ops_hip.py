@@ -239,19 +239,11 @@ def _same(ref, t: torch.Tensor) -> bool:
     return ref is not None and ref() is t
 
 
-def _decide_anew() -> None:
-    """Products that the native call path (csrc/host.cpp) serves without asking this module are all
-    decided again on their next call."""
-    if native._host is not None:
-        native._host.advance()
-
-
 def forget(*objs) -> None:
     """Drop everything this module has derived from the given tensors (or from the tensors of the
     given STensors, results, lists): the next call inspects, plans and copies anew.  For writes that
     PyTorch's version counter does not see -- ``t.data``, raw pointers, numpy / DLPack aliases,
     kernels of other libraries, replays of recorded graphs."""
-    _decide_anew()
     for t in _tensors_of(objs):
         for name in _CACHE_ATTRIBUTES:
             if hasattr(t, name):
@@ -260,7 +252,8 @@ def forget(*objs) -> None:
                 except AttributeError:
                     pass
         try:
-            t._scorch_epoch = _epoch(t) + 1      # plans that live on a partner tensor name this one's epoch
+            # plans that live on a partner tensor, and what the native call path has decided, name this one's epoch
+            t._scorch_epoch = _epoch(t) + 1
         except (AttributeError, RuntimeError):
             pass
 
@@ -270,7 +263,6 @@ def mark_volatile(*objs, volatile: bool = True) -> None:
     recorded graph, buffers another library writes): nothing derived from their values -- the
     column-tile copy, the all-ones verdict -- is kept or used from now on.  What is derived from an
     index tensor (a sparsity pattern) is not affected: use forget() when a pattern is rewritten."""
-    _decide_anew()
     for t in _tensors_of(objs):
         if volatile:
             for name in ("_scorch_tiled", "_scorch_seen", "_scorch_ones", "_scorch_listed"):

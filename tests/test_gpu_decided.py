@@ -320,3 +320,50 @@ def test_decided_products_of_inference_and_of_wrapped_tensors(N, monkeypatch):
     with pytest.raises(RuntimeError):
         torch.func.grad(lambda x: scorch.matmul(A, x).sum())(b)
     assert native.host().spmm(A, torch.randn(300, N, device="cuda"), None, 0) is not None
+
+
+def test_forget_and_mark_volatile_concern_the_tensors_they_name():
+    """What is forgotten, or marked, is decided anew; another operand's decisions stand."""
+    from scorch_amd import workloads
+    rng = np.random.default_rng(11)
+    (A, _), (other, _) = (_operand(rng, 300, 300, np.float32, "csr") for _ in range(2))
+    b = torch.randn(300, 20, device="cuda")
+    S = _operand(rng, 200, 170, np.float32, "csr")[0]
+    q, k = torch.randn(200, 48, device="cuda"), torch.randn(170, 48, device="cuda")
+    rp, ci = (dev(x) for x in workloads.longformer_mask(256))
+    h = torch.randn(2, 256, 64, device="cuda")
+    stands = {
+        "spmm": lambda: native.host().spmm(A, b, None, 0) is not None,
+        "other": lambda: native.host().spmm(other, b, None, 0) is not None,
+        "sddmm": lambda: native.host().sddmm(S, q, k) is not None,
+        "attention": lambda: native.host().attention(h, h, h, rp, ci, 0.2, 1) is not None,
+    }
+
+    def decide():
+        for _ in range(4):
+            scorch.matmul(A, b), scorch.matmul(other, b), scorch.einsum("ij,ik,jk->ij", S, q, k)
+            H.sparse_attention_f32(h, h, h, rp, ci, 0.2)
+        assert all(check() for check in stands.values())
+
+    a_pos, a_crd = A.index.mode_indices[1]
+    for act, gone in ((lambda: H.forget(b), ""), (lambda: H.forget(torch.zeros(3, device="cuda")), ""),
+                      (lambda: H.mark_volatile(b), ""), (lambda: H.mark_volatile(b, volatile=False), ""),
+                      (lambda: H.forget(A), "spmm"), (lambda: H.forget(A.values), "spmm"), (lambda: H.forget(a_pos), "spmm"),
+                      (lambda: H.forget(a_crd), "spmm"), (lambda: H.forget(S.values), "sddmm"),
+                      (lambda: H.mark_volatile(S.values), "sddmm"), (lambda: H.forget(rp), "attention"),
+                      (lambda: H.forget(ci), "attention"), (lambda: H.forget(rp, ci, S, A, other), "spmm other sddmm attention")):
+        decide()
+        act()
+        assert [name for name, check in stands.items() if not check()] == gone.split()
+        H.mark_volatile(S.values, volatile=False)
+    # values rewritten while they were volatile, behind the version counter's back
+    S.values.fill_(1.0)
+    decide()
+    H.mark_volatile(S.values)
+    S.values.data.fill_(2.0)
+    H.mark_volatile(S.values, volatile=False)
+    twice = scorch.einsum("ij,ik,jk->ij", S, q, k).values
+    for _ in range(4):
+        assert torch.equal(scorch.einsum("ij,ik,jk->ij", S, q, k).values, twice)
+    at = [x[0].long().cpu() for x in scorch.einsum("ij,ik,jk->ij", S, q, k).index.mode_indices]
+    assert torch.allclose(twice.cpu(), 2 * (q.double() @ k.double().t()).float().cpu()[at[0], at[1]], rtol=1e-4, atol=1e-4)
