@@ -265,19 +265,19 @@ Route *find_route(Operand *o, int64_t width, int act) {
   return nullptr;
 }
 
-// Whether a dense operand without a column-tile copy is a new one: then it is marked as seen once, as
-// the general path does (its second product makes the copy), and this product goes without.
+// Whether a dense operand without a (valid) column-tile copy comes along for the first time as it is now:
+// then that is noted with it, as the general path does (the second product of the same unchanged
+// operand makes the copy), and this product goes without.
 bool first_sight(PyObject *b, int64_t K, int64_t N) {
   const at::Tensor &t = THPVariable_Unpack(b);
   // (an inference tensor has no version counter: writes go unseen, so no copy is ever kept of it)
   if (t.is_inference() || is_volatile(b)) return true;
-  PyObject *d = dict_of(b);
-  if (item(d, n_seen) || item(d, n_tiled)) return false;
-  PyObject *epoch = epoch_of(b);
+  PyObject *seen = item(dict_of(b), n_seen), *epoch = epoch_of(b);
   PyObject *stamp = Py_BuildValue("(kKLLl)", (unsigned long)version_of(t),
                                   (unsigned long long)reinterpret_cast<uintptr_t>(t.const_data_ptr()), (long long)K, (long long)N,
                                   epoch ? PyLong_AsLong(epoch) : 0L);
-  const bool marked = stamp && PyObject_SetAttr(b, n_seen, stamp) == 0;
+  const int again = stamp && seen ? PyObject_RichCompareBool(seen, stamp, Py_EQ) : 0;
+  const bool marked = stamp && again == 0 && PyObject_SetAttr(b, n_seen, stamp) == 0;
   Py_XDECREF(stamp);
   if (!marked) PyErr_Clear();
   return marked;

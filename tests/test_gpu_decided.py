@@ -367,3 +367,22 @@ def test_forget_and_mark_volatile_concern_the_tensors_they_name():
         assert torch.equal(scorch.einsum("ij,ik,jk->ij", S, q, k).values, twice)
     at = [x[0].long().cpu() for x in scorch.einsum("ij,ik,jk->ij", S, q, k).index.mode_indices]
     assert torch.allclose(twice.cpu(), 2 * (q.double() @ k.double().t()).float().cpu()[at[0], at[1]], rtol=1e-4, atol=1e-4)
+
+
+def test_a_wide_operand_that_is_rewritten_before_every_product_is_served_by_the_native_path():
+    """A width at which a dense operand that stays as it is gets a copy by column tiles: one that does not is
+    multiplied as it lies, without asking Python; left alone, it gets its copy on the second product."""
+    rng = np.random.default_rng(12)
+    A, dense = _operand(rng, 1024, 256, np.float32, "csr")
+    b = torch.randn(256, 1024, device="cuda")
+    for _ in range(2):
+        scorch.matmul(A, b)
+    for step in range(4):
+        b.mul_(0.5)
+        out = native.host().spmm(A, b, None, 0)
+        assert out is not None and _close(out, dense @ b.double().cpu(), np.float32)
+    copied = native.lib().scorch_hip_dense_tiled_recommended(256, 1024, A.values.numel(), 4)
+    assert (native.host().spmm(A, b, None, 0) is None) == bool(copied)      # unchanged since: the general path's turn
+    for _ in range(3):
+        assert _close(scorch.matmul(A, b), dense @ b.double().cpu(), np.float32)
+    assert copied and b._scorch_tiled[0] == b._version and native.host().spmm(A, b, None, 0) is not None
