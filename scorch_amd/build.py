@@ -102,10 +102,26 @@ HOST_SRC = os.path.join(SRC_DIR, "host.cpp")
 HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 
 
+def host_built_for() -> str:
+    """What a module built here is bound to: torch's C++ interface and the interpreter's.  The text is
+    compiled into it (csrc/host.cpp)."""
+    import torch
+    return "scorch_amd._host for torch %s, Python %d.%d" % ((torch.__version__,) + sys.version_info[:2])
+
+
+def host_fits() -> bool:
+    """Whether the module is there and was built for this torch and this Python."""
+    try:
+        with open(HOST_PATH, "rb") as f:
+            return (host_built_for() + ".").encode() in f.read()
+    except OSError:
+        return False
+
+
 def build_host(force: bool = False, verbose: bool = False) -> str:
     """Compile csrc/host.cpp, the native call path of the Python layer (no device code), against
     torch's headers and libscorch_hip.so.  Returns the module's path."""
-    if not force and not _newer(HOST_PATH, [HOST_SRC] + _headers()):
+    if not force and not _newer(HOST_PATH, [HOST_SRC] + _headers()) and host_fits():
         return HOST_PATH
     import sysconfig
     import torch
@@ -114,18 +130,19 @@ def build_host(force: bool = False, verbose: bool = False) -> str:
         raise RuntimeError("g++ not found: cannot build _host.so")
     base = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = "%s.%d.tmp" % (HOST_PATH, os.getpid())     # (the ranks of a job may find it missing at the same time)
     cmd = [gxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           "-DUSE_ROCM=1", '-DSCORCH_BUILT_FOR="%s."' % host_built_for(), "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
            "-isystem", os.path.join(base, "include"), "-isystem", os.path.join(base, "include", "torch", "csrc", "api", "include"),
            "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"], HOST_SRC,
            "-L", PKG_DIR, "-l:libscorch_hip.so", "-L", os.path.join(base, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
-           "-ltorch_python", "-lamdhip64", "-Wl,-rpath,$ORIGIN", "-o", HOST_PATH + ".tmp"]
+           "-ltorch_python", "-lamdhip64", "-Wl,-rpath,$ORIGIN", "-o", tmp]
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError("g++ failed:\n" + proc.stdout)
-    os.replace(HOST_PATH + ".tmp", HOST_PATH)
+    os.replace(tmp, HOST_PATH)
     return HOST_PATH
 
 

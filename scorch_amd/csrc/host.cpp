@@ -710,7 +710,8 @@ PyMethodDef methods[] = {
     {"remember_attention", host_remember_attention, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Calls of decided products, in native code.", -1, methods};
+// (build.py looks for what the module was built for in its file before it is loaded)
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Calls of decided products, in native code: " SCORCH_BUILT_FOR, -1, methods};
 
 }  // namespace
 

@@ -197,21 +197,44 @@ def lib() -> ctypes.CDLL:
 _host = None
 
 
+class _GeneralWay:
+    """In the place of the native call path where it cannot be loaded: nothing is ever decided, and every
+    call goes the general way, which launches the same kernels (10 us more host time a call)."""
+
+    @staticmethod
+    def spmm(*args):
+        return None
+
+    sddmm = attention = remember = remember_attention = spmm
+
+
+def _load_host():
+    """The module csrc/host.cpp, built (again) if it is missing or was built for another torch or Python."""
+    try:
+        if not _build.host_fits():
+            _build.build_host(force=True)
+        from . import _host as module
+        return module
+    except (ImportError, OSError, RuntimeError) as error:
+        import warnings
+        warnings.warn(f"scorch_amd: the native call path (_host.so) cannot be loaded, calls take the general way: {error}",
+                      RuntimeWarning, stacklevel=3)
+        return None
+
+
 def host():
     """The native call path for products that have been decided (csrc/host.cpp), bound to this package."""
     global _host
     if _host is None:
-        handle = lib()          # (also builds both libraries if they are missing)
+        lib()          # (built first if it is missing: the module is linked against it)
         with _lock:
             if _host is None:
-                if not os.path.exists(_build.HOST_PATH):
-                    _build.build_host()
-                from . import _host as module
-                from . import scorch_ops_hip
-                from .stensor import STensor
-                module.bind(vars(scorch_ops_hip), STensor, scorch_ops_hip._torch_empty, check)
-                _host = module
-        del handle
+                module = _load_host()
+                if module is not None:
+                    from . import scorch_ops_hip
+                    from .stensor import STensor
+                    module.bind(vars(scorch_ops_hip), STensor, scorch_ops_hip._torch_empty, check)
+                _host = module if module is not None else _GeneralWay
     return _host
 
 

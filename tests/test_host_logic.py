@@ -604,3 +604,29 @@ def test_format_arguments_of_every_documented_form_reach_the_dispatch(fmt):
                  lambda: scorch.einsum("ij,jk->ik", A, b, format=fmt)):
         with pytest.raises(RuntimeError, match="HIP devices only"):
             call()
+
+
+def test_the_native_call_path_is_built_for_this_torch_or_done_without(monkeypatch, tmp_path):
+    """A module that was built for another torch or Python is built again before it is loaded; where it can be
+    neither built nor loaded, calls go the general way, with a warning."""
+    from scorch_amd import build, native
+    native.host()
+    assert build.host_fits()
+    other = tmp_path / "_host.so"
+    other.write_bytes(open(build.HOST_PATH, "rb").read().replace(torch.__version__.encode() + b", Python", b"0.0" + b" " * (
+        len(torch.__version__) - 3) + b", Python"))
+    monkeypatch.setattr(build, "HOST_PATH", str(other))
+    assert not build.host_fits()
+    calls = []
+    monkeypatch.setattr(build, "build_host", lambda **kw: calls.append(kw))
+    assert native._load_host() is not None and calls == [{"force": True}]
+
+    def cannot(**kw):
+        raise RuntimeError("g++ not found")
+
+    monkeypatch.setattr(build, "build_host", cannot)
+    monkeypatch.setattr(native, "_host", None)
+    with pytest.warns(RuntimeWarning, match="general way.*g\\+\\+ not found"):
+        host = native.host()
+    assert host.spmm(1, 2, None, 0) is None and host.sddmm(1, 2, 3) is None and host.attention(*range(7)) is None
+    assert host.remember() is None and host.remember_attention() is None
