@@ -30,7 +30,7 @@ namespace {
 
 // ---- names and objects looked up once ---------------------------------------------------------
 PyObject *n_storage, *n_index, *n_value, *n_shape, *n_mode_indices, *n_format, *n_routes, *n_spmm_path, *n_blocked_path,
-    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_ones, *n_dtype, *n_device;
+    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_ones, *n_streams, *n_dtype, *n_device;
 PyObject *g_ops = nullptr;        // scorch_ops_hip's namespace
 PyObject *g_stensor = nullptr;    // the STensor type
 PyObject *g_torch_empty = nullptr;
@@ -96,6 +96,7 @@ enum Kind { kRows = 0, kPlanned = 1, kBlockedSpmm = 2, kSpmv = 3, kSddmmCsr = 4,
 
 // One decided product: everything about the call that does not change from call to call.
 struct Route {
+  hipStream_t stream; // what `q` and `row_ptr` point at may be read by kernels on this one
   int64_t width;      // columns of the dense operand (SDDMM: its depth; SpMV: -1)
   int act;            // 0: none, 1: bias, 2: bias and ReLU
   int kind;
@@ -259,9 +260,9 @@ PyObject *finished(int rc, const at::Tensor &out) {
   return THPVariable_Wrap(out);
 }
 
-Route *find_route(Operand *o, int64_t width, int act) {
+Route *find_route(Operand *o, hipStream_t stream, int64_t width, int act) {
   for (Route &r : *o->routes)
-    if (r.width == width && r.act == act) return &r;
+    if (r.width == width && r.act == act && r.stream == stream) return &r;
   return nullptr;
 }
 
@@ -284,7 +285,7 @@ bool first_sight(PyObject *b, int64_t K, int64_t N) {
 }
 
 // The column-tile copy of a dense operand, if the operand carries a valid one.
-const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N) {
+const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N, hipStream_t stream) {
   PyObject *d = dict_of(b);
   PyObject *c = item(d, n_tiled);
   if (!c || !PyTuple_CheckExact(c) || PyTuple_GET_SIZE(c) != 6) return nullptr;
@@ -298,7 +299,13 @@ const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N) {
       PyLong_AsLong(PyTuple_GET_ITEM(c, 5)) != e)
     return nullptr;
   PyObject *copy = PyTuple_GET_ITEM(c, 4);
-  return THPVariable_Check(copy) ? &THPVariable_Unpack(copy) : nullptr;
+  if (!THPVariable_Check(copy)) return nullptr;
+  PyObject *streams = item(dict_of(copy), n_streams);  // (whose kernels may read it)
+  PyObject *mine = streams ? PyLong_FromUnsignedLongLong(reinterpret_cast<unsigned long long>(stream)) : nullptr;
+  const int among = mine ? PySequence_Contains(streams, mine) : 0;
+  Py_XDECREF(mine);
+  if (among < 0) PyErr_Clear();
+  return among > 0 ? &THPVariable_Unpack(copy) : nullptr;
 }
 
 bool tiles_switched_off() {
@@ -321,7 +328,9 @@ PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
   const bool transposed = !bt.is_contiguous();
   if (!fits(b, o, dims, o->dtype, transposed) || (transposed && o->dtype != at::kFloat)) return none();
   const int64_t N = dims == 2 ? bt.size(1) : -1;
-  Route *r = find_route(o, N, act);
+  if (c10::hip::current_device() != o->device) return none();
+  hipStream_t stream = c10::hip::getCurrentHIPStream(o->device).stream();
+  Route *r = find_route(o, stream, N, act);
   if (!r || r->spmm_path != item(g_ops, n_spmm_path) || r->other_path != item(g_ops, n_blocked_path)) return none();
   const at::Tensor &vt = THPVariable_Unpack(o->value);
   if (vt.scalar_type() != o->dtype || vt.numel() != o->second.numel || !vt.is_contiguous() || vt.get_device() != o->device)
@@ -333,8 +342,6 @@ PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
     if (t.numel() != N) return none();
     bias_ptr = t.const_data_ptr();
   }
-  if (c10::hip::current_device() != o->device) return none();
-  hipStream_t stream = c10::hip::getCurrentHIPStream(o->device).stream();
   void *ws = nullptr, *counters = nullptr;
   size_t ws_bytes = 0, n_counted = 0;
   const at::Tensor *tiles = nullptr;
@@ -342,7 +349,7 @@ PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
   if (r->workspace || r->may_tile) {
     if (capturing(stream)) return none();
     if (r->may_tile && !transposed && !tiles_switched_off()) {
-      tiles = tile_copy(b, o->cols, N);
+      tiles = tile_copy(b, o->cols, N, stream);
       if (!tiles && !first_sight(b, o->cols, N)) return none();  // the general path makes the copy
       if (!r->p[5]) tiles = nullptr;                             // (which is for other products of this operand)
     }
@@ -419,14 +426,14 @@ PyObject *sddmm_body(PyObject *const *args, Py_ssize_t n) {
   const at::Tensor &A = THPVariable_Unpack(args[1]), &B = THPVariable_Unpack(args[2]);
   const int64_t K = A.size(1);
   if (A.size(0) != o->rows || B.size(0) != o->cols || B.size(1) != K) return none();
-  Route *r = find_route(o, K, 3);
+  if (c10::hip::current_device() != o->device) return none();
+  hipStream_t stream = c10::hip::getCurrentHIPStream(o->device).stream();
+  Route *r = find_route(o, stream, K, 3);
   if (!r || r->spmm_path != item(g_ops, n_sddmm_path) || r->other_path != item(g_ops, n_blocked_path)) return none();
   // what is known about the mask's values was found out about these values
   const at::Tensor &vt = THPVariable_Unpack(o->value);
   if (item(dict_of(o->value), n_ones) != r->verdict) return none();  // (mark_volatile() takes it away)
   if (vt.const_data_ptr() != r->value_data || version_of(vt) != r->value_version || vt.numel() != o->second.numel) return none();
-  if (c10::hip::current_device() != o->device) return none();
-  hipStream_t stream = c10::hip::getCurrentHIPStream(o->device).stream();
   if (capturing(stream)) return none();
   at::Tensor out;
   const int64_t M = o->rows, N = o->cols, nnz = o->second.numel;
@@ -495,6 +502,7 @@ PyObject *remember_body(PyObject *args) {
     Py_DECREF(o);  // the storage's now
   }
   Route r = {};
+  r.stream = c10::hip::getCurrentHIPStream(o->device).stream();
   r.width = width, r.act = act, r.kind = kind, r.may_tile = may_tile, r.mask_values = mask_values, r.workspace = ws;
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(ints); ++i) r.p[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(ints, i));
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tensors); ++i) {
@@ -511,11 +519,11 @@ PyObject *remember_body(PyObject *args) {
   auto drop = [](Route &x) {
     for (PyObject *y : {x.keep, x.spmm_path, x.other_path, x.rows, x.verdict}) Py_XDECREF(y);
   };
-  if (Route *old = find_route(o, width, act)) {
+  if (Route *old = find_route(o, r.stream, width, act)) {
     std::swap(*old, r);
     drop(r);
   } else {
-    constexpr size_t kMost = 16;  // widths one operand is multiplied with at a time
+    constexpr size_t kMost = 32;  // widths and streams one operand is multiplied with at a time
     if (o->routes->size() >= kMost) {
       drop(o->routes->front());
       o->routes->erase(o->routes->begin());
@@ -528,6 +536,7 @@ PyObject *remember_body(PyObject *args) {
 // ---- attention over a CSR mask -------------------------------------------------------------------
 enum AttentionKind { kRowsBf16 = 0, kItemsBf16 = 1, kF32 = 2 };
 struct AttentionRoute {
+  hipStream_t stream;  // as in Route
   int64_t H, S, D;
   at::ScalarType dtype;
   int kind;
@@ -590,12 +599,13 @@ PyObject *attention_body(PyObject *const *args, Py_ssize_t n) {
       q.is_neg() || k.is_neg() || v.is_neg() || !q.has_storage() || !k.has_storage() || !v.has_storage())
     return none();
   const int64_t H = q.size(0), S = q.size(1), D = q.size(2);
+  const int device = q.get_device();
+  if (c10::hip::current_device() != device) return none();
+  hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
   AttentionRoute *r = nullptr;
   for (AttentionRoute &x : *t->routes)
-    if (x.H == H && x.S == S && x.D == D && x.dtype == q.scalar_type()) r = &x;
-  const int device = q.get_device();
-  if (!r || (form == 2 && !r->p[7]) || c10::hip::current_device() != device) return none();
-  hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
+    if (x.H == H && x.S == S && x.D == D && x.dtype == q.scalar_type() && x.stream == stream) r = &x;
+  if (!r || (form == 2 && !r->p[7])) return none();
   void *ws = nullptr;
   size_t ws_bytes = 0;
   if (r->workspace && (capturing(stream) || !(ws = workspace(device, stream, r->workspace, &ws_bytes)))) return none();
@@ -658,14 +668,16 @@ PyObject *remember_attention_body(PyObject *args) {
   }
   AttentionRoute r = {};
   r.H = H, r.S = S, r.D = D, r.kind = kind, r.workspace = ws;
-  r.dtype = THPVariable_Unpack(model).scalar_type();
+  const at::Tensor &of = THPVariable_Unpack(model);
+  r.dtype = of.scalar_type();
+  r.stream = of.is_cuda() ? c10::hip::getCurrentHIPStream(of.get_device()).stream() : nullptr;
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(ints); ++i) r.p[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(ints, i));
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tensors); ++i) {
     PyObject *x = PyTuple_GET_ITEM(tensors, i);
     r.q[i] = THPVariable_Check(x) && THPVariable_Unpack(x).numel() ? THPVariable_Unpack(x).const_data_ptr() : nullptr;
   }
   if (PyErr_Occurred()) return nullptr;
-  constexpr size_t kMost = 16;
+  constexpr size_t kMost = 32;
   if (t->routes->size() >= kMost) {
     Py_XDECREF(t->routes->front().keep);
     t->routes->erase(t->routes->begin());
@@ -724,7 +736,7 @@ PyMODINIT_FUNC PyInit__host() {
                {&n_spmm_path, "SPMM_PATH"}, {&n_blocked_path, "BLOCKED_PATH"}, {&n_sddmm_path, "SDDMM_PATH"},
                {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_counters, "_counter_buffers"}, {&n_tiled, "_scorch_tiled"}, {&n_seen, "_scorch_seen"},
                {&n_volatile, "_scorch_volatile"}, {&n_epoch, "_scorch_epoch"}, {&n_attention, "_scorch_attention"},
-               {&n_ones, "_scorch_ones"}, {&n_dtype, "dtype"}, {&n_device, "device"}};
+               {&n_ones, "_scorch_ones"}, {&n_streams, "_scorch_streams"}, {&n_dtype, "dtype"}, {&n_device, "device"}};
   for (const auto &x : names) *x.slot = PyUnicode_InternFromString(x.text);
   OperandType.tp_name = "scorch_amd._host.Operand";
   OperandType.tp_basicsize = sizeof(Operand);

@@ -281,6 +281,28 @@ def is_volatile(t: torch.Tensor) -> bool:
         bool(getattr(getattr(t, "_scorch_origin", None), "_scorch_volatile", False))
 
 
+# What is kept was queued on the stream of the call that made it, and its memory is that stream's to torch's
+# allocator.  A caller who multiplies by one operand on two streams has ordered what it passes in, but
+# cannot know of these: the first call on another stream waits for the device, once.
+def _made_on(stream: int, *tensors: Optional[torch.Tensor]) -> None:
+    for t in tensors:
+        if t is not None:
+            t._scorch_streams = [stream]         # the streams whose kernels may read it
+
+
+def _for_use_on(dev: torch.device, stream: int, first: Optional[torch.Tensor], *made_with_it: Optional[torch.Tensor]) -> None:
+    """Before kernels on `stream`, torch's current one, read kept tensors (a caller's own carry no note and are
+    the caller's to order).  Under a capture nothing can be waited for: what a graph reads is made, and the device
+    waited for, before the capture begins."""
+    if first is None or stream in getattr(first, "_scorch_streams", (stream,)) or torch.cuda.is_current_stream_capturing():
+        return
+    torch.cuda.synchronize(dev)
+    for t in (first,) + made_with_it:
+        if t is not None and stream not in getattr(t, "_scorch_streams", (stream,)):
+            t.record_stream(torch.cuda.current_stream(dev))
+            t._scorch_streams.append(stream)
+
+
 # ---- what is computed once per operand ---------------------------------------------
 def plans_enabled() -> bool:
     """Sparse operands are inspected and planned unless SCORCH_HIP_PLAN=0."""
@@ -403,7 +425,9 @@ def _chunk_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, N: int, el
                              device=pos.device)
         native.check(L.scorch_hip_spmm_csr_bounds(M, nnz, N, elem, pos.data_ptr(), bounds.data_ptr(),
                                                   bounds.numel(), stream))
+        _made_on(stream, bounds)
         plan.bounds[(N, elem)] = bounds
+    _for_use_on(pos.device, stream, bounds)
     return bounds
 
 
@@ -433,7 +457,7 @@ class BlockedCsr:
     the CSR position of the row's first entry in the block, and the two lists of work items."""
     __slots__ = ("n_active", "block_row_ptr", "block_col_idx", "block_words", "block_off", "block_cols", "block_nnz",
                  "sddmm_items", "spmm_items", "n_spmm_items", "spmm_split_rows", "n_spmm_split_rows", "n_spmm_slots",
-                 "n_block_rows", "longest_block_row", "fill")
+                 "n_block_rows", "longest_block_row", "fill", "kept")
 
     def sddmm_items_for(self, heads: int):
         """(work items, their number) of an SDDMM of so many heads: the largest that still give every
@@ -562,6 +586,9 @@ def _blocked_csr(plan: "CsrPlan", pos: torch.Tensor, crd: torch.Tensor, M: int, 
     bl.n_block_rows = nbr
     bl.longest_block_row = longest
     bl.fill = nnz / (n_active * block * block)
+    bl.kept = (bl.block_row_ptr, bl.block_col_idx, bl.block_words, bl.block_off, bl.block_cols, bl.block_nnz, bl.spmm_items,
+               bl.spmm_split_rows, *(items for items, _ in bl.sddmm_items.values()))
+    _made_on(_stream(dev), *bl.kept)
     return bl
 
 
@@ -590,6 +617,7 @@ def _blocked(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, width: int)
 def _blocked_sddmm(L, bl: BlockedCsr, heads: int, M: int, n_cols: int, K: int, nnz: int, mask_vals,
                    a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, rows_ptr, stream: int) -> int:
     """Launch the block SDDMM for `heads` pairs of dense operands over one pattern."""
+    _for_use_on(out.device, stream, *bl.kept)
     items, n_items = bl.sddmm_items_for(heads)
     return L.scorch_hip_sddmm_csr_blocked_f32(
         heads, M, n_cols, K, nnz, bl.n_active, bl.block_col_idx.data_ptr(), bl.block_words.data_ptr(),
@@ -617,6 +645,7 @@ def _listed_mask_values(values: torch.Tensor, lists: torch.Tensor, L, stream):
     key = _stamp(values)
     cached = getattr(values, "_scorch_listed", None)
     if cached is not None and cached[0] == key and cached[1] is lists:
+        _for_use_on(values.device, stream, cached[2])
         return values.data_ptr(), cached[2].data_ptr()
     seen = getattr(values, "_scorch_ones", None)
     if seen is None or seen[0] != key or seen[1] is not False:
@@ -624,6 +653,7 @@ def _listed_mask_values(values: torch.Tensor, lists: torch.Tensor, L, stream):
     listed = _empty_like(values)
     native.check(L.scorch_hip_sddmm_csr_list_values_f32(values.numel(), lists.data_ptr(), lists.numel(),
                                                         values.data_ptr(), listed.data_ptr(), stream))
+    _made_on(stream, listed)
     try:
         values._scorch_listed = (key, lists, listed)
     except (AttributeError, RuntimeError):
@@ -659,6 +689,7 @@ def _known_all_ones(values: torch.Tensor) -> bool:
 def _blocked_spmm(L, bl: BlockedCsr, heads: int, M: int, K: int, N: int, nnz: int, vals: torch.Tensor,
                   b: torch.Tensor, out: torch.Tensor, stream: int) -> int:
     """Launch the block SpMM for `heads` value arrays over one pattern."""
+    _for_use_on(out.device, stream, *bl.kept)
     ws = None
     if bl.n_spmm_slots:
         ws = _workspace(out.device, stream, L.scorch_hip_spmm_csr_blocked_workspace_bytes(heads, bl.n_spmm_slots, N))
@@ -701,6 +732,7 @@ def prepare_dense_operand(values: torch.Tensor, K: int, N: int) -> Optional[torc
     with _on_device(dev):
         native.check(L.scorch_hip_dense_to_tiled_f32(K, N, flat.data_ptr(), bt.data_ptr(), bt.numel() * 4,
                                                      _stream(dev)))
+        _made_on(_stream(dev), bt)
     owner._scorch_tiled = (owner._version, values.data_ptr(), K, N, bt, _epoch(owner))
     return bt
 
@@ -723,6 +755,7 @@ def _tiled_operand(values: torch.Tensor, K: int, N: int, nnz: int, L) -> Optiona
     stamp = (owner._version, values.data_ptr(), K, N)
     cached = getattr(owner, "_scorch_tiled", None)
     if cached is not None and cached[:4] == stamp and cached[5] == _epoch(owner):
+        _for_use_on(values.device, _stream(values.device), cached[4])
         return cached[4]
     stamp = stamp + (_epoch(owner),)
     if getattr(owner, "_scorch_seen", None) == stamp:
@@ -881,6 +914,8 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
     def remember(kind, ints=(), tensors=(), workspace=0, may_tile=False):
         if pos_of_coo:
             tensors = tuple(tensors) + pos_of_coo[len(tensors):]
+        for t in tensors:
+            _for_use_on(dev, _stream(dev), t)
         host.remember(a, kind, width, act, tuple(ints), tuple(tensors), workspace, may_tile, 0, None, SPMM_PATH, BLOCKED_PATH)
 
     if width < 0:
@@ -1119,7 +1154,9 @@ def _spmv_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, L, stream) 
     if bounds is None and M > 0:
         bounds = _empty(L.scorch_hip_spmv_csr_bounds_bytes(M, nnz), dtype=torch.uint8, device=pos.device)
         native.check(L.scorch_hip_spmv_csr_bounds(M, nnz, pos.data_ptr(), bounds.data_ptr(), bounds.numel(), stream))
+        _made_on(stream, bounds)
         plan.bounds["spmv"] = bounds
+    _for_use_on(pos.device, stream, bounds)
     return bounds
 
 
@@ -1186,7 +1223,9 @@ def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int,
         lists = _empty(L.scorch_hip_sddmm_csr_lists_bytes(crd.numel()), dtype=torch.uint8, device=pos.device)
         native.check(L.scorch_hip_sddmm_csr_lists(M, n_cols, crd.numel(), pos.data_ptr(), crd.data_ptr(),
                                                   lists.data_ptr(), lists.numel(), stream))
+        _made_on(stream, lists)
         plan.sddmm_lists = lists
+    _for_use_on(pos.device, stream, plan.sddmm_lists)
     return plan.sddmm_lists
 
 
@@ -1221,13 +1260,17 @@ def _coo_mask_row_ptr(row: torch.Tensor, col: torch.Tensor, M: int, n_cols: int,
     if seen is not None and seen[0] == key and _same(seen[2], col):
         if seen[1] is None and not torch.cuda.is_current_stream_capturing():
             pos = coo_row_ptr(row, M)
+            _made_on(_stream(row.device), pos)
             seen = (key, pos if pos is not None else False, seen[2])
             row._scorch_coo_pos = seen
             if pos is not None:
                 plan = csr_plan(pos, col, M, n_cols, "S")
                 if plan is not None:
                     plan.blocked_uses = 1           # this is the mask's second product already
-        return seen[1] if isinstance(seen[1], torch.Tensor) else None
+        if not isinstance(seen[1], torch.Tensor):
+            return None
+        _for_use_on(row.device, _stream(row.device), seen[1])
+        return seen[1]
     try:
         row._scorch_coo_pos = (key, None, weakref.ref(col))
     except (AttributeError, RuntimeError):
@@ -1273,9 +1316,11 @@ def _result_rows(plan: Optional[CsrPlan], crd: torch.Tensor):
     the same tensor -- as the reference hands out a coordinate mask's own index tensors
     (src/scorch/ops.py:416-423) -- so a result's index tensors are not for writing to."""
     if plan is not None and plan.rows is not None:
+        _for_use_on(crd.device, _stream(crd.device), plan.rows)
         return plan.rows, None
     rows = _empty_like(crd)
     if plan is not None and not torch.cuda.is_current_stream_capturing():
+        _made_on(_stream(crd.device), rows)
         plan.rows = rows
     return rows, rows.data_ptr()
 
@@ -1329,6 +1374,8 @@ def remember_sddmm(mask, K: int) -> None:
     host = native.host()
 
     def remember(kind, ints=(), tensors=(), rows=None):
+        for t in tensors:
+            _for_use_on(vals.device, _stream(vals.device), t)
         host.remember(mask, kind, K, 3, tuple(ints), tuple(tensors), 0, False, read_values, rows, SDDMM_PATH, BLOCKED_PATH)
 
     def remember_blocked(bl, rows):
@@ -1453,6 +1500,7 @@ def _coo_as_csr(mode_indices, values, n_rows: int, what: str):
     rows, cols = _index(mode_indices[0][0], what + " rows"), _index(mode_indices[1][0], what + " columns")
     if rows.numel() != cols.numel() or rows.numel() != values.numel():
         raise ValueError(f"scorch_ops_hip: {what}: coordinate and value arrays differ in length")
+    stream = _stream(_device_of(rows))
     known = _known_row_order(rows, n_rows)
     if known is None:
         pos, order = coo_row_ptr(rows, n_rows), None
@@ -1461,6 +1509,7 @@ def _coo_as_csr(mode_indices, values, n_rows: int, what: str):
                 raise ValueError(f"scorch_ops_hip: {what} has a row coordinate outside [0, {n_rows})")
             in_order, order = torch.sort(rows, stable=True)
             pos = coo_row_ptr(in_order, n_rows)
+        _made_on(stream, pos, order)
         known = (pos, order, {})
         if plans_enabled():
             try:
@@ -1468,11 +1517,14 @@ def _coo_as_csr(mode_indices, values, n_rows: int, what: str):
             except (AttributeError, RuntimeError):
                 pass
     pos, order, sorted_cols = known
+    _for_use_on(rows.device, stream, pos, order)
     if order is not None:
         key = _stamp(cols)
         kept = sorted_cols.get("cols")
         if kept is None or kept[0] != key or not _same(kept[1], cols):
             kept = sorted_cols["cols"] = (key, weakref.ref(cols), cols[order])
+            _made_on(stream, kept[2])
+        _for_use_on(rows.device, stream, kept[2])
         cols, values = kept[2], values[order]
     return pos, cols, values
 
@@ -1691,6 +1743,9 @@ class BlockMask:
         self.block_cols = None      # int64 per active block: the columns some row of it refers to (None: all)
         self.pairing = {}           # (item list, heads, head dimension) -> (workgroups take two items?, priority step)
 
+    def kept(self):
+        return self.block_col_idx, self.block_row_ptr, self.block_mask_index, self.block_masks, self.block_cols
+
     def row_lens(self):
         """Active blocks per block row as a numpy array on the host (read from the device once)."""
         if self.block_row_lens is None:
@@ -1758,6 +1813,7 @@ def _block_mask(pos: torch.Tensor, crd: torch.Tensor, S: int) -> BlockMask:
     bm.block_row_lens = brp[1:] - brp[:-1]
     if partial.numel():
         bm.block_cols = arrays["block_cols"]
+    _made_on(_stream(dev), *bm.kept())
     return bm
 
 
@@ -1853,6 +1909,8 @@ def split_long_block_rows(bm: BlockMask, longest: Optional[int] = None, list_une
     dev = bm.block_row_ptr.device
     bm.items = torch.from_numpy(items).to(dev).reshape(-1)
     bm.split_rows = torch.from_numpy(split_rows).to(dev).reshape(-1)
+    if dev.type == "cuda":
+        _made_on(_stream(dev), bm.items, bm.split_rows)
     bm.n_slots = n_slots
     return bm
 
@@ -2037,6 +2095,8 @@ def attn_blocksparse_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bm: 
     L = native.lib()
     with _on_device(dev):
         stream = _stream(dev)
+        _for_use_on(dev, stream, *bm.kept())
+        _for_use_on(dev, stream, items, split_rows)
         need = L.scorch_hip_attn_blocksparse_f32_workspace_bytes(H, n_slots, D) if n_items else 0
         ws = _workspace(dev, stream, need) if need else None
         n_masks = bm.n_masks if bm.block_masks is not None else 0
@@ -2073,6 +2133,8 @@ def _attn_bf16_items(q, k, v, bm: BlockMask, items: torch.Tensor, split_rows: Op
     L = native.lib()
     with _on_device(dev):
         stream = _stream(dev)
+        _for_use_on(dev, stream, *bm.kept())
+        _for_use_on(dev, stream, items, split_rows)
         need = L.scorch_hip_attn_blocksparse_split_workspace_bytes(H, n_slots, D)
         ws = _workspace(dev, stream, need) if need else None
         rc = L.scorch_hip_attn_blocksparse_split_bf16(
@@ -2185,6 +2247,8 @@ def _block_row_schedule(brp: torch.Tensor):
     lens = ptrs[1:] - ptrs[:-1]
     items, _, _ = _stretches(lens, max(int(lens.max()), 1) if lens.size else 1, True)
     entry = (_stamp(brp), lens, torch.from_numpy(items).to(brp.device).reshape(-1), {})
+    if brp.is_cuda:
+        _made_on(_stream(brp.device), entry[2])
     try:
         brp._scorch_rows = entry
     except (AttributeError, RuntimeError):
@@ -2241,6 +2305,7 @@ def attn_blocksparse_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
             return _attn_bf16_items(q, k, v, rows, items, None, 0, scale, pair, priority_step)
     out = _empty_like(q)
     with _on_device(dev):
+        _for_use_on(dev, _stream(dev), bci, brp, bmi, block_masks)
         if bmi is None:
             rc = native.lib().scorch_hip_attn_blocksparse_bf16(H, S, D, block, bci.numel(), brp.data_ptr(),
                                                                bci.data_ptr(), q.data_ptr(), k.data_ptr(),
