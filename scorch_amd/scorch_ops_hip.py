@@ -417,9 +417,13 @@ def _malformed(what: str, problems) -> ValueError:
     return ValueError(f"scorch_ops_hip: {what}: malformed CSR index: " + "; ".join(problems))
 
 
-def _chunk_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, N: int, elem: int, L, stream) -> torch.Tensor:
-    """Chunk boundaries of the merge-path split for dense width N, computed once."""
+def _chunk_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, N: int, elem: int, L, stream) -> Optional[torch.Tensor]:
+    """Chunk boundaries of the merge-path split for dense width N, computed once.  None while the
+    stream is being captured and there are none: made there they would be the graph's memory, and hold
+    nothing until it is replayed (the kernels then search row_ptr)."""
     bounds = plan.bounds.get((N, elem))
+    if bounds is None and torch.cuda.is_current_stream_capturing():
+        return None
     if bounds is None:
         bounds = _empty(L.scorch_hip_spmm_csr_bounds_bytes(M, nnz, N, elem), dtype=torch.uint8,
                              device=pos.device)
@@ -733,7 +737,8 @@ def prepare_dense_operand(values: torch.Tensor, K: int, N: int) -> Optional[torc
         native.check(L.scorch_hip_dense_to_tiled_f32(K, N, flat.data_ptr(), bt.data_ptr(), bt.numel() * 4,
                                                      _stream(dev)))
         _made_on(_stream(dev), bt)
-    owner._scorch_tiled = (owner._version, values.data_ptr(), K, N, bt, _epoch(owner))
+    if not torch.cuda.is_current_stream_capturing():
+        owner._scorch_tiled = (owner._version, values.data_ptr(), K, N, bt, _epoch(owner))
     return bt
 
 
@@ -1149,9 +1154,9 @@ prebuilt_spmspm_csr_i64 = _make_spgemm(torch.int64)
 
 
 def _spmv_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, L, stream) -> Optional[torch.Tensor]:
-    """Chunk boundaries of the matrix-vector product, computed once."""
+    """Chunk boundaries of the matrix-vector product, computed once (not under a capture, as above)."""
     bounds = plan.bounds.get("spmv")
-    if bounds is None and M > 0:
+    if bounds is None and M > 0 and not torch.cuda.is_current_stream_capturing():
         bounds = _empty(L.scorch_hip_spmv_csr_bounds_bytes(M, nnz), dtype=torch.uint8, device=pos.device)
         native.check(L.scorch_hip_spmv_csr_bounds(M, nnz, pos.data_ptr(), bounds.data_ptr(), bounds.numel(), stream))
         _made_on(stream, bounds)
@@ -1217,8 +1222,10 @@ def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int,
         if not _lists_apply(crd.numel(), n_cols, K):
             return None
         plan.sddmm_uses += 1
-        if plan.sddmm_lists is None and (plan.sddmm_uses < 2 or torch.cuda.is_current_stream_capturing()):
+        if plan.sddmm_lists is None and plan.sddmm_uses < 2:
             return None
+    if plan.sddmm_lists is None and torch.cuda.is_current_stream_capturing():
+        return None
     if plan.sddmm_lists is None:
         lists = _empty(L.scorch_hip_sddmm_csr_lists_bytes(crd.numel()), dtype=torch.uint8, device=pos.device)
         native.check(L.scorch_hip_sddmm_csr_lists(M, n_cols, crd.numel(), pos.data_ptr(), crd.data_ptr(),
@@ -1522,8 +1529,10 @@ def _coo_as_csr(mode_indices, values, n_rows: int, what: str):
         key = _stamp(cols)
         kept = sorted_cols.get("cols")
         if kept is None or kept[0] != key or not _same(kept[1], cols):
-            kept = sorted_cols["cols"] = (key, weakref.ref(cols), cols[order])
-            _made_on(stream, kept[2])
+            kept = (key, weakref.ref(cols), cols[order])
+            if not torch.cuda.is_current_stream_capturing():      # (a recorded gather is the graph's alone)
+                sorted_cols["cols"] = kept
+                _made_on(stream, kept[2])
         _for_use_on(rows.device, stream, kept[2])
         cols, values = kept[2], values[order]
     return pos, cols, values

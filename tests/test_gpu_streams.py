@@ -154,3 +154,34 @@ def test_kept_memory_is_not_handed_out_while_another_stream_reads_it():
     assert all(t.data_ptr() != where for t in fresh)
     torch.cuda.synchronize()
     assert torch.equal(late, want)
+
+
+@pytest.mark.parametrize("N", [None, 24, 200])
+@pytest.mark.parametrize("pin", ["auto", "merge"])
+def test_what_a_capture_would_make_is_not_kept(N, pin, monkeypatch):
+    """A product of a planned operand at a width that is new, recorded first and replayed never: the eager product
+    after it does not read what the recording alone would have filled.  Then the replays."""
+    monkeypatch.setattr(H, "SPMM_PATH", pin)
+    rng = np.random.default_rng(8)
+    n = 900
+    rp, ci, v = _graph(rng, n, 4000)
+    A = STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (n, n))
+    b = torch.randn(n, N, device="cuda") if N else torch.randn(n, device="cuda")
+    dense = torch.zeros(n, n, dtype=torch.float64)
+    dense.index_put_((torch.from_numpy(np.repeat(np.arange(n), np.diff(rp))), torch.from_numpy(ci).long()),
+                     torch.from_numpy(v).double(), accumulate=True)
+    want = dense @ b.double().cpu()
+    scorch.matmul(A, torch.randn(n, 5, device="cuda"))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = scorch.matmul(A, b)
+    assert ((N, 4) if N else "spmv") not in A.index.mode_indices[1][0]._scorch_plan.bounds
+    eager = scorch.matmul(A, b)
+    for _ in range(3):
+        assert float((eager.double().cpu() - want).norm()) <= 1e-5 * float(want.norm())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((recorded.double().cpu() - want).norm()) <= 1e-5 * float(want.norm())
+        recorded.zero_()
+        eager = scorch.matmul(A, b)
