@@ -9,7 +9,7 @@
 // still the same unwritten tensors (identity, address, version counter, and the epoch that
 // forget() advances), that the dense operand fits, allocates the result, and
 // calls the library.  Anything else -- another dtype, a view, a graph being captured that would
-// need scratch memory, a pinned kernel path -- is answered with None, and the caller takes the
+// need scratch memory or reads kept data, a pinned kernel path -- is answered with None, and the caller takes the
 // general way, which also words every error.
 #include <Python.h>
 
@@ -346,8 +346,8 @@ PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
   size_t ws_bytes = 0, n_counted = 0;
   const at::Tensor *tiles = nullptr;
   const bool panels = (r->kind == kRows || r->kind == kPlanned) && (r->p[4] & (transposed ? 2 : 1));
-  if (r->workspace || r->may_tile) {
-    if (capturing(stream)) return none();
+  if (r->workspace || r->may_tile || r->row_ptr) {
+    if (capturing(stream)) return none();  // (the general path, which tells the recording what it reads)
     if (r->may_tile && !transposed && !tiles_switched_off()) {
       tiles = tile_copy(b, o->cols, N, stream);
       if (!tiles && !first_sight(b, o->cols, N)) return none();  // the general path makes the copy
@@ -608,7 +608,7 @@ PyObject *attention_body(PyObject *const *args, Py_ssize_t n) {
   if (!r || (form == 2 && !r->p[7])) return none();
   void *ws = nullptr;
   size_t ws_bytes = 0;
-  if (r->workspace && (capturing(stream) || !(ws = workspace(device, stream, r->workspace, &ws_bytes)))) return none();
+  if (capturing(stream) || (r->workspace && !(ws = workspace(device, stream, r->workspace, &ws_bytes)))) return none();
   at::Tensor out;
   if (!allocate(out, q.sizes(), q.scalar_type(), device, q)) return nullptr;
   const void *Q = q.const_data_ptr(), *K = k.const_data_ptr(), *V = v.const_data_ptr();

@@ -13,7 +13,7 @@ masks) are built on an operand's first or second use and need a
 synchronisation, which a capturing stream does not allow; the step is run
 eagerly on a side stream first, ``warmup`` times, so that they exist.  The plans
 of a sparse operand's index arrays (and of an attention mask) become part of the
-recording: values may be rewritten in place between replays, index arrays may
+recording, which keeps them alive: values may be rewritten in place between replays, index arrays may
 not.  Nothing derived from an operand's *values* is recorded (the column-tile
 copy of a wide dense operand, the verdict that a mask's values are all 1): a
 recorded product runs from the operand itself and reads every value array it
@@ -47,7 +47,7 @@ class CapturedStep:
             raise RuntimeError("scorch_amd.graphs: no GPU")
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("scorch_amd.graphs: capture() called while the stream is already capturing")
-        self.args = args
+        self.fn, self.args = fn, args       # (fn: the operands it closes over are read by every replay)
         scorch_ops_hip.mark_volatile(args)
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -57,8 +57,13 @@ class CapturedStep:
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            self.result = fn(*args)
+        self._kept: list = []
+        scorch_ops_hip._recordings.append(self._kept)
+        try:
+            with torch.cuda.graph(self.graph):
+                self.result = fn(*args)
+        finally:
+            scorch_ops_hip._recordings[:] = [r for r in scorch_ops_hip._recordings if r is not self._kept]
         self._result_tensors = list(scorch_ops_hip._tensors_of(self.result))
         scorch_ops_hip.mark_volatile(self._result_tensors)
 

@@ -284,6 +284,11 @@ def is_volatile(t: torch.Tensor) -> bool:
 # What is kept was queued on the stream of the call that made it, and its memory is that stream's to torch's
 # allocator.  A caller who multiplies by one operand on two streams has ordered what it passes in, but
 # cannot know of these: the first call on another stream waits for the device, once.
+# graphs.CapturedStep puts a list here while it records: a recording holds the addresses of the kept tensors
+# that it reads, and has to hold the tensors as well -- forget() drops them, and so does a rewritten index.
+_recordings: list = []
+
+
 def _made_on(stream: int, *tensors: Optional[torch.Tensor]) -> None:
     for t in tensors:
         if t is not None:
@@ -294,7 +299,12 @@ def _for_use_on(dev: torch.device, stream: int, first: Optional[torch.Tensor], *
     """Before kernels on `stream`, torch's current one, read kept tensors (a caller's own carry no note and are
     the caller's to order).  Under a capture nothing can be waited for: what a graph reads is made, and the device
     waited for, before the capture begins."""
-    if first is None or stream in getattr(first, "_scorch_streams", (stream,)) or torch.cuda.is_current_stream_capturing():
+    if first is None:
+        return
+    if _recordings and torch.cuda.is_current_stream_capturing():
+        _recordings[-1].extend(t for t in (first,) + made_with_it if t is not None)
+        return
+    if stream in getattr(first, "_scorch_streams", (stream,)) or torch.cuda.is_current_stream_capturing():
         return
     torch.cuda.synchronize(dev)
     for t in (first,) + made_with_it:

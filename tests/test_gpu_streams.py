@@ -185,3 +185,38 @@ def test_what_a_capture_would_make_is_not_kept(N, pin, monkeypatch):
         assert float((recorded.double().cpu() - want).norm()) <= 1e-5 * float(want.norm())
         recorded.zero_()
         eager = scorch.matmul(A, b)
+
+
+@pytest.mark.parametrize("kind", ["csr", "coo", "vector", "sddmm", "attention"])
+def test_a_recording_holds_what_it_reads(kind):
+    """forget() drops what is kept with an operand; a recorded step goes on reading it."""
+    from scorch_amd import graphs
+    rng = np.random.default_rng(9)
+    n, N = 640, 48
+    rp, ci, v = _graph(rng, n, 5000)
+    rows = np.repeat(np.arange(n), np.diff(rp)).astype(np.int32)
+    A = STensor._coo((n, n), [dev(rows), dev(ci)], dev(v), "A") if kind == "coo" else \
+        STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (n, n))
+    X = torch.randn(n, device="cuda") if kind == "vector" else torch.randn(n, N, device="cuda")
+    forgotten, X2 = A, torch.randn_like(X)
+    if kind == "sddmm":
+        step = lambda x: scorch.einsum("ij,ik,jk->ij", A, x, X2).values
+    elif kind == "attention":
+        X, X2 = torch.randn(2, n, 64, device="cuda"), torch.randn(2, n, 64, device="cuda")
+        mask = forgotten = tuple(dev(x) for x in workloads.longformer_mask(n))
+        step = lambda x: H.sparse_attention_f32(x, X2, X2, *mask, 0.125)
+    else:
+        step = lambda x: scorch.matmul(A, x)
+    recorded = graphs.capture(step, X, warmup=4)
+    want = step(X)
+    # (fp32 sums by another kernel, or in another order)
+    close = lambda got: float((got - want).norm()) <= 2e-5 * float(want.norm())
+    assert close(recorded())
+    H.forget(forgotten)
+    junk = [torch.full((size,), 0x7F, dtype=torch.uint8, device="cuda") for size in (512, 2048, 8192, 65_536, 1 << 20)
+            for _ in range(40)]
+    for _ in range(3):
+        recorded.result.zero_()
+        assert close(recorded())
+        torch.cuda.synchronize()
+    del junk
