@@ -288,7 +288,7 @@ bool first_sight(PyObject *b, int64_t K, int64_t N) {
 const at::Tensor *tile_copy(PyObject *b, int64_t K, int64_t N, hipStream_t stream) {
   PyObject *d = dict_of(b);
   PyObject *c = item(d, n_tiled);
-  if (!c || !PyTuple_CheckExact(c) || PyTuple_GET_SIZE(c) != 6) return nullptr;
+  if (!c || !PyTuple_Check(c) || PyTuple_GET_SIZE(c) != 6) return nullptr;
   const at::Tensor &t = THPVariable_Unpack(b);
   if (t.is_inference() || is_volatile(b)) return nullptr;
   PyObject *epoch = epoch_of(b);
@@ -688,12 +688,15 @@ PyObject *remember_attention_body(PyObject *args) {
   return none();
 }
 
-// What copy and pickle make of these objects: nothing (a copied operand decides anew).
-PyObject *reduce_to_none(PyObject *, PyObject *) {
-  PyObject *type = reinterpret_cast<PyObject *>(Py_TYPE(Py_None));
-  return Py_BuildValue("O()", type);
+// What copy and pickle make of these objects: an empty container, which is no decision (a copied operand
+// decides anew) and which torch.load takes with weights_only.
+PyObject *reduce_to_nothing(PyObject *, PyObject *) {
+  PyObject *collections = PyImport_ImportModule("collections");
+  PyObject *type = collections ? PyObject_GetAttrString(collections, "OrderedDict") : nullptr;
+  Py_XDECREF(collections);
+  return type ? Py_BuildValue("N()", type) : nullptr;
 }
-PyMethodDef kept_methods[] = {{"__reduce__", reduce_to_none, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef kept_methods[] = {{"__reduce__", reduce_to_nothing, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 
 // ---- module ----------------------------------------------------------------------------------------
 // bind(namespace of scorch_ops_hip, STensor type, torch.empty, native.check)

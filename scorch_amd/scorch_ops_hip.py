@@ -21,6 +21,7 @@ is re-stored once by column tiles (see CsrPlan and _tiled_operand below).
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 import math
 import os
@@ -194,6 +195,21 @@ _CACHE_ATTRIBUTES = ("_scorch_plan", "_scorch_tiled", "_scorch_seen", "_scorch_o
                      "_scorch_block_mask", "_scorch_mask_checked", "_scorch_rows", "_scorch_row_order", "_scorch_attention")
 
 
+class _Kept(tuple):
+    """What an attribute of a tensor holds.  It belongs to that one tensor object: a copy made by
+    copy.deepcopy, pickle or torch.save gets an empty dictionary in its place (a plain container, so
+    that torch.load still reads the file with weights_only)."""
+    __slots__ = ()
+
+    def __reduce_ex__(self, protocol):
+        return collections.OrderedDict, ()
+
+
+def _kept(t: torch.Tensor, name: str) -> Optional[_Kept]:
+    found = getattr(t, name, None)
+    return found if type(found) is _Kept else None
+
+
 def _tensors_of(obj, seen=None):
     """The torch tensors reachable from `obj`: a tensor, an STensor (values and index arrays), a result
     carrier of this module, or lists / tuples / dicts of those."""
@@ -359,10 +375,17 @@ class CsrPlan:
         self.attention_uses = 0                            # sparse_attention_csr calls
         self.other_columns = None                          # (weak reference, stamp): column indices last multiplied over these rows
 
+    __reduce_ex__ = _Kept.__reduce_ex__
+
+
+def _plan_kept(pos: torch.Tensor) -> Optional[CsrPlan]:
+    plan = getattr(pos, "_scorch_plan", None)
+    return plan if type(plan) is CsrPlan else None          # (a copy of the tensor has none: see _Kept)
+
 
 def _plan_at_hand(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int) -> Optional[CsrPlan]:
     """The plan of (pos, crd) if it has been made and both tensors are what they were."""
-    plan = getattr(pos, "_scorch_plan", None)
+    plan = _plan_kept(pos)
     if plan is not None and plan.key == (_stamp(pos), _stamp(crd), n_rows, n_cols) and _same(plan.partner, crd):
         return plan
     return None
@@ -372,7 +395,7 @@ def _plan_of_rows(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int
     """The plan of these unchanged row pointers with other column indices, for column indices that
     come along for the first time: what it knows about rows holds for them too, and only their
     range is open.  From their second product on they get a plan of their own."""
-    plan = getattr(pos, "_scorch_plan", None)
+    plan = _plan_kept(pos)
     if plan is None or n_cols == 0 or crd.numel() == 0 or not plans_enabled() or torch.cuda.is_current_stream_capturing():
         return None
     (of_pos, of_crd, *sizes), stamp = plan.key, _stamp(crd)
@@ -657,11 +680,11 @@ def _listed_mask_values(values: torch.Tensor, lists: torch.Tensor, L, stream):
     if torch.cuda.is_current_stream_capturing() or is_volatile(values):
         return values.data_ptr(), None
     key = _stamp(values)
-    cached = getattr(values, "_scorch_listed", None)
+    cached = _kept(values, "_scorch_listed")
     if cached is not None and cached[0] == key and cached[1] is lists:
         _for_use_on(values.device, stream, cached[2])
         return values.data_ptr(), cached[2].data_ptr()
-    seen = getattr(values, "_scorch_ones", None)
+    seen = _kept(values, "_scorch_ones")
     if seen is None or seen[0] != key or seen[1] is not False:
         return values.data_ptr(), None          # not yet seen twice unchanged
     listed = _empty_like(values)
@@ -669,7 +692,7 @@ def _listed_mask_values(values: torch.Tensor, lists: torch.Tensor, L, stream):
                                                         values.data_ptr(), listed.data_ptr(), stream))
     _made_on(stream, listed)
     try:
-        values._scorch_listed = (key, lists, listed)
+        values._scorch_listed = _Kept((key, lists, listed))
     except (AttributeError, RuntimeError):
         return values.data_ptr(), None
     return values.data_ptr(), listed.data_ptr()
@@ -683,18 +706,18 @@ def _known_all_ones(values: torch.Tensor) -> bool:
         # a recording holds pointers, not verdicts: the values may be rewritten before a replay
         return False
     key = _stamp(values)
-    seen = getattr(values, "_scorch_ones", None)
+    seen = _kept(values, "_scorch_ones")
     if seen is not None and seen[0] == key:
         if seen[1] is None:
             differ = _empty(1, dtype=torch.int32, device=values.device)
             with _on_device(values.device):
                 native.check(native.lib().scorch_hip_values_differ_f32(values.numel(), values.data_ptr(), 1.0,
                                                                        differ.data_ptr(), _stream(values.device)))
-            seen = (key, values.dtype == torch.float32 and not differ.item())
+            seen = _Kept((key, values.dtype == torch.float32 and not differ.item()))
             values._scorch_ones = seen
         return bool(seen[1])
     try:
-        values._scorch_ones = (key, None)
+        values._scorch_ones = _Kept((key, None))
     except (AttributeError, RuntimeError):
         pass
     return False
@@ -748,7 +771,7 @@ def prepare_dense_operand(values: torch.Tensor, K: int, N: int) -> Optional[torc
                                                      _stream(dev)))
         _made_on(_stream(dev), bt)
     if not torch.cuda.is_current_stream_capturing():
-        owner._scorch_tiled = (owner._version, values.data_ptr(), K, N, bt, _epoch(owner))
+        owner._scorch_tiled = _Kept((owner._version, values.data_ptr(), K, N, bt, _epoch(owner)))
     return bt
 
 
@@ -768,7 +791,7 @@ def _tiled_operand(values: torch.Tensor, K: int, N: int, nnz: int, L) -> Optiona
     if is_volatile(owner) or is_volatile(values):
         return None
     stamp = (owner._version, values.data_ptr(), K, N)
-    cached = getattr(owner, "_scorch_tiled", None)
+    cached = _kept(owner, "_scorch_tiled")
     if cached is not None and cached[:4] == stamp and cached[5] == _epoch(owner):
         _for_use_on(values.device, _stream(values.device), cached[4])
         return cached[4]
@@ -1273,12 +1296,12 @@ def _coo_mask_row_ptr(row: torch.Tensor, col: torch.Tensor, M: int, n_cols: int,
     if not _coo_mask_may_be_blocked(row, M, n_cols, K):
         return None
     key = (_stamp(row), _stamp(col), M)
-    seen = getattr(row, "_scorch_coo_pos", None)
+    seen = _kept(row, "_scorch_coo_pos")
     if seen is not None and seen[0] == key and _same(seen[2], col):
         if seen[1] is None and not torch.cuda.is_current_stream_capturing():
             pos = coo_row_ptr(row, M)
             _made_on(_stream(row.device), pos)
-            seen = (key, pos if pos is not None else False, seen[2])
+            seen = _Kept((key, pos if pos is not None else False, seen[2]))
             row._scorch_coo_pos = seen
             if pos is not None:
                 plan = csr_plan(pos, col, M, n_cols, "S")
@@ -1289,7 +1312,7 @@ def _coo_mask_row_ptr(row: torch.Tensor, col: torch.Tensor, M: int, n_cols: int,
         _for_use_on(row.device, _stream(row.device), seen[1])
         return seen[1]
     try:
-        row._scorch_coo_pos = (key, None, weakref.ref(col))
+        row._scorch_coo_pos = _Kept((key, None, weakref.ref(col)))
     except (AttributeError, RuntimeError):
         pass
     return None
@@ -1383,7 +1406,7 @@ def remember_sddmm(mask, K: int) -> None:
     if SDDMM_PATH != "auto" or BLOCKED_PATH not in BLOCKED_PATHS or vals.dtype != torch.float32 or K == 0 \
             or torch.cuda.is_current_stream_capturing() or is_volatile(vals) or vals.numel() == 0:
         return
-    seen = getattr(vals, "_scorch_ones", None)
+    seen = _kept(vals, "_scorch_ones")
     if seen is None or seen[0] != _stamp(vals) or seen[1] is None:
         return
     M, n_cols, nnz = int(mask.shape[0]), int(mask.shape[1]), vals.numel()
@@ -1412,7 +1435,7 @@ def remember_sddmm(mask, K: int) -> None:
                 remember_blocked(bl, plan.rows)
                 return
         if _lists_apply(crd.numel(), n_cols, K):
-            listed = getattr(vals, "_scorch_listed", None)
+            listed = _kept(vals, "_scorch_listed")
             if plan.sddmm_lists is None or (read_values and (listed is None or listed[0] != _stamp(vals)
                                                              or listed[1] is not plan.sddmm_lists)):
                 return
@@ -1423,7 +1446,7 @@ def remember_sddmm(mask, K: int) -> None:
     elif len(modes) == 2 and len(modes[0]) == 1 and len(modes[1]) == 1:
         row, col = modes[0][0], modes[1][0]
         if _coo_mask_may_be_blocked(row, M, n_cols, K):
-            seen = getattr(row, "_scorch_coo_pos", None)
+            seen = _kept(row, "_scorch_coo_pos")
             if seen is None or seen[0] != (_stamp(row), _stamp(col), M) or not _same(seen[2], col) or seen[1] is None:
                 return
             if seen[1] is not False:
@@ -1444,7 +1467,7 @@ SOFTMAX_SHORT_ROW = 4096     # rows up to this length never reach the row softma
 def _known_longest_row(pos: torch.Tensor, n_rows: int, nnz: int) -> Optional[int]:
     """The longest row of the pattern if a plan made for this row pointer says so (a product with
     the same pattern has inspected it), else None."""
-    plan = getattr(pos, "_scorch_plan", None)
+    plan = _plan_kept(pos)
     if plan is not None and plan.key[0] == _stamp(pos) and plan.key[1][3] == nnz and plan.key[2] == n_rows:
         return plan.max_row
     return None
@@ -1530,7 +1553,7 @@ def _coo_as_csr(mode_indices, values, n_rows: int, what: str):
         known = (pos, order, {})
         if plans_enabled():
             try:
-                rows._scorch_row_order = (_stamp(rows), n_rows, known)
+                rows._scorch_row_order = _Kept((_stamp(rows), n_rows, known))
             except (AttributeError, RuntimeError):
                 pass
     pos, order, sorted_cols = known
@@ -1552,7 +1575,7 @@ def _known_row_order(rows: torch.Tensor, n_rows: int):
     """(row pointer, permutation into row order or None if they are in it, the columns in that order
     once asked for) of row coordinates, kept with their tensor since an earlier product; None if
     there is nothing (valid) kept."""
-    kept = getattr(rows, "_scorch_row_order", None)
+    kept = _kept(rows, "_scorch_row_order")
     return kept[2] if kept is not None and kept[0] == _stamp(rows) and kept[1] == n_rows else None
 
 
@@ -1938,7 +1961,7 @@ def attention_block_mask(row_ptr: torch.Tensor, col_idx: torch.Tensor, S: int) -
     """block_mask_from_csr, kept with the mask's row_ptr tensor and rebuilt when either index
     array is replaced or written to."""
     key = (_stamp(row_ptr), _stamp(col_idx), S)
-    cached = getattr(row_ptr, "_scorch_block_mask", None)
+    cached = _kept(row_ptr, "_scorch_block_mask")
     if cached is not None and cached[0] == key and _same(cached[2], col_idx):
         return cached[1]
     if torch.cuda.is_current_stream_capturing():
@@ -1946,7 +1969,7 @@ def attention_block_mask(row_ptr: torch.Tensor, col_idx: torch.Tensor, S: int) -
                            "attention_block_mask(row_ptr, col_idx, S) once before capturing")
     bm = split_long_block_rows(block_mask_from_csr(row_ptr, col_idx, S))
     try:
-        row_ptr._scorch_block_mask = (key, bm, weakref.ref(col_idx))
+        row_ptr._scorch_block_mask = _Kept((key, bm, weakref.ref(col_idx)))
     except AttributeError:
         pass
     return bm
@@ -2125,7 +2148,7 @@ def attn_blocksparse_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bm: 
             q.data_ptr(), k.data_ptr(), v.data_ptr(), float(scale), out.data_ptr(),
             ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, stream)
     native.check(rc)
-    if ws is not None:
+    if ws is not None and torch.cuda.is_current_stream_capturing():
         out._scorch_workspace = ws     # a buffer handed out during a graph capture lives as long as the result
     return out
 
@@ -2164,7 +2187,7 @@ def _attn_bf16_items(q, k, v, bm: BlockMask, items: torch.Tensor, split_rows: Op
             v.data_ptr(), float(scale), out.data_ptr(), ws.data_ptr() if ws is not None else None,
             ws.numel() if ws is not None else 0, stream)
     native.check(rc)
-    if ws is not None:
+    if ws is not None and torch.cuda.is_current_stream_capturing():
         out._scorch_workspace = ws     # a buffer handed out during a graph capture lives as long as the result
     return out
 
@@ -2257,7 +2280,7 @@ def _block_row_schedule(brp: torch.Tensor):
     decisions) of a block row pointer, read back once and kept with the tensor; None while the
     stream is capturing and nothing is known yet."""
     import numpy as np
-    cached = getattr(brp, "_scorch_rows", None)
+    cached = _kept(brp, "_scorch_rows")
     if cached is not None and cached[0] == _stamp(brp):
         return cached[1:]
     if torch.cuda.is_current_stream_capturing():
@@ -2265,7 +2288,7 @@ def _block_row_schedule(brp: torch.Tensor):
     ptrs = brp.cpu().numpy().astype(np.int64)
     lens = ptrs[1:] - ptrs[:-1]
     items, _, _ = _stretches(lens, max(int(lens.max()), 1) if lens.size else 1, True)
-    entry = (_stamp(brp), lens, torch.from_numpy(items).to(brp.device).reshape(-1), {})
+    entry = _Kept((_stamp(brp), lens, torch.from_numpy(items).to(brp.device).reshape(-1), {}))
     if brp.is_cuda:
         _made_on(_stream(brp.device), entry[2])
     try:
@@ -2305,11 +2328,11 @@ def attn_blocksparse_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, blo
         n_masks = block_masks.numel() // block
         # the kernel trusts the mask indices as it trusts block_col_idx; a caller that built them by
         # hand gets them checked here, once per index tensor
-        if getattr(bmi, "_scorch_mask_checked", None) != (_stamp(bmi), n_masks):
+        if _kept(bmi, "_scorch_mask_checked") != (_stamp(bmi), n_masks):
             if bmi.numel() and int(bmi.max()) >= n_masks:
                 raise ValueError("scorch_ops_hip: block_mask_index names a mask beyond block_masks")
             try:
-                bmi._scorch_mask_checked = (_stamp(bmi), n_masks)
+                bmi._scorch_mask_checked = _Kept((_stamp(bmi), n_masks))
             except AttributeError:
                 pass
     schedule = _block_row_schedule(brp) if block == 64 and D in ATTENTION_WORKGROUPS_PER_CU else None

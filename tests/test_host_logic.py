@@ -630,3 +630,42 @@ def test_the_native_call_path_is_built_for_this_torch_or_done_without(monkeypatc
         host = native.host()
     assert host.spmm(1, 2, None, 0) is None and host.sddmm(1, 2, 3) is None and host.attention(*range(7)) is None
     assert host.remember() is None and host.remember_attention() is None
+
+
+@pytest.mark.parametrize("how", ["save", "pickle", "deepcopy"])
+def test_copies_of_a_tensor_get_nothing_of_what_is_kept_with_it(how):
+    """A row pointer, a value tensor or a mask that has been multiplied with can be saved, pickled and copied, the
+    file is read with weights_only, and the copy starts without plans and decisions."""
+    import copy
+    import io
+    import pickle
+    import weakref
+
+    from scorch_amd import native
+    kept, H = scorch_ops_hip._Kept, scorch_ops_hip
+    t, partner = torch.arange(5, dtype=torch.int32), torch.arange(4, dtype=torch.int32)
+    plan = H.CsrPlan((1, 2), 3, 4)
+    plan.partner = weakref.ref(partner)
+    plan.bounds[(1, 4)] = torch.zeros(1000)
+    t._scorch_plan = plan
+    t._scorch_epoch = 3
+    H._made_on(7, t)
+    for name in H._CACHE_ATTRIBUTES:
+        if not hasattr(t, name):
+            setattr(t, name, kept((H._stamp(t), torch.zeros(1000), weakref.ref(partner), None, None, {})))
+    del t._scorch_attention
+    native.host().remember_attention(t, partner, weakref.ref(partner), 2, (1, 64, 32), torch.zeros(1), (), (), 0)
+    if how == "save":
+        buffer = io.BytesIO()
+        torch.save(t, buffer)
+        assert buffer.tell() < 4000
+        buffer.seek(0)
+        twin = torch.load(buffer, weights_only=True)
+    else:
+        twin = pickle.loads(pickle.dumps(t)) if how == "pickle" else copy.deepcopy(t)
+    assert torch.equal(twin, t)
+    assert H._plan_kept(t) is plan and H._plan_kept(twin) is None
+    assert all(H._kept(twin, name) is None for name in H._CACHE_ATTRIBUTES)
+    assert H._plan_at_hand(twin, partner, 4, 5) is None and H._known_row_order(twin, 4) is None
+    H.forget(twin)
+    assert not any(hasattr(twin, name) for name in H._CACHE_ATTRIBUTES)
