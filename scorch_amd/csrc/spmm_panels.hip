@@ -217,11 +217,14 @@ int launch_panels(int64_t M, int64_t K, int64_t N, const int *row_ptr, const int
   const int64_t panels = (N + P - 1) / P;
   const int64_t grid = round_up_8(panels * shares);
   if (grid > INT32_MAX) return fail(SCORCH_HIP_EUNSUPPORTED, "SpMM (panels): %lld workgroups exceed the launch limit", (long long)grid);
-  static std::atomic<int> allowed{0};  // (per kernel)
-  if (!allowed.load(std::memory_order_acquire)) {
+  static std::atomic<uint64_t> allowed{0};  // (per kernel) a bit per device: the attribute is a device's own
+  int device = 0;
+  SCORCH_HIP_CHECK(hipGetDevice(&device));
+  const uint64_t bit = 1ull << (device & 63);
+  if (device > 63 || !(allowed.load(std::memory_order_acquire) & bit)) {
     SCORCH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&spmm_panels_kernel<P, R>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, kPanelLds));
-    allowed.store(1, std::memory_order_release);
+    allowed.fetch_or(bit, std::memory_order_release);
   }
   mark_launch(s);
   spmm_panels_kernel<P, R><<<dim3((unsigned)grid), kPanelThreads, (size_t)panel_lds(K, P, R), s>>>(
