@@ -669,3 +669,57 @@ def test_copies_of_a_tensor_get_nothing_of_what_is_kept_with_it(how):
     assert H._plan_at_hand(twin, partner, 4, 5) is None and H._known_row_order(twin, 4) is None
     H.forget(twin)
     assert not any(hasattr(twin, name) for name in H._CACHE_ATTRIBUTES)
+
+
+def _rows(*stretches):
+    return np.concatenate([np.full(count, length, np.int64) for length, count in stretches])
+
+
+@pytest.mark.parametrize("lens, heads, D, want", [
+    # share of a CU below two blocks: stretches of two (S = 3,001, 8 heads, window: 47 rows, one of them long)
+    (_rows((3, 46), (47, 1)), 8, 64, 4), (_rows((3, 46), (47, 1)), 1, 64, 2),
+    # the longest row against half as much again as a CU's share
+    (_rows((24, 256)), 1, 64, None), (_rows((23, 255), (36, 1)), 1, 64, 8), (_rows((24, 255), (36, 1)), 1, 64, None),
+    # rows of two blocks are never cut
+    (_rows((2, 8)), 1, 64, None), (_rows((2, 8), (3, 1)), 1, 64, 2),
+    # four blocks up to a share of 16 (at D = 64), eight up to 64, whole rows beyond; twice and half of that at 32 and 128
+    (_rows((15, 255), (64, 1)), 1, 64, 4), (_rows((17, 255), (64, 1)), 1, 64, 8), (_rows((17, 255), (64, 1)), 1, 32, 4),
+    (_rows((15, 255), (64, 1)), 1, 128, 8), (_rows((62, 255), (128, 1)), 1, 64, 8), (_rows((64, 255), (256, 1)), 1, 64, None),
+    (_rows((33, 255), (256, 1)), 1, 128, None), (_rows((33, 255), (256, 1)), 1, 32, 8),
+    (np.zeros(0, np.int64), 1, 64, None), (_rows((0, 5)), 1, 64, None),
+])
+def test_stretches_of_the_fused_fp32_kernel_on_either_side_of_every_rule(lens, heads, D, want):
+    assert scorch_ops_hip._fp32_stretch(lens, heads, D, 256) == want
+
+
+@pytest.mark.parametrize("lens, heads, D, want", [
+    # no row stands out: whole rows, unless half the CUs at most have one and some row has 16 blocks or more
+    (_rows((7, 128)), 1, 64, None), (_rows((16, 128)), 1, 64, 8), (_rows((15, 128)), 1, 64, None), (_rows((16, 129)), 1, 64, None),
+    (_rows((16, 64)), 2, 64, 8), (_rows((16, 65)), 2, 64, None),
+    # a row stands out beyond eight blocks and twice the mean, rounded up
+    (_rows((1, 511), (8, 1)), 16, 64, None), (_rows((1, 511), (9, 1)), 16, 64, 8), (_rows((10, 255), (22, 1)), 16, 64, None),
+    (_rows((10, 255), (23, 1)), 16, 64, 20),
+    # a launch that leaves a quarter of the chip idle (768 of 1,024 workgroups at D = 64): half of that, four at least
+    (_rows((3, 63), (64, 1)), 11, 64, 4), (_rows((3, 63), (64, 1)), 12, 64, 8), (_rows((10, 63), (64, 1)), 11, 64, 10),
+    (_rows((3, 63), (64, 1)), 5, 128, 4), (_rows((3, 63), (64, 1)), 6, 128, 8), (_rows((3, 63), (64, 1)), 14, 32, 4),
+    (_rows((3, 63), (64, 1)), 15, 32, 8), (_rows((3, 63), (64, 1)), 8, 48, None), (np.zeros(0, np.int64), 8, 64, None),
+])
+def test_stretches_of_the_fused_bf16_kernel_on_either_side_of_every_rule(lens, heads, D, want):
+    assert scorch_ops_hip._bf16_stretch(lens, heads, D, 256) == want
+
+
+@pytest.mark.parametrize("lens, heads, want", [          # D = 64: the chip holds 1,024 workgroups at once
+    (_rows((4, 613)), 1, False), (_rows((4, 615)), 1, True),                                   # 0.6 rounds
+    (_rows((4, 64)), 64, True), (_rows((4, 4097)), 1, False),                                  # 4 rounds
+    (_rows((4, 2048)), 1, True), (_rows((4, 2049)), 1, False), (_rows((4, 2730)), 1, False), (_rows((4, 2731)), 1, True),
+    (_rows((6, 1024)), 1, True), (_rows((7, 1024)), 1, False),                                 # equal rows: at most six blocks
+    (_rows((4, 768), (5, 256)), 1, True),                                                      # equal within a quarter of the mean
+    (_rows((6, 512), (8, 512)), 1, False), (_rows((6, 512), (8, 512)), 2, False),              # (7 on average: 8 is within a quarter)
+    (_rows((5, 512), (9, 512)), 2, False), (_rows((5, 512), (10, 512)), 2, True),              # unequal: more than seven on average
+    (_rows((8, 512), (14, 512)), 1, False), (_rows((8, 538), (14, 538)), 1, True),             # and more than 1.05 rounds
+    (_rows((8, 900), (20, 124)), 1, True),                                                     # or a row of more than 1.75 times the mean
+    (_rows((60, 1023), (64, 1)), 1, False), (_rows((63, 1000), (200, 24)), 1, False),          # equal rows of many blocks; 66 on average
+    (_rows((58, 1000), (200, 24)), 1, True), (_rows((4, 1)), 1024, False),                     # a single item has no partner
+])
+def test_pairs_of_the_fused_bf16_kernel_on_either_side_of_every_rule(lens, heads, want):
+    assert scorch_ops_hip.pair_attention_items(lens, heads, 64) is want
