@@ -21,10 +21,12 @@
 // carry_row[chunk].  The chunk holding the marker stores only its own part.
 // spmm_fixup_kernel then adds, in chunk order, the carries of each such row
 // to C: a fixed summation order, so results are bit-reproducible, and no
-// atomics.  A fused bias/ReLU epilogue is applied at the store when the row
-// lies wholly inside the chunk, and by the fix-up otherwise.
+// floating-point atomics.  A fused bias/ReLU epilogue is applied at the store when the row
+// lies wholly inside the chunk, and by the fix-up otherwise.  A caller with counters for the
+// launch saves the second one: the last of a row's chunks to finish adds the carries up, in
+// the same order (finish_part).
 //
-// Columns beyond 64 * VEC are covered by column tiles (each tile walks the same
+// Columns beyond 64 * VEC are covered by column tiles (tile_lanes; each tile walks the same
 // chunks again; A's indices are small next to the B rows gathered).  Tiles are
 // placed on XCDs so that a tile's slice of B stays in one L2 (map_workgroup).
 #include "spmm.hpp"
