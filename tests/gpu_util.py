@@ -60,6 +60,15 @@ def hip_spmv(row_ptr, col_idx, vals, x):
     return host(out.storage.value)
 
 
+def three_step_attention(row_ptr, col_idx, q, k, v, scale):
+    """SDDMM, row softmax and SpMM of all heads, a launch each (sparse_attention_csr itself goes to the fused kernel
+    where the mask fills its blocks and has come back)."""
+    S = int(q.shape[1])
+    mask = [[], [row_ptr, col_idx]]
+    scores, _ = H.sddmm_csr_float_batched([S, S], mask, None, q, k)
+    return H.spmm_csr_float_batched([S, S], mask, H.softmax_csr_float_batched(row_ptr, scores, scale), v)
+
+
 def hip_sddmm_coo(row_idx, col_idx, svals, A, B, shape):
     r, c = dev(row_idx), dev(col_idx)
     out = H.sddmm_coo_float_prebuilt(list(shape), list(shape), [[r], [c]], dev(svals), list(A.shape),

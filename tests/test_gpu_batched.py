@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import dev, spmm_path
+from gpu_util import dev, spmm_path, three_step_attention
 from scorch_amd import scorch_ops_hip as H
 from scorch_amd import workloads
 
@@ -87,10 +87,14 @@ def test_sparse_attention_at_the_reference_benchmarks_shape():
         ref = p @ v[h].double()
         worst = max(worst, (torch.linalg.norm(out[h].double() - ref) / torch.linalg.norm(ref)).item())
     assert worst <= 1e-5, worst          # fp32 throughout (the bf16 bar of the fused kernel is 1e-2)
-    # the mask has come back: its two products now run by blocks (same bar), and from here on the
-    # result is the same bits from call to call
+    # the mask has come back: the fused kernel takes it now, the three steps' products run by blocks (same
+    # bar), and from here on the result is the same bits from call to call
     again = H.sparse_attention_csr(rp, ci, q, k, v, scale)
-    assert isinstance(rp._scorch_plan.blocked, H.BlockedCsr)
+    assert isinstance(rp._scorch_plan.attention, H.BlockMask) and isinstance(rp._scorch_plan.blocked, H.BlockedCsr)
+    steps = three_step_attention(rp, ci, q, k, v, scale)
+    assert torch.equal(steps, three_step_attention(rp, ci, q, k, v, scale))
+    assert max((torch.linalg.norm(steps[h].double() - out[h].double()) / torch.linalg.norm(out[h].double())).item()
+               for h in range(heads)) <= 2e-6
     worst = max((torch.linalg.norm(again[h].double() - out[h].double()) / torch.linalg.norm(out[h].double())).item()
                 for h in range(heads))
     assert worst <= 2e-6, worst

@@ -214,7 +214,11 @@ def test_batched_equals_per_head_and_repeats_bit_for_bit():
         assert torch.equal(prod.storage.value.view(M, 64), c[h])
 
 
-def test_sparse_attention_through_the_block_kernels(oracle):
+@pytest.mark.parametrize("path", ["auto", "always"])
+def test_sparse_attention_through_the_block_kernels(oracle, path, monkeypatch):
+    """With the block kernels pinned the two products are theirs; left alone, a mask that fills its blocks goes to the
+    fused kernel when it comes back."""
+    monkeypatch.setattr(H, "BLOCKED_PATH", path)
     rng = np.random.default_rng(11)
     S, heads, D = 512, 4, 64
     mask = pattern("window", S, S, rng)
@@ -224,11 +228,14 @@ def test_sparse_attention_through_the_block_kernels(oracle):
     H.sparse_attention_csr(pos, crd, dev(q), dev(k), dev(v), D ** -0.5)
     got = host(H.sparse_attention_csr(pos, crd, dev(q), dev(k), dev(v), D ** -0.5))
     assert isinstance(pos._scorch_plan.blocked, H.BlockedCsr)
+    assert (pos._scorch_plan.attention is None) == (path == "always")
     for h in range(heads):
         assert oracle.rel_fro(got[h], oracle.attention_dense_fp64(q[h], k[h], v[h], mask, D ** -0.5)) <= TOL
 
 
-def test_recorded_step_replays_the_block_kernels(oracle):
+@pytest.mark.parametrize("path", ["auto", "always"])
+def test_recorded_step_replays_the_block_kernels(oracle, path, monkeypatch):
+    monkeypatch.setattr(H, "BLOCKED_PATH", path)         # (auto: the fused kernel's)
     rng = np.random.default_rng(12)
     S, heads, D = 256, 2, 32
     mask = pattern("causal", S, S, rng)
