@@ -597,10 +597,10 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
 // last of the row's chunks (finish_part) where the caller has counters, else by spmv_fixup_kernel.
 //
 // Bound: the gathers of x, one L2 request each; past 4 MB of x most of them miss their XCD's L2 and
-// are bound by the fabric (1 M rows, 11 M entries, fp64, power-law: 203 us, 7 TB/s of 128-byte lines;
-// without a plan's boundaries and with the second launch 211 us).  Small matrices are bound by the launch: 2000
-// rows 19.1 -> 6.1 us per call, 100 k rows x 10 19.7 -> 10.8 us with one launch instead of two and
-// boundaries read instead of searched for.
+// are bound by the fabric (1 M rows, 17.8 M entries, fp64, power-law: 203 us; 1.4 GB fetched, 10.9 M of
+// 18.4 M line requests past their L2, 7.0 TB/s; without a plan's boundaries and with the second
+// launch 211 us).  Small matrices are bound by the launch: 2000 rows 19.1 -> 6.1 us per call, 100 k
+// rows x 10 19.7 -> 10.8 us with one launch instead of two and boundaries read instead of searched for.
 constexpr int kSpmvItems = 512;
 // large matrices take chunks twice the size: 16 loads per lane in flight instead of 8, half
 // the chunks to start and to fix up (0.124 -> 0.117 ms on a 17 M-nonzero graph); smaller
