@@ -243,8 +243,9 @@ def _epoch(t: torch.Tensor) -> int:
 
 
 def _stamp(t: torch.Tensor):
-    """What must be unchanged for data derived from `t` to be served again."""
-    return (t.data_ptr(), t._version, _epoch(t), t.numel())
+    """What must be unchanged for data derived from `t` to be served again.  An inference tensor has no
+    version counter, and no two of its stamps are equal: what is derived from it serves one call."""
+    return (t.data_ptr(), object() if t.is_inference() else t._version, _epoch(t), t.numel())
 
 
 def _same(ref, t: torch.Tensor) -> bool:

@@ -13,7 +13,7 @@ import torch
 import scorch_amd as scorch
 from conftest import random_csr
 from gpu_util import dev, host
-from scorch_amd import graphs
+from scorch_amd import graphs, workloads
 from scorch_amd import scorch_ops_hip as H
 
 pytestmark = pytest.mark.gpu
@@ -195,3 +195,48 @@ def test_a_new_index_tensor_at_a_freed_tensors_address_is_not_taken_for_it():
             break
     with pytest.raises(ValueError, match="column index"):
         product(crd)
+
+
+@pytest.mark.parametrize("form", ["csr", "coo", "coo_unsorted"])
+def test_operands_made_in_inference_mode(form):
+    """Tensors without version counters: nothing derived from them is served to a second call, so a write
+    that nothing can see is seen -- values, columns, a dense operand of a width that would be tiled, masks."""
+    rng = np.random.default_rng(90)
+    n, N = 256, 512
+    rp, ci, v = random_csr(rng, n, n, 0.05)
+    rows = np.repeat(np.arange(n), np.diff(rp)).astype(np.int32)
+    order = rng.permutation(rows.size) if form == "coo_unsorted" else np.arange(rows.size)
+    with torch.inference_mode():
+        dr, dc, dv = (dev(x) + 0 for x in (rows[order], ci[order], v[order]))
+        A = scorch.STensor.from_csr_arrays(dev(rp) + 0, dc, dv, (n, n)) if form == "csr" else \
+            scorch.STensor._coo((n, n), [dr, dc], dv, "A")
+        assert A.values.is_inference()
+        for turn in range(4):
+            for width in (N, 24, None):
+                b = torch.randn(n, width, device="cuda") if width else torch.randn(n, device="cuda")
+                if width is None and form != "csr":
+                    continue
+                dense = torch.zeros(n, n, dtype=torch.float64)
+                dense.index_put_((dr.long().cpu(), dc.long().cpu()), dv.double().cpu(), accumulate=True)
+                for _ in range(3):
+                    got = scorch.matmul(A, b)
+                    want = dense @ b.double().cpu()
+                    assert float((got.double().cpu() - want).norm()) <= 1e-5 * float(want.norm())
+                    b.mul_(0.5)
+            q, k = torch.randn(n, 64, device="cuda"), torch.randn(n, 64, device="cuda")
+            for _ in range(3):
+                out = scorch.einsum("ij,ik,jk->ij", A, q, k).values.double().cpu()
+                want = (dv.double() * (q.double()[dr.long()] * k.double()[dc.long()]).sum(1)).cpu()
+                assert float((out - want).norm()) <= 1e-5 * float(want.norm())
+                dv.fill_(1.0) if turn == 1 else dv.mul_(1.5)
+            dc.copy_(torch.randint(n, (dc.numel(),), device="cuda", dtype=torch.int32))
+        if form == "csr":
+            pos, crd = (dev(x) + 0 for x in workloads.longformer_mask(n))
+            h = torch.randn(2, n, 64, device="cuda")
+            want = H.sparse_attention_csr(pos.clone(), crd.clone(), h, h, h, 0.1)
+            for _ in range(3):
+                assert float((H.sparse_attention_csr(pos, crd, h, h, h, 0.1) - want).norm()) <= 1e-5 * float(want.norm())
+                assert float((H.sparse_attention_f32(h, h, h, pos, crd, 0.1) - want).norm()) <= 1e-5 * float(want.norm())
+            dc[0] = n + 5
+            with pytest.raises(ValueError, match="column"):
+                scorch.matmul(A, b)
