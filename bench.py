@@ -63,9 +63,9 @@ MEASURED_TRAFFIC = {
     ("sae_decoder", "merge"): {"bytes": 1_767_200_000, "sources": _SPMM_SOURCES, "sha16": "4adff1435fde6270",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
     ("sddmm_uniform", "listed"): {"bytes": 277_700_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
-                                  "sha16": "d2d68c326f9e656a", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
+                                  "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
     ("sddmm_uniform", "plain"): {"bytes": 848_400_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
-                                 "sha16": "d2d68c326f9e656a", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
+                                 "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
     ("attention_blocksparse", "fused"): {"bytes": 81_050_000, "sources": (_CSRC + "attn.hip", _CSRC + "common.hpp"),
                                          "sha16": "93359f7faeb90848", "profile": "profiles/attn_blocksparse_kernel_s8192_h16.md"},
 }
@@ -513,7 +513,7 @@ def run_sddmm(args):
                       "seed": workloads.SEEDS["sddmm_uniform"]},
            "warmup_ms": warm,
            "path": "listed" if listed else "plain",
-           "roofline": _hbm_roofline("sddmm_listed_kernel<16,4>" if listed else "sddmm_kernel<16,4,false,false>",
+           "roofline": _hbm_roofline("sddmm_listed_kernel<8,2,false>" if listed else "sddmm_kernel<8,2,false,false>",
                                      kernel_ms, algo, traffic, provenance,
                                      {"kernel_ms_queued": round(ms, 5),
                                       "row_coordinate_output_bytes": 4 * nnz, "gather_model_bytes": gather,

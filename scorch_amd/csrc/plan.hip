@@ -31,7 +31,7 @@ namespace {
 constexpr int kPlanWidths = 8;              // chunk boundaries kept for this many values of N
 constexpr int64_t kSoftmaxShortRow = 4096;  // rows up to this length: the one-launch softmax
 constexpr int64_t kFillFirstBytes = (int64_t)32 << 20;
-constexpr int64_t kListsMinDense = (int64_t)8 << 20, kListsMaxDense = (int64_t)20 << 20;
+constexpr int64_t kListsMinDense = (int64_t)9 << 19, kListsMaxDense = (int64_t)20 << 20;
 
 struct Boundaries {
   int64_t N = -1;

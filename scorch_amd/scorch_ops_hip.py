@@ -1241,8 +1241,10 @@ SDDMM_PATH = os.environ.get("SCORCH_HIP_SDDMM_PATH", "auto")
 
 def _lists_apply(nnz: int, n_cols: int, K: int) -> bool:
     """Whether SDDMMs of this shape are served from per-XCD entry lists when their mask comes back: B
-    beyond one L2 and within the eight together, and used often enough."""
-    return 0 < K <= 256 and (8 << 20) <= n_cols * K * 4 <= (20 << 20) and nnz >= 4 * n_cols
+    beyond one L2 (4 MiB) and within the eight together, and used often enough.  Where B is 4 MiB the plain
+    kernel is as fast (20,000 columns, 600 K entries, K = 50: 17.8 us, by lists 18.0), at 4.9 MiB it no longer
+    is (4 M entries, K = 64: 72.7 against 65.1; 6.1 MiB, 10 M entries, K = 16: 99 against 73)."""
+    return 0 < K <= 256 and (9 << 19) <= n_cols * K * 4 <= (20 << 20) and nnz >= 4 * n_cols
 
 
 def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int, L, stream) -> Optional[torch.Tensor]:

@@ -60,6 +60,44 @@ def test_inner_dimensions(oracle, K):
     np.testing.assert_allclose(coo, oracle.sddmm_coo_f32(rows, ci, s, A, B), rtol=1e-4, atol=1e-5)
 
 
+# K on either side of every shape of a lane group (4, 8 and 16 lanes, one to four 16-byte pieces) and where a row's
+# last piece is shared with the one before
+@pytest.mark.parametrize("K", [3, 4, 7, 17, 33, 36, 50, 63, 67, 97, 99, 129, 130, 191, 193, 253, 255])
+def test_rows_staged_in_lds_and_rows_read_by_every_entry(oracle, monkeypatch, K):
+    """Entries in row order share their row of A through LDS, entries in any order (64 rows among 64 entries) read
+    their own: the same bits.  An infinity in a row's last element reaches the entries of that row and column only."""
+    rng = np.random.default_rng(K)
+    rp, ci, s = random_csr(rng, 300, 90, 0.3, empty_rows=(0, 150, 299))
+    rows = oracle.rows_of(rp)
+    A, B = rng.standard_normal((300, K)).astype(np.float32), rng.standard_normal((90, K)).astype(np.float32)
+    r, c, csr = hip_sddmm_csr(rp, ci, s, A, B, (300, 90))
+    perm = rng.permutation(s.size)
+    assert np.array_equal(csr[perm], hip_sddmm_coo(rows[perm], ci[perm], s[perm], A, B, (300, 90)))
+    assert oracle.rel_fro(csr, oracle.sddmm_fp64(rows, ci, s, A, B)) <= TOL
+    monkeypatch.setattr(H, "SDDMM_PATH", "listed")
+    assert np.array_equal(csr, hip_sddmm_csr(rp, ci, s, A, B, (300, 90))[2])
+    monkeypatch.setattr(H, "SDDMM_PATH", "plain")
+    A[7, K - 1], B[11, K - 1], B[12, 0] = np.inf, -np.inf, np.nan
+    wild = hip_sddmm_csr(rp, ci, s, A, B, (300, 90))[2]
+    apart = (rows != 7) & (ci != 11) & (ci != 12)
+    assert np.array_equal(wild[apart], csr[apart])
+    with np.errstate(invalid="ignore"):
+        expected = s[~apart] * np.einsum("ek,ek->e", A[rows[~apart]].astype(np.float64), B[ci[~apart]].astype(np.float64))
+    np.testing.assert_allclose(wild[~apart], expected.astype(np.float32), rtol=1e-3, atol=1e-4)
+
+
+@pytest.mark.parametrize("nnz", [1, 63, 64, 65, 256, 257, 16385])
+def test_short_and_ragged_last_pieces(oracle, nnz):
+    rng = np.random.default_rng(nnz)
+    flat = np.sort(rng.choice(400 * 300, nnz, replace=False))
+    rows, ci, s = (flat // 300).astype(np.int32), (flat % 300).astype(np.int32), rng.standard_normal(nnz).astype(np.float32)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=400))]).astype(np.int32)
+    A, B = rng.standard_normal((400, 64)).astype(np.float32), rng.standard_normal((300, 64)).astype(np.float32)
+    r, c, csr = hip_sddmm_csr(rp, ci, s, A, B, (400, 300))
+    assert np.array_equal(r, rows) and np.array_equal(csr, hip_sddmm_coo(rows, ci, s, A, B, (400, 300)))
+    assert oracle.rel_fro(csr, oracle.sddmm_fp64(rows, ci, s, A, B)) <= TOL
+
+
 def test_coo_entries_in_any_order(oracle):
     rng = np.random.default_rng(5)
     rp, ci, s = random_csr(rng, 300, 300, 0.05)
