@@ -52,15 +52,15 @@ CONFIG_WORKLOADS = ("spmm_uniform", "sddmm_uniform", "attention_blocksparse", "s
 _CSRC = "scorch_amd/csrc/"
 _SPMM_SOURCES = (_CSRC + "spmm.hip", _CSRC + "spmm.hpp", _CSRC + "common.hpp")
 MEASURED_TRAFFIC = {
-    ("gcn_powerlaw", "merge"): {"bytes": 9_789_900_000, "sources": _SPMM_SOURCES, "sha16": "4adff1435fde6270",
+    ("gcn_powerlaw", "merge"): {"bytes": 9_789_900_000, "sources": _SPMM_SOURCES, "sha16": "",
                                 "profile": "profiles/spmm_merge_kernel_gcn_powerlaw.md"},
     ("spmm_uniform", "rows"): {"bytes": 10_834_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp",
-                                                                _CSRC + "common.hpp"), "sha16": "d867733f2e85735c",
+                                                                _CSRC + "common.hpp"), "sha16": "",
                                "profile": "profiles/spmm_rows_kernel_uniform_4096.md"},
     ("sae_decoder", "tiled"): {"bytes": 344_300_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp",
-                                                                 _CSRC + "common.hpp"), "sha16": "aeffb325fcf43940",
+                                                                 _CSRC + "common.hpp"), "sha16": "",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
-    ("sae_decoder", "merge"): {"bytes": 1_767_200_000, "sources": _SPMM_SOURCES, "sha16": "4adff1435fde6270",
+    ("sae_decoder", "merge"): {"bytes": 1_767_200_000, "sources": _SPMM_SOURCES, "sha16": "",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
     ("sddmm_uniform", "listed"): {"bytes": 277_700_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
                                   "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},

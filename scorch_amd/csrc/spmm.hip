@@ -182,6 +182,226 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
   }
 }
 
+// ---- narrow column tiles: a lane group per stretch of entries ---------------------------------
+// When a row of B is narrower than a wavefront's 64 lanes can cover with full vectors (at most 256
+// bytes, see narrow_tile_bytes), LPR lanes take an entry, and a workgroup takes a chunk of up to
+// kGroupedItems merge items: its 256 / LPR lane groups walk equal, contiguous stretches of the chunk's
+// entries, whatever rows those belong to, four entries at a time and the next four requested meanwhile.
+//
+// What bounds such a product is a chain of a few reads (boundaries, then columns and values, then B),
+// a microsecond or more each, and how many chunks have to go through it one after the other: so
+// grouped_split sizes the chunks such that all of them are resident at once where they can be.  Chunks
+// of a workgroup instead of a wavefront leave a quarter of the parts of a long row to be folded through memory
+// (the fold is still 2 to 3 us of products of 6 to 20).  50,021 power-law rows of 12, N = 37: 27.0 -> 20.3 us; 2,708 rows
+// of 5, N = 16: 7.6 -> 6.3; 929 rows of 7, N = 41: 8.2 -> 6.6.
+//
+// Rows end inside stretches and go on in the next.  The last entry of every row is marked; at a mark the
+// group stores its sum, unless the row began in an earlier group: that sum waits until the walk is over,
+// and the sums that the groups before had left at the end of their stretches are then added up in their
+// order.  The summation order depends on the chunk alone.
+constexpr int kGroupedSlots = kGroupedItems + kSnapItems;
+
+// A barrier for what is exchanged through LDS: unlike __syncthreads() it does not wait for stores to C.
+__device__ __forceinline__ void workgroup_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <typename T, int VEC, int LPR, int EPI>
+__global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
+    int M, int N, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
+    const T *__restrict__ vals, const T *__restrict__ B, T *__restrict__ C,
+    const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int64_t chunks,
+    int *__restrict__ carry_row, T *__restrict__ carry_val,
+    const Boundary *__restrict__ bounds, SpmmBatch batch, int *__restrict__ counters) {
+  using A = typename Acc<T>::type;
+  using VecT = Vec<T, VEC>;
+  constexpr int kGroups = kBlockThreads / LPR;
+  constexpr int kPadded = (kGroupedSlots + 4 * kGroups - 1) / (4 * kGroups) * (4 * kGroups);
+  vals += blockIdx.y * batch.vals;  // problem blockIdx.y of a batch over one pattern
+  B += blockIdx.y * batch.b;
+  C += blockIdx.y * batch.c;
+  carry_val += blockIdx.y * batch.carry;
+
+  // (behind the chunk's entries the last stretches are filled up with zeros that no row's mark follows)
+  __shared__ __attribute__((aligned(16))) int s_col[kPadded];
+  __shared__ __attribute__((aligned(16))) T s_val[kPadded];
+  __shared__ __attribute__((aligned(16))) unsigned short s_mark[kPadded];  // last entries of rows: the row's slot + 1
+  __shared__ int s_rp[kGroupedSlots + 2];
+  __shared__ VecT s_last[kBlockThreads];
+
+  const int tid = threadIdx.x;
+  const int group = tid / LPR;
+  const int t = tid % LPR;
+  const int64_t span = xcd_contiguous(blockIdx.x, gridDim.x);
+  if (span >= chunks) return;
+  const int col0 = lane_column<VEC>(t * VEC, N);
+  const bool active = col0 < N;
+
+  const int64_t d0 = span * items_per_chunk;
+  const Boundary from = bounds ? load_boundary(bounds, span) : chunk_boundary(d0, M, total_items, row_ptr, kSnapItems);
+  const Boundary to = bounds ? load_boundary(bounds, span + 1)
+                             : chunk_boundary(d0 + items_per_chunk, M, total_items, row_ptr, kSnapItems);
+  const int x0 = from.x, y0 = from.y, x1 = to.x, y1 = to.y;
+  const int n_nz = y1 - y0;
+  const int n_rows = x1 - x0;
+  const int stretch = (n_nz + 4 * kGroups - 1) / (4 * kGroups) * 4;
+
+  for (int k = tid * 4; k < stretch * kGroups; k += kBlockThreads * 4)
+    *reinterpret_cast<unsigned long long *>(&s_mark[k]) = 0ull;
+  workgroup_lds_sync();
+  T bias_v[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) bias_v[v] = (EPI != kEpiNone && active) ? bias[col0 + v] : (T)0;
+
+  // Row slot r is row x0 + r; slot n_rows is the row that continues past the chunk.
+  struct Range { int lo, hi; };  // its entries, counted from y0
+  auto entries_of = [&](int begin, int end) {
+    Range r;
+    r.lo = (begin > y0 ? begin : y0) - y0;
+    r.hi = (end < y1 ? end : y1) - y0;
+    if (r.hi < r.lo) r.hi = r.lo;
+    return r;
+  };
+  bool empty_rows = false;  // of this thread's
+  for (int k = tid; k < stretch * kGroups; k += kBlockThreads) {
+    s_col[k] = k < n_nz ? col_idx[y0 + k] : 0;
+    s_val[k] = k < n_nz ? vals[y0 + k] : (T)0;
+  }
+  for (int k = tid; k <= n_rows; k += kBlockThreads) {
+    const int begin = row_ptr[x0 + k], end = row_ptr[x0 + k < M ? x0 + k + 1 : M];
+    s_rp[k] = begin;
+    if (k == n_rows) s_rp[k + 1] = end;
+    const Range r = entries_of(begin, end);
+    if (r.hi > r.lo) s_mark[r.hi - 1] = (unsigned short)(k + 1);
+    else empty_rows |= k < n_rows;
+  }
+  const bool any_empty = __syncthreads_or(empty_rows);
+
+  const bool carry_in = uniform(s_rp[0]) < y0;  // row x0 began in an earlier chunk
+  auto store_row = [&](int slot, const A (&sum)[VEC]) {
+    if (!active) return;
+    VecT o;
+    if (slot < n_rows) {
+      const bool partial = carry_in && slot == 0;
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) o.v[v] = partial ? (T)sum[v] : apply_epilogue<T, EPI>(sum[v], bias_v[v]);
+      T *dst = C + (size_t)(x0 + slot) * (size_t)N + col0;
+      if (partial && counters) store_part<T, VEC>(dst, o);
+      else if constexpr (sizeof(VecT) * LPR > 128) store_streaming(dst, o);
+      else store_vec<T, VEC>(dst, o);
+    } else {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) o.v[v] = (T)sum[v];
+      T *dst = carry_val + (size_t)span * (size_t)N + col0;
+      if (counters) store_part<T, VEC>(dst, o);
+      else store_vec<T, VEC>(dst, o);
+    }
+  };
+  if (any_empty) {  // rows without an entry here are stored as zeros
+    const A zeros[VEC] = {};
+    for (int slot = group; slot < n_rows; slot += kGroups) {
+      const Range r = entries_of(s_rp[slot], s_rp[slot + 1]);
+      if (r.hi == r.lo) store_row(slot, zeros);
+    }
+  }
+
+  const int first = group * stretch;
+  bool open = first > 0 && first < n_nz && s_mark[first - 1] == 0;  // the row under way began in an earlier group
+  A acc[VEC], head[VEC];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) acc[v] = head[v] = (A)0;
+  int head_slot = -1;
+  const T *const from_b = B + (active ? col0 : 0);
+  const int stop = first + stretch;
+  struct Four { VecT b[4]; } even, odd;
+  auto request = [&](Four &four, int k) {
+    const int4 c = *reinterpret_cast<const int4 *>(&s_col[k]);
+    four.b[0] = load_vec<T, VEC>(from_b + (size_t)(unsigned)c.x * (size_t)(unsigned)N);
+    four.b[1] = load_vec<T, VEC>(from_b + (size_t)(unsigned)c.y * (size_t)(unsigned)N);
+    four.b[2] = load_vec<T, VEC>(from_b + (size_t)(unsigned)c.z * (size_t)(unsigned)N);
+    four.b[3] = load_vec<T, VEC>(from_b + (size_t)(unsigned)c.w * (size_t)(unsigned)N);
+  };
+  auto add = [&](const Four &four, int k) {
+    const unsigned long long marks = *reinterpret_cast<const unsigned long long *>(&s_mark[k]);
+    A a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[u] = (A)s_val[k + u];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) acc[v] += a[u] * (A)four.b[u].v[v];
+      const int mark = (int)(marks >> (16 * u)) & 0xffff;
+      if (mark) {
+        if (open) {
+          head_slot = mark - 1;
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) head[v] = acc[v];
+          open = false;
+        } else {
+          store_row(mark - 1, acc);
+        }
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) acc[v] = (A)0;
+      }
+    }
+  };
+  if (first < n_nz) {  // (a group that has nothing of its own asks for nothing)
+    request(even, first);
+    for (int k = first; k < stop; k += 8) {
+      if (k + 4 < stop) request(odd, k + 4);
+      add(even, k);
+      if (k + 4 < stop) {
+        if (k + 8 < stop) request(even, k + 8);
+        add(odd, k + 4);
+      }
+    }
+  }
+
+  // rows that more than one group has entries of
+  VecT last;
+#pragma unroll
+  for (int v = 0; v < VEC; ++v) last.v[v] = (T)acc[v];
+  s_last[tid] = last;
+  workgroup_lds_sync();
+  if (head_slot >= 0) {
+    A sum[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) sum[v] = (A)0;
+#pragma unroll 4
+    for (int j = entries_of(s_rp[head_slot], s_rp[head_slot + 1]).lo / stretch; j < group; ++j) {
+      const VecT part = s_last[j * LPR + t];
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) sum[v] += (A)part.v[v];
+    }
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) sum[v] += head[v];
+    store_row(head_slot, sum);
+  }
+
+  const int tail_begin = uniform(s_rp[n_rows]);
+  const bool carry_out = y1 > (tail_begin > y0 ? tail_begin : y0);
+  if (!counters) {
+    if (tid == 0 && blockIdx.y == 0) carry_row[span] = carry_out ? x1 : -1;
+    return;
+  }
+  const bool ends_cut_row = carry_in && n_rows > 0;
+  if (!ends_cut_row && !carry_out) return;
+  // the row's parts of all wavefronts are in memory when one of them takes the chunk's ticket
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  workgroup_lds_sync();
+  if (tid >= kWaveSize) return;
+  counters += 2 * (int64_t)blockIdx.y * chunks;
+  auto finish = [&](int row, int begin, int end, bool carry) {
+    finish_part<T, VEC, EPI>(row, begin, end, span, carry, items_per_chunk, kSnapItems, chunks, counters, N, col0,
+                             active && group == 0, carry_val, C, bias_v);
+  };
+  if (ends_cut_row) finish(x0, uniform(s_rp[0]), uniform(s_rp[1]), false);
+  if (carry_out) finish(x1, tail_begin, uniform(s_rp[n_rows + 1]), true);
+}
+
+
 // ---- narrow column tiles: one lane group per row --------------------------------------------
 // When a column tile is narrower than a wavefront's 64 lanes can cover with
 // full vectors, the wavefront is divided into G = 64 / LPR groups of LPR lanes
@@ -192,15 +412,16 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_merge_kernel(
 // nonzeros in the chunk would leave the other groups idle: such rows are summed
 // by all groups together (strided over its nonzeros, then combined with
 // shuffles in a fixed order).  Used when a row of B is at most 256 bytes (see
-// narrow_tile_bytes).
+// narrow_tile_bytes) and the product is a large one, bound by what it moves past the L2s: rows that lie
+// side by side are stored side by side, by one instruction, where spmm_grouped_kernel stores each when it ends (1 M nodes,
+// N = 31, 9 M entries: 309 against 326 us; N = 16 166 against 172).
 constexpr int kGroupRowMax = 24;  // longer in-chunk rows are shared by all groups
 
 template <typename T, int VEC, int LPR, int EPI>
-__global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
+__global__ __launch_bounds__(kBlockThreads) void spmm_row_groups_kernel(
     int M, int N, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
     const T *__restrict__ vals, const T *__restrict__ B, T *__restrict__ C,
-    const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int n_tiles,
-    int64_t blocks_per_tile, int *__restrict__ carry_row, T *__restrict__ carry_val,
+    const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int *__restrict__ carry_row, T *__restrict__ carry_val,
     const Boundary *__restrict__ bounds, SpmmBatch batch, int *__restrict__ counters) {
   using A = typename Acc<T>::type;
   using VecT = Vec<T, VEC>;
@@ -219,9 +440,8 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
   const int w = threadIdx.x / kWaveSize;
   const int g = lane / LPR;
   const int t = lane % LPR;
-  const TileMap where = map_workgroup(blockIdx.x, n_tiles, blocks_per_tile);
-  const int64_t span = where.block * kWavesPerBlock + w;
-  const int col0 = lane_column<VEC>((where.tile * LPR + t) * VEC, N);
+  const int64_t span = xcd_contiguous(blockIdx.x, gridDim.x) * kWavesPerBlock + w;
+  const int col0 = lane_column<VEC>(t * VEC, N);
   const bool active = col0 < N;
 
   const int64_t d0 = span * items_per_chunk;
@@ -328,12 +548,12 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_grouped_kernel(
         else store_vec<T, VEC>(dst, o);
       }
     }
-    if (!counters && live && slot == n_rows && where.tile == 0 && t == 0 && blockIdx.y == 0)
+    if (!counters && live && slot == n_rows && t == 0 && blockIdx.y == 0)
       carry_row[span] = len > 0 ? x1 : -1;
   }
   if (counters) {
     const int64_t chunks = (total_items + items_per_chunk - 1) >> __builtin_ctz(items_per_chunk);
-    counters += 2 * ((int64_t)blockIdx.y * n_tiles + where.tile) * chunks;
+    counters += 2 * (int64_t)blockIdx.y * chunks;
     auto finish = [&](int row, int begin, int end, bool carry) {
       finish_part<T, VEC, EPI>(row, begin, end, span, carry, items_per_chunk, snap, chunks, counters, N, col0, active && g == 0,
                                carry_val, C, bias_v);
@@ -386,9 +606,6 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_bounds_kernel(int M, int64
   bounds[c] = b;
 }
 
-inline size_t spmm_bounds_bytes(int64_t M, int64_t nnz, int64_t N, size_t elem) {
-  return (size_t)(spmm_split(M, nnz, N, elem).spans + 1) * sizeof(Boundary);
-}
 
 // Optional per-kernel timing: events recorded on the launch stream around each
 // of the two kernels.
@@ -455,27 +672,17 @@ int launch_spmm(int M, int N, int64_t nnz, const int *row_ptr, const int *col_id
   return SCORCH_HIP_OK;
 }
 
-// Narrow-tile variant: lane groups of LPR lanes, tiles of LPR * VEC columns, one
-// chunk per wavefront.  The fix-up does not care how the main kernel tiled the
+// Narrow-tile variant: lane groups of LPR lanes, one tile of LPR * VEC columns, a
+// chunk per workgroup or per wavefront.  The fix-up does not care how the main kernel tiled the
 // columns; it runs with scalar lanes over ceil(N / 64) tiles.
 template <typename T, int VEC, int LPR, int EPI>
 int launch_spmm_grouped(int M, int N, int64_t nnz, const int *row_ptr, const int *col_idx,
                         const T *vals, const T *B, const T *bias, T *C, void *workspace,
                         hipStream_t stream, const Boundary *bounds, int batch, int64_t K, int *counters,
                         int64_t counters_given) {
-  const int64_t total = (int64_t)M + nnz;
-  const int tile = LPR * VEC;
-  const int n_tiles = (N + tile - 1) / tile;
-  // as in spmm_split, with the real tile count: fill 8192 wavefront slots, at most 256 items each
-  const int64_t per_wave = total * n_tiles / 8192;
-  int ipc = kMinItemsPerWave;
-  while (ipc < kItemsPerWave && ipc * 2 <= per_wave) ipc *= 2;
-  const int wide_ipc = spmm_split(M, nnz, N, sizeof(T)).items_per_chunk;
-  if (ipc < wide_ipc) ipc = wide_ipc;  // never more carry records than the workspace holds
-  if (bounds && ipc != wide_ipc)
-    return fail(SCORCH_HIP_ERUNTIME, "SpMM: the chunk boundaries were built for %d items per chunk, not %d",
-                wide_ipc, ipc);
-  const int64_t spans = (total + ipc - 1) / ipc;
+  const bool by_workgroup = grouped_chunks(M, nnz, N, sizeof(T));
+  const SpmmSplit split = planned_split(M, nnz, N, sizeof(T));
+  const int64_t spans = split.spans;
   if (spans > spmm_num_chunks(M, nnz, N, sizeof(T)))
     return fail(SCORCH_HIP_ERUNTIME, "SpMM: %lld carry records exceed the workspace's %lld",
                 (long long)spans, (long long)spmm_num_chunks(M, nnz, N, sizeof(T)));
@@ -483,17 +690,21 @@ int launch_spmm_grouped(int M, int N, int64_t nnz, const int *row_ptr, const int
   T *carry_val = reinterpret_cast<T *>(
       static_cast<char *>(workspace) +
       align_up((size_t)spmm_num_chunks(M, nnz, N, sizeof(T)) * sizeof(int), 256));
-  const int64_t blocks_per_tile = round_up_8((spans + kWavesPerBlock - 1) / kWavesPerBlock);
-  if (blocks_per_tile * n_tiles > INT32_MAX)
-    return fail(SCORCH_HIP_EUNSUPPORTED, "SpMM: %lld workgroups exceed the launch limit",
-                (long long)(blocks_per_tile * n_tiles));
+  const int64_t blocks = round_up_8(by_workgroup ? spans : (spans + kWavesPerBlock - 1) / kWavesPerBlock);
+  if (blocks > INT32_MAX)
+    return fail(SCORCH_HIP_EUNSUPPORTED, "SpMM: %lld workgroups exceed the launch limit", (long long)blocks);
   mark_launch(stream);
   const SpmmBatch strides = {nnz, K * N, (int64_t)M * N, spans * N};
-  if (counters_given < 2 * (int64_t)batch * n_tiles * spans) counters = nullptr;  // the launch below folds the carries
-  spmm_grouped_kernel<T, VEC, LPR, EPI><<<dim3((unsigned)(blocks_per_tile * n_tiles), (unsigned)batch), kBlockThreads,
-                                          0, stream>>>(
-      M, N, row_ptr, col_idx, vals, B, C, bias, total, ipc, ipc < kSnapItems ? ipc : kSnapItems, n_tiles,
-      blocks_per_tile, carry_row, carry_val, bounds, strides, counters);
+  if (counters_given < 2 * (int64_t)batch * spans) counters = nullptr;  // the launch below folds the carries
+  const dim3 grid((unsigned)blocks, (unsigned)batch);
+  if (by_workgroup)
+    spmm_grouped_kernel<T, VEC, LPR, EPI><<<grid, kBlockThreads, 0, stream>>>(
+        M, N, row_ptr, col_idx, vals, B, C, bias, (int64_t)M + nnz, split.items_per_chunk, spans, carry_row, carry_val,
+        bounds, strides, counters);
+  else
+    spmm_row_groups_kernel<T, VEC, LPR, EPI><<<grid, kBlockThreads, 0, stream>>>(
+        M, N, row_ptr, col_idx, vals, B, C, bias, (int64_t)M + nnz, split.items_per_chunk, split.snap, carry_row,
+        carry_val, bounds, strides, counters);
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(stream);
   if (counters) return SCORCH_HIP_OK;
@@ -503,17 +714,6 @@ int launch_spmm_grouped(int M, int N, int64_t nnz, const int *row_ptr, const int
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(stream);
   return SCORCH_HIP_OK;
-}
-
-// Narrow tiles pay off when N is small: a row of B is at most 256 bytes, so
-// full-width tiles would leave lanes idle or fall back to 4-byte loads.  Returns the tile width in
-// bytes, or 0 for wide tiles.  (Tiling a wide B by columns so that K narrow rows
-// stay in one XCD's L2 was measured and lost: the workgroups resident on an XCD
-// span several tiles at once and evict each other's slices.)
-inline int narrow_tile_bytes(int64_t K, int64_t N, int64_t nnz, size_t elem) {
-  (void)K; (void)nnz;
-  const int64_t row_bytes = N * (int64_t)elem;
-  return row_bytes <= 256 ? (int)row_bytes : 0;
 }
 
 template <typename T, int EPI>
@@ -553,7 +753,7 @@ int spmm_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, con
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int m = (int)M, n = (int)N;
-  if (const int tile_bytes = timer ? 0 : narrow_tile_bytes(K, N, nnz, sizeof(T))) {
+  if (const int tile_bytes = timer ? 0 : narrow_tile_bytes(N, sizeof(T))) {
     const int vec = narrow_vec<T>(N);
     const int64_t lanes = (tile_bytes / (int)sizeof(T) + vec - 1) / vec;  // at most 16: 256 bytes in vectors of 16
 #define SCORCH_GROUPED(VEC, LPR) \
@@ -1063,7 +1263,7 @@ int scorch_hip_spmm_csr_bounds(int64_t M, int64_t nnz, int64_t N, size_t elem_si
   if (bounds_bytes < need)
     return scorch::fail(SCORCH_HIP_EWORKSPACE, "%s: %zu bytes needed for the boundaries, %zu given", fn, need,
                         bounds_bytes);
-  const scorch::SpmmSplit split = scorch::spmm_split(M, nnz, N, elem_size);
+  const scorch::SpmmSplit split = scorch::planned_split(M, nnz, N, elem_size);
   const int64_t num_bounds = split.spans + 1;
   scorch::spmm_bounds_kernel<<<dim3((unsigned)((num_bounds + scorch::kBlockThreads - 1) / scorch::kBlockThreads)),
                                scorch::kBlockThreads, 0, static_cast<hipStream_t>(stream)>>>(

@@ -236,6 +236,16 @@ __device__ __forceinline__ void finish_part(int row, int begin, int end, int64_t
   store_vec<T, VEC>(dst, o);
 }
 
+// Narrow tiles pay off when N is small: a row of B is at most 256 bytes, so
+// full-width tiles would leave lanes idle or fall back to 4-byte loads.  Returns the tile width in
+// bytes, or 0 for wide tiles.  (Tiling a wide B by columns so that K narrow rows
+// stay in one XCD's L2 was measured and lost: the workgroups resident on an XCD
+// span several tiles at once and evict each other's slices.)
+inline int narrow_tile_bytes(int64_t N, size_t elem) {
+  const int64_t row_bytes = N * (int64_t)elem;
+  return row_bytes <= 256 ? (int)row_bytes : 0;
+}
+
 inline SpmmSplit spmm_split(int64_t M, int64_t nnz, int64_t N, size_t elem) {
   const int64_t total = M + nnz;
   SpmmSplit sp;
@@ -248,6 +258,31 @@ inline SpmmSplit spmm_split(int64_t M, int64_t nnz, int64_t N, size_t elem) {
   sp.snap = sp.items_per_chunk < kSnapItems ? sp.items_per_chunk : kSnapItems;
   sp.spans = (total + sp.items_per_chunk - 1) / sp.items_per_chunk;
   return sp;
+}
+
+// Chunks of spmm_grouped_kernel, one to a workgroup: few enough to be resident at once, six workgroups to a
+// CU (20,000 nodes, 820 K items, N = 32: 2,000 chunks, which take two rounds, 15.0 us, 1,500 13.3), of 128
+// items at least (2,708 nodes, N = 16: 6.3 us, of 256 7.1) and 1,024 at most.
+constexpr int kGroupedItems = 1024, kGroupedItemsMin = 128;
+inline SpmmSplit grouped_split(int64_t M, int64_t nnz) {
+  const int64_t total = M + nnz, resident = 1536;
+  int64_t items = ((total + resident - 1) / resident + 31) / 32 * 32;
+  items = items < kGroupedItemsMin ? kGroupedItemsMin : items > kGroupedItems ? kGroupedItems : items;
+  return {(int)items, kSnapItems, (total + items - 1) / items};
+}
+// Where narrow rows are split that way.  Large products are bound by their traffic, of which the kernel with
+// a lane group per row makes less (see there); up to here the chain of reads counts (100,000 nodes of 3 + 1,
+// N = 16: 17.5 -> 13.2 us, of 12 + 1, N = 64: 54.9 -> 51.7; 300,000 of 6 + 1, 2.1 M items: N = 31 75.4 against 77.7).
+constexpr int64_t kGroupedMost = 2 << 20;  // merge items
+inline bool grouped_chunks(int64_t M, int64_t nnz, int64_t N, size_t elem) {
+  return narrow_tile_bytes(N, elem) && M + nnz <= kGroupedMost;
+}
+// The split whose boundaries a plan keeps for products with N columns.
+inline SpmmSplit planned_split(int64_t M, int64_t nnz, int64_t N, size_t elem) {
+  return grouped_chunks(M, nnz, N, elem) ? grouped_split(M, nnz) : spmm_split(M, nnz, N, elem);
+}
+inline size_t spmm_bounds_bytes(int64_t M, int64_t nnz, int64_t N, size_t elem) {
+  return (size_t)(planned_split(M, nnz, N, elem).spans + 1) * sizeof(Boundary);
 }
 
 // Carry records the workspace must hold: the most any kernel variant produces

@@ -272,6 +272,8 @@ int spmm_tiled_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nn
     split = resident;
     bounds = nullptr;
   }
+  // (boundaries kept for narrow rows may be those of other chunks)
+  if (grouped_chunks(M, nnz, N, sizeof(T))) bounds = nullptr;
   if (split.items_per_chunk + split.snap > kTiledSlots)
     return fail(SCORCH_HIP_ERUNTIME, "%s: chunks of %d + %d items exceed the %d staging slots", fn,
                 split.items_per_chunk, split.snap, kTiledSlots);

@@ -468,6 +468,38 @@ def test_direct_calls_on_a_large_square_like_the_references_perf_test():
     assert torch.allclose(out.cpu(), reference, atol=1e-3, rtol=1e-3)
 
 
+# every shape of a lane group, and rows whose last vector overlaps the one before
+@pytest.mark.parametrize("dtype, N", [(np.float32, n) for n in (1, 2, 3, 4, 7, 8, 16, 17, 31, 33, 37, 64)]
+                         + [(np.float64, n) for n in (1, 2, 5, 8, 15, 32)] + [(np.int32, 13), (np.int64, 9)])
+def test_narrow_rows_whose_ends_fall_anywhere_in_a_chunk(oracle, dtype, N):
+    """Chunks of a workgroup, walked in equal stretches by its lane groups: rows that end with a stretch, begin or end
+    inside one, span several groups or several chunks (up to 40: folded in two levels), and empty rows in front of, between and
+    behind them.  With boundaries from the plan and without, with the fold in the launch and behind it: the same bits."""
+    rng = np.random.default_rng(N)
+    ladder = [k for n in range(1, 70) for k in (n, 0)]
+    lens = np.array([0, 0, 5000] + ladder + [128, 64, 64, 63, 65, 1, 0, 0, 256, 31] + [4] * 300 + [700, 0, 3] + [1] * 500 + [129, 0], np.int64)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = rng.integers(0, 977, rp[-1]).astype(np.int32)
+    if np.dtype(dtype).kind == "i":
+        v, B = rng.integers(-9, 9, rp[-1]).astype(dtype), rng.integers(-99, 99, (977, N)).astype(dtype)
+    else:
+        v, B = rng.standard_normal(rp[-1]).astype(dtype), rng.standard_normal((977, N)).astype(dtype)
+    planned, unplanned = (hip_spmm(rp, ci, v, B, path=path) for path in ("merge", "merge_unplanned"))
+    assert np.array_equal(planned, unplanned)
+    if np.dtype(dtype).kind == "i":
+        np.testing.assert_array_equal(planned, oracle.spmm_csr_typed(rp, ci, v, B))
+    else:
+        assert oracle.rel_fro(planned, oracle.spmm_fp64(rp, ci, v, B)) <= (1e-6 if dtype is np.float32 else 1e-14)
+        if dtype is np.float32:
+            bias = rng.standard_normal(N).astype(np.float32)
+            np.testing.assert_array_equal(hip_spmm(rp, ci, v, B, bias=bias, relu=True, path="merge"),
+                                          np.maximum(planned + bias, 0))
+        # an infinity reaches the rows that refer to it and no others
+        B[0, N - 1] = np.inf
+        apart = ~np.isin(np.arange(len(lens)), np.repeat(np.arange(len(lens)), lens)[ci == 0])
+        assert np.array_equal(hip_spmm(rp, ci, v, B, path="merge")[apart], planned[apart])
+
+
 @pytest.mark.parametrize("M, K, N, per_row", [(1, 1, 1, 1), (3, 40, 33, 20), (17, 5000, 7, 100), (40, 10_239, 9, 300), (33, 1247, 64, 65),
                                              (70, 1300, 61, 64), (1040, 2500, 40, 30), (257, 200, 1000, 129)])
 @pytest.mark.parametrize("transposed", [0, 1])
