@@ -404,6 +404,40 @@ __device__ __forceinline__ void end_of_symbolic(int *counters, unsigned long lon
   counters[counter(3)] = 0;
 }
 
+// A thread's kScanPerThread consecutive elements, four to a request (one at a time, a wavefront's request touches 64 lines
+// for 256 bytes: the one-workgroup scan below took 21 us for 21,648 rows and 43 for 45,000); 0 beyond the end.
+__device__ __forceinline__ void load_run(const int *data, int64_t first, int64_t n, int (&v)[kScanPerThread]) {
+  if (first + kScanPerThread <= n) {
+#pragma unroll
+    for (int q = 0; q < kScanPerThread / 4; ++q) {
+      const Vec<int, 4> x = load_vec<int, 4>(data + first + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * q + e] = x.v[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < kScanPerThread; ++e) v[e] = first + e < n ? data[first + e] : 0;
+  }
+}
+// Their exclusive sums, starting from `running`.
+__device__ __forceinline__ void store_run(int *data, int64_t first, int64_t n, int running, const int (&v)[kScanPerThread]) {
+  int sums[kScanPerThread];
+#pragma unroll
+  for (int e = 0; e < kScanPerThread; ++e) {
+    sums[e] = running;
+    running += v[e];
+  }
+  if (first + kScanPerThread <= n) {
+#pragma unroll
+    for (int q = 0; q < kScanPerThread / 4; ++q)
+      store_vec<int, 4>(data + first + 4 * q, Vec<int, 4>{{sums[4 * q], sums[4 * q + 1], sums[4 * q + 2], sums[4 * q + 3]}});
+  } else {
+#pragma unroll
+    for (int e = 0; e < kScanPerThread; ++e)
+      if (first + e < n) data[first + e] = sums[e];
+  }
+}
+
 // (*grand_total also receives the sum of all counts in 64 bits: the row pointer is int32,
 // and a result of 2^31 entries or more must be reported, not wrapped)
 __global__ __launch_bounds__(kBlockThreads) void scan_tile_totals_kernel(const int *__restrict__ data,
@@ -412,12 +446,14 @@ __global__ __launch_bounds__(kBlockThreads) void scan_tile_totals_kernel(const i
                                                                          unsigned long long *__restrict__ grand_total) {
   __shared__ int s_scan[kWavesPerBlock + 1];
   const int64_t first = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
+  int v[kScanPerThread];
+  load_run(data, first, n, v);
   int mine = 0;
   long long wide = 0;
+#pragma unroll
   for (int e = 0; e < kScanPerThread; ++e) {
-    const int v = first + e < n ? data[first + e] : 0;
-    mine += v;
-    wide += v;
+    mine += v[e];
+    wide += v[e];
   }
   int total = 0;
   (void)block_exclusive_scan(mine, s_scan, total);
@@ -445,52 +481,50 @@ __global__ __launch_bounds__(kBlockThreads) void scan_spine_kernel(int *__restri
 }
 
 // (the last element, the total, becomes -1 when the 64-bit total does not fit an int32)
+// SPINE: `totals` has been through scan_spine_kernel; else a workgroup adds up the totals of the tiles before its own,
+// and the first one ends the symbolic pass.
+constexpr int64_t kScanOwnTotals = 4096;  // most tiles for that
+template <bool SPINE>
 __global__ __launch_bounds__(kBlockThreads) void scan_apply_kernel(int *__restrict__ data, int64_t n,
-                                                                   const int *__restrict__ totals,
-                                                                   const unsigned long long *__restrict__ grand_total) {
+                                                                   const int *__restrict__ totals, int *__restrict__ counters,
+                                                                   int64_t *__restrict__ report, int64_t sequence) {
   __shared__ int s_scan[kWavesPerBlock + 1];
+  const unsigned long long grand_total = *reinterpret_cast<const unsigned long long *>(counters + counter(6));
+  if (!SPINE && blockIdx.x == 0 && threadIdx.x == 0) end_of_symbolic(counters, grand_total, report, sequence);
   const int64_t first = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
   int v[kScanPerThread];
-  int mine = 0;
-  for (int e = 0; e < kScanPerThread; ++e) {
-    v[e] = first + e < n ? data[first + e] : 0;
-    mine += v[e];
+  load_run(data, first, n, v);
+  int mine = 0, total = 0, before = 0;
+#pragma unroll
+  for (int e = 0; e < kScanPerThread; ++e) mine += v[e];
+  if (SPINE) {
+    before = totals[blockIdx.x];
+  } else {
+    int part = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kBlockThreads) part += totals[i];
+    (void)block_exclusive_scan(part, s_scan, before);
   }
-  int total = 0;
-  int running = totals[blockIdx.x] + block_exclusive_scan(mine, s_scan, total);
-  for (int e = 0; e < kScanPerThread; ++e) {
-    if (first + e < n) data[first + e] = first + e == n - 1 && *grand_total > (unsigned long long)INT32_MAX ? -1 : running;
-    running += v[e];
-  }
+  const int running = before + block_exclusive_scan(mine, s_scan, total);
+  store_run(data, first, n, running, v);
+  if (first <= n - 1 && n - 1 < first + kScanPerThread && grand_total > (unsigned long long)INT32_MAX) data[n - 1] = -1;
 }
 
 // The same for few rows, in one workgroup and one launch.
-constexpr int kScanOneGroup = 65536;
 constexpr int kScanThreads = 1024;
+constexpr int kScanOneGroup = kScanThreads * kScanPerThread;  // one round (more rows: two launches of 4 us)
 __global__ __launch_bounds__(kScanThreads) void scan_one_group_kernel(int *__restrict__ data, int n, int *__restrict__ counters,
                                                                       int64_t *__restrict__ report, int64_t sequence) {
-  constexpr int kPer = 16;
   __shared__ int s_scan[kScanThreads / kWaveSize];
-  int carried = 0;
   unsigned long long wide = 0;
-  for (int base = 0; base < n; base += kScanThreads * kPer) {
-    const int first = base + (int)threadIdx.x * kPer;
-    int v[kPer], mine = 0;
+  const int first = (int)threadIdx.x * kScanPerThread;
+  int v[kScanPerThread], mine = 0, total = 0;
+  load_run(data, first, n, v);
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      v[e] = first + e < n ? data[first + e] : 0;
-      mine += v[e];
-      wide += (unsigned)v[e];
-    }
-    int total = 0;
-    int running = carried + block_exclusive_scan_n<kScanThreads / kWaveSize>(mine, s_scan, total);
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      if (first + e < n) data[first + e] = running;
-      running += v[e];
-    }
-    carried += total;
+  for (int e = 0; e < kScanPerThread; ++e) {
+    mine += v[e];
+    wide += (unsigned)v[e];
   }
+  store_run(data, first, n, block_exclusive_scan_n<kScanThreads / kWaveSize>(mine, s_scan, total), v);
 #pragma unroll
   for (int off = kWaveSize / 2; off > 0; off >>= 1) {
     const unsigned lo = (unsigned)__shfl_xor((int)(unsigned)wide, off), hi = (unsigned)__shfl_xor((int)(unsigned)(wide >> 32), off);
@@ -643,8 +677,8 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bounds_kernel(
     const int r = s_very_long[i];
     long long part = 0;
     const int hi = a_pos[r + 1];
-    for (int p = a_pos[r] + (int)threadIdx.x; p < hi; p += 8 * kBlockThreads)
-      part += products_of_entries<8>(p, kBlockThreads, hi, a_crd, b_pos);
+    for (int p = a_pos[r] + (int)threadIdx.x; p < hi; p += 16 * kBlockThreads)
+      part += products_of_entries<16>(p, kBlockThreads, hi, a_crd, b_pos);
 #pragma unroll
     for (int off = kWaveSize / 2; off > 0; off >>= 1) part += __shfl_xor(part, off);
     __syncthreads();
@@ -1624,9 +1658,11 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
 // For products of up to kNarrowColumns columns whose two passes share what they find out.
 constexpr int kBinThreads = kBinEntries;
 constexpr int kBinProducts = 4 * kBinThreads;  // to a window
-constexpr int kBinShare = 4 * kBinProducts;    // products of a batch of entries to a workgroup
+constexpr int kBinShare = 4 * kBinProducts;    // products of a batch of entries to a workgroup, where there are many
+constexpr int64_t kBinManyProducts = (int64_t)512 * kBinShare;
 constexpr int kBinColumns = 8192;              // most columns to a range; a power of two
-constexpr int kMaxBins = kNarrowColumns / kBinColumns;
+constexpr int kMaxBins = 32;
+static_assert(kMaxBins * kBinColumns >= kNarrowColumns, "the widest B in ranges of the most columns");
 constexpr int64_t kBinBudget = (int64_t)4 << 30;
 
 struct BinWindow {
@@ -1642,6 +1678,7 @@ struct BinItem {
 
 struct Bins {
   int shift = 0, n = 0;                 // ranges of 2^shift columns, n of them; n 0: not used
+  int share = kBinShare;                // products of a batch of entries to a workgroup
   int64_t rows = 0, items = 0;
   int *totals;                          // products, windows, items handed out to rows so far (counters of pass 0)
   BinRow *row;
@@ -1657,11 +1694,19 @@ struct Bins {
 inline Bins spgemm_bins(char *base, int *counters, int64_t N, size_t elem, int64_t rows, int64_t products, int64_t batches) {
   Bins b;
   if (rows == 0 || N > kNarrowColumns || products * (int64_t)(2 + elem) > kBinBudget || products > INT32_MAX / 2) return b;
-  b.shift = 10;  // eight ranges and more, for the sake of narrow matrices' hubs
-  while ((2 << b.shift) <= kBinColumns && (8 << b.shift) < N) ++b.shift;
+  // Narrow ranges while that makes workgroups the chip has room for, of 512 products and more (45,000 nodes of 11, ranges of
+  // 2,048 columns instead of 4,096: sums 29 -> 22 us, counts 21 -> 17; 131,072 nodes of 4, 49 such rows of few
+  // products, 4,096 instead of 8,192: 9 -> 12; of 17, 1,074 such rows: 117 -> 186).
+  b.shift = 10;
+  const auto ranges = [&](int shift) { return rows * ((N + (1 << shift) - 1) >> shift); };
+  while ((2 << b.shift) <= kBinColumns &&
+         ((kMaxBins << b.shift) < N || ranges(b.shift) > 4096 || ranges(b.shift) * 512 > products))
+    ++b.shift;
   b.n = (int)((N + (1 << b.shift) - 1) >> b.shift);
   b.rows = rows;
-  b.items = batches + products / kBinShare;
+  // (21,648 rows of 7: 120 workgroups that make four windows one after the other 18 us, of one window each 8.4)
+  if (products < kBinManyProducts) b.share = kBinProducts;
+  b.items = batches + products / b.share;
   size_t off = 0;
   auto take = [&](size_t bytes) { char *p = base ? base + off : nullptr; off += (bytes + 255) / 256 * 256; return p; };
   b.totals = counters ? counters + counter(16) : nullptr;
@@ -1691,7 +1736,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bin_rows_kernel(int M, B
     r.row = huge_row(huge_rows, M, counters[counter(5)], (int)i);
     p = products[r.row];
     r.batches = (a_pos[r.row + 1] - a_pos[r.row] + kBinEntries - 1) / kBinEntries;
-    r.items = r.batches + p / kBinShare;  // at most
+    r.items = r.batches + p / bins.share;  // at most
   }
   const int want[3] = {p, mine ? p / kBinProducts + r.batches : 0, r.items};
   int at[3];
@@ -1712,7 +1757,7 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bin_rows_kernel(int M, B
 }
 
 // A row's work items: a wavefront to a batch of entries.
-constexpr int kBinItemThreads = 512;
+constexpr int kBinItemThreads = 1024;  // (a row of 50,000 entries is what the launch waits for)
 __global__ __launch_bounds__(kBinItemThreads) void spgemm_bin_items_kernel(Bins bins, const int *__restrict__ a_pos,
                                                                            const int *__restrict__ a_crd,
                                                                            const int *__restrict__ b_pos) {
@@ -1735,7 +1780,7 @@ __global__ __launch_bounds__(kBinItemThreads) void spgemm_bin_items_kernel(Bins 
       if (at[i] >= 0) total += b_pos[at[i] + 1] - b_pos[at[i]];
 #pragma unroll
     for (int off = kWaveSize / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
-    const int shares = 1 + total / kBinShare;
+    const int shares = 1 + total / bins.share;
     int first = 0;
     if (lane == 0) first = atomicAdd(&s_items, shares);
     first = r.first_item + uniform(first);
@@ -2164,9 +2209,13 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
     const unsigned tiles = (unsigned)((n + kScanTile - 1) / kScanTile);
     scan_tile_totals_kernel<<<tiles, kBlockThreads, 0, stream>>>(c_pos, n, ws.scan_totals, grand_total);
     SCORCH_HIP_CHECK(hipGetLastError());
-    scan_spine_kernel<<<1, kBlockThreads, 0, stream>>>(ws.scan_totals, tiles, ws.counters, report, sequence);
-    SCORCH_HIP_CHECK(hipGetLastError());
-    scan_apply_kernel<<<tiles, kBlockThreads, 0, stream>>>(c_pos, n, ws.scan_totals, grand_total);
+    if (tiles <= kScanOwnTotals) {
+      scan_apply_kernel<false><<<tiles, kBlockThreads, 0, stream>>>(c_pos, n, ws.scan_totals, ws.counters, report, sequence);
+    } else {
+      scan_spine_kernel<<<1, kBlockThreads, 0, stream>>>(ws.scan_totals, tiles, ws.counters, report, sequence);
+      SCORCH_HIP_CHECK(hipGetLastError());
+      scan_apply_kernel<true><<<tiles, kBlockThreads, 0, stream>>>(c_pos, n, ws.scan_totals, ws.counters, report, sequence);
+    }
     SCORCH_HIP_CHECK(hipGetLastError());
   }
   return SCORCH_HIP_OK;

@@ -494,3 +494,30 @@ def test_without_memory_for_the_sorted_products_the_long_rows_go_the_other_way(o
     monkeypatch.setattr(H, "_empty", without_memory)
     other_rp, other_ci, _ = check(oracle, arp, aci, av, brp, bci, bv, N)
     assert len(refused) == 1 and np.array_equal(rp, other_rp) and np.array_equal(ci, other_ci)
+
+
+@pytest.mark.parametrize("M", [15, 16, 17, 4096, 16_382, 16_383, 16_384, 20_479, 20_480, 65_537])
+def test_row_pointers_on_either_side_of_a_scans_tiles(oracle, M):
+    """The result's row pointer has M + 1 elements: one workgroup sums up to 16,384 of them, tiles of 4,096 and a second
+    launch the rest; a thread takes sixteen, four to a request, the last ones one at a time."""
+    rng = np.random.default_rng(M)
+    lens = rng.integers(0, 3, M)
+    arp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    aci = np.concatenate([np.sort(rng.choice(50, n, replace=False)) for n in lens if n]).astype(np.int32)
+    brp, bci, bv = random_csr(rng, 50, 70, 0.1, empty_rows=(0, 49))
+    check(oracle, arp, aci, rng.integers(-9, 9, aci.size).astype(np.int64), brp, bci, rng.integers(-9, 9, bci.size).astype(np.int64), 70)
+
+
+@pytest.mark.parametrize("hubs, hub, N", [(1, 9000, 9000), (4, 3000, 20_000), (40, 1200, 60_000), (300, 300, 131_072)])
+def test_ranges_of_columns_of_every_width(oracle, hubs, hub, N):
+    """Few long rows of many products take narrow ranges of columns and a window to a work item, many long rows wide ranges."""
+    rng = np.random.default_rng(N)
+    K = 9000
+    blens = rng.integers(0, 40, K)
+    brp = np.concatenate([[0], np.cumsum(blens)]).astype(np.int32)
+    bci = np.concatenate([np.sort(rng.choice(N, n, replace=False)) for n in blens if n]).astype(np.int32)
+    lens = np.concatenate([np.full(hubs, hub), rng.integers(0, 5, 200)])
+    rng.shuffle(lens)
+    arp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    aci = np.concatenate([np.sort(rng.choice(K, n, replace=False)) for n in lens if n]).astype(np.int32)
+    check(oracle, arp, aci, rng.uniform(-1, 1, aci.size).astype(np.float32), brp, bci, rng.uniform(-1, 1, bci.size).astype(np.float32), N)
