@@ -388,6 +388,326 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
   }
 }
 
+// ---- masks whose blocks are live in part: sixteen queries to a team of wavefronts ---------------------------------------
+// A sliding window leaves a third of the 16-key tiles of its blocks dead, and different ones to every sixteen queries: the
+// kernel above skips them, but its four wavefronts meet at two barriers per key block and wait for whichever has most
+// tiles; and a launch of a few hundred workgroups leaves most of the chip's SIMDs with one wavefront's chain.  Here
+// sixteen queries have a list of the tiles that are live for them, which up to four wavefronts take in turn: no tile
+// of K or V goes through LDS, no barrier until the end, when they put their sums together.  K and V are read
+// four times as often, out of the L2s (8 KB for a tile's 32 matrix instructions, 1,024 clocks: 32 bytes a
+// clock and CU), the next tile's while one is computed.
+//
+// Features are numbered for the second product so that a lane's four V operands are one 16-byte piece of a row: tile
+// dt = VW h + v holds features 16 VW h + VW i + v, i = 0 .. 15.
+//
+// SPLIT wavefronts take the tiles of sixteen queries in turn; a workgroup of four has 4 / SPLIT times sixteen.
+//
+// Bound: a wavefront's chain of reads (work item, block, mask words, K: about 4 us of launches of 6 to 20), then a SIMD's matrix
+// and vector instructions, which hardly overlap: 1,024 and about 400 clocks a tile.  See team_wavefronts for what it takes.
+template <int D, int SPLIT>
+__global__ __launch_bounds__(kBlockThreads)
+__attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kernel(
+    int S, int n_blocks, int n_heads, const int *__restrict__ block_row_ptr,
+    const int *__restrict__ block_col_idx, const int *__restrict__ block_mask_index,
+    const unsigned long long *__restrict__ block_masks,
+    const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float scale_log2e,
+    float *__restrict__ O, int n_items, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
+  constexpr int kQueries = 16, kTeams = kWavesPerBlock / SPLIT;  // queries to a team of SPLIT wavefronts; teams
+  constexpr int kSlabs = D / 16, kFeat = D / 16;
+  constexpr int VW = D == 32 ? 2 : 4, NH = kFeat / VW;
+  constexpr int kBlocksAtOnce = 16;                           // 64 tiles: one to a lane
+  constexpr int kStride = D + 4;
+  constexpr int kOthers = SPLIT > 1 ? SPLIT - 1 : 1;
+  __shared__ unsigned long long s_words[kTeams][kBlocksAtOnce][kQueries];
+  __shared__ int s_col[kBlocksAtOnce];
+  __shared__ __attribute__((aligned(16))) float s_sums[SPLIT > 1 ? kTeams : 1][kOthers][SPLIT > 1 ? kQueries : 1][kStride];
+  __shared__ unsigned s_flags[SPLIT > 1 ? kTeams : 1][kOthers][3][kWaveSize];
+
+  const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), w = uniform(tid / kWaveSize);
+  const int team = w / SPLIT, part = w % SPLIT;
+  const int g = lane >> 4, n = lane & 15;
+  int head, rank;
+  const int ranks = n_items * SPLIT;
+  if (n_heads % 8 == 0) {  // a head's workgroups on one XCD, as above
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    head = xcd + 8 * (slot / ranks);
+    rank = slot % ranks;
+  } else {
+    head = blockIdx.x / ranks;
+    rank = blockIdx.x % ranks;
+  }
+  const int sub = rank % SPLIT * kTeams + team;  // sixteen queries of the block row
+  int qb, kb_begin, kb_end, part_slot = -1;
+  if (items) {
+    const int4 item = items[rank / SPLIT];
+    qb = uniform(item.x);
+    kb_begin = uniform(item.y);
+    kb_end = uniform(item.z);
+    part_slot = uniform(item.w);
+  } else {
+    qb = n_blocks - 1 - rank / SPLIT;
+    kb_begin = block_row_ptr[qb];
+    kb_end = block_row_ptr[qb + 1];
+  }
+  const int first_query = qb * kBlock + sub * kQueries;
+  const size_t head_off = (size_t)head * (size_t)S * D;
+  const float *Kh = K + head_off, *Vh = V + head_off;
+  const int query = first_query + n < S ? first_query + n : S - 1;
+
+  floatx4 q_op[kSlabs];
+#pragma unroll
+  for (int j = 0; j < kSlabs; ++j) q_op[j] = *reinterpret_cast<const floatx4 *>(Q + head_off + (size_t)query * D + 16 * j + 4 * g);
+
+  floatx4 o_acc[kFeat];
+#pragma unroll
+  for (int dt = 0; dt < kFeat; ++dt) o_acc[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float m_run = kDead, l_run = 0.0f;
+  unsigned nan_at = 0, up_at = 0, down_at = 0;  // results (bit 4 dt + r) that a NaN or infinity in V belongs to
+  bool flagged = false;
+
+  floatx4 k_op[kSlabs];
+  float v_op[4][NH][VW];
+  unsigned long long live_tiles = 0;  // of the blocks at hand; a team's wavefronts take them in turn
+  int number = 0;
+  unsigned my_keys = 0;               // of tile `lane`: keys that some query of the sixteen attends to
+  auto next_tile = [&]() {            // -1: no more
+    while (live_tiles) {
+      const int at = __ffsll(live_tiles) - 1;
+      live_tiles &= live_tiles - 1;
+      if (number++ % SPLIT == part) return at;
+    }
+    return -1;
+  };
+  // Rows of K and V that none of the sixteen attends to are not read -- there may be none, or anything -- and zeros
+  // stand in: their requests go beyond the buffer (host: S * D * 4 < 2^31), which the hardware answers with
+  // zeros and no traffic, and without a branch.  `at`: 4 * block + tile.
+  constexpr int kNowhere = (int)0x80000000;
+  const __amdgpu_buffer_rsrc_t k_rows = __builtin_amdgcn_make_buffer_rsrc((void *)Kh, 0, S * D * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t v_rows = __builtin_amdgcn_make_buffer_rsrc((void *)Vh, 0, S * D * 4, 0x00020000);
+  const int k_lane = (n * D + 4 * g) * 4, v_lane = (4 * g * D + VW * n) * 4;
+  auto first_key_of = [&](int at) { return uniform(s_col[at >> 2]) * kBlock + 16 * (at & 3); };
+  auto keys_of = [&](int at) { return (unsigned)__builtin_amdgcn_readlane((int)my_keys, at); };
+  auto fetch_k = [&](int at) __attribute__((always_inline)) {
+    const int from = (keys_of(at) >> n) & 1u ? first_key_of(at) * (D * 4) + k_lane : kNowhere;
+#pragma unroll
+    for (int j = 0; j < kSlabs; ++j)
+      k_op[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(k_rows, from + 64 * j, 0, 0));
+  };
+  auto fetch_v = [&](int at) __attribute__((always_inline)) {
+    const int from = first_key_of(at) * (D * 4) + v_lane;
+    const unsigned keys = keys_of(at) >> (4 * g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = (keys >> r) & 1u ? from + r * (D * 4) : kNowhere;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        Vec<float, VW> x;
+        if constexpr (VW == 4)
+          x = __builtin_bit_cast(Vec<float, VW>, __builtin_amdgcn_raw_buffer_load_b128(v_rows, row + 64 * VW * h, 0, 0));
+        else
+          x = __builtin_bit_cast(Vec<float, VW>, __builtin_amdgcn_raw_buffer_load_b64(v_rows, row + 64 * VW * h, 0, 0));
+#pragma unroll
+        for (int v = 0; v < VW; ++v) v_op[r][h][v] = x.v[v];
+      }
+    }
+  };
+  // One tile, whose rows of K have been requested; `next`: the one whose rows are, as soon as these have been used.
+  auto compute = [&](int at, int next) __attribute__((always_inline)) {
+    fetch_v(at);
+    const int block = at >> 2, t = at & 3;
+    const unsigned half = reinterpret_cast<const unsigned *>(&s_words[team][block][n])[t >> 1];  // keys 32 (t / 2) ..
+    const unsigned live = half >> (16 * (t & 1) + 4 * g);
+    floatx4 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < kSlabs; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) st = __builtin_amdgcn_mfma_f32_16x16x4f32(k_op[j][c], q_op[j][c], st, 0, 0, 0);
+    if (next >= 0) fetch_k(next);
+    const bool partly = !__all((live & 0xfu) == 0xfu);
+    if (partly) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[r] = (live >> r) & 1u ? st[r] : kDead;
+    }
+    const float mx = fmaxf(fmaxf(st[0], st[1]), fmaxf(st[2], st[3]));
+    if (__any(mx > m_run)) {
+      const float m_new = fmaxf(m_run, combine_query_lanes(mx, [](float a, float b) { return fmaxf(a, b); }));
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kFeat; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o_acc[dt][r] *= alpha;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) st[r] = __builtin_amdgcn_exp2f(st[r] - m_run);
+    if (partly) {  // (a query without a live key so far has kDead for its maximum: its dead keys are set to 0)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[r] = (live >> r) & 1u ? st[r] : 0.0f;
+    }
+    l_run += (st[0] + st[1]) + (st[2] + st[3]);
+    if (partly) {  // a NaN or infinity in V belongs to the queries that attend to its key (see the file's head)
+      float sum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+          for (int v = 0; v < VW; v += 2) sum = fmaf(v_op[r][h][v], v_op[r][h][v + 1], sum);
+      if (__any(!(fabsf(sum) < __builtin_inff()))) {
+        flagged = true;
+        const unsigned row = (unsigned)(s_words[team][block][n] >> (16 * t)) & 0xffffu;
+#pragma unroll 1
+        for (int key = 0; key < 16; ++key) {
+          if (!((row >> key) & 1u)) continue;
+          const float *from = Vh + (size_t)(first_key_of(at) + key) * D;
+#pragma unroll 1
+          for (int i = 0; i < 4 * kFeat; ++i) {
+            const int dt = i / 4, r = i % 4;
+            const float x = from[16 * VW * (dt / VW) + VW * (4 * g + r) + dt % VW];
+            if (fabsf(x) < __builtin_inff()) continue;
+            const unsigned bit = 1u << i;
+            up_at |= x > 0.0f ? bit : 0u;
+            down_at |= x < 0.0f ? bit : 0u;
+            nan_at |= x > 0.0f || x < 0.0f ? 0u : bit;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int v = 0; v < VW; ++v) v_op[r][h][v] = fabsf(v_op[r][h][v]) < __builtin_inff() ? v_op[r][h][v] : 0.0f;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int v = 0; v < VW; ++v)
+          o_acc[h * VW + v] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_op[r][h][v], st[r], o_acc[h * VW + v], 0, 0, 0);
+  };
+
+  for (int base = kb_begin; base < kb_end; base += kBlocksAtOnce) {  // uniform over the workgroup
+    if (base > kb_begin) __syncthreads();  // everyone is done with the words before
+    {
+      const int i = tid / kQueries, it = base + i;
+      unsigned long long word[kTeams];
+#pragma unroll
+      for (int p = 0; p < kTeams; ++p) word[p] = 0;
+      if (it < kb_end) {
+        const int mask_at = block_mask_index ? block_mask_index[it] : -1;
+        if (tid % kQueries == 0) s_col[i] = block_col_idx[it];
+        const unsigned long long *words = block_masks + (size_t)mask_at * kBlock + rank % SPLIT * kTeams * kQueries + tid % kQueries;
+#pragma unroll
+        for (int p = 0; p < kTeams; ++p) word[p] = mask_at >= 0 ? words[p * kQueries] : ~0ull;
+      }
+#pragma unroll
+      for (int p = 0; p < kTeams; ++p) s_words[p][i][tid % kQueries] = word[p];
+    }
+    __syncthreads();
+    unsigned long long any = 0;
+#pragma unroll
+    for (int i = 0; i < kQueries; ++i) any |= s_words[team][lane >> 2][i];
+    my_keys = (unsigned)(any >> (16 * (lane & 3))) & 0xffffu;
+    live_tiles = __ballot(my_keys != 0);
+    if (base == kb_begin)
+#pragma unroll
+      for (int j = 0; j < kSlabs; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) q_op[j][c] *= scale_log2e;
+    int at = next_tile();
+    if (at >= 0) fetch_k(at);
+    while (at >= 0) {
+      const int next = next_tile();
+      compute(at, next);
+      at = next;
+    }
+  }
+
+  float l = combine_query_lanes(l_run, [](float a, float b) { return a + b; });
+  if constexpr (SPLIT > 1) {
+    if (part > 0) {
+      float *mine = s_sums[team][part - 1][n];
+#pragma unroll
+      for (int dt = 0; dt < kFeat; ++dt) *reinterpret_cast<floatx4 *>(mine + 16 * dt + 4 * g) = o_acc[dt];
+      if (g == 0) {
+        mine[D] = m_run;
+        mine[D + 1] = l;
+      }
+      s_flags[team][part - 1][0][lane] = nan_at;
+      s_flags[team][part - 1][1][lane] = up_at;
+      s_flags[team][part - 1][2][lane] = down_at;
+    }
+    flagged = __syncthreads_or(flagged);
+    if (part > 0) return;
+    float m_all = m_run;
+#pragma unroll
+    for (int p = 0; p < kOthers; ++p) m_all = fmaxf(m_all, s_sums[team][p][n][D]);
+    const float own = __builtin_amdgcn_exp2f(m_run - m_all);
+    m_run = m_all;
+    l *= own;
+#pragma unroll
+    for (int dt = 0; dt < kFeat; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o_acc[dt][r] *= own;
+#pragma unroll
+    for (int p = 0; p < kOthers; ++p) {
+      const float *theirs = s_sums[team][p][n];
+      const float weight = __builtin_amdgcn_exp2f(theirs[D] - m_all);
+      l += weight * theirs[D + 1];
+#pragma unroll
+      for (int dt = 0; dt < kFeat; ++dt) {
+        const floatx4 o = *reinterpret_cast<const floatx4 *>(theirs + 16 * dt + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o_acc[dt][r] += weight * o[r];
+      }
+    }
+    if (flagged) {
+#pragma unroll
+      for (int p = 0; p < kOthers; ++p) {
+        nan_at |= s_flags[team][p][0][lane];
+        up_at |= s_flags[team][p][1][lane];
+        down_at |= s_flags[team][p][2][lane];
+      }
+    }
+  }
+  if (flagged) {
+#pragma unroll
+    for (int dt = 0; dt < kFeat; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const unsigned bit = 1u << (4 * dt + r);
+        if ((nan_at & bit) || ((up_at & bit) && (down_at & bit))) o_acc[dt][r] = __builtin_nanf("");
+        else if (up_at & bit) o_acc[dt][r] += __builtin_inff();
+        else if (down_at & bit) o_acc[dt][r] -= __builtin_inff();
+      }
+  }
+  float inv = 1.0f;
+  float *out;
+  if (part_slot >= 0) {
+    out = partials + (((size_t)head * n_slots + part_slot) * kBlock + (sub * kQueries + n)) * (D + 4);
+    if (g == 0) {
+      out[D] = m_run;
+      out[D + 1] = l;
+    }
+  } else {
+    if (first_query + n >= S) return;
+    inv = l > 0.0f ? 1.0f / l : 0.0f;  // queries without a live key give zeros
+    out = O + head_off + (size_t)query * D;
+  }
+#pragma unroll
+  for (int h = 0; h < NH; ++h)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      Vec<float, VW> o;
+#pragma unroll
+      for (int v = 0; v < VW; ++v) o.v[v] = o_acc[h * VW + v][r] * inv;
+      *reinterpret_cast<Vec<float, VW> *>(out + 16 * VW * h + VW * (4 * g + r)) = o;
+    }
+}
+
 // Combines the stretches of a block row that was shared out: with m* the largest of the
 // stretches' reference maxima, O = sum_p 2^(m_p - m*) O_p / sum_p 2^(m_p - m*) l_p.
 // One workgroup per (split row, head); thread t takes query t / 4 and a quarter of the features.
@@ -423,6 +743,22 @@ __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, in
   *reinterpret_cast<floatx4 *>(O + ((size_t)head * S + (size_t)row.x * kBlock + q) * D + feature) = acc;
 }
 
+// Wavefronts to sixteen queries in attn_f32_tiles_kernel for masks whose blocks are live in part, 0: the other kernel.
+// As many as leave every workgroup a place at once (four to a CU, two for D = 128); what is longer than that goes best with one,
+// and with D = 32, whose tiles are half as long as the reads in front of them, by the other kernel.  Windows of 64 and a
+// global token, (tokens, heads, D, workgroups of a block row): the other kernel, 1, 2 and 4 wavefronts, us:
+//   (300, 4, 64, 20) 10.8, 11.1, 8.2, 6.6     (2,048, 4, 64, 176) 19.0, 18.5, 15.3, 13.4   (960, 16, 64, 288) 23.6, 22.8, 19.5, 19.5
+//   (3,001, 8, 64, 464) 24.6, 23.7, 23.1, 26.5   (2,048, 16, 64, 704) 31.8, 30.3, 30.4, 33.8   (8,192, 16, 64, 2,288) 92.6, 90.2, 92.1, 111
+//   (1,472, 8, 32, 224) 13.4, 14.0, 11.9, 11.0   (2,944, 12, 32, 684) 20.0, 22.3, 20.8, 24.0   (6,141, 16, 32, 1,904) 43.6, 44.4, 44.5, 51.0
+//   (7,744, 1, 128, 151) 30.8, 30.1, 23.8, 22.4   (2,048, 12, 128, 468) 45.0, 43.2, 45.9, 54.2   (4,992, 16, 128, 1,392) 130, 109, 113, 133
+// (Whole blocks: 13.5 for 15.9 at (1,024, 8, 64, 128), but 13.8 for 11.6 at (4,096, 1, 64, 254); they stay with the other kernel.)
+inline int team_wavefronts(int D, unsigned workgroups) {
+  const unsigned places = D == 128 ? 160 : 320;
+  if (workgroups <= places) return 4;
+  if (workgroups <= 2 * places - 64) return 2;
+  return D == 32 || workgroups > INT32_MAX / 4 ? 0 : 1;
+}
+
 template <int D>
 static int launch(dim3 grid, hipStream_t s, int S, int n_blocks, int H, const int32_t *block_row_ptr,
                   const int32_t *block_col_idx, const int32_t *block_mask_index,
@@ -430,9 +766,16 @@ static int launch(dim3 grid, hipStream_t s, int S, int n_blocks, int H, const in
                   const float *k, const float *v, float scale_log2e, float *o, int n_items, const int4 *items, int n_slots, float *partials,
                   int n_split_rows, const int4 *split_rows) {
   mark_launch(s);
-  auto kernel = block_mask_index ? &attn_f32_kernel<D, true> : &attn_f32_kernel<D, false>;
-  kernel<<<grid, kBlockThreads, 0, s>>>(S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index, block_masks,
-                                        block_cols, q, k, v, scale_log2e, o, n_items, items, n_slots, partials);
+  if (const int split = block_mask_index ? team_wavefronts(D, grid.x) : 0; split && (int64_t)S * D * 4 < INT32_MAX) {
+    auto kernel = split == 4 ? &attn_f32_tiles_kernel<D, 4> : split == 2 ? &attn_f32_tiles_kernel<D, 2> : &attn_f32_tiles_kernel<D, 1>;
+    kernel<<<dim3(grid.x * split), kBlockThreads, 0, s>>>(
+        S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index, block_masks, q, k, v, scale_log2e, o, n_items, items,
+        n_slots, partials);
+  } else {
+    auto kernel = block_mask_index ? &attn_f32_kernel<D, true> : &attn_f32_kernel<D, false>;
+    kernel<<<grid, kBlockThreads, 0, s>>>(S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index, block_masks,
+                                          block_cols, q, k, v, scale_log2e, o, n_items, items, n_slots, partials);
+  }
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(s);
   if (n_split_rows > 0) {

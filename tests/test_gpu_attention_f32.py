@@ -211,3 +211,33 @@ def test_a_non_finite_row_of_v_reaches_the_queries_that_attend_to_it_and_no_othe
     assert isinstance(rp._scorch_plan.attention, H.BlockMask)
     if S % 64 == 0:
         assert np.array_equal(H.sparse_attention_f32(dq, dk, dv, rp, ci, scale).cpu().numpy(), out, equal_nan=True)
+
+
+# seven block rows: 7 workgroups of a block row to a head, more with the global token's row in stretches
+@pytest.mark.parametrize("heads", [1, 24, 40, 50, 90])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_teams_of_four_two_and_one_wavefront_to_sixteen_queries(oracle, heads, D):
+    """Launches of more and more workgroups: the tiles of sixteen queries are shared out to fewer and fewer
+    wavefronts.  Sixteen queries without any key, sixteen with a single one, and a NaN that reaches one head's queries of key 99."""
+    S = 447
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = (abs(i - j) <= 40) | (i == 0) | (j == 0)
+    mask[160:192] = False
+    mask[176:192, 300] = True
+    rng = np.random.default_rng(heads + D)
+    q, k, v = (rng.standard_normal((heads, S, D)).astype(np.float32) for _ in range(3))
+    scale = D ** -0.5
+    ref = {h: oracle.attention_dense_fp64(q[h], k[h], v[h], mask, scale) for h in {0, heads // 2, heads - 1}}
+    v[heads - 1, 99, D - 1] = np.nan
+    rp, ci = (dev(x) for x in csr_of(mask))
+    dq, dk, dv = (dev(x) for x in (q, k, v))
+    for call in range(3):
+        out = H.sparse_attention_csr(rp, ci, dq, dk, dv, scale).cpu().numpy()
+    assert isinstance(rp._scorch_plan.attention, H.BlockMask)
+    reached = np.zeros((S, D), bool)
+    reached[mask[:, 99], D - 1] = True
+    for h, want in ref.items():
+        hit = reached if h == heads - 1 else np.zeros_like(reached)
+        assert np.isnan(out[h][hit]).all()
+        assert oracle.rel_fro(np.where(hit, 0, out[h]), np.where(hit, 0, want)) <= TOL
+        assert np.all(out[h, 160:176] == 0)
