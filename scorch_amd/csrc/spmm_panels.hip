@@ -7,20 +7,19 @@
 // its 8 bytes of A from the L2 and P * 4 bytes from LDS.  A panel of B is P columns, so a B that is
 // handed over as its transpose (the usual W @ x.T) is read where it lies, P rows of x at a time.
 //
-// A row is a wavefront's, P / 4 lanes to an entry with 16 bytes each.  The next entries, or the next row's
-// first, are on their way while those at hand are used: with four or eight lanes to an entry they
-// come one to a lane and go through a strip of LDS of the wavefront's own, from which the lanes that
-// share one read it (a load for every share fetches 32 bytes at a time: 88 -> 63 us for 8,192 rows of
-// 50, N = 1,024); with one or two lanes to an entry every lane loads what it uses, four or eight
-// entries at a time.  At the end of a row the partial sums are added up by exchanging halves: a
-// lane keeps two of its four columns, then one, so that the last steps move one value.
+// A row is a wavefront's, P / 4 lanes to an entry with 16 bytes each.  Its entries come one to a lane, one, two, four or
+// eight batches of 64 at a time, by buffer loads whose range is the batch (what lies beyond it costs no bounds check and
+// no traffic), and the lanes that share an entry get it by a move inside a quad that the address calculation carries.
+// The next batch, or the next row's first, is on its way while the one at hand is used.  (Through a strip of LDS for four
+// and eight lanes to an entry, and with a checked load for every share for one and two: 16.5 us for 13.2 with 1,024 x 4,096,
+// 205 k entries, N = 256, P = 8; 15.0 for 12.3 with 4,096 x 1,024, P = 32; 70 for 56 with 8,192 x 1,024, N = 1,024, P = 32;
+// 101 for 75 with 1,024 x 8,192, P = 4.)  At the end of a row the partial sums are added up by exchanging halves and then
+// rows of 16 lanes between registers: a lane keeps two of its four columns, then one; the last steps are rotations.
 //
-// The panel's LDS reads are at random rows, so the entries that one access serves fall on the
-// same banks now and then (1,024 x 4,096, 205 k entries, N = 256: 58 bytes a clock and CU at P = 8, 42 % of the
-// cycles conflicts; at P = 32 17 %); wider panels lose less to that and read A
-// less often, and they take more LDS per row of B.  The LDS is busy for half of a launch: the rest is
-// the panel's way into it, the entries' loads and the end of every row.  The host picks P and the number of row shares
-// from K, N and nnz.
+// The panel's LDS reads are at random rows, so the entries that one access serves fall on the same banks now and then;
+// wider panels lose less to that and read A less often, and they take more LDS per row of B.  A launch of 12 us is 2 us of
+// panel on its way into LDS, 3 to 4 of LDS reads without conflicts, twice that with them, and the end of every row.
+// The host picks P and the number of row shares from K, N and nnz.
 #include <atomic>
 
 #include "spmm.hpp"
@@ -32,26 +31,48 @@ constexpr int kPanelLds = 160 * 1024;
 
 constexpr int kPanelWaves = kPanelThreads / kWaveSize;
 
+// x of the lane of each lane's group of LPE that holds the group's entry u mod LPE (u a constant once the caller's
+// loop is unrolled), by moves inside a quad, which the instruction that uses the value carries.  With eight lanes to an
+// entry, `low` holds the first four lanes' values in both quads of the group and `high` the last four's.
+template <int LPE>
+struct Shared {
+  int low, high;
+  Shared() = default;
+  __device__ __forceinline__ explicit Shared(int x) : low(x), high(x) {
+    if constexpr (LPE == 8) {
+      low = __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xa, false);   // row_shr:4 into the odd quads
+      high = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xf, 0x5, false);  // row_shl:4 into the even ones
+    }
+  }
+  __device__ __forceinline__ int of(int u) const {
+    if constexpr (LPE == 1) return low;
+    if constexpr (LPE == 2)
+      return u % 2 ? __builtin_amdgcn_update_dpp(0, low, 0xf5, 0xf, 0xf, true) : __builtin_amdgcn_update_dpp(0, low, 0xa0, 0xf, 0xf, true);
+    const int x = LPE == 8 && u % 8 >= 4 ? high : low;
+    switch (u % 4) {
+      case 0: return __builtin_amdgcn_update_dpp(0, x, 0x00, 0xf, 0xf, true);
+      case 1: return __builtin_amdgcn_update_dpp(0, x, 0x55, 0xf, 0xf, true);
+      case 2: return __builtin_amdgcn_update_dpp(0, x, 0xaa, 0xf, 0xf, true);
+      default: return __builtin_amdgcn_update_dpp(0, x, 0xff, 0xf, 0xf, true);
+    }
+  }
+};
+
 template <int P, int R>
 __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
     int M, int K, int N, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
     const float *__restrict__ vals, const float *__restrict__ B, int transposed, const float *__restrict__ bias,
     int relu, float *__restrict__ C, int n_panels, int shares, int rows_per_share) {
   constexpr int LPE = P / 4;              // lanes to an entry
-  constexpr int SLOTS = kWaveSize / LPE;  // entries a wavefront takes at once
-  constexpr bool STAGED = LPE >= 4;
-  constexpr int APART = STAGED ? kWaveSize : SLOTS;  // a lane's R entries
-  constexpr int BATCH = R * APART;
-  constexpr int STEPS = BATCH / SLOTS;
-  extern __shared__ float4 s_panel[];     // [K + 1][LPE], row K is zero; then the wavefronts' strips
-  int2 *strip = reinterpret_cast<int2 *>(s_panel + (size_t)(K + 1) * LPE) + (threadIdx.x / kWaveSize) * 2 * BATCH;
+  constexpr int BATCH = R * kWaveSize;    // entries at hand: R to a lane
+  extern __shared__ float4 s_panel[];     // [K + 1][LPE], row K is zero
 
   const int id = (int)xcd_contiguous(blockIdx.x, gridDim.x);
   const int panel = id / shares, share = id % shares;
   if (panel >= n_panels) return;
   const int n0 = panel * P;
   const int row_end = min(M, (share + 1) * rows_per_share);
-  const int lane = wave_lane(), slot = lane / LPE, part = lane % LPE;
+  const int lane = wave_lane(), part = lane % LPE;
 
   // The wavefront's rows are first, first + 16, ...; lane i holds the i-th's pointers, 64 rows at a time.
   int row = uniform(share * rows_per_share + (int)threadIdx.x / kWaveSize);
@@ -63,13 +84,15 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
   };
   int c[R];
   float a[R];
-  auto load_entries = [&](int first, int end) {
+  auto load_entries = [&](int first, int end) {  // (loads beyond the row's end give zeros)
+    first = uniform(first);
+    const int bytes = uniform(max(min(end - first, BATCH), 0) * 4);
+    const __amdgpu_buffer_rsrc_t columns = __builtin_amdgcn_make_buffer_rsrc((void *)(col_idx + first), 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t values = __builtin_amdgcn_make_buffer_rsrc((void *)(vals + first), 0, bytes, 0x00020000);
 #pragma unroll
     for (int e = 0; e < R; ++e) {
-      const int p = first + (STAGED ? lane : slot) + e * APART;
-      const bool ok = p < end;
-      c[e] = ok ? col_idx[p] : K;
-      a[e] = ok ? vals[p] : 0.0f;
+      c[e] = __builtin_amdgcn_raw_buffer_load_b32(columns, (e * kWaveSize + lane) * 4, 0, 0);
+      a[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(values, (e * kWaveSize + lane) * 4, 0, 0));
     }
   };
   hold(row);
@@ -95,35 +118,43 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
           s_panel[k * LPE + l] = make_float4(v[i][4 * l], v[i][4 * l + 1], v[i][4 * l + 2], v[i][4 * l + 3]);
       }
     }
-  } else {
-    for (int i = threadIdx.x; i < K * LPE; i += kPanelThreads) {
-      const int k = i / LPE, col = n0 + i % LPE * 4;
-      const float *from = B + (size_t)k * (size_t)N + col;
-      float4 x = make_float4(0, 0, 0, 0);
-      if (col + 4 <= N) {
-        const Vec<float, 4> v = load_vec<float, 4>(from);
-        x = make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
-      } else {
-        if (col < N) x.x = from[0];
-        if (col + 1 < N) x.y = from[1];
-        if (col + 2 < N) x.z = from[2];
+  } else if (N >= 4) {
+    constexpr int AHEAD = 8, ROWS = kPanelThreads / LPE;
+    const int l = threadIdx.x % LPE, col = n0 + 4 * l;
+    const int from = min(col, N - 4), beyond = col - from;  // the last columns are loaded with those in front of them
+    for (int k0 = threadIdx.x / LPE; k0 < K; k0 += AHEAD * ROWS) {
+      Vec<float, 4> x[AHEAD];
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) x[j] = load_vec<float, 4>(B + (size_t)min(k0 + j * ROWS, K - 1) * (size_t)N + from);
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        float4 y = make_float4(x[j].v[0], x[j].v[1], x[j].v[2], x[j].v[3]);
+        if (beyond & 1) y = make_float4(y.y, y.z, y.w, 0);
+        if (beyond & 2) y = make_float4(y.z, y.w, 0, 0);
+        if (beyond >= 4) y = make_float4(0, 0, 0, 0);
+        s_panel[min(k0 + j * ROWS, K - 1) * LPE + l] = y;
       }
-      s_panel[i] = x;
+    }
+  } else {
+    for (int k = threadIdx.x; k < K; k += kPanelThreads) {
+      const float *row_of_B = B + (size_t)k * (size_t)N;
+      s_panel[k * LPE] = make_float4(row_of_B[0], N > 1 ? row_of_B[1] : 0.0f, N > 2 ? row_of_B[2] : 0.0f, 0);
+#pragma unroll
+      for (int l = 1; l < LPE; ++l) s_panel[k * LPE + l] = make_float4(0, 0, 0, 0);
     }
   }
   if (threadIdx.x < LPE) s_panel[K * LPE + threadIdx.x] = make_float4(0, 0, 0, 0);
   __syncthreads();
 
   // (k: the first entry of the batch in c and a; begin, end: its row's)
-  int k = begin, buffer = 0;
+  int k = begin;
   float acc[4] = {0, 0, 0, 0};
   while (row < row_end) {
-    int cc[R];
-    float aa[R];
+    Shared<LPE> from[R], with[R];  // the byte an entry's row of the panel begins at, and its value
 #pragma unroll
     for (int e = 0; e < R; ++e) {
-      if constexpr (STAGED) strip[buffer * BATCH + e * kWaveSize + lane] = make_int2(c[e], __builtin_bit_cast(int, a[e]));
-      cc[e] = c[e], aa[e] = a[e];
+      from[e] = Shared<LPE>((e * kWaveSize + lane < end - k ? c[e] : K) * (P * 4));
+      with[e] = Shared<LPE>(__builtin_bit_cast(int, a[e]));
     }
     k += BATCH;
     const bool row_done = k >= end;
@@ -139,36 +170,42 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
       k = begin;
     }
     if (row < row_end) load_entries(k, end);
-    if constexpr (STAGED) wave_lds_sync();
+    constexpr int STEPS = R * LPE, AT_ONCE = STEPS < 4 ? STEPS : 4;  // LDS reads in flight
 #pragma unroll
-    for (int u = 0; u < STEPS; ++u) {
-      int col;
-      float v;
-      if constexpr (STAGED) {
-        const int2 entry = strip[buffer * BATCH + u * SLOTS + slot];
-        col = entry.x, v = __builtin_bit_cast(float, entry.y);
-      } else {
-        col = cc[u], v = aa[u];
+    for (int s0 = 0; s0 < STEPS; s0 += AT_ONCE) {
+      float4 b[AT_ONCE];
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int u = s0 + i;
+        b[i] = *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(s_panel) + from[u / LPE].of(u % LPE) + part * 16);
       }
-      const float4 b = s_panel[col * LPE + part];
-      acc[0] += v * b.x;
-      acc[1] += v * b.y;
-      acc[2] += v * b.z;
-      acc[3] += v * b.w;
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int u = s0 + i;
+        const float value = __builtin_bit_cast(float, with[u / LPE].of(u % LPE));
+        acc[0] += value * b[i].x;
+        acc[1] += value * b[i].y;
+        acc[2] += value * b[i].z;
+        acc[3] += value * b[i].w;
+      }
     }
-    buffer ^= 1;
     if (!row_done) continue;
-    // slots whose lowest bit is set keep columns 2 and 3 of their four; those with the next bit set the odd one of two
-    const bool upper = slot & 1, odd = slot & 2;
-    float two[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      two[j] = (upper ? acc[2 + j] : acc[j]) + __shfl_xor(upper ? acc[j] : acc[2 + j], LPE);
-    float sum = (odd ? two[1] : two[0]) + __shfl_xor(odd ? two[0] : two[1], 2 * LPE);
-#pragma unroll
-    for (int off = 4 * LPE; off < kWaveSize; off <<= 1) sum += __shfl_xor(sum, off);
-    const int col = n0 + part * 4 + (upper ? 2 : 0) + (odd ? 1 : 0);
-    if (slot < 4 && col < N) {
+    // The upper half of the wavefront keeps columns 2 and 3 of a lane's four, then odd rows of 16 lanes the odd one of two.
+    // (a's upper half changes places with b's lower one, then a's odd rows with b's even ones)
+    auto exchanged = [](float a, float b, auto swap) {
+      const auto r = swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b));
+      const unsigned x = r[0], y = r[1];
+      return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+    };
+    auto halves = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+    auto rows = [](unsigned a, unsigned b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
+    float sum = exchanged(exchanged(acc[0], acc[2], halves), exchanged(acc[1], acc[3], halves), rows);
+    sum += row_rotated<8>(sum);
+    if constexpr (LPE <= 4) sum += row_rotated<4>(sum);
+    if constexpr (LPE <= 2) sum += row_rotated<2>(sum);
+    if constexpr (LPE <= 1) sum += row_rotated<1>(sum);
+    const int col = n0 + part * 4 + lane / 32 * 2 + lane / 16 % 2;
+    if (lane % 16 < LPE && col < N) {
       if (bias) sum += bias[col];
       if (relu) sum = sum > 0.0f ? sum : 0.0f;
       C[(size_t)this_row * (size_t)N + col] = sum;
@@ -184,30 +221,31 @@ struct PanelShape {
   double us;     // estimated
 };
 
-inline int64_t panel_lds(int64_t K, int width, int in_flight) {
-  return (K + 1) * width * 4 + (width >= 16 ? kPanelWaves * 2 * kWaveSize * in_flight * 8 : 0);
-}
+inline int64_t panel_lds(int64_t K, int width) { return (K + 1) * width * 4; }
 
-// Panel width and row shares with the least estimated time: rounds of workgroups (one to a CU, or two of
-// half its LDS), each a panel's load at 24 bytes a clock and its share of the entries, in clocks each what
-// LDS takes for their pieces of B, and of the rows.
+// Panel width and row shares with the least estimated time: what the busiest CU has to do, a panel's load at 24 bytes a clock
+// and its share of the entries for each of its workgroups, in clocks each what LDS takes for their pieces of B, and of the
+// rows.  (Measured against the estimate, us: 1,024 x 4,096, 200 to a row, N = 256, P = 8 13.2 for 13.9; 7,989 x 3,994, 194,
+// N = 379, P = 8 113 for 115; 1,024 x 8,192, 400, N = 1,024, P = 4 75 for 81; 4,096 x 1,024, 49, N = 256, P = 32 12.3 for 11.5;
+// 465 x 1,863, 90, N = 167, P = 8 6.4 for 5.9.  The row kernel in its place: 17.0, 167, -, 17.0, 8.5; and at the line between the
+// two, 663 x 226, 48, N = 716 6.9 for 8.1, 1,448 x 517, 64, N = 244 6.4 for 7.9, 2,301 x 702, 64, N = 122 6.2 for 7.2.)
 inline PanelShape panel_shape(int64_t M, int64_t K, int64_t N, int64_t nnz) {
   PanelShape best = {0, 0, 0, 0};
   if (M <= 0 || N <= 0 || K > kPanelLds / 16) return best;
   const int64_t mean = (nnz + M - 1) / M;
   for (int width : {32, 16, 8, 4}) {
-    const int in_flight = width >= 16 ? 1 : width == 8 ? (mean > 192 ? 8 : 4) : mean > 256 ? 8 : mean > 128 ? 4 : 2;
-    const int64_t lds = panel_lds(K, width, in_flight);
+    const int in_flight = width >= 16 ? 1 : width == 8 ? (mean > 192 ? 4 : 2) : mean > 256 ? 8 : mean > 128 ? 4 : 2;
+    const int64_t lds = panel_lds(K, width);
     if (lds > kPanelLds) continue;
-    const int64_t batch = width >= 16 ? kWaveSize : kWaveSize / (width / 4) * in_flight;
-    const double per_entry = width == 32 ? 1.55 : width == 16 ? 1.1 : width == 8 ? 0.57 : 0.30;
+    const int64_t batch = kWaveSize * in_flight;
+    const double per_entry = width == 32 ? 1.2 : width == 16 ? 0.8 : width == 8 ? 0.47 : 0.25;
     const double work = (double)M * ((double)((mean + batch - 1) / batch * batch) * per_entry + 50);
-    const int64_t per_cu = lds <= kPanelLds / 2 ? 2 : 1, slots = 256 * per_cu, panels = (N + width - 1) / width;
+    const int64_t panels = (N + width - 1) / width;
     for (int64_t shares = 1; shares <= 512 && (shares == 1 || shares * kPanelWaves <= M); ++shares) {
-      const double rounds = (double)((panels * shares + slots - 1) / slots * per_cu);
+      const double rounds = (double)((panels * shares + 255) / 256);
       const double us = 2.5 + rounds * ((double)lds / 24 + work / (double)shares) / 2400;
       if (best.width == 0 || us < best.us) best = {width, in_flight, (int)shares, us};
-      if (panels * shares >= 4 * slots) break;
+      if (panels * shares >= 2048) break;
     }
   }
   return best;
@@ -229,7 +267,7 @@ int launch_panels(int64_t M, int64_t K, int64_t N, const int *row_ptr, const int
     allowed.fetch_or(bit, std::memory_order_release);
   }
   mark_launch(s);
-  spmm_panels_kernel<P, R><<<dim3((unsigned)grid), kPanelThreads, (size_t)panel_lds(K, P, R), s>>>(
+  spmm_panels_kernel<P, R><<<dim3((unsigned)grid), kPanelThreads, (size_t)panel_lds(K, P), s>>>(
       (int)M, (int)K, (int)N, row_ptr, col_idx, vals, B, transposed, bias, relu, C, (int)panels, shares,
       (int)((M + shares - 1) / shares));
   SCORCH_HIP_CHECK(hipGetLastError());
@@ -278,8 +316,8 @@ int scorch_hip_spmm_csr_rows_panels_f32(int64_t M, int64_t K, int64_t N, int64_t
   SCORCH_PANELS(4, 2);
   SCORCH_PANELS(4, 4);
   SCORCH_PANELS(4, 8);
+  SCORCH_PANELS(8, 2);
   SCORCH_PANELS(8, 4);
-  SCORCH_PANELS(8, 8);
   SCORCH_PANELS(16, 1);
   SCORCH_PANELS(32, 1);
 #undef SCORCH_PANELS

@@ -534,6 +534,42 @@ def test_panels_of_the_dense_operand_in_lds(oracle, M, K, N, per_row, transposed
     assert L.scorch_hip_spmm_csr_rows_panels_recommended(M, 20_000, N, ci.size, per_row, transposed) == 0   # no panel fits
 
 
+@pytest.mark.parametrize("K", [300, 1300, 2600, 5200])                # panels of 32, 16, 8 and 4 columns
+@pytest.mark.parametrize("N", [1, 3, 4, 6, 31, 35])
+def test_panels_of_rows_that_end_anywhere_in_a_batch(oracle, K, N):
+    """Rows of one entry to two past eight batches' (K allowing) and empty ones, columns to both sides of a
+    panel's last and of a 16-byte piece's, an infinity in a row of the dense operand that few rows refer to:
+    it reaches those and nothing else, whatever the lanes without an entry add.  fp32 sums of at most K products
+    in any order: 1e-5 of the Frobenius norm."""
+    from scorch_amd import native
+    rng = np.random.default_rng(K + N)
+    ends = [n for b in (64, 128, 256, 512) for n in (b - 1, b, b + 1) if n < K]
+    lens = np.array([0, 1, 2, 15, 16, 17, 0, 33] + ends + [K - 1, 0])
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = np.concatenate([1 + np.sort(rng.choice(K - 1, n, replace=False)) for n in lens]).astype(np.int32)
+    marked = [3, 9]
+    ci[rp[marked]] = 0
+    v = rng.uniform(0.5, 1, ci.size).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    L, stream = native.lib(), torch.cuda.current_stream().cuda_stream
+    want = oracle.spmm_fp64(rp, ci, v, B)
+    M = len(lens)
+    d_rp, d_ci, d_v = dev(rp), dev(ci), dev(v)
+    for transposed in (0, 1):
+        outs = []
+        for top in (B[0], np.full(N, np.inf, dtype=np.float32)):
+            B2 = np.concatenate([top[None], B[1:]])
+            d_B = dev(np.ascontiguousarray(B2.T) if transposed else B2)
+            out = torch.full((M, N), float("nan"), device="cuda")
+            native.check(L.scorch_hip_spmm_csr_rows_panels_f32(
+                M, K, N, ci.size, d_rp.data_ptr(), d_ci.data_ptr(), d_v.data_ptr(), d_B.data_ptr(), transposed, None, 0,
+                out.data_ptr(), stream))
+            outs.append(host(out))
+        assert oracle.rel_fro(outs[0], want) <= 1e-5
+        others = np.setdiff1d(np.arange(M), marked)
+        assert np.array_equal(outs[0][others], outs[1][others]) and np.isposinf(outs[1][marked]).all()
+
+
 @pytest.mark.parametrize("M, K, per_row", [(2, 900, 900), (100, 64, 33), (512, 1024, 64), (520, 1024, 65), (4096, 2000, 64), (3000, 2000, 70)])
 def test_tiled_kernel_with_several_lane_groups_to_a_row(oracle, M, K, per_row):
     """Chunks of one, two and four rows (eight, four and two lane groups to each), rows that end at a chunk's
