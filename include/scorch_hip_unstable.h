@@ -381,6 +381,8 @@ SCORCH_HIP_API int scorch_hip_csr_block_fill(int64_t M, int64_t n_cols, int64_t 
  *   _sddmm_csr_batched: out_row_idx (may be NULL) is written once, nnz entries.
  *   _softmax_csr_batched: workspace as for scorch_hip_softmax_csr_f32.
  *   _spmm_csr_rows_batched: the row-split kernel (short rows), no workspace.
+ *   _spmm_csr_rows_panels_batched: scorch_hip_spmm_csr_rows_panels_f32, for what its _recommended says of a single
+ *     product (no bias, B as it lies).
  *   _spmm_csr_batched: the merge-path kernels; workspace of
  *     scorch_hip_spmm_csr_batched_workspace_bytes(batch, M, nnz, N) bytes;
  *     `bounds` as for scorch_hip_spmm_csr_planned_f32 (may be NULL).
@@ -395,6 +397,10 @@ SCORCH_HIP_API int scorch_hip_softmax_csr_batched_f32(int64_t batch, int64_t M, 
                                        float *out /* [batch, nnz] */, void *workspace, size_t workspace_bytes,
                                        void *stream);
 SCORCH_HIP_API int scorch_hip_spmm_csr_rows_batched_f32(int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz,
+                                         const int32_t *row_ptr, const int32_t *col_idx,
+                                         const float *vals /* [batch, nnz] */, const float *B /* [batch, K, N] */,
+                                         float *C /* [batch, M, N] */, void *stream);
+SCORCH_HIP_API int scorch_hip_spmm_csr_rows_panels_batched_f32(int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz,
                                          const int32_t *row_ptr, const int32_t *col_idx,
                                          const float *vals /* [batch, nnz] */, const float *B /* [batch, K, N] */,
                                          float *C /* [batch, M, N] */, void *stream);

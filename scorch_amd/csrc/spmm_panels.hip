@@ -62,14 +62,18 @@ template <int P, int R>
 __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
     int M, int K, int N, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
     const float *__restrict__ vals, const float *__restrict__ B, int transposed, const float *__restrict__ bias,
-    int relu, float *__restrict__ C, int n_panels, int shares, int rows_per_share) {
+    int relu, float *__restrict__ C, int batch, int n_panels, int shares, int rows_per_share, int64_t nnz) {
   constexpr int LPE = P / 4;              // lanes to an entry
   constexpr int BATCH = R * kWaveSize;    // entries at hand: R to a lane
   extern __shared__ float4 s_panel[];     // [K + 1][LPE], row K is zero
 
   const int id = (int)xcd_contiguous(blockIdx.x, gridDim.x);
-  const int panel = id / shares, share = id % shares;
-  if (panel >= n_panels) return;
+  const int share = id % shares, panel = id / shares % n_panels;
+  const int product = id / shares / n_panels;  // of a batch over one pattern
+  if (product >= batch) return;
+  vals += (size_t)product * (size_t)nnz;
+  B += (size_t)product * (size_t)K * (size_t)N;
+  C += (size_t)product * (size_t)M * (size_t)N;
   const int n0 = panel * P;
   const int row_end = min(M, (share + 1) * rows_per_share);
   const int lane = wave_lane(), part = lane % LPE;
@@ -229,33 +233,39 @@ inline int64_t panel_lds(int64_t K, int width) { return (K + 1) * width * 4; }
 // N = 379, P = 8 113 for 115; 1,024 x 8,192, 400, N = 1,024, P = 4 75 for 81; 4,096 x 1,024, 49, N = 256, P = 32 12.3 for 11.5;
 // 465 x 1,863, 90, N = 167, P = 8 6.4 for 5.9.  The row kernel in its place: 17.0, 167, -, 17.0, 8.5; and at the line between the
 // two, 663 x 226, 48, N = 716 6.9 for 8.1, 1,448 x 517, 64, N = 244 6.4 for 7.9, 2,301 x 702, 64, N = 122 6.2 for 7.2.)
+inline PanelShape panel_shape_of_width(int64_t M, int64_t K, int64_t N, int64_t nnz, int width, int64_t batch) {
+  const int64_t mean = (nnz + M - 1) / M;
+  const int in_flight = width >= 16 ? 1 : width == 8 ? (mean > 192 ? 4 : 2) : mean > 256 ? 8 : mean > 128 ? 4 : 2;
+  PanelShape best = {0, in_flight, 0, 0};
+  const int64_t lds = panel_lds(K, width);
+  if (lds > kPanelLds) return best;
+  const int64_t in_batch = kWaveSize * in_flight, panels = (N + width - 1) / width * batch;
+  const double per_entry = width == 32 ? 1.2 : width == 16 ? 0.8 : width == 8 ? 0.47 : 0.25;
+  const double work = (double)M * ((double)((mean + in_batch - 1) / in_batch * in_batch) * per_entry + 50);
+  for (int64_t shares = 1; shares <= 512 && (shares == 1 || shares * kPanelWaves <= M); ++shares) {
+    const double rounds = (double)((panels * shares + 255) / 256);
+    const double us = 2.5 + rounds * ((double)lds / 24 + work / (double)shares) / 2400;
+    if (best.width == 0 || us < best.us) best = {width, in_flight, (int)shares, us};
+    if (panels * shares >= 2048) break;
+  }
+  return best;
+}
+
 inline PanelShape panel_shape(int64_t M, int64_t K, int64_t N, int64_t nnz) {
   PanelShape best = {0, 0, 0, 0};
   if (M <= 0 || N <= 0 || K > kPanelLds / 16) return best;
-  const int64_t mean = (nnz + M - 1) / M;
   for (int width : {32, 16, 8, 4}) {
-    const int in_flight = width >= 16 ? 1 : width == 8 ? (mean > 192 ? 4 : 2) : mean > 256 ? 8 : mean > 128 ? 4 : 2;
-    const int64_t lds = panel_lds(K, width);
-    if (lds > kPanelLds) continue;
-    const int64_t batch = kWaveSize * in_flight;
-    const double per_entry = width == 32 ? 1.2 : width == 16 ? 0.8 : width == 8 ? 0.47 : 0.25;
-    const double work = (double)M * ((double)((mean + batch - 1) / batch * batch) * per_entry + 50);
-    const int64_t panels = (N + width - 1) / width;
-    for (int64_t shares = 1; shares <= 512 && (shares == 1 || shares * kPanelWaves <= M); ++shares) {
-      const double rounds = (double)((panels * shares + 255) / 256);
-      const double us = 2.5 + rounds * ((double)lds / 24 + work / (double)shares) / 2400;
-      if (best.width == 0 || us < best.us) best = {width, in_flight, (int)shares, us};
-      if (panels * shares >= 2048) break;
-    }
+    const PanelShape shape = panel_shape_of_width(M, K, N, nnz, width, 1);
+    if (shape.width != 0 && (best.width == 0 || shape.us < best.us)) best = shape;
   }
   return best;
 }
 
 template <int P, int R>
-int launch_panels(int64_t M, int64_t K, int64_t N, const int *row_ptr, const int *col_idx, const float *vals, const float *B,
-                  int transposed, const float *bias, int relu, float *C, int shares, hipStream_t s) {
+int launch_panels(int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int *row_ptr, const int *col_idx,
+                  const float *vals, const float *B, int transposed, const float *bias, int relu, float *C, int shares, hipStream_t s) {
   const int64_t panels = (N + P - 1) / P;
-  const int64_t grid = round_up_8(panels * shares);
+  const int64_t grid = round_up_8(batch * panels * shares);
   if (grid > INT32_MAX) return fail(SCORCH_HIP_EUNSUPPORTED, "SpMM (panels): %lld workgroups exceed the launch limit", (long long)grid);
   static std::atomic<uint64_t> allowed{0};  // (per kernel) a bit per device: the attribute is a device's own
   int device = 0;
@@ -268,11 +278,49 @@ int launch_panels(int64_t M, int64_t K, int64_t N, const int *row_ptr, const int
   }
   mark_launch(s);
   spmm_panels_kernel<P, R><<<dim3((unsigned)grid), kPanelThreads, (size_t)panel_lds(K, P), s>>>(
-      (int)M, (int)K, (int)N, row_ptr, col_idx, vals, B, transposed, bias, relu, C, (int)panels, shares,
-      (int)((M + shares - 1) / shares));
+      (int)M, (int)K, (int)N, row_ptr, col_idx, vals, B, transposed, bias, relu, C, (int)batch, (int)panels,
+      shares, (int)((M + shares - 1) / shares), nnz);
   SCORCH_HIP_CHECK(hipGetLastError());
   mark_launch(s);
   return SCORCH_HIP_OK;
+}
+
+// `batch` products over one pattern, vals[h], B[h] and C[h] one behind the other: the panel width that a single one gets, so that
+// each has the bits it would have by itself, and row shares for all of them.
+int panels_entry(const char *fn, int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,
+                 const int32_t *col_idx, const float *vals, const float *B, int transposed, const float *bias, int act, float *C,
+                 void *stream) {
+  if (int rc = check_csr_args(fn, M, K, nnz, row_ptr, col_idx, vals)) return rc;
+  SCORCH_REQUIRE(N >= 0, "%s: negative N=%lld", fn, (long long)N);
+  SCORCH_REQUIRE(batch >= 0, "%s: negative batch=%lld", fn, (long long)batch);
+  if (N > INT32_MAX - kWaveSize * 4)
+    return fail(SCORCH_HIP_EUNSUPPORTED, "%s: N=%lld is too large", fn, (long long)N);
+  SCORCH_REQUIRE(act == SCORCH_HIP_ACT_NONE || act == SCORCH_HIP_ACT_RELU, "%s: unknown activation %d", fn, act);
+  SCORCH_REQUIRE(act == SCORCH_HIP_ACT_NONE || bias != nullptr, "%s: an activation needs a bias", fn);
+  if (batch == 0 || M == 0 || N == 0) return SCORCH_HIP_OK;  // nothing to write
+  SCORCH_REQUIRE(C != nullptr, "%s: C is NULL", fn);
+  SCORCH_REQUIRE(K == 0 || B != nullptr, "%s: B is NULL", fn);
+  SCORCH_REQUIRE(aligned_to(B, 4) && aligned_to(C, 4) && aligned_to(vals, 4) && aligned_to(bias, 4),
+                 "%s: value arrays must be aligned to their element size", fn);
+  PanelShape shape = panel_shape(M, K, N, nnz);
+  if (shape.width == 0) return fail(SCORCH_HIP_EUNSUPPORTED, "%s: K=%lld rows of B do not fit a CU's LDS", fn, (long long)K);
+  if (batch > INT32_MAX / N)
+    return fail(SCORCH_HIP_EUNSUPPORTED, "%s: a batch of %lld exceeds the launch limit", fn, (long long)batch);
+  if (batch > 1) shape = panel_shape_of_width(M, K, N, nnz, shape.width, batch);
+  const int relu = act == SCORCH_HIP_ACT_RELU;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define SCORCH_PANELS(P, R)                                                                                            \
+  if (shape.width == P && shape.in_flight == R)                                                                        \
+    return launch_panels<P, R>(batch, M, K, N, nnz, row_ptr, col_idx, vals, B, transposed, bias, relu, C, shape.shares, s)
+  SCORCH_PANELS(4, 2);
+  SCORCH_PANELS(4, 4);
+  SCORCH_PANELS(4, 8);
+  SCORCH_PANELS(8, 2);
+  SCORCH_PANELS(8, 4);
+  SCORCH_PANELS(16, 1);
+  SCORCH_PANELS(32, 1);
+#undef SCORCH_PANELS
+  return fail(SCORCH_HIP_ERUNTIME, "%s: no kernel for panels of %d columns", fn, shape.width);
 }
 
 }  // namespace scorch
@@ -291,37 +339,17 @@ int scorch_hip_spmm_csr_rows_panels_recommended(int64_t M, int64_t K, int64_t N,
 }
 
 int scorch_hip_spmm_csr_rows_panels_f32(int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,
-                                   const int32_t *col_idx, const float *vals, const float *B, int transposed,
-                                   const float *bias, int act, float *C, void *stream) {
-  using namespace scorch;
-  const char *fn = "scorch_hip_spmm_csr_rows_panels_f32";
-  if (int rc = check_csr_args(fn, M, K, nnz, row_ptr, col_idx, vals)) return rc;
-  SCORCH_REQUIRE(N >= 0, "%s: negative N=%lld", fn, (long long)N);
-  if (N > INT32_MAX - kWaveSize * 4)
-    return fail(SCORCH_HIP_EUNSUPPORTED, "%s: N=%lld is too large", fn, (long long)N);
-  SCORCH_REQUIRE(act == SCORCH_HIP_ACT_NONE || act == SCORCH_HIP_ACT_RELU, "%s: unknown activation %d", fn, act);
-  SCORCH_REQUIRE(act == SCORCH_HIP_ACT_NONE || bias != nullptr, "%s: an activation needs a bias", fn);
-  if (M == 0 || N == 0) return SCORCH_HIP_OK;  // nothing to write
-  SCORCH_REQUIRE(C != nullptr, "%s: C is NULL", fn);
-  SCORCH_REQUIRE(K == 0 || B != nullptr, "%s: B is NULL", fn);
-  SCORCH_REQUIRE(aligned_to(B, 4) && aligned_to(C, 4) && aligned_to(vals, 4) && aligned_to(bias, 4),
-                 "%s: value arrays must be aligned to their element size", fn);
-  const PanelShape shape = panel_shape(M, K, N, nnz);
-  if (shape.width == 0) return fail(SCORCH_HIP_EUNSUPPORTED, "%s: K=%lld rows of B do not fit a CU's LDS", fn, (long long)K);
-  const int relu = act == SCORCH_HIP_ACT_RELU;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-#define SCORCH_PANELS(P, R)                           \
-  if (shape.width == P && shape.in_flight == R)       \
-    return launch_panels<P, R>(M, K, N, row_ptr, col_idx, vals, B, transposed, bias, relu, C, shape.shares, s)
-  SCORCH_PANELS(4, 2);
-  SCORCH_PANELS(4, 4);
-  SCORCH_PANELS(4, 8);
-  SCORCH_PANELS(8, 2);
-  SCORCH_PANELS(8, 4);
-  SCORCH_PANELS(16, 1);
-  SCORCH_PANELS(32, 1);
-#undef SCORCH_PANELS
-  return fail(SCORCH_HIP_ERUNTIME, "%s: no kernel for panels of %d columns", fn, shape.width);
+                                        const int32_t *col_idx, const float *vals, const float *B, int transposed,
+                                        const float *bias, int act, float *C, void *stream) {
+  return scorch::panels_entry("scorch_hip_spmm_csr_rows_panels_f32", 1, M, K, N, nnz, row_ptr, col_idx, vals, B, transposed, bias,
+                              act, C, stream);
+}
+
+int scorch_hip_spmm_csr_rows_panels_batched_f32(int64_t batch, int64_t M, int64_t K, int64_t N, int64_t nnz,
+                                                const int32_t *row_ptr, const int32_t *col_idx, const float *vals,
+                                                const float *B, float *C, void *stream) {
+  return scorch::panels_entry("scorch_hip_spmm_csr_rows_panels_batched_f32", batch, M, K, N, nnz, row_ptr, col_idx, vals, B, 0,
+                              nullptr, SCORCH_HIP_ACT_NONE, C, stream);
 }
 
 }  // extern "C"

@@ -114,6 +114,8 @@ SIGNATURES = {
                                                           _size, _ptr]),
     "scorch_hip_spmm_csr_rows_batched_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
                                                             _ptr, _ptr]),
+    "scorch_hip_spmm_csr_rows_panels_batched_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
+                                                                   _ptr, _ptr]),
     "scorch_hip_spmm_csr_batched_workspace_bytes": (_size, [_i64, _i64, _i64, _i64]),
     "scorch_hip_spmm_csr_batched_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,
                                                        _ptr, _size, _ptr, _size, _ptr]),

@@ -357,7 +357,7 @@ class CsrPlan:
     row-pointer tensor, so it is dropped with the operand, and is rebuilt when
     either index tensor has been written to since."""
     __slots__ = ("key", "partner", "max_row", "empty_rows", "sorted_rows", "runs", "bounds", "sddmm_lists",
-                 "sddmm_uses", "rows", "blocked", "blocked_uses", "attention", "attention_uses", "other_columns")
+                 "sddmm_uses", "rows", "blocked", "blocked_uses", "attention", "attention_uses", "other_columns", "panels")
 
     def __init__(self, key, max_row: int, empty_rows: int, sorted_rows: bool = False, runs: int = 0):
         self.key = key
@@ -375,6 +375,7 @@ class CsrPlan:
         self.attention = None                              # BlockMask, False (blocks too thinly filled), None (not yet)
         self.attention_uses = 0                            # sparse_attention_csr calls
         self.other_columns = None                          # (weak reference, stamp): column indices last multiplied over these rows
+        self.panels: Dict[int, int] = {}                   # by dense width: whether products go to the panel kernel
 
     __reduce_ex__ = _Kept.__reduce_ex__
 
@@ -449,6 +450,14 @@ def csr_plan(pos: torch.Tensor, crd: torch.Tensor, n_rows: int, n_cols: int, wha
 
 def _malformed(what: str, problems) -> ValueError:
     return ValueError(f"scorch_ops_hip: {what}: malformed CSR index: " + "; ".join(problems))
+
+
+def _takes_panels(plan: CsrPlan, M: int, K: int, N: int, nnz: int, L) -> int:
+    """Whether an fp32 product over these rows goes to the kernel with the dense operand in LDS."""
+    known = plan.panels.get(N)
+    if known is None:
+        known = plan.panels[N] = L.scorch_hip_spmm_csr_rows_panels_recommended(M, K, N, nnz, plan.max_row, 0)
+    return known
 
 
 def _chunk_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, N: int, elem: int, L, stream) -> Optional[torch.Tensor]:
@@ -886,7 +895,7 @@ def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N
                 native.check(_blocked_spmm(L, bl, 1, M, K, N, nnz, a_val, b_val, out, stream))
                 return Tensor(out, [[], []])
         if tiled is None and path == "auto" and plan is not None and dtype == torch.float32 and \
-                L.scorch_hip_spmm_csr_rows_panels_recommended(M, K, N, nnz, plan.max_row, 0):
+                _takes_panels(plan, M, K, N, nnz, L):
             native.check(L.scorch_hip_spmm_csr_rows_panels_f32(M, K, N, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(),
                                                           b_val.data_ptr(), 0, bias_ptr, act, out.data_ptr(), stream))
             return Tensor(out, [[], []])
@@ -1696,6 +1705,9 @@ def spmm_csr_float_batched(A_shape, A_mode_indices, A_values: torch.Tensor, B: t
         bl = _blocked(plan, pos, crd, M, K, N) if SPMM_PATH == "auto" else None
         if bl is not None:
             rc = _blocked_spmm(L, bl, H, M, K, N, nnz, a_val, b, out, stream)
+        elif SPMM_PATH == "auto" and plan is not None and _takes_panels(plan, M, K, N, nnz, L):
+            rc = L.scorch_hip_spmm_csr_rows_panels_batched_f32(H, M, K, N, nnz, pos.data_ptr(), crd.data_ptr(),
+                                                               a_val.data_ptr(), b.data_ptr(), out.data_ptr(), stream)
         elif SPMM_PATH == "rows" or (SPMM_PATH == "auto" and plan is not None and
                                     L.scorch_hip_spmm_csr_rows_recommended(M, nnz, plan.max_row)):
             rc = L.scorch_hip_spmm_csr_rows_batched_f32(H, M, K, N, nnz, pos.data_ptr(), crd.data_ptr(),

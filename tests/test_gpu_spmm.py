@@ -568,6 +568,17 @@ def test_panels_of_rows_that_end_anywhere_in_a_batch(oracle, K, N):
         assert oracle.rel_fro(outs[0], want) <= 1e-5
         others = np.setdiff1d(np.arange(M), marked)
         assert np.array_equal(outs[0][others], outs[1][others]) and np.isposinf(outs[1][marked]).all()
+    # three products over the pattern in one launch: the bits of three separate ones
+    d_v3 = dev(np.stack([v, 2 * v, -v]))
+    d_B3 = dev(np.stack([B, B[::-1], B]))
+    three, alone = torch.full((3, M, N), float("nan"), device="cuda"), torch.empty(M, N, device="cuda")
+    native.check(L.scorch_hip_spmm_csr_rows_panels_batched_f32(
+        3, M, K, N, ci.size, d_rp.data_ptr(), d_ci.data_ptr(), d_v3.data_ptr(), d_B3.data_ptr(), three.data_ptr(), stream))
+    for h in range(3):
+        native.check(L.scorch_hip_spmm_csr_rows_panels_f32(
+            M, K, N, ci.size, d_rp.data_ptr(), d_ci.data_ptr(), d_v3[h].data_ptr(), d_B3[h].data_ptr(), 0, None, 0,
+            alone.data_ptr(), stream))
+        assert torch.equal(three[h], alone)
 
 
 @pytest.mark.parametrize("M, K, per_row", [(2, 900, 900), (100, 64, 33), (512, 1024, 64), (520, 1024, 65), (4096, 2000, 64), (3000, 2000, 70)])
