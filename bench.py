@@ -52,20 +52,20 @@ CONFIG_WORKLOADS = ("spmm_uniform", "sddmm_uniform", "attention_blocksparse", "s
 _CSRC = "scorch_amd/csrc/"
 _SPMM_SOURCES = (_CSRC + "spmm.hip", _CSRC + "spmm.hpp", _CSRC + "common.hpp")
 MEASURED_TRAFFIC = {
-    ("gcn_powerlaw", "merge"): {"bytes": 9_789_900_000, "sources": _SPMM_SOURCES, "sha16": "",
+    ("gcn_powerlaw", "merge"): {"bytes": 9_790_000_000, "sources": _SPMM_SOURCES, "sha16": "29d6cd6f4ca103a4",
                                 "profile": "profiles/spmm_merge_kernel_gcn_powerlaw.md"},
-    ("spmm_uniform", "rows"): {"bytes": 10_834_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp",
-                                                                _CSRC + "common.hpp"), "sha16": "",
+    ("spmm_uniform", "rows"): {"bytes": 10_832_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp",
+                                                                _CSRC + "common.hpp"), "sha16": "be5ce2017146dd01",
                                "profile": "profiles/spmm_rows_kernel_uniform_4096.md"},
-    ("sae_decoder", "tiled"): {"bytes": 344_300_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp",
-                                                                 _CSRC + "common.hpp"), "sha16": "",
+    ("sae_decoder", "tiled"): {"bytes": 344_100_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp",
+                                                                 _CSRC + "common.hpp"), "sha16": "6412349773054a07",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
-    ("sae_decoder", "merge"): {"bytes": 1_767_200_000, "sources": _SPMM_SOURCES, "sha16": "",
+    ("sae_decoder", "merge"): {"bytes": 1_766_000_000, "sources": _SPMM_SOURCES, "sha16": "29d6cd6f4ca103a4",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
-    ("sddmm_uniform", "listed"): {"bytes": 277_700_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
-                                  "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
-    ("sddmm_uniform", "plain"): {"bytes": 848_400_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
-                                 "sha16": "", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
+    ("sddmm_uniform", "listed"): {"bytes": 258_100_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
+                                  "sha16": "2766274460e3afef", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
+    ("sddmm_uniform", "plain"): {"bytes": 880_200_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
+                                 "sha16": "2766274460e3afef", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
     ("attention_blocksparse", "fused"): {"bytes": 81_050_000, "sources": (_CSRC + "attn.hip", _CSRC + "common.hpp"),
                                          "sha16": "93359f7faeb90848", "profile": "profiles/attn_blocksparse_kernel_s8192_h16.md"},
 }
