@@ -225,16 +225,20 @@ __device__ __forceinline__ int block_scan_min_max(int v, int &total, int &lo, in
 // TEAM entries of A at once -- thread t reads entry t, its B row's start and
 // length -- turns the lengths into offsets with a prefix sum, and then walks the
 // batch's products flat: product x belongs to the entry e with off[e] <= x <
-// off[e + 1].  Workgroups find it by bisection in LDS.  Teams of up to a wavefront
+// off[e + 1].  Teams of up to a wavefront
 // mark the first product of every entry that has any and take the running maximum of
 // the marks: six vector instructions per product instead of six dependent LDS reads with their
-// compares.  All lanes stay busy and consecutive lanes read consecutive entries of a B row.
+// compares.  The wavefronts of a workgroup take up to 256 products each, mark the first products of
+// entries by a bit, and count the bits up to a product's (entries_of_products); entries without products are left
+// out of the batch.  All lanes stay busy and consecutive lanes read consecutive entries of a B row.
 constexpr int kProductsInFlight = 4;
 
 template <int TEAM, typename A>
-struct ProductBatch {
-  int index[2 * TEAM];  // [e]: first product of entry e within the batch; [TEAM + e]: where its B row starts
+struct ProductBatch {  // of the entries that have products, in their order, INT_MAX behind them:
+  int first[TEAM];     // first product within the batch
+  int start[TEAM];     // where the B row starts, less that
   A a_val[TEAM];
+  uint4 begins[TEAM / kWaveSize][2];  // a wavefront's: a bit per product of its step that is an entry's first
 };
 template <typename A>
 struct MarkedBatch {
@@ -265,35 +269,70 @@ __device__ __forceinline__ int team_exclusive_scan(int v, int *scratch, int &tot
   return incl - v;
 }
 
-// One step of the walk over a batch's products: products x0, x0 + TEAM, ... (U of
-// them) of this thread.  Their bisections interleave and their loads from B are all
-// issued before the first is used; a step of one product waits out a whole memory
-// round trip for it.  PARTIAL: the batch may end within the step; slots beyond its
-// last product read that product again and hand nothing to fn.
-template <int TEAM, bool NUMERIC, int U, bool PARTIAL, typename T, typename A, typename Fn>
-__device__ __forceinline__ void product_step(int x0, int total, const int *__restrict__ b_crd,
-                                             const T *__restrict__ b_val,
-                                             const ProductBatch<TEAM, A> &batch, Fn &fn) {
-  int q[U], e[U];
+// Entries of a batch for a team of wavefronts: thread t's entry has `len` products, its B row starts at `lo`.  Returns
+// the number of products.  Two barriers, and one behind which the batch may be read.
+template <int TEAM, bool NUMERIC, typename A>
+__device__ __forceinline__ int fill_batch(int len, int lo, A av, ProductBatch<TEAM, A> &batch, int *scan_scratch) {
+  constexpr int WAVES = TEAM / kWaveSize;
+  const int t = threadIdx.x, lane = wave_lane(), w = t / kWaveSize;
+  const unsigned long long has = __ballot(len > 0);
+  const int incl = team_inclusive_sum<kWaveSize>(len);
+  __syncthreads();  // the previous batch has been read by everyone
+  if (lane == kWaveSize - 1) {
+    scan_scratch[w] = incl;
+    batch.begins[w][0].x = (unsigned)__popcll(has);
+  }
+  __syncthreads();
+  int first = incl - len, total = 0, entries = 0;
+  int at = __builtin_amdgcn_mbcnt_hi((unsigned)(has >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)has, 0u));
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) {
+    if (i == w) first += total, at += entries;
+    total += scan_scratch[i];
+    entries += (int)batch.begins[i][0].x;
+  }
+  if (len > 0) {
+    batch.first[at] = first;
+    batch.start[at] = lo - first;
+    if (NUMERIC) batch.a_val[at] = av;
+  }
+  if (t >= entries) batch.first[t] = INT_MAX;
+  __syncthreads();
+  return total;
+}
+
+// The entries e[u] that products xs + 64 u + lane, u < U, belong to, for a wavefront whose products are [xs, xe),
+// 0 <= xs < xe <= xs + 64 U.  The entry of the first is looked for by the whole wavefront at once; every entry that begins
+// behind it leaves a bit, and an entry's number is the bits up to the product: a third of the LDS reads and half of the vector
+// instructions of a bisection for every product.  (131,072 nodes, 16 a row, us: products made and sorted 108 -> 100, rows of up to
+// 4,096 products counted 19.6 -> 18.2 and summed 70.3 -> 66.7, of up to 1,024 28.6 -> 26.6 and 79.8 -> 78.2; what is left of the sort
+// is the gathers from B and its own writes, 4.4 TB/s.)
+template <int TEAM, int U, typename A>
+__device__ __forceinline__ void entries_of_products(int xs, int xe, ProductBatch<TEAM, A> &batch, int (&e)[U]) {
+  static_assert(U <= 4, "a bit per product");
+  constexpr int S = TEAM / kWaveSize;
+  const int lane = wave_lane(), w = uniform((int)threadIdx.x / kWaveSize);
+  unsigned *const begins = reinterpret_cast<unsigned *>(batch.begins[w]);
+  if (lane < 8) begins[lane] = 0u;
+  const int stretch = __popcll(__ballot(batch.first[lane * S] <= xs)) - 1;
+  const int e0 = stretch * S + __popcll(__ballot(lane < S && batch.first[stretch * S + lane % S] <= xs)) - 1;
+  wave_lds_sync();
+  for (int i = e0 + 1 + lane;; i += kWaveSize) {  // (64 of them begin in the step: there may be more)
+    const int first = i < TEAM ? batch.first[i] : INT_MAX;
+    if (first < xe) atomicOr(&begins[(first - xs) >> 5], 1u << ((first - xs) & 31));
+    if (!__all(first < xe)) break;
+  }
+  wave_lds_sync();
+  const uint4 b0 = batch.begins[w][0], b1 = batch.begins[w][1];
+  const unsigned words[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+  int before = e0;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int x = PARTIAL ? min(x0 + u * TEAM, total - 1) : x0 + u * TEAM;
-    e[u] = 0;  // the last entry whose offset is <= x (entries without products share an offset)
-#pragma unroll
-    for (int step = TEAM / 2; step > 0; step >>= 1)
-      if (batch.index[e[u] + step] <= x) e[u] += step;
-    q[u] = batch.index[TEAM + e[u]] + (x - batch.index[e[u]]);
+    const unsigned long long m = (unsigned long long)(unsigned)uniform((int)words[2 * u + 1]) << 32 | (unsigned)uniform((int)words[2 * u]);
+    const unsigned long long behind = m >> 1;  // bits up to a lane's own: the first, and of these those below it
+    e[u] = before + (int)(m & 1u) + __builtin_amdgcn_mbcnt_hi((unsigned)(behind >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)behind, 0u));
+    before += __popcll(m);
   }
-  int col[U];
-  A b[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    col[u] = b_crd[q[u]];
-    b[u] = NUMERIC ? (A)b_val[q[u]] : (A)0;
-  }
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (!PARTIAL || x0 + u * TEAM < total) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
 }
 
 // The same for a team of up to a wavefront, U = kProductsInFlight: `first` and `len` are this lane's entry's
@@ -350,28 +389,38 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
       len = b_pos[j + 1] - lo;
       if (NUMERIC) av = (A)a_val[p];
     }
-    int total = 0;
-    const int first = team_exclusive_scan<TEAM>(len, scan_scratch, total);
-    team_sync<TEAM>();  // the previous batch has been read by everyone
     if constexpr (TEAM <= kWaveSize) {
+      int total = 0;
+      const int first = team_exclusive_scan<TEAM>(len, scan_scratch, total);
+      team_sync<TEAM>();  // the previous batch has been read by everyone
       batch.start[t] = lo - first;
       if (NUMERIC) batch.a_val[t] = av;
       int carried = 0;
       for (int x = 0; x < total; x += U * TEAM)
         marked_step<TEAM, NUMERIC, T, A>(x, total, t, first, len, carried, b_crd, b_val, batch, fn);
-      continue;
     } else {
-    batch.index[t] = first;
-    batch.index[TEAM + t] = lo;
-    if (NUMERIC) batch.a_val[t] = av;
-    team_sync<TEAM>();
-    int x = 0;  // the team's first product of the step
-    for (; x + U * TEAM <= total; x += U * TEAM)
-      product_step<TEAM, NUMERIC, U, false, T, A>(x + t, total, b_crd, b_val, batch, fn);
-    if (x + TEAM < total)  // more than one product a thread is left
-      product_step<TEAM, NUMERIC, U, true, T, A>(x + t, total, b_crd, b_val, batch, fn);
-    else if (x + t < total)
-      product_step<TEAM, NUMERIC, 1, false, T, A>(x + t, total, b_crd, b_val, batch, fn);
+      const int total = fill_batch<TEAM, NUMERIC, A>(len, lo, av, batch, scan_scratch);
+      const int lane = wave_lane(), w = uniform(t / kWaveSize);
+      for (int x = 0; x < total; x += U * TEAM) {
+        // as many products to a thread as leave no wavefront without
+        const int each = min(U, (total - x + TEAM - 1) / TEAM), xs = x + w * each * kWaveSize;
+        const int xe = min(xs + each * kWaveSize, total);
+        if (xs >= xe) break;
+        int e[U], q[U], col[U];
+        A b[U];
+        entries_of_products<TEAM, U, A>(xs, xe, batch, e);
+#pragma unroll
+        for (int u = 0; u < U; ++u) q[u] = min(xs + u * kWaveSize + lane, total - 1) + batch.start[e[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (u > 0 && xs + u * kWaveSize >= xe) break;  // uniform over the wavefront
+          col[u] = b_crd[q[u]];
+          b[u] = NUMERIC ? (A)b_val[q[u]] : (A)0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (xs + u * kWaveSize + lane < xe) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
+      }
     }
   }
 }
@@ -1651,7 +1700,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
 // in LDS, by a workgroup that reads its runs from all of the row's windows: streams instead of
 // gathers, as many workgroups to a row as it has ranges, and a hub shared out by itself.
 // Both passes over these rows of a power-law graph squared (131,072 nodes, 16 entries a row, 19 M
-// products of this kind), fp32: 300 us (lists 19, sort 106, count 52, sums 123); the numeric pass alone took 512.  The sort is
+// products of this kind), fp32: 290 us (lists 17, sort 100, count 52, sums 121); the numeric pass alone took 512.  The sort is
 // bound by the gathers from B (a line for about two entries), the sums by LDS atomics.  (Ranges
 // without the windows, each item bisecting the rows of B for its piece, fetch those lines once
 // per range: 411 us for the numeric pass alone.)
@@ -1806,44 +1855,33 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
   if (item.shares == 0) return;
   const BinRow r = bins.row[item.row];
   const int lo = a_pos[r.row] + item.batch * kBinEntries, hi = min(lo + kBinEntries, a_pos[r.row + 1]);
-  {
-    int first = 0, len = 0;
-    A av = (A)0;
-    if (lo + tid < hi) {
-      const int j = a_crd[lo + tid];
-      first = b_pos[j];
-      len = b_pos[j + 1] - first;
-      av = (A)a_val[lo + tid];
-    }
-    int unused = 0;
-    s_batch.index[tid] = block_exclusive_scan_n<kBinThreads / kWaveSize>(len, s_scan, unused);
-    s_batch.index[kBinEntries + tid] = first;
-    s_batch.a_val[tid] = av;
-    if (tid == kBinThreads - 1) s_first = unused;
+  int start = 0, len = 0;
+  A av = (A)0;
+  if (lo + tid < hi) {
+    const int j = a_crd[lo + tid];
+    start = b_pos[j];
+    len = b_pos[j + 1] - start;
+    av = (A)a_val[lo + tid];
   }
-  __syncthreads();
-  const int total = s_first;
+  const int total = fill_batch<kBinEntries, true, A>(len, start, av, s_batch, s_scan);
+  const int lane = wave_lane(), w = uniform(tid / kWaveSize);
   for (int x0 = item.share * kBinProducts; x0 < total; x0 += item.shares * kBinProducts) {  // uniform
     const int n = min(kBinProducts, total - x0);
-    int q[U], e[U], col[U], rank[U];
+    const int each = (n + kBinThreads - 1) / kBinThreads, xs = x0 + w * each * kWaveSize, xe = min(xs + each * kWaveSize, x0 + n);
+    int e[U], col[U], rank[U];
     A b[U];
     unsigned long long used = 0;  // (the round trip passes while the products are gathered)
     if (tid == kBinThreads - 1) used = atomicAdd(&bins.used[item.row], (1ull << 32) + (unsigned)n);
+    if (xs < xe) {
+      entries_of_products<kBinEntries, U, A>(xs, xe, s_batch, e);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int x = min(x0 + u * kBinThreads + tid, total - 1);
-      e[u] = 0;  // as in product_step
-#pragma unroll
-      for (int step = kBinEntries / 2; step > 0; step >>= 1)
-        if (s_batch.index[e[u] + step] <= x) e[u] += step;
-      q[u] = s_batch.index[kBinEntries + e[u]] + (x - s_batch.index[e[u]]);
+      for (int u = 0; u < U; ++u) {
+        const int q = min(xs + u * kWaveSize + lane, total - 1) + s_batch.start[e[u]];
+        col[u] = b_crd[q];
+        b[u] = (A)b_val[q];
+      }
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      col[u] = b_crd[q[u]];
-      b[u] = (A)b_val[q[u]];
-    }
-    __syncthreads();  // everyone is done with the previous window (and has read s_first)
+    __syncthreads();  // everyone is done with the previous window
     if (tid <= kMaxBins) s_count[tid] = 0;
     if (tid == kBinThreads - 1) {
       s_first = (int)(unsigned)used;
@@ -1854,7 +1892,7 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       bin[u] = col[u] >> bins.shift;
-      if (u * kBinThreads + tid < n) rank[u] = atomicAdd(&s_count[bin[u]], 1);
+      if (xs + u * kWaveSize + lane < xe) rank[u] = atomicAdd(&s_count[bin[u]], 1);
     }
     __syncthreads();
     if (tid <= bins.n) {
@@ -1867,7 +1905,7 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (u * kBinThreads + tid < n) {
+      if (xs + u * kWaveSize + lane < xe) {
         const int at = s_at[bin[u]] + rank[u];
         s_column[at] = (unsigned short)(col[u] - (bin[u] << bins.shift));
         s_value[at] = s_batch.a_val[e[u]] * b[u];

@@ -521,3 +521,26 @@ def test_ranges_of_columns_of_every_width(oracle, hubs, hub, N):
     arp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     aci = np.concatenate([np.sort(rng.choice(K, n, replace=False)) for n in lens if n]).astype(np.int32)
     check(oracle, arp, aci, rng.uniform(-1, 1, aci.size).astype(np.float32), brp, bci, rng.uniform(-1, 1, bci.size).astype(np.float32), N)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int64])
+@pytest.mark.parametrize("products", [256, 257, 319, 320, 512, 1023, 1024, 1025, 2047, 2048, 4096, 4097, 9000])
+def test_products_of_rows_whose_entries_have_none_one_or_many(oracle, dtype, products):
+    """Rows of a workgroup's: entries of A whose row of B is empty, has one entry (256 begin in a wavefront's step of 256
+    products), or fills many steps, in every order; numbers of products on either side of a step's, a wavefront's and a tier's."""
+    rng = np.random.default_rng(products)
+    N, K, longest = 5000, 12_000, min(products, 3000)
+    blens = np.concatenate([np.zeros(K // 3, dtype=np.int64), np.ones(K - K // 3 - 1, dtype=np.int64), [longest]])
+    brp = np.concatenate([[0], np.cumsum(blens)]).astype(np.int32)
+    bci = np.concatenate([np.sort(rng.choice(N, n, replace=False)) for n in blens if n]).astype(np.int32)
+    ones, none, many = np.arange(K // 3, K - 1), np.arange(K // 3), np.array([K - 1])
+    rows = [np.concatenate([rng.choice(ones, products, replace=False) if products <= ones.size else ones]),
+            np.concatenate([rng.choice(ones, products - longest, replace=False), many]),
+            np.concatenate([none, rng.choice(ones, min(products, ones.size), replace=False)]),
+            np.concatenate([rng.choice(none, 700, replace=False), rng.choice(ones, min(products, ones.size), replace=False)]),
+            none, many]
+    rows = [np.sort(r) if i % 2 else rng.permutation(r) for i, r in enumerate(rows)]
+    aci = np.concatenate(rows).astype(np.int32)
+    arp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    value = (lambda n: rng.integers(-9, 9, n).astype(dtype)) if dtype == np.int64 else (lambda n: rng.uniform(-1, 1, n).astype(dtype))
+    check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
