@@ -1700,7 +1700,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
 // in LDS, by a workgroup that reads its runs from all of the row's windows: streams instead of
 // gathers, as many workgroups to a row as it has ranges, and a hub shared out by itself.
 // Both passes over these rows of a power-law graph squared (131,072 nodes, 16 entries a row, 19 M
-// products of this kind), fp32: 283 us (lists 17, sort 100, count 45, sums 121); the numeric pass alone took 512.  The sort is
+// products of this kind), fp32: 282 us (lists 17, sort 100, count 44, sums 121); the numeric pass alone took 512.  The sort is
 // bound by the gathers from B (a line for about two entries), the sums by LDS atomics.  (Ranges
 // without the windows, each item bisecting the rows of B for its piece, fetch those lines once
 // per range: 411 us for the numeric pass alone.)
@@ -1959,32 +1959,45 @@ __global__ __launch_bounds__(kBinCountThreads) void spgemm_bin_count_kernel(Bins
   for (int i = threadIdx.x; i < words; i += kBinCountThreads) s_bits[i] = 0u;
   __syncthreads();
   // Four runs of a wavefront's at a time, of clamped places (a load behind a condition is waited for before the next, and four
-  // runs gain nothing): 131,072 nodes, 16 a row 52 -> 45 us, 45,000, 10 a row 18.0 -> 14.9.  (The sums: 120 -> 126.)
+  // runs gain nothing): 131,072 nodes, 16 a row 52 -> 44 us, 45,000, 10 a row 18.0 -> 14.5, with a hub of 50,000 entries 72 -> 63.
+  // (The sums: 120 -> 126.)  Not where a wavefront has up to three, many of them of a few products: rows of at most 5,000 entries
+  // 28, four at a time 35.
   constexpr int kRuns = 4, kEach = 4;
-  for_each_runs<kWaves>(bins, r, windows, bin, [&](int first, int last, int here) {
-    for (int i = 0; i < here; i += kRuns) {
-      int p[kRuns], to[kRuns], longest = 0;
+  if (windows <= 3 * kWaves) {
+    for_each_binned<kWaves>(bins, r, windows, bin, [&](int p, int to) {
+      int c[4];
 #pragma unroll
-      for (int j = 0; j < kRuns; ++j) {
-        const int run = min(i + j, kWaveSize - 1), from = __builtin_amdgcn_readlane(first, run);
-        to[j] = i + j < here ? __builtin_amdgcn_readlane(last, run) : from;
-        longest = max(longest, to[j] - from);
-        p[j] = from + wave_lane();
+      for (int u = 0; u < 4; ++u) c[u] = p + u * kWaveSize < to ? bins.columns[p + u * kWaveSize] : -1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (c[u] >= 0) atomicOr(&s_bits[c[u] >> 5], 1u << (c[u] & 31));
+    });
+  } else {
+    for_each_runs<kWaves>(bins, r, windows, bin, [&](int first, int last, int here) {
+      for (int i = 0; i < here; i += kRuns) {
+        int p[kRuns], to[kRuns], longest = 0;
+#pragma unroll
+        for (int j = 0; j < kRuns; ++j) {
+          const int run = min(i + j, kWaveSize - 1), from = __builtin_amdgcn_readlane(first, run);
+          to[j] = i + j < here ? __builtin_amdgcn_readlane(last, run) : from;
+          longest = max(longest, to[j] - from);
+          p[j] = from + wave_lane();
+        }
+        for (int o = 0; o < longest; o += kEach * kWaveSize) {
+          int c[kRuns][kEach];
+#pragma unroll
+          for (int j = 0; j < kRuns; ++j)
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) c[j][u] = bins.columns[max(min(p[j] + o + u * kWaveSize, to[j] - 1), 0)];
+#pragma unroll
+          for (int j = 0; j < kRuns; ++j)
+#pragma unroll
+            for (int u = 0; u < kEach; ++u)
+              if (p[j] + o + u * kWaveSize < to[j]) atomicOr(&s_bits[c[j][u] >> 5], 1u << (c[j][u] & 31));
+        }
       }
-      for (int o = 0; o < longest; o += kEach * kWaveSize) {
-        int c[kRuns][kEach];
-#pragma unroll
-        for (int j = 0; j < kRuns; ++j)
-#pragma unroll
-          for (int u = 0; u < kEach; ++u) c[j][u] = bins.columns[max(min(p[j] + o + u * kWaveSize, to[j] - 1), 0)];
-#pragma unroll
-        for (int j = 0; j < kRuns; ++j)
-#pragma unroll
-          for (int u = 0; u < kEach; ++u)
-            if (p[j] + o + u * kWaveSize < to[j]) atomicOr(&s_bits[c[j][u] >> 5], 1u << (c[j][u] & 31));
-      }
-    }
-  });
+    });
+  }
   __syncthreads();
   int mine = 0, total = 0;
   for (int i = threadIdx.x; i < words; i += kBinCountThreads) mine += __popc(s_bits[i]);
