@@ -254,17 +254,9 @@ struct ProductBatch<16, A> {
   unsigned mark[kProductsInFlight * 16 / 4];
 };
 
-// Teams of up to a wavefront (64 lanes, or an aligned part of one) need no
-// barrier: a wavefront's LDS operations complete in program order.
 template <int TEAM>
-__device__ __forceinline__ void team_sync() {
-  if (TEAM <= kWaveSize) wave_lds_sync(); else __syncthreads();
-}
-
-template <int TEAM>
-__device__ __forceinline__ int team_exclusive_scan(int v, int *scratch, int &total) {
-  if (TEAM > kWaveSize) return block_exclusive_scan_n<TEAM / kWaveSize>(v, scratch, total);
-  const int incl = team_inclusive_sum<TEAM <= kWaveSize ? TEAM : kWaveSize>(v);
+__device__ __forceinline__ int team_exclusive_scan(int v, int &total) {
+  const int incl = team_inclusive_sum<TEAM>(v);
   total = team_last<TEAM>(incl);
   return incl - v;
 }
@@ -391,8 +383,8 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
     }
     if constexpr (TEAM <= kWaveSize) {
       int total = 0;
-      const int first = team_exclusive_scan<TEAM>(len, scan_scratch, total);
-      team_sync<TEAM>();  // the previous batch has been read by everyone
+      const int first = team_exclusive_scan<TEAM>(len, total);
+      wave_lds_sync();  // the previous batch has been read by everyone (LDS operations of a wavefront complete in program order)
       batch.start[t] = lo - first;
       if (NUMERIC) batch.a_val[t] = av;
       int carried = 0;
@@ -905,7 +897,7 @@ __device__ __forceinline__ void spgemm_team_row(
     wave_lds_sync();
     const int c0 = cnt[2 * t], c1 = cnt[2 * t + 1];  // lane t places buckets 2t and 2t + 1
     int unused = 0;
-    const int before = team_exclusive_scan<TEAM>(c0 + c1, nullptr, unused);
+    const int before = team_exclusive_scan<TEAM>(c0 + c1, unused);
     int crowd = c0 > c1 ? c0 : c1;
     crowd = team_last<TEAM>(team_inclusive_max<TEAM>(crowd));
     if (crowd <= kCrowd) {  // uniform
