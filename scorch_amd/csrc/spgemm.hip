@@ -41,6 +41,7 @@
 // integer results are exact.
 #include <climits>
 
+#include "products.hpp"
 #include "sync.hpp"
 
 namespace scorch {
@@ -293,15 +294,16 @@ __device__ __forceinline__ int fill_batch(int len, int lo, A av, ProductBatch<TE
   return total;
 }
 
-// The entries e[u] that products xs + 64 u + lane, u < U, belong to, for a wavefront whose products are [xs, xe),
-// 0 <= xs < xe <= xs + 64 U.  The entry of the first is looked for by the whole wavefront at once; every entry that begins
+// The entries e[u] that the products of a wavefront's step belong to, slot u < U and lane: those of step.product(u, lane), which
+// is below the step's end (an entry that begins there or later leaves no bit).  0 <= step.first < step.last.  The entry of the first is looked for by the whole wavefront at once; every entry that begins
 // behind it leaves a bit, and an entry's number is the bits up to the product: a third of the LDS reads and half of the vector
 // instructions of a bisection for every product.  (131,072 nodes, 16 a row, us: products made and sorted 108 -> 100, rows of up to
 // 4,096 products counted 19.6 -> 18.2 and summed 70.3 -> 66.7, of up to 1,024 28.6 -> 26.6 and 79.8 -> 78.2; what is left of the sort
 // is the gathers from B and its own writes, 4.4 TB/s.)
 template <int TEAM, int U, typename A>
-__device__ __forceinline__ void entries_of_products(int xs, int xe, ProductBatch<TEAM, A> &batch, int (&e)[U]) {
-  static_assert(U <= 4, "a bit per product");
+__device__ __forceinline__ void entries_of_products(const ProductStep &step, ProductBatch<TEAM, A> &batch, int (&e)[U]) {
+  static_assert(U <= 4 && kProductLanes == kWaveSize, "a bit per product");
+  const int xs = step.first, xe = step.last;
   constexpr int S = TEAM / kWaveSize;
   const int lane = wave_lane(), w = uniform((int)threadIdx.x / kWaveSize);
   unsigned *const begins = reinterpret_cast<unsigned *>(batch.begins[w]);
@@ -394,24 +396,22 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
       const int total = fill_batch<TEAM, NUMERIC, A>(len, lo, av, batch, scan_scratch);
       const int lane = wave_lane(), w = uniform(t / kWaveSize);
       for (int x = 0; x < total; x += U * TEAM) {
-        // as many products to a thread as leave no wavefront without
-        const int each = min(U, (total - x + TEAM - 1) / TEAM), xs = x + w * each * kWaveSize;
-        const int xe = min(xs + each * kWaveSize, total);
-        if (xs >= xe) break;
+        const ProductStep step = product_step(x, min(U * TEAM, total - x), TEAM / kWaveSize, w);
+        if (step.first >= step.last) break;
         int e[U], q[U], col[U];
         A b[U];
-        entries_of_products<TEAM, U, A>(xs, xe, batch, e);
+        entries_of_products<TEAM, U, A>(step, batch, e);
 #pragma unroll
-        for (int u = 0; u < U; ++u) q[u] = min(xs + u * kWaveSize + lane, total - 1) + batch.start[e[u]];
+        for (int u = 0; u < U; ++u) q[u] = step.product(u, lane) + batch.start[e[u]];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (u > 0 && xs + u * kWaveSize >= xe) break;  // uniform over the wavefront
+          if (u > 0 && !step.has(u)) break;  // uniform over the wavefront
           col[u] = b_crd[q[u]];
           b[u] = NUMERIC ? (A)b_val[q[u]] : (A)0;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (xs + u * kWaveSize + lane < xe) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
+          if (step.first + u * kWaveSize + lane < step.last) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
       }
     }
   }
@@ -1859,16 +1859,17 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
   const int lane = wave_lane(), w = uniform(tid / kWaveSize);
   for (int x0 = item.share * kBinProducts; x0 < total; x0 += item.shares * kBinProducts) {  // uniform
     const int n = min(kBinProducts, total - x0);
-    const int each = (n + kBinThreads - 1) / kBinThreads, xs = x0 + w * each * kWaveSize, xe = min(xs + each * kWaveSize, x0 + n);
+    const ProductStep step = product_step(x0, n, kBinThreads / kWaveSize, w);
     int e[U], col[U], rank[U];
     A b[U];
     unsigned long long used = 0;  // (the round trip passes while the products are gathered)
     if (tid == kBinThreads - 1) used = atomicAdd(&bins.used[item.row], (1ull << 32) + (unsigned)n);
-    if (xs < xe) {
-      entries_of_products<kBinEntries, U, A>(xs, xe, s_batch, e);
+    if (step.first < step.last) {
+      entries_of_products<kBinEntries, U, A>(step, s_batch, e);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int q = min(xs + u * kWaveSize + lane, total - 1) + s_batch.start[e[u]];
+        if (u > 0 && !step.has(u)) break;  // uniform over the wavefront
+        const int q = step.product(u, lane) + s_batch.start[e[u]];
         col[u] = b_crd[q];
         b[u] = (A)b_val[q];
       }
@@ -1882,10 +1883,11 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
     __syncthreads();
     int bin[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      bin[u] = col[u] >> bins.shift;
-      if (xs + u * kWaveSize + lane < xe) rank[u] = atomicAdd(&s_count[bin[u]], 1);
-    }
+    for (int u = 0; u < U; ++u)
+      if (step.first + u * kWaveSize + lane < step.last) {
+        bin[u] = col[u] >> bins.shift;
+        rank[u] = atomicAdd(&s_count[bin[u]], 1);
+      }
     __syncthreads();
     if (tid <= bins.n) {
       int at = 0;
@@ -1897,7 +1899,7 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (xs + u * kWaveSize + lane < xe) {
+      if (step.first + u * kWaveSize + lane < step.last) {
         const int at = s_at[bin[u]] + rank[u];
         s_column[at] = (unsigned short)(col[u] - (bin[u] << bins.shift));
         s_value[at] = s_batch.a_val[e[u]] * b[u];
