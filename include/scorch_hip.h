@@ -286,8 +286,9 @@ SCORCH_HIP_API int scorch_hip_softmax_csr_f32(int64_t M, int64_t nnz, const int3
  *                                   terms up in another grouping (equal to rounding).  Both are
  *                                   bit-reproducible from call to call.
  * scorch_hip_sddmm_csr_plan_f32     like scorch_hip_sddmm_csr_f32 (mask_vals and out_row_idx may
- *                                   be NULL); a mask with a dense right operand of 8 to 20 MB is
- *                                   served from per-XCD entry lists built once.  Bit-identical.
+ *                                   be NULL); a mask with a dense right operand of 4.5 to 20 MiB and
+ *                                   four entries a column or more is served from per-XCD entry
+ *                                   lists built once.  Bit-identical.
  * scorch_hip_softmax_csr_plan_f32   like scorch_hip_softmax_csr_f32; one launch when no row is
  *                                   longer than 4096.  Bit-identical.
  *

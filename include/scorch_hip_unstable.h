@@ -214,7 +214,9 @@ SCORCH_HIP_API int scorch_hip_spmm_csr_tiled_recommended(int64_t M, int64_t K, i
  * (listed_vals[e] = vals[position of list entry e]); handed to the listed kernel as `listed_vals`
  * they are read with the entries, coalesced, instead of one scattered load per entry (mask_vals is
  * then not read).  The copy is the caller's to redo when the values change.  listed_vals may be
- * NULL, and so may mask_vals (a mask of ones). */
+ * NULL, and so may mask_vals (a mask of ones).
+ * scorch_hip_sddmm_csr_lists_recommended is 1 where the lists pay for a mask that comes back. */
+SCORCH_HIP_API int scorch_hip_sddmm_csr_lists_recommended(int64_t n_cols, int64_t K, int64_t nnz);
 SCORCH_HIP_API size_t scorch_hip_sddmm_csr_lists_bytes(int64_t nnz);
 SCORCH_HIP_API int scorch_hip_sddmm_csr_lists(int64_t M, int64_t n_cols, int64_t nnz, const int32_t *row_ptr,
                                const int32_t *col_idx, void *lists, size_t lists_bytes, void *stream);

@@ -31,7 +31,6 @@ namespace {
 constexpr int kPlanWidths = 8;              // chunk boundaries kept for this many values of N
 constexpr int64_t kSoftmaxShortRow = 4096;  // rows up to this length: the one-launch softmax
 constexpr int64_t kFillFirstBytes = (int64_t)32 << 20;
-constexpr int64_t kListsMinDense = (int64_t)9 << 19, kListsMaxDense = (int64_t)20 << 20;
 
 struct Boundaries {
   int64_t N = -1;
@@ -152,9 +151,7 @@ int prepare_spmm(scorch_hip_csr_plan *plan, int64_t N, hipStream_t stream, Bound
 }
 
 bool sddmm_by_lists(const scorch_hip_csr_plan *plan, int64_t K) {
-  const int64_t dense = plan->n_cols * K * 4;
-  return K > 0 && K <= 256 && plan->nnz > 0 && dense >= kListsMinDense && dense <= kListsMaxDense &&
-         plan->nnz >= 4 * plan->n_cols;
+  return scorch_hip_sddmm_csr_lists_recommended(plan->n_cols, K, plan->nnz) != 0;
 }
 
 int prepare_sddmm(scorch_hip_csr_plan *plan, int64_t K, hipStream_t stream) {

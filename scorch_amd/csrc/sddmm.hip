@@ -483,8 +483,8 @@ __global__ __launch_bounds__(kBlockThreads) void sddmm_bucket_fill_kernel(
     }
   }
   // every entry's slot: the wavefront's entries keep their order inside a list, so that a row's
-  // entries stay next to each other there (its row of A is then kept in registers, and the
-  // entry's mask value and result lie next to its neighbours')
+  // entries stay next to each other there (its row of A is then staged in LDS once for all of them,
+  // and the entry's mask value and result lie next to its neighbours')
   int base[kBuckets];
   int start = 0;
 #pragma unroll
@@ -716,6 +716,16 @@ int scorch_hip_sddmm_csr_batched_f32(int64_t batch, int64_t M, int64_t n_cols, i
                                      void *stream) {
   return scorch::sddmm_entry<false>("scorch_hip_sddmm_csr_batched_f32", M, n_cols, K, nnz, row_ptr, col_idx,
                                     mask_vals, A, B, out_vals, out_row_idx, stream, batch);
+}
+
+// B beyond one L2 (4 MiB) and within the eight together, and its rows used often enough.  Where B is 4 MiB the plain kernel
+// is as fast (20,000 columns, 600 K entries, K = 50: 17.8 us, by lists 18.0), at 4.9 MiB it no longer is (4 M entries,
+// K = 64: 72.7 against 65.1; 6.1 MiB, 10 M entries, K = 16: 99 against 73).
+int scorch_hip_sddmm_csr_lists_recommended(int64_t n_cols, int64_t K, int64_t nnz) {
+  constexpr int64_t kLeastB = (int64_t)9 << 19, kMostB = (int64_t)20 << 20;  // bytes
+  if (K <= 0 || K > 256 || n_cols <= 0 || n_cols > kMostB) return 0;
+  const int64_t bytes = n_cols * K * (int64_t)sizeof(float);
+  return bytes >= kLeastB && bytes <= kMostB && nnz >= 4 * n_cols;
 }
 
 size_t scorch_hip_sddmm_csr_lists_bytes(int64_t nnz) {

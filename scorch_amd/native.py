@@ -119,6 +119,7 @@ SIGNATURES = {
     "scorch_hip_spmm_csr_batched_workspace_bytes": (_size, [_i64, _i64, _i64, _i64]),
     "scorch_hip_spmm_csr_batched_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _ptr,
                                                        _ptr, _size, _ptr, _size, _ptr]),
+    "scorch_hip_sddmm_csr_lists_recommended": (ctypes.c_int, [_i64, _i64, _i64]),
     "scorch_hip_sddmm_csr_lists_bytes": (_size, [_i64]),
     "scorch_hip_sddmm_csr_lists": (ctypes.c_int, [_i64, _i64, _i64, _ptr, _ptr, _ptr, _size, _ptr]),
     "scorch_hip_sddmm_csr_list_values_f32": (ctypes.c_int, [_i64, _ptr, _size, _ptr, _ptr, _ptr]),

@@ -1242,18 +1242,14 @@ prebuilt_spmv_csr_i64 = _make_spmv(torch.int64)
 
 
 SDDMM_PATHS = ("auto", "plain", "listed")
-# "auto": a CSR mask seen for the second time, with a dense right operand between 8 and 20 MB
-# (beyond one L2, within the eight together), is served from per-XCD entry lists; "plain" /
-# "listed" pin one path (SCORCH_HIP_SDDMM_PATH sets the default).
+# "auto": a CSR mask seen for the second time, where the library recommends it, is served from
+# per-XCD entry lists; "plain" / "listed" pin one path (SCORCH_HIP_SDDMM_PATH sets the default).
 SDDMM_PATH = os.environ.get("SCORCH_HIP_SDDMM_PATH", "auto")
 
 
 def _lists_apply(nnz: int, n_cols: int, K: int) -> bool:
-    """Whether SDDMMs of this shape are served from per-XCD entry lists when their mask comes back: B
-    beyond one L2 (4 MiB) and within the eight together, and used often enough.  Where B is 4 MiB the plain
-    kernel is as fast (20,000 columns, 600 K entries, K = 50: 17.8 us, by lists 18.0), at 4.9 MiB it no longer
-    is (4 M entries, K = 64: 72.7 against 65.1; 6.1 MiB, 10 M entries, K = 16: 99 against 73)."""
-    return 0 < K <= 256 and (9 << 19) <= n_cols * K * 4 <= (20 << 20) and nnz >= 4 * n_cols
+    """Whether SDDMMs of this shape are served from per-XCD entry lists when their mask comes back."""
+    return bool(native.lib().scorch_hip_sddmm_csr_lists_recommended(n_cols, K, nnz))
 
 
 def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int, L, stream) -> Optional[torch.Tensor]:

@@ -69,6 +69,26 @@ def test_abi_version(L):
     assert L.scorch_hip_abi_version() == int(m.group(1))
 
 
+@pytest.mark.parametrize("n_cols, K, nnz, want", [
+    (18_432, 64, 1 << 20, True), (18_431, 64, 1 << 20, False),                # B of 4.5 MiB
+    (81_920, 64, 1 << 20, True), (81_921, 64, 1 << 20, False),                # ... and of 20
+    (65_536, 32, 4 * 65_536, True), (65_536, 32, 4 * 65_536 - 1, False),      # four entries a column
+    (8192, 256, 1 << 20, True), (8192, 257, 1 << 20, False), (1 << 20, 0, 1 << 24, False), (0, 64, 0, False)])
+def test_where_the_lists_of_an_sddmm_pay_is_the_librarys_answer(L, monkeypatch, n_cols, K, nnz, want):
+    """One rule for the plan handle and for the package: the package asks the library."""
+    from scorch_amd import scorch_ops_hip as H
+    assert L.scorch_hip_sddmm_csr_lists_recommended(n_cols, K, nnz) == want
+    asked = []
+
+    class Other:
+        def scorch_hip_sddmm_csr_lists_recommended(self, *of):
+            asked.append(of)
+            return int(not want)
+
+    monkeypatch.setattr(native, "lib", Other)
+    assert H._lists_apply(nnz, n_cols, K) is not want and asked == [(n_cols, K, nnz)]
+
+
 def test_workspace_bytes_formula(L):
     f = L.scorch_hip_spmm_csr_workspace_bytes
     assert f(-1, 0, 4, 4) == 0 and f(4, 4, 4, 0) == 0
