@@ -294,7 +294,8 @@ SCORCH_HIP_API int scorch_hip_softmax_csr_f32(int64_t M, int64_t nnz, const int3
  *
  * The first product of a kind and width allocates device memory (hipMalloc: not under graph
  * capture); scorch_hip_csr_plan_prepare does that ahead of time, after which the product calls
- * of that kind and width allocate nothing and do not synchronise.  `width` is N for
+ * of that kind and width allocate nothing and do not synchronise.  (An SDDMM whose lists are
+ * not there goes without them under capture, and where there is no memory for them.)  `width` is N for
  * SCORCH_HIP_PLAN_SPMM_F32 and SCORCH_HIP_PLAN_SPMM_DENSE_F32, K for SCORCH_HIP_PLAN_SDDMM_F32
  * and ignored for SCORCH_HIP_PLAN_SOFTMAX_F32.  A plan holds boundaries for at most 8 widths of N; a ninth
  * replaces the oldest.

@@ -154,11 +154,20 @@ bool sddmm_by_lists(const scorch_hip_csr_plan *plan, int64_t K) {
   return scorch_hip_sddmm_csr_lists_recommended(plan->n_cols, K, plan->nnz) != 0;
 }
 
-int prepare_sddmm(scorch_hip_csr_plan *plan, int64_t K, hipStream_t stream) {
+// (`no_memory`, if given: set instead of an error where the lists' memory cannot be had)
+int prepare_sddmm(scorch_hip_csr_plan *plan, int64_t K, hipStream_t stream, bool *no_memory = nullptr) {
   if (K < 0) return fail(SCORCH_HIP_EINVAL, "scorch_hip_csr_plan: negative K");
   if (!sddmm_by_lists(plan, K) || plan->lists_built) return SCORCH_HIP_OK;
   const size_t bytes = scorch_hip_sddmm_csr_lists_bytes(plan->nnz);
-  SCORCH_HIP_CHECK(hipMalloc(&plan->lists, bytes));
+  if (const hipError_t err = hipMalloc(&plan->lists, bytes)) {
+    (void)hipGetLastError();  // (the next launch would report it as its own)
+    plan->lists = nullptr;
+    if (no_memory && err == hipErrorOutOfMemory) {
+      *no_memory = true;
+      return SCORCH_HIP_OK;
+    }
+    return fail(SCORCH_HIP_ERUNTIME, "scorch_hip_csr_plan: hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(err));
+  }
   plan->lists_bytes = bytes;
   if (int rc = scorch_hip_sddmm_csr_lists(plan->M, plan->n_cols, plan->nnz, plan->row_ptr, plan->col_idx,
                                           plan->lists, bytes, stream)) {
@@ -296,8 +305,19 @@ int scorch_hip_spmm_csr_plan_f32(scorch_hip_csr_plan *plan, int64_t N, const flo
 int scorch_hip_sddmm_csr_plan_f32(scorch_hip_csr_plan *plan, int64_t K, const float *mask_vals, const float *A,
                                   const float *B, float *out_vals, int32_t *out_row_idx, void *stream) {
   if (int rc = check_plan("scorch_hip_sddmm_csr_plan_f32", plan)) return rc;
-  if (int rc = prepare_sddmm(plan, K, static_cast<hipStream_t>(stream))) return rc;
-  if (sddmm_by_lists(plan, K))
+  if (K < 0) return fail(SCORCH_HIP_EINVAL, "scorch_hip_csr_plan: negative K");
+  // Without the lists the plain kernel gives the same bits: it serves a product that is being recorded before they are made
+  // (nothing can be allocated there), and one for whose lists there is no memory.
+  bool listed = sddmm_by_lists(plan, K);
+  if (listed && !plan->lists_built) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    SCORCH_HIP_CHECK(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture));
+    bool without = capture != hipStreamCaptureStatusNone;
+    if (!without)
+      if (int rc = prepare_sddmm(plan, K, static_cast<hipStream_t>(stream), &without)) return rc;
+    listed = !without;
+  }
+  if (listed)
     return scorch_hip_sddmm_csr_listed_f32(1, plan->M, plan->n_cols, K, plan->nnz, plan->lists, plan->lists_bytes,
                                            mask_vals, nullptr, A, B, out_vals, out_row_idx, stream);
   return scorch_hip_sddmm_csr_f32(plan->M, plan->n_cols, K, plan->nnz, plan->row_ptr, plan->col_idx, mask_vals, A, B,

@@ -697,7 +697,10 @@ def _listed_mask_values(values: torch.Tensor, lists: torch.Tensor, L, stream):
     seen = _kept(values, "_scorch_ones")
     if seen is None or seen[0] != key or seen[1] is not False:
         return values.data_ptr(), None          # not yet seen twice unchanged
-    listed = _empty_like(values)
+    try:
+        listed = _empty_like(values)
+    except torch.OutOfMemoryError:
+        return values.data_ptr(), None
     native.check(L.scorch_hip_sddmm_csr_list_values_f32(values.numel(), lists.data_ptr(), lists.numel(),
                                                         values.data_ptr(), listed.data_ptr(), stream))
     _made_on(stream, listed)
@@ -1268,7 +1271,13 @@ def _sddmm_lists(plan: Optional[CsrPlan], pos, crd, M: int, n_cols: int, K: int,
     if plan.sddmm_lists is None and torch.cuda.is_current_stream_capturing():
         return None
     if plan.sddmm_lists is None:
-        lists = _empty(L.scorch_hip_sddmm_csr_lists_bytes(crd.numel()), dtype=torch.uint8, device=pos.device)
+        try:
+            lists = _empty(L.scorch_hip_sddmm_csr_lists_bytes(crd.numel()), dtype=torch.uint8, device=pos.device)
+        except torch.OutOfMemoryError:
+            if SDDMM_PATH == "listed":
+                raise
+            plan.sddmm_uses = 0             # (asked for again two products on; the plain kernel needs none)
+            return None
         native.check(L.scorch_hip_sddmm_csr_lists(M, n_cols, crd.numel(), pos.data_ptr(), crd.data_ptr(),
                                                   lists.data_ptr(), lists.numel(), stream))
         _made_on(stream, lists)

@@ -154,6 +154,25 @@ def test_sddmm_through_a_plan(oracle):
     assert oracle.rel_fro(ones, oracle.sddmm_fp64(oracle.rows_of(rp), ci, np.ones_like(s), A, B)) <= TOL
 
 
+def test_an_sddmm_recorded_before_its_lists_are_made_goes_without_them():
+    """B of 4.9 MiB: a product of its own makes the lists; one that is recorded first cannot, and has the same bits."""
+    M, n_cols, K = 3000, 20_000, 64
+    w = workloads.sddmm_uniform(M=M, n_cols=n_cols, per_row=40, K=K, seed=6, unit_mask=False)
+    rp, ci, sv, A, B = (dev(w[name]) for name in ("row_ptr", "col_idx", "vals", "A", "B"))
+    with CsrPlanHandle(rp, ci, n_cols) as plan:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            recorded = plan.sddmm(sv, A, B)
+        assert plan.info()["device_bytes"] == 0
+        eager = plan.sddmm(sv, A, B)
+        assert plan.info()["device_bytes"] >= 12 * ci.numel()            # the lists
+        for factor in (1.0, 2.0, 0.5):
+            A.copy_(dev(w["A"]) * factor)
+            recorded.fill_(float("nan"))
+            graph.replay()
+            assert torch.equal(recorded, plan.sddmm(sv, A, B)) and torch.equal(recorded, eager * factor)
+
+
 @pytest.mark.parametrize("longest", [300, 9000])
 def test_softmax_through_a_plan(longest, oracle):
     rng = np.random.default_rng(longest)

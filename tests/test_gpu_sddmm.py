@@ -6,6 +6,8 @@ mask's own index tensors come back; for a CSR mask the result is the
 coordinate list (row of each entry, col_idx) in mask order, one entry per mask
 entry, explicit zeros kept.
 """
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -241,6 +243,33 @@ def test_auto_builds_the_lists_on_the_second_product_at_full_size(oracle):
     second = call()
     assert rp._scorch_plan.sddmm_lists is not None
     assert torch.equal(first, second) and torch.equal(second, call())
+
+
+@pytest.mark.parametrize("refused", ["lists", "values"])
+def test_without_memory_for_the_lists_the_plain_kernel_serves(refused, monkeypatch):
+    """The lists, and the values in their order, are memory that a product can do without."""
+    M, n_cols, K = 3000, 20_000, 64                              # B of 4.9 MiB
+    w = workloads.sddmm_uniform(M=M, n_cols=n_cols, per_row=40, K=K, seed=5, unit_mask=False)
+    rp, ci, sv, A, B = (dev(w[name]).reshape(-1) for name in ("row_ptr", "col_idx", "vals", "A", "B"))
+    call = lambda: H.sddmm_csr_float([M, n_cols], [M, n_cols], [[], [rp, ci]], sv, [M, K], [[], []], A, [n_cols, K],
+                                     [[], []], B).storage.value
+    first, refusals = call(), []
+    name, asker = {"lists": ("_empty", "_sddmm_lists"), "values": ("_empty_like", "_listed_mask_values")}[refused]
+    allocate = getattr(H, name)
+
+    def without_memory(*args, **kwargs):
+        if sys._getframe(1).f_code.co_name != asker:
+            return allocate(*args, **kwargs)
+        refusals.append(args)
+        raise torch.OutOfMemoryError("no memory, says the test")
+
+    with monkeypatch.context() as m:
+        m.setattr(H, name, without_memory)
+        assert all(torch.equal(call(), first) for _ in range(4)) and refusals
+        assert (rp._scorch_plan.sddmm_lists is None) == (refused == "lists")
+        assert getattr(sv, "_scorch_listed", None) is None
+    assert all(torch.equal(call(), first) for _ in range(4))     # ... and are made once there is memory again
+    assert rp._scorch_plan.sddmm_lists is not None and sv._scorch_listed is not None
 
 
 @pytest.mark.parametrize("mask_format", ["ds", "oo"])
