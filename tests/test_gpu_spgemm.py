@@ -508,6 +508,20 @@ def test_row_pointers_on_either_side_of_a_scans_tiles(oracle, M):
     check(oracle, arp, aci, rng.integers(-9, 9, aci.size).astype(np.int64), brp, bci, rng.integers(-9, 9, bci.size).astype(np.int64), 70)
 
 
+@pytest.mark.parametrize("M", [4096 * 4096 - 1, 4096 * 4096, 4096 * 4096 + 12_345])
+def test_row_pointers_on_either_side_of_4096_tiles(oracle, M):
+    """Beyond 4,096 tiles of 4,096 elements a launch of its own sums the tiles' totals: few entries, in rows all over the
+    matrix, the first and the last among them."""
+    rng = np.random.default_rng(M)
+    rows = np.unique(np.concatenate([[0, 4095, 4096, M - 2, M - 1], rng.integers(0, M, 200_000)]))
+    lens = np.zeros(M, dtype=np.int32)
+    lens[rows] = rng.integers(1, 4, rows.size)
+    arp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    aci = rng.integers(0, 50, arp[-1]).astype(np.int32)
+    brp, bci, bv = random_csr(rng, 50, 70, 0.1, empty_rows=(0, 49))
+    check(oracle, arp, aci, rng.integers(-9, 9, aci.size).astype(np.int64), brp, bci, rng.integers(-9, 9, bci.size).astype(np.int64), 70)
+
+
 @pytest.mark.parametrize("hubs, hub, N", [(1, 9000, 9000), (4, 3000, 20_000), (40, 1200, 60_000), (300, 300, 131_072)])
 def test_ranges_of_columns_of_every_width(oracle, hubs, hub, N):
     """Few long rows of many products take narrow ranges of columns and a window to a work item, many long rows wide ranges."""
