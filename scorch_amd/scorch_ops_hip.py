@@ -487,8 +487,11 @@ def _chunk_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, N: int, el
 BLOCKED_PATHS = ("auto", "off", "always")
 BLOCKED_PATH = os.environ.get("SCORCH_HIP_BLOCKED", "auto")
 # dense width -> share of the active blocks' positions that must be stored for the block kernels to
-# be the faster ones (measured on uniformly filled 4,096 x 4,096 masks, 8 heads: the general
-# kernels' time grows with the entries, the block kernels' with the blocks)
+# be taken: about where the SDDMM's is the faster one (uniformly filled 4,096 x 4,096 masks, 8 heads, us, general
+# against blocks: 137 / 133 at 0.15 and width 32, 215 / 211 at 0.15 and 64, 295 / 350 at 0.12 and 371 / 350 at 0.15
+# and 128; the general kernels' time grows with the entries, the block kernels' with the blocks).  The SpMM's line
+# was near it against the merge-path kernels; against the panels, which masks of about equal rows now go to, it lies
+# higher: 113 / 156 and 214 / 229 at 0.3, 371 / 378 at 0.25
 BLOCKED_MIN_FILL = {32: 0.17, 64: 0.15, 128: 0.12}
 BLOCKED_WIDTHS = tuple(BLOCKED_MIN_FILL)
 BLOCKED_STRETCH = 16         # blocks per work item at most
