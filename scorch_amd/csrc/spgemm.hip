@@ -1296,16 +1296,20 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_huge_kernel(
 // row's first kAccEntries output entries (the others are added into the output
 // with global atomics as above).
 constexpr int kLdsBudget = 160 * 1024 - 1024;
+// The tier of up to kMediumProducts products: with 16-bit ranks, and sums of the last hundred of the longest rows in the
+// output, four workgroups of eight wavefronts fill a CU (256 threads, four of four, 2,600 rows: 67 us, 512 60).
+constexpr int kBitmapThreads = 512, kBitmapSums = 3968;
 
 // THREADS: workgroup size.  ACC: LDS sums to provide (0: all the LDS that is left).
 // LIST, WORK: which of the counters holds the length of `rows` and the next row to hand out.
 template <typename A, bool NUMERIC, int WORDS, int THREADS, int ACC>
 struct BitmapTables {
   static constexpr int kGroups = WORDS / 4;
-  static constexpr int kFixed = WORDS * 4 + (NUMERIC ? kGroups * 4 : 0) + (int)sizeof(ProductBatch<THREADS, A>) + 512;
+  using Rank = std::conditional_t<(ACC > 0), unsigned short, int>;  // (ACC: of rows with at most kMediumProducts columns)
+  static constexpr int kFixed = WORDS * 4 + (NUMERIC ? kGroups * (int)sizeof(Rank) : 0) + (int)sizeof(ProductBatch<THREADS, A>) + 512;
   static constexpr int kAccEntries = !NUMERIC ? 1 : ACC > 0 ? ACC : (kLdsBudget - kFixed) / (int)sizeof(A);
   alignas(16) unsigned bits[WORDS];
-  int rank[NUMERIC ? kGroups : 1];  // rank of the first column of every group of four words
+  Rank rank[NUMERIC ? kGroups : 1];  // rank of the first column of every group of four words
   A acc[kAccEntries];
   ProductBatch<THREADS, A> batch;
   int scan[THREADS / kWaveSize];
@@ -1409,7 +1413,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
                 __popc(s_bits[4 * g + 3]);
         int total = 0;
         const int at = block_exclusive_scan_n<kWaves>(cnt, s_scan, total);
-        if (NUMERIC && g < groups) s_rank[g] = n + at;
+        if (NUMERIC && g < groups) s_rank[g] = (typename Tables::Rank)(n + at);
         n += total;
       }
       if (NUMERIC && n > 0) {  // uniform
@@ -2204,8 +2208,8 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
       }
       if (bitmap_blocks && narrow) {
         // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
-        spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts, 0, 4>
-            <<<bitmap_blocks, kBlockThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
+        spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kBitmapThreads, kBitmapSums, 0, 4>
+            <<<bitmap_blocks, kBitmapThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
                                                           narrow_rows, ws.counters, c_pos, c_crd, c_val);
       } else if (bitmap_blocks) {
         // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit

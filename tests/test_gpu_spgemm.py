@@ -558,3 +558,23 @@ def test_products_of_rows_whose_entries_have_none_one_or_many(oracle, dtype, pro
     arp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
     value = (lambda n: rng.integers(-9, 9, n).astype(dtype)) if dtype == np.int64 else (lambda n: rng.uniform(-1, 1, n).astype(dtype))
     check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+@pytest.mark.parametrize("N", [70_001, 131_072])
+def test_rows_at_the_edges_of_the_tiers_of_a_large_matrix(oracle, dtype, N):
+    """Rows of as many distinct columns as a tier's tables hold, one fewer and one more (among them more than have sums in LDS
+    beside the bitmap), and clustered ones, in a matrix whose tiers are launched apart."""
+    M, lens = 32_768 + 5, [1, 31, 32, 33, 64, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2048, 3967, 3968, 3969, 4095, 4096]
+    rng = np.random.default_rng(N)
+    b_rows = [np.sort(rng.choice(N, n, replace=False)) for n in lens] + [np.arange(n) + 17 for n in lens]
+    brp = np.concatenate([[0], np.cumsum([len(r) for r in b_rows])]).astype(np.int32)
+    bci = np.concatenate(b_rows).astype(np.int32)
+    K = len(b_rows)
+    aci = (np.arange(M) % 3).astype(np.int32)                      # most rows: one short row of B
+    longer = rng.choice(M, 4 * K, replace=False)
+    aci[longer] = np.tile(np.arange(K), 4)
+    arp = np.arange(M + 1, dtype=np.int32)
+    draw = (lambda n: rng.integers(-9, 10, n).astype(dtype)) if np.issubdtype(dtype, np.integer) else \
+        (lambda n: (rng.random(n) + 0.5).astype(dtype))
+    check(oracle, arp, aci, draw(M), brp, bci, draw(len(bci)), N)
