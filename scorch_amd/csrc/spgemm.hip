@@ -1708,8 +1708,8 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
 // in LDS, by a workgroup that reads its runs from all of the row's windows: streams instead of
 // gathers, as many workgroups to a row as it has ranges, and a hub shared out by itself.
 // Both passes over these rows of a power-law graph squared (131,072 nodes, 16 entries a row, 19 M
-// products of this kind), fp32: 282 us (lists 17, sort 100, count 44, sums 121); the numeric pass alone took 512.  The sort is
-// bound by the gathers from B (a line for about two entries), the sums by LDS atomics.  (Ranges
+// products of this kind), fp32: 250 us (lists 17, sort 80, count 44, sums 111); the numeric pass alone took 512.  The sort is
+// bound by the gathers from B (a line for about two entries), the sums by a workgroup's chain of reads.  (Ranges
 // without the windows, each item bisecting the rows of B for its piece, fetch those lines once
 // per range: 411 us for the numeric pass alone.)
 // For products of up to kNarrowColumns columns whose two passes share what they find out.
@@ -1902,7 +1902,21 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
     for (int u = 0; u < U; ++u)
       if (step.first + u * kWaveSize + lane < step.last) {
         bin[u] = col[u] >> bins.shift;
-        rank[u] = atomicAdd(&s_count[bin[u]], 1);
+        // The wavefront's products of this range, and one add for all of them: 64 adds to some sixteen counters
+        // queue up in the LDS (kernel 99 -> 80 us: vector instructions instead, which had time).
+        unsigned long long alike = __ballot(true);
+#pragma unroll
+        for (int bit = 0; (1 << bit) < kMaxBins; ++bit) {
+          const int set = -((bin[u] >> bit) & 1);
+          const unsigned long long with = __ballot(set != 0);
+          const unsigned lo = (unsigned)alike & ~((unsigned)with ^ (unsigned)set);
+          const unsigned hi = (unsigned)(alike >> 32) & ~((unsigned)(with >> 32) ^ (unsigned)set);
+          alike = (unsigned long long)hi << 32 | lo;
+        }
+        const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(alike >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)alike, 0u));
+        int base = 0;
+        if (before == 0) base = atomicAdd(&s_count[bin[u]], __popcll(alike));
+        rank[u] = before + __shfl(base, __ffsll(alike) - 1);
       }
     __syncthreads();
     if (tid <= bins.n) {
@@ -2023,8 +2037,9 @@ template <typename T>
 __global__ __launch_bounds__(kBinSumThreads) void spgemm_bin_sums_kernel(Bins bins, const int *__restrict__ c_pos,
                                                                          int *__restrict__ c_crd, T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
-  constexpr int kWaves = kBinSumThreads / kWaveSize;
-  __shared__ A s_sum[kBinColumns];
+  constexpr int kWaves = kBinSumThreads / kWaveSize, kFour = (int)(16 / sizeof(A));
+  static_assert(2 * kBinColumns / 32 <= kBinSumThreads, "a thread to half a word of the bitmap");
+  alignas(16) __shared__ A s_sum[kBinColumns];
   __shared__ unsigned s_bits[kBinColumns / 32];
   __shared__ int s_rank[kBinColumns / 32];
   __shared__ int s_scan[kWaves];
@@ -2034,7 +2049,7 @@ __global__ __launch_bounds__(kBinSumThreads) void spgemm_bin_sums_kernel(Bins bi
   const int n = counts[bin];
   const BinRow r = bins.row[idx];
   const int windows = (int)(bins.used[idx] >> 32), columns = 1 << bins.shift, words = columns / 32;
-  for (int i = tid; i < columns; i += kBinSumThreads) s_sum[i] = (A)0;
+  for (int i = tid; i < columns / kFour; i += kBinSumThreads) reinterpret_cast<uint4 *>(s_sum)[i] = make_uint4(0u, 0u, 0u, 0u);
   for (int i = tid; i < words; i += kBinSumThreads) s_bits[i] = 0u;
   int out = c_pos[r.row];
   for (int i = 0; i < bin; ++i) out += counts[i];
@@ -2059,20 +2074,19 @@ __global__ __launch_bounds__(kBinSumThreads) void spgemm_bin_sums_kernel(Bins bi
   });
   __syncthreads();
   int unused = 0;
-  const int rank = block_exclusive_scan_n<kWaves>(tid < words ? __popc(s_bits[tid]) : 0, s_scan, unused);
+  const unsigned half = tid < 2 * words ? (s_bits[tid >> 1] >> (16 * (tid & 1))) & 0xffffu : 0u;
+  const int rank = block_exclusive_scan_n<kWaves>(__popc(half), s_scan, unused);
   const int first_column = bin << bins.shift;
-  if (4 * n < columns) {  // a thread per word of the bitmap
-    if (tid < words) {
-      int at = out + rank;
-      for (unsigned bits = s_bits[tid]; bits; bits &= bits - 1, ++at) {
-        const int col = tid * 32 + __ffs(bits) - 1;
-        c_crd[at] = first_column + col;
-        c_val[at] = (T)s_sum[col];
-      }
+  if (4 * n < columns) {  // a thread per half word of the bitmap (per word, and cleared four bytes at a time: 120 us, 111)
+    int at = out + rank;
+    for (unsigned bits = half; bits; bits &= bits - 1, ++at) {
+      const int col = tid * 16 + __ffs(bits) - 1;
+      c_crd[at] = first_column + col;
+      c_val[at] = (T)s_sum[col];
     }
     return;
   }
-  if (tid < words) s_rank[tid] = rank;
+  if (tid < 2 * words && !(tid & 1)) s_rank[tid >> 1] = rank;
   __syncthreads();
   // two bitmap words, 64 columns, per wavefront and step
   for (int w = 2 * (tid / kWaveSize); w < words; w += 2 * kWaves) {
