@@ -429,10 +429,10 @@ constexpr int kScanTile = kBlockThreads * kScanPerThread;
 // counters: [0] medium rows, [1] huge rows, [2] small rows, [5] giant rows listed; [3], [4] next row to hand out;
 // [6] (64 bits) the number of entries of the result; [8] rows shared out, [9] their slices; [10] (64 bits) the giant
 // rows' products; [12] (64 bits) the products of all rows beyond kMediumProducts, and [14] their batches of kBinEntries
-// entries; [15] workgroups of pass 0 that are through; [16..18] the bins' totals (Bins)
+// entries; [15] workgroups of pass 0 that are through; [16..20] the bins' totals (Bins)
 // Every counter has a 128-byte line of its own: atomics on one line follow one another at 12 ns each, whatever
 // they address (512 workgroups with eight counts each: 71 us on one line).
-constexpr int kSpgemmCounters = 20;
+constexpr int kSpgemmCounters = 22;
 __host__ __device__ constexpr int counter(int i) { return 32 * i; }
 constexpr int kBinEntries = 512;
 
@@ -1708,7 +1708,7 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_split_emit_kernel(
 // in LDS, by a workgroup that reads its runs from all of the row's windows: streams instead of
 // gathers, as many workgroups to a row as it has ranges, and a hub shared out by itself.
 // Both passes over these rows of a power-law graph squared (131,072 nodes, 16 entries a row, 19 M
-// products of this kind), fp32: 250 us (lists 17, sort 80, count 44, sums 111); the numeric pass alone took 512.  The sort is
+// products of this kind), fp32: 240 us (lists 17, sort 80, count 34, sums 111); the numeric pass alone took 512.  The sort is
 // bound by the gathers from B (a line for about two entries), the sums by a workgroup's chain of reads.  (Ranges
 // without the windows, each item bisecting the rows of B for its piece, fetch those lines once
 // per range: 411 us for the numeric pass alone.)
@@ -1719,6 +1719,7 @@ constexpr int kBinShare = 4 * kBinProducts;    // products of a batch of entries
 constexpr int64_t kBinManyProducts = (int64_t)512 * kBinShare;
 constexpr int kBinColumns = 8192;              // most columns to a range; a power of two
 constexpr int kMaxBins = 32;
+constexpr int kHubProducts = 4 * kGiantProducts;
 static_assert(kMaxBins * kBinColumns >= kNarrowColumns, "the widest B in ranges of the most columns");
 constexpr int64_t kBinBudget = (int64_t)4 << 30;
 
@@ -1735,9 +1736,11 @@ struct BinItem {
 
 struct Bins {
   int shift = 0, n = 0;                 // ranges of 2^shift columns, n of them; n 0: not used
+  int giant = 0;                        // rows of kGiantProducts products and more: they come first, the longest of them before the others
+  int counted_wide = 0;                 // the first rows, whose ranges are counted by a workgroup each, the others' by a wavefront
   int share = kBinShare;                // products of a batch of entries to a workgroup
   int64_t rows = 0, items = 0;
-  int *totals;                          // products, windows, items handed out to rows so far (counters of pass 0)
+  int *totals;                          // products, windows, items and places handed out to rows so far (counters of pass 0)
   BinRow *row;
   unsigned long long *used;             // per row: windows (upper half) and products written
   BinItem *item;
@@ -1748,7 +1751,8 @@ struct Bins {
   size_t total = 0;
 };
 
-inline Bins spgemm_bins(char *base, int *counters, int64_t N, size_t elem, int64_t rows, int64_t products, int64_t batches) {
+inline Bins spgemm_bins(char *base, int *counters, int64_t N, size_t elem, int64_t rows, int64_t giant, int64_t products,
+                        int64_t batches) {
   Bins b;
   if (rows == 0 || N > kNarrowColumns || products * (int64_t)(2 + elem) > kBinBudget || products > INT32_MAX / 2) return b;
   // Narrow ranges while that makes workgroups the chip has room for, of 512 products and more (45,000 nodes of 11, ranges of
@@ -1761,6 +1765,9 @@ inline Bins spgemm_bins(char *base, int *counters, int64_t N, size_t elem, int64
     ++b.shift;
   b.n = (int)((N + (1 << b.shift) - 1) >> b.shift);
   b.rows = rows;
+  b.giant = (int)giant;
+  // (Where workgroups for all of them fit the chip, a wavefront's chain is the longer one: 2,500 to 9,800 nodes, the whole product 82 -> 86 us.)
+  b.counted_wide = (int)(rows * b.n <= 2048 ? rows : giant);
   // (21,648 rows of 7: 120 workgroups that make four windows one after the other 18 us, of one window each 8.4)
   if (products < kBinManyProducts) b.share = kBinProducts;
   b.items = batches + products / b.share;
@@ -1784,7 +1791,8 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bin_rows_kernel(int M, B
                                                                         const int *__restrict__ huge_rows,
                                                                         const int *__restrict__ counters,
                                                                         int *__restrict__ c_pos) {
-  __shared__ int s_scan[kWavesPerBlock], s_base[3];
+  constexpr int kWants = 4;
+  __shared__ int s_scan[kWavesPerBlock], s_base[kWants + 1];
   const int64_t i = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x;
   const bool mine = i < bins.rows;
   BinRow r = {};
@@ -1795,21 +1803,26 @@ __global__ __launch_bounds__(kBlockThreads) void spgemm_bin_rows_kernel(int M, B
     r.batches = (a_pos[r.row + 1] - a_pos[r.row] + kBinEntries - 1) / kBinEntries;
     r.items = r.batches + p / bins.share;  // at most
   }
-  const int want[3] = {p, mine ? p / kBinProducts + r.batches : 0, r.items};
-  int at[3];
+  // A workgroup takes a range of a row, and the longest rows decide when the counts and sums end: they go first.
+  const bool hub = p >= kHubProducts, giant = i < bins.giant && mine;
+  const int want[kWants] = {p, mine ? p / kBinProducts + r.batches : 0, r.items, hub ? 1 << 16 : giant ? 1 : 0};
+  int at[kWants];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
+  for (int k = 0; k < kWants; ++k) {
     int total = 0;
     at[k] = block_exclusive_scan(want[k], s_scan, total);
-    if (threadIdx.x == (unsigned)k) s_base[k] = atomicAdd(bins.totals + counter(k), total);
+    if (threadIdx.x == (unsigned)k && k < 3) s_base[k] = atomicAdd(bins.totals + counter(k), total);
+    if (k == 3 && threadIdx.x == 3) s_base[3] = total >> 16 ? atomicAdd(bins.totals + counter(3), total >> 16) : 0;
+    if (k == 3 && threadIdx.x == 4) s_base[4] = total & 0xffff ? atomicAdd(bins.totals + counter(4), total & 0xffff) : 0;
   }
   __syncthreads();
   if (!mine) return;
   r.first_product = s_base[0] + at[0];
   r.first_window = s_base[1] + at[1];
   r.first_item = s_base[2] + at[2];
-  bins.row[i] = r;
-  bins.used[i] = 0;
+  const int64_t place = hub ? s_base[3] + (at[3] >> 16) : giant ? bins.giant - 1 - (s_base[4] + (at[3] & 0xffff)) : i;
+  bins.row[place] = r;
+  bins.used[place] = 0;
   c_pos[r.row] = 0;
 }
 
@@ -1948,7 +1961,7 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
 // time by each of WAVES wavefronts, lane i < here has the i-th's ends.
 template <int WAVES, typename Fn>
 __device__ __forceinline__ void for_each_runs(const Bins &bins, const BinRow &r, int windows, int bin, Fn fn) {
-  const int lane = wave_lane(), w = threadIdx.x / kWaveSize;
+  const int lane = wave_lane(), w = WAVES == 1 ? 0 : threadIdx.x / kWaveSize;
   for (int base = w; base < windows; base += WAVES * kWaveSize) {
     int first = 0, last = 0;
     if (base + lane * WAVES < windows) {
@@ -1972,14 +1985,46 @@ __device__ __forceinline__ void for_each_binned(const Bins &bins, const BinRow &
   });
 }
 
-constexpr int kBinCountThreads = 256;
+// Rows of kGiantProducts products and more: a workgroup to a range; the others: a wavefront to a range, eight of them to a
+// workgroup (131,072 nodes, 16 a row: a workgroup of 256 to every range 44 us; with 512 threads for the longest rows, which are
+// what the launch waits for, those first, and wavefronts for the others 34).
+constexpr int kBinCountThreads = 512;
 __global__ __launch_bounds__(kBinCountThreads) void spgemm_bin_count_kernel(Bins bins, int *__restrict__ c_pos) {
   constexpr int kWaves = kBinCountThreads / kWaveSize;
-  __shared__ unsigned s_bits[kBinColumns / 32];
+  __shared__ unsigned s_all_bits[kWaves][kBinColumns / 32];
   __shared__ int s_scan[kWaves];
+  const int words = (1 << bins.shift) / 32;
+  if (blockIdx.x >= (unsigned)bins.counted_wide * (unsigned)bins.n) {
+    const unsigned groups = (unsigned)(bins.n + kWaves - 1) / kWaves, at = blockIdx.x - (unsigned)bins.counted_wide * (unsigned)bins.n;
+    const int idx = bins.counted_wide + (int)(at / groups), w = uniform((int)threadIdx.x / kWaveSize), bin = (int)(at % groups) * kWaves + w;
+    if (bin >= bins.n) return;
+    unsigned *const bits = s_all_bits[w];
+    const BinRow r = bins.row[idx];
+    const int windows = (int)(bins.used[idx] >> 32);
+    for (int i = wave_lane(); i < words; i += kWaveSize) bits[i] = 0u;
+    wave_lds_sync();
+    for_each_binned<1>(bins, r, windows, bin, [&](int p, int to) {
+      int c[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) c[u] = p + u * kWaveSize < to ? bins.columns[p + u * kWaveSize] : -1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (c[u] >= 0) atomicOr(&bits[c[u] >> 5], 1u << (c[u] & 31));
+    });
+    wave_lds_sync();
+    int mine = 0;
+    for (int i = wave_lane(); i < words; i += kWaveSize) mine += __popc(bits[i]);
+    mine = team_inclusive_sum<kWaveSize>(mine);
+    if (wave_lane() == kWaveSize - 1) {
+      bins.counts[(size_t)idx * bins.n + bin] = mine;
+      if (mine) atomicAdd(&c_pos[r.row], mine);
+    }
+    return;
+  }
+  unsigned *const s_bits = s_all_bits[0];
   const int idx = (int)(blockIdx.x / (unsigned)bins.n), bin = (int)(blockIdx.x % (unsigned)bins.n);
   const BinRow r = bins.row[idx];
-  const int windows = (int)(bins.used[idx] >> 32), words = (1 << bins.shift) / 32;
+  const int windows = (int)(bins.used[idx] >> 32);
   for (int i = threadIdx.x; i < words; i += kBinCountThreads) s_bits[i] = 0u;
   __syncthreads();
   // Four runs of a wavefront's at a time, of clamped places (a load behind a condition is waited for before the next, and four
@@ -2341,7 +2386,7 @@ int spgemm_numeric_entry(const char *fn, int64_t M, int64_t K, int64_t N, const 
   if (report) {
     known = report_of(report);
     if (bin_memory) bins = spgemm_bins(static_cast<char *>(bin_memory), ws.counters, N, sizeof(T), known.huge + known.giant,
-                                       known.products, known.batches);
+                                       known.giant, known.products, known.batches);
     if (bins.total > bin_bytes)
       return fail(SCORCH_HIP_EWORKSPACE, "%s: bins of %zu bytes needed, %zu given", fn, bins.total, bin_bytes);
   }
@@ -2367,7 +2412,7 @@ int spgemm_symbolic_entry(const char *fn, int64_t M, int64_t K, int64_t N, const
   const SpgemmWorkspace ws = spgemm_layout(static_cast<char *>(workspace), M, N, sizeof(T));
   Bins bins;
   if (bin_memory) bins = spgemm_bins(static_cast<char *>(bin_memory), ws.counters, N, sizeof(T), known.huge + known.giant,
-                                     known.products, known.batches);
+                                     known.giant, known.products, known.batches);
   if (bins.total > bin_bytes)
     return fail(SCORCH_HIP_EWORKSPACE, "%s: bins of %zu bytes needed, %zu given", fn, bins.total, bin_bytes);
   SyncCall sync;
@@ -2380,7 +2425,9 @@ int spgemm_symbolic_entry(const char *fn, int64_t M, int64_t K, int64_t N, const
     SCORCH_HIP_CHECK(hipGetLastError());
     spgemm_bin_kernel<T><<<(unsigned)bins.items, kBinThreads, 0, s>>>(bins, a_pos, a_crd, a_val, b_pos, b_crd, b_val);
     SCORCH_HIP_CHECK(hipGetLastError());
-    spgemm_bin_count_kernel<<<(unsigned)(bins.rows * bins.n), kBinCountThreads, 0, s>>>(bins, c_pos);
+    constexpr int kWaves = kBinCountThreads / kWaveSize;
+    const int64_t count_blocks = (int64_t)bins.counted_wide * bins.n + (bins.rows - bins.counted_wide) * ((bins.n + kWaves - 1) / kWaves);
+    spgemm_bin_count_kernel<<<(unsigned)count_blocks, kBinCountThreads, 0, s>>>(bins, c_pos);
     SCORCH_HIP_CHECK(hipGetLastError());
   }
   if (int rc = spgemm_run<float, false>((int)M, (int)N, a_pos, a_crd, nullptr, b_pos, b_crd, nullptr, c_pos, nullptr, nullptr, ws,
@@ -2448,7 +2495,7 @@ int scorch_hip_spgemm_csr_symbolic_planned_begin(int64_t M, int64_t K, int64_t N
   if (int rc = sync.wait(fn, s, words, 6)) return rc;  // (the short rows' kernels are still at work)
   for (int i = 0; i < 4; ++i) report[1 + i] = words[i];
   report[7] = words[4], report[8] = words[5];
-  *bin_bytes = spgemm_bins(nullptr, nullptr, N, elem_size, words[2] + words[3], words[4], words[5]).total;
+  *bin_bytes = spgemm_bins(nullptr, nullptr, N, elem_size, words[2] + words[3], words[3], words[4], words[5]).total;
   return SCORCH_HIP_OK;
 }
 
