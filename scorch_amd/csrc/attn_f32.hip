@@ -405,47 +405,46 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_kernel(
 // Bound: a wavefront's chain of reads (work item, block, mask words, K: about 4 us of launches of 6 to 20), then a SIMD's matrix
 // and vector instructions, which hardly overlap: 1,024 and about 400 clocks a tile.  See team_wavefronts for what it takes.
 template <int D, int SPLIT>
-__global__ __launch_bounds__(kBlockThreads)
-__attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kernel(
-    int S, int n_blocks, int n_heads, const int *__restrict__ block_row_ptr,
+struct TeamTables {
+  static constexpr int kQueries = 16, kTeams = kWavesPerBlock / SPLIT;  // queries to a team of SPLIT wavefronts; teams
+  static constexpr int kBlocksAtOnce = 16;                              // 64 tiles: one to a lane
+  static constexpr int kOthers = SPLIT > 1 ? SPLIT - 1 : 1;
+  unsigned long long words[kTeams][kBlocksAtOnce][kQueries];
+  int col[kBlocksAtOnce];
+  alignas(16) float sums[SPLIT > 1 ? kTeams : 1][kOthers][SPLIT > 1 ? kQueries : 1][D + 4];
+  unsigned flags[SPLIT > 1 ? kTeams : 1][kOthers][3][kWaveSize];
+};
+
+// Of a head's work item number `item`, the queries of the `quarter`-th of SPLIT workgroups.
+template <int D, int SPLIT>
+__device__ __forceinline__ void team_rows(
+    TeamTables<D, SPLIT> &lds, int head, int item_at, int quarter, int S, int n_blocks, const int *__restrict__ block_row_ptr,
     const int *__restrict__ block_col_idx, const int *__restrict__ block_mask_index,
     const unsigned long long *__restrict__ block_masks,
     const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float scale_log2e,
-    float *__restrict__ O, int n_items, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
-  constexpr int kQueries = 16, kTeams = kWavesPerBlock / SPLIT;  // queries to a team of SPLIT wavefronts; teams
+    float *__restrict__ O, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
+  using Tables = TeamTables<D, SPLIT>;
+  constexpr int kQueries = Tables::kQueries, kTeams = Tables::kTeams, kBlocksAtOnce = Tables::kBlocksAtOnce, kOthers = Tables::kOthers;
   constexpr int kSlabs = D / 16, kFeat = D / 16;
   constexpr int VW = D == 32 ? 2 : 4, NH = kFeat / VW;
-  constexpr int kBlocksAtOnce = 16;                           // 64 tiles: one to a lane
-  constexpr int kStride = D + 4;
-  constexpr int kOthers = SPLIT > 1 ? SPLIT - 1 : 1;
-  __shared__ unsigned long long s_words[kTeams][kBlocksAtOnce][kQueries];
-  __shared__ int s_col[kBlocksAtOnce];
-  __shared__ __attribute__((aligned(16))) float s_sums[SPLIT > 1 ? kTeams : 1][kOthers][SPLIT > 1 ? kQueries : 1][kStride];
-  __shared__ unsigned s_flags[SPLIT > 1 ? kTeams : 1][kOthers][3][kWaveSize];
+  auto &s_words = lds.words;
+  auto &s_col = lds.col;
+  auto &s_sums = lds.sums;
+  auto &s_flags = lds.flags;
 
   const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), w = uniform(tid / kWaveSize);
   const int team = w / SPLIT, part = w % SPLIT;
   const int g = lane >> 4, n = lane & 15;
-  int head, rank;
-  const int ranks = n_items * SPLIT;
-  if (n_heads % 8 == 0) {  // a head's workgroups on one XCD, as above
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    head = xcd + 8 * (slot / ranks);
-    rank = slot % ranks;
-  } else {
-    head = blockIdx.x / ranks;
-    rank = blockIdx.x % ranks;
-  }
-  const int sub = rank % SPLIT * kTeams + team;  // sixteen queries of the block row
+  const int sub = quarter * kTeams + team;  // sixteen queries of the block row
   int qb, kb_begin, kb_end, part_slot = -1;
   if (items) {
-    const int4 item = items[rank / SPLIT];
+    const int4 item = items[item_at];
     qb = uniform(item.x);
     kb_begin = uniform(item.y);
     kb_end = uniform(item.z);
     part_slot = uniform(item.w);
   } else {
-    qb = n_blocks - 1 - rank / SPLIT;
+    qb = n_blocks - 1 - item_at;
     kb_begin = block_row_ptr[qb];
     kb_end = block_row_ptr[qb + 1];
   }
@@ -599,7 +598,7 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kerne
       if (it < kb_end) {
         const int mask_at = block_mask_index ? block_mask_index[it] : -1;
         if (tid % kQueries == 0) s_col[i] = block_col_idx[it];
-        const unsigned long long *words = block_masks + (size_t)mask_at * kBlock + rank % SPLIT * kTeams * kQueries + tid % kQueries;
+        const unsigned long long *words = block_masks + (size_t)mask_at * kBlock + quarter * kTeams * kQueries + tid % kQueries;
 #pragma unroll
         for (int p = 0; p < kTeams; ++p) word[p] = mask_at >= 0 ? words[p * kQueries] : ~0ull;
       }
@@ -708,6 +707,54 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kerne
     }
 }
 
+// WIDE: the first n_wide items are four workgroups' each, whatever SPLIT: where a few of the items are stretches of a shared-out row, that
+// is a row with a query that attends to everything, and the sixteen queries with it have all of the stretch's tiles, the others
+// next to none.  A wavefront for the sixteen was what launches waited for.  Window of 64 and a global token, us before and now:
+// (3,001 tokens, 8 heads, D = 64) 24.9, 22.4; (4,500, 12, 64) 59.1, 38.4; (8,192, 16, 64) 87.4, 75.8; (2,198, 4, 128) 30.5, 24.3;
+// (2,048, 12, 128) 45.0, 38.9; (6,075, 16, 32) 47.1, 41.5.  (In the same kernel without any: 52.3 -> 53.2 for a window of 256, so it is one of its own.)
+template <int D, int SPLIT, bool WIDE>
+__global__ __launch_bounds__(kBlockThreads)
+__attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kernel(
+    int S, int n_blocks, int n_heads, const int *__restrict__ block_row_ptr,
+    const int *__restrict__ block_col_idx, const int *__restrict__ block_mask_index,
+    const unsigned long long *__restrict__ block_masks,
+    const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float scale_log2e,
+    float *__restrict__ O, int n_items, int n_wide, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
+  __shared__ union {
+    TeamTables<D, SPLIT> usual;
+    TeamTables<D, WIDE ? 4 : SPLIT> wide;
+  } lds;
+  // First, of every head, a quarter of the wide items and all of the others, and at the end of the launch the wide ones' other quarters,
+  // of which most have nothing to do.  (The four of an item one after the other: an XCD's workgroups go to its four shader
+  // engines in turn, and one engine got all the long ones; a head's at the end of the head: workgroups with nothing to do
+  // took the places of others.)
+  const int first = WIDE ? n_wide + (n_items - n_wide) * SPLIT : n_items * SPLIT;
+  int id = blockIdx.x, ranks = first, quarter = 0;
+  if (WIDE && id >= n_heads * first) {
+    id -= n_heads * first;
+    ranks = 3 * n_wide;
+    quarter = 1;
+  }
+  int head, rank;
+  if (n_heads % 8 == 0) {  // a head's workgroups on one XCD, as above
+    const int xcd = id & 7, slot = id >> 3;
+    head = xcd + 8 * (slot / ranks);
+    rank = slot % ranks;
+  } else {
+    head = id / ranks;
+    rank = id % ranks;
+  }
+  if (WIDE && (quarter > 0 || rank < n_wide)) {
+    quarter += rank / n_wide;
+    team_rows<D, WIDE ? 4 : SPLIT>(lds.wide, head, rank % n_wide, quarter, S, n_blocks, block_row_ptr, block_col_idx, block_mask_index,
+                                   block_masks, Q, K, V, scale_log2e, O, items, n_slots, partials);
+    return;
+  }
+  if (WIDE) rank -= n_wide;
+  team_rows<D, SPLIT>(lds.usual, head, (WIDE ? n_wide : 0) + rank / SPLIT, rank % SPLIT, S, n_blocks, block_row_ptr, block_col_idx,
+                      block_mask_index, block_masks, Q, K, V, scale_log2e, O, items, n_slots, partials);
+}
+
 // Combines the stretches of a block row that was shared out: with m* the largest of the
 // stretches' reference maxima, O = sum_p 2^(m_p - m*) O_p / sum_p 2^(m_p - m*) l_p.
 // One workgroup per (split row, head); thread t takes query t / 4 and a quarter of the features.
@@ -745,18 +792,19 @@ __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, in
 
 // Wavefronts to sixteen queries in attn_f32_tiles_kernel for masks whose blocks are live in part, 0: the other kernel.
 // As many as leave every workgroup a place at once (four to a CU, two for D = 128); what is longer than that goes best with one,
-// and with D = 32, whose tiles are half as long as the reads in front of them, by the other kernel.  Windows of 64 and a
-// global token, (tokens, heads, D, workgroups of a block row): the other kernel, 1, 2 and 4 wavefronts, us:
+// and with D = 32, whose tiles are half as long as the reads in front of them, by the other kernel unless a few long rows are
+// shared out (causal, 2,048 tokens, 16 heads, D = 32: 61 us for 68; window and a global token, 6,075 tokens: 47 for 41).  Windows of 64 and a
+// global token, (tokens, heads, D, workgroups of a block row): the other kernel, 1, 2 and 4 wavefronts, us, all without WIDE:
 //   (300, 4, 64, 20) 10.8, 11.1, 8.2, 6.6     (2,048, 4, 64, 176) 19.0, 18.5, 15.3, 13.4   (960, 16, 64, 288) 23.6, 22.8, 19.5, 19.5
 //   (3,001, 8, 64, 464) 24.6, 23.7, 23.1, 26.5   (2,048, 16, 64, 704) 31.8, 30.3, 30.4, 33.8   (8,192, 16, 64, 2,288) 92.6, 90.2, 92.1, 111
 //   (1,472, 8, 32, 224) 13.4, 14.0, 11.9, 11.0   (2,944, 12, 32, 684) 20.0, 22.3, 20.8, 24.0   (6,141, 16, 32, 1,904) 43.6, 44.4, 44.5, 51.0
 //   (7,744, 1, 128, 151) 30.8, 30.1, 23.8, 22.4   (2,048, 12, 128, 468) 45.0, 43.2, 45.9, 54.2   (4,992, 16, 128, 1,392) 130, 109, 113, 133
 // (Whole blocks: 13.5 for 15.9 at (1,024, 8, 64, 128), but 13.8 for 11.6 at (4,096, 1, 64, 254); they stay with the other kernel.)
-inline int team_wavefronts(int D, unsigned workgroups) {
+inline int team_wavefronts(int D, unsigned workgroups, bool few_stretches) {
   const unsigned places = D == 128 ? 160 : 320;
   if (workgroups <= places) return 4;
   if (workgroups <= 2 * places - 64) return 2;
-  return D == 32 || workgroups > INT32_MAX / 4 ? 0 : 1;
+  return (D == 32 && !few_stretches) || workgroups > INT32_MAX / 16 ? 0 : 1;
 }
 
 template <int D>
@@ -766,10 +814,15 @@ static int launch(dim3 grid, hipStream_t s, int S, int n_blocks, int H, const in
                   const float *k, const float *v, float scale_log2e, float *o, int n_items, const int4 *items, int n_slots, float *partials,
                   int n_split_rows, const int4 *split_rows) {
   mark_launch(s);
-  if (const int split = block_mask_index ? team_wavefronts(D, grid.x) : 0; split && (int64_t)S * D * 4 < INT32_MAX) {
-    auto kernel = split == 4 ? &attn_f32_tiles_kernel<D, 4> : split == 2 ? &attn_f32_tiles_kernel<D, 2> : &attn_f32_tiles_kernel<D, 1>;
-    kernel<<<dim3(grid.x * split), kBlockThreads, 0, s>>>(
-        S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index, block_masks, q, k, v, scale_log2e, o, n_items, items,
+  const bool few_stretches = items && n_slots > 0 && 3 * (int64_t)n_slots <= n_items;  // (of a few long rows: see the tiles' kernel)
+  if (const int split = block_mask_index ? team_wavefronts(D, grid.x, few_stretches) : 0; split && (int64_t)S * D * 4 < INT32_MAX) {
+    const bool wide = split < 4 && few_stretches;
+    const int n_wide = wide ? n_slots : 0;
+    auto kernel = split == 4   ? &attn_f32_tiles_kernel<D, 4, false>
+                  : split == 2 ? (wide ? &attn_f32_tiles_kernel<D, 2, true> : &attn_f32_tiles_kernel<D, 2, false>)
+                               : (wide ? &attn_f32_tiles_kernel<D, 1, true> : &attn_f32_tiles_kernel<D, 1, false>);
+    kernel<<<dim3((unsigned)H * (unsigned)(4 * n_wide + (n_items - n_wide) * split)), kBlockThreads, 0, s>>>(
+        S, n_blocks, H, block_row_ptr, block_col_idx, block_mask_index, block_masks, q, k, v, scale_log2e, o, n_items, n_wide, items,
         n_slots, partials);
   } else {
     auto kernel = block_mask_index ? &attn_f32_kernel<D, true> : &attn_f32_kernel<D, false>;

@@ -554,9 +554,10 @@ def _describe_blocks(pos: torch.Tensor, crd: torch.Tensor, M: int, n_cols: int, 
     return brp, arrays
 
 
-def _stretches(lens, longest, split_slots: bool):
+def _stretches(lens, longest, split_slots: bool, stretches_first: bool = False):
     """Work items (block row, begin, end, slot) over block rows of `lens` active blocks each, as an
-    int32 array of shape (n, 4) sorted longest first (ties in row order): a block row with more
+    int32 array of shape (n, 4) sorted longest first (ties in row order; with `stretches_first`, where whole rows are at least
+    twice as many, the stretches before them: the fp32 kernel has more wavefronts for the first n_slots items): a block row with more
     than `longest` blocks goes out in ceil(n / longest) stretches of nearly equal length.  With
     `split_slots` a whole row's slot is -1 and the stretches of a shared-out row get consecutive
     slots, returned with the list of those rows (block row, first slot, stretches, 0) and the number
@@ -579,6 +580,8 @@ def _stretches(lens, longest, split_slots: bool):
         rows = np.nonzero(shared)[0]
         split_rows = np.stack([rows, first_slot[rows], parts[rows], np.zeros_like(rows)], axis=1).astype(np.int32)
     order = np.argsort(-(hi - lo), kind="stable")          # longest first
+    if stretches_first and 3 * n_slots <= row.size:
+        order = order[np.argsort(slot[order] < 0, kind="stable")]
     items = np.stack([row, lo, hi, slot], axis=1)[order].astype(np.int32)
     return items, split_rows, n_slots
 
@@ -2008,7 +2011,8 @@ def attention_priority_step(lens, heads: int, D: int, pair: bool, n_cus: int = 2
     return max(1, -(-most // 4))
 
 
-def split_long_block_rows(bm: BlockMask, longest: Optional[int] = None, list_unequal_rows: bool = False) -> BlockMask:
+def split_long_block_rows(bm: BlockMask, longest: Optional[int] = None, list_unequal_rows: bool = False,
+                          stretches_first: bool = False) -> BlockMask:
     """Share block rows with more than `longest` key blocks out among several workgroups (in
     stretches of equal length up to `longest`); by default `longest` is twice the mean number of
     key blocks per block row, at least 8, so that masks whose rows are of similar length are left
@@ -2026,7 +2030,7 @@ def split_long_block_rows(bm: BlockMask, longest: Optional[int] = None, list_une
     if longest < 1 or most <= longest:
         if not (list_unequal_rows and nb and int(lens.min()) != most):
             return bm
-    items, split_rows, n_slots = _stretches(lens, longest if longest >= 1 else max(most, 1), True)
+    items, split_rows, n_slots = _stretches(lens, longest if longest >= 1 else max(most, 1), True, stretches_first)
     dev = bm.block_row_ptr.device
     bm.items = torch.from_numpy(items).to(dev).reshape(-1)
     bm.split_rows = torch.from_numpy(split_rows).to(dev).reshape(-1)
@@ -2150,7 +2154,7 @@ def _fp32_schedule(bm: BlockMask):
         longest = int(lens.max()) if lens.size else 0
         if longest > 1.25 * mean:      # (rows of similar length are best left whole)
             longest = min(FP32_ATTENTION_STRETCH, max(8, 2 * math.ceil(mean)))
-        split_long_block_rows(plain, longest, list_unequal_rows=True)
+        split_long_block_rows(plain, longest, list_unequal_rows=True, stretches_first=True)
         bm.schedule32 = (plain.items, plain.split_rows, plain.n_slots)
     return bm.schedule32
 
@@ -2184,7 +2188,7 @@ def _fp32_launch_schedule(bm: BlockMask, heads: int, D: int):
         if stretch is not None and not torch.cuda.is_current_stream_capturing():
             plain = BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)
             plain.block_row_lens = bm.row_lens()
-            split_long_block_rows(plain, stretch, list_unequal_rows=True)
+            split_long_block_rows(plain, stretch, list_unequal_rows=True, stretches_first=True)
             kept = (plain.items, plain.split_rows, plain.n_slots)
         elif stretch is not None:
             return kept

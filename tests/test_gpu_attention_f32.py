@@ -241,3 +241,30 @@ def test_teams_of_four_two_and_one_wavefront_to_sixteen_queries(oracle, heads, D
         assert np.isnan(out[h][hit]).all()
         assert oracle.rel_fro(np.where(hit, 0, out[h]), np.where(hit, 0, want)) <= TOL
         assert np.all(out[h, 160:176] == 0)
+
+
+# twenty block rows, and five or so stretches of the row with the global token: 384 to 800 workgroups of a block row
+@pytest.mark.parametrize("heads, token", [(16, 0), (24, 40), (25, 17), (32, 1100), (33, 1218)])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_a_few_long_rows_in_stretches_of_four_workgroups_each(oracle, heads, token, D):
+    """One query that attends to everything, in every sixteen of its block row: its stretches go to more wavefronts than the
+    other rows, whatever the order of the items."""
+    S = 1219
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = (abs(i - j) <= 40) | (i == token) | (j == token)
+    rng = np.random.default_rng(heads + D)
+    q, k, v = (rng.standard_normal((heads, S, D)).astype(np.float32) for _ in range(3))
+    scale = D ** -0.5
+    rp, ci = (dev(x) for x in csr_of(mask))
+    dq, dk, dv = (dev(x) for x in (q, k, v))
+    for call in range(3):
+        out = H.sparse_attention_csr(rp, ci, dq, dk, dv, scale).cpu().numpy()
+    for h in {0, heads // 2, heads - 1}:
+        assert oracle.rel_fro(out[h], oracle.attention_dense_fp64(q[h], k[h], v[h], mask, scale)) <= TOL
+    bm = rp._scorch_plan.attention
+    items, split_rows, n_slots = H._fp32_launch_schedule(bm, heads, D)
+    rows = items.view(-1, 4)
+    assert 0 < 3 * n_slots <= rows.shape[0] and bool((rows[:n_slots, 3] >= 0).all())
+    bm.pairing["fp32", heads, D] = (rows.flip(0).contiguous().view(-1), split_rows, n_slots)
+    turned = H.attn_blocksparse_f32(dq, dk, dv, bm, scale).cpu().numpy()
+    assert oracle.rel_fro(turned, out) <= TOL
