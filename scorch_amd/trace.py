@@ -198,7 +198,7 @@ def _try_prebuilt_fused(spec: FusionSpec, args: tuple) -> Optional[Callable]:
             scorch_ops_hip.remember_spmm(lhs, cols, act)
         return out.storage.value.view(rows, cols)
 
-    run.fused_symbol = resolved.symbol_name
+    run.fused_symbol, run.act = resolved.symbol_name, act
     return run
 
 
@@ -238,8 +238,17 @@ class compile:
         self.fn = fn
         self._fx_graph: Optional[torch.fx.GraphModule] = None
         self._cache: Dict[tuple, tuple] = {}
+        self._decided: Optional[tuple] = None     # (the arguments of its decided product, activation), once a runner was a fused one
 
     def __call__(self, *args: Any) -> Any:
+        # A product that has been decided is served whatever runner it was decided by: only those of the fused kernel's formats and
+        # types are, and the function is the same.  (Two layers: 5.8 -> 4.8 us each before the runner is looked up.)
+        if self._decided is not None:
+            a, b, bias, act, count = self._decided
+            if len(args) == count:
+                result = ops._decided_spmm(args[a], args[b], args[bias], act)
+                if result is not None:
+                    return result
         if self._fx_graph is None:
             self._fx_graph = _symbolic_trace(self.fn)
         key = self._build_cache_key(args)
@@ -248,6 +257,8 @@ class compile:
             spec = analyze_fx_graph(self._fx_graph.graph, args)
             cached = (compile_fused(spec, args), spec)
             self._cache[key] = cached
+            if cached[0].fused_symbol is not None and spec.complete:
+                self._decided = (*spec.matmul_arg_indices, spec.extra_arg_indices[0], cached[0].act, len(args))
         runner, spec = cached
         result = runner(args)
         if spec.complete:
