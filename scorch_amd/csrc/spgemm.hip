@@ -368,6 +368,30 @@ __device__ __forceinline__ void marked_step(int x0, int total, int t, int first,
     if (x0 + u * TEAM + t < total) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
 }
 
+// The columns and products of a wavefront's step, 0 <= step.first < step.last: slot u's are those of step.product(u, lane) if the
+// wavefront has any there.
+template <int TEAM, bool NUMERIC, typename T, typename A, int U>
+__device__ __forceinline__ void products_of_step(const ProductStep &step, const int *__restrict__ b_crd, const T *__restrict__ b_val,
+                                                 ProductBatch<TEAM, A> &batch, int (&col)[U], A (&product)[U]) {
+  const int lane = wave_lane();
+  int e[U], q[U];
+  A b[U];
+  entries_of_products<TEAM, U, A>(step, batch, e);
+#pragma unroll
+  for (int u = 0; u < U; ++u) q[u] = step.product(u, lane) + batch.start[e[u]];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u > 0 && !step.has(u)) break;  // uniform over the wavefront
+    col[u] = b_crd[q[u]];
+    b[u] = NUMERIC ? (A)b_val[q[u]] : (A)0;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u > 0 && !step.has(u)) break;
+    product[u] = NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0;
+  }
+}
+
 // fn(column, product) for every product of A entries [a_lo, a_hi); `t` is the
 // thread's number in the team.  Uniform over the team.
 template <int TEAM, bool NUMERIC, typename T, typename A, typename Fn>
@@ -401,20 +425,12 @@ __device__ __forceinline__ void for_each_product(int a_lo, int a_hi, int t, cons
       for (int x = 0; x < total; x += U * TEAM) {
         const ProductStep step = product_step(x, min(U * TEAM, total - x), TEAM / kWaveSize, w);
         if (step.first >= step.last) break;
-        int e[U], q[U], col[U];
-        A b[U];
-        entries_of_products<TEAM, U, A>(step, batch, e);
-#pragma unroll
-        for (int u = 0; u < U; ++u) q[u] = step.product(u, lane) + batch.start[e[u]];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (u > 0 && !step.has(u)) break;  // uniform over the wavefront
-          col[u] = b_crd[q[u]];
-          b[u] = NUMERIC ? (A)b_val[q[u]] : (A)0;
-        }
+        int col[U];
+        A product[U];
+        products_of_step<TEAM, NUMERIC, T, A>(step, b_crd, b_val, batch, col, product);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (step.first + u * kWaveSize + lane < step.last) fn(col[u], NUMERIC ? batch.a_val[e[u]] * b[u] : (A)0);
+          if (step.first + u * kWaveSize + lane < step.last) fn(col[u], product[u]);
       }
     }
   }
@@ -1333,6 +1349,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
   using Tables = BitmapTables<A, NUMERIC, WORDS, THREADS, ACC>;
   constexpr int kAccEntries = Tables::kAccEntries;
   constexpr int kWaves = THREADS / kWaveSize;
+  constexpr bool kHolds = NUMERIC && ACC > 0;
   auto &s_bits = lds.bits;
   auto &s_rank = lds.rank;
   auto &s_acc = lds.acc;
@@ -1381,6 +1398,35 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
     const int out = NUMERIC ? c_pos[row] : 0;
     int done = 0;  // distinct columns found in the ranges before this one
 
+    // Rows of as many products as the threads hold in registers are walked once (131,072 nodes, 16 a row, 2,600 rows: 60 -> 52 us).
+    constexpr int U = kProductsInFlight, kSteps = kHolds ? kMediumProducts / (U * THREADS) : 1;
+    static_assert(!kHolds || (kSteps * U * THREADS == kMediumProducts && WORDS * 32 >= kNarrowColumns), "all products of a row of one range");
+    int col[kSteps][U];
+    A product[kSteps][U];
+    ProductStep steps[kSteps] = {};
+    bool held = kHolds && !sums_by_column && a_hi - a_lo <= THREADS;
+    if constexpr (kHolds) {
+      if (held) {  // uniform
+        int start = 0, len = 0;
+        A av = (A)0;
+        if (a_lo + tid < a_hi) {
+          const int j = a_crd[a_lo + tid];
+          start = b_pos[j];
+          len = b_pos[j + 1] - start;
+          av = (A)a_val[a_lo + tid];
+        }
+        const int total = fill_batch<THREADS, true, A>(len, start, av, s_batch, s_scan);
+        held = total <= kMediumProducts;
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+          const int x = s * U * THREADS;
+          if (!held || x >= total) break;
+          steps[s] = product_step(x, min(U * THREADS, total - x), kWaves, uniform(tid / kWaveSize));
+          if (steps[s].first < steps[s].last) products_of_step<THREADS, true, T, A>(steps[s], b_crd, b_val, s_batch, col[s], product[s]);
+        }
+      }
+    }
+
     // B wider than the bitmap: one range of kRangeColumns columns after the other,
     // walking the row's products again for each (ranges ascend, so the row comes
     // out sorted all the same)
@@ -1398,12 +1444,22 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
               atomicOr(&s_bits[k >> 5], 1u << (k & 31));
               lds_accumulate<A>(&s_acc[k], product);
             });
+      } else if (held) {
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (steps[s].first + u * kWaveSize + wave_lane() < steps[s].last) atomicOr(&s_bits[col[s][u] >> 5], 1u << (col[s][u] & 31));
       } else {
         for_each_product<THREADS, false, T, A>(
             a_lo, a_hi, tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan, [&](int k, A) {
               const unsigned rel = (unsigned)(k - c0);
               if (rel < (unsigned)columns) atomicOr(&s_bits[rel >> 5], 1u << (rel & 31));
             });
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)  // (nothing is held: no registers for it during the walk)
+#pragma unroll
+          for (int u = 0; u < U; ++u) col[s][u] = 0, product[s][u] = (A)0;
       }
       __syncthreads();
 
@@ -1447,23 +1503,31 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
         for (int e = in_lds + tid; e < n; e += THREADS) workgroup_store(&acc[first + e], (A)0);
         for (int e = tid; e < in_lds; e += THREADS) s_acc[e] = (A)0;
         __syncthreads();
-        for_each_product<THREADS, true, T, A>(
-            a_lo, a_hi, tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan, [&](int k, A product) {
-              const unsigned rel = (unsigned)(k - c0);
-              if (rel >= (unsigned)columns) return;
-              // rank = the group's + the bits below the column's in the group's four words,
-              // which come in one read (a loop over the words before the column's
-              // would chain up to three more LDS round trips)
-              const int w = (int)(rel >> 5), sub = w & 3;
-              const uint4 grp = *reinterpret_cast<const uint4 *>(&s_bits[w & ~3]);
-              const unsigned below = (1u << (rel & 31)) - 1u;
-              const int at = s_rank[w >> 2] + __popc(grp.x & (sub == 0 ? below : ~0u)) +
-                             __popc(grp.y & (sub == 1 ? below : sub > 1 ? ~0u : 0u)) +
-                             __popc(grp.z & (sub == 2 ? below : sub > 2 ? ~0u : 0u)) +
-                             __popc(grp.w & (sub == 3 ? below : 0u));
-              if (at < kAccEntries) lds_accumulate<A>(&s_acc[at], product);
-              else __hip_atomic_fetch_add(&acc[first + at], product, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            });
+        const auto add = [&](int k, A product) {
+          const unsigned rel = (unsigned)(k - c0);
+          if (rel >= (unsigned)columns) return;
+          // rank = the group's + the bits below the column's in the group's four words,
+          // which come in one read (a loop over the words before the column's
+          // would chain up to three more LDS round trips)
+          const int w = (int)(rel >> 5), sub = w & 3;
+          const uint4 grp = *reinterpret_cast<const uint4 *>(&s_bits[w & ~3]);
+          const unsigned below = (1u << (rel & 31)) - 1u;
+          const int at = s_rank[w >> 2] + __popc(grp.x & (sub == 0 ? below : ~0u)) +
+                         __popc(grp.y & (sub == 1 ? below : sub > 1 ? ~0u : 0u)) +
+                         __popc(grp.z & (sub == 2 ? below : sub > 2 ? ~0u : 0u)) +
+                         __popc(grp.w & (sub == 3 ? below : 0u));
+          if (at < kAccEntries) lds_accumulate<A>(&s_acc[at], product);
+          else __hip_atomic_fetch_add(&acc[first + at], product, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        if (held) {
+#pragma unroll
+          for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (steps[s].first + u * kWaveSize + wave_lane() < steps[s].last) add(col[s][u], product[s][u]);
+        } else {
+          for_each_product<THREADS, true, T, A>(a_lo, a_hi, tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan, add);
+        }
         __syncthreads();
         for (int e = tid; e < in_lds; e += THREADS) c_val[first + e] = (T)s_acc[e];
       }
@@ -1485,45 +1549,49 @@ __global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
                                                                       counters, c_pos, c_crd, c_val);
 }
 
-// ---- a matrix of few rows: the three kinds of 256-thread work in one launch --------------------
+// ---- a matrix of few rows: the three kinds of work in one launch --------------------------------
 // Below 32,768 rows the tiers' kernels are short and what a product costs is launches, 3 to 5 us
 // each: workgroups [0, n_bitmap) take bitmap rows, the next n_medium hash rows of up to
-// kSmallProducts products, the rest four rows of up to kTinyProducts each, the longest kinds first.
+// kSmallProducts products, the rest a row of up to kTinyProducts to each wavefront, the longest kinds first.
 // The kinds share the workgroup's LDS (40 KB with fp32 sums, four workgroups to a CU).
+// (512 threads: with 256, rows of 1,024 to 4,096 products took twice the steps, and there are few of them to fill the chip with:
+// 1,500 nodes of 16 86 -> 82 us in all, 25,000 of 10 140 -> 135.)
+constexpr int kSmallMatrixThreads = 512;
 template <typename T, bool NUMERIC>
-__global__ __launch_bounds__(kBlockThreads) void spgemm_small_matrix_kernel(
+__global__ __launch_bounds__(kSmallMatrixThreads) void spgemm_small_matrix_kernel(
     int M, int N, int n_bitmap, int n_medium, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
     const T *__restrict__ a_val, const int *__restrict__ b_pos, const int *__restrict__ b_crd,
     const T *__restrict__ b_val, const int *__restrict__ products, const int *__restrict__ small_rows,
     const int *__restrict__ medium_rows, const int *__restrict__ narrow_rows, int *__restrict__ counters,
     int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
+  constexpr int kWaves = kSmallMatrixThreads / kWaveSize;
   union Tables {
-    BitmapTables<A, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts> bitmap;
-    MediumTables<A, NUMERIC, kSmallProducts, kBlockThreads> medium;
-    TeamTables<A, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts> tiny;
+    BitmapTables<A, NUMERIC, kNarrowColumns / 32, kSmallMatrixThreads, kBitmapSums> bitmap;
+    MediumTables<A, NUMERIC, kSmallProducts, kSmallMatrixThreads> medium;
+    TeamTables<A, NUMERIC, kWaveSize, kWaves, kTinySlots, kTinyProducts> tiny;
   };
   __shared__ Tables lds;
   int block = blockIdx.x;
   if (block < n_bitmap) {
-    spgemm_lds_bitmap_rows<T, NUMERIC, kNarrowColumns / 32, kBlockThreads, kMediumProducts, 0, 4>(
+    spgemm_lds_bitmap_rows<T, NUMERIC, kNarrowColumns / 32, kSmallMatrixThreads, kBitmapSums, 0, 4>(
         lds.bitmap, block, n_bitmap, M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, medium_rows, narrow_rows, counters,
         c_pos, c_crd, c_val);
     return;
   }
   block -= n_bitmap;
   if (block < n_medium) {
-    spgemm_medium_rows<T, NUMERIC, kSmallProducts, 2, kBlockThreads>(lds.medium, block, n_medium, a_pos, a_crd, a_val, b_pos,
+    spgemm_medium_rows<T, NUMERIC, kSmallProducts, 2, kSmallMatrixThreads>(lds.medium, block, n_medium, a_pos, a_crd, a_val, b_pos,
                                                                     b_crd, b_val, products, small_rows, counters, c_pos,
                                                                     c_crd, c_val);
     return;
   }
   block -= n_medium;
   const int w = threadIdx.x / kWaveSize;
-  const int row = block * kWavesPerBlock + w;
+  const int row = block * kWaves + w;
   const int bound = row < M ? products[row] : INT_MAX;
   if (bound > kTinyProducts) return;
-  spgemm_team_row<T, NUMERIC, kWaveSize, kWavesPerBlock, kTinySlots, kTinyProducts>(
+  spgemm_team_row<T, NUMERIC, kWaveSize, kWaves, kTinySlots, kTinyProducts>(
       lds.tiny, w, wave_lane(), row, bound, a_pos, a_crd, a_val, b_pos, b_crd, b_val, c_pos, c_crd, c_val);
 }
 
@@ -2252,8 +2320,8 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
     const unsigned small_blocks = blocks_for(known ? known->small : M);
     const unsigned bitmap_blocks = blocks_for(known ? known->medium + (narrow_rows ? known->huge : 0) : M);
     if (M < 4 * 8192 && narrow) {
-      const unsigned tiny_blocks = (unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock);
-      spgemm_small_matrix_kernel<T, NUMERIC><<<bitmap_blocks + small_blocks + tiny_blocks, kBlockThreads, 0, stream>>>(
+      const unsigned tiny_blocks = (unsigned)((M + kSmallMatrixThreads / kWaveSize - 1) / (kSmallMatrixThreads / kWaveSize));
+      spgemm_small_matrix_kernel<T, NUMERIC><<<bitmap_blocks + small_blocks + tiny_blocks, kSmallMatrixThreads, 0, stream>>>(
           M, N, (int)bitmap_blocks, (int)small_blocks, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows,
           ws.medium_rows, narrow_rows, ws.counters, c_pos, c_crd, c_val);
       SCORCH_HIP_CHECK(hipGetLastError());
