@@ -86,22 +86,24 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
     held_begin = r < row_end ? row_ptr[r] : 0;
     held_end = r < row_end ? row_ptr[r + 1] : 0;
   };
-  int c[R];
-  float a[R];
-  auto load_entries = [&](int first, int end) {  // (loads beyond the row's end give zeros)
+  struct Entries {
+    int c[R];
+    float a[R];
+  } even, odd;
+  auto load_entries = [&](Entries &to, int first, int end) __attribute__((always_inline)) {  // (loads beyond the row's end give zeros)
     first = uniform(first);
     const int bytes = uniform(max(min(end - first, BATCH), 0) * 4);
     const __amdgpu_buffer_rsrc_t columns = __builtin_amdgcn_make_buffer_rsrc((void *)(col_idx + first), 0, bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t values = __builtin_amdgcn_make_buffer_rsrc((void *)(vals + first), 0, bytes, 0x00020000);
 #pragma unroll
     for (int e = 0; e < R; ++e) {
-      c[e] = __builtin_amdgcn_raw_buffer_load_b32(columns, (e * kWaveSize + lane) * 4, 0, 0);
-      a[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(values, (e * kWaveSize + lane) * 4, 0, 0));
+      to.c[e] = __builtin_amdgcn_raw_buffer_load_b32(columns, (e * kWaveSize + lane) * 4, 0, 0);
+      to.a[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(values, (e * kWaveSize + lane) * 4, 0, 0));
     }
   };
   hold(row);
   int begin = __builtin_amdgcn_readlane(held_begin, 0), end = __builtin_amdgcn_readlane(held_end, 0);
-  load_entries(begin, end);
+  load_entries(even, begin, end);
 
   if (transposed) {  // B[k][n] lies at n * K + k
     constexpr int AHEAD = 32 / P;  // 32 loads in flight
@@ -150,15 +152,16 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
   if (threadIdx.x < LPE) s_panel[K * LPE + threadIdx.x] = make_float4(0, 0, 0, 0);
   __syncthreads();
 
-  // (k: the first entry of the batch in c and a; begin, end: its row's)
+  // A batch at hand, of the row's entries from k on, while the next one is requested: the two change places from step to step (copied
+  // from one to the other they were 16 of a step's 105 vector instructions with four batches to a lane).
   int k = begin;
   float acc[4] = {0, 0, 0, 0};
-  while (row < row_end) {
+  auto step = [&](const Entries &at_hand, Entries &next) __attribute__((always_inline)) {
     Shared<LPE> from[R], with[R];  // the byte an entry's row of the panel begins at, and its value
 #pragma unroll
     for (int e = 0; e < R; ++e) {
-      from[e] = Shared<LPE>((e * kWaveSize + lane < end - k ? c[e] : K) * (P * 4));
-      with[e] = Shared<LPE>(__builtin_bit_cast(int, a[e]));
+      from[e] = Shared<LPE>((e * kWaveSize + lane < end - k ? at_hand.c[e] : K) * (P * 4));
+      with[e] = Shared<LPE>(__builtin_bit_cast(int, at_hand.a[e]));
     }
     k += BATCH;
     const bool row_done = k >= end;
@@ -173,7 +176,7 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
       end = __builtin_amdgcn_readlane(held_end, held & (kWaveSize - 1));
       k = begin;
     }
-    if (row < row_end) load_entries(k, end);
+    if (row < row_end) load_entries(next, k, end);
     constexpr int STEPS = R * LPE, AT_ONCE = STEPS < 4 ? STEPS : 4;  // LDS reads in flight
 #pragma unroll
     for (int s0 = 0; s0 < STEPS; s0 += AT_ONCE) {
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
         acc[3] += value * b[i].w;
       }
     }
-    if (!row_done) continue;
+    if (!row_done) return;
     // The upper half of the wavefront keeps columns 2 and 3 of a lane's four, then odd rows of 16 lanes the odd one of two.
     // (a's upper half changes places with b's lower one, then a's odd rows with b's even ones)
     auto exchanged = [](float a, float b, auto swap) {
@@ -215,6 +218,10 @@ __global__ __launch_bounds__(kPanelThreads) void spmm_panels_kernel(
       C[(size_t)this_row * (size_t)N + col] = sum;
     }
     acc[0] = acc[1] = acc[2] = acc[3] = 0.0f;
+  };
+  while (row < row_end) {
+    step(even, odd);
+    if (row < row_end) step(odd, even);
   }
 }
 
