@@ -1906,16 +1906,28 @@ __global__ __launch_bounds__(kBinItemThreads) void spgemm_bin_items_kernel(Bins 
   const int lane = wave_lane();
   const BinRow r = bins.row[blockIdx.x];
   const int lo = a_pos[r.row], hi = a_pos[r.row + 1];
-  for (int batch = threadIdx.x / kWaveSize; batch < r.batches; batch += kBinItemThreads / kWaveSize) {
-    int at[kPer], total = 0;
+  int next[kPer];  // columns of the batch to come
+  auto request = [&](int batch) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int p = lo + batch * kBinEntries + i * kWaveSize + lane;
-      at[i] = p < hi ? a_crd[p] : -1;
+      next[i] = p < hi ? a_crd[p] : -1;
     }
+  };
+  constexpr int kBatchWaves = kBinItemThreads / kWaveSize;
+  int batch = threadIdx.x / kWaveSize;
+  if (batch < r.batches) request(batch);
+  for (; batch < r.batches; batch += kBatchWaves) {
+    Vec<int, 2> b[kPer];
+    int total = 0;
 #pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      if (at[i] >= 0) total += b_pos[at[i] + 1] - b_pos[at[i]];
+    for (int i = 0; i < kPer; ++i) {
+      b[i].v[0] = b[i].v[1] = 0;
+      if (next[i] >= 0) b[i] = load_vec<int, 2>(b_pos + next[i]);
+    }
+    if (batch + kBatchWaves < r.batches) request(batch + kBatchWaves);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) total += b[i].v[1] - b[i].v[0];
 #pragma unroll
     for (int off = kWaveSize / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
     const int shares = 1 + total / bins.share;
@@ -1988,6 +2000,7 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
         unsigned long long alike = __ballot(true);
 #pragma unroll
         for (int bit = 0; (1 << bit) < kMaxBins; ++bit) {
+          if (bins.n <= 1 << bit) break;  // uniform
           const int set = -((bin[u] >> bit) & 1);
           const unsigned long long with = __ballot(set != 0);
           const unsigned lo = (unsigned)alike & ~((unsigned)with ^ (unsigned)set);
@@ -2000,11 +2013,12 @@ __global__ __launch_bounds__(kBinThreads) void spgemm_bin_kernel(
         rank[u] = before + __shfl(base, __ffsll(alike) - 1);
       }
     __syncthreads();
-    if (tid <= bins.n) {
-      int at = 0;
-      for (int i = 0; i < tid; ++i) at += s_count[i];
-      s_at[tid] = at;
-      bins.window[r.first_window + s_window].at[tid] = (unsigned short)at;
+    if (w == 0) {  // (the others wait: a scan by the lanes, not a chain of reads)
+      const int count = lane < bins.n ? s_count[lane] : 0, at = team_inclusive_sum<kWaveSize>(count) - count;
+      if (lane <= bins.n) {
+        s_at[lane] = at;
+        bins.window[r.first_window + s_window].at[lane] = (unsigned short)at;
+      }
     }
     if (tid == 0) bins.window[r.first_window + s_window].first = r.first_product + s_first;
     __syncthreads();
