@@ -2176,6 +2176,16 @@ def _fp32_stretch(lens, heads: int, D: int, n_cus: int) -> Optional[int]:
     return 2 if share < 2 else 4 if share * D / 64 < 16 else 8
 
 
+def _eight_at_once(lens, heads: int, D: int, n_cus: int) -> bool:
+    """Whether stretches of eight key blocks serve a few long rows at D = 32 better than four: a stretch's tiles go to
+    four wavefronts (csrc/attn_f32.hip) and are half as long, and a CU's share is five blocks or more (in units of D = 64).
+    Window of 64 and a global token, 16 heads, us: S = 3,001 23.7 -> 22.6, 6,075 41.3 -> 37.3; 1,024, 12 heads 13.9 -> 15.6."""
+    if D != 32 or float(lens.sum()) * heads / n_cus * D / 64 < 5:
+        return False
+    slots = int(-(-lens[lens > 8] // 8).sum())
+    return 0 < 3 * slots <= int((lens <= 8).sum()) + slots
+
+
 def _fp32_launch_schedule(bm: BlockMask, heads: int, D: int):
     """_fp32_schedule for a launch of so many heads, kept with the BlockMask."""
     key = ("fp32", heads, D)
@@ -2185,6 +2195,8 @@ def _fp32_launch_schedule(bm: BlockMask, heads: int, D: int):
         if bm.schedule32 is None:          # (being recorded, with nothing decided before)
             return kept
         stretch = _fp32_stretch(bm.row_lens(), heads, D, _cu_count(bm.block_row_ptr.device))
+        if stretch == 4 and _eight_at_once(bm.row_lens(), heads, D, _cu_count(bm.block_row_ptr.device)):
+            stretch = 8
         if stretch is not None and not torch.cuda.is_current_stream_capturing():
             plain = BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)
             plain.block_row_lens = bm.row_lens()

@@ -693,6 +693,16 @@ def test_stretches_of_the_fused_fp32_kernel_on_either_side_of_every_rule(lens, h
 
 
 @pytest.mark.parametrize("lens, heads, D, want", [
+    # a CU's share of five blocks (in units of D = 64), one long row among short ones, D = 32
+    (_rows((3, 90), (90, 1)), 16, 32, True), (_rows((3, 90), (90, 1)), 6, 32, False), (_rows((3, 90), (90, 1)), 16, 64, False),
+    # stretches of eight are a third of the items at most; rows of eight blocks are whole
+    (_rows((4, 24), (90, 1)), 40, 32, True), (_rows((4, 23), (90, 1)), 40, 32, False), (_rows((8, 90)), 16, 32, False),
+])
+def test_stretches_of_eight_for_a_few_long_rows(lens, heads, D, want):
+    assert scorch_ops_hip._eight_at_once(lens, heads, D, 256) == want
+
+
+@pytest.mark.parametrize("lens, heads, D, want", [
     # no row stands out: whole rows, unless half the CUs at most have one and some row has 16 blocks or more
     (_rows((7, 128)), 1, 64, None), (_rows((16, 128)), 1, 64, 8), (_rows((15, 128)), 1, 64, None), (_rows((16, 129)), 1, 64, None),
     (_rows((16, 64)), 2, 64, 8), (_rows((16, 65)), 2, 64, None),
