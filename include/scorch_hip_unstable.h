@@ -182,6 +182,14 @@ SCORCH_HIP_API int scorch_hip_spmm_csr_tiled_f32(int64_t M, int64_t K, int64_t N
                                   const float *Bt, size_t bt_bytes, const float *bias, int act, float *C,
                                   const void *bounds, size_t bounds_bytes,
                                   void *workspace, size_t workspace_bytes, int64_t longest_row, void *stream);
+/* The same for column indices that nobody has looked at yet, under row pointers that are known to be well formed, where every wavefront has one
+ * chunk (scorch_hip_spmm_csr_tiled_recommended): the product reads row 0 for a column outside [0, K), and
+ * scorch_hip_csr_inspect_columns_end(*pending, ...) says while it runs whether there was one, i.e. the product is not to be used.
+ * *pending is NULL if nothing has been queued.  Not for a stream that is being captured. */
+SCORCH_HIP_API int scorch_hip_spmm_csr_tiled_new_columns_f32(int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,
+                                                 const int32_t *col_idx, const float *vals, const float *Bt, size_t bt_bytes, float *C,
+                                                 void *workspace, size_t workspace_bytes, int64_t longest_row, void *stream,
+                                                 void **pending);
 
 /* SpMM of a matrix of up to 10,239 columns whose rows are about equally long -- a sparse weight
  * matrix -- with B by column panels in LDS: C = act(A * B + bias), bias NULL or of N elements.

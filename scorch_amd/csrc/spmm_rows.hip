@@ -415,12 +415,6 @@ __global__ __launch_bounds__(kBlockThreads) void csr_inspect_kernel(int M, int K
 // verdict before it returns, reads it while the product runs.  (The decoder product of 4,096 x 32
 // activations, N = 4,096, kept the GPU idle for 45 of 166 us while the host waited for the inspection
 // of the whole pattern, boundaries and launches.)
-struct ColumnsSync {
-  int *tickets;      // [0]: see SyncSlot; [16]: whether a column lies outside, left 0
-  unsigned tickets_before;
-  int64_t *to;
-  int64_t sequence;
-};
 __global__ __launch_bounds__(kBlockThreads) void csr_columns_kernel(int K, int64_t nnz, const int *__restrict__ col_idx,
                                                                     int *__restrict__ checked, ColumnsSync sync) {
   const int64_t stride = (int64_t)gridDim.x * kBlockThreads;
@@ -432,20 +426,8 @@ __global__ __launch_bounds__(kBlockThreads) void csr_columns_kernel(int K, int64
     checked[p] = outside ? 0 : c;
   }
   bad = __syncthreads_or(bad);
-  if (threadIdx.x != 0) return;
-  if (bad) (void)__hip_atomic_fetch_or(sync.tickets + 16, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned ticket = __hip_atomic_fetch_add(reinterpret_cast<unsigned *>(sync.tickets), 1u, __ATOMIC_ACQ_REL,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-  if (ticket - sync.tickets_before != gridDim.x - 1) return;  // not the last workgroup
-  const int64_t verdict = __hip_atomic_exchange(sync.tickets + 16, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  sync_publish(sync.to, sync.sequence, &verdict, 1);
+  if (threadIdx.x == 0) columns_checked(sync, bad, gridDim.x);
 }
-
-// A check whose verdict has not been read yet.
-struct ColumnsPending {
-  SyncCall sync;
-  hipStream_t stream;
-};
 
 }  // namespace scorch
 

@@ -27,7 +27,11 @@
 // workgroup waits for another: with few enough requests in flight per wavefront
 // (kTiledBatch) the wavefronts of an XCD, which all have about the same work per
 // tile, stay together well enough by themselves.
+#include <memory>
+#include <new>
+
 #include "spmm.hpp"
+#include "sync.hpp"
 
 namespace scorch {
 
@@ -72,13 +76,16 @@ __global__ __launch_bounds__(kBlockThreads) void dense_to_tiled_kernel(int64_t K
   *reinterpret_cast<Vec<T, VEC> *>(Bt + idx * VEC) = o;
 }
 
-template <typename T, int EPI>
+// CHECKED: nobody has looked whether the columns lie in [0, K).  A wavefront that stages its chunk (single chunks only) reads row 0 for those
+// that do not, and one XCD's workgroups, which have all of the entries among them, tell the host: the verdict is there
+// before the first tile is through, and a launch in front that reads the columns is saved (decoder shape: 5.4 us and the gap behind it).
+template <typename T, int EPI, bool CHECKED>
 __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
     int M, int N, int K, const int *__restrict__ row_ptr, const int *__restrict__ col_idx,
     const T *__restrict__ vals, const T *__restrict__ Bt, T *__restrict__ C,
     const T *__restrict__ bias, int64_t total_items, int items_per_chunk, int snap, int n_tiles,
     int wgs_per_xcd, int64_t spans, int vector_stores, int *__restrict__ carry_row,
-    T *__restrict__ carry_val, const Boundary *__restrict__ bounds) {
+    T *__restrict__ carry_val, const Boundary *__restrict__ bounds, ColumnsSync sync) {
   using A = typename Acc<T>::type;
   constexpr int VEC = (int)(16 / sizeof(T));
   constexpr int LPR = kTileBytes / 16;
@@ -104,6 +111,18 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
   bool carry_in = false, staged = false;
   const bool has_work = first_span < spans;
 
+  __shared__ int s_bad, s_through;  // CHECKED: of the workgroup's wavefronts
+  if constexpr (CHECKED) {
+    if (threadIdx.x == 0) s_bad = s_through = 0;
+    __syncthreads();
+  }
+  const auto looked_at = [&](bool bad) {  // once by every wavefront
+    if (!CHECKED || xcd != 0 || lane != 0) return;
+    if (bad) atomicOr(&s_bad, 1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    if (atomicAdd(&s_through, 1) == kWavesPerBlock - 1) columns_checked(sync, atomicOr(&s_bad, 0), gridDim.x >> 3);
+  };
+  if (!has_work) looked_at(false);
   for (int tile = xcd; tile < n_tiles; tile += 8) {
     // A gathered row's address is the slice's (the same for the whole wavefront: scalar registers) plus
     // a byte offset of 32 bits (the entry's, staged as such, plus the lane's 16 bytes of the tile row):
@@ -127,10 +146,14 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_tiled_kernel(
         x0 = from.x, y0 = from.y, x1 = to.x, y1 = to.y;
         n_nz = y1 - y0;
         n_rows = x1 - x0;
+        bool bad = false;
         for (int k = lane; k < n_nz; k += kWaveSize) {
-          s_col[w][k] = (int)((unsigned)col_idx[y0 + k] * (unsigned)kTileBytes);  // byte offset within a slice
+          unsigned col = (unsigned)col_idx[y0 + k];
+          if (CHECKED && col >= (unsigned)K) bad = true, col = 0u;
+          s_col[w][k] = (int)(col * (unsigned)kTileBytes);  // byte offset within a slice
           s_val[w][k] = vals[y0 + k];
         }
+        if (CHECKED) looked_at(__any(bad));
         for (int k = lane; k <= n_rows + 1; k += kWaveSize) {
           const int r = x0 + k < M ? x0 + k : M;
           s_rp[w][k] = row_ptr[r];
@@ -243,7 +266,7 @@ template <typename T, int EPI>
 int spmm_tiled_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,
                      const int32_t *col_idx, const T *vals, const T *Bt, size_t bt_bytes, const T *bias, T *C,
                      const void *bounds_buffer, size_t bounds_bytes, void *workspace, size_t workspace_bytes,
-                     int64_t longest_row, void *stream) {
+                     int64_t longest_row, void *stream, void **pending = nullptr) {
   if (int rc = check_csr_args(fn, M, K, nnz, row_ptr, col_idx, vals)) return rc;
   SCORCH_REQUIRE(N >= 0, "%s: negative N=%lld", fn, (long long)N);
   if (N > INT32_MAX - kWaveSize * 4)
@@ -292,11 +315,24 @@ int spmm_tiled_entry(const char *fn, int64_t M, int64_t K, int64_t N, int64_t nn
   const int vector_stores = N % VEC == 0 && aligned_to(C, 16) && aligned_to(carry_val, 16);
   int64_t wgs = (split.spans + kWavesPerBlock - 1) / kWavesPerBlock;
   if (wgs > kTiledMaxWorkgroupsPerXcd) wgs = kTiledMaxWorkgroupsPerXcd;
+  std::unique_ptr<ColumnsPending> call;
+  ColumnsSync how = {};
+  auto kernel = &spmm_tiled_kernel<T, EPI, false>;
+  if (pending) {
+    if constexpr (EPI == kEpiNone) kernel = &spmm_tiled_kernel<T, EPI, true>;
+    if (split.spans > wgs * kWavesPerBlock || K == 0 || nnz == 0 || EPI != kEpiNone)
+      return fail(SCORCH_HIP_EUNSUPPORTED, "%s: %lld chunks for %lld wavefronts of an XCD", fn, (long long)split.spans,
+                  (long long)(wgs * kWavesPerBlock));
+    call.reset(new (std::nothrow) ColumnsPending{{}, s});
+    if (!call || call->sync.null()) return fail(SCORCH_HIP_ERUNTIME, "%s: no memory for the verdict", fn);
+    how = {call->sync.scratch(), call->sync.tickets_before((unsigned)wgs), call->sync.target(), call->sync.sequence()};
+  }
   mark_launch(s);
-  spmm_tiled_kernel<T, EPI><<<dim3((unsigned)(wgs * 8)), kBlockThreads, 0, s>>>(
+  kernel<<<dim3((unsigned)(wgs * 8)), kBlockThreads, 0, s>>>(
       (int)M, (int)N, (int)K, row_ptr, col_idx, vals, Bt, C, bias, M + nnz, split.items_per_chunk, split.snap,
-      (int)tiled_tiles(N, sizeof(T)), (int)wgs, split.spans, vector_stores, carry_row, carry_val, bounds);
+      (int)tiled_tiles(N, sizeof(T)), (int)wgs, split.spans, vector_stores, carry_row, carry_val, bounds, how);
   SCORCH_HIP_CHECK(hipGetLastError());
+  if (pending) *pending = call.release();
   mark_launch(s);
   // A boundary that falls inside a row moves to the row's end when that is at most `snap` items
   // away (chunk_boundary): with no row longer than that no chunk leaves a carry, and a caller who
@@ -376,6 +412,17 @@ int scorch_hip_spmm_csr_tiled_f32(int64_t M, int64_t K, int64_t N, int64_t nnz, 
                                                                  workspace, workspace_bytes, longest_row, stream);
   return scorch::fail(SCORCH_HIP_EINVAL, "%s: activation %d (with%s bias) is not supported", fn, act,
                       bias ? "" : "out");
+}
+
+int scorch_hip_spmm_csr_tiled_new_columns_f32(int64_t M, int64_t K, int64_t N, int64_t nnz, const int32_t *row_ptr,
+                                              const int32_t *col_idx, const float *vals, const float *Bt, size_t bt_bytes, float *C,
+                                              void *workspace, size_t workspace_bytes, int64_t longest_row, void *stream,
+                                              void **pending) {
+  const char *fn = "scorch_hip_spmm_csr_tiled_new_columns_f32";
+  SCORCH_REQUIRE(pending != nullptr, "%s: pending is NULL", fn);
+  *pending = nullptr;
+  return scorch::spmm_tiled_entry<float, scorch::kEpiNone>(fn, M, K, N, nnz, row_ptr, col_idx, vals, Bt, bt_bytes, nullptr, C,
+                                                           nullptr, 0, workspace, workspace_bytes, longest_row, stream, pending);
 }
 
 }  // extern "C"

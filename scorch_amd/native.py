@@ -102,6 +102,7 @@ SIGNATURES = {
     **{"scorch_hip_spmv_csr_listed_" + t: (ctypes.c_int, [_i64] * 3 + [_ptr, _ptr, _size] + [_ptr] * 3 + [_size, _i64, _ptr]) for t in ("f32", "f64")},
     "scorch_hip_dense_to_rows_f32": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr]),
     "scorch_hip_csr_inspect_columns_begin": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr, ctypes.POINTER(_ptr)]),
+    "scorch_hip_spmm_csr_tiled_new_columns_f32": (ctypes.c_int, [_i64] * 4 + [_ptr] * 4 + [_size, _ptr, _ptr, _size, _i64, _ptr, ctypes.POINTER(_ptr)]),
     "scorch_hip_csr_inspect_columns_end": (ctypes.c_int, [_ptr, ctypes.POINTER(ctypes.c_int32)]),
     "scorch_hip_spmm_csr_rows_panels_f32": (ctypes.c_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr, ctypes.c_int, _ptr,
                                                       ctypes.c_int, _ptr, _ptr]),

@@ -859,20 +859,37 @@ def _spmm(dtype, result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mod
     return _spmm_launch(plan, True, dtype, M, K, N, pos, crd, a_val, b_val, B_values, bias_ptr, act)
 
 
+_UNDECIDED = object()
+
+
 def _spmm_new_columns(plan: CsrPlan, dtype, M, K, N, pos, crd, a_val, b_val, B_values, bias_ptr, act):
     """A product with new column indices over row pointers that `plan` knows: the product is queued
     behind the check of the columns' range (it reads a copy without columns out of range), and the
     verdict is read while it runs."""
-    L, dev = native.lib(), pos.device
-    checked = _empty(crd.numel(), dtype=torch.int32, device=dev)
+    L, dev, nnz = native.lib(), pos.device, crd.numel()
     pending, outside = ctypes.c_void_p(), ctypes.c_int32(1)
     with _on_device(dev):
-        native.check(L.scorch_hip_csr_inspect_columns_begin(K, crd.numel(), crd.data_ptr(), checked.data_ptr(), _stream(dev),
-                                                    ctypes.byref(pending)))
-        try:
-            result = _spmm_launch(plan, False, dtype, M, K, N, pos, checked, a_val, b_val, B_values, bias_ptr, act)
-        finally:
-            rc = L.scorch_hip_csr_inspect_columns_end(pending, ctypes.byref(outside))
+        stream = _stream(dev)
+        tiled = _tiled_operand(B_values, K, N, nnz, L)
+        if tiled is not None and not L.scorch_hip_spmm_csr_tiled_recommended(M, K, N, nnz):
+            tiled = None
+        if tiled is not None and bias_ptr is None and act == 0:
+            # the product looks at the columns itself
+            out = _empty(M * N, dtype=dtype, device=dev)
+            ws = _workspace(dev, stream, L.scorch_hip_spmm_csr_workspace_bytes(M, nnz, N, 4))
+            rc = L.scorch_hip_spmm_csr_tiled_new_columns_f32(
+                M, K, N, nnz, pos.data_ptr(), crd.data_ptr(), a_val.data_ptr(), tiled.data_ptr(), tiled.numel() * 4, out.data_ptr(),
+                ws.data_ptr(), ws.numel(), plan.max_row, stream, ctypes.byref(pending))
+            ended = L.scorch_hip_csr_inspect_columns_end(pending, ctypes.byref(outside)) if pending.value else 0
+            native.check(rc)
+            rc, result = ended, Tensor(out, [[], []])
+        else:
+            checked = _empty(nnz, dtype=torch.int32, device=dev)
+            native.check(L.scorch_hip_csr_inspect_columns_begin(K, nnz, crd.data_ptr(), checked.data_ptr(), stream, ctypes.byref(pending)))
+            try:
+                result = _spmm_launch(plan, False, dtype, M, K, N, pos, checked, a_val, b_val, B_values, bias_ptr, act, tiled)
+            finally:
+                rc = L.scorch_hip_csr_inspect_columns_end(pending, ctypes.byref(outside))
         native.check(rc)
     if outside.value:
         raise _malformed("A", [f"a column index lies outside [0, {K})"])
@@ -880,9 +897,10 @@ def _spmm_new_columns(plan: CsrPlan, dtype, M, K, N, pos, crd, a_val, b_val, B_v
 
 
 def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N, pos, crd, a_val, b_val, B_values,
-                 bias_ptr, act):
+                 bias_ptr, act, tiled=_UNDECIDED):
     """Choose the kernel of a checked product and queue it.  `of_these_columns`: `plan` was made for
-    these column indices, not only for the row pointers."""
+    these column indices, not only for the row pointers.  `tiled`: the column-tile copy of B to use or
+    None, where the caller has decided that."""
     dev, nnz = pos.device, a_val.numel()
     out = _empty(M * N, dtype=dtype, device=dev)
     L = native.lib()
@@ -892,8 +910,10 @@ def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N
     with _on_device(dev):
         stream = _stream(dev)
         # a wide dense operand that keeps coming back is served from its column-tile copy
-        tiled = None
-        if path == "auto":
+        decided, tiled = tiled is not _UNDECIDED, None if tiled is _UNDECIDED else tiled
+        if decided:
+            pass
+        elif path == "auto":
             tiled = _tiled_operand(B_values, K, N, nnz, L)
             if tiled is not None and not L.scorch_hip_spmm_csr_tiled_recommended(M, K, N, nnz):
                 tiled = None

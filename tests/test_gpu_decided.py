@@ -264,6 +264,48 @@ def test_new_columns_under_known_row_pointers(rows, K, N, per_row):
         product(torch.zeros_like(ci), vals)
 
 
+@pytest.mark.parametrize("rows, K, N, longest", [(4099, 2048, 1000, 40), (1500, 16_384, 2050, 70), (90, 3000, 8200, 1500)])
+def test_new_columns_with_a_dense_operand_stored_by_column_tiles(rows, K, N, longest, monkeypatch):
+    """The kernel looks at the columns itself: the same bits as with columns that were checked before, columns out of range at the
+    first, some and the last entry refused, rows without entries and rows that chunks cut, several streams."""
+    rng = np.random.default_rng(rows)
+    lens = rng.integers(0, longest + 1, rows)
+    lens[[0, rows // 2]] = [longest, 0]
+    rp = dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    nnz = int(lens.sum())
+    assert native.lib().scorch_hip_spmm_csr_tiled_recommended(rows, K, N, nnz)
+    b = torch.randn(K, N, device="cuda")
+    vals = torch.randn(nnz, device="cuda")
+    product = lambda ci: scorch.matmul(STensor.from_csr_arrays(rp, ci, vals, (rows, K)), b)
+    columns = lambda: dev(rng.integers(0, K, nnz).astype(np.int32))
+    for _ in range(3):
+        product(columns())                                # (the copy by column tiles is made for the second one)
+    for at in (0, nnz // 3, nnz - 1):
+        for outside in (K, -1, 2**31 - 1, -2**31):
+            bad = columns()
+            bad[at] = outside
+            with pytest.raises(ValueError, match="column"):
+                product(bad)
+        ci = columns()
+        got = product(ci)
+        with monkeypatch.context() as m:
+            m.setattr(H, "SPMM_PATH", "tiled")
+            assert torch.equal(got, scorch.matmul(STensor.from_csr_arrays(rp.clone(), ci, vals, (rows, K)), b))
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    some = [(s, columns()) for s in streams for _ in range(3)]
+    results = []
+    for s, ci in some:
+        with torch.cuda.stream(s):
+            s.wait_stream(torch.cuda.default_stream())
+            results.append(product(ci))
+    torch.cuda.synchronize()
+    for (_, ci), got in zip(some, results):
+        at = torch.repeat_interleave(torch.arange(rows), torch.from_numpy(lens))
+        want = torch.zeros(rows, K, dtype=torch.float64).index_put_((at, ci.long().cpu()), vals.double().cpu(), accumulate=True)
+        assert _close(got, want @ b.double().cpu(), np.float32)
+
+
 def test_no_memory_for_a_decided_products_result_is_an_error_to_catch(monkeypatch):
     """The native call path allocates the result itself: without memory for it the caller gets torch's
     OutOfMemoryError, as from the general way, and the next product works."""
