@@ -9,12 +9,12 @@
 // it sums (sum over its entries of the length of the B row they select):
 //
 //   up to 32 products    a quarter wavefront, hash table of 64 slots in LDS
-//   up to 256 products   one wavefront, hash table of 512 slots in LDS
+//   up to 256 products   one wavefront, hash table of up to 512 slots in LDS
 //                        (a wavefront takes four consecutive rows: the first kind
 //                        all at once, then the second kind one after the other)
 //   up to 1024 products  one workgroup, hash table of 2048 slots in LDS
 //   up to 4096 products  B of at most 131,072 columns: a bitmap of the columns in LDS
-//                        (256 threads, see below); wider B: one workgroup, hash
+//                        (512 threads, see below); wider B: one workgroup, hash
 //                        table of 8192 slots in LDS
 //   more, B of at most 131,072 columns, and the two passes share what they find out
 //                        the products sorted by ranges of columns (see "the longest rows by
@@ -2325,7 +2325,7 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
                                                                     sync ? sync->target() : nullptr, sync ? sync->sequence() : 0);
       SCORCH_HIP_CHECK(hipGetLastError());
     }
-    // rows the 256-thread bitmap kernel goes through; with the result's row pointer known, also those of the tier above
+    // rows the smaller bitmap kernel goes through; with the result's row pointer known, also those of the tier above
     // that turn out to have few distinct columns
     const int *narrow_rows = NUMERIC && narrow && !bins ? ws.huge_rows : nullptr;
     const auto blocks_for = [&](int64_t rows) {
