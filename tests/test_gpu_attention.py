@@ -415,3 +415,27 @@ def test_rows_shared_out_by_the_size_of_the_launch(oracle, D, S, heads, window, 
         ref = oracle.attention_dense_fp64(q[h].float().cpu().numpy(), k[h].float().cpu().numpy(),
                                           v[h].float().cpu().numpy(), mask, D ** -0.5)
         assert oracle.rel_fro(out[h].float().cpu().numpy(), ref) <= 5e-3
+
+
+# a block row in so many stretches: the combining kernel asks for eight of them at once
+@pytest.mark.parametrize("stretches", [2, 7, 8, 9, 17])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_combining_the_stretches_of_a_long_row(oracle, stretches, D):
+    S, heads, token = 128 * stretches - 64, 2, 70
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = (abs(i - j) <= 20) | (i == token)
+    rows, cols = np.nonzero(mask)
+    row_ptr = np.concatenate(([0], np.cumsum(np.bincount(rows, minlength=S)))).astype(np.int32)
+    g = torch.Generator().manual_seed(stretches + D)
+    q, k, v = (torch.randn(heads, S, D, generator=g) for _ in range(3))
+    k *= torch.linspace(0.1, 4.0, S)[:, None]  # the stretches' maxima differ
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    bm = H.attention_block_mask(dev(row_ptr), dev(cols.astype(np.int32)), S)
+    plain = H.BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)
+    plain.block_row_lens = bm.row_lens()
+    H.split_long_block_rows(plain, 2, list_unequal_rows=True)
+    assert int(plain.split_rows.view(-1, 4)[:, 2].max()) == stretches
+    out = H._attn_bf16_items(q.cuda(), k.cuda(), v.cuda(), bm, plain.items, plain.split_rows, plain.n_slots, D ** -0.5, False)
+    for h in range(heads):
+        ref = oracle.attention_dense_fp64(*(t[h].float().numpy() for t in (q, k, v)), mask, D ** -0.5)
+        assert oracle.rel_fro(out[h].float().cpu().numpy(), ref) <= TOL_BF16
