@@ -343,7 +343,11 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(D
 }
 
 // The block rows that went out in stretches: C = the stretches' sums added in their order.
-// One workgroup per (split row, head); split_rows: x = block row, y = first slot, z = stretches.
+// A workgroup to 1,024 elements of a (split row, head); split_rows: x = block row, y = first slot, z = stretches.
+// What bounds it is the chain of reads: eight stretches are requested together.  The product with a workgroup to the whole tile and a
+// stretch's read waiting for the one before, and so, us: window of 64 and a global token (4,096 rows, 1 head, N = 64) 28.6, 19.7, (8 heads)
+// 37.9, 28.4; window of 128 (2,048, 8, 128) 47.6, 41.2, (8,192, 4, 64, three such tokens) 57.9, 48.1; causal (4,096, 2, 128) 89.8, 84.3.
+constexpr int kMergeAtOnce = 8;
 template <int D>
 __global__ __launch_bounds__(kBlockThreads) void spmm_blocked_merge_kernel(int M, int n_slots,
                                                                            const int4 *__restrict__ split_rows,
@@ -351,18 +355,24 @@ __global__ __launch_bounds__(kBlockThreads) void spmm_blocked_merge_kernel(int M
                                                                            float *__restrict__ C) {
   const int4 row = split_rows[blockIdx.x];
   const int head = blockIdx.y;
-  constexpr int kTile = kBlock * D;  // floats; 256 threads x 4 floats per pass
-  const float *base = partials + ((size_t)head * n_slots + row.y) * kTile;
-  float *out = C + ((size_t)head * M + (size_t)row.x * kBlock) * D;
-  for (int at = threadIdx.x * 4; at < kTile; at += kBlockThreads * 4) {
-    floatx4 sum = *reinterpret_cast<const floatx4 *>(base + at);
-    for (int p = 1; p < row.z; ++p) {
-      const floatx4 x = *reinterpret_cast<const floatx4 *>(base + (size_t)p * kTile + at);
+  constexpr int kTile = kBlock * D;  // floats
+  static_assert(kTile % (kBlockThreads * 4) == 0, "whole workgroups");
+  const int at = ((int)blockIdx.z * kBlockThreads + (int)threadIdx.x) * 4;
+  const float *base = partials + ((size_t)head * n_slots + row.y) * kTile + at;
+  floatx4 sum = *reinterpret_cast<const floatx4 *>(base);
+  for (int p = 1; p < row.z; p += kMergeAtOnce) {
+    floatx4 x[kMergeAtOnce];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sum[r] += x[r];
-    }
-    *reinterpret_cast<floatx4 *>(out + at) = sum;
+    for (int u = 0; u < kMergeAtOnce; ++u)  // (past the last: the last again)
+      x[u] = *reinterpret_cast<const floatx4 *>(base + (size_t)min(p + u, row.z - 1) * kTile);
+#pragma unroll
+    for (int u = 0; u < kMergeAtOnce; ++u)
+      if (p + u < row.z) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[r] += x[u][r];
+      }
   }
+  *reinterpret_cast<floatx4 *>(C + ((size_t)head * M + (size_t)row.x * kBlock) * D + at) = sum;
 }
 
 static int check_blocked(const char *fn, int64_t H, int64_t M, int64_t K, int64_t D, int64_t nnz, int64_t n_active,
@@ -469,7 +479,7 @@ extern "C" int scorch_hip_spmm_csr_blocked_f32(int64_t H, int64_t M, int64_t K, 
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)(n_items * H));
-  const dim3 merge_grid((unsigned)n_split_rows, (unsigned)H);
+  const dim3 merge_grid((unsigned)n_split_rows, (unsigned)H, (unsigned)(blocked::kBlock * N / (4 * kBlockThreads)));
   SCORCH_REQUIRE(aligned_to(block_cols, 8), "%s: block_cols must be 8-byte aligned", fn);
   const unsigned long long *words = reinterpret_cast<const unsigned long long *>(block_words);
   const unsigned long long *cols = reinterpret_cast<const unsigned long long *>(block_cols);

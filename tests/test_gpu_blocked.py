@@ -117,6 +117,20 @@ def test_rectangular_masks_and_head_counts(oracle, shape, heads):
     check_values(oracle, rp, ci, mv, A, B, P, V, out, rows, c)
 
 
+# a block row that holds everything, in stretches of five: the kernel that adds them up asks for eight at once
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("stretches", [2, 8, 9, 10, 18])
+def test_adding_up_the_stretches_of_a_long_row(oracle, stretches, D):
+    rng = np.random.default_rng(D + stretches)
+    M = 64 * 5 * stretches
+    i, j = np.arange(M)[:, None], np.arange(M)[None, :]
+    rp, ci = csr_of((abs(i - j) <= 40) | (i == 70))
+    mv, A, B, P, V = operands(rng, 2, M, M, D, ci.size)
+    out, rows, c, plan = products(rp, ci, mv, A, B, P, V)
+    assert plan.blocked.spmm_split_rows.view(-1, 4)[:, 2].tolist() == [stretches]
+    check_values(oracle, rp, ci, mv, A, B, P, V, out, rows, c)
+
+
 @pytest.mark.parametrize("D", [32, 128])
 def test_thinly_filled_blocks_when_forced(oracle, D):
     """Two stored entries in a hundred: every row of every block is partly stored, most words
