@@ -538,23 +538,6 @@ SCORCH_HIP_API int scorch_hip_spmv_csr_planned_i64(
     const void *bounds, size_t bounds_bytes, void *workspace, size_t workspace_bytes, int32_t *counters, int64_t n_counters,
     void *stream);
 
-/* SpMV over a copy of the entries in which the whole chip reads x from one end to the other: for a matrix that comes
- * back with the same values and an x that does not fit an L2 (_recommended; at most 2^22 columns).  The copy takes
- * _bytes and is made from checked indices by _copy_; `copy` is 256-byte aligned.  longest_row: of the matrix, 0 if not
- * known (a launch that folds rows cut between wavefronts is left out where it tells that there are none).  Results
- * repeat bit for bit; they differ from the other entry points' in rounding (products are added up in fp64, by columns). */
-SCORCH_HIP_API int scorch_hip_spmv_csr_listed_recommended(int64_t M, int64_t K, int64_t nnz, size_t elem_size);
-SCORCH_HIP_API size_t scorch_hip_spmv_csr_listed_bytes(int64_t M, int64_t nnz, size_t elem_size);
-SCORCH_HIP_API size_t scorch_hip_spmv_csr_listed_workspace_bytes(int64_t M, int64_t nnz);
-SCORCH_HIP_API int scorch_hip_spmv_csr_listed_copy_f32(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
-                                           const float *vals, void *copy, size_t copy_bytes, void *stream);
-SCORCH_HIP_API int scorch_hip_spmv_csr_listed_copy_f64(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const int32_t *col_idx,
-                                           const double *vals, void *copy, size_t copy_bytes, void *stream);
-SCORCH_HIP_API int scorch_hip_spmv_csr_listed_f32(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const void *copy, size_t copy_bytes, const float *x,
-                                      float *y, void *workspace, size_t workspace_bytes, int64_t longest_row, void *stream);
-SCORCH_HIP_API int scorch_hip_spmv_csr_listed_f64(int64_t M, int64_t K, int64_t nnz, const int32_t *row_ptr, const void *copy, size_t copy_bytes, const double *x,
-                                      double *y, void *workspace, size_t workspace_bytes, int64_t longest_row, void *stream);
-
 /* B (K, N) row by row from its transpose X, an (N, K) array: what a product with a transposed view
  * needs first. */
 SCORCH_HIP_API int scorch_hip_dense_to_rows_f32(int64_t K, int64_t N, const float *X, float *B, void *stream);

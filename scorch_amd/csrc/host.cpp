@@ -30,7 +30,7 @@ namespace {
 
 // ---- names and objects looked up once ---------------------------------------------------------
 PyObject *n_storage, *n_index, *n_value, *n_shape, *n_mode_indices, *n_format, *n_routes, *n_spmm_path, *n_blocked_path,
-    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_ones, *n_swept, *n_streams, *n_dtype, *n_device;
+    *n_sddmm_path, *n_empty, *n_workspaces, *n_counters, *n_tiled, *n_seen, *n_volatile, *n_epoch, *n_attention, *n_ones, *n_streams, *n_dtype, *n_device;
 PyObject *g_ops = nullptr;        // scorch_ops_hip's namespace
 PyObject *g_stensor = nullptr;    // the STensor type
 PyObject *g_torch_empty = nullptr;
@@ -92,7 +92,7 @@ bool unchanged(const Mark &m) {
   return t.const_data_ptr() == m.data && version_of(t) == m.version && t.numel() == m.numel && epoch_of(m.obj) == m.epoch;
 }
 
-enum Kind { kRows = 0, kPlanned = 1, kBlockedSpmm = 2, kSpmv = 3, kSddmmCsr = 4, kSddmmListed = 5, kSddmmCoo = 6, kBlockedSddmm = 7, kSpmvSwept = 8 };
+enum Kind { kRows = 0, kPlanned = 1, kBlockedSpmm = 2, kSpmv = 3, kSddmmCsr = 4, kSddmmListed = 5, kSddmmCoo = 6, kBlockedSddmm = 7 };
 
 // One decided product: everything about the call that does not change from call to call.
 struct Route {
@@ -109,8 +109,8 @@ struct Route {
   PyObject *keep;     // strong: what `q` and `row_ptr` point into
   PyObject *spmm_path, *other_path;   // strong: the module settings the decision was made under
   uint32_t value_version;
-  PyObject *verdict;                  // SDDMM: the attribute that says whether the mask's values are all 1; kSpmvSwept: the copy's note (strong, or null)
-  const void *value_data;             // the values that is about
+  PyObject *verdict;                  // SDDMM: the attribute that says whether the mask's values are all 1 (strong, or null)
+  const void *value_data;             // SDDMM: the mask's values the verdict in mask_values is about
   PyObject *rows;                     // SDDMM over a CSR mask: the result's row coordinates (strong)
 };
 
@@ -335,10 +335,6 @@ PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
   const at::Tensor &vt = THPVariable_Unpack(o->value);
   if (vt.scalar_type() != o->dtype || vt.numel() != o->second.numel || !vt.is_contiguous() || vt.get_device() != o->device)
     return none();
-  // (a copy of the values holds while they are as they were; mark_volatile() takes its note away)
-  if (r->kind == kSpmvSwept && (vt.const_data_ptr() != r->value_data || version_of(vt) != r->value_version ||
-                                item(dict_of(o->value), n_swept) != r->verdict))
-    return none();
   const void *bias_ptr = nullptr;
   if (act) {
     if (!fits(bias, o, 1, at::kFloat)) return none();
@@ -411,13 +407,6 @@ PyObject *spmm_body(PyObject *const *args, Py_ssize_t n) {
                                   stream)
     SCORCH_BY_TYPE(SCORCH_CALL)
 #undef SCORCH_CALL
-  } else if (r->kind == kSpmvSwept) {
-    if (o->dtype == at::kDouble)
-      rc = scorch_hip_spmv_csr_listed_f64(M, K, nnz, pos, r->q[0], (size_t)r->p[0], at_<double>(B), static_cast<double *>(C), ws, ws_bytes,
-                                         r->p[2], stream);
-    else
-      rc = scorch_hip_spmv_csr_listed_f32(M, K, nnz, pos, r->q[0], (size_t)r->p[0], at_<float>(B), static_cast<float *>(C), ws, ws_bytes,
-                                         r->p[2], stream);
   } else if (r->kind == kBlockedSpmm) {
     rc = scorch_hip_spmm_csr_blocked_f32(1, M, K, N, nnz, r->p[0], at_<int32_t>(r->q[0]), at_<uint64_t>(r->q[1]),
                                          at_<int32_t>(r->q[2]), at_<uint64_t>(r->q[3]), r->p[1], at_<int32_t>(r->q[4]),
@@ -525,7 +514,7 @@ PyObject *remember_body(PyObject *args) {
   r.value_data = vt.const_data_ptr();
   r.value_version = version_of(vt);
   r.keep = tensors, r.spmm_path = path, r.other_path = other, r.rows = rows == Py_None ? nullptr : rows;
-  r.verdict = item(dict_of(p.value), kind == kSpmvSwept ? n_swept : n_ones);
+  r.verdict = item(dict_of(p.value), n_ones);
   for (PyObject *x : {r.keep, r.spmm_path, r.other_path, r.rows, r.verdict}) Py_XINCREF(x);
   auto drop = [](Route &x) {
     for (PyObject *y : {x.keep, x.spmm_path, x.other_path, x.rows, x.verdict}) Py_XDECREF(y);
@@ -750,7 +739,7 @@ PyMODINIT_FUNC PyInit__host() {
                {&n_spmm_path, "SPMM_PATH"}, {&n_blocked_path, "BLOCKED_PATH"}, {&n_sddmm_path, "SDDMM_PATH"},
                {&n_empty, "_empty"}, {&n_workspaces, "_workspaces"}, {&n_counters, "_counter_buffers"}, {&n_tiled, "_scorch_tiled"}, {&n_seen, "_scorch_seen"},
                {&n_volatile, "_scorch_volatile"}, {&n_epoch, "_scorch_epoch"}, {&n_attention, "_scorch_attention"},
-               {&n_ones, "_scorch_ones"}, {&n_swept, "_scorch_swept"}, {&n_streams, "_scorch_streams"}, {&n_dtype, "dtype"}, {&n_device, "device"}};
+               {&n_ones, "_scorch_ones"}, {&n_streams, "_scorch_streams"}, {&n_dtype, "dtype"}, {&n_device, "device"}};
   for (const auto &x : names) *x.slot = PyUnicode_InternFromString(x.text);
   OperandType.tp_name = "scorch_amd._host.Operand";
   OperandType.tp_basicsize = sizeof(Operand);

@@ -23,7 +23,6 @@ hipError_t preload_spmm();
 hipError_t preload_spmm_panels();
 hipError_t preload_spmm_rows();
 hipError_t preload_spmm_tiled();
-hipError_t preload_spmv_swept();
 hipError_t preload_sync();
 }  // namespace scorch
 
@@ -194,7 +193,7 @@ int scorch_hip_init(void) {
   hipError_t (*const loaders[])() = {scorch::preload_attn,      scorch::preload_attn_f32, scorch::preload_blockdesc,
                                      scorch::preload_blocked,   scorch::preload_misc,     scorch::preload_sddmm,
                                      scorch::preload_spgemm,    scorch::preload_spmm,     scorch::preload_spmm_rows, scorch::preload_spmm_panels,
-                                     scorch::preload_spmm_tiled, scorch::preload_spmv_swept, scorch::preload_sync};
+                                     scorch::preload_spmm_tiled, scorch::preload_sync};
   for (auto load : loaders) SCORCH_HIP_CHECK(load());
   return SCORCH_HIP_OK;
 }

@@ -95,11 +95,6 @@ SIGNATURES = {
     "scorch_hip_spmv_csr_bounds": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _size, _ptr]),
     **{"scorch_hip_spmv_csr_planned_" + t: (ctypes.c_int, [_i64] * 3 + [_ptr] * 6 + [_size, _ptr, _size, _ptr, _i64, _ptr])
        for t in ("f32", "f64", "i32", "i64")},
-    "scorch_hip_spmv_csr_listed_recommended": (ctypes.c_int, [_i64, _i64, _i64, _size]),
-    "scorch_hip_spmv_csr_listed_bytes": (_size, [_i64, _i64, _size]),
-    "scorch_hip_spmv_csr_listed_workspace_bytes": (_size, [_i64, _i64]),
-    **{"scorch_hip_spmv_csr_listed_copy_" + t: (ctypes.c_int, [_i64] * 3 + [_ptr] * 4 + [_size, _ptr]) for t in ("f32", "f64")},
-    **{"scorch_hip_spmv_csr_listed_" + t: (ctypes.c_int, [_i64] * 3 + [_ptr, _ptr, _size] + [_ptr] * 3 + [_size, _i64, _ptr]) for t in ("f32", "f64")},
     "scorch_hip_dense_to_rows_f32": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr]),
     "scorch_hip_csr_inspect_columns_begin": (ctypes.c_int, [_i64, _i64, _ptr, _ptr, _ptr, ctypes.POINTER(_ptr)]),
     "scorch_hip_spmm_csr_tiled_new_columns_f32": (ctypes.c_int, [_i64] * 4 + [_ptr] * 4 + [_size, _ptr, _ptr, _size, _i64, _ptr, ctypes.POINTER(_ptr)]),

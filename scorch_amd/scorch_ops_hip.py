@@ -185,16 +185,14 @@ class _on_device:
 #   from index tensors   the CsrPlan (validity, longest row, chunk boundaries, entry lists, block
 #                        description), the row pointer of a coordinate mask, an attention mask's blocks
 #   from value tensors   the column-tile copy of a wide dense operand, "this mask's values are all 1", a
-#                        mask's values in the order of its SDDMM entry lists, a matrix's entries in the order of
-#                        the columns for products with vectors
+#                        mask's values in the order of its SDDMM entry lists
 # Each is stamped with the tensor's address, its version counter and its epoch (below), and rebuilt
 # when the stamp no longer matches.  PyTorch bumps the version counter for every in-place operation
 # of its own on the tensor or on a view of it.  It does not for writes through ``t.data``, a raw
 # pointer, a numpy or DLPack alias, a kernel of another library, or the replay of a recorded graph:
 # after such a write call forget(t), or mark the tensor volatile once.
 _CACHE_ATTRIBUTES = ("_scorch_plan", "_scorch_tiled", "_scorch_seen", "_scorch_ones", "_scorch_listed", "_scorch_coo_pos",
-                     "_scorch_block_mask", "_scorch_mask_checked", "_scorch_rows", "_scorch_row_order", "_scorch_attention",
-                     "_scorch_swept")
+                     "_scorch_block_mask", "_scorch_mask_checked", "_scorch_rows", "_scorch_row_order", "_scorch_attention")
 
 
 class _Kept(tuple):
@@ -284,7 +282,7 @@ def mark_volatile(*objs, volatile: bool = True) -> None:
     index tensor (a sparsity pattern) is not affected: use forget() when a pattern is rewritten."""
     for t in _tensors_of(objs):
         if volatile:
-            for name in ("_scorch_tiled", "_scorch_seen", "_scorch_ones", "_scorch_listed", "_scorch_swept"):
+            for name in ("_scorch_tiled", "_scorch_seen", "_scorch_ones", "_scorch_listed"):
                 if hasattr(t, name):
                     delattr(t, name)
         try:
@@ -960,7 +958,7 @@ def _spmm_launch(plan: Optional[CsrPlan], of_these_columns: bool, dtype, M, K, N
 
 # What the native call path does with a decided product (the enum Kind of csrc/host.cpp)
 _ROUTE_ROWS, _ROUTE_PLANNED, _ROUTE_BLOCKED_SPMM, _ROUTE_SPMV, _ROUTE_SDDMM_CSR, _ROUTE_SDDMM_LISTED, _ROUTE_SDDMM_COO, \
-    _ROUTE_BLOCKED_SDDMM, _ROUTE_SPMV_SWEPT = range(9)
+    _ROUTE_BLOCKED_SDDMM = range(8)
 
 
 def remember_spmm(a, width: int, act: int = 0) -> None:
@@ -999,12 +997,6 @@ def remember_spmm(a, width: int, act: int = 0) -> None:
 
     if width < 0:
         if not pos_of_coo:
-            if _swept_applies(plan, M, K, vals, L):
-                kept = _kept(vals, "_scorch_swept")
-                if kept is not None and kept[0] == _stamp(vals) and kept[1] is plan and isinstance(kept[2], torch.Tensor):
-                    remember(_ROUTE_SPMV_SWEPT, (kept[2].numel(), 0, plan.max_row), (kept[2],),
-                             L.scorch_hip_spmv_csr_listed_workspace_bytes(M, nnz))
-                return              # (open until the copy is made)
             bounds = plan.bounds.get("spmv")
             if bounds is None:
                 return
@@ -1246,47 +1238,6 @@ def _spmv_bounds(plan: CsrPlan, pos: torch.Tensor, M: int, nnz: int, L, stream) 
 
 
 # ---- SpMV ----------------------------------------------------------------------
-def _swept_applies(plan: Optional[CsrPlan], M: int, K: int, values: torch.Tensor, L) -> bool:
-    """Whether products of this matrix with vectors are served from a copy of its entries, if it comes back unchanged."""
-    return plan is not None and values.dtype in (torch.float32, torch.float64) and not is_volatile(values) \
-        and bool(L.scorch_hip_spmv_csr_listed_recommended(M, K, values.numel(), values.element_size()))
-
-
-# The copy costs about what four products gain by it (1 M rows, 17.8 M entries, fp64: 346 us, 100 a product): it is made when
-# that many have gone without.  Results differ from the merge kernel's in rounding, and repeat bit for bit from then on.
-SWEPT_AFTER = 4
-
-
-def _swept_copy(plan: Optional[CsrPlan], pos, crd, M: int, K: int, values: torch.Tensor, L, stream) -> Optional[torch.Tensor]:
-    """The matrix's entries in the order in which the chip sweeps x, as kept with its values: made
-    after SWEPT_AFTER products in a row with the same unchanged values and pattern, else None.  Never while
-    a stream is capturing: the values may be rewritten before a replay."""
-    if torch.cuda.is_current_stream_capturing() or not _swept_applies(plan, M, K, values, L):
-        return None
-    key = _stamp(values)
-    kept = _kept(values, "_scorch_swept")
-    uses = kept[2] if kept is not None and kept[0] == key and kept[1] is plan else 0
-    if isinstance(uses, int):
-        if uses < SWEPT_AFTER:
-            try:
-                values._scorch_swept = _Kept((key, plan, uses + 1))
-            except (AttributeError, RuntimeError):
-                pass
-            return None
-        nnz, elem = values.numel(), values.element_size()
-        try:
-            copy = _empty(L.scorch_hip_spmv_csr_listed_bytes(M, nnz, elem), dtype=torch.uint8, device=values.device)
-        except torch.OutOfMemoryError:
-            del values._scorch_swept        # (asked for again as many products on; the merge kernel needs none)
-            return None
-        native.check(getattr(L, "scorch_hip_spmv_csr_listed_copy_" + _SUFFIX[values.dtype])(
-            M, K, nnz, pos.data_ptr(), crd.data_ptr(), values.data_ptr(), copy.data_ptr(), copy.numel(), stream))
-        _made_on(stream, copy)
-        kept = values._scorch_swept = _Kept((key, plan, copy))
-    _for_use_on(values.device, stream, kept[2])
-    return kept[2]
-
-
 def _make_spmv(dtype):
     def kernel(result_shape, A_shape, A_mode_indices, A_values, B_shape, B_mode_indices, B_values):
         M, K = int(A_shape[0]), int(A_shape[1])
@@ -1302,13 +1253,6 @@ def _make_spmv(dtype):
         nnz = a_val.numel()
         with _on_device(dev):
             stream = _stream(dev)
-            swept = _swept_copy(plan, pos, crd, M, K, a_val, L, stream)
-            if swept is not None:
-                ws = _workspace(dev, stream, L.scorch_hip_spmv_csr_listed_workspace_bytes(M, nnz))
-                native.check(getattr(L, "scorch_hip_spmv_csr_listed_" + _SUFFIX[dtype])(
-                    M, K, nnz, pos.data_ptr(), swept.data_ptr(), swept.numel(), x.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel(),
-                    plan.max_row, stream))
-                return Tensor(y, [[]])
             ws = _workspace(dev, stream, L.scorch_hip_spmv_csr_workspace_bytes(M, nnz, a_val.element_size()))
             bounds = _spmv_bounds(plan, pos, M, nnz, L, stream) if plan is not None else None
             fn = getattr(L, "scorch_hip_spmv_csr_planned_" + _SUFFIX[dtype])

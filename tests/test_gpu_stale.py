@@ -240,3 +240,36 @@ def test_operands_made_in_inference_mode(form):
             dc[0] = n + 5
             with pytest.raises(ValueError, match="column"):
                 scorch.matmul(A, b)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_products_with_vectors_read_the_values_that_are_in_memory(dtype):
+    """A matrix whose vector is larger than an L2 keeps, multiplied time and again, its values written in
+    between by ``.data`` and by a recorded step that closes over them: nobody is told, and nothing may be derived
+    from values of before."""
+    rng = np.random.default_rng(60)
+    M, K, per_row = 3000, 900_000, 600
+    rp = np.arange(0, M * per_row + 1, per_row, dtype=np.int32)
+    ci = np.sort(rng.integers(0, K, (M, per_row)), axis=1).astype(np.int32)
+    v, x = rng.uniform(0.5, 1, ci.shape).astype(dtype), rng.uniform(0.5, 1, K).astype(dtype)
+    A = scorch.STensor.from_csr_arrays(dev(rp), dev(ci.reshape(-1)), dev(v.reshape(-1)), (M, K))
+    t_x = dev(x)
+    want = (v.astype(np.float64) * x.astype(np.float64)[ci]).sum(axis=1)
+    rel = 600 * (2.0 ** -24 if dtype == np.float32 else 2.0 ** -53)     # a rounding a term, all of one sign
+
+    def products(scale, n=7):
+        for _ in range(n):
+            np.testing.assert_allclose(host(scorch.matmul(A, t_x)).astype(np.float64), want * scale, rtol=rel)
+
+    products(1.0)
+    version = A.values._version
+    A.values.data.mul_(2.0)
+    assert A.values._version == version                      # the write the stamp cannot see
+    products(2.0)
+    step = graphs.capture(lambda b: (A.values.mul_(0.5), scorch.matmul(A, b))[1], t_x)
+    torch.cuda.synchronize()
+    A.values.copy_(dev(v.reshape(-1)))
+    products(1.0)
+    for scale in (0.5, 0.25, 0.125):
+        step()
+        products(scale)
