@@ -1448,8 +1448,11 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
 #pragma unroll
         for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (steps[s].first + u * kWaveSize + wave_lane() < steps[s].last) atomicOr(&s_bits[col[s][u] >> 5], 1u << (col[s][u] & 31));
+          for (int u = 0; u < U; ++u) {  // (a column outside of B is left out, as by the walk and by `add` below)
+            const unsigned rel = (unsigned)col[s][u];
+            if (steps[s].first + u * kWaveSize + wave_lane() < steps[s].last && rel < (unsigned)columns)
+              atomicOr(&s_bits[rel >> 5], 1u << (rel & 31));
+          }
       } else {
         for_each_product<THREADS, false, T, A>(
             a_lo, a_hi, tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan, [&](int k, A) {

@@ -578,3 +578,51 @@ def test_rows_at_the_edges_of_the_tiers_of_a_large_matrix(oracle, dtype, N):
     draw = (lambda n: rng.integers(-9, 10, n).astype(dtype)) if np.issubdtype(dtype, np.integer) else \
         (lambda n: (rng.random(n) + 0.5).astype(dtype))
     check(oracle, arp, aci, draw(M), brp, bci, draw(len(bci)), N)
+
+
+@pytest.mark.parametrize("suffix, dtype", [("f32", np.float32), ("i64", np.int64)])
+@pytest.mark.parametrize("M", [60, 32_768 + 7])
+def test_columns_outside_of_b_are_left_out_of_rows_summed_by_a_bitmap(suffix, dtype, M):
+    """The bare C calls look at no indices beforehand.  Rows of 1,025 to 4,096 products, of few entries and of more than
+    threads: both passes leave a column outside [0, N) out.  Whole numbers: every sum is exact."""
+    from scorch_amd import native
+    N, rng = 70_001, np.random.default_rng(M)
+    lens = [1025, 2048, 4096, 300, 5]
+    bci = [rng.choice(N, n, replace=False) for n in lens]
+    outside = np.array([N, N + 31, 131_071, 131_072, 2**31 - 1, -1, -(2**31)])
+    for at in bci:
+        k = min(at.size - 1, outside.size)
+        at[rng.choice(at.size, k, replace=False)] = outside[:k]
+    rows = {0: [0], 7: [1], 8: [2], M - 1: [0, 1, 3], 40: [3] * 4 + [4] * 500}
+    aci = np.concatenate([rows[r] for r in sorted(rows)]).astype(np.int32)
+    arp = np.zeros(M + 1, np.int32)
+    for r, entries in rows.items():
+        arp[r + 1] = len(entries)
+    arp = np.cumsum(arp).astype(np.int32)
+    brp, bci = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), np.concatenate(bci).astype(np.int32)
+    av, bv = (rng.integers(-3, 4, n).astype(dtype) for n in (aci.size, bci.size))
+    assert all(1024 < sum(lens[j] for j in e) <= 4096 for e in rows.values())
+    L, K = native.lib(), len(lens)
+    d = [dev(x) for x in (arp, aci, av, brp, bci, bv)]
+    ap, ac, a, bp, bc, b = (x.data_ptr() for x in d)
+    ws = torch.full((L.scorch_hip_spgemm_csr_workspace_bytes(M, N, 8),), 0x7F, dtype=torch.uint8, device="cuda")
+    c_pos = torch.empty(M + 1, dtype=torch.int32, device="cuda")
+    native.check(L.scorch_hip_spgemm_csr_symbolic(M, K, N, ap, ac, bp, bc, c_pos.data_ptr(), ws.data_ptr(), ws.numel(), None))
+    want = np.zeros((len(rows), N), np.int64)
+    stored = np.zeros((len(rows), N), bool)
+    for i, r in enumerate(sorted(rows)):
+        for p in range(arp[r], arp[r + 1]):
+            q = np.arange(brp[aci[p]], brp[aci[p] + 1])
+            q = q[(bci[q] >= 0) & (bci[q] < N)]
+            want[i, bci[q]] += int(av[p]) * bv[q].astype(np.int64)
+            stored[i, bci[q]] = True
+    counts = np.zeros(M + 1, np.int64)
+    counts[np.array(sorted(rows)) + 1] = stored.sum(axis=1)
+    assert np.array_equal(host(c_pos), np.cumsum(counts))
+    nnz = int(counts.sum())
+    c_crd = torch.full((nnz,), -1, dtype=torch.int32, device="cuda")
+    c_val = torch.zeros(nnz, dtype=d[2].dtype, device="cuda")
+    native.check(getattr(L, "scorch_hip_spgemm_csr_numeric_" + suffix)(
+        M, K, N, ap, ac, a, bp, bc, b, c_pos.data_ptr(), c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), None))
+    assert np.array_equal(host(c_crd), np.nonzero(stored)[1])
+    assert np.array_equal(host(c_val), want[stored].astype(dtype))
