@@ -1316,8 +1316,9 @@ __global__ __launch_bounds__(kHugeThreads) void spgemm_huge_kernel(
 // row's first kAccEntries output entries (the others are added into the output
 // with global atomics as above).
 constexpr int kLdsBudget = 160 * 1024 - 1024;
-// The tier of up to kMediumProducts products: with 16-bit ranks, and sums of the last hundred of the longest rows in the
-// output, four workgroups of eight wavefronts fill a CU (256 threads, four of four, 2,600 rows: 67 us, 512 60).
+// The numeric pass of the tier of up to kMediumProducts products: with 16-bit ranks, and sums of the last hundred of the longest rows
+// in the output, four workgroups of eight wavefronts fill a CU (256 threads, four of four, 2,600 rows: 67 us, 512 60).  The symbolic
+// pass has neither ranks nor sums in LDS and needs no larger workgroups to fill a CU: kBlockThreads (512: 19.2 us, 256 18.1).
 constexpr int kBitmapThreads = 512, kBitmapSums = 3968;
 
 // THREADS: workgroup size.  ACC: LDS sums to provide (0: all the LDS that is left).
@@ -2356,8 +2357,9 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
       }
       if (bitmap_blocks && narrow) {
         // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
-        spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kBitmapThreads, kBitmapSums, 0, 4>
-            <<<bitmap_blocks, kBitmapThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
+        constexpr int kThreads = NUMERIC ? kBitmapThreads : kBlockThreads;
+        spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kThreads, kBitmapSums, 0, 4>
+            <<<bitmap_blocks, kThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
                                                           narrow_rows, ws.counters, c_pos, c_crd, c_val);
       } else if (bitmap_blocks) {
         // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
