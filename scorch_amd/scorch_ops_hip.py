@@ -2141,9 +2141,13 @@ def _fp32_stretch(lens, heads: int, D: int, n_cus: int) -> Optional[int]:
 
 
 def _eight_at_once(lens, heads: int, D: int, n_cus: int) -> bool:
-    """Whether stretches of eight key blocks serve a few long rows at D = 32 better than four: a stretch's tiles go to
-    four wavefronts (csrc/attn_f32.hip) and are half as long, and a CU's share is five blocks or more (in units of D = 64).
-    Window of 64 and a global token, 16 heads, us: S = 3,001 23.7 -> 22.6, 6,075 41.3 -> 37.3; 1,024, 12 heads 13.9 -> 15.6."""
+    """Whether stretches of eight key blocks serve a few long rows at D = 32 better than four, in a mask of partly live blocks: a
+    stretch's tiles go to four wavefronts (csrc/attn_f32.hip) and are half as long, and a CU's share is five blocks or more (in units
+    of D = 64).  Fours and eights, us, by that share.  Window of 64 and a global token, (tokens, heads): 1.7 (1,024, 12) 13.7, 15.6;
+    3.6 (2,048, 12) 17.6, 19.1; 3.6 (3,008, 8) 18.0, 17.5; 4.8 (2,048, 16) 18.7, 20.8; 4.9 (4,096, 8) 21.3, 20.3; 5.4 (3,008, 12)
+    23.4, 21.6; 7.4 (4,096, 12) 27.7, 25.6; 9.6 (2,048, 32) 28.5, 28.6; 9.9 (8,192, 8) 33.0, 30.0; 14.7 (6,080, 16) 42.9, 37.9.  Window of
+    128: 6.6 (2,048, 16) 32.4, 24.9; 64 global tokens: 7.2 (3,008, 16) 32.9, 30.7.  Below five it depends on more than the share.
+    (Whole blocks go to the other kernel, a workgroup to a stretch: 5.4 (3,008, 12) 25.5, 32.6; 9.8 (4,096, 16) 34.7, 40.0.)"""
     if D != 32 or float(lens.sum()) * heads / n_cus * D / 64 < 5:
         return False
     slots = int(-(-lens[lens > 8] // 8).sum())
@@ -2159,7 +2163,7 @@ def _fp32_launch_schedule(bm: BlockMask, heads: int, D: int):
         if bm.schedule32 is None:          # (being recorded, with nothing decided before)
             return kept
         stretch = _fp32_stretch(bm.row_lens(), heads, D, _cu_count(bm.block_row_ptr.device))
-        if stretch == 4 and _eight_at_once(bm.row_lens(), heads, D, _cu_count(bm.block_row_ptr.device)):
+        if stretch == 4 and bm.block_masks is not None and bm.n_masks and _eight_at_once(bm.row_lens(), heads, D, _cu_count(bm.block_row_ptr.device)):
             stretch = 8
         if stretch is not None and not torch.cuda.is_current_stream_capturing():
             plain = BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)

@@ -702,6 +702,21 @@ def test_stretches_of_eight_for_a_few_long_rows(lens, heads, D, want):
     assert scorch_ops_hip._eight_at_once(lens, heads, D, 256) == want
 
 
+@pytest.mark.parametrize("n_masks, want", [(None, 4), (0, 4), (1, 8)])
+def test_stretches_of_eight_are_for_masks_of_partly_live_blocks(monkeypatch, n_masks, want):
+    """The kernel for whole blocks has one workgroup to a stretch and keeps stretches of four."""
+    lens = _rows((3, 63), (64, 1))
+    block_row_ptr = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    n = int(lens.sum())
+    bm = scorch_ops_hip.BlockMask(4096, 64, block_row_ptr, torch.zeros(n, dtype=torch.int32), torch.full((n,), -1, dtype=torch.int32),
+                                  None if n_masks is None else torch.zeros(64 * n_masks, dtype=torch.int64), 4096 * n)
+    monkeypatch.setattr(scorch_ops_hip, "_cu_count", lambda device: 256)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    items, split_rows, n_slots = scorch_ops_hip._fp32_launch_schedule(bm, 16, 32)
+    rows = items.view(-1, 4)
+    assert int((rows[:, 2] - rows[:, 1]).max()) == want and n_slots == 64 // want
+
+
 @pytest.mark.parametrize("lens, heads, D, want", [
     # no row stands out: whole rows, unless half the CUs at most have one and some row has 16 blocks or more
     (_rows((7, 128)), 1, 64, None), (_rows((16, 128)), 1, 64, 8), (_rows((15, 128)), 1, 64, None), (_rows((16, 129)), 1, 64, None),
