@@ -270,6 +270,50 @@ def test_a_few_long_rows_in_stretches_of_four_workgroups_each(oracle, heads, tok
     assert oracle.rel_fro(turned, out) <= TOL
 
 
+@pytest.mark.parametrize("heads, token", [(16, 0), (33, 700)])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_non_finite_values_in_stretches_of_four_workgroups_each(heads, token, D):
+    """NaN, either infinity, both in one sum, values whose products overflow and a NaN in K: in keys that only the query that attends to
+    everything and a window's queries refer to, and in the key that every query does."""
+    S = 1219
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = (abs(i - j) <= 40) | (i == token) | (j == token)
+    rng = np.random.default_rng(heads + D)
+    q, k, v = (rng.standard_normal((heads, S, D)).astype(np.float32) for _ in range(3))
+    last = heads - 1
+    v[0, token, 3] = np.inf
+    v[0, S // 2] = np.nan
+    v[0, S - 1, ::2] = -np.inf
+    v[0, S - 2, 1::3] = np.inf
+    v[1, 7], v[1, 9] = 3e38, -3e38                        # finite, though a product of two is not
+    v[1, S // 3, D - 1] = -np.inf
+    k[last, 300, D // 2] = np.nan                         # a score of NaN: the whole row
+    scale = 0.5 * D ** -0.5                               # (no probability underflows)
+    rp, ci = (dev(x) for x in csr_of(mask))
+    dq, dk, dv = (dev(x) for x in (q, k, v))
+    for call in range(3):
+        out = H.sparse_attention_csr(rp, ci, dq, dk, dv, scale).cpu().numpy()
+    n_items, n_slots = (lambda items, split_rows, slots: (items.numel() // 4, slots))(
+        *H._fp32_launch_schedule(rp._scorch_plan.attention, heads, D))
+    assert 0 < 3 * n_slots <= n_items and heads * n_items > (160 if D == 128 else 320)
+    for h in (0, 1, 2, last):
+        want = np.empty((S, D))
+        with np.errstate(all="ignore"):
+            for row in range(S):
+                keys = np.flatnonzero(mask[row])
+                x = scale * (k[h, keys].astype(np.float64) @ q[h, row].astype(np.float64))
+                p = np.exp(x - x.max())
+                want[row] = (p / p.sum()) @ v[h, keys].astype(np.float64)
+        finite = np.isfinite(want)
+        assert finite.all() == (h == 2) and finite.any()
+        np.testing.assert_array_equal(np.isnan(out[h]), np.isnan(want))
+        np.testing.assert_array_equal(np.isposinf(out[h]), np.isposinf(want))
+        np.testing.assert_array_equal(np.isneginf(out[h]), np.isneginf(want))
+        # sums that may cancel, each rounded a few times: against the magnitudes that go in
+        size = np.abs(want[finite])
+        assert (np.abs(out[h][finite] - want[finite]) <= 1e-5 * np.maximum(size, np.where(size > 1e6, 3e38, 4.0))).all()
+
+
 # a block row in so many stretches: the combining kernel asks for eight of them at once
 @pytest.mark.parametrize("stretches", [2, 7, 8, 9, 17])
 @pytest.mark.parametrize("D", [32, 64, 128])
