@@ -1558,36 +1558,37 @@ __global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
 // each: workgroups [0, n_bitmap) take bitmap rows, the next n_medium hash rows of up to
 // kSmallProducts products, the rest a row of up to kTinyProducts to each wavefront, the longest kinds first.
 // The kinds share the workgroup's LDS (40 KB with fp32 sums, four workgroups to a CU).
-// (512 threads: with 256, rows of 1,024 to 4,096 products took twice the steps, and there are few of them to fill the chip with:
-// 1,500 nodes of 16 86 -> 82 us in all, 25,000 of 10 140 -> 135.)
-constexpr int kSmallMatrixThreads = 512;
-template <typename T, bool NUMERIC>
-__global__ __launch_bounds__(kSmallMatrixThreads) void spgemm_small_matrix_kernel(
+// THREADS: symbolic 256.  Numeric with sums of 8 bytes, whose tables take the LDS, 512: with 256 half of a CU's wavefronts find no room.
+// With sums of 4 bytes 512 for the rows of up to kTinyProducts, and 256 where more than half of the rows have more products (a
+// workgroup's barriers are what these wait for).  The product, us, all with 256 and so, M x N with rows of (products): fp32 30,000 x 30,000
+// (100) 99, 91; fp64 (100) 135, 104; (400) 474, 439; (2,000) 681, 609; all with 512 and so: fp32 30,000 x 30,000 (400) 376, 296;
+// (1,000) 465, 388; (2,000) 515, 455; 8,000 x 3,000 (400) 120, 100.  Graphs of 1,500 nodes of 16 and 25,000 of 10, fp32: 96 and 135 with 256, 92 and 128 so.
+template <typename T, bool NUMERIC, int THREADS>
+__global__ __launch_bounds__(THREADS) void spgemm_small_matrix_kernel(
     int M, int N, int n_bitmap, int n_medium, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
     const T *__restrict__ a_val, const int *__restrict__ b_pos, const int *__restrict__ b_crd,
     const T *__restrict__ b_val, const int *__restrict__ products, const int *__restrict__ small_rows,
     const int *__restrict__ medium_rows, const int *__restrict__ narrow_rows, int *__restrict__ counters,
     int *__restrict__ c_pos, int *__restrict__ c_crd, T *__restrict__ c_val) {
   using A = typename Acc<T>::type;
-  constexpr int kWaves = kSmallMatrixThreads / kWaveSize;
+  constexpr int kWaves = THREADS / kWaveSize;
   union Tables {
-    BitmapTables<A, NUMERIC, kNarrowColumns / 32, kSmallMatrixThreads, kBitmapSums> bitmap;
-    MediumTables<A, NUMERIC, kSmallProducts, kSmallMatrixThreads> medium;
+    BitmapTables<A, NUMERIC, kNarrowColumns / 32, THREADS, kBitmapSums> bitmap;
+    MediumTables<A, NUMERIC, kSmallProducts, THREADS> medium;
     TeamTables<A, NUMERIC, kWaveSize, kWaves, kTinySlots, kTinyProducts> tiny;
   };
   __shared__ Tables lds;
   int block = blockIdx.x;
   if (block < n_bitmap) {
-    spgemm_lds_bitmap_rows<T, NUMERIC, kNarrowColumns / 32, kSmallMatrixThreads, kBitmapSums, 0, 4>(
+    spgemm_lds_bitmap_rows<T, NUMERIC, kNarrowColumns / 32, THREADS, kBitmapSums, 0, 4>(
         lds.bitmap, block, n_bitmap, M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, medium_rows, narrow_rows, counters,
         c_pos, c_crd, c_val);
     return;
   }
   block -= n_bitmap;
   if (block < n_medium) {
-    spgemm_medium_rows<T, NUMERIC, kSmallProducts, 2, kSmallMatrixThreads>(lds.medium, block, n_medium, a_pos, a_crd, a_val, b_pos,
-                                                                    b_crd, b_val, products, small_rows, counters, c_pos,
-                                                                    c_crd, c_val);
+    spgemm_medium_rows<T, NUMERIC, kSmallProducts, 2, THREADS>(lds.medium, block, n_medium, a_pos, a_crd, a_val, b_pos, b_crd, b_val,
+                                                               products, small_rows, counters, c_pos, c_crd, c_val);
     return;
   }
   block -= n_medium;
@@ -2338,8 +2339,14 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
     const unsigned small_blocks = blocks_for(known ? known->small : M);
     const unsigned bitmap_blocks = blocks_for(known ? known->medium + (narrow_rows ? known->huge : 0) : M);
     if (M < 4 * 8192 && narrow) {
-      const unsigned tiny_blocks = (unsigned)((M + kSmallMatrixThreads / kWaveSize - 1) / (kSmallMatrixThreads / kWaveSize));
-      spgemm_small_matrix_kernel<T, NUMERIC><<<bitmap_blocks + small_blocks + tiny_blocks, kSmallMatrixThreads, 0, stream>>>(
+      // (see spgemm_small_matrix_kernel)
+      constexpr int kMore = NUMERIC ? kBitmapThreads : kBlockThreads;
+      const bool few = known && 2 * (known->small + known->medium) < M;
+      const bool more = sizeof(A) > 4 || few;
+      const int threads = more ? kMore : kBlockThreads;
+      const unsigned tiny_blocks = (unsigned)((M + threads / kWaveSize - 1) / (threads / kWaveSize));
+      auto kernel = more ? &spgemm_small_matrix_kernel<T, NUMERIC, kMore> : &spgemm_small_matrix_kernel<T, NUMERIC, kBlockThreads>;
+      kernel<<<bitmap_blocks + small_blocks + tiny_blocks, threads, 0, stream>>>(
           M, N, (int)bitmap_blocks, (int)small_blocks, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows,
           ws.medium_rows, narrow_rows, ws.counters, c_pos, c_crd, c_val);
       SCORCH_HIP_CHECK(hipGetLastError());

@@ -626,3 +626,22 @@ def test_columns_outside_of_b_are_left_out_of_rows_summed_by_a_bitmap(suffix, dt
         M, K, N, ap, ac, a, bp, bc, b, c_pos.data_ptr(), c_crd.data_ptr(), c_val.data_ptr(), ws.data_ptr(), ws.numel(), None))
     assert np.array_equal(host(c_crd), np.nonzero(stored)[1])
     assert np.array_equal(host(c_val), want[stored].astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+@pytest.mark.parametrize("N", [1, 3967, 3968, 3969, 9000])
+@pytest.mark.parametrize("M, short", [(200, 0), (200, 150), (32_767, 20_000), (32_768, 20_000)])
+def test_many_and_few_rows_beyond_a_wavefronts_and_sums_by_column(oracle, dtype, N, M, short):
+    """Most rows of up to 256 products or most of more, the last matrix whose tiers share a launch and the first whose tiers
+    do not, on either side of the number of columns that have a sum each."""
+    rng = np.random.default_rng(N + M)
+    lens = [3, 40, 256, 257, 1024, 1025, 2500, 4096, 4097]
+    brp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    bci = np.concatenate([np.sort(rng.integers(0, N, n)) for n in lens]).astype(np.int32)
+    which = rng.integers(2, 4, M)                          # 256 and 257 products
+    which[:short] = rng.integers(0, 3, short)
+    which[rng.choice(M, 90, replace=False)] = np.tile(np.arange(9), 10)
+    aci = np.sort(np.concatenate([which[:, None], rng.integers(0, 2, (M, 1))], axis=1), axis=1).astype(np.int32).reshape(-1)
+    arp = np.arange(0, 2 * M + 1, 2, dtype=np.int32)
+    value = (lambda n: rng.integers(-9, 10, n).astype(dtype)) if dtype == np.int64 else (lambda n: (rng.random(n) + 0.5).astype(dtype))
+    check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
