@@ -1350,7 +1350,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
   using Tables = BitmapTables<A, NUMERIC, WORDS, THREADS, ACC>;
   constexpr int kAccEntries = Tables::kAccEntries;
   constexpr int kWaves = THREADS / kWaveSize;
-  constexpr bool kHolds = NUMERIC && ACC > 0;
+  constexpr bool kByColumn = NUMERIC && ACC > 0 && 32 * WORDS <= ACC, kHolds = NUMERIC && ACC > 0 && !kByColumn;
   auto &s_bits = lds.bits;
   auto &s_rank = lds.rank;
   auto &s_acc = lds.acc;
@@ -1366,8 +1366,10 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
   A *acc = reinterpret_cast<A *>(c_val);
   // B with no more columns than the LDS holds sums: the numeric pass keeps a sum
   // per column and walks the row's products once (bits and sums together)
-  // instead of twice (bits, then sums at their ranks).
-  const bool sums_by_column = NUMERIC && N <= kAccEntries && N <= kRangeColumns;
+  // instead of twice (bits, then sums at their ranks).  The tier of up to kMediumProducts products has kernels of its own for it
+  // (kByColumn), with a bitmap for as many columns and no registers for held products: fp32 40,000 x 3,000, rows of 2,000 products
+  // 832 -> 715 us, 8,000 x 1,000, 1,600 182 -> 139; fp64 1,102 -> 772, 286 -> 153.
+  const bool sums_by_column = ACC > 0 ? kByColumn : NUMERIC && N <= kAccEntries && N <= kRangeColumns;
 
   // The longest rows are handed out through a counter, one at a time, so that the
   // workgroups stay evenly loaded; the rows of the tier below are short enough
@@ -1405,7 +1407,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
     int col[kSteps][U];
     A product[kSteps][U];
     ProductStep steps[kSteps] = {};
-    bool held = kHolds && !sums_by_column && a_hi - a_lo <= THREADS;
+    bool held = kHolds && a_hi - a_lo <= THREADS;
     if constexpr (kHolds) {
       if (held) {  // uniform
         int start = 0, len = 0;
@@ -1442,6 +1444,7 @@ __device__ __forceinline__ void spgemm_lds_bitmap_rows(
       if (sums_by_column) {
         for_each_product<THREADS, true, T, A>(
             a_lo, a_hi, tid, a_crd, a_val, b_pos, b_crd, b_val, s_batch, s_scan, [&](int k, A product) {
+              if ((unsigned)k >= (unsigned)columns) return;
               atomicOr(&s_bits[k >> 5], 1u << (k & 31));
               lds_accumulate<A>(&s_acc[k], product);
             });
@@ -1562,8 +1565,8 @@ __global__ __launch_bounds__(THREADS) void spgemm_lds_bitmap_kernel(
 // With sums of 4 bytes 512 for the rows of up to kTinyProducts, and 256 where more than half of the rows have more products (a
 // workgroup's barriers are what these wait for).  The product, us, all with 256 and so, M x N with rows of (products): fp32 30,000 x 30,000
 // (100) 99, 91; fp64 (100) 135, 104; (400) 474, 439; (2,000) 681, 609; all with 512 and so: fp32 30,000 x 30,000 (400) 376, 296;
-// (1,000) 465, 388; (2,000) 515, 455; 8,000 x 3,000 (400) 120, 100.  Graphs of 1,500 nodes of 16 and 25,000 of 10, fp32: 96 and 135 with 256, 92 and 128 so.
-template <typename T, bool NUMERIC, int THREADS>
+// (1,000) 465, 388; (2,000) 515, 455; 8,000 x 3,000 (400) 120, 88.  Graphs of 1,500 nodes of 16 and 25,000 of 10, fp32: 96 and 135 with 256, 92 and 128 so.
+template <typename T, bool NUMERIC, int THREADS, int WORDS>
 __global__ __launch_bounds__(THREADS) void spgemm_small_matrix_kernel(
     int M, int N, int n_bitmap, int n_medium, const int *__restrict__ a_pos, const int *__restrict__ a_crd,
     const T *__restrict__ a_val, const int *__restrict__ b_pos, const int *__restrict__ b_crd,
@@ -1573,14 +1576,14 @@ __global__ __launch_bounds__(THREADS) void spgemm_small_matrix_kernel(
   using A = typename Acc<T>::type;
   constexpr int kWaves = THREADS / kWaveSize;
   union Tables {
-    BitmapTables<A, NUMERIC, kNarrowColumns / 32, THREADS, kBitmapSums> bitmap;
+    BitmapTables<A, NUMERIC, WORDS, THREADS, kBitmapSums> bitmap;
     MediumTables<A, NUMERIC, kSmallProducts, THREADS> medium;
     TeamTables<A, NUMERIC, kWaveSize, kWaves, kTinySlots, kTinyProducts> tiny;
   };
   __shared__ Tables lds;
   int block = blockIdx.x;
   if (block < n_bitmap) {
-    spgemm_lds_bitmap_rows<T, NUMERIC, kNarrowColumns / 32, THREADS, kBitmapSums, 0, 4>(
+    spgemm_lds_bitmap_rows<T, NUMERIC, WORDS, THREADS, kBitmapSums, 0, 4>(
         lds.bitmap, block, n_bitmap, M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, medium_rows, narrow_rows, counters,
         c_pos, c_crd, c_val);
     return;
@@ -2333,6 +2336,8 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
     // rows the smaller bitmap kernel goes through; with the result's row pointer known, also those of the tier above
     // that turn out to have few distinct columns
     const int *narrow_rows = NUMERIC && narrow && !bins ? ws.huge_rows : nullptr;
+    const bool by_column = NUMERIC && N <= kBitmapSums;  // sums of rows of up to kMediumProducts products (spgemm_lds_bitmap_rows)
+    constexpr int kByColumnWords = NUMERIC ? kBitmapSums / 32 : kNarrowColumns / 32;
     const auto blocks_for = [&](int64_t rows) {
       return (unsigned)std::min<int64_t>(rows, known ? kKnownWorkgroups : kMediumWorkgroups);
     };
@@ -2342,10 +2347,12 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
       // (see spgemm_small_matrix_kernel)
       constexpr int kMore = NUMERIC ? kBitmapThreads : kBlockThreads;
       const bool few = known && 2 * (known->small + known->medium) < M;
-      const bool more = sizeof(A) > 4 || few;
+      const bool more = !by_column && (sizeof(A) > 4 || few);
       const int threads = more ? kMore : kBlockThreads;
       const unsigned tiny_blocks = (unsigned)((M + threads / kWaveSize - 1) / (threads / kWaveSize));
-      auto kernel = more ? &spgemm_small_matrix_kernel<T, NUMERIC, kMore> : &spgemm_small_matrix_kernel<T, NUMERIC, kBlockThreads>;
+      auto kernel = by_column ? &spgemm_small_matrix_kernel<T, NUMERIC, kBlockThreads, kByColumnWords>
+                    : more    ? &spgemm_small_matrix_kernel<T, NUMERIC, kMore, kNarrowColumns / 32>
+                              : &spgemm_small_matrix_kernel<T, NUMERIC, kBlockThreads, kNarrowColumns / 32>;
       kernel<<<bitmap_blocks + small_blocks + tiny_blocks, threads, 0, stream>>>(
           M, N, (int)bitmap_blocks, (int)small_blocks, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.small_rows,
           ws.medium_rows, narrow_rows, ws.counters, c_pos, c_crd, c_val);
@@ -2364,10 +2371,12 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
       }
       if (bitmap_blocks && narrow) {
         // narrow enough for a bitmap in LDS beside other workgroups: no hashing, nothing to sort
-        constexpr int kThreads = NUMERIC ? kBitmapThreads : kBlockThreads;
-        spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kThreads, kBitmapSums, 0, 4>
-            <<<bitmap_blocks, kThreads, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.medium_rows,
-                                                          narrow_rows, ws.counters, c_pos, c_crd, c_val);
+        constexpr int kMore = NUMERIC ? kBitmapThreads : kBlockThreads;
+        auto kernel = by_column ? &spgemm_lds_bitmap_kernel<T, NUMERIC, kByColumnWords, kBlockThreads, kBitmapSums, 0, 4>
+                                : &spgemm_lds_bitmap_kernel<T, NUMERIC, kNarrowColumns / 32, kMore, kBitmapSums, 0, 4>;
+        kernel<<<bitmap_blocks, by_column ? kBlockThreads : kMore, 0, stream>>>(M, N, a_pos, a_crd, a_val, b_pos, b_crd, b_val,
+                                                                                ws.medium_rows, narrow_rows, ws.counters, c_pos,
+                                                                                c_crd, c_val);
       } else if (bitmap_blocks) {
         // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
         // beside them (with 8-byte sums, no more than 256)

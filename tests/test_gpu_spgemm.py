@@ -582,13 +582,14 @@ def test_rows_at_the_edges_of_the_tiers_of_a_large_matrix(oracle, dtype, N):
 
 @pytest.mark.parametrize("suffix, dtype", [("f32", np.float32), ("i64", np.int64)])
 @pytest.mark.parametrize("M", [60, 32_768 + 7])
-def test_columns_outside_of_b_are_left_out_of_rows_summed_by_a_bitmap(suffix, dtype, M):
+@pytest.mark.parametrize("N", [70_001, 3001])
+def test_columns_outside_of_b_are_left_out_of_rows_summed_by_a_bitmap(suffix, dtype, M, N):
     """The bare C calls look at no indices beforehand.  Rows of 1,025 to 4,096 products, of few entries and of more than
-    threads: both passes leave a column outside [0, N) out.  Whole numbers: every sum is exact."""
+    threads, summed by rank and by column: both passes leave a column outside [0, N) out.  Whole numbers: every sum is exact."""
     from scorch_amd import native
-    N, rng = 70_001, np.random.default_rng(M)
+    rng = np.random.default_rng(M)
     lens = [1025, 2048, 4096, 300, 5]
-    bci = [rng.choice(N, n, replace=False) for n in lens]
+    bci = [rng.choice(N, n, replace=n > N) for n in lens]
     outside = np.array([N, N + 31, 131_071, 131_072, 2**31 - 1, -1, -(2**31)])
     for at in bci:
         k = min(at.size - 1, outside.size)
@@ -614,7 +615,7 @@ def test_columns_outside_of_b_are_left_out_of_rows_summed_by_a_bitmap(suffix, dt
         for p in range(arp[r], arp[r + 1]):
             q = np.arange(brp[aci[p]], brp[aci[p] + 1])
             q = q[(bci[q] >= 0) & (bci[q] < N)]
-            want[i, bci[q]] += int(av[p]) * bv[q].astype(np.int64)
+            np.add.at(want[i], bci[q], int(av[p]) * bv[q].astype(np.int64))
             stored[i, bci[q]] = True
     counts = np.zeros(M + 1, np.int64)
     counts[np.array(sorted(rows)) + 1] = stored.sum(axis=1)
