@@ -334,3 +334,26 @@ def test_combining_the_stretches_of_a_long_row(oracle, stretches, D):
     out = H.attn_blocksparse_f32(*(dev(x) for x in (q, k, v)), bm, D ** -0.5).cpu().numpy()
     for h in range(heads):
         assert oracle.rel_fro(out[h], oracle.attention_dense_fp64(q[h], k[h], v[h], mask, D ** -0.5)) <= TOL
+
+
+# rows of two stretches beside one of so many, four or fewer on average: the combining kernel asks for four at once
+@pytest.mark.parametrize("stretches", [3, 4, 5, 9, 12])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_combining_a_long_rows_stretches_beside_many_rows_of_two(oracle, stretches, D):
+    S, heads, token = 128 * stretches, 2, 70
+    i, j = np.arange(S)[:, None], np.arange(S)[None, :]
+    mask = (abs(i - j) <= 80) | (i == token)
+    rng = np.random.default_rng(stretches + D)
+    q, k, v = (rng.standard_normal((heads, S, D)).astype(np.float32) for _ in range(3))
+    k *= np.linspace(0.1, 4.0, S, dtype=np.float32)[:, None]  # the stretches' maxima differ
+    rp, ci = (dev(x) for x in csr_of(mask))
+    bm = H.attention_block_mask(rp, ci, S)
+    plain = H.BlockMask(bm.S, bm.block, bm.block_row_ptr, bm.block_col_idx, None, None, bm.nnz)
+    plain.block_row_lens = bm.row_lens()
+    H.split_long_block_rows(plain, 2, list_unequal_rows=True)
+    rows = plain.split_rows.view(-1, 4)
+    assert int(rows[:, 2].max()) == stretches and plain.n_slots <= 4 * len(rows)
+    bm.pairing["fp32", heads, D] = (plain.items, plain.split_rows, plain.n_slots)
+    out = H.attn_blocksparse_f32(*(dev(x) for x in (q, k, v)), bm, D ** -0.5).cpu().numpy()
+    for h in range(heads):
+        assert oracle.rel_fro(out[h], oracle.attention_dense_fp64(q[h], k[h], v[h], mask, D ** -0.5)) <= TOL
