@@ -409,16 +409,21 @@ struct TeamTables {
   static constexpr int kQueries = 16, kTeams = kWavesPerBlock / SPLIT;  // queries to a team of SPLIT wavefronts; teams
   static constexpr int kBlocksAtOnce = 16;                              // 64 tiles: one to a lane
   static constexpr int kOthers = SPLIT > 1 ? SPLIT - 1 : 1;
-  unsigned long long words[kTeams][kBlocksAtOnce][kQueries];
-  int col[kBlocksAtOnce];
-  alignas(16) float sums[SPLIT > 1 ? kTeams : 1][kOthers][SPLIT > 1 ? kQueries : 1][D + 4];
-  unsigned flags[SPLIT > 1 ? kTeams : 1][kOthers][3][kWaveSize];
+  using Words = unsigned long long[kTeams][kBlocksAtOnce][kQueries];
+  using Col = int[kBlocksAtOnce];
+  using Sums = float[SPLIT > 1 ? kTeams : 1][kOthers][SPLIT > 1 ? kQueries : 1][D + 4];
+  using Flags = unsigned[SPLIT > 1 ? kTeams : 1][kOthers][3][kWaveSize];
+  Words words;
+  Col col;
+  alignas(16) Sums sums;
+  Flags flags;
 };
 
 // Of a head's work item number `item`, the queries of the `quarter`-th of SPLIT workgroups.
 template <int D, int SPLIT>
 __device__ __forceinline__ void team_rows(
-    TeamTables<D, SPLIT> &lds, int head, int item_at, int quarter, int S, int n_blocks, const int *__restrict__ block_row_ptr,
+    typename TeamTables<D, SPLIT>::Words &s_words, typename TeamTables<D, SPLIT>::Col &s_col,
+    typename TeamTables<D, SPLIT>::Sums &s_sums, typename TeamTables<D, SPLIT>::Flags &s_flags, int head, int item_at, int quarter, int S, int n_blocks, const int *__restrict__ block_row_ptr,
     const int *__restrict__ block_col_idx, const int *__restrict__ block_mask_index,
     const unsigned long long *__restrict__ block_masks,
     const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float scale_log2e,
@@ -427,10 +432,6 @@ __device__ __forceinline__ void team_rows(
   constexpr int kQueries = Tables::kQueries, kTeams = Tables::kTeams, kBlocksAtOnce = Tables::kBlocksAtOnce, kOthers = Tables::kOthers;
   constexpr int kSlabs = D / 16, kFeat = D / 16;
   constexpr int VW = D == 32 ? 2 : 4, NH = kFeat / VW;
-  auto &s_words = lds.words;
-  auto &s_col = lds.col;
-  auto &s_sums = lds.sums;
-  auto &s_flags = lds.flags;
 
   const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), w = uniform(tid / kWaveSize);
   const int team = w / SPLIT, part = w % SPLIT;
@@ -720,10 +721,6 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kerne
     const unsigned long long *__restrict__ block_masks,
     const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V, float scale_log2e,
     float *__restrict__ O, int n_items, int n_wide, const int4 *__restrict__ items, int n_slots, float *__restrict__ partials) {
-  __shared__ union {
-    TeamTables<D, SPLIT> usual;
-    TeamTables<D, WIDE ? 4 : SPLIT> wide;
-  } lds;
   // First, of every head, a quarter of the wide items and all of the others, and at the end of the launch the wide ones' other quarters,
   // of which most have nothing to do.  (The four of an item one after the other: an XCD's workgroups go to its four shader
   // engines in turn, and one engine got all the long ones; a head's at the end of the head: workgroups with nothing to do
@@ -744,15 +741,30 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kerne
     head = id / ranks;
     rank = id % ranks;
   }
-  if (WIDE && (quarter > 0 || rank < n_wide)) {
-    quarter += rank / n_wide;
-    team_rows<D, WIDE ? 4 : SPLIT>(lds.wide, head, rank % n_wide, quarter, S, n_blocks, block_row_ptr, block_col_idx, block_mask_index,
-                                   block_masks, Q, K, V, scale_log2e, O, items, n_slots, partials);
-    return;
+  if constexpr (WIDE) {
+    __shared__ union {
+      TeamTables<D, SPLIT> usual;
+      TeamTables<D, 4> wide;
+    } lds;
+    if (quarter > 0 || rank < n_wide) {
+      quarter += rank / n_wide;
+      team_rows<D, 4>(lds.wide.words, lds.wide.col, lds.wide.sums, lds.wide.flags, head, rank % n_wide, quarter, S, n_blocks, block_row_ptr,
+                      block_col_idx, block_mask_index, block_masks, Q, K, V, scale_log2e, O, items, n_slots, partials);
+      return;
+    }
+    rank -= n_wide;
+    team_rows<D, SPLIT>(lds.usual.words, lds.usual.col, lds.usual.sums, lds.usual.flags, head, n_wide + rank / SPLIT, rank % SPLIT, S,
+                        n_blocks, block_row_ptr, block_col_idx, block_mask_index, block_masks, Q, K, V, scale_log2e, O, items, n_slots,
+                        partials);
+  } else {
+    using Tables = TeamTables<D, SPLIT>;
+    __shared__ typename Tables::Words words;
+    __shared__ typename Tables::Col col;
+    __shared__ alignas(16) typename Tables::Sums sums;
+    __shared__ typename Tables::Flags flags;
+    team_rows<D, SPLIT>(words, col, sums, flags, head, rank / SPLIT, rank % SPLIT, S, n_blocks, block_row_ptr, block_col_idx,
+                        block_mask_index, block_masks, Q, K, V, scale_log2e, O, items, n_slots, partials);
   }
-  if (WIDE) rank -= n_wide;
-  team_rows<D, SPLIT>(lds.usual, head, (WIDE ? n_wide : 0) + rank / SPLIT, rank % SPLIT, S, n_blocks, block_row_ptr, block_col_idx,
-                      block_mask_index, block_masks, Q, K, V, scale_log2e, O, items, n_slots, partials);
 }
 
 // Combines the stretches of a block row that was shared out: with m* the largest of the
