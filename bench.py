@@ -66,8 +66,8 @@ MEASURED_TRAFFIC = {
                                   "sha16": "6bec361246ba8e16", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
     ("sddmm_uniform", "plain"): {"bytes": 880_200_000, "sources": (_CSRC + "sddmm.hip", _CSRC + "common.hpp"),
                                  "sha16": "6bec361246ba8e16", "profile": "profiles/sddmm_kernels_uniform_65536.md"},
-    ("attention_blocksparse", "fused"): {"bytes": 81_010_000, "sources": (_CSRC + "attn.hip", _CSRC + "common.hpp"),
-                                         "sha16": "fcae0aa15a99558d", "profile": "profiles/attn_blocksparse_kernel_s8192_h16.md"},
+    ("attention_blocksparse", "fused"): {"bytes": 80_990_000, "sources": (_CSRC + "attn.hip", _CSRC + "attn_parts.hpp", _CSRC + "common.hpp"),
+                                         "sha16": "1caf9703227a300a", "profile": "profiles/attn_blocksparse_kernel_s8192_h16.md"},
 }
 
 

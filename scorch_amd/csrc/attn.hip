@@ -27,6 +27,7 @@
 // the softmax state of its query; the 16 probabilities it holds after the
 // first product (4 tiles x 4 keys) are exactly the B operand of the second
 // one, provided the V^T operand is gathered with the same key order.
+#include "attn_parts.hpp"
 #include "common.hpp"
 
 namespace scorch {
@@ -417,7 +418,6 @@ __attribute__((amdgpu_waves_per_eu(AttnTile<D>::kWavesPerSimd))) void attn_block
 // A thread takes four features of a query: a row has few stretches (a dozen) and a launch few such rows (a
 // global token's), so it is the number of loads in flight that counts (S = 8,192, 16 heads, one shared-out
 // row of 13 stretches: 10.3 us with a quarter of the features per thread and one workgroup per row and head).
-constexpr int kMergeAtOnce = 8;
 template <int D>
 __global__ __launch_bounds__(kBlockThreads) void attn_merge_kernel(int S, int n_slots,
                                                                    const int4 *__restrict__ split_rows,
@@ -428,45 +428,9 @@ __global__ __launch_bounds__(kBlockThreads) void attn_merge_kernel(int S, int n_
   const int head = blockIdx.y;
   const int q = blockIdx.z * kQueries + threadIdx.x / kLanes, feature = threadIdx.x % kLanes * 4;
   const float *base = partials + (((size_t)head * n_slots + row.y) * kAttnBlock + q) * (D + 4);
-  const size_t part_stride = (size_t)kAttnBlock * (D + 4);
-  // The first stretches' sums are requested with their maxima, one round trip instead of two: windows of 64 and a global token, (tokens,
-  // heads, D) (1,024, 4, 64) 9.3 -> 8.5 us, (4,480, 12, 64) 19.8 -> 18.9, (2,048, 12, 128) 21.2 -> 20.4, (8,192, 16, 64) 31.4 -> 31.1.
-  constexpr float kNothing = -3.0e38f;
-  floatx4 first_o[kMergeAtOnce];
-  float first_m[kMergeAtOnce], first_l[kMergeAtOnce];
-  if (row.z > 0) {
-#pragma unroll
-    for (int p = 0; p < kMergeAtOnce; ++p) {  // (past the last: the last again)
-      const float *part = base + min(p, row.z - 1) * part_stride;
-      first_o[p] = *reinterpret_cast<const floatx4 *>(part + feature);
-      first_m[p] = part[D];
-      first_l[p] = part[D + 1];
-    }
-  } else {
-#pragma unroll
-    for (int p = 0; p < kMergeAtOnce; ++p) first_m[p] = kNothing;
-  }
-  float m_star = kNothing;
-#pragma unroll
-  for (int p = 0; p < kMergeAtOnce; ++p) m_star = fmaxf(m_star, first_m[p]);
-#pragma unroll 8
-  for (int p = kMergeAtOnce; p < row.z; ++p) m_star = fmaxf(m_star, base[p * part_stride + D]);
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  float l = 0.0f;
-  const auto add = [&](float m, float sum, const floatx4 &o) __attribute__((always_inline)) {
-    const float weight = __builtin_amdgcn_exp2f(m - m_star);
-    l += weight * sum;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[r] += weight * o[r];
-  };
-#pragma unroll
-  for (int p = 0; p < kMergeAtOnce; ++p)
-    if (p < row.z) add(first_m[p], first_l[p], first_o[p]);
-#pragma unroll 4
-  for (int p = kMergeAtOnce; p < row.z; ++p) {
-    const float *part = base + p * part_stride;
-    add(part[D], part[D + 1], *reinterpret_cast<const floatx4 *>(part + feature));
-  }
+  floatx4 acc;
+  float l;
+  combine_parts<D, kAttnBlock *(D + 4)>(base, row.z, feature, acc, l);
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
   bf16x4 o;
 #pragma unroll

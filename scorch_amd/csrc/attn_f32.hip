@@ -37,6 +37,7 @@
 // block has something non-finite in V, those elements become zeros in LDS and leave a flag (NaN,
 // infinity, -infinity) at the result elements they belong to, which are given it at the end.  (The
 // look costs 1 % -- S = 3,001, 8 heads, D = 64, window of 64 and a global token: 27.0 -> 27.3 us.)
+#include "attn_parts.hpp"
 #include "common.hpp"
 
 namespace scorch {
@@ -770,7 +771,7 @@ __attribute__((amdgpu_waves_per_eu(D == 128 ? 2 : 4))) void attn_f32_tiles_kerne
 // Combines the stretches of a block row that was shared out: with m* the largest of the
 // stretches' reference maxima, O = sum_p 2^(m_p - m*) O_p / sum_p 2^(m_p - m*) l_p.
 // One workgroup per (split row, head); thread t takes query t / 4 and a quarter of the features.
-template <int D, int AT_ONCE>
+template <int D>
 __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, int n_slots,
                                                                        const int4 *__restrict__ split_rows,
                                                                        const float *__restrict__ partials,
@@ -780,46 +781,9 @@ __global__ __launch_bounds__(kBlockThreads) void attn_f32_merge_kernel(int S, in
   constexpr int kLanes = D / 4, kQueries = kBlockThreads / kLanes;  // threads per query, queries per workgroup
   const int q = blockIdx.z * kQueries + threadIdx.x / kLanes, feature = threadIdx.x % kLanes * 4;
   const float *base = partials + (((size_t)head * n_slots + row.y) * kBlock + q) * (D + 4);
-  const size_t part_stride = (size_t)kBlock * (D + 4);
-  // The first AT_ONCE stretches' sums are requested with their maxima, one round trip instead of two: windows of 64 and a global token, (tokens,
-  // heads, D) (2,048, 12, 128) 39.2 -> 38.3 us, (4,096, 4, 32) 17.2 -> 16.7, (3,001, 8, 64) 22.5 -> 22.3.  Eight of them, four where
-  // rows have four or fewer on average: reading the last again costs more there than is waited for (rows of two, the two launches, us, none at
-  // once, eight, four: (2,048, 16, 64), window of 256 73.7, 74.8, 73.2; (3,008, 8, 64), 128 43.8, 45.1, 43.7; (8,192, 4, 128), 256 152.3, 154.9, 153.5).
-  floatx4 first_o[AT_ONCE];
-  float first_m[AT_ONCE], first_l[AT_ONCE];
-  if (row.z > 0) {
-#pragma unroll
-    for (int p = 0; p < AT_ONCE; ++p) {  // (past the last: the last again; a branch to each puts the waits between them, +0.7 us)
-      const float *part = base + min(p, row.z - 1) * part_stride;
-      first_o[p] = *reinterpret_cast<const floatx4 *>(part + feature);
-      first_m[p] = part[D];
-      first_l[p] = part[D + 1];
-    }
-  } else {
-#pragma unroll
-    for (int p = 0; p < AT_ONCE; ++p) first_m[p] = kDead;
-  }
-  float m_star = kDead;
-#pragma unroll
-  for (int p = 0; p < AT_ONCE; ++p) m_star = fmaxf(m_star, first_m[p]);
-#pragma unroll 8
-  for (int p = AT_ONCE; p < row.z; ++p) m_star = fmaxf(m_star, base[p * part_stride + D]);
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  float l = 0.0f;
-  const auto add = [&](float m, float sum, const floatx4 &o) __attribute__((always_inline)) {
-    const float weight = __builtin_amdgcn_exp2f(m - m_star);
-    l += weight * sum;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[r] += weight * o[r];
-  };
-#pragma unroll
-  for (int p = 0; p < AT_ONCE; ++p)
-    if (p < row.z) add(first_m[p], first_l[p], first_o[p]);
-#pragma unroll 4
-  for (int p = AT_ONCE; p < row.z; ++p) {
-    const float *part = base + p * part_stride;
-    add(part[D], part[D + 1], *reinterpret_cast<const floatx4 *>(part + feature));
-  }
+  floatx4 acc;
+  float l;
+  combine_parts<D, kBlock *(D + 4)>(base, row.z, feature, acc, l);
   if (row.x * kBlock + q >= S) return;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
@@ -870,8 +834,7 @@ static int launch(dim3 grid, hipStream_t s, int S, int n_blocks, int H, const in
   mark_launch(s);
   if (n_split_rows > 0) {
     const dim3 merge_grid((unsigned)n_split_rows, (unsigned)H, (unsigned)(kBlock * D / 4 / kBlockThreads));
-    auto kernel = n_slots <= 4 * (int64_t)n_split_rows ? &attn_f32_merge_kernel<D, 4> : &attn_f32_merge_kernel<D, 8>;
-    kernel<<<merge_grid, kBlockThreads, 0, s>>>(S, n_slots, split_rows, partials, o);
+    attn_f32_merge_kernel<D><<<merge_grid, kBlockThreads, 0, s>>>(S, n_slots, split_rows, partials, o);
     SCORCH_HIP_CHECK(hipGetLastError());
     mark_launch(s);
   }

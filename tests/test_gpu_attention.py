@@ -417,8 +417,8 @@ def test_rows_shared_out_by_the_size_of_the_launch(oracle, D, S, heads, window, 
         assert oracle.rel_fro(out[h].float().cpu().numpy(), ref) <= 5e-3
 
 
-# a block row in so many stretches: the combining kernel asks for eight of them at once
-@pytest.mark.parametrize("stretches", [2, 7, 8, 9, 17])
+# a block row in so many stretches: the combining kernel asks for four or eight of them at once, and for the others in batches
+@pytest.mark.parametrize("stretches", [2, 4, 5, 7, 8, 9, 16, 17, 25])
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_combining_the_stretches_of_a_long_row(oracle, stretches, D):
     S, heads, token = 128 * stretches - 64, 2, 70

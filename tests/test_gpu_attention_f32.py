@@ -314,8 +314,8 @@ def test_non_finite_values_in_stretches_of_four_workgroups_each(heads, token, D)
         assert (np.abs(out[h][finite] - want[finite]) <= 1e-5 * np.maximum(size, np.where(size > 1e6, 3e38, 4.0))).all()
 
 
-# a block row in so many stretches: the combining kernel asks for eight of them at once
-@pytest.mark.parametrize("stretches", [2, 7, 8, 9, 17])
+# a block row in so many stretches: the combining kernel asks for four or eight of them at once, and for the others in batches
+@pytest.mark.parametrize("stretches", [2, 4, 5, 7, 8, 9, 16, 17, 25])
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_combining_the_stretches_of_a_long_row(oracle, stretches, D):
     S, heads, token = 128 * stretches - 64, 2, 70
@@ -336,7 +336,7 @@ def test_combining_the_stretches_of_a_long_row(oracle, stretches, D):
         assert oracle.rel_fro(out[h], oracle.attention_dense_fp64(q[h], k[h], v[h], mask, D ** -0.5)) <= TOL
 
 
-# rows of two stretches beside one of so many, four or fewer on average: the combining kernel asks for four at once
+# rows of two stretches beside one of so many
 @pytest.mark.parametrize("stretches", [3, 4, 5, 9, 12])
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_combining_a_long_rows_stretches_beside_many_rows_of_two(oracle, stretches, D):
