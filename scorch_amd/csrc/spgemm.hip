@@ -2378,9 +2378,11 @@ int spgemm_run(int M, int N, const int *a_pos, const int *a_crd, const T *a_val,
                                                                                 ws.medium_rows, narrow_rows, ws.counters, c_pos,
                                                                                 c_crd, c_val);
       } else if (bitmap_blocks) {
-        // tables for 4096 products leave room for one workgroup per CU: as many threads as still fit
-        // beside them (with 8-byte sums, no more than 256)
-        constexpr int kThreads = sizeof(A) > 4 ? kBlockThreads : kHugeThreads;
+        // Two workgroups of 512 threads to a CU with sums of 4 bytes, one of 8 wavefronts with 8.  Sorted in the table's place by 1,024
+        // threads, with sums of 8 bytes by 256 (as many as had fitted beside separate tables), rows of 1,200 to 2,000 products had lost
+        // against those.  20,000 x 200,000, us, separate tables, those threads, now: fp32 (1,200 products) 995, 1,006, 491; (1,600) 1,074,
+        // 1,091, 552; (3,600) 1,536, 1,540, 945; fp64 (1,200) 1,204, 1,222, 789; (1,600) 1,404, 1,432, 901; (3,600) 2,547, 2,502, 1,531.
+        constexpr int kThreads = kBitmapThreads;
         spgemm_medium_kernel<T, NUMERIC, kMediumProducts, 0, kThreads><<<bitmap_blocks, kThreads, 0, stream>>>(
             a_pos, a_crd, a_val, b_pos, b_crd, b_val, ws.products, ws.medium_rows, ws.counters, c_pos, c_crd, c_val);
       }

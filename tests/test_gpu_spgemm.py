@@ -646,3 +646,21 @@ def test_many_and_few_rows_beyond_a_wavefronts_and_sums_by_column(oracle, dtype,
     arp = np.arange(0, 2 * M + 1, 2, dtype=np.int32)
     value = (lambda n: rng.integers(-9, 10, n).astype(dtype)) if dtype == np.int64 else (lambda n: (rng.random(n) + 0.5).astype(dtype))
     check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+@pytest.mark.parametrize("N", [131_073, 2_000_000])
+def test_rows_of_a_wide_b_that_are_sorted_in_the_place_of_their_table(oracle, dtype, N):
+    """A B beyond the bitmaps: rows at the edges of the table's sizes, spread out (sorted by buckets) and crowded around one column with
+    another far away (sorted as a whole)."""
+    rng = np.random.default_rng(N)
+    lens = [257, 1024, 1025, 2047, 2048, 2049, 3000, 4095, 4096]
+    rows = [np.sort(rng.choice(N, n, replace=False)) for n in lens]
+    rows += [np.concatenate([np.arange(n - 1) + 60_000, [N - 1]]) for n in lens]
+    brp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    bci = np.concatenate(rows).astype(np.int32)
+    K = len(rows)
+    aci = np.concatenate([np.arange(K), np.full(5, 2), [0, 9]]).astype(np.int32)
+    arp = np.concatenate([np.arange(K + 1), [K + 3, K + 5, K + 7]]).astype(np.int32)     # (and rows of two and of three entries)
+    value = (lambda n: rng.integers(-9, 10, n).astype(dtype)) if dtype == np.int64 else (lambda n: (rng.random(n) + 0.5).astype(dtype))
+    check(oracle, arp, aci, value(aci.size), brp, bci, value(bci.size), N)
