@@ -54,11 +54,11 @@ _SPMM_SOURCES = (_CSRC + "spmm.hip", _CSRC + "spmm.hpp", _CSRC + "common.hpp")
 MEASURED_TRAFFIC = {
     ("gcn_powerlaw", "merge"): {"bytes": 9_790_000_000, "sources": _SPMM_SOURCES, "sha16": "29d6cd6f4ca103a4",
                                 "profile": "profiles/spmm_merge_kernel_gcn_powerlaw.md"},
-    ("spmm_uniform", "rows"): {"bytes": 10_834_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp",
-                                                                _CSRC + "common.hpp"), "sha16": "a8c3814230e5c123",
+    ("spmm_uniform", "rows"): {"bytes": 10_834_000, "sources": (_CSRC + "spmm_rows.hip", _CSRC + "spmm.hpp", _CSRC + "sync.hpp",
+                                                                _CSRC + "common.hpp"), "sha16": "373d7749cd57a444",
                                "profile": "profiles/spmm_rows_kernel_uniform_4096.md"},
-    ("sae_decoder", "tiled"): {"bytes": 344_200_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp",
-                                                                 _CSRC + "common.hpp"), "sha16": "6fc9000e2bf14019",
+    ("sae_decoder", "tiled"): {"bytes": 344_200_000, "sources": (_CSRC + "spmm_tiled.hip", _CSRC + "spmm.hpp", _CSRC + "sync.hpp",
+                                                                 _CSRC + "common.hpp"), "sha16": "62afa656a2ca0a2b",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},
     ("sae_decoder", "merge"): {"bytes": 1_766_000_000, "sources": _SPMM_SOURCES, "sha16": "29d6cd6f4ca103a4",
                                "profile": "profiles/spmm_tiled_kernel_sae_decoder.md"},

@@ -1,5 +1,6 @@
 """bench.py's table of measured memory traffic must not outlive the kernels it was measured on."""
 import os
+import re
 
 import bench
 
@@ -14,6 +15,16 @@ def test_measured_traffic_is_stamped_with_the_sources_it_was_measured_on():
             assert os.path.exists(os.path.join(bench.ROOT, f)), (key, f)
         assert rec["sha16"] in ("", bench.source_hash(rec["sources"])), \
             f"{key}: the kernel's sources changed after its traffic was measured"
+
+
+def test_a_record_names_every_header_its_kernels_are_built_from():
+    """Device code of a kernel stands in headers too: a change there makes its record stale as well."""
+    for key, rec in bench.MEASURED_TRAFFIC.items():
+        for f in rec["sources"]:
+            with open(os.path.join(bench.ROOT, f)) as fh:
+                included = re.findall(r'^#include "([^"/]+)"', fh.read(), re.M)
+            missing = [h for h in included if os.path.join(os.path.dirname(f), h) not in rec["sources"]]
+            assert not missing, (key, f, missing)
 
 
 def test_a_stale_record_reports_no_traffic(monkeypatch):
