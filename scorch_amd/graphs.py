@@ -23,18 +23,48 @@ A replay writes the results, and whatever the caller copied into the static
 inputs arrived there, without PyTorch's version counters necessarily noticing.
 ``capture`` therefore marks the static inputs and the results volatile
 (scorch_ops_hip.mark_volatile: eager calls that take them as operands keep
-nothing derived from their values), and every replay bumps the results' version
-counters, so that data other code derived from them is seen to be stale.
+nothing derived from their values), and every replay bumps the version counters
+of the results and of the tensors that the step writes in place by operations of
+PyTorch (an operand it closes over and updates), so that data other code derived
+from them is seen to be stale.
 
 The reference has no counterpart: its kernels run on the host.
 """
 from __future__ import annotations
 
-from typing import Any, Callable
+import weakref
+from typing import Any, Callable, Dict, List
 
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from . import scorch_ops_hip
+
+
+class _Writes(TorchDispatchMode):
+    """Notes the tensors that operations run under it write in place (of a view, the tensor it is a view of)."""
+
+    def __init__(self) -> None:
+        super().__init__()
+        self._seen: Dict[int, "weakref.ref[torch.Tensor]"] = {}
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        kwargs = kwargs or {}
+        result = func(*args, **kwargs)
+        schema = getattr(func, "_schema", None)
+        for i, spec in enumerate(schema.arguments if schema is not None else ()):
+            if spec.alias_info is None or not spec.alias_info.is_write:
+                continue
+            value = args[i] if i < len(args) else kwargs.get(spec.name)
+            for t in value if isinstance(value, (list, tuple)) else (value,):
+                if isinstance(t, torch.Tensor):
+                    t = t._base if t._is_view() else t
+                    self._seen[id(t)] = weakref.ref(t)
+        return result
+
+    def surviving(self) -> List[torch.Tensor]:
+        """Those that are still there: the step's own temporaries are not."""
+        return [t for t in (ref() for ref in self._seen.values()) if t is not None and not t.is_inference()]
 
 
 class CapturedStep:
@@ -52,7 +82,9 @@ class CapturedStep:
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
-            for _ in range(max(int(warmup), 2)):     # twice at least: some plans are built on the second use
+            for _ in range(max(int(warmup), 2) - 1):  # twice at least: some plans are built on the second use
+                fn(*args)
+            with _Writes() as writes:
                 fn(*args)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
@@ -66,12 +98,13 @@ class CapturedStep:
             scorch_ops_hip._recordings[:] = [r for r in scorch_ops_hip._recordings if r is not self._kept]
         self._result_tensors = list(scorch_ops_hip._tensors_of(self.result))
         scorch_ops_hip.mark_volatile(self._result_tensors)
+        self._written = self._result_tensors + writes.surviving()
 
     def replay(self) -> Any:
         self.graph.replay()
-        if self._result_tensors:
+        if self._written:
             # the replay has rewritten them in place behind the version counters' back
-            torch.autograd.graph.increment_version(self._result_tensors)
+            torch.autograd.graph.increment_version(self._written)
         return self.result
 
     __call__ = replay

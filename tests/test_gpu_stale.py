@@ -273,3 +273,44 @@ def test_products_with_vectors_read_the_values_that_are_in_memory(dtype):
     for scale in (0.5, 0.25, 0.125):
         step()
         products(scale)
+
+
+@pytest.mark.parametrize("write", ["whole", "view", "out", "foreach"])
+def test_an_operand_that_a_recorded_step_closes_over_and_writes(oracle, write):
+    """B is neither an input of the step nor its result: a replay rewrites it all the same, and eager products whose column-tile copy
+    of it was made before must see what is in memory then."""
+    rng = np.random.default_rng(61)
+    M, K, N = 384, 1024, 512
+    rp, ci, v = _wide_case(rng, M, K, N)
+    A = scorch.STensor.from_csr_arrays(dev(rp), dev(ci), dev(v), (M, K))
+    B, X = torch.randn(K, N, device="cuda"), torch.randn(K, N, device="cuda")
+
+    def update(x):
+        if write == "whole":
+            B.mul_(0.5).add_(x)
+        elif write == "view":
+            B[:K // 2, 3:].copy_(x[:K // 2, 3:])
+        elif write == "out":
+            torch.add(B, x, out=B)
+        else:
+            torch._foreach_add_([B], 0.25)
+        return scorch.matmul(A, B, format="dd")
+
+    step = graphs.capture(update, X)
+    torch.cuda.synchronize()
+    assert not H.is_volatile(B)
+
+    def products():
+        for _ in range(3):                                   # the second product is the one that may build a copy
+            want = oracle.spmm_fp64(rp, ci, v, host(B).astype(np.float64))
+            assert oracle.rel_fro(host(scorch.matmul(A, B, format="dd")), want) <= TOL
+        assert hasattr(B, "_scorch_tiled")
+
+    products()
+    for _ in range(3):
+        X.copy_(torch.randn(K, N, device="cuda"))
+        version = B._version
+        R = step()
+        assert B._version > version
+        assert oracle.rel_fro(host(R), oracle.spmm_fp64(rp, ci, v, host(B).astype(np.float64))) <= TOL
+        products()
