@@ -14,8 +14,8 @@
 //                        all at once, then the second kind one after the other)
 //   up to 1024 products  one workgroup, hash table of 2048 slots in LDS
 //   up to 4096 products  B of at most 131,072 columns: a bitmap of the columns in LDS
-//                        (512 threads, see below); wider B: one workgroup, hash
-//                        table of 8192 slots in LDS
+//                        (see below), or, with up to 3,968, a sum to each of them; wider B: one
+//                        workgroup, hash table of 8192 slots in LDS
 //   more, B of at most 131,072 columns, and the two passes share what they find out
 //                        the products sorted by ranges of columns (see "the longest rows by
 //                        bins of columns")
