@@ -43,6 +43,7 @@ from . import scorch_ops_hip
 
 class _Writes(TorchDispatchMode):
     """Notes the tensors that operations run under it write in place (of a view, the tensor it is a view of)."""
+    supports_higher_order_operators = True      # (they run as without it; what they write is not noted)
 
     def __init__(self) -> None:
         super().__init__()

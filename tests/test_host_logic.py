@@ -748,3 +748,28 @@ def test_stretches_of_the_fused_bf16_kernel_on_either_side_of_every_rule(lens, h
 ])
 def test_pairs_of_the_fused_bf16_kernel_on_either_side_of_every_rule(lens, heads, want):
     assert scorch_ops_hip.pair_attention_items(lens, heads, 64) is want
+
+
+def test_writes_of_a_step_are_noted_whatever_their_form():
+    """What graphs.capture counts as written by every replay: in place, through views of views, as out= and in lists, by an
+    optimiser; not what is read, a temporary, or an inference tensor, which has no version counter."""
+    from scorch_amd.graphs import _Writes
+    whole, view, out, listed, read = (torch.zeros(4, 4) for _ in range(5))
+    weight = torch.nn.Parameter(torch.ones(3))
+    weight.grad = torch.ones(3)
+    step = torch.optim.SGD([weight], lr=0.1)
+    with torch.inference_mode():
+        inference = torch.zeros(4)
+    with _Writes() as writes:
+        whole.mul_(2.0)
+        view[1].t()[2:].add_(1.0)
+        torch.add(read, 1.0, out=out)
+        torch._foreach_add_([listed], 1.0)
+        step.step()
+        (read + 1.0).relu_()
+        with torch.inference_mode():
+            inference.add_(1.0)
+        branch = torch.cond(torch.tensor(True), lambda a: a + 1.0, lambda a: a - 1.0, (read,))
+    assert torch.equal(branch, read + 1.0)
+    found = writes.surviving()
+    assert {id(t) for t in found} == {id(t) for t in (whole, view, out, listed, weight)} and len(found) == 5
